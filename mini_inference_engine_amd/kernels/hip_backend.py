@@ -218,6 +218,34 @@ class HipBackend(KernelBackend):
                                            self._stream()))
         return y
 
+    # ---- products of the float32 path (csrc/gemm_f32.hip): one order of summation whatever the number of rows
+    F32_STORE, F32_ADD, F32_SWIGLU = 0, 1, 2
+
+    @staticmethod
+    def _f32_ok(x, w, bias, out_dtype) -> bool:
+        """Whether the 32-bit matrix-unit kernels take x w^T: float32 throughout and 16-byte pieces everywhere.  What
+        they refuse goes to mie_gemm_nt.  Nothing here depends on the number of rows."""
+        return (out_dtype == torch.float32 and x.dtype == torch.float32 and w.dtype == torch.float32
+                and w.shape[0] % 4 == 0 and w.shape[1] % 4 == 0 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
+                and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and (bias is None or (bias.dtype == torch.float32 and bias.is_contiguous() and bias.data_ptr() % 16 == 0)))
+
+    def _f32_product(self, x, w, epi, out, bias=None):
+        """out = x w^T, out += x w^T, or out = silu(gate) * up (w = [gate rows; up rows]); False: this many rows of a
+        gated product are better cut without the epilogue."""
+        lib = self.lib("gemm_f32")
+        M, K = x.shape
+        cols, part = w.shape[0], None
+        if M > 16:
+            units = lib.mie_f32_units(M, cols)
+            if units > 1:
+                part = torch.empty((units, M, cols), dtype=torch.float32, device=x.device)
+            elif epi == self.F32_SWIGLU:
+                return False
+        library.check(lib, lib.mie_gemm_f32(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), epi, _ptr(bias),
+                                            _ptr(part), M, cols // 2 if epi == self.F32_SWIGLU else cols, K, self._stream()))
+        return True
+
     # ---- few-row products of the bfloat16 path: one fused kernel each
     SKINNY_MAX_ROWS = 16      # the kernel's own limit (one tile of rows); a decode step of 16 rows of 512 keys at the
                               # benchmark's sizes takes 1.15 ms, one of 17 rows with the split product 1.27
@@ -377,6 +405,13 @@ class HipBackend(KernelBackend):
                 return self._lt_product(x, w, self.LT_BF16, torch.empty((M, N), dtype=torch.bfloat16, device=w.device))
             y = torch.nn.functional.linear(x, w, None if bias is None else bias.to(torch.bfloat16))
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
+        if self._f32_ok(x, w, bias, out_dtype):
+            if sink is not None:
+                self._f32_product(x, w, self.F32_ADD, sink.stream, bias)
+                return None if sink.norm_weight is None else Normed(self, None, sink.stream, sink.norm_weight, sink.norm_eps)
+            out = torch.empty((M, N), dtype=torch.float32, device=w.device)
+            self._f32_product(x, w, self.F32_STORE, out, bias)
+            return out
         return self._gemm(x, w, bias, out_dtype)
 
     def silu_mul(self, gu, intermediate):
@@ -406,6 +441,13 @@ class HipBackend(KernelBackend):
             out = torch.empty((x.shape[0], intermediate), dtype=torch.bfloat16, device=w_gate_up.device)
             self._skinny(x, w_gate_up, self.EPI_SWIGLU, out, intermediate)
             return out
+        if self.act_dtype == torch.float32 and intermediate % 4 == 0 and self._f32_ok(x, w_gate_up, None, torch.float32):
+            self._on_device(x, w_gate_up)
+            _rows_ok(x, "linear_silu_mul: x")
+            _rows_ok(w_gate_up, "linear_silu_mul: w")
+            out = torch.empty((x.shape[0], intermediate), dtype=torch.float32, device=w_gate_up.device)
+            if self._f32_product(x, w_gate_up, self.F32_SWIGLU, out):
+                return out
         return self.silu_mul(self.linear(x, w_gate_up), intermediate)
 
     ACT_CODES = {"none": 0, "silu": 1, "gelu_tanh": 2, "relu2": 3}

@@ -37,6 +37,10 @@ register_kernel_module("gemm", {
     "mie_clamped_glu": [P, L, P, L, I, I, I, F, F, F, I, P],
     "mie_clamped_glu_bf16": [P, L, P, L, I, I, F, F, F, P],
 })
+register_kernel_module("gemm_f32", {
+    "mie_f32_units": [I, I],
+    "mie_gemm_f32": [P, L, P, L, P, L, I, P, P, I, I, I, P],
+})
 register_kernel_module("grouped_gemm", {
     "mie_grouped_linear": [P, I, L, L, I, P, I, L, L, P, I, L, L, P, P, L, P, P, I, I, I, I, I, I, P, P],
     "mie_grouped_glu": [P, I, L, P, I, L, L, P, I, L, P, P, I, I, I, I, I, F, F, F, P, P],

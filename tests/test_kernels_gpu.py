@@ -112,6 +112,37 @@ def test_linear_float32_is_batch_invariant(ops):
     for a, b in ((0, 1), (63, 130), (199, 200), (17, 19)):
         assert torch.equal(ops[torch.float32].linear(x[a:b].contiguous(), w), whole[a:b])
 
+# (rows, K, N): few rows and many, K with quarters and segments missing (4, 16, 176), one step beyond a stage, tile edges
+F32_SHAPES = [(1, 2048, 2048), (16, 176, 64), (5, 4, 36), (17, 64, 132), (64, 1040, 260), (65, 528, 4100), (128, 2048, 96),
+              (300, 332, 640), (513, 256, 8196)]
+
+
+@pytest.mark.parametrize("shape", F32_SHAPES)
+def test_linear_float32_matrix_unit(ops, shape):
+    """The 32-bit products on the matrix unit: against 64 bits within the worst case of their chains (K / 16 terms in a
+    segment, 32 joins; half an ulp each of the sum of magnitudes), a row the same bits in any cut (few-row kernel, tiles,
+    units of K), the added and the gated form the same bits as the product and a step of its own."""
+    M, K, N = shape
+    o = ops[torch.float32]
+    torch.manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) / math.sqrt(K)
+    y = o.linear(x, w)
+    bound = (K / 16 + 32) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30
+    assert bool(((y.double() - x.double() @ w.double().T).abs() <= bound).all())
+    for a, b in ((0, 1), (M // 2, M // 2 + 1), (max(0, M - 17), M), (0, min(M, 16)), (0, M // 2 + 1)):
+        assert torch.equal(o.linear(x[a:b].contiguous(), w), y[a:b])
+    big = torch.cat([x, torch.randn(700, K, device=DEV)])
+    assert torch.equal(o.linear(big, w)[:M], y)
+    stream = torch.randn(M, N, device=DEV)
+    expect = stream + y
+    assert o.linear(x, w, add_to=stream) is None
+    assert torch.equal(stream, expect)
+    inter = N // 2
+    if inter % 4 == 0:
+        assert torch.equal(o.linear_silu_mul(x, w, inter), o.silu_mul(y, inter))
+    bias = torch.randn(N, device=DEV)
+    assert torch.equal(o.linear(x, w, bias=bias), y + bias)
+
 
 def test_linear_mixed_storage(ops):
     """A matrix stored in 32-bit beside bfloat16 activations: computed, not refused."""
