@@ -1680,6 +1680,9 @@ class HipBackend(KernelBackend):
             else:
                 library.check(lib, lib.mie_prefill_attention(*args, self._stream()))
             end = step.num_decode_rows
+        if (done < end and qkv.dtype == torch.float32 and not (force_generic or scored or has_sink or num_splits is not None)
+                and self._attention_f32(qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window)):
+            return out
         if done < end:
             lib = self.lib("attention")
             esz = qkv.element_size()
@@ -1694,6 +1697,38 @@ class HipBackend(KernelBackend):
             else:
                 library.check(lib, lib.mie_paged_attention(*args, self._stream()))
         return out
+
+    def _attention_f32(self, qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window) -> bool:
+        """Plain causal (windowed) softmax attention of a float32 step on the 32-bit matrix unit (csrc/attention_f32.hip);
+        False where that does not take the operands.  Head sizes, strides and alignment decide, never the step's rows: a
+        request's tokens take the same arithmetic in every step."""
+        T, window = qkv.shape[0], int(window or 0)
+        single = step.num_decode_rows
+        rows_known = step.row_start is not None and step.row_position is not None
+        if (D % 16 or D > 128 or page % 16 or qkv.stride(0) % 4 or any(t.data_ptr() % 16 for t in (qkv, k_cache, v_cache))
+                or (single < T and not rows_known) or single > 65535):
+            return False
+        lib = self.lib("attention_f32")
+        caches = (_ptr(qkv), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(bt), bt.shape[1])
+        if single:
+            seg = lib.mie_attention_f32_segment()
+            splits = -(-step.max_context // seg)
+            if window:
+                splits = min(splits, (window - 1) // seg + 2)
+            o_part = ml = None
+            if splits > 1:
+                o_part = torch.empty((single, Hq, splits, D), dtype=torch.float32, device=qkv.device)
+                ml = torch.empty((single, Hq, splits, 2), dtype=torch.float32, device=qkv.device)
+            library.check(lib, lib.mie_attention_f32_single(*caches, _ptr(step.token_row), _ptr(step.positions), single, Hq, Hkv, D,
+                                                            page, float(scale), window, splits, _ptr(o_part), _ptr(ml), self._stream()))
+        if single < T:
+            for name, t, n in (("row_start", step.row_start, step.num_rows + 1), ("row_position", step.row_position, step.num_rows)):
+                if t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous():
+                    raise ValueError(f"paged_attention: {name} must be contiguous int32 [{n}]")
+            library.check(lib, lib.mie_attention_f32_portions(*caches, _ptr(step.row_start), _ptr(step.row_position), single,
+                                                              step.num_rows, step.max_row_tokens, Hq, Hkv, D, page, float(scale),
+                                                              window, self._stream()))
+        return True
 
     def sample(self, logits, temperatures, seeds, counters, out=None):
         self._on_device(logits, temperatures, seeds, counters, out)

@@ -41,6 +41,11 @@ register_kernel_module("gemm_f32", {
     "mie_f32_units": [I, I],
     "mie_gemm_f32": [P, L, P, L, P, L, I, P, P, I, I, I, P],
 })
+register_kernel_module("attention_f32", {
+    "mie_attention_f32_segment": [],
+    "mie_attention_f32_single": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, P, P],
+    "mie_attention_f32_portions": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, P],
+})
 register_kernel_module("grouped_gemm", {
     "mie_grouped_linear": [P, I, L, L, I, P, I, L, L, P, I, L, L, P, P, L, P, P, I, I, I, I, I, I, P, P],
     "mie_grouped_glu": [P, I, L, P, I, L, L, P, I, L, P, P, I, I, I, I, I, F, F, F, P, P],

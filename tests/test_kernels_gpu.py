@@ -1015,6 +1015,30 @@ def test_attention_ignores_stale_pages(ops):
     assert torch.equal(clean, dirty)
 
 
+# heads, kv heads, head size, page: groups that fill 16 queries, leave some of them empty, and take several tiles
+@pytest.mark.parametrize("window", [None, 1, 100, 128, 300])
+@pytest.mark.parametrize("geom", [(32, 4, 64, 16), (3, 1, 32, 16), (5, 5, 48, 32), (40, 2, 16, 16), (16, 1, 128, 16), (10, 2, 112, 48)])
+def test_attention_float32_matrix_unit(ops, geom, window):
+    """The 32-bit attention on the matrix unit, against 64 bits and against itself: a request's tokens as one portion, as
+    portions cut in the middle of a segment of 128 keys, and one by one give the same bits."""
+    Hq, Hkv, D, page = geom
+    o, n = ops[torch.float32], 389
+    q, kc, vc, group, step = paged_setup([n, 131], [n, 131], Hq, Hkv, D, page, torch.float32, seed=D)
+    whole, expect = run_attention(ops, torch.float32, q, kc, vc, group, step, Hq, Hkv, D, 1 / math.sqrt(D), window)
+    torch.testing.assert_close(whole.double(), expect, **ATT_TOL[torch.float32])
+    for a, b in ((0, 2), (2, 129), (129, 256), (256, n)):
+        part = SimpleNamespace(token_row=step.token_row[a:b], positions=step.positions[a:b], num_rows=1, max_context=b, num_tokens=b - a,
+                               num_decode_rows=0, max_row_tokens=b - a, row_start=torch.tensor([0, b - a], dtype=torch.int32, device=DEV),
+                               row_position=torch.tensor([a], dtype=torch.int32, device=DEV))
+        assert torch.equal(o.paged_attention(q[a:b], Hq, Hkv, D, kc, vc, group, part, 1 / math.sqrt(D), window), whole[a:b])
+    for bound in (n, 2000):                     # a static bound on the context, as under capture
+        wide = SimpleNamespace(block_tables=torch.nn.functional.pad(group.block_tables, (0, 2000 // page + 1 - group.block_tables.shape[1])))
+        wide.max_blocks = wide.block_tables.shape[1]
+        single = SimpleNamespace(token_row=step.token_row, positions=step.positions, num_rows=2, max_context=bound, num_tokens=n + 131,
+                                 num_decode_rows=n + 131, max_row_tokens=1, row_start=None, row_position=None)
+        assert torch.equal(o.paged_attention(q, Hq, Hkv, D, kc, vc, wide, single, 1 / math.sqrt(D), window), whole)
+
+
 # ------------------------------------------------------------------- sampling
 def test_sample_greedy_and_ties(ops):
     torch.manual_seed(0)
