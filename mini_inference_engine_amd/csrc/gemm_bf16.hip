@@ -37,7 +37,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // what a k-step beyond a wave's range or beyond K loads instead of weights, so that every load is unconditional
-__device__ __align__(64) const uint32_t mie_zero_words[16] = {0};
+__device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
 
 // wait until at most n vector memory loads of this wave are still on their way
 #define SG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
@@ -50,20 +50,18 @@ constexpr int RING_U = 2;         // k-steps a slot of a wave's ring
 // in one piece of assembly: the compiler knows nothing of the loads that write the LDS, so a read it could see
 // would make it wait for every load on its way, and it must never see a register whose value is still to arrive.
 typedef uint32_t sg_u32x4 __attribute__((ext_vector_type(4)));
-template <int U> struct RingRead;
-template <> struct RingRead<2> {
-  static __device__ __forceinline__ void run(uint32_t at, sg_u32x4 (&f)[4]) {
-    asm volatile(
-      "ds_read_b128 %0, %4\n\t"
-      "ds_read_b128 %1, %4 offset:1024\n\t"
-      "ds_read_b128 %2, %4 offset:2048\n\t"
-      "ds_read_b128 %3, %4 offset:3072\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
-      : "v"(at)
-      : "memory");
-  }
-};
+// at0 / at1: this lane's piece of the slot's first / second k-step.
+__device__ __forceinline__ void ring_read(uint32_t at0, uint32_t at1, sg_u32x4 (&f)[4]) {
+  asm volatile(
+    "ds_read_b128 %0, %4\n\t"
+    "ds_read_b128 %1, %4 offset:2048\n\t"
+    "ds_read_b128 %2, %5\n\t"
+    "ds_read_b128 %3, %5 offset:2048\n\t"
+    "s_waitcnt lgkmcnt(0)"
+    : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
+    : "v"(at0), "v"(at1)
+    : "memory");
+}
 
 // The wait of round `it` < SLOTS - 1 (the counter's limit must be a constant of the instruction).
 template <int SLOTS, int IT> struct RingStart {
@@ -136,7 +134,7 @@ template <int EPI, bool NF, int SLOTS>
 __global__ void __launch_bounds__(SG_THREADS)
 skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, void* __restrict__ outv,
                    long ldo, int M, int N, int K, int up_offset, RopeArgs rope, NormArgs nf) {
-  constexpr int SLOT_BYTES = RING_U * 2 * 1024;            // a k-step: the weight fragment, then the x fragment, 1 KB each
+  constexpr int SLOT_BYTES = RING_U * 2 * 1024;            // 16 weight rows of 64 k (128 bytes), then 16 x rows
   constexpr int WAVE_BYTES = SLOTS * SLOT_BYTES;
   constexpr int L = RING_U * 2;                            // loads a slot
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
@@ -147,17 +145,18 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
   const int col = lane & 15, kb = lane >> 4;
   const int tile = blockIdx.x;
   const int ksteps = (K + 31) >> 5;
-  const int per_wave = (ksteps + SG_WAVES - 1) / SG_WAVES;
+  const int per_wave = ((ksteps + SG_WAVES - 1) / SG_WAVES + 1) & ~1;       // whole cache lines of a row
   const int ks0 = wave * per_wave;
   const int ks1 = ks0 + per_wave < ksteps ? ks0 + per_wave : ksteps;
 
-  // What this lane brings in: row lrow (of the weight tile; of x), k-block lkb of every k-step.  And the one
+  // What this lane brings in: rows lrow and lrow + 8 (of the weight tile; of x), block lblk of every 64 k.  And the one
   // result this thread owns after the waves are summed: x row m, column c of the tile.  The gather of x's
   // rows, if there is one, and the positions are the first things asked for: addresses depend on them.
-  const int lrow = lane >> 2, lkb = (lane & 3) ^ ((lrow >> 2) & 3);
+  const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;
   const int m = threadIdx.x >> 4, c = threadIdx.x & 15;
   const bool gather = NF && EPI != EPI_ADD && nf.rows;
-  const int lsrc = lrow < M ? (gather ? nf.rows[lrow] : lrow) : 0;
+  const int lsrc0 = lrow < M ? (gather ? nf.rows[lrow] : lrow) : 0;
+  const int lsrc1 = lrow + 8 < M ? (gather ? nf.rows[lrow + 8] : lrow + 8) : lsrc0;
   const int msrc = m < M ? (gather ? nf.rows[m] : m) : 0;
 
   bool ok;
@@ -175,32 +174,33 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
 
   // The ring.  Slots beyond the wave's range load zeros only, so that it is always filled and drained the
   // same way.
-  bool lok;
-  const long lwr = tile_column<EPI>(tile, lrow, N, up_offset, rope.D, lok);
-  const bf16* wsrc = W + (size_t)(lok ? lwr : 0) * ldw + lkb * 8;   // a row that does not exist is never stored
-  const bf16* xsrc = X + (size_t)lsrc * ldx + lkb * 8;              // rows beyond M read row 0 along with the lanes that own it
-  const bf16* zero_lane = reinterpret_cast<const bf16*>(mie_zero_words) + lkb * 8;   // per lane, so that choosing it is a select
+  bool lok0, lok1;
+  const long lwr0 = tile_column<EPI>(tile, lrow, N, up_offset, rope.D, lok0);
+  const long lwr1 = tile_column<EPI>(tile, lrow + 8, N, up_offset, rope.D, lok1);
+  // a row that does not exist is never stored; rows beyond M read another row along with the lanes that own it
+  const bf16* wsrc0 = W + (size_t)(lok0 ? lwr0 : 0) * ldw + lblk * 8;
+  const bf16* wsrc1 = W + (size_t)(lok1 ? lwr1 : 0) * ldw + lblk * 8;
+  const bf16* xsrc0 = X + (size_t)lsrc0 * ldx + lblk * 8;
+  const bf16* xsrc1 = X + (size_t)lsrc1 * ldx + lblk * 8;
+  const bf16* zero_lane = reinterpret_cast<const bf16*>(mie_zero_words) + lblk * 8;  // per lane, so that choosing it is a select
   char* mine = ring_lds + wave * WAVE_BYTES;
-  // what: 1 the weight fragments of slot s, 2 the x fragments, 3 both (weight, x, weight, x)
+  // what: 1 the weights of slot s, 2 its x, 3 both
   auto issue = [&](int s, int what) {
     char* base = mine + (s % SLOTS) * SLOT_BYTES;
     const int ks = ks0 + s * RING_U;
+    const bool kok = ks + (lblk >> 2) < ks1 && ks * 32 + lblk * 8 < K;
+    const size_t k = (size_t)ks * 32;
+    const bf16* src[4] = {kok ? wsrc0 + k : zero_lane, kok ? wsrc1 + k : zero_lane, kok ? xsrc0 + k : zero_lane, kok ? xsrc1 + k : zero_lane};
 #pragma unroll
-    for (int u = 0; u < RING_U; ++u) {
-      const bool kok = ks + u < ks1 && (ks + u) * 32 + lkb * 8 < K;
-      const bf16* a = kok ? wsrc + (size_t)(ks + u) * 32 : zero_lane;
-      const bf16* b = kok ? xsrc + (size_t)(ks + u) * 32 : zero_lane;
-      if (what & 1)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)a,
-                                         (__attribute__((address_space(3))) void*)(base + (2 * u) * 1024), 16, 0, 0);
-      if (what & 2)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)b,
-                                         (__attribute__((address_space(3))) void*)(base + (2 * u + 1) * 1024), 16, 0, 0);
-    }
+    for (int j = 0; j < 4; ++j)
+      if (what & (j < 2 ? 1 : 2))
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[j],
+                                         (__attribute__((address_space(3))) void*)(base + j * 1024), 16, 0, 0);
   };
   const int rounds = ks1 > ks0 ? (ks1 - ks0 + RING_U - 1) / RING_U : 0;
-  // this lane's piece of a fragment: row col, block kb
-  const uint32_t at0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine + (col * 4 + (kb ^ ((col >> 2) & 3))) * 16;
+  // this lane's pieces of a slot: row col, blocks kb and 4 + kb
+  const uint32_t row0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine + col * 128;
+  const uint32_t at0 = row0 + (kb ^ (col & 7)) * 16, at1 = row0 + ((4 + kb) ^ (col & 7)) * 16;
   // The ring starts with the weights of its first slots; their x follows below, after what the epilogue reads
   // has been asked for: all that waits for the row numbers of a gather, the weights do not.
 #pragma unroll
@@ -245,7 +245,7 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     if (it >= SLOTS - 1) SG_VMCNT((SLOTS - 1) * L);
     else RingStart<SLOTS, 0>::wait(it);
     sg_u32x4 f[2 * RING_U];
-    RingRead<RING_U>::run(at0 + (it % SLOTS) * SLOT_BYTES, f);
+    ring_read(at0 + (it % SLOTS) * SLOT_BYTES, at1 + (it % SLOTS) * SLOT_BYTES, f);
 #pragma unroll
     for (int u = 0; u < RING_U; ++u)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f[2 * u]), __builtin_bit_cast(bf16x8, f[2 * u + 1]),
