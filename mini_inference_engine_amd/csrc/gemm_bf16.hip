@@ -13,13 +13,16 @@
 // values, 16 bytes) of row r.  Loaded in that order, a quarter wave (16 lanes) touches 16 cache lines for 16
 // bytes each, and the address unit, which looks lines up one at a time, is then what bounds the kernel: the x
 // loads alone (all of them hits) cost a seventh to a third of its time, and the weights stream at 4.2 to
-// 4.7 TB/s where a plain read of the same bytes runs at 5.4 to 5.8.  So the loads are issued in the order lane
-// 4 r + b (a quarter wave reads 64 contiguous bytes of 4 rows) and write the wave's own piece of the LDS
-// directly (no registers, nothing the compiler waits for): a ring of slots of two k-steps, all but one on their
-// way while that one is multiplied.  Within a row the four blocks are permuted (block b at 16-byte slot
-// 4 r + (b ^ (r / 4) % 4)), so that the fragment reads (lane 16 b + r) are spread over all banks.  No barrier
-// in the loop: a wave reads only what it brought in itself.  (The same order with nontemporal loads reads a
-// fifth faster still when nothing else is loaded, but slower beside the x loads: measured, not used.)
+// 4.7 TB/s where a plain read of the same bytes runs at 5.4 to 5.8.  So a load takes whole cache lines, 8 rows of
+// 64 k (lane 8 r + b), and writes the wave's own piece of the LDS directly (no registers, nothing the compiler
+// waits for): a ring of slots of two k-steps, all but one on their way while that one is multiplied.  Within a
+// row the eight blocks are permuted (block b at 16-byte slot 8 r + (b ^ r % 8)), so that the fragment reads
+// (lane 16 b + r) are spread over all banks.  No barrier in the loop: a wave reads only what it brought in itself.
+// Up to 8 rows bring in half as much x and a slot more of the weights.  Measured (decode steps of 1 / 8 rows at
+// TinyLlama sizes, 8 rows at four layers of Llama-3-8B's, us): half lines, 16 rows of 64 bytes a load, 936 / 1064 /
+// 821; whole lines 927 / 1021 / 795; the smaller slots beside that 898 / 999 / 786.
+// (Half lines with nontemporal loads read a fifth faster still when nothing else is loaded, but slower beside the
+// x loads: measured, not used.)
 //
 // Epilogues: STORE (bfloat16 or float32 y), ADD (r[m, n] += y, the residual add of the 32-bit stream),
 //   SWIGLU (W holds gate rows then up rows; a tile is 8 gate rows and the matching 8 up rows, and the
@@ -50,24 +53,24 @@ constexpr int RING_U = 2;         // k-steps a slot of a wave's ring
 // in one piece of assembly: the compiler knows nothing of the loads that write the LDS, so a read it could see
 // would make it wait for every load on its way, and it must never see a register whose value is still to arrive.
 typedef uint32_t sg_u32x4 __attribute__((ext_vector_type(4)));
-// at0 / at1: this lane's piece of the slot's first / second k-step.
-__device__ __forceinline__ void ring_read(uint32_t at0, uint32_t at1, sg_u32x4 (&f)[4]) {
+// w0 / w1, x0 / x1: this lane's pieces of the slot's first and second k-step.
+__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1, uint32_t x1, sg_u32x4 (&f)[4]) {
   asm volatile(
     "ds_read_b128 %0, %4\n\t"
-    "ds_read_b128 %1, %4 offset:2048\n\t"
-    "ds_read_b128 %2, %5\n\t"
-    "ds_read_b128 %3, %5 offset:2048\n\t"
+    "ds_read_b128 %1, %5\n\t"
+    "ds_read_b128 %2, %6\n\t"
+    "ds_read_b128 %3, %7\n\t"
     "s_waitcnt lgkmcnt(0)"
     : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
-    : "v"(at0), "v"(at1)
+    : "v"(w0), "v"(x0), "v"(w1), "v"(x1)
     : "memory");
 }
 
 // The wait of round `it` < SLOTS - 1 (the counter's limit must be a constant of the instruction).
-template <int SLOTS, int IT> struct RingStart {
+template <int SLOTS, int XL, int IT> struct RingStart {
   static __device__ __forceinline__ void wait(int it) {
-    if (it == IT) SG_VMCNT((SLOTS - 2 - IT) * RING_U + (IT + 1) * RING_U * 2);
-    else if constexpr (IT + 1 < SLOTS - 1) RingStart<SLOTS, IT + 1>::wait(it);
+    if (it == IT) SG_VMCNT((SLOTS - 2 - IT) * XL + (IT + 1) * (2 + XL));
+    else if constexpr (IT + 1 < SLOTS - 1) RingStart<SLOTS, XL, IT + 1>::wait(it);
   }
 };
 
@@ -130,13 +133,14 @@ __device__ __forceinline__ long tile_column(int tile, int c, int N, int up_offse
   return n;
 }
 
-template <int EPI, bool NF, int SLOTS>
+// XL: loads of x a slot: one for up to 8 rows (columns 8 to 15 of the tile then take rows 0 to 7 again), else two.
+template <int EPI, bool NF, int SLOTS, int XL>
 __global__ void __launch_bounds__(SG_THREADS)
 skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, void* __restrict__ outv,
                    long ldo, int M, int N, int K, int up_offset, RopeArgs rope, NormArgs nf) {
-  constexpr int SLOT_BYTES = RING_U * 2 * 1024;            // 16 weight rows of 64 k (128 bytes), then 16 x rows
+  constexpr int L = 2 + XL;                                // loads a slot
+  constexpr int SLOT_BYTES = L * 1024;                     // 16 weight rows of 64 k (128 bytes), then the x rows
   constexpr int WAVE_BYTES = SLOTS * SLOT_BYTES;
-  constexpr int L = RING_U * 2;                            // loads a slot
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(16) char ring_lds[];         // WAVE_BYTES a wave
   __shared__ float s_acc[SG_WAVES][256];
@@ -192,15 +196,16 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     const size_t k = (size_t)ks * 32;
     const bf16* src[4] = {kok ? wsrc0 + k : zero_lane, kok ? wsrc1 + k : zero_lane, kok ? xsrc0 + k : zero_lane, kok ? xsrc1 + k : zero_lane};
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < L; ++j)
       if (what & (j < 2 ? 1 : 2))
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[j],
                                          (__attribute__((address_space(3))) void*)(base + j * 1024), 16, 0, 0);
   };
   const int rounds = ks1 > ks0 ? (ks1 - ks0 + RING_U - 1) / RING_U : 0;
   // this lane's pieces of a slot: row col, blocks kb and 4 + kb
-  const uint32_t row0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine + col * 128;
-  const uint32_t at0 = row0 + (kb ^ (col & 7)) * 16, at1 = row0 + ((4 + kb) ^ (col & 7)) * 16;
+  const uint32_t ring0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine;
+  const uint32_t blk0 = (kb ^ (col & 7)) * 16, blk1 = ((4 + kb) ^ (col & 7)) * 16;
+  const uint32_t wrow0 = ring0 + col * 128, xrow0 = ring0 + 2048 + (XL == 1 ? col & 7 : col) * 128;
   // The ring starts with the weights of its first slots; their x follows below, after what the epilogue reads
   // has been asked for: all that waits for the row numbers of a gather, the weights do not.
 #pragma unroll
@@ -243,9 +248,10 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     // SLOTS - 1 slots after it; before, the x fragments of the first slots that follow its own and the slots
     // issued in the loop so far.  (Anything else asked for in between only makes this wait for more.)
     if (it >= SLOTS - 1) SG_VMCNT((SLOTS - 1) * L);
-    else RingStart<SLOTS, 0>::wait(it);
+    else RingStart<SLOTS, XL, 0>::wait(it);
     sg_u32x4 f[2 * RING_U];
-    ring_read(at0 + (it % SLOTS) * SLOT_BYTES, at1 + (it % SLOTS) * SLOT_BYTES, f);
+    const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
+    ring_read(w0 + blk0, x0 + blk0, w0 + blk1, x0 + blk1, f);
 #pragma unroll
     for (int u = 0; u < RING_U; ++u)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f[2 * u]), __builtin_bit_cast(bf16x8, f[2 * u + 1]),
@@ -350,13 +356,13 @@ static int allow_lds(const void* kernel, int bytes) {
   return 0;
 }
 
-template <bool NF, int SLOTS>
+template <bool NF, int SLOTS, int XL>
 static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
                       long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& nf) {
-  constexpr int lds = SG_WAVES * SLOTS * RING_U * 2 * 1024;
+  constexpr int lds = SG_WAVES * SLOTS * (2 + XL) * 1024;
 #define SG_LAUNCH(E)                                                                                                    \
   {                                                                                                                     \
-    auto kernel = skinny_gemm_kernel<E, NF, SLOTS>;                                                                     \
+    auto kernel = skinny_gemm_kernel<E, NF, SLOTS, XL>;                                                                     \
     if (allow_lds((const void*)kernel, lds)) return -1;                                                                 \
     hipLaunchKernelGGL(kernel, grid, dim3(SG_THREADS), lds, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, nf); \
   }
@@ -375,8 +381,8 @@ static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx
   return 0;
 }
 
-// Slots a wave's ring has.  Four (64 KB a workgroup, two workgroups a compute unit) stream best; three (48 KB,
-// three workgroups a compute unit) when that lets all tiles run at once instead of in two rounds.  Chosen from
+// Slots a wave's ring has.  Four (64 KB a workgroup, two workgroups a compute unit; five of 60 KB for up to 8 rows) stream
+// best; three (48 KB, three workgroups a compute unit; four of 48 KB for up to 8 rows) when that lets all tiles run at once instead of in two rounds.  Chosen from
 // the weight's shape alone, never from the batch (the sums do not depend on it anyway).
 static int compute_units() {
   static int units[64];
@@ -396,11 +402,12 @@ static int slots_for(int tiles) {
 static int launch_rows(int tiles, int epi, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
                        long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& n, bool fused) {
   dim3 grid(tiles);
-  if (slots_for(tiles) == 3)
-    return fused ? launch_epi<true, 3>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n)
-                 : launch_epi<false, 3>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n);
-  return fused ? launch_epi<true, 4>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n)
-            : launch_epi<false, 4>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n);
+  const bool three = slots_for(tiles) == 3;
+#define SG_ROWS(NF, SLOTS, XL) launch_epi<NF, SLOTS, XL>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n)
+  if (M <= 8)             // a slot is a quarter smaller: as many workgroups a compute unit with one slot more
+    return three ? (fused ? SG_ROWS(true, 4, 1) : SG_ROWS(false, 4, 1)) : (fused ? SG_ROWS(true, 5, 1) : SG_ROWS(false, 5, 1));
+  return three ? (fused ? SG_ROWS(true, 3, 2) : SG_ROWS(false, 3, 2)) : (fused ? SG_ROWS(true, 4, 2) : SG_ROWS(false, 4, 2));
+#undef SG_ROWS
 }
 
 static int check_operands(const char* what, const void* X, long ldx, const void* W, long ldw, int M, int K) {
