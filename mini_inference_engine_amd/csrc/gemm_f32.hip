@@ -20,8 +20,8 @@
 //   whose sums go to memory and meet in reduce_f32_kernel.
 //
 // Measured on MI355X against the vector-unit kernel gemm_nt_kernel (gemm.hip) with its 64 x 64 tiles walking all of K:
-// 4 rows of [2048, 2048] / [2048, 5632] 330 / 900 -> 9 / 18 us (1.9 / 2.6 TB/s of weights), of [11264, 2048] with the gate
-// 340 -> 27 (3.4 TB/s); 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225 (105 TFLOP/s of the 157 that
+// a step's products at 4 rows 47 -> 6.1 ms with the kernels beside them unchanged, and whole cache lines a load (half lines and
+// 16 rows of x before) took a whole step 2,057 -> 1,853 us; 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225 (105 TFLOP/s of the 157 that
 // the 32-bit matrix unit has).  Error against 64 bits of a 22-layer step's logits 2.5e-6 -> 2.1e-6.
 #include "common.hpp"
 #include <mutex>
@@ -31,7 +31,7 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __align__(64) const uint32_t mie_zero_words[16] = {0};
+__device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
 
 #define GF_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
@@ -65,33 +65,33 @@ enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2 };
 
 // ------------------------------------------------------------------------------------------------ few rows
 constexpr int GF_U = 2;                       // steps a slot of a wave's ring
-constexpr int GF_SLOTS = 4;
-constexpr int GF_SLOT_BYTES = GF_U * 2 * 1024;
 
-// The fragments of a slot (weights, x, weights, x) out of the LDS, read and waited for in one piece of assembly: the
-// compiler knows nothing of the loads that write the LDS and would wait for all of them at a read it could see.
-__device__ __forceinline__ void ring_read(uint32_t at, u32x4 (&f)[4]) {
+// The fragments of a slot out of the LDS, read and waited for in one piece of assembly: the compiler knows nothing of the
+// loads that write the LDS and would wait for all of them at a read it could see.
+__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1, uint32_t x1, u32x4 (&f)[4]) {
   asm volatile(
     "ds_read_b128 %0, %4\n\t"
-    "ds_read_b128 %1, %4 offset:1024\n\t"
-    "ds_read_b128 %2, %4 offset:2048\n\t"
-    "ds_read_b128 %3, %4 offset:3072\n\t"
+    "ds_read_b128 %1, %5\n\t"
+    "ds_read_b128 %2, %6\n\t"
+    "ds_read_b128 %3, %7\n\t"
     "s_waitcnt lgkmcnt(0)"
     : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
-    : "v"(at)
+    : "v"(w0), "v"(x0), "v"(w1), "v"(x1)
     : "memory");
 }
 
+// XL: loads of x a slot: one for up to 8 rows (columns 8 to 15 of the tile then take rows 0 to 7 again), else two.
 // SWIGLU: W is gate rows then up rows (up_offset apart); a tile is 8 gate rows and the 8 up rows of the same columns.
-template <int EPI, int WAVES>
+template <int EPI, int WAVES, int SLOTS, int XL>
 __global__ void __launch_bounds__(WAVES * 64)
 skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ out,
                   long ldo, const float* __restrict__ bias, int M, int N, int K, int up_offset) {
   constexpr int SPW = 16 / WAVES;             // segments a wave
-  constexpr int L = GF_U * 2;                 // loads a slot
+  constexpr int L = 2 + XL, SLOT_BYTES = L * 1024;       // loads a slot: 16 weight rows of 128 bytes, then the x rows
+  static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(16) char gf_lds[];
-  char* ring = gf_lds;                                            // WAVES * GF_SLOTS slots
-  float* s_acc = reinterpret_cast<float*>(gf_lds + WAVES * GF_SLOTS * GF_SLOT_BYTES);    // [16][256]
+  char* ring = gf_lds;                                            // WAVES * SLOTS slots
+  float* s_acc = reinterpret_cast<float*>(gf_lds);                // [16][256], once every wave is done with its ring
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tile = blockIdx.x;
   const KCut cut = k_cut(K);
@@ -103,41 +103,46 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
     for (int i = 0; i < SPW; ++i) segment_range(cut, wave * SPW + i, b, seg_end[i]);
     ks1 = seg_end[SPW - 1];
   }
-  const int lrow = lane >> 2, lkb = (lane & 3) ^ ((lrow >> 2) & 3);
-  int wr = EPI == GF_SWIGLU ? tile * 8 + (lrow & 7) : tile * 16 + lrow;
-  if (wr >= N) wr = 0;                        // a row that does not exist is never stored
-  if (EPI == GF_SWIGLU) wr += (lrow >> 3) * up_offset;
-  const float* wsrc = W + (size_t)wr * ldw + lkb * 4;
-  const float* xsrc = X + (size_t)(lrow < M ? lrow : 0) * ldx + lkb * 4;
-  const float* zero = reinterpret_cast<const float*>(mie_zero_words) + lkb * 4;
-  char* mine = ring + wave * GF_SLOTS * GF_SLOT_BYTES;
-  auto issue = [&](int s) {
-    char* base = mine + (s % GF_SLOTS) * GF_SLOT_BYTES;
-    const int ks = ks0 + s * GF_U;
+  const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;            // this lane's place in a load of 8 rows
+  const float *wsrc[2], *xsrc[2];
 #pragma unroll
-    for (int u = 0; u < GF_U; ++u) {
-      const bool kok = ks + u < ks1 && (ks + u) * 16 + lkb * 4 < K;
-      const float* a = kok ? wsrc + (size_t)(ks + u) * 16 : zero;
-      const float* b = kok ? xsrc + (size_t)(ks + u) * 16 : zero;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)a,
-                                       (__attribute__((address_space(3))) void*)(base + (2 * u) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)b,
-                                       (__attribute__((address_space(3))) void*)(base + (2 * u + 1) * 1024), 16, 0, 0);
-    }
+  for (int j = 0; j < 2; ++j) {
+    const int r = lrow + 8 * j;
+    int wr = EPI == GF_SWIGLU ? tile * 8 + (r & 7) : tile * 16 + r;
+    if (wr >= N) wr = 0;                      // a row that does not exist is never stored
+    if (EPI == GF_SWIGLU) wr += (r >> 3) * up_offset;
+    wsrc[j] = W + (size_t)wr * ldw + lblk * 4;
+    xsrc[j] = X + (size_t)(r < M ? r : 0) * ldx + lblk * 4;
+  }
+  const float* zero = reinterpret_cast<const float*>(mie_zero_words) + lblk * 4;
+  char* mine = ring + wave * SLOTS * SLOT_BYTES;
+  auto issue = [&](int s) {
+    char* base = mine + (s % SLOTS) * SLOT_BYTES;
+    const int ks = ks0 + s * GF_U;
+    const bool kok = ks + (lblk >> 2) < ks1 && ks * 16 + lblk * 4 < K;
+    const size_t k = (size_t)ks * 16;
+    const float* src[4] = {kok ? wsrc[0] + k : zero, kok ? wsrc[1] + k : zero, kok ? xsrc[0] + k : zero, kok ? xsrc[1] + k : zero};
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[j],
+                                       (__attribute__((address_space(3))) void*)(base + j * 1024), 16, 0, 0);
   };
 #pragma unroll
-  for (int s = 0; s < GF_SLOTS - 1; ++s) issue(s);
+  for (int s = 0; s < SLOTS - 1; ++s) issue(s);
   const int col = lane & 15, kb = lane >> 4;
-  const uint32_t at0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine + (col * 4 + (kb ^ ((col >> 2) & 3))) * 16;
+  const uint32_t ring0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine;
+  const uint32_t blk0 = (kb ^ (col & 7)) * 16, blk1 = ((4 + kb) ^ (col & 7)) * 16;
+  const uint32_t wrow0 = ring0 + col * 128, xrow0 = ring0 + 2048 + (XL == 1 ? col & 7 : col) * 128;
   f32x4 acc[SPW];
 #pragma unroll
   for (int i = 0; i < SPW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int rounds = ks1 > ks0 ? (ks1 - ks0 + GF_U - 1) / GF_U : 0;
   for (int it = 0; it < rounds; ++it) {
-    issue(it + GF_SLOTS - 1);                 // into the slot that was read a round ago
-    GF_VMCNT((GF_SLOTS - 1) * L);             // slot `it` has landed
+    issue(it + SLOTS - 1);                    // into the slot that was read a round ago
+    GF_VMCNT((SLOTS - 1) * L);                // slot `it` has landed
     u32x4 f[2 * GF_U];
-    ring_read(at0 + (it % GF_SLOTS) * GF_SLOT_BYTES, f);
+    const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
+    ring_read(w0 + blk0, x0 + blk0, w0 + blk1, x0 + blk1, f);
 #pragma unroll
     for (int u = 0; u < GF_U; ++u) {
       const int ks = ks0 + it * GF_U + u;     // a step beyond ks1 loaded zeros and joins the last segment: it adds nothing
@@ -148,7 +153,8 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
           acc[i] = step_mfma(w4, x4, acc[i]);
     }
   }
-  GF_VMCNT(0);                                // nothing of this wave may still be writing the LDS when it ends
+  GF_VMCNT(0);                                // nothing of this wave is writing the LDS any more
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < SPW; ++i) *reinterpret_cast<f32x4*>(s_acc + (wave * SPW + i) * 256 + lane * 4) = acc[i];
   __syncthreads();
@@ -408,11 +414,20 @@ template <int EPI>
 static int launch_skinny(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int M, int N,
                          int K, hipStream_t s) {
   const int tiles = EPI == GF_SWIGLU ? (N + 7) / 8 : (N + 15) / 16;
-  const int waves = tiles <= 256 ? 8 : 4;
-  const int lds = waves * GF_SLOTS * GF_SLOT_BYTES + 16 * 256 * 4;
-  auto kernel = waves == 8 ? skinny_f32_kernel<EPI, 8> : skinny_f32_kernel<EPI, 4>;
-  if (allow_lds((const void*)kernel, lds)) return -1;
-  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(waves * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, M, N, K, N);
+  // 8 waves, 144 KB of ring and one workgroup a compute unit, or 4 waves, 48 KB and three
+#define GF_SKINNY(WAVES, SLOTS, XL)                                                                                       \
+  {                                                                                                                       \
+    auto kernel = skinny_f32_kernel<EPI, WAVES, SLOTS, XL>;                                                               \
+    constexpr int lds = WAVES * SLOTS * (2 + XL) * 1024;                                                                  \
+    if (allow_lds((const void*)kernel, lds)) return -1;                                                                   \
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, M, N, K, N);        \
+  }
+  if (tiles <= 256) {
+    if (M <= 8) GF_SKINNY(8, 6, 1) else GF_SKINNY(8, 4, 2)
+  } else {
+    if (M <= 8) GF_SKINNY(4, 4, 1) else GF_SKINNY(4, 3, 2)
+  }
+#undef GF_SKINNY
   MIE_CHECK_LAUNCH("skinny_f32");
   return 0;
 }
