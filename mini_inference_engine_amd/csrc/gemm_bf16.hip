@@ -20,9 +20,8 @@
 // (lane 16 b + r) are spread over all banks.  No barrier in the loop: a wave reads only what it brought in itself.
 // Up to 8 rows bring in half as much x and a slot more of the weights.  Measured (decode steps of 1 / 8 rows at
 // TinyLlama sizes, 8 rows at four layers of Llama-3-8B's, us): half lines, 16 rows of 64 bytes a load, 936 / 1064 /
-// 821; whole lines 927 / 1021 / 795; the smaller slots beside that 898 / 999 / 786.
-// (Half lines with nontemporal loads read a fifth faster still when nothing else is loaded, but slower beside the
-// x loads: measured, not used.)
+// 821; whole lines 927 / 1021 / 795; the smaller slots beside that 898 / 999 / 786; the weights by nontemporal loads
+// beside that 862 / 995 / 755 (with half lines the hint had made the kernel slower: it dropped the line's other half).
 //
 // Epilogues: STORE (bfloat16 or float32 y), ADD (r[m, n] += y, the residual add of the 32-bit stream),
 //   SWIGLU (W holds gate rows then up rows; a tile is 8 gate rows and the matching 8 up rows, and the
@@ -44,6 +43,8 @@ __device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
 
 // wait until at most n vector memory loads of this wave are still on their way
 #define SG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
+
+constexpr int SG_NONTEMPORAL = 2;  // the hint of loads whose lines nobody reads again: the weights
 
 constexpr int SG_WAVES = 4;       // waves a workgroup
 constexpr int SG_THREADS = SG_WAVES * 64;
@@ -196,10 +197,12 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     const size_t k = (size_t)ks * 32;
     const bf16* src[4] = {kok ? wsrc0 + k : zero_lane, kok ? wsrc1 + k : zero_lane, kok ? xsrc0 + k : zero_lane, kok ? xsrc1 + k : zero_lane};
 #pragma unroll
-    for (int j = 0; j < L; ++j)
-      if (what & (j < 2 ? 1 : 2))
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[j],
-                                         (__attribute__((address_space(3))) void*)(base + j * 1024), 16, 0, 0);
+    for (int j = 0; j < L; ++j) {
+      const auto* from = (const __attribute__((address_space(1))) void*)src[j];
+      auto* to = (__attribute__((address_space(3))) void*)(base + j * 1024);
+      if (j < 2 && (what & 1)) __builtin_amdgcn_global_load_lds(from, to, 16, 0, SG_NONTEMPORAL);
+      if (j >= 2 && (what & 2)) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+    }
   };
   const int rounds = ks1 > ks0 ? (ks1 - ks0 + RING_U - 1) / RING_U : 0;
   // this lane's pieces of a slot: row col, blocks kb and 4 + kb

@@ -64,6 +64,7 @@ __device__ __forceinline__ f32x4 step_mfma(const f32x4& w, const f32x4& x, f32x4
 enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2 };
 
 // ------------------------------------------------------------------------------------------------ few rows
+constexpr int GF_NONTEMPORAL = 2;             // the hint of loads whose lines nobody reads again: the weights
 constexpr int GF_U = 2;                       // steps a slot of a wave's ring
 
 // The fragments of a slot out of the LDS, read and waited for in one piece of assembly: the compiler knows nothing of the
@@ -123,9 +124,12 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
     const size_t k = (size_t)ks * 16;
     const float* src[4] = {kok ? wsrc[0] + k : zero, kok ? wsrc[1] + k : zero, kok ? xsrc[0] + k : zero, kok ? xsrc[1] + k : zero};
 #pragma unroll
-    for (int j = 0; j < L; ++j)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[j],
-                                       (__attribute__((address_space(3))) void*)(base + j * 1024), 16, 0, 0);
+    for (int j = 0; j < L; ++j) {
+      const auto* from = (const __attribute__((address_space(1))) void*)src[j];
+      auto* to = (__attribute__((address_space(3))) void*)(base + j * 1024);
+      if (j < 2) __builtin_amdgcn_global_load_lds(from, to, 16, 0, GF_NONTEMPORAL);
+      else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+    }
   };
 #pragma unroll
   for (int s = 0; s < SLOTS - 1; ++s) issue(s);
