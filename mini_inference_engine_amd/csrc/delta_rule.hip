@@ -10,8 +10,8 @@
 //     in through the LDS, eight tokens at a time, the next eight on their way meanwhile.  The head's output is divided by
 //     its root mean square, times the weight and the sigmoid of the output gate, and rounded once.
 //
-// Rows run whole (one chunk: S from state[slot], left there afterwards), or, long rows, in chunks of L tokens side by
-// side in three passes, since a chunk acts on the state it starts from as S_end = P S_start + B with P and B of the
+// Rows run whole (one chunk: S from state[slot], left there afterwards), or, long rows, in chunks on the matrix cores (below) or,
+// what those do not take, in chunks of L tokens side by side in three passes, since a chunk acts on the state it starts from as S_end = P S_start + B with P and B of the
 // chunk's own tokens:  (1) every chunk but a row's last computes P (the recurrence without k v^T on the identity) and
 // B (the recurrence on zero), a thread carrying the same column of both;  (2) per row and head, chunk after chunk, S_start(c + 1) = P_c S_start(c) + B_c from
 // state[slot] (16 columns a workgroup; columns do not mix);  (3) every chunk runs its tokens from its S_start and writes
@@ -323,7 +323,491 @@ delta_fold_kernel(const float* __restrict__ summaries, float* __restrict__ start
   }
 }
 
+// ---- long rows on the matrix cores: chunks of 64 tokens, heads of up to 64, in 32-bit (v_mfma_f32_16x16x4_f32)
+//
+// With w = a * u, G_t the sum of log2 decays over a chunk's tokens up to t and y_t = S_(t-1)^T u_t, unrolled from the state S_0
+// the chunk starts from:
+//     S_t = 2^G_t S_0 + sum_(s <= t) 2^(G_t - G_s) (k_s v_s^T - w_s y_s^T)
+//     (I + A) y = (2^G_(t-1) u) S_0 + B v,      A_ts = sum_i u_ti w_si 2^(G_(t-1) - G_s)  (s < t),   B the same with k_s for w_s
+//     o = (2^G_t r) S_0 + Qk v - Qw y,          Qk_ts = sum_i r_ti k_si 2^(G_t - G_s)  (s <= t),     Qw the same with w_s
+// so with [W | U] = (I + A)^-1 [2^G_(t-1) u | B v] a chunk acts on S_0 by four 64 x 64 matrices:
+//     S_end = P S_0 + E,  P = 2^G_end - (2^(G_end - G) w)^T W,  E = (2^(G_end - G) k)^T v - (2^(G_end - G) w)^T U
+//     o = R S_0 + F,      R = 2^G r - Qw W,                     F = Qk v - Qw U
+// (1) chunk_solve, a workgroup a (chunk, head): from the projection's sums to P, E, R, F;  (2) chunk_fold, per (row, head, 16
+// columns), chunk after chunk: S_0 of every chunk;  (3) chunk_outputs: o, its norm, weight and gate.
+// Powers for tokens t of one 16 and s of the same or an earlier 16 are taken against the start of t's 16, so that the products
+// run on the matrix cores; the one positive exponent is that of 16 tokens' decay at most (DELTA_SCALE_MAX keeps it finite).
+// What bounds it: the solve's chain of small products (about 440 matrix instructions a SIMD and chunk) and its 32-bit arithmetic,
+// a workgroup a compute unit.  2,048 tokens of 16 heads of 64 (MI355X): 40 + 168 + 142 + 175 us (preparation, summaries, fold,
+// chunks, token by token through the LDS) -> 73 + 27 + 17 us.  The token-by-token chunks stay for heads of 65 to 128, other inner
+// sizes and stronger decays.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int CH = 64, MS = CH + 4;
+constexpr float LOG2E = 1.4426950408889634f, DELTA_SCALE_MAX = 4.f;
+constexpr int SOLVE_THREADS = 512;
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x); }
+// The waves meet over the LDS only: loads and stores of global memory stay on their way (__syncthreads would wait for them)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+struct ChunkArgs {
+  const float* sums; long ld; int r_col, k_col, v_col, g_col, a_col, w_col;
+  const float* w_decay; int rank; const float* decay_bias; float decay_scale; const float* removal_bias;
+  const float* norm_weight; float eps;
+  float* state; const int* row_start; const int* slots; void* out;
+  float *P, *E, *R, *F, *S0;       // [units * H][DP or 64][DP]; S0 [units * H][DP][DP]
+  int H, d, first_row, max_chunks, units;     // units: rows * max_chunks; the launch's rows begin at first_row
+};
+
+#define CHUNK_OF_ROW                                                                                                    \
+  const int place = blockIdx.y + gridDim.y * blockIdx.z;                                                                \
+  if (place >= a.units) return;                                                                                         \
+  const int rr = place / a.max_chunks, ci = place - rr * a.max_chunks, row = a.first_row + rr, h = blockIdx.x;          \
+  const int t0 = a.row_start[row] + ci * CH, t_end = a.row_start[row + 1];                                              \
+  if (t0 >= t_end) return;                                                                                              \
+  const int nt = t_end - t0 < CH ? t_end - t0 : CH;                                                                     \
+  const size_t unit = (size_t)place * a.H + h
+
+template <int DP>
+__global__ void __launch_bounds__(SOLVE_THREADS)
+chunk_solve_kernel(ChunkArgs a) {
+  constexpr int DS = DP + 4, CT = DP / 16, WAVES = SOLVE_THREADS / 64;
+  extern __shared__ __align__(16) float lds[];
+  float* sU = lds;                   // [64][DS] unit keys, then 2^G_(t-1) u
+  float* sK = sU + CH * DS;          // keys, then 2^(G_end - G) k
+  float* sW = sK + CH * DS;          // a * u, then 2^(G_end - G) w
+  float* sR = sW + CH * DS;          // r, then 2^G r
+  float* sG = sR + CH * DS;          // G from the start of a token's 16 on; then [64][MS] B
+  float* M = sG + CH * MS;           // [64][MS] the inner activations; then A
+  float* X = M + CH * MS;            // [64][MS] (I + A)^-1
+  float* Qw = X + CH * MS;
+  float* Qk = Qw + CH * MS;
+  float* so = Qk + CH * MS;          // [4][DP] sums of 16 tokens, then 2^G_end
+  CHUNK_OF_ROW;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int d = a.d, nH = a.H * d;
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  // ---- a wave eight tokens, lane a channel
+  {
+    const int i = lane < d ? lane : d - 1, c = h * d + i;
+    const float rb = a.removal_bias[c];
+    float k[8], r[8], al[8], in[8], kk[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int tt = 8 * wave + q;
+      const float* src = a.sums + (size_t)(t0 + (tt < nt ? tt : nt - 1)) * a.ld;
+      k[q] = src[a.k_col + c];
+      r[q] = src[a.r_col + c];
+      al[q] = src[a.a_col + c];
+      in[q] = src[a.w_col + (lane < a.rank ? lane : a.rank - 1)];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) kk[q] = lane < d ? k[q] * k[q] : 0.f;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) kk[q] += __shfl_xor(kk[q], o, 64);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int tt = 8 * wave + q;
+      const bool ok = lane < d && tt < nt;
+      const float u = k[q] / sqrtf(kk[q] + 1e-6f);
+      if (lane < DP) {
+        sU[tt * DS + lane] = ok ? u : 0.f;
+        sK[tt * DS + lane] = ok ? k[q] : 0.f;
+        sR[tt * DS + lane] = ok ? r[q] : 0.f;
+        sW[tt * DS + lane] = ok ? mie_sigmoid(al[q] + rb) * u : 0.f;
+      }
+      M[tt * MS + lane] = lane < a.rank && tt < nt ? tanhf(in[q]) : 0.f;
+    }
+  }
+  lds_barrier();
+  // ---- decays: (inner activations) (matrix of the head's channels)^T
+  for (int tile = wave; tile < 4 * CT; tile += WAVES) {
+    const int x = tile & 3, c = (tile >> 2) * 16 + n;
+    const int cc = h * d + (c < d ? c : d - 1);
+    const float* __restrict__ wd = a.w_decay + (size_t)cc * a.rank + 4 * g;
+    f32x4 z = none;
+    for (int kb = 0; kb < a.rank; kb += 16) {
+      const f32x4 w = *reinterpret_cast<const f32x4*>(wd + kb);
+      const f32x4 in = *reinterpret_cast<const f32x4*>(M + (16 * x + n) * MS + kb + 4 * g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) z = mfma4(in[j], w[j], z);
+    }
+    const float b = a.decay_bias[cc];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * x + 4 * g + e;
+      sG[t * DS + c] = t < nt && c < d ? -a.decay_scale * LOG2E * mie_sigmoid(z[e] + b) : 0.f;
+    }
+  }
+  lds_barrier();
+  // ---- sums over the tokens of a 16 (differences of sums over all 64 would lose more to rounding)
+  if (tid < 4 * DP) {
+    const int i = tid % DP, part = tid / DP;
+    float run = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float* at = sG + (16 * part + t) * DS + i;
+      run += *at;
+      *at = run;
+    }
+    so[part * DP + i] = run;
+  }
+  lds_barrier();
+  // ---- A, B, Qw, Qk: the ten 16 x 16 blocks on and below the diagonal over the waves, results kept until all have read
+  f32x4 accA[2], accB[2], accW[2], accK[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    accA[q] = accB[q] = accW[q] = accK[q] = none;
+    const int blk = wave + WAVES * q;
+    if (blk >= 10) break;
+    const int x = blk < 4 ? 3 : blk < 7 ? 2 : blk < 9 ? 1 : 0, y = blk - (blk < 4 ? 0 : blk < 7 ? 4 : blk < 9 ? 7 : 9);
+    const int t = 16 * x + n, s = 16 * y + n;
+    const float inside = n > 0 ? 1.f : 0.f;                        // the token before the 16's first: nothing
+    const float* gb = sG + (t - (n > 0 ? 1 : 0)) * DS;
+#pragma unroll
+    for (int i = 4 * g; i < DP; i += 16) {
+      f32x4 between = none;                                         // the sum over the tokens from s's 16 up to t's
+      for (int z = y; z < x; ++z) between += *reinterpret_cast<const f32x4*>(so + z * DP + i);
+      const f32x4 gt = *reinterpret_cast<const f32x4*>(sG + t * DS + i), gp = *reinterpret_cast<const f32x4*>(gb + i) * inside;
+      const f32x4 gs = between - *reinterpret_cast<const f32x4*>(sG + s * DS + i);
+      const f32x4 u = *reinterpret_cast<const f32x4*>(sU + t * DS + i), r = *reinterpret_cast<const f32x4*>(sR + t * DS + i);
+      const f32x4 w = *reinterpret_cast<const f32x4*>(sW + s * DS + i), k = *reinterpret_cast<const f32x4*>(sK + s * DS + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lu = u[e] * pow2(gp[e]), lr = r[e] * pow2(gt[e]), es = pow2(gs[e]);
+        const float rw = w[e] * es, rk = k[e] * es;
+        accA[q] = mfma4(lu, rw, accA[q]);
+        accB[q] = mfma4(lu, rk, accB[q]);
+        accW[q] = mfma4(lr, rw, accW[q]);
+        accK[q] = mfma4(lr, rk, accK[q]);
+      }
+    }
+  }
+  lds_barrier();
+  // ---- the vectors times their powers, in place, 2^G_end beside them
+  for (int e = tid; e < CH * DP; e += SOLVE_THREADS) {
+    const int t = e / DP, i = e % DP, x = t >> 4;
+    float before = 0.f, after = so[x * DP + i] - sG[t * DS + i];
+    for (int z = 0; z < x; ++z) before += so[z * DP + i];
+    for (int z = x + 1; z < 4; ++z) after += so[z * DP + i];
+    const float G = sG[t * DS + i], Gb = t & 15 ? sG[(t - 1) * DS + i] : 0.f, to_end = pow2(after);
+    sU[t * DS + i] *= pow2(before + Gb);
+    sR[t * DS + i] *= pow2(before + G);
+    sK[t * DS + i] *= to_end;
+    sW[t * DS + i] *= to_end;
+    if (t == CH - 1) so[4 * DP + i] = pow2(before + G);
+  }
+  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) M[e] = X[e] = Qw[e] = Qk[e] = 0.f;
+  lds_barrier();
+  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) sG[e] = 0.f;
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int blk = wave + WAVES * q;
+    if (blk >= 10) break;
+    const int x = blk < 4 ? 3 : blk < 7 ? 2 : blk < 9 ? 1 : 0, y = blk - (blk < 4 ? 0 : blk < 7 ? 4 : blk < 9 ? 7 : 9);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * x + 4 * g + e, s = 16 * y + n;
+      M[t * MS + s] = s < t ? accA[q][e] : 0.f;
+      sG[t * MS + s] = s < t ? accB[q][e] : 0.f;
+      Qw[t * MS + s] = s <= t ? accW[q][e] : 0.f;
+      Qk[t * MS + s] = s <= t ? accK[q][e] : 0.f;
+    }
+  }
+  lds_barrier();
+  // ---- the inverse: diagonal blocks by substitution, a lane a column; X_ab = -X_aa sum_c M_ac X_cb below them
+  if (wave < 4) {
+    const float* __restrict__ m = M + 16 * wave * MS + 16 * wave;
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float v = t == n ? 1.f : 0.f;
+#pragma unroll
+      for (int s = 0; s < t; ++s) v = fmaf(-m[t * MS + s], x[s], v);
+      x[t] = v;
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) X[(16 * wave + t) * MS + 16 * wave + n] = x[t];
+    }
+  }
+  lds_barrier();
+#pragma unroll 1
+  for (int dist = 1; dist < 4; ++dist) {
+    if (wave + dist < 4) {
+      const int x = wave + dist, y = wave;
+      f32x4 s = none, r = none;
+      for (int c = y; c < x; ++c) {
+        const f32x4 m = *reinterpret_cast<const f32x4*>(M + (16 * x + n) * MS + 16 * c + 4 * g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s = mfma4(m[j], X[(16 * c + 4 * g + j) * MS + 16 * y + n], s);
+      }
+      // a result's rows 4 g + e are what the next product's operand wants as its rows 4 g + j
+      const f32x4 xx = *reinterpret_cast<const f32x4*>(X + (16 * x + n) * MS + 16 * x + 4 * g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r = mfma4(xx[j], s[j], r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) X[(16 * x + 4 * g + e) * MS + 16 * y + n] = -r[e];
+    }
+    lds_barrier();
+  }
+  // ---- the four matrices, a wave 16 columns: first W, R, P, then U, F, E
+  auto lower = [&](const float* L, const f32x4 (&b)[4], f32x4 (&acc)[4], float sign) {      // acc += sign L b, L lower triangular
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+      for (int x = y; x < 4; ++x) {
+        const f32x4 m = *reinterpret_cast<const f32x4*>(L + (16 * x + n) * MS + 16 * y + 4 * g) * sign;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[x] = mfma4(m[j], b[y][j], acc[x]);
+      }
+  };
+  auto turned = [&](const float* T, const f32x4 (&b)[4], f32x4 (&acc)[CT], float sign) {    // acc += sign T^T b, T [64][DS]
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < CT; ++x) acc[x] = mfma4(sign * T[(16 * y + 4 * g + j) * DS + 16 * x + n], b[y][j], acc[x]);
+  };
+  for (int ct = wave; ct < 2 * CT; ct += WAVES) {
+    const bool of_v = ct >= CT;
+    const int c = (of_v ? ct - CT : ct) * 16 + n;
+    f32x4 b[4], w[4], o[4], st[CT];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) w[x] = o[x] = none;
+#pragma unroll
+    for (int x = 0; x < CT; ++x) st[x] = none;
+    if (of_v) {
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int s = 16 * y + 4 * g + j;
+          b[y][j] = s < nt && c < d ? a.sums[(size_t)(t0 + s) * a.ld + a.v_col + h * d + c] : 0.f;
+        }
+      lower(Qk, b, o, 1.f);
+      turned(sK, b, st, 1.f);
+      lower(sG, b, w, 1.f);              // B v
+#pragma unroll
+      for (int y = 0; y < 4; ++y) { b[y] = w[y]; w[y] = none; }
+    } else {
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          b[y][j] = sU[(16 * y + 4 * g + j) * DS + c];
+          o[y][j] = sR[(16 * y + 4 * g + j) * DS + c];
+        }
+#pragma unroll
+      for (int x = 0; x < CT; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[x][e] = 16 * x + 4 * g + e == c ? so[4 * DP + c] : 0.f;
+    }
+    lower(X, b, w, 1.f);                 // W or U
+    lower(Qw, w, o, -1.f);
+    turned(sW, w, st, -1.f);
+    float* __restrict__ to = (of_v ? a.F : a.R) + unit * CH * DP + c;
+    float* __restrict__ se = (of_v ? a.E : a.P) + unit * DP * DP + c;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[(size_t)(16 * x + 4 * g + e) * DP] = o[x][e];
+#pragma unroll
+    for (int x = 0; x < CT; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) se[(size_t)(16 * x + 4 * g + e) * DP] = st[x][e];
+  }
+}
+
+// (2) grid (H, rows, DP / 16): a wave 16 rows of the state's 16 columns; every chunk's S_0 out, S = P S + E
+template <int DP>
+__global__ void __launch_bounds__(DP * 4)
+chunk_fold_kernel(ChunkArgs a) {
+  constexpr int CS = 20, KB = DP / 16;
+  __shared__ __align__(16) float sS[2][DP * CS];
+  const int h = blockIdx.x, rr = blockIdx.y, row = a.first_row + rr, col = blockIdx.z * 16 + (threadIdx.x & 15);
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int d = a.d, tokens = a.row_start[row + 1] - a.row_start[row], chunks = (tokens + CH - 1) / CH;
+  if (chunks <= 0) return;
+  float* __restrict__ st = a.state + ((size_t)a.slots[row] * a.H + h) * d * d;
+  f32x4 S;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int r = 16 * wave + 4 * g + e;
+    S[e] = r < d && col < d ? st[(size_t)r * d + col] : 0.f;
+  }
+  struct Ahead { f32x4 p[KB], e; };      // what a chunk needs, asked for two chunks ahead
+  auto fetch = [&](Ahead& A, int c) {
+    const size_t unit = ((size_t)rr * a.max_chunks + (c < chunks ? c : chunks - 1)) * a.H + h;
+    const float* __restrict__ P = a.P + unit * DP * DP + (size_t)(16 * wave + n) * DP + 4 * g;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) A.p[kb] = *reinterpret_cast<const f32x4*>(P + 16 * kb);
+    const float* __restrict__ E = a.E + unit * DP * DP + (size_t)(16 * wave + 4 * g) * DP + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) A.e[e] = E[(size_t)e * DP];
+  };
+  auto step = [&](Ahead& A, int c) {
+    float* __restrict__ s = sS[c & 1];
+    float* __restrict__ S0 = a.S0 + (((size_t)rr * a.max_chunks + c) * a.H + h) * DP * DP + (size_t)(16 * wave + 4 * g) * DP + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[(16 * wave + 4 * g + e) * CS + n] = S[e];
+      S0[(size_t)e * DP] = S[e];
+    }
+    lds_barrier();                       // (two buffers: the one written next was read before this barrier)
+    f32x4 acc[2] = {A.e, f32x4{0.f, 0.f, 0.f, 0.f}};
+    float right[KB][4];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) right[kb][j] = s[(16 * kb + 4 * g + j) * CS + n];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) acc[kb & 1] = mfma4(A.p[kb][j], right[kb][j], acc[kb & 1]);
+    S = acc[0] + acc[1];
+    fetch(A, c + 2);
+  };
+  Ahead even, odd;
+  fetch(even, 0);
+  fetch(odd, 1);
+  for (int c = 0; c < chunks; c += 2) {
+    step(even, c);
+    if (c + 1 < chunks) step(odd, c + 1);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int r = 16 * wave + 4 * g + e;
+    if (r < d && col < d) st[(size_t)r * d + col] = S[e];
+  }
+}
+
+// (3) a wave 16 tokens of a head: o = R S_0 + F, S_0 through the LDS; then the norm, the weight and the gate
+template <int DP, typename TO>
+__global__ void __launch_bounds__(256)
+chunk_outputs_kernel(ChunkArgs a) {
+  constexpr int CT = DP / 16, SS = DP + 4;
+  __shared__ __align__(16) float sS[DP * SS];
+  CHUNK_OF_ROW;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int d = a.d;
+  const float* __restrict__ S0 = a.S0 + unit * DP * DP;
+  const float* __restrict__ R = a.R + unit * CH * DP + (size_t)(16 * wave + n) * DP + 4 * g;
+  const float* __restrict__ F = a.F + unit * CH * DP + (size_t)(16 * wave + 4 * g) * DP + n;
+  f32x4 r[CT], o[CT];
+#pragma unroll
+  for (int kb = 0; kb < CT; ++kb) r[kb] = *reinterpret_cast<const f32x4*>(R + 16 * kb);
+#pragma unroll
+  for (int x = 0; x < CT; ++x)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[x][e] = F[(size_t)e * DP + 16 * x];
+  for (int e = tid; e < DP * DP / 4; e += 256) {
+    const int i = e / (DP / 4), c = e % (DP / 4);
+    *reinterpret_cast<f32x4*>(sS + i * SS + 4 * c) = *reinterpret_cast<const f32x4*>(S0 + 4 * e);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int kb = 0; kb < CT; ++kb)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int x = 0; x < CT; ++x) o[x] = mfma4(r[kb][j], sS[(16 * kb + 4 * g + j) * SS + 16 * x + n], o[x]);
+  float ss[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    ss[e] = 0.f;
+#pragma unroll
+    for (int x = 0; x < CT; ++x) ss[e] = fmaf(o[x][e], o[x][e], ss[e]);
+  }
+#pragma unroll
+  for (int q = 8; q > 0; q >>= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss[e] += __shfl_xor(ss[e], q, 64);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int tt = 16 * wave + 4 * g + e;
+    if (tt >= nt) continue;
+    const float rstd = 1.0f / sqrtf(ss[e] / (float)d + a.eps);
+    const size_t t = t0 + tt;
+#pragma unroll
+    for (int x = 0; x < CT; ++x) {
+      const int c = 16 * x + n;
+      if (c < d)
+        ((TO*)a.out)[t * a.H * d + h * d + c] =
+            from_float<TO>(o[x][e] * rstd * a.norm_weight[h * d + c] * mie_sigmoid(a.sums[t * a.ld + a.g_col + h * d + c]));
+    }
+  }
+}
+
 MIE_EXPORT const char* delta_rule_last_error() { return g_mie_error; }
+
+template <int DP>
+static int chunks_launch(const ChunkArgs& a, int rows, int out_dtype, hipStream_t s) {
+  const size_t lds = ((size_t)4 * CH * (DP + 4) + (size_t)5 * CH * MS + 5 * DP) * sizeof(float);
+  static bool allowed[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("delta_rule: no current device");
+  if (!allowed[dev]) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_solve_kernel<DP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) MIE_FAIL("delta_rule: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    allowed[dev] = true;
+  }
+  const dim3 units(a.H, a.units < 32768 ? a.units : 32768, (a.units + 32767) / 32768);
+  hipLaunchKernelGGL(chunk_solve_kernel<DP>, units, dim3(SOLVE_THREADS), lds, s, a);
+  MIE_CHECK_LAUNCH("delta_rule (chunks: solve)");
+  hipLaunchKernelGGL(chunk_fold_kernel<DP>, dim3(a.H, rows, DP / 16), dim3(DP * 4), 0, s, a);
+  MIE_CHECK_LAUNCH("delta_rule (chunks: fold)");
+  if (out_dtype == MIE_F32) hipLaunchKernelGGL((chunk_outputs_kernel<DP, float>), units, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((chunk_outputs_kernel<DP, bf16>), units, dim3(256), 0, s, a);
+  MIE_CHECK_LAUNCH("delta_rule (chunks: outputs)");
+  return 0;
+}
+
+// Whether mie_delta_rule_chunks takes heads of d, an inner size and a decay's scale.
+MIE_EXPORT int mie_delta_rule_chunks_take(int d, int rank, float decay_scale) {
+  return d >= 1 && d <= 64 && rank >= 16 && rank <= 64 && rank % 16 == 0 && decay_scale >= 0.f && decay_scale <= DELTA_SCALE_MAX;
+}
+// floats of scratch a (chunk, head) takes
+MIE_EXPORT int mie_delta_rule_unit_floats(int d) { const int DP = d <= 32 ? 32 : 64; return 2 * CH * DP + 3 * DP * DP; }
+
+// Rows [first_row, first_row + rows) in chunks of 64 tokens, at most max_chunks a row; scratch: rows * max_chunks * H *
+// mie_delta_rule_unit_floats(d) floats.
+MIE_EXPORT int mie_delta_rule_chunks(const float* sums, long ld, int r_col, int k_col, int v_col, int g_col, int a_col, int w_col,
+                                     const float* w_decay, int rank, const float* decay_bias, float decay_scale,
+                                     const float* removal_bias, const float* norm_weight, float eps, float* state,
+                                     const int* row_start, const int* slots, void* out, int out_dtype, int first_row, int rows,
+                                     int H, int d, int max_chunks, float* scratch, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (H <= 0 || first_row < 0 || !mie_delta_rule_chunks_take(d, rank, decay_scale))
+    MIE_FAIL("delta_rule: chunks of %d heads of %d, inner size %d, decays' scale %g", H, d, rank, (double)decay_scale);
+  if (rows > 65535 || H > 65535 || max_chunks < 1 || (long)rows * max_chunks > 2147483647L) MIE_FAIL("delta_rule: %d rows of %d chunks, %d heads are beyond the grid", rows, max_chunks, H);
+  if (out_dtype != MIE_F32 && out_dtype != MIE_BF16) MIE_FAIL("delta_rule: out dtype code %d", out_dtype);
+  if (!scratch || (((uintptr_t)scratch | (uintptr_t)w_decay) & 15)) MIE_FAIL("delta_rule: scratch and the decay's matrix must be 16-byte aligned");
+  const int DP = d <= 32 ? 32 : 64;
+  const size_t units = (size_t)rows * max_chunks * H;
+  ChunkArgs a{sums, ld, r_col, k_col, v_col, g_col, a_col, w_col, w_decay, rank, decay_bias, decay_scale, removal_bias, norm_weight,
+              eps, state, row_start, slots, out, nullptr, nullptr, nullptr, nullptr, nullptr, H, d, first_row, max_chunks, rows * max_chunks};
+  float* at = scratch;
+  auto take = [&](size_t per) { float* q = at; at += units * per; return q; };
+  a.P = take((size_t)DP * DP);
+  a.E = take((size_t)DP * DP);
+  a.S0 = take((size_t)DP * DP);
+  a.R = take((size_t)CH * DP);
+  a.F = take((size_t)CH * DP);
+  return DP == 32 ? chunks_launch<32>(a, rows, out_dtype, s) : chunks_launch<64>(a, rows, out_dtype, s);
+}
 
 // prep: scratch of tokens * 3 * H * d floats.  chunk_tokens 0: rows run whole.  Else rows run in chunks of that many
 // tokens, at most max_chunks a row, with scratch summaries [rows * max_chunks * H * 2 * d * d] and starts

@@ -1253,20 +1253,37 @@ class HipBackend(KernelBackend):
         if int(step.host["state_slots"].max()) >= state.shape[0]:
             raise ValueError("delta_rule: a state slot beyond the state's slots")
         out = torch.empty((T, n), dtype=self.act_dtype, device=sums.device)
-        prep = torch.empty((T, 3 * n), dtype=torch.float32, device=sums.device)
+        lib = self.lib("delta_rule")
         longest = int(getattr(step, "max_row_tokens", 0) or (step.host["row_start"][1:] - step.host["row_start"][:-1]).max())
         chunk, chunks, summaries, starts = 0, 0, None, None
-        if longest > self.DELTA_CHUNK and not self.true_fp32 and d <= self.DELTA_CHUNKED_MAX_DIM:
+        whole, rows, tokens = 0, step.num_rows, T
+        if (longest > self.DELTA_CHUNK and not self.true_fp32 and lib.mie_delta_rule_chunks_take(d, rank, float(decay_scale))
+                and w_decay.data_ptr() % 16 == 0):
+            # rows of many tokens, in chunks on the matrix cores; the single tokens that lead the step one by one, below
+            whole = int(getattr(step, "num_decode_rows", 0) or 0)
+            chunks = -(-longest // 64)
+            scratch = torch.empty((rows - whole) * chunks * H * lib.mie_delta_rule_unit_floats(d), dtype=torch.float32, device=sums.device)
+            library.check(lib, lib.mie_delta_rule_chunks(
+                _ptr(sums), sums.stride(0), cols["r"], cols["k"], cols["v"], cols["g"], cols["a"], cols["w"], _ptr(w_decay), rank,
+                _ptr(decay_bias), float(decay_scale), _ptr(removal_bias), _ptr(norm_weight), float(eps), _ptr(state),
+                _ptr(step.row_start), _ptr(step.state_slots), _ptr(out), _code(out.dtype), whole, rows - whole, H, d, chunks,
+                _ptr(scratch), self._stream()))
+            if not whole:
+                return out
+            rows = tokens = whole
+        elif longest > self.DELTA_CHUNK and not self.true_fp32 and d <= self.DELTA_CHUNKED_MAX_DIM:
             # rows of many tokens: chunks side by side (whether a step takes this path depends on its longest row alone;
             # the two paths differ by the rounding of the fold over whole chunks, so the 32-bit mode keeps to one)
             chunk, chunks = self.DELTA_CHUNK, -(-longest // self.DELTA_CHUNK)
             scratch = torch.empty((3, step.num_rows * chunks * H, d, d), dtype=torch.float32, device=sums.device)
             summaries, starts = scratch[:2], scratch[2]
-        lib = self.lib("delta_rule")
+        if whole:
+            chunk, chunks = 0, 0
+        prep = torch.empty((tokens, 3 * n), dtype=torch.float32, device=sums.device)
         library.check(lib, lib.mie_delta_rule(
             _ptr(sums), sums.stride(0), cols["r"], cols["k"], cols["v"], cols["g"], cols["a"], cols["w"], _ptr(w_decay), rank,
             _ptr(decay_bias), float(decay_scale), _ptr(removal_bias), _ptr(norm_weight), float(eps), _ptr(state),
-            _ptr(step.row_start), _ptr(step.state_slots), _ptr(prep), _ptr(out), _code(out.dtype), T, step.num_rows, H, d,
+            _ptr(step.row_start), _ptr(step.state_slots), _ptr(prep), _ptr(out), _code(out.dtype), tokens, rows, H, d,
             chunk, chunks, _ptr(summaries), _ptr(starts), self._stream()))
         return out
 

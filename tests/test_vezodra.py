@@ -585,6 +585,33 @@ def test_delta_rule_kernel(hip, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,d,rank,lens,scale", [
+    (2, 64, 64, [1, 1, 65, 300], 0.6065), (1, 48, 16, [64, 128, 129], 0.6), (3, 20, 32, [1, 70], 0.6), (5, 32, 48, [192], 0.6),
+    (2, 16, 16, [2, 63, 200], 0.6), (2, 64, 16, [100, 67], 4.0), (1, 33, 64, [80], 0.0), (2, 64, 64, [130], 4.5)])
+def test_delta_rule_in_chunks_on_the_matrix_cores(hip, H, d, rank, lens, scale):
+    """Heads of up to 64 with inner sizes in steps of 16: rows beyond 64 tokens as chunks of 64 by matrix products, single tokens
+    beside them one by one, against the recurrence in 64 bits; the strongest decay the chunks take, none at all, and one beyond
+    them (the token-by-token kernels).  The states within the bound of test_delta_rule_kernel; twice it for the strongest decay,
+    whose sums over 16 tokens in units of log 2 reach 92 and carry an absolute rounding of 92 * 2^-24 = 5e-6 into their powers."""
+    ops, g = hip[torch.bfloat16], torch.Generator().manual_seed(d + rank)
+    step = FakeStep(lens, list(range(len(lens), 0, -1)))
+    step.num_decode_rows = next(i for i, m in enumerate(lens) if m > 1)
+    T, n = step.num_tokens, H * d
+    cols = dict(r=0, k=n, v=2 * n, g=3 * n, a=4 * n, w=5 * n)
+    sums = _rand((T, 5 * n + rank + 3), torch.float32, g)
+    w_decay, db, rb = _rand((n, rank), torch.float32, g, 1.5), _rand((n,), torch.float32, g), _rand((n,), torch.float32, g)
+    nw = _rand((n,), torch.float32, g) + 1
+    state = _rand((len(lens) + 1, H, d, d), torch.float32, g, 0.5)
+    st_w = state.cpu().clone()
+    want = ref.ref_delta_rule(sums.cpu(), cols, H, d, w_decay.cpu(), db.cpu(), scale, rb.cpu(), nw.cpu(), 1e-5, st_w,
+                              step.host["row_start"], step.host["state_slots"], torch.float64)
+    got = ops.delta_rule(sums, cols, H, d, w_decay, db, scale, rb, nw, 1e-5, state, step)
+    close(got.double(), want, 1e-2, f"delta rule {H} x {d}")
+    close(state, st_w, 3e-5 if scale < 1 else 6e-5, "state")
+    assert torch.equal(state[0].cpu(), st_w[0]), "slots of no row are left alone"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_kernels_with_a_sink(hip, dtype):
     """The three attention kernels (32-bit, matrix-core decode with and without splits, matrix-core prompt portions)
