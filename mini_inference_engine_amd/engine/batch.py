@@ -65,7 +65,8 @@ class StepContext:
 
 
 class StepArena:
-    """Fixed-address int32 storage for step metadata, with a pinned host mirror."""
+    """Fixed-address int32 storage for step metadata, with two pinned host mirrors that take turns: a step is built in
+    one while the copy of the step before may still be reading the other."""
 
     def __init__(self, max_tokens: int, max_rows: int, max_blocks: int, num_groups: int, device):
         self.max_tokens, self.max_rows, self.max_blocks, self.num_groups = max_tokens, max_rows, max_blocks, num_groups
@@ -86,35 +87,49 @@ class StepArena:
         self.tables_begin = self.offsets["block_tables0"][0] if num_groups else off
         self.size = off
         pin = self.device.type == "cuda"
-        self.host = torch.zeros(off, dtype=torch.int32, pin_memory=pin)
-        self.host_np = self.host.numpy()
-        self.dev = torch.zeros(off, dtype=torch.int32, device=self.device) if pin else self.host
-        self._copied = None
+        self.mirrors = [torch.zeros(off, dtype=torch.int32, pin_memory=pin) for _ in range(2 if pin else 1)]
+        self.mirrors_np = [m.numpy() for m in self.mirrors]
+        self.dev = torch.zeros(off, dtype=torch.int32, device=self.device) if pin else self.mirrors[0]
+        self._turn = 0                       # the mirror the step being built is written to
+        self._copied = [None] * len(self.mirrors)     # event behind the last copy out of each mirror
+        self._views = {}                     # device views by (name, length): an address and a length each, the same every step
+        self.ramp = np.arange(max(max_tokens, max_rows) + 1, dtype=np.int64)
 
     def host_view(self, name: str) -> np.ndarray:
         o, n = self.offsets[name]
-        return self.host_np[o:o + n]
+        return self.mirrors_np[self._turn][o:o + n]
 
     def dev_view(self, name: str, n: int | None = None) -> torch.Tensor:
-        o, cap = self.offsets[name]
-        return self.dev[o:o + (cap if n is None else n)]
+        v = self._views.get((name, n))
+        if v is None:
+            o, cap = self.offsets[name]
+            v = self.dev[o:o + (cap if n is None else n)]
+            if len(self._views) >= 4096:     # many step sizes: start over rather than grow
+                self._views.clear()
+            self._views[(name, n)] = v
+        return v
+
+    def next_mirror(self) -> None:
+        """Take the other mirror, once the copy that last read it is done."""
+        self._turn = (self._turn + 1) % len(self.mirrors)
+        if self._copied[self._turn] is not None:
+            self._copied[self._turn].synchronize()
 
     def upload(self, table_rows: int) -> None:
-        """One copy of everything before the block tables plus the used rows of the tables."""
-        if self.dev is self.host:
+        """Everything before the block tables with the used rows of the first group's tables behind it in one copy; the used
+        rows of the other groups' tables."""
+        host = self.mirrors[self._turn]
+        if self.dev is host:
             return
-        end = self.tables_begin
-        self.dev[:end].copy_(self.host[:end], non_blocking=True)
-        for g in range(self.num_groups):
+        n = table_rows * self.max_blocks
+        end = self.tables_begin + (n if self.num_groups else 0)
+        self.dev[:end].copy_(host[:end], non_blocking=True)
+        for g in range(1, self.num_groups):
             o, _ = self.offsets[f"block_tables{g}"]
-            n = table_rows * self.max_blocks
-            self.dev[o:o + n].copy_(self.host[o:o + n], non_blocking=True)
-        self._copied = torch.cuda.Event()
-        self._copied.record()
-
-    def wait_uploaded(self) -> None:
-        if self._copied is not None:
-            self._copied.synchronize()
+            self.dev[o:o + n].copy_(host[o:o + n], non_blocking=True)
+        if self._copied[self._turn] is None:
+            self._copied[self._turn] = torch.cuda.Event()
+        self._copied[self._turn].record()
 
 
 def order_rows(rows: Sequence[StepRow]) -> list[int]:
@@ -134,9 +149,11 @@ def build_step(rows: Sequence[StepRow], arena: StepArena, page_size: int, *, pad
     ``sampling``: (temperatures, seeds, counters), one entry for each wanted row of logits in their order
     (with ``want_all``: one for each of ``rows``; scratch rows are greedy), for a step whose tokens are
     chosen on the device."""
-    arena.wait_uploaded()           # the last step's copy may still be reading the host mirror
-    order = order_rows(rows)
+    arena.next_mirror()
     n_rows = len(rows)
+    if not pad_portion_to and n_rows and all(len(r.tokens) == 1 for r in rows):
+        return _build_single(rows, arena, page_size, max(n_rows, pad_rows_to), static_context, want_all, sampling)
+    order = order_rows(rows)
     lens = np.fromiter((len(rows[i].tokens) for i in order), dtype=np.int64, count=n_rows)
     if pad_portion_to:
         if n_rows != 1 or pad_rows_to or pad_portion_to < lens[0]:
@@ -206,16 +223,7 @@ def build_step(rows: Sequence[StepRow], arena: StepArena, page_size: int, *, pad
     R = len(wanted)
     arena.host_view("logit_rows")[:R] = wanted
     if sampling is not None:
-        temps, seeds, counters = sampling
-        n = len(temps)
-        if not (len(seeds) == len(counters) == n) or n != (n_rows if want_all else R) or R > arena.max_rows:
-            raise ValueError(f"sampling inputs for {n} rows; the step has {n_rows if want_all else R} rows of wanted "
-                             f"logits (at most {arena.max_rows})")
-        ht, hc, hs = arena.host_view("sample_temps"), arena.host_view("sample_counters"), arena.host_view("sample_seeds")
-        ht[:R], hc[:R], hs[:2 * R] = 0, 0, 0
-        ht[:n] = np.asarray(temps, dtype=np.float32).view(np.int32)
-        hc[:n] = np.asarray(counters, dtype=np.int32)
-        hs[:2 * n] = np.asarray([s & 0xFFFFFFFFFFFFFFFF for s in seeds], dtype=np.uint64).view(np.int32)
+        _put_sampling(arena, sampling, n_rows, R, want_all)
 
     mb = arena.max_blocks
     for g in range(arena.num_groups):
@@ -235,6 +243,85 @@ def build_step(rows: Sequence[StepRow], arena: StepArena, page_size: int, *, pad
             page_of[len(rows[0].tokens):] = 0
         arena.host_view(f"slot_mapping{g}")[:T] = page_of * page_size + positions % page_size
 
+    return _finish(arena, page_size, T, total_rows, num_decode, R, int(row_len.max()), int(static_context or ctx.max()), sampling,
+                   {"row_start": row_start, "row_position": row_pos, "row_context": ctx, "row_len": row_len,
+                    "positions": positions, "token_row": token_row, "state_slots": slots_state[:total_rows].copy()})
+
+
+def _put_sampling(arena, sampling, n_rows, R, want_all):
+    temps, seeds, counters = sampling
+    n = len(temps)
+    if not (len(seeds) == len(counters) == n) or n != (n_rows if want_all else R) or R > arena.max_rows:
+        raise ValueError(f"sampling inputs for {n} rows; the step has {n_rows if want_all else R} rows of wanted "
+                         f"logits (at most {arena.max_rows})")
+    ht, hc, hs = arena.host_view("sample_temps"), arena.host_view("sample_counters"), arena.host_view("sample_seeds")
+    ht[:R], hc[:R], hs[:2 * R] = 0, 0, 0
+    ht[:n] = np.asarray(temps, dtype=np.float32).view(np.int32)
+    hc[:n] = np.asarray(counters, dtype=np.int32)
+    hs[:2 * n] = np.asarray([s & 0xFFFFFFFFFFFFFFFF for s in seeds], dtype=np.uint64).view(np.int32)
+
+
+def _build_single(rows, arena, page_size, total_rows, static_context, want_all, sampling):
+    """A step of single-token rows (and scratch rows up to ``total_rows``): token r is row r, so every array is a value a
+    row, without the general step's repeats and sums over row lengths."""
+    n = len(rows)
+    if total_rows > arena.max_tokens or total_rows > arena.max_rows:
+        raise ValueError(f"step of {total_rows} tokens in {total_rows} rows exceeds the arena "
+                         f"({arena.max_tokens} tokens, {arena.max_rows} rows)")
+    positions = np.zeros(total_rows, dtype=np.int64)
+    positions[:n] = [r.start for r in rows]
+    ctx = positions + 1
+    most = int(ctx.max())
+    width = -(-most // page_size)
+    if width > arena.max_blocks:
+        raise ValueError(f"a row needs {width} pages; the arena holds {arena.max_blocks} per row")
+    ramp = arena.ramp
+    ids, taken, slots_state = arena.host_view("input_ids"), arena.host_view("taken_from"), arena.host_view("state_slots")
+    ids[:total_rows] = 0
+    taken[:total_rows] = -1
+    slots_state[:total_rows] = 0
+    ids[:n] = [r.tokens[0] if r.taken_from < 0 else 0 for r in rows]
+    taken[:n] = [r.taken_from if r.taken_from >= 0 else -1 for r in rows]
+    slots_state[:n] = [r.cache.state_slot for r in rows]
+    arena.host_view("positions")[:total_rows] = positions
+    arena.host_view("token_row")[:total_rows] = ramp[:total_rows]
+    arena.host_view("row_start")[:total_rows + 1] = ramp[:total_rows + 1]
+    arena.host_view("row_position")[:total_rows] = positions
+    arena.host_view("row_context")[:total_rows] = ctx
+    if want_all:
+        wanted = ramp[:total_rows]
+    else:
+        wanted = []
+        for i, r in enumerate(rows):
+            for w in r.want:
+                if w != 0:
+                    raise ValueError(f"wanted offset {w} outside a row of 1 tokens")
+                wanted.append(i)
+    R = len(wanted)
+    arena.host_view("logit_rows")[:R] = wanted
+    if sampling is not None:
+        _put_sampling(arena, sampling, n, R, want_all)
+    mb = arena.max_blocks
+    for g in range(arena.num_groups):
+        bt = arena.host_view(f"block_tables{g}")[:total_rows * mb].reshape(total_rows, mb)
+        bt[:, :width] = 0
+        slots = np.zeros(total_rows, dtype=np.int64)
+        for i, r in enumerate(rows):
+            t, last = r.cache.tables[g], r.start // page_size
+            if len(t) <= last:
+                raise ValueError(f"row {i}: {len(t)} pages reserved in group {g}, {last + 1} needed")
+            bt[i, :last + 1] = t if len(t) == last + 1 else t[:last + 1]
+            slots[i] = t[last] * page_size + r.start % page_size
+        arena.host_view(f"slot_mapping{g}")[:total_rows] = slots
+    return _finish(arena, page_size, total_rows, total_rows, total_rows, R, 1, int(static_context or most), sampling,
+                   {"row_start": ramp[:total_rows + 1].copy(), "row_position": positions, "row_context": ctx,
+                    "row_len": np.ones(total_rows, dtype=np.int64), "positions": positions, "token_row": ramp[:total_rows].copy(),
+                    "state_slots": slots_state[:total_rows].copy()})
+
+
+def _finish(arena, page_size, T, total_rows, num_decode, R, max_row_tokens, max_context, sampling, host):
+    """Send the arrays and describe the step by views of where they arrive."""
+    mb = arena.max_blocks
     arena.upload(total_rows)
     step = StepContext(
         num_tokens=T, num_rows=total_rows, num_decode_rows=num_decode, num_logits=R,
@@ -243,11 +330,7 @@ def build_step(rows: Sequence[StepRow], arena: StepArena, page_size: int, *, pad
         token_row=arena.dev_view("token_row", T), row_start=arena.dev_view("row_start", total_rows + 1),
         row_position=arena.dev_view("row_position", total_rows), row_context=arena.dev_view("row_context", total_rows),
         state_slots=arena.dev_view("state_slots", total_rows), logit_rows=arena.dev_view("logit_rows", R),
-        page_size=page_size, max_row_tokens=int(row_len.max()),
-        max_context=int(static_context or ctx.max()),
-        host={"row_start": row_start, "row_position": row_pos, "row_context": ctx, "row_len": row_len,
-              "positions": positions, "token_row": token_row, "state_slots": slots_state[:total_rows].copy()},
-    )
+        page_size=page_size, max_row_tokens=max_row_tokens, max_context=max_context, host=host)
     if sampling is not None:
         step.sample_temps = arena.dev_view("sample_temps", R).view(torch.float32)
         step.sample_counters = arena.dev_view("sample_counters", R)

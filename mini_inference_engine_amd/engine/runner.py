@@ -10,6 +10,8 @@ finished prompts only.)
 """
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from ..cache import CacheManager, CacheStorage, GroupSpec
@@ -22,6 +24,9 @@ _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.
            torch.bfloat16: torch.bfloat16, torch.float32: torch.float32}
 
 
+_NO_RANGE = contextlib.nullcontext()
+
+
 class PhaseRanges:
     """Named ranges around the phases of a step, for a profiler's timeline (rocprofv3 --marker-trace shows them;
     the reference marks the same four phases with NVTX, inference_engine/engine.py:183-210).  Off by default:
@@ -31,10 +36,7 @@ class PhaseRanges:
         self.on = bool(on)
 
     def __call__(self, name: str):
-        if self.on:
-            return torch.cuda.nvtx.range(name)
-        import contextlib
-        return contextlib.nullcontext()
+        return torch.cuda.nvtx.range(name) if self.on else _NO_RANGE
 
 
 def parse_dtype(d) -> torch.dtype:

@@ -308,3 +308,50 @@ def test_a_portion_lengthened_to_a_captured_size_writes_to_the_scratch_page():
         build_step([StepRow(req, [1, 2], 0, []), StepRow(req, [3, 4], 2, [])], arena, page, pad_portion_to=16)
     with pytest.raises(ValueError, match="one row"):
         build_step([StepRow(req, list(range(9)), 0, [])], arena, page, pad_portion_to=8)
+
+
+@pytest.mark.parametrize("pad,static", [(0, 0), (5, 64), (3, 64)])
+def test_step_of_single_tokens_is_what_the_general_step_would_hold(pad, static):
+    """Rows of one token take a path of their own through build_step: every array against its definition, at page edges, with a
+    token still on the device, scratch rows, two page groups, and again after a step that left other numbers behind."""
+    from mini_inference_engine_amd.engine.batch import StepArena, StepRow, build_step
+    cache = CacheManager(16, [GroupSpec(None, 30), GroupSpec(None, 30)], 8)
+    arena = StepArena(8, 6, 4, 2, "cpu")
+    starts = [0, 15, 16]
+    rcs = []
+    for i, s in enumerate(starts):
+        rc = cache.open(i)
+        assert cache.reserve(rc, 0, s + 1)
+        rcs.append(rc)
+    long_rc = cache.open("long")
+    assert cache.reserve(long_rc, 0, 8)
+    build_step([StepRow(long_rc, [9, 8, 7, 6, 5, 4, 3, 2], 0, [7])], arena, 16)
+    rows = [StepRow(rcs[0], [11], 0, [0]), StepRow(rcs[1], [0], 15, [], taken_from=2), StepRow(rcs[2], [13], 16, [0])]
+    step = build_step(rows, arena, 16, pad_rows_to=pad, static_context=static, want_all=bool(pad),
+                      sampling=([0.5, 0.0, 1.0], [3, 4, 5], [0, 1, 2]) if pad else None)
+    n = max(3, pad)
+    more = [0] * (n - 3)
+    assert (step.num_tokens, step.num_rows, step.num_decode_rows, step.max_row_tokens) == (n, n, n, 1)
+    assert step.max_context == (static or 17) and step.num_logits == (n if pad else 2)
+    assert step.input_ids.tolist() == [11, 0, 13] + more and step.taken_from.tolist() == [-1, 2, -1] + [-1] * (n - 3)
+    assert step.positions.tolist() == starts + more == step.row_position.tolist()
+    assert step.row_context.tolist() == [s + 1 for s in starts] + [1] * (n - 3)
+    assert step.token_row.tolist() == list(range(n)) and step.row_start.tolist() == list(range(n + 1))
+    assert step.state_slots.tolist() == [rc.state_slot for rc in rcs] + more
+    assert step.logit_rows.tolist() == (list(range(n)) if pad else [0, 2])
+    for g in range(2):
+        want = [rc.tables[g][s // 16] * 16 + s % 16 for rc, s in zip(rcs, starts)] + more
+        assert step.groups[g].slot_mapping.tolist() == want
+        for r, (rc, s) in enumerate(zip(rcs, starts)):
+            used = s // 16 + 1
+            assert step.groups[g].block_tables[r].tolist()[:2] == (rc.tables[g][:used] + [0])[:2]
+    if pad:
+        assert step.sample_temps.tolist() == [0.5, 0.0, 1.0] + more and step.sample_seeds.tolist() == [3, 4, 5] + more
+    for name, t in (("row_start", step.row_start), ("positions", step.positions), ("row_context", step.row_context)):
+        assert step.host[name].tolist() == t.tolist()
+    with pytest.raises(ValueError, match="pages reserved"):
+        build_step([StepRow(rcs[0], [1], 16, [0])], arena, 16)
+    with pytest.raises(ValueError, match="wanted offset"):
+        build_step([StepRow(rcs[0], [1], 0, [1])], arena, 16)
+    with pytest.raises(ValueError, match="exceeds the arena"):
+        build_step(rows, arena, 16, pad_rows_to=7)
