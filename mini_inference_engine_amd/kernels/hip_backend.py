@@ -1515,8 +1515,12 @@ class HipBackend(KernelBackend):
                              f"({bt.shape[1]} pages of {page})")
         return T, page, bt
 
-    # workgroups the decode attention kernel should at least be spread over (two per compute unit)
+    # Workgroups the decode attention kernel should at least be spread over: two a compute unit, or, where rows and heads alone
+    # give at most 64, four (the bound on the context is often far above the contexts, and the splits beyond them are empty).
+    # Decode steps with four / two, us: 16 rows at TinyLlama sizes 1,110 / 1,142, 8 rows of up to 6,000 of 8,192 keys at four
+    # layers of Llama-3-8B's 748 / 755; 128 workgroups without a split (4 rows, 32 kv heads) 543 / 521.
     DECODE_TARGET_WORKGROUPS = 512
+    DECODE_FEW_WORKGROUPS = 64
     DECODE_WHOLE_WORKGROUPS = 256
 
     def decode_splits(self, rows: int, Hq: int, Hkv: int, context_bound: int, window, block_keys: int,
@@ -1537,7 +1541,8 @@ class HipBackend(KernelBackend):
         base = rows * Hkv * -(-(Hq // Hkv) // 16)
         most = max(1, -(-context_bound // block_keys))
         whole_from = min(self.DECODE_WHOLE_WORKGROUPS, 32 + context_bound * head_dim // (64 * 18))
-        target = self.DECODE_TARGET_WORKGROUPS if base < whole_from else base
+        few = base <= self.DECODE_FEW_WORKGROUPS
+        target = self.DECODE_TARGET_WORKGROUPS * (2 if few else 1) if base < whole_from else base
         splits = max(1, min(-(-target // base), most))
         partition = -(-(-(-context_bound // splits)) // block_keys) * block_keys
         return partition, max(1, -(-context_bound // partition))
