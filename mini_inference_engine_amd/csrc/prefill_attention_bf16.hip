@@ -22,8 +22,8 @@
 // registers: block i + 1 waits in registers while block i is computed, block i + 2 is on its way, the pages
 // of block i + 3 are looked up), in rows padded so that the fragment reads meet no bank conflict.  The more
 // queries share a block the better: what bounds the kernel at long contexts is the traffic from the L2 into
-// the workgroups.  Work per stretch grows with its place in the row (causal), so a workgroup takes stretch
-// NS - 1 - i and then stretch i: every workgroup of a row has the same number of blocks.  A block every
+// the workgroups.  Work per stretch grows with its place in the row (causal), so where stretches outnumber the
+// compute units a workgroup takes stretch NS - 1 - i and then stretch i: every workgroup of a row has the same number of blocks.  A block every
 // query of a wave sees whole takes a path without masks; the running maximum m is kept in units of
 // scale * log2(e); l is a per-lane partial sum, joined over a query's two lanes at the end.
 //
@@ -623,35 +623,38 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
     compute_units[dev] = n;
   }
   // the grid for `waves` waves a workgroup: waves side by side over the heads of a group (a power of two), the rest
-  // over 32-query tiles; a workgroup takes a late stretch and an early one
-  int paired = 1;
-  auto plan = [&](int waves, int* waves_h, dim3* grid) {
+  // over 32-query tiles; a workgroup takes a late stretch and an early one (in pairs) or one stretch
+  auto plan = [&](int waves, bool in_pairs, int* waves_h, dim3* grid) {
     int wh = 1;
     while (wh < G && wh < waves) wh <<= 1;
     const int head_chunks = (G + wh - 1) / wh;
     const int stretch = (waves / wh) * PF_QW;
     const long stretches = (max_row_tokens + stretch - 1) / stretch;
     *waves_h = wh;
-    *grid = dim3((unsigned)((stretches + 1) / 2), rows, Hkv * head_chunks);
+    *grid = dim3((unsigned)(in_pairs ? (stretches + 1) / 2 : stretches), rows, Hkv * head_chunks);
     return (long)grid->x * grid->y * grid->z;
   };
-  // Eight waves over twice the queries where that still gives every compute unit a workgroup; else, at head
-  // sizes that leave room, eight waves in two halves over the keys (the grid of four waves); else four waves.
+  // How the stretches meet the compute units (a compute unit holds one workgroup of eight waves), at head sizes that leave room
+  // for eight waves; measured at one row of 128 to 2,048 tokens behind 0, 1,000 and 4,096, 16 or 32 heads (MI355X, us):
+  //   two halves over the keys, a stretch a workgroup, while that is no more than a workgroup a compute unit: in pairs half the
+  //     compute units and twice the chain (512 tokens of 32 / 4 heads of 64 19 -> 14, of 32 / 8 of 128 behind 4,096 283 -> 153);
+  //   else above head size 64 twice the queries, a stretch a workgroup, while that is: a step brings half the keys in for the same
+  //     products (2,048 tokens of 32 / 8 of 128 alone 87 in halves and pairs, 84; behind 4,096 344 -> 229; at head size 64
+  //     42 -> 55 and 150 -> 146, so not there);
+  //   else two halves in pairs, while they are (two rounds of it, the second half empty, are slower: 2,560 tokens of 32 / 4 of 64
+  //     95 us against 45 for 2,048);
+  //   else twice the queries in pairs.
   enum { FOUR, EIGHT_QUERIES, EIGHT_KEYS } kind = FOUR;
   int waves_h;
   dim3 grid;
+  bool paired = true;
   if (PF_MAX_WAVES == 8) {
-    // A compute unit holds one workgroup of eight waves (registers): more of the two-halves kind than compute
-    // units would run in two rounds, the second half empty (2,560 tokens: 95 us, against 45 for 2,048).
-    const long n4 = plan(4, &waves_h, &grid);
-    kind = n4 > compute_units[dev] ? EIGHT_QUERIES : EIGHT_KEYS;
+    const long units = compute_units[dev];
+    if (plan(4, false, &waves_h, &grid) <= units) { kind = EIGHT_KEYS; paired = false; }
+    else if (D > 64 && plan(8, false, &waves_h, &grid) <= units) { kind = EIGHT_QUERIES; paired = false; }
+    else kind = plan(4, true, &waves_h, &grid) <= units ? EIGHT_KEYS : EIGHT_QUERIES;
   }
-  const long pairs = plan(kind == EIGHT_QUERIES ? 8 : 4, &waves_h, &grid);
-  if (2 * pairs <= compute_units[dev]) {        // every stretch its own compute unit (512 tokens of 32 / 4 heads of 64: 64
-                                                // workgroups in pairs, prompt of 333 tokens in a step of 512 2,933 -> 2,803 us)
-    paired = 0;
-    grid.x = (unsigned)((max_row_tokens + (kind == EIGHT_QUERIES ? 8 : 4) / waves_h * PF_QW - 1) / ((kind == EIGHT_QUERIES ? 8 : 4) / waves_h * PF_QW));
-  }
+  plan(kind == EIGHT_QUERIES ? 8 : 4, paired, &waves_h, &grid);
   if (grid.y > 65535 || grid.z > 65535) MIE_FAIL("prefill_attention: grid too large (%d rows)", rows);
   const float scale_log2 = sigmoid ? scale : scale * 1.4426950408889634f;      // the sigmoid kernels fold their own constants
   // more LDS than a kernel gets by default is asked for once per kernel and device
@@ -668,7 +671,7 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
     hipLaunchKernelGGL(kernel, grid, dim3(waves * 64), lds_bytes, stream, (const bf16*)q, q_stride, (const bf16*)k_cache,
                        (const bf16*)v_cache, (bf16*)out, block_tables, max_blocks, row_start, row_position, first_row, Hq, Hkv,
                        waves_h, page, scale_log2, window, sink_log2, chunk, softcap, head_bias, dist_bias, dist_n, keep,
-                       head_sinks, paired);
+                       head_sinks, paired ? 1 : 0);
     return 0;
   };
   int rc = 0;
