@@ -1,0 +1,266 @@
+// Matrix products of the bfloat16 path with more than 128 rows, where more than the library's product is gained beside it:
+//
+//   gate and up with silu(gate) * up on their float32 sums (the separate pass over the library's output reads and writes both
+//   once more), and narrow weights over a long K in parts of K, whose sums meet in the add + norm kernel that follows anyway
+//   (reduce_rows in gemm_mid_bf16.hip).          x [M, K], W [N, K] bfloat16, float32 sums
+//
+// A workgroup makes BM x BN outputs with waves of 64 x 64 (v_mfma_f32_16x16x32_bf16, A = 16 weight rows, B = 16 x rows).
+// Stages of 64 k come into a ring in the LDS by loads that write it directly, 8 rows x 128 bytes a load: whole cache lines
+// (in halves of 64 bytes large tiles were up to a third slower: the L2s are asked twice for every line).  Row r's block b of
+// 16 bytes stands at 8 r + (b ^ r % 8), so that the fragment reads (lane 16 g + r: row r, block g) spread over all banks.
+//
+// What bounds it: the traffic from the L2s into the workgroups, 8 to 13 TB/s with every tile, ring and number of workgroups
+// tried (the library's kernels move 11); reading the next fragments while one set is multiplied, across the barrier too,
+// changed nothing.  So what counts is bytes a workgroup brings in, and that every compute unit has one: TILE_STAGE_US, the
+// time of a stage of each tile, times the rounds of its grid picks the tile.
+#include "common.hpp"
+#include <mutex>
+#include <set>
+#include <utility>
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define TG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
+
+enum { TG_F32, TG_SWIGLU };
+
+// 16 bytes a lane from base + offset into the LDS at byte `at` + 16 lane.  The compiler does not see that memory is on its
+// way: the waits are the kernel's own (TG_VMCNT and a barrier before a stage is read).
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t at) {
+  asm volatile(
+    "s_mov_b32 m0, %0\n\t"
+    "s_nop 0\n\t"
+    "global_load_lds_dwordx4 %1, %2"
+    :
+    : "s"(at), "v"(offset), "s"(base)
+    : "memory");
+}
+
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(a)) | ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(b)) << 16);
+}
+
+// grid: tiles over m (fastest), then n, then units of K, re-dealt so that an XCD takes a contiguous run of them.
+// K in units of stages; unit z's sums go to out + z * unit_stride.
+template <int WR, int WC, int STAGES, int EPI>
+__global__ void __launch_bounds__(WR * WC * 64)
+tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, void* __restrict__ outv, long ldo,
+                 int M, int N, int stages_all, int stages_unit, long unit_stride, int mt, int nt, int up_offset) {
+  constexpr int WAVES = WR * WC, BM = WR * 64, BN = WC * 64, XL = BM / 8, LOADS = XL + BN / 8;
+  constexpr int STAGE = LOADS * 1024, L = (LOADS + WAVES - 1) / WAVES;
+  static_assert((STAGES - 2) * L <= 63, "more loads in flight than the counter holds");
+  extern __shared__ __align__(1024) char tg_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kb = lane >> 4;
+  // workgroup i runs on XCD i % 8: give every XCD a run of neighbours, so that a weight tile is fetched into one L2
+  int id = blockIdx.x;
+  {
+    const int total = gridDim.x, q = total >> 3, r = total & 7, x = id & 7, y = id >> 3;
+    id = x * q + (x < r ? x : r) + y;
+  }
+  const int tm = id % mt, rest = id / mt, tn = rest % nt, unit = rest / nt;
+  const int m0 = tm * BM;
+  const int st0 = unit * stages_unit;
+  const int nst = st0 + stages_unit < stages_all ? stages_unit : stages_all - st0;
+
+  const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;          // this lane's place in a load of 8 rows
+  uint32_t off[L], at[L];
+  bool is_w[L];
+#pragma unroll
+  for (int j = 0; j < L; ++j) {
+    const int f = wave * L + j < LOADS ? wave * L + j : LOADS - 1;      // (the last one again)
+    is_w[j] = f >= XL;
+    long row;
+    if (f < XL) {
+      row = m0 + f * 8 + lrow;
+      if (row >= M) row = M - 1;
+      off[j] = (uint32_t)(row * ldx * 2) + lblk * 16;
+    } else {
+      const int r = (f - XL) * 8 + lrow;
+      if (EPI == TG_SWIGLU) {                  // a wave's 64 weight rows: 32 gate rows, then the up rows of the same columns
+        row = (long)tn * (BN / 2) + (r >> 6) * 32 + (r & 31);
+        if (row >= N) row = N - 1;
+        row += ((r >> 5) & 1) * (long)up_offset;
+      } else {
+        row = (long)tn * BN + r;
+        if (row >= N) row = N - 1;
+      }
+      off[j] = (uint32_t)(row * ldw * 2) + lblk * 16;
+    }
+    at[j] = f * 1024;
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)tg_lds;
+  auto issue = [&](int s) {
+    const char* xb = reinterpret_cast<const char*>(X) + (size_t)(st0 + s) * 128;
+    const char* wb = reinterpret_cast<const char*>(W) + (size_t)(st0 + s) * 128;
+    const uint32_t base = lds0 + (s % STAGES) * STAGE;
+#pragma unroll
+    for (int j = 0; j < L; ++j) load_to_lds(is_w[j] ? wb : xb, off[j], base + at[j]);
+  };
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wr = wave % WR, wc = wave / WR;
+  const char* xl = tg_lds + (wr * 64 + col) * 128;
+  const char* wl = tg_lds + (BM + wc * 64 + col) * 128;
+
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nst) issue(s);
+  for (int it = 0; it < nst; ++it) {
+    if (it + STAGES - 1 <= nst) TG_VMCNT((STAGES - 2) * L);      // this wave's loads of stage `it` have landed
+    else TG_VMCNT(0);
+    __builtin_amdgcn_s_barrier();                                // and everybody else's; everybody is done with stage it - 1
+    asm volatile("" ::: "memory");
+    if (it + STAGES - 1 < nst) issue(it + STAGES - 1);
+    const int stage = (it % STAGES) * STAGE;
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const int blk = stage + ((4 * kc + kb) ^ (col & 7)) * 16;
+      bf16x8 wf[4], xf[4];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) wf[a] = *reinterpret_cast<const bf16x8*>(wl + blk + a * 2048);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) xf[b] = *reinterpret_cast<const bf16x8*>(xl + blk + b * 2048);
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf[b], acc[a][b], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // this wave has read the stage before the next barrier
+  }
+
+  // acc[a][b][i] of lane (col, kb): weight row 16 a + 4 kb + i of the wave's 64, x row 16 b + col
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int m = m0 + wr * 64 + b * 16 + col;
+    if (m >= M) continue;
+    if (EPI == TG_SWIGLU) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int n = tn * (BN / 2) + wc * 32 + a * 16 + 4 * kb;
+        if (n >= N) continue;
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = acc[a][b][i];
+          o[i] = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * acc[a + 2][b][i];
+        }
+        *reinterpret_cast<uint2*>((bf16*)outv + (size_t)m * ldo + n) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+      }
+      continue;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int n = tn * BN + wc * 64 + a * 16 + 4 * kb;
+      if (n >= N) continue;                    // N is a multiple of 4
+      *reinterpret_cast<f32x4*>((float*)outv + unit * unit_stride + (size_t)m * ldo + n) = acc[a][b];
+    }
+  }
+}
+
+MIE_EXPORT const char* tile_gemm_bf16_last_error() { return g_mie_error; }
+
+static int allow_lds(const void* kernel, int bytes) {
+  static std::mutex lock;
+  static std::set<std::pair<int, const void*>> done;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) MIE_FAIL("tile_gemm: no current device");
+  std::lock_guard<std::mutex> g(lock);
+  if (done.count({dev, kernel})) return 0;
+  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) MIE_FAIL("tile_gemm: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
+  done.insert({dev, kernel});
+  return 0;
+}
+
+template <int WR, int WC, int STAGES, int EPI>
+static int launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, long ldo, int M, int N, int K, int units, hipStream_t s) {
+  constexpr int BM = WR * 64, BN = WC * 64, cols = EPI == TG_SWIGLU ? BN / 2 : BN;
+  constexpr int lds = STAGES * (BM + BN) * 128;
+  static_assert(lds <= 160 * 1024, "LDS");
+  auto kernel = tile_gemm_kernel<WR, WC, STAGES, EPI>;
+  if (allow_lds((const void*)kernel, lds)) return -1;
+  const int mt = (M + BM - 1) / BM, nt = (N + cols - 1) / cols, stages = K / 64, per = (stages + units - 1) / units;
+  if ((long)mt * nt * units > 0x7FFFFFFF) MIE_FAIL("tile_gemm: %d x %d tiles are beyond the grid", mt, nt);
+  hipLaunchKernelGGL(kernel, dim3(mt * nt * units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, M, N, stages, per,
+                     (long)M * N, mt, nt, N);
+  MIE_CHECK_LAUNCH("tile_gemm");
+  return 0;
+}
+
+static int check_operands(const void* X, long ldx, const void* W, long ldw, const void* out, int M, long w_rows, int N, int K) {
+  if (K <= 0 || (K & 63) || (N & 7)) MIE_FAIL("tile_gemm: K = %d (multiples of 64), N = %d (of 8)", K, N);
+  if (ldx < K || ldw < K || (ldx & 7) || (ldw & 7)) MIE_FAIL("tile_gemm: leading dims %ld, %ld for K %d", ldx, ldw, K);
+  if (((uintptr_t)X | (uintptr_t)W | (uintptr_t)out) & 15) MIE_FAIL("tile_gemm: operands must be 16-byte aligned");
+  if ((long)M * ldx > 0x40000000L || w_rows * ldw > 0x40000000L) MIE_FAIL("tile_gemm: an operand of more than 2 GiB");
+  return 0;
+}
+
+static int compute_units() {
+  static int units[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!units[dev]) {
+    int n = 0;
+    units[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+  }
+  return units[dev];
+}
+
+// Time of a stage (64 k) of a grid that gives every compute unit one workgroup, us: measured at 160 to 2,048 rows of
+// [11264, 2048] (MI355X).
+constexpr struct { int bm, bn; float us; } TILE_STAGE_US[5] = {
+  {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}};
+
+static int best_tile(int M, long cols, float& us) {
+  int best = 0;
+  us = 1e30f;
+  for (int i = 0; i < 5; ++i) {
+    const long tiles = (long)((M + TILE_STAGE_US[i].bm - 1) / TILE_STAGE_US[i].bm) * ((cols + TILE_STAGE_US[i].bn - 1) / TILE_STAGE_US[i].bn);
+    const long rounds = (tiles + compute_units() - 1) / compute_units();
+    if (rounds * TILE_STAGE_US[i].us < us) {
+      us = rounds * TILE_STAGE_US[i].us;
+      best = i;
+    }
+  }
+  return best;
+}
+
+// Estimated time of mie_tile_gemm_swiglu, in units of 0.01 us.
+MIE_EXPORT int mie_tile_gemm_swiglu_cost(int M, int N, int K) {
+  float us;
+  best_tile(M, 2L * N, us);
+  return (int)(100.f * us * (K / 64));
+}
+
+// out [M, ldo] bfloat16 = silu(x Wg^T) * (x Wu^T), W = [gate rows (N of them); up rows].
+MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long ldw, void* out, long ldo, int M, int N, int K, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  if (check_operands(X, ldx, W, ldw, out, M, 2L * N, N, K)) return -1;
+  if (ldo < N || (ldo & 3)) MIE_FAIL("tile_gemm_swiglu: output leading dim %ld for %d columns", ldo, N);
+  const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
+  float us;
+  switch (best_tile(M, 2L * N, us)) {
+    case 0: return launch<2, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 1: return launch<3, 2, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 2: return launch<4, 2, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 3: return launch<4, 3, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    default: return launch<4, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+  }
+}
+
+// part [units, M, N] float32: the sums over unit u's part of K.  Every unit has at least one stage of 64 k.
+MIE_EXPORT int mie_tile_gemm_units(const void* X, long ldx, const void* W, long ldw, float* part, int M, int N, int K, int units, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  if (check_operands(X, ldx, W, ldw, part, M, N, N, K)) return -1;
+  const int stages = K / 64, per = units > 0 ? (stages + units - 1) / units : 0;
+  if (units < 1 || (units - 1) * per >= stages) MIE_FAIL("tile_gemm_units: %d units of %d stages", units, stages);
+  const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
+  // a workgroup a compute unit and a deep ring, or two and a short one
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * units;
+  return tiles <= compute_units() ? launch<2, 2, 4, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s)
+                                  : launch<2, 2, 2, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s);
+}

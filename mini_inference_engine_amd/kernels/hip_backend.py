@@ -334,6 +334,57 @@ class HipBackend(KernelBackend):
             int(g is not None and g.dtype == torch.float32), _ptr(x_next), x_next.stride(0) if x_next is not None else 0,
             float(eps), self._stream()))
 
+    def _add_parts(self, part, sink):
+        """The partial sums into the sink's stream, and the norm that reads it next if there is one."""
+        _, M, N = part.shape
+        g = sink.norm_weight
+        if g is None or g.dtype not in (torch.bfloat16, torch.float32) or tuple(g.shape) != (N,) or not g.is_contiguous():
+            self._mid_reduce(part, self.RED_ADD, stream=sink.stream)
+            return None
+        normed = torch.empty((M, N), dtype=torch.bfloat16, device=part.device)
+        self._mid_reduce(part, self.RED_ADD_NORM, stream=sink.stream, g=g, x_next=normed, eps=sink.norm_eps)
+        done = Normed(self, None, sink.stream, g, sink.norm_eps)
+        done._value = normed            # the norm is computed: materialize() hands this out
+        return done
+
+    # ---- more rows: the engine's own tiles (csrc/tile_gemm_bf16.hip) where they gain over the library's product
+    def _tile_ok(self, x, w, bias) -> bool:
+        return (not self.true_fp32 and bias is None and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+                and x.shape[0] > self.MID_MAX_ROWS and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0
+                and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and x.shape[0] * x.stride(0) < 1 << 30 and w.shape[0] * w.stride(0) < 1 << 30)
+
+    TILE_SPLIT_MAX_ROWS = 512
+    TILE_SPLIT_MIN_K = 4096
+
+    def _tile_split(self, x, w, bias) -> int:
+        """Parts of K for a product that is added into the stream, 0: the library's.  The library walks all of a long K on few
+        workgroups; parts give every compute unit one, and their sums meet in the kernel that adds and norms anyway, until
+        those sums cost more than they save.  Product, add and norm against the library's and the norm kernel, us: 512 rows
+        of [2048, 5632] 27.9 / 29.6, 384 23.9 / 27.2, of [4096, 14336] 85 / 101 and 68 / 83; 768 rows 128 / 127, and of
+        [2048, 2048] 512 rows 21.4 / 16.7."""
+        M, (N, K) = x.shape[0], w.shape
+        if (M > self.TILE_SPLIT_MAX_ROWS or K < self.TILE_SPLIT_MIN_K or N > 8192 or not self._tile_ok(x, w, bias)):
+            return 0
+        tiles = -(-M // 128) * -(-N // 128)
+        units = 256 // tiles
+        if units * tiles < 205:                 # one workgroup a compute unit would leave many without: two
+            units = 512 // tiles
+        units = min(units, 8, K // 256)
+        return -(-(K // 64) // -(-(K // 64) // units)) if units >= 2 else 0      # as many as their stages come out at
+
+    def _tile_swiglu_gains(self, x, w, intermediate) -> bool:
+        """Whether the own gate/up product with SwiGLU on its sums beats the library's and silu_mul: its estimate (a stage's time
+        of each tile times the rounds of its grid) against what the library was measured at, 7 us + weights at 3.5 TB/s +
+        1.2 PFLOP/s, for K up to 2,048 (us, [11264, 2048]: 256 rows 25 / 30, 512 33.6 / 35.6, 1,132 55 / 60, 1,536 86 / 83 by
+        the library, 2,048 90 / 96; at K = 4,096 the library's largest tiles are as fast: 1,024 rows of [28672, 4096] 212 /
+        221, 2,048 403 / 395)."""
+        M, K = x.shape
+        if K > 2048 or intermediate % 8 or not self._tile_ok(x, w, None):
+            return False
+        library_us = 7.0 + w.shape[0] * K * 2 / 3.5e6 + 2.0 * M * w.shape[0] * K / 1.2e9
+        return self.lib("tile_gemm_bf16").mie_tile_gemm_swiglu_cost(M, intermediate, K) <= 100 * library_us
+
     def linear(self, x, w, bias=None, out_dtype=None, add_to=None):
         self._on_device(w, bias)
         _rows_ok(w, "linear: w")
@@ -373,15 +424,14 @@ class HipBackend(KernelBackend):
                 out = torch.empty((M, N), dtype=out_dtype, device=w.device)
                 self._mid_reduce(part, self.RED_BF16 if out_dtype == torch.bfloat16 else self.RED_F32, out=out)
                 return out
-            g = sink.norm_weight
-            if g is None or g.dtype not in (torch.bfloat16, torch.float32) or tuple(g.shape) != (N,) or not g.is_contiguous():
-                self._mid_reduce(part, self.RED_ADD, stream=sink.stream)
-                return None
-            normed = torch.empty((M, N), dtype=torch.bfloat16, device=w.device)
-            self._mid_reduce(part, self.RED_ADD_NORM, stream=sink.stream, g=g, x_next=normed, eps=sink.norm_eps)
-            done = Normed(self, None, sink.stream, g, sink.norm_eps)
-            done._value = normed            # the norm is computed: materialize() hands this out
-            return done
+            return self._add_parts(part, sink)
+        units = self._tile_split(x, w, bias) if sink is not None else 0
+        if units:
+            part = torch.empty((units, M, N), dtype=torch.float32, device=w.device)
+            lib = self.lib("tile_gemm_bf16")
+            library.check(lib, lib.mie_tile_gemm_units(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(part), M, N, K, units,
+                                                       self._stream()))
+            return self._add_parts(part, sink)
         if not self.true_fp32 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
             # library matrix product, 32-bit accumulation, as the reference's F.linear.  What goes into the
             # float32 stream or out as logits leaves the product in float32: the sums are not rounded to
@@ -448,6 +498,15 @@ class HipBackend(KernelBackend):
             out = torch.empty((x.shape[0], intermediate), dtype=torch.float32, device=w_gate_up.device)
             if self._f32_product(x, w_gate_up, self.F32_SWIGLU, out):
                 return out
+        if self._tile_swiglu_gains(x, w_gate_up, intermediate):
+            self._on_device(x, w_gate_up)
+            _rows_ok(x, "linear_silu_mul: x")
+            _rows_ok(w_gate_up, "linear_silu_mul: w")
+            out = torch.empty((x.shape[0], intermediate), dtype=torch.bfloat16, device=w_gate_up.device)
+            lib = self.lib("tile_gemm_bf16")
+            library.check(lib, lib.mie_tile_gemm_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0),
+                                                        x.shape[0], intermediate, x.shape[1], self._stream()))
+            return out
         return self.silu_mul(self.linear(x, w_gate_up), intermediate)
 
     ACT_CODES = {"none": 0, "silu": 1, "gelu_tanh": 2, "relu2": 3}

@@ -253,6 +253,52 @@ def test_mid_linear(engine_ops, shape):
         torch.testing.assert_close(out.materialize().double(), want, atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("shape", [(129, 4096, 264), (300, 4160, 2048), (512, 5632, 136), (385, 4096, 4104)])
+def test_tile_product_in_parts(engine_ops, shape):
+    """A long K in parts on the own tiles, added into the stream with and without the norm behind it: rows and columns beyond
+    the tiles, K whose stages do not divide over the parts; the float32 sums within the worst case of their additions."""
+    from mini_inference_engine_amd.kernels.api import Sink
+    o, (M, K, N) = engine_ops, shape
+    torch.manual_seed(M)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    units = o._tile_split(x, w, None)
+    assert units >= 2 and (units - 1) * -(-(K // 64) // units) < K // 64, "the case must take the path it is for"
+    stream = torch.randn(M, N, device=DEV)
+    expect = stream.double() + x.double() @ w.double().T
+    bound = (K + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -22 * expect.abs()
+    plain = stream.clone()
+    assert o.linear(x, w, add_to=plain) is None
+    assert bool(((plain.double() - expect).abs() <= bound).all())
+    g = torch.randn(N, device=DEV).to(torch.bfloat16)
+    normed = o.linear(x, w, add_to=Sink(stream, g, 1e-5))
+    assert torch.equal(stream, plain)
+    torch.testing.assert_close(normed.materialize().float(), torch.nn.functional.rms_norm(plain, (N,), g.float(), 1e-5), atol=2e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("shape", [(129, 64, 104), (192, 2048, 5632), (300, 192, 96), (513, 128, 5640), (1300, 2048, 2816), (2047, 64, 1000)])
+def test_tile_product_swiglu(engine_ops, shape):
+    """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
+    sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
+    from mini_inference_engine_amd.kernels import library
+    o, (M, K, inter) = engine_ops, shape
+    torch.manual_seed(K + inter)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    out = torch.full((M, inter + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    lib = o.lib("tile_gemm_bf16")
+    library.check(lib, lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K,
+                                                torch.cuda.current_stream().cuda_stream))
+    gu = x.double() @ w.double().T
+    expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
+    assert bool(((out[:, :inter].double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
+    assert bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
+    if o._tile_swiglu_gains(x, w, inter):
+        assert torch.equal(o.linear_silu_mul(x, w, inter), out[:, :inter])
+    assert lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K - 8, None) != 0
+    assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
+
+
 def test_mid_linear_refuses_what_it_cannot_run(engine_ops):
     o = engine_ops
     lib = o.lib("gemm_mid_bf16")
