@@ -36,7 +36,9 @@ rotary_kv_store_kernel(T* __restrict__ qkv, long row_stride, const int* __restri
       T* hp = row + (size_t)head * D;
       const float x1 = to_float(hp[j]), x2 = to_float(hp[j + half]);
       const float c = cr[j], s = sr[j];
-      const T o1 = from_float<T>(x1 * c - x2 * s), o2 = from_float<T>(x2 * c + x1 * s);
+      float r1, r2;
+      rotate_pair(x1, x2, c, s, r1, r2);
+      const T o1 = from_float<T>(r1), o2 = from_float<T>(r2);
       hp[j] = o1;
       hp[j + half] = o2;
       if (head >= Hq) {

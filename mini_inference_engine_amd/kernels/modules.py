@@ -40,6 +40,7 @@ register_kernel_module("gemm", {
 register_kernel_module("gemm_f32", {
     "mie_f32_units": [I, I],
     "mie_gemm_f32": [P, L, P, L, P, L, I, P, P, I, I, I, P],
+    "mie_qkv_rope_f32": [P, L, P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, I, P],
 })
 register_kernel_module("tile_gemm_bf16", {
     "mie_tile_gemm_swiglu_cost": [I, I, I],

@@ -589,6 +589,30 @@ def test_fused_projection_rotary_store(ops, geom, M):
         torch.testing.assert_close(full.float()[:, :Hq * D], q_ref[:, :Hq * D], atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("geom", [(2, 1, 16), (3, 3, 80), (5, 1, 112), (32, 4, 64), (2, 2, 256)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17])
+def test_float32_projection_rotary_store(ops, geom, M):
+    """The float32 product that rotates and writes to the cache by itself (up to 16 rows) against the product and the
+    rotary kernel in turn: the same sums, rotated with the same expression, so the same bits (17 rows: two kernels)."""
+    from mini_inference_engine_amd.kernels.api import KernelBackend
+    from mini_inference_engine_amd.parts.rope import rotary_tables
+    Hq, Hkv, D = geom
+    o = ops[torch.float32]
+    torch.manual_seed(D + M)
+    K, page, pages = 136, 16, 12
+    cos, sin = (t.to(DEV) for t in rotary_tables(10000.0, D, 300))
+    x = torch.randn(M, K, device=DEV)
+    w = torch.randn((Hq + 2 * Hkv) * D, K, device=DEV) / math.sqrt(K)
+    pos = torch.randint(0, 300, (M,), device=DEV, dtype=torch.int32)
+    slots = (torch.randperm((pages - 1) * page, device=DEV)[:M] + page).to(torch.int32)
+    kc, vc = make_cache(pages, Hkv, page, D, torch.float32)
+    kc2, vc2 = kc.clone(), vc.clone()
+    want = KernelBackend.linear_rotary_kv_store(o, x, w, pos, cos, sin, D, Hq, Hkv, D, kc2, vc2, slots)
+    out = o.linear_rotary_kv_store(x, w, pos, cos, sin, D, Hq, Hkv, D, kc, vc, slots)
+    assert (out.shape[1] == Hq * D) == (M <= 16), "one kernel for up to 16 rows, which returns q alone"
+    assert torch.equal(out[:, :Hq * D], want[:, :Hq * D]) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
+
+
 def test_rotary_q_only(ops):
     from mini_inference_engine_amd.parts.rope import rotary_tables
     cos, sin = (t.to(DEV) for t in rotary_tables(500000.0, 32, 100))
