@@ -16,8 +16,8 @@
 // positions back adds a number of its head's table to the score.  With a window and kept first keys a query also
 // sees keys 0 .. keep - 1, taken before the window's.  The sink may be a number a query head.
 //
-// This is the reference kernel of the engine: the float32 path runs on it, and the
-// bfloat16 path uses it wherever a faster kernel does not take the shape.
+// This is the reference kernel of the engine: both paths use it wherever a faster kernel (attention_f32.hip,
+// attention_bf16.hip, prefill_attention_bf16.hip) does not take the shape or the kind of attention.
 #include "common.hpp"
 
 template <typename T> struct Pack;

@@ -1,8 +1,8 @@
 // C = A W^T (+ bias): A [M, K], W [N, K] (the layout of a checkpoint's weight matrices),
 // C [M, N], for any mix of float and bfloat16 operands, accumulated in true 32-bit FMAs.
 //
-// This is the kernel of the float32 path and the fallback for operand mixes the fast
-// bfloat16 kernels do not take.  Every output element adds its K products in increasing k, sixteen
+// This is the kernel of operand mixes that the bfloat16 kernels do not take and of float32 operands that are not
+// multiples of 4 or not on 16 bytes (gemm_f32.hip takes the others).  Every output element adds its K products in increasing k, sixteen
 // at a time into a partial sum that then joins the total, whatever M, N and the tile it falls in
 // are: a token's result is bit-identical however the batch around it is cut.
 // Also here: silu(gate) * up on the fused gate/up projection output.

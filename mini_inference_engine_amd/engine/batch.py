@@ -4,7 +4,8 @@ The reference builds three device tensors and per-portion masks with Python
 loops per token (inference_engine/engine.py:133-179).  Here a step is described
 by a handful of int32 arrays that live in one arena with fixed device addresses
 (so a captured decode step can be replayed on them), filled with vectorised host
-code and sent with one copy.  Single-token rows come first, then longer portions
+code in one of two pinned mirrors in turn and sent with one copy.  A step of single
+tokens only, the common one, is filled without the general step's sums.  Single-token rows come first, then longer portions
 (inference_engine/engine.py:137); every row, whatever its length, reads the
 cache through its block table, so no mask or gathered context exists.
 """

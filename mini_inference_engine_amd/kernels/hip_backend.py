@@ -3,8 +3,9 @@
 Every wrapper checks on the host that operand shapes, dtypes and strides are what
 its kernel and grid assume before anything is launched, launches on torch's
 current stream, and raises with the library's message on a refusal.  Matrix
-products of the bfloat16 path with many rows go to the library GEMM behind
-torch (hipBLASLt), as the reference's go to cuBLAS (inference_engine/model.py:172-185);
+products of the bfloat16 path with many rows go to the library GEMM (hipBLASLt),
+as the reference's go to cuBLAS (inference_engine/model.py:172-185), unless a kernel
+here gains more than the product by what it does beside it (csrc/tile_gemm_bf16.hip);
 everything else, and every product of the float32 path, is a kernel of this
 package.  There is no CPU path and no fallback: a missing library is an error.
 """
@@ -1591,35 +1592,33 @@ class HipBackend(KernelBackend):
                              f"({bt.shape[1]} pages of {page})")
         return T, page, bt
 
-    # Workgroups the decode attention kernel should at least be spread over: two a compute unit, or, where rows and heads alone
-    # give at most 64, four (the bound on the context is often far above the contexts, and the splits beyond them are empty).
-    # Decode steps with four / two, us: 16 rows at TinyLlama sizes 1,110 / 1,142, 8 rows of up to 6,000 of 8,192 keys at four
-    # layers of Llama-3-8B's 748 / 755; 128 workgroups without a split (4 rows, 32 kv heads) 543 / 521.
+    # Workgroups of the decode attention kernel where a context is split: two a compute unit and never more, since a few beyond
+    # that wait for a round of their own.  Decode steps of full contexts with at most / at least 512, ms: Llama-3-8B sizes 3 rows
+    # 3.84 / 3.89, 6 rows 4.41 / 4.58, 10 rows 5.25 / 5.49, 12 rows 5.74 / 6.14; TinyLlama sizes 28 rows 1.515 / 1.553.  1,024 where
+    # rows and heads alone give at most 64 helps uneven contexts (16 rows 1.142 -> 1.110) and costs full ones more
+    # (8 rows of Llama-3-8B 4.70 -> 4.90, 16 rows at TinyLlama sizes 1.175 -> 1.190).
     DECODE_TARGET_WORKGROUPS = 512
-    DECODE_FEW_WORKGROUPS = 64
     DECODE_WHOLE_WORKGROUPS = 256
 
     def decode_splits(self, rows: int, Hq: int, Hkv: int, context_bound: int, window, block_keys: int,
                       head_dim: int = 64):
         """(keys per split, number of splits) for single-token rows: split the context only as far
         as the rows and heads alone do not fill the GPU (inference_engine/kernels/decode_attention.py:117-125
-        follows the same idea), in whole blocks of the kernel.
+        follows the same idea), in whole blocks of the kernel.  How far: the target above.
 
         Not split at all (no partial results, no merge kernel): always when rows and heads give every compute unit
         a workgroup; and with fewer workgroups where the contexts are short, because a workgroup then reads its
         whole context in less time than the merge kernel takes.  Measured at head size 64 (keys of 256 bytes a kv
         head): the unsplit kernel wins from 64 workgroups on at 512 keys, from 96 at 1,024, from 144 at 2,048:
         about 32 + keys / 18.  At head size 128 (8 and 32 kv heads, 1 to 16 rows, 512 to 8,192 keys) whole decode
-        steps with half the target, or unsplit at 512 keys, are within 3 % of this rule's, faster or slower by the
-        case: the rule holds there."""
+        steps that go unsplit at 512 keys are within 3 % of this rule's, faster or slower by the case: it holds there."""
         if window:
             context_bound = min(context_bound, window + 32)
         base = rows * Hkv * -(-(Hq // Hkv) // 16)
         most = max(1, -(-context_bound // block_keys))
         whole_from = min(self.DECODE_WHOLE_WORKGROUPS, 32 + context_bound * head_dim // (64 * 18))
-        few = base <= self.DECODE_FEW_WORKGROUPS
-        target = self.DECODE_TARGET_WORKGROUPS * (2 if few else 1) if base < whole_from else base
-        splits = max(1, min(-(-target // base), most))
+        target = self.DECODE_TARGET_WORKGROUPS if base < whole_from else base
+        splits = max(1, min(target // base, most))
         partition = -(-(-(-context_bound // splits)) // block_keys) * block_keys
         return partition, max(1, -(-context_bound // partition))
 
