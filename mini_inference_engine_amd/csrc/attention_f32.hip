@@ -34,10 +34,12 @@ struct AttArgs {
 };
 
 // What segment `seg` gives 16 queries of kv head kvh: fragments qf, each lane's query at position pos (-1: none) with
-// keys from lo on; last / first: the largest position and smallest lo among the 16.
+// keys from lo on; first / last: the smallest lo and the largest position among the 16.  Every query sees the keys from all_lo to
+// all_pos; a value that is not finite at another key, one that only some of them see, sets `odd`: a query that does not see
+// the key has weight 0 there, and 0 times that value is not 0, so m and l are right and o is not.
 template <int DT>
 __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, int kvh, int seg, const f32x4 (&qf)[DT], int pos, int lo,
-                                             int first, int last, float& m, float& l, f32x4 (&o)[DT]) {
+                                             int first, int last, int all_lo, int all_pos, float& m, float& l, f32x4 (&o)[DT], bool& odd) {
   constexpr int D = DT * 16;
   const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const f32x4 none = {0.f, 0.f, 0.f, 0.f};
@@ -96,6 +98,7 @@ __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, in
   l = sum;
 #pragma unroll
   for (int c = 0; c < DT; ++c) o[c] = none;
+  bool some = false;
 #pragma unroll
   for (int u = 0; u < AF_TILES; u += AHEAD) {
     f32x4 vf[AHEAD][DT];
@@ -108,11 +111,15 @@ __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, in
 #pragma unroll
     for (int t = 0; t < AHEAD; ++t) {
       const int key = base + (u + t) * 16 + 4 * g;
-      if (key - 4 * g < first || key - 4 * g + 15 > last) {        // keys nobody wrote, or whose page went back: no numbers
+      if (key - 4 * g < all_lo || key - 4 * g + 15 > all_pos) {
+        // keys none of the queries sees: nobody wrote them, or their page went back; and keys some of them see
 #pragma unroll
         for (int c = 0; c < DT; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) vf[t][c][i] = key + i >= first && key + i <= last ? vf[t][c][i] : 0.f;
+          for (int i = 0; i < 4; ++i) {
+            vf[t][c][i] = key + i >= first && key + i <= last ? vf[t][c][i] : 0.f;
+            some |= !(fabsf(vf[t][c][i]) < INFINITY) && (key + i < all_lo || key + i > all_pos);
+          }
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -120,6 +127,7 @@ __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, in
         for (int c = 0; c < DT; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][c][i], s[u + t][i], o[c], 0, 0, 0);
     }
   }
+  odd = __builtin_amdgcn_ballot_w64(some) != 0;
 }
 
 // weights of what is there and of what joins
@@ -169,16 +177,35 @@ portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ r
 #pragma unroll
   for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int* bt = a.block_tables + (size_t)row * a.max_blocks;
-  for (int seg = first / AF_SEG; seg * AF_SEG <= last; ++seg) {
+  const auto first_of = [&](int p) { return a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0; };
+  bool odd = false;
+  auto add = [&](int seg, int qpos, int f, int e, int all_lo, int all_pos, bool mine) {
     float m, l, wa, wb;
     f32x4 o[DT];
-    segment_sums<DT>(a, bt, kvh, seg, qf, pos, lo, first, last, m, l, o);
+    segment_sums<DT>(a, bt, kvh, seg, qf, qpos, lo, f, e, all_lo, all_pos, m, l, o, odd);
+    if (!mine) return;
     join_weights(M, m, wa, wb);
     L = joined(L, wa, l, wb);
 #pragma unroll
     for (int c = 0; c < DT; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) O[c][i] = joined(O[c][i], wa, o[c][i], wb);
+  };
+  for (int seg = first / AF_SEG; seg * AF_SEG <= last && !odd; ++seg) add(seg, pos, first, last, first_of(last), p0, true);
+  if (odd) {
+    // (values of the row's later tokens, or, beside padding tokens, of slots of its last page that nobody wrote)  All over
+    // again, one token after the other: the same bits for what is a number
+    M = -INFINITY;
+    L = 0.f;
+#pragma unroll
+    for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int p = p0; p <= last; ++p) {
+      const bool mine = pos == p;
+      const int f = first_of(p);
+#pragma unroll 1
+      for (int seg = f / AF_SEG; seg * AF_SEG <= p; ++seg) add(seg, mine ? pos : -1, f, p, f, p, mine);
+    }
   }
   if (!live) return;
   const float inv = 1.0f / L;
@@ -207,7 +234,8 @@ single_f32_kernel(AttArgs a, float* __restrict__ out, float* __restrict__ o_part
   f32x4 qf[DT], o[DT];
   load_queries<DT>(a, live ? t : -1, h, qf);
   float m, l;
-  segment_sums<DT>(a, a.block_tables + (size_t)token_row[t] * a.max_blocks, kvh, seg, qf, live ? p : -1, first, first, p, m, l, o);
+  bool odd;                                   // (of no account: all queries are one token's)
+  segment_sums<DT>(a, a.block_tables + (size_t)token_row[t] * a.max_blocks, kvh, seg, qf, live ? p : -1, first, first, p, first, p, m, l, o, odd);
   if (!live) return;
   if (splits == 1) {                          // joined with nothing: O 0 + o 1, L 0 + l 1
     const float inv = 1.0f / l;

@@ -390,6 +390,36 @@ def test_full_budget_portions_through_the_captured_graph(tiny_models, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float32"])
+@pytest.mark.parametrize("model", ["A", "B"])
+def test_padded_portions_see_nothing_that_the_request_did_not_write(tiny_models, model, dtype):
+    """Captured portions lengthened with padding tokens, and single tokens behind them, on a cache that holds NaN in every slot
+    the request has not written, the scratch page among them: the logits of the same steps on a cache of zeros, bit for bit."""
+    from mini_inference_engine_amd.engine.batch import StepRow
+    from mini_inference_engine_amd.engine.runner import ModelRunner
+    m = tiny_models[model]
+    toks = prompts_for(m, [60], seed=12)[0]
+    runner = ModelRunner(m["folder_f32"] if dtype == "float32" else m["folder_bf16"], dtype=dtype, device="cuda", num_pages=12,
+                         max_rows=4, max_step_tokens=48)
+    runner.capture_portion_graphs([16, 48])
+    seen = []
+    for fill in (0.0, float("nan")):
+        rc = runner.cache.open(str(fill))
+        for e in runner.storage.entries.values():
+            for t in e.tensors.values():
+                t.fill_(fill)
+        start, logits = 0, []
+        for n in (7, 29, 5, 1, 13):
+            assert runner.cache.reserve(rc, start, n)
+            logits.append(runner.forward_step([StepRow(rc, toks[start:start + n], start, [n - 1])]).clone())
+            assert runner.last_step_captured == (n > 1)
+            start += n
+        runner.cache.close(rc)
+        seen.append(torch.cat(logits))
+    assert bool(torch.isfinite(seen[0]).all()) and torch.equal(seen[0], seen[1])
+
+
+@pytest.mark.gpu
 def test_phase_ranges_change_nothing(tiny_models):
     """EngineConfig.trace_ranges marks schedule / prepare / forward / sample of every step for a profiler (the
     reference marks the same phases, inference_engine/engine.py:183-210); with or without them the same tokens."""

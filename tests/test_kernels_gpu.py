@@ -1109,6 +1109,44 @@ def test_attention_float32_matrix_unit(ops, geom, window):
         assert torch.equal(o.paged_attention(q, Hq, Hkv, D, kc, vc, wide, single, 1 / math.sqrt(D), window), whole)
 
 
+# 16 queries of a wave: 16, 2, 5 and 1 neighbouring tokens; a window whose first key lies inside a tile of 16 keys
+@pytest.mark.parametrize("window", [None, 21])
+@pytest.mark.parametrize("geom", [(4, 4, 64, 16), (32, 4, 64, 16), (3, 1, 32, 48), (32, 2, 16, 16)])
+def test_attention_float32_looks_at_no_other_querys_keys(ops, geom, window):
+    """A row lengthened with padding tokens whose keys lie in the scratch page, with NaN in every slot the row did not write:
+    the row's own tokens get the bits of the step without padding.  And what is not a number in a value of the row itself
+    reaches the tokens that see it, in the dimension it stands in, and no others."""
+    Hq, Hkv, D, page = geom
+    o, n, real, padded = ops[torch.float32], 170, 29, 48
+    q, kc, vc, group, step = paged_setup([n], [real], Hq, Hkv, D, page, torch.float32, seed=D + Hq)
+    clean = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 0.2, window)
+    bt = torch.nn.functional.pad(group.block_tables, (0, 4))
+    lo = 0 if window is None else n - real - window + 1
+    own = torch.zeros(kc.shape[0], page, dtype=torch.bool, device=DEV)
+    for p in range(lo, n):
+        own[int(bt[0, p // page]), p % page] = True
+    kd, vd = kc.clone(), vc.clone()
+    kd.permute(0, 2, 1, 3)[~own] = float("nan")
+    vd.permute(0, 3, 1, 2)[~own] = float("nan")
+    longer = SimpleNamespace(token_row=torch.zeros(padded, dtype=torch.int32, device=DEV), num_rows=1, num_tokens=padded,
+                             positions=torch.arange(n - real, n - real + padded, dtype=torch.int32, device=DEV),
+                             max_context=n - real + padded, num_decode_rows=0, max_row_tokens=padded,
+                             row_start=torch.tensor([0, padded], dtype=torch.int32, device=DEV), row_position=step.row_position)
+    wide = SimpleNamespace(block_tables=bt, max_blocks=bt.shape[1])
+    got = o.paged_attention(torch.cat([q, torch.full_like(q[:1], float("nan")).expand(padded - real, -1)]), Hq, Hkv, D, kd, vd, wide,
+                            longer, 0.2, window)
+    assert torch.equal(got[:real], clean)
+    for at, what in ((n - 3, float("inf")), (n - real + 1, float("-inf")), (n - 20, float("nan"))):
+        ve = vd.clone()
+        ve[int(bt[0, at // page]), 0, 5, at % page] = what
+        odd = o.paged_attention(q, Hq, Hkv, D, kc, ve, group, step, 0.2, window).view(real, Hkv, Hq // Hkv, D)
+        sees = torch.arange(n - real, n, device=DEV)
+        sees = (sees >= at) & (sees - at < (window or n))
+        want = clean.clone().view(real, Hkv, Hq // Hkv, D)
+        want[sees, 0, :, 5] = what
+        assert torch.equal(torch.nan_to_num(odd, 1e6, 2e6, 3e6), torch.nan_to_num(want, 1e6, 2e6, 3e6))
+
+
 # ------------------------------------------------------------------- sampling
 def test_sample_greedy_and_ties(ops):
     torch.manual_seed(0)
