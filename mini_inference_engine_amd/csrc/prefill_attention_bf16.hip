@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(PF_WAVES * 64)
 prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* __restrict__ k_cache,
                          const bf16* __restrict__ v_cache, bf16* __restrict__ out,
                          const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ row_start,
-                         const int* __restrict__ row_position, int first_row, int Hq, int Hkv, int waves_h,
+                         const int* __restrict__ row_position, const int* __restrict__ row_written, int first_row, int Hq, int Hkv, int waves_h,
                          int page, float scale_log2, int window, float sink_log2, int chunk, float softcap,
                          const float* __restrict__ head_bias, const float* __restrict__ dist_bias, int dist_n, int keep,
                          const float* __restrict__ head_sinks, int paired) {
@@ -133,6 +133,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // the same in all lanes: kept in a scalar register
   const int col = lane & 31, g = lane >> 5;
   const int t0 = row_start[row], q_len = row_start[row + 1] - t0, p0 = row_position[row];
+  const int written = row_written ? row_written[row] : p0 + q_len;     // keys from there on are nobody's: padding tokens'
   const int STRETCH = PF_QW * waves_q;
   const int NS = (q_len + STRETCH - 1) / STRETCH;              // stretches of this row
   if (bx >= (paired ? (NS + 1) / 2 : NS)) return;              // the whole workgroup, before any barrier
@@ -178,6 +179,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
     const int kmax = p0 + end_q - 1;
     int kmin = window > 0 ? p0 + s * STRETCH - window + 1 : 0;
     kmin = kmin > 0 ? kmin : 0;
+    const int vmax = kmax < written ? kmax : written - 1;      // last key whose value counts
     int q_lo = 0, tile_lo = 0;                                 // with chunks: first key of the lane's query's, of the tile's last query's
     float sg_c1 = 0.f, sg_c2 = 0.f, sg_c3 = 0.f;
     if constexpr (SIG || CHUNK) {
@@ -202,6 +204,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
         sg_c3 = -L2E * hb;
       }
     }
+    const int vmin = kmin;
     int gap = 0, kept_end = 0;
     if constexpr (KEEP) {
       kept_end = (keep + FK - 1) / FK * FK;
@@ -308,12 +311,15 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
           const int cv = c - KPIECES, t = cv % T16, dim = cv / T16;
           uint32_t w[8] = {P.lo[i].x, P.lo[i].y, P.lo[i].z, P.lo[i].w, P.hi[i].x, P.hi[i].y, P.hi[i].z, P.hi[i].w};
           const int key0 = blk + t * 16;
-          if (key0 + 15 > kmax) {
-            // slots after the row's last key may be stale: zero them (0 * NaN must not reach the sum)
+          if (key0 + 15 > vmax || key0 < vmin) {
+            // values that nobody may look at: behind the row's last key slots that were never written (also beside padding
+            // tokens, whose keys lie elsewhere), before a window's or a chunk's first key pages that went back.  Zero: their
+            // weight is 0, but 0 * NaN would reach the sum.
+            auto dead = [&](int key) { return key > vmax || (key < vmin && !(KEEP && key < keep)); };
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-              if (key0 + 2 * e > kmax) w[e] &= 0xFFFF0000u;
-              if (key0 + 2 * e + 1 > kmax) w[e] &= 0x0000FFFFu;
+              if (dead(key0 + 2 * e)) w[e] &= 0xFFFF0000u;
+              if (dead(key0 + 2 * e + 1)) w[e] &= 0x0000FFFFu;
             }
           }
           // within a row the keys stand in the order the second product wants them: for lane half 0 keys
@@ -593,10 +599,11 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 MIE_EXPORT const char* prefill_attention_bf16_last_error() { return g_mie_error; }
 
 // Rows first_row .. first_row + rows - 1 of the step (those of more than one token).  q and out are
-// indexed by flat token; row_start [all rows + 1], row_position [all rows] as the step gives them.
+// indexed by flat token; row_start [all rows + 1], row_position [all rows] as the step gives them, row_written (or null) [all
+// rows] too: a row's keys from there on are its padding tokens', which are not in its pages (null: rows have no padding tokens).
 static int prefill_attention_launch(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                     const int* block_tables, int max_blocks, const int* row_start,
-                                    const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                    const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                     int Hkv, int head_dim, int page, float scale, int window, float sink_log2,
                                     hipStream_t stream, bool sigmoid = false, int chunk = 0, float softcap = 0.f,
                                     const float* head_bias = nullptr, const float* dist_bias = nullptr, int dist_n = 0,
@@ -669,7 +676,7 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
       lds_allowed[which][dev] = true;
     }
     hipLaunchKernelGGL(kernel, grid, dim3(waves * 64), lds_bytes, stream, (const bf16*)q, q_stride, (const bf16*)k_cache,
-                       (const bf16*)v_cache, (bf16*)out, block_tables, max_blocks, row_start, row_position, first_row, Hq, Hkv,
+                       (const bf16*)v_cache, (bf16*)out, block_tables, max_blocks, row_start, row_position, row_written, first_row, Hq, Hkv,
                        waves_h, page, scale_log2, window, sink_log2, chunk, softcap, head_bias, dist_bias, dist_n, keep,
                        head_sinks, paired ? 1 : 0);
     return 0;
@@ -700,20 +707,20 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
 
 MIE_EXPORT int mie_prefill_attention(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                      const int* block_tables, int max_blocks, const int* row_start,
-                                     const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                     const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                      int Hkv, int head_dim, int page, float scale, int window, hipStream_t stream) {
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream);
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream);
 }
 
 // The same with a sink: one more term exp(sink) in every softmax's denominator that has no value.
 MIE_EXPORT int mie_prefill_attention_sink(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                           const int* block_tables, int max_blocks, const int* row_start,
-                                          const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                          const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                           int Hkv, int head_dim, int page, float scale, int window, float sink,
                                           hipStream_t stream) {
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window,
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window,
                                   sink * 1.4426950408889634f, stream);
 }
 
@@ -722,11 +729,11 @@ MIE_EXPORT int mie_prefill_attention_sink(const void* q, long q_stride, const vo
 // floor(position / n) n.  Nothing is normalised.
 MIE_EXPORT int mie_prefill_attention_sigmoid(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                              const int* block_tables, int max_blocks, const int* row_start,
-                                             const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                             const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                              int Hkv, int head_dim, int page, float scale, int window, int chunk,
                                              float softcap, const float* head_bias, hipStream_t stream) {
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
                                   true, chunk, softcap, head_bias);
 }
 
@@ -734,12 +741,12 @@ MIE_EXPORT int mie_prefill_attention_sigmoid(const void* q, long q_stride, const
 // log2 e; a key n positions back of the query adds entry min(n, dist_n - 1) of the head's row to score * scale.
 MIE_EXPORT int mie_prefill_attention_biased(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                             const int* block_tables, int max_blocks, const int* row_start,
-                                            const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                            const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                             int Hkv, int head_dim, int page, float scale, int window, const float* dist_bias,
                                             int dist_n, hipStream_t stream) {
   if (!dist_bias) MIE_FAIL("prefill_attention_biased: no table");
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
                                   false, 0, 0.f, nullptr, dist_bias, dist_n);
 }
 
@@ -747,11 +754,11 @@ MIE_EXPORT int mie_prefill_attention_biased(const void* q, long q_stride, const 
 // head_sinks float32 [Hq] or null, the numbers already times log2 e.
 MIE_EXPORT int mie_prefill_attention_kept(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                           const int* block_tables, int max_blocks, const int* row_start,
-                                          const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                          const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                           int Hkv, int head_dim, int page, float scale, int window, int keep,
                                           const float* head_sinks, hipStream_t stream) {
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
                                   false, 0, 0.f, nullptr, nullptr, 0, keep, head_sinks);
 }
 
@@ -759,11 +766,11 @@ MIE_EXPORT int mie_prefill_attention_kept(const void* q, long q_stride, const vo
 // ``window`` of them, if that is not 0).
 MIE_EXPORT int mie_prefill_attention_chunked(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out,
                                              const int* block_tables, int max_blocks, const int* row_start,
-                                             const int* row_position, int first_row, int rows, int max_row_tokens, int Hq,
+                                             const int* row_position, const int* row_written, int first_row, int rows, int max_row_tokens, int Hq,
                                              int Hkv, int head_dim, int page, float scale, int window, int chunk,
                                              hipStream_t stream) {
   if (chunk < 1) MIE_FAIL("prefill_attention_chunked: chunks of %d positions", chunk);
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
-                                  first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
+                                  row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
                                   false, chunk);
 }

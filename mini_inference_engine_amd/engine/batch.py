@@ -51,6 +51,7 @@ class StepContext:
     row_context: torch.Tensor        # [rows] int32 keys visible after this step = position + length
     state_slots: torch.Tensor        # [rows] int32
     logit_rows: torch.Tensor         # [num_logits] int32 flat token positions, in the caller's order
+    row_written: torch.Tensor | None = None     # [rows] int32: row_context without the padding tokens of a lengthened portion
     taken_from: torch.Tensor | None = None      # [T] int32, see StepRow.taken_from; -1 where input_ids holds the token
     sample_temps: torch.Tensor | None = None    # [num_logits] float32: temperature of each wanted row (0 = greedy), if
     sample_seeds: torch.Tensor | None = None    # [num_logits] int64    the step's caller wants tokens chosen from its
@@ -74,7 +75,7 @@ class StepArena:
         self.device = torch.device(device)
         fields_ = [("input_ids", max_tokens), ("taken_from", max_tokens), ("positions", max_tokens), ("token_row", max_tokens),
                    ("logit_rows", max_tokens), ("row_start", max_rows + 1), ("row_position", max_rows),
-                   ("row_context", max_rows), ("state_slots", max_rows),
+                   ("row_context", max_rows), ("row_written", max_rows), ("state_slots", max_rows),
                    # what choosing a token from a row's logits needs: they travel with the step's other arrays
                    ("sample_temps", max_rows), ("sample_counters", max_rows), ("sample_seeds", 2 * max_rows)]
         for g in range(num_groups):
@@ -212,6 +213,7 @@ def build_step(rows: Sequence[StepRow], arena: StepArena, page_size: int, *, pad
     arena.host_view("row_start")[:total_rows + 1] = row_start
     arena.host_view("row_position")[:total_rows] = row_pos
     arena.host_view("row_context")[:total_rows] = ctx
+    arena.host_view("row_written")[:total_rows] = row_pos + len(rows[0].tokens) if pad_portion_to else ctx
 
     # wanted logits, in the caller's order of rows and of ``want``
     wanted = list(range(T)) if want_all else []
@@ -289,6 +291,7 @@ def _build_single(rows, arena, page_size, total_rows, static_context, want_all, 
     arena.host_view("row_start")[:total_rows + 1] = ramp[:total_rows + 1]
     arena.host_view("row_position")[:total_rows] = positions
     arena.host_view("row_context")[:total_rows] = ctx
+    arena.host_view("row_written")[:total_rows] = ctx
     if want_all:
         wanted = ramp[:total_rows]
     else:
@@ -330,7 +333,8 @@ def _finish(arena, page_size, T, total_rows, num_decode, R, max_row_tokens, max_
         positions=arena.dev_view("positions", T),
         token_row=arena.dev_view("token_row", T), row_start=arena.dev_view("row_start", total_rows + 1),
         row_position=arena.dev_view("row_position", total_rows), row_context=arena.dev_view("row_context", total_rows),
-        state_slots=arena.dev_view("state_slots", total_rows), logit_rows=arena.dev_view("logit_rows", R),
+        row_written=arena.dev_view("row_written", total_rows), state_slots=arena.dev_view("state_slots", total_rows),
+        logit_rows=arena.dev_view("logit_rows", R),
         page_size=page_size, max_row_tokens=max_row_tokens, max_context=max_context, host=host)
     if sampling is not None:
         step.sample_temps = arena.dev_view("sample_temps", R).view(torch.float32)

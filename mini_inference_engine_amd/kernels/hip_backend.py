@@ -1758,9 +1758,12 @@ class HipBackend(KernelBackend):
                                ("row_position", step.row_position, step.num_rows)):
                 if t is None or t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous():
                     raise ValueError(f"paged_attention: {name} must be contiguous int32 [{n}]")
+            written = getattr(step, "row_written", None)        # where rows end that padding tokens lengthen
+            if written is not None and (written.dtype != torch.int32 or written.shape[0] < step.num_rows or not written.is_contiguous()):
+                raise ValueError(f"paged_attention: row_written must be contiguous int32 [{step.num_rows}]")
             lib = self.lib("prefill_attention_bf16", (f"-DHEAD_DIM={D}",))
             args = (_ptr(qkv), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(bt), bt.shape[1],
-                    _ptr(step.row_start), _ptr(step.row_position), step.num_decode_rows,
+                    _ptr(step.row_start), _ptr(step.row_position), _ptr(written), step.num_decode_rows,
                     step.num_rows - step.num_decode_rows, step.max_row_tokens, Hq, Hkv, D, page, float(scale),
                     int(window or 0))
             if sigmoid:

@@ -133,12 +133,12 @@ register_kernel_module("attention_bf16", {
 # the compiler parks the outputs in accumulation registers and copies all of them back and forth around
 # every key block for the sake of the (rare) rescaling.
 register_kernel_module("prefill_attention_bf16", {
-    "mie_prefill_attention": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, P],
-    "mie_prefill_attention_sink": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, F, P],
-    "mie_prefill_attention_sigmoid": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, I, F, P, P],
-    "mie_prefill_attention_biased": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, P, I, P],
-    "mie_prefill_attention_chunked": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, I, P],
-    "mie_prefill_attention_kept": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, I, P, P],
+    "mie_prefill_attention": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P],
+    "mie_prefill_attention_sink": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, F, P],
+    "mie_prefill_attention_sigmoid": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, F, P, P],
+    "mie_prefill_attention_biased": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P, I, P],
+    "mie_prefill_attention_chunked": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
+    "mie_prefill_attention_kept": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, P, P],
 }, variants=_head_variants, flags=["-mllvm", "-amdgpu-mfma-vgpr-form"])
 # lt_gemm: host code only, the engine's own way into the library's matrix products (hipBLASLt) with the choice of
 # kernel per shape kept here.

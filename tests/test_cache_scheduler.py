@@ -300,6 +300,7 @@ def test_a_portion_lengthened_to_a_captured_size_writes_to_the_scratch_page():
     table = arena.dev_view("block_tables0", 16).tolist()
     assert table[:3] == [7, 3, 9] and table[3:6] == [0, 0, 0]
     assert step.host["row_context"].tolist() == [21]
+    assert step.row_context.tolist() == [21] and step.row_written.tolist() == [10], "what the row's own tokens have written"
     # positions 5 .. 9 need three pages; two are not enough, padding or not
     short = SimpleNamespace(tables=[[7, 3]], state_slot=0)
     with pytest.raises(ValueError, match="pages reserved"):
@@ -336,6 +337,7 @@ def test_step_of_single_tokens_is_what_the_general_step_would_hold(pad, static):
     assert step.input_ids.tolist() == [11, 0, 13] + more and step.taken_from.tolist() == [-1, 2, -1] + [-1] * (n - 3)
     assert step.positions.tolist() == starts + more == step.row_position.tolist()
     assert step.row_context.tolist() == [s + 1 for s in starts] + [1] * (n - 3)
+    assert step.row_written.tolist() == step.row_context.tolist()
     assert step.token_row.tolist() == list(range(n)) and step.row_start.tolist() == list(range(n + 1))
     assert step.state_slots.tolist() == [rc.state_slot for rc in rcs] + more
     assert step.logit_rows.tolist() == (list(range(n)) if pad else [0, 2])

@@ -390,7 +390,7 @@ def test_full_budget_portions_through_the_captured_graph(tiny_models, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["float32"])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("model", ["A", "B"])
 def test_padded_portions_see_nothing_that_the_request_did_not_write(tiny_models, model, dtype):
     """Captured portions lengthened with padding tokens, and single tokens behind them, on a cache that holds NaN in every slot

@@ -1047,6 +1047,48 @@ def test_prefill_attention_ignores_stale_pages_bf16(ops):
     assert torch.equal(clean, dirty)
 
 
+# portions that take four waves, eight in two halves over the keys and eight over the queries; pages of 16 and 48; (kept keys, window,
+# chunk) of the forms that hide a row's first keys
+@pytest.mark.parametrize("form", ["plain", "window", "kept", "chunk", "sigmoid", "sigmoid chunk", "biased"])
+@pytest.mark.parametrize("geom", [(8, 2, 64, 16, 170, 29, 48), (32, 4, 64, 48, 600, 333, 512), (4, 4, 256, 16, 90, 35, 64), (16, 8, 128, 16, 1500, 1025, 1400)])
+def test_prefill_attention_looks_at_no_slot_its_row_did_not_write(ops, geom, form):
+    """A row lengthened with padding tokens, whose keys are not in its pages, with NaN in every slot the row did not write and in
+    the pages whose keys lie before all its queries' first: its own tokens get the bits they get from a cache of zeros there."""
+    Hq, Hkv, D, page, n, real, padded = geom
+    dtype = torch.bfloat16
+    q, kc, vc, group, step = paged_setup([n], [real], Hq, Hkv, D, page, dtype, seed=D + n)
+    window, kw, first = None, {}, 0
+    if form in ("window", "kept"):
+        window, first = 21, n - real - 20
+    if form == "kept":
+        kw = dict(keep_first=5)
+    if form.endswith("chunk"):
+        kw, first = dict(chunk=40), (n - real) // 40 * 40
+    if form.startswith("sigmoid"):
+        kw["weights"] = "sigmoid"
+    if form == "biased":
+        kw = dict(distance_bias=torch.randn(Hq, 30, device=DEV))
+    own = torch.zeros(kc.shape[0], page, dtype=torch.bool, device=DEV)
+    for p in [*range(kw.get("keep_first", 0)), *range(first, n)]:
+        own[int(group.block_tables[0, p // page]), p % page] = True
+    more = padded - real
+    longer = SimpleNamespace(token_row=torch.zeros(padded, dtype=torch.int32, device=DEV), num_rows=1, num_tokens=padded,
+                             positions=torch.arange(n - real, n + more, dtype=torch.int32, device=DEV),
+                             max_context=n + more, num_decode_rows=0, max_row_tokens=padded, row_position=step.row_position,
+                             row_start=torch.tensor([0, padded], dtype=torch.int32, device=DEV),
+                             row_written=torch.tensor([n], dtype=torch.int32, device=DEV))
+    bt = torch.nn.functional.pad(group.block_tables, (0, more // page + 2))
+    wide = SimpleNamespace(block_tables=bt, max_blocks=bt.shape[1])
+    seen = []
+    for fill in (0.0, float("nan")):
+        kd, vd = kc.clone(), vc.clone()
+        kd.permute(0, 2, 1, 3)[~own] = fill
+        vd.permute(0, 3, 1, 2)[~own] = fill
+        qd = torch.cat([q, torch.full_like(q[:1], fill).expand(more, -1)])
+        seen.append(ops[dtype].paged_attention(qd, Hq, Hkv, D, kd, vd, wide, longer, 0.2, window, **kw)[:real])
+    assert bool(torch.isfinite(seen[0]).all()) and torch.equal(seen[0], seen[1])
+
+
 def test_prefill_last_row_equals_decode(ops):
     """The last token of a portion, computed by the prefill kernel, equals the same token computed as a
     single-token row by the decode kernel (same keys, same cache), within bfloat16 rounding."""
