@@ -1800,13 +1800,17 @@ class HipBackend(KernelBackend):
 
     def _attention_f32(self, qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window) -> bool:
         """Plain causal (windowed) softmax attention of a float32 step on the 32-bit matrix unit (csrc/attention_f32.hip);
-        False where that does not take the operands.  Head sizes, strides and alignment decide, never the step's rows: a
-        request's tokens take the same arithmetic in every step."""
+        False where that does not take the operands, or a step does not say where its portions lie (the kernel of
+        attention.hip goes by tokens alone).  Head sizes, strides and alignment decide, never how many rows of how many tokens
+        a step has: a request's tokens take the same arithmetic in every step of the engine."""
         T, window = qkv.shape[0], int(window or 0)
         single = step.num_decode_rows
-        rows_known = step.row_start is not None and step.row_position is not None
+        longest = int(getattr(step, "max_row_tokens", 0) or 0)
         if (D % 16 or D > 128 or page % 16 or qkv.stride(0) % 4 or any(t.data_ptr() % 16 for t in (qkv, k_cache, v_cache))
-                or (single < T and not rows_known) or single > 65535):
+                or Hkv * -(-(Hq // Hkv) // 16) > 65535 or single > 65535 or step.num_rows - single > 65535):
+            return False
+        if single < T and (longest < 1 or any(t is None or t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous()
+                                              for t, n in ((step.row_start, step.num_rows + 1), (step.row_position, step.num_rows)))):
             return False
         lib = self.lib("attention_f32")
         caches = (_ptr(qkv), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(bt), bt.shape[1])
@@ -1822,12 +1826,9 @@ class HipBackend(KernelBackend):
             library.check(lib, lib.mie_attention_f32_single(*caches, _ptr(step.token_row), _ptr(step.positions), single, Hq, Hkv, D,
                                                             page, float(scale), window, splits, _ptr(o_part), _ptr(ml), self._stream()))
         if single < T:
-            for name, t, n in (("row_start", step.row_start, step.num_rows + 1), ("row_position", step.row_position, step.num_rows)):
-                if t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous():
-                    raise ValueError(f"paged_attention: {name} must be contiguous int32 [{n}]")
             library.check(lib, lib.mie_attention_f32_portions(*caches, _ptr(step.row_start), _ptr(step.row_position), single,
-                                                              step.num_rows, step.max_row_tokens, Hq, Hkv, D, page, float(scale),
-                                                              window, self._stream()))
+                                                              step.num_rows, longest, Hq, Hkv, D, page, float(scale), window,
+                                                              self._stream()))
         return True
 
     def sample(self, logits, temperatures, seeds, counters, out=None):
