@@ -358,15 +358,17 @@ class HipBackend(KernelBackend):
     TILE_SPLIT_MAX_ROWS = 512
     TILE_SPLIT_MIN_K = 4096
 
-    def _tile_split(self, x, w, bias) -> int:
+    def _tile_split(self, x, w, bias, sink=None) -> int:
         """Parts of K for a product that is added into the stream, 0: the library's.  The library walks all of a long K on few
         workgroups; parts give every compute unit one, and their sums meet in the kernel that adds and norms anyway, until
         those sums cost more than they save.  Product, add and norm against the library's and the norm kernel, us: 512 rows
         of [2048, 5632] 27.9 / 29.6, 384 23.9 / 27.2, of [4096, 14336] 85 / 101 and 68 / 83; 768 rows 128 / 127, and of
         [2048, 2048] 512 rows 21.4 / 16.7."""
         M, (N, K) = x.shape[0], w.shape
-        if (M > self.TILE_SPLIT_MAX_ROWS or K < self.TILE_SPLIT_MIN_K or N > 8192 or not self._tile_ok(x, w, bias)):
+        if M > self.TILE_SPLIT_MAX_ROWS or K < self.TILE_SPLIT_MIN_K or N > 8192 or not self._tile_ok(x, w, bias):
             return 0
+        if sink is not None and any(t is not None and t.data_ptr() % 16 for t in (sink.stream, sink.norm_weight)):
+            return 0                            # the kernel that joins the parts takes 16 bytes at a time
         tiles = -(-M // 128) * -(-N // 128)
         units = 256 // tiles
         if units * tiles < 205:                 # one workgroup a compute unit would leave many without: two
@@ -426,7 +428,7 @@ class HipBackend(KernelBackend):
                 self._mid_reduce(part, self.RED_BF16 if out_dtype == torch.bfloat16 else self.RED_F32, out=out)
                 return out
             return self._add_parts(part, sink)
-        units = self._tile_split(x, w, bias) if sink is not None else 0
+        units = self._tile_split(x, w, bias, sink) if sink is not None else 0
         if units:
             part = torch.empty((units, M, N), dtype=torch.float32, device=w.device)
             lib = self.lib("tile_gemm_bf16")
@@ -456,7 +458,7 @@ class HipBackend(KernelBackend):
                 return self._lt_product(x, w, self.LT_BF16, torch.empty((M, N), dtype=torch.bfloat16, device=w.device))
             y = torch.nn.functional.linear(x, w, None if bias is None else bias.to(torch.bfloat16))
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
-        if self._f32_ok(x, w, bias, out_dtype):
+        if self._f32_ok(x, w, bias, out_dtype) and (sink is None or sink.stream.data_ptr() % 16 == 0):
             if sink is not None:
                 self._f32_product(x, w, self.F32_ADD, sink.stream, bias)
                 return None if sink.norm_weight is None else Normed(self, None, sink.stream, sink.norm_weight, sink.norm_eps)

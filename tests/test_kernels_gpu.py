@@ -276,6 +276,30 @@ def test_tile_product_in_parts(engine_ops, shape):
     torch.testing.assert_close(normed.materialize().float(), torch.nn.functional.rms_norm(plain, (N,), g.float(), 1e-5), atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("case", [(torch.float32, 5, 64, 36), (torch.float32, 70, 64, 132), (torch.bfloat16, 300, 4096, 264)])
+def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
+    """A contiguous float32 stream (and a norm weight) that starts anywhere: what the kernels for 16-byte pieces do not take goes
+    where it went without them, and the sum arrives either way."""
+    from mini_inference_engine_amd.kernels.api import Normed, Sink
+    dtype, M, K, N = case
+    o = engine_ops if dtype == torch.bfloat16 else ops[dtype]
+    torch.manual_seed(K)
+    x = torch.randn(M, K, device=DEV).to(dtype)
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(dtype)
+    base, g = torch.randn(M, N, device=DEV), torch.randn(N + 1, device=DEV)[1:]
+    want = base.double() + x.double() @ w.double().T
+    for off in (0, 1):
+        stream = torch.empty(M * N + off, device=DEV)[off:].view(M, N).copy_(base)
+        normed = o.linear(x, w, add_to=Sink(stream, g, 1e-5))
+        if torch.is_tensor(normed):                 # not added yet: the caller's to do
+            stream += normed
+        else:
+            assert isinstance(normed, Normed)
+            y = torch.nn.functional.rms_norm(want, (N,), g.double(), 1e-5)
+            torch.testing.assert_close(normed.materialize().double(), y, **tol(dtype))
+        torch.testing.assert_close(stream.double(), want, atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("shape", [(129, 64, 104), (192, 2048, 5632), (300, 192, 96), (513, 128, 5640), (1300, 2048, 2816), (2047, 64, 1000)])
 def test_tile_product_swiglu(engine_ops, shape):
     """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
