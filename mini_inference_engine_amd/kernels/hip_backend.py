@@ -1487,6 +1487,7 @@ class HipBackend(KernelBackend):
             page = self._check_rope_operands("linear_rotary_kv_store", M, K, w_qkv, positions, cos, sin, Hq, Hkv, D, k_cache,
                                              v_cache, slot_mapping, torch.float32)
             _rows_ok(x, "linear_rotary_kv_store: x")
+            _rows_ok(w_qkv, "linear_rotary_kv_store: w")
             q = torch.empty((M, Hq * D), dtype=torch.float32, device=x.device)
             lib = self.lib("gemm_f32")
             library.check(lib, lib.mie_qkv_rope_f32(_ptr(x), x.stride(0), _ptr(w_qkv), w_qkv.stride(0), _ptr(q), q.stride(0),

@@ -637,6 +637,23 @@ def test_float32_projection_rotary_store(ops, geom, M):
     assert torch.equal(out[:, :Hq * D], want[:, :Hq * D]) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
 
 
+@pytest.mark.parametrize("M", [5, 17])
+def test_float32_projection_rotary_store_refuses_strided_weights(ops, M):
+    """A weight matrix whose rows are not contiguous (or x so) is refused with any number of rows, and nothing is written."""
+    from mini_inference_engine_amd.parts.rope import rotary_tables
+    Hq, Hkv, D, K, page, pages = 2, 1, 16, 64, 16, 4
+    o = ops[torch.float32]
+    cos, sin = (t.to(DEV) for t in rotary_tables(10000.0, D, 30))
+    wide, x2 = torch.randn((Hq + 2 * Hkv) * D, 2 * K, device=DEV), torch.randn(M, 2 * K, device=DEV)
+    pos = torch.arange(M, device=DEV, dtype=torch.int32)
+    kc, vc = make_cache(pages, Hkv, page, D, torch.float32)
+    kept = kc.clone()
+    for x, w in ((x2[:, :K], wide[:, ::2]), (x2[:, ::2], wide[:, :K])):
+        with pytest.raises(ValueError, match="unit inner stride"):
+            o.linear_rotary_kv_store(x, w, pos, cos, sin, D, Hq, Hkv, D, kc, vc, pos + page)
+    assert torch.equal(kc, kept)
+
+
 def test_rotary_q_only(ops):
     from mini_inference_engine_amd.parts.rope import rotary_tables
     cos, sin = (t.to(DEV) for t in rotary_tables(500000.0, 32, 100))
