@@ -325,29 +325,42 @@ delta_fold_kernel(const float* __restrict__ summaries, float* __restrict__ start
 
 // ---- long rows on the matrix cores: chunks of 64 tokens, heads of up to 64, in 32-bit (v_mfma_f32_16x16x4_f32)
 //
-// With w = a * u, G_t the sum of log2 decays over a chunk's tokens up to t and y_t = S_(t-1)^T u_t, unrolled from the state S_0
-// the chunk starts from:
-//     S_t = 2^G_t S_0 + sum_(s <= t) 2^(G_t - G_s) (k_s v_s^T - w_s y_s^T)
-//     (I + A) y = (2^G_(t-1) u) S_0 + B v,      A_ts = sum_i u_ti w_si 2^(G_(t-1) - G_s)  (s < t),   B the same with k_s for w_s
-//     o = (2^G_t r) S_0 + Qk v - Qw y,          Qk_ts = sum_i r_ti k_si 2^(G_t - G_s)  (s <= t),     Qw the same with w_s
-// so with [W | U] = (I + A)^-1 [2^G_(t-1) u | B v] a chunk acts on S_0 by four 64 x 64 matrices:
-//     S_end = P S_0 + E,  P = 2^G_end - (2^(G_end - G) w)^T W,  E = (2^(G_end - G) k)^T v - (2^(G_end - G) w)^T U
-//     o = R S_0 + F,      R = 2^G r - Qw W,                     F = Qk v - Qw U
+// With w = a * u, P_t the product of a chunk's decays up to token t (a number a channel) and y_t = S_(t-1)^T u_t, unrolled from
+// the state S_0 the chunk starts from (the triangular-solve form of the chunked delta rule: the WY representation of a product of
+// rank-one updates, with a decay a channel):
+//     S_t = P_t S_0 + sum_(s <= t) P_t / P_s (k_s v_s^T - w_s y_s^T)
+//     (I + A) y = (P_(t-1) u) S_0 + B v,      A_ts = sum_i u_ti w_si P_(t-1)i / P_si  (s < t),   B the same with k_s for w_s
+//     o = (P_t r) S_0 + Qk v - Qw y,          Qk_ts = sum_i r_ti k_si P_ti / P_si  (s <= t),     Qw the same with w_s
+// so with [W | U] = (I + A)^-1 [P_(t-1) u | B v] a chunk acts on S_0 by four 64 x 64 matrices:
+//     S_end = P S_0 + E,  P = P_end - (P_end / P_s w)^T W,  E = (P_end / P_s k)^T v - (P_end / P_s w)^T U
+//     o = R S_0 + F,      R = P_t r - Qw W,                 F = Qk v - Qw U
 // (1) chunk_solve, a workgroup a (chunk, head): from the projection's sums to P, E, R, F;  (2) chunk_fold, per (row, head, 16
 // columns), chunk after chunk: S_0 of every chunk;  (3) chunk_outputs: o, its norm, weight and gate.
-// Powers for tokens t of one 16 and s of the same or an earlier 16 are taken against the start of t's 16, so that the products
-// run on the matrix cores; the one positive exponent is that of 16 tokens' decay at most (DELTA_SCALE_MAX keeps it finite).
+// The products run on the matrix cores, so a quotient P_t / P_s is the factor of t from the start of its 16 on, the decays of the
+// 16s between, and the factor of s up to the end of its own 16; inside one 16 the reciprocal of s's factor from its start on.
+// Every factor is a product of decays, and every sum of 64 terms is four chains of 16 that meet at the end: each number is then
+// a few roundings from true, as in the token-by-token recurrence.  (Powers of differences of summed logarithms carry a logarithm's
+// absolute rounding, and one chain over 64 or 128 terms four times as many roundings.)  Relative error of the state
+// against 64 bits, 1e-8, 512 tokens of heads of 64, decay scales 0.61 / 1 / 2 / 4 (MI355X): 9.6 / 8.2 / 9.1 / 9.5; with powers and
+// long chains 24 / 24 / 33 / 55; token by token 9.6 / 8.4 / 8.8 / 9.5.  Beyond DELTA_SCALE_MAX the token-by-token chunks are up to
+// a third more exact with other weights (heads of 32, scale 4: 4.4 against 6.2), so they take what lies there.
 // What bounds it: the solve's chain of small products (about 440 matrix instructions a SIMD and chunk) and its 32-bit arithmetic,
 // a workgroup a compute unit.  2,048 tokens of 16 heads of 64 (MI355X): 40 + 168 + 142 + 175 us (preparation, summaries, fold,
 // chunks, token by token through the LDS) -> 73 + 27 + 17 us.  The token-by-token chunks stay for heads of 65 to 128, other inner
 // sizes and stronger decays.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int CH = 64, MS = CH + 4;
-constexpr float LOG2E = 1.4426950408889634f, DELTA_SCALE_MAX = 4.f;
+constexpr float DELTA_SCALE_MAX = 1.f;
 constexpr int SOLVE_THREADS = 512;
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x); }
+// four chains of a sum meet
+__device__ __forceinline__ f32x4 meet(const f32x4 (&p)[4]) { return (p[0] + p[1]) + (p[2] + p[3]); }
+// 1 / x to within a rounding or so, x a normal number
+__device__ __forceinline__ float reciprocal(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.f), r, r);
+}
 // The waves meet over the LDS only: loads and stores of global memory stay on their way (__syncthreads would wait for them)
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -378,16 +391,17 @@ __global__ void __launch_bounds__(SOLVE_THREADS)
 chunk_solve_kernel(ChunkArgs a) {
   constexpr int DS = DP + 4, CT = DP / 16, WAVES = SOLVE_THREADS / 64;
   extern __shared__ __align__(16) float lds[];
-  float* sU = lds;                   // [64][DS] unit keys, then 2^G_(t-1) u
-  float* sK = sU + CH * DS;          // keys, then 2^(G_end - G) k
-  float* sW = sK + CH * DS;          // a * u, then 2^(G_end - G) w
-  float* sR = sW + CH * DS;          // r, then 2^G r
-  float* sG = sR + CH * DS;          // G from the start of a token's 16 on; then [64][MS] B
+  float* sU = lds;                   // [64][DS] unit keys, then P_(t-1) u
+  float* sK = sU + CH * DS;          // keys, then P_end / P_s k
+  float* sW = sK + CH * DS;          // a * u, then P_end / P_s w
+  float* sR = sW + CH * DS;          // r, then P_t r
+  float* sG = sR + CH * DS;          // decays, their products from the start of a token's 16 on; then [64][MS] B
   float* M = sG + CH * MS;           // [64][MS] the inner activations; then A
   float* X = M + CH * MS;            // [64][MS] (I + A)^-1
   float* Qw = X + CH * MS;
   float* Qk = Qw + CH * MS;
-  float* so = Qk + CH * MS;          // [4][DP] sums of 16 tokens, then 2^G_end
+  float* sT = Qk;                    // first [64][DS] products from a token's next to the end of its 16
+  float* so = Qk + CH * MS;          // [4][DP] products of a 16's decays, then P_end
   CHUNK_OF_ROW;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -433,30 +447,38 @@ chunk_solve_kernel(ChunkArgs a) {
     const int x = tile & 3, c = (tile >> 2) * 16 + n;
     const int cc = h * d + (c < d ? c : d - 1);
     const float* __restrict__ wd = a.w_decay + (size_t)cc * a.rank + 4 * g;
-    f32x4 z = none;
+    f32x4 zs[4] = {none, none, none, none};
     for (int kb = 0; kb < a.rank; kb += 16) {
       const f32x4 w = *reinterpret_cast<const f32x4*>(wd + kb);
       const f32x4 in = *reinterpret_cast<const f32x4*>(M + (16 * x + n) * MS + kb + 4 * g);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) z = mfma4(in[j], w[j], z);
+      for (int j = 0; j < 4; ++j) zs[j] = mfma4(in[j], w[j], zs[j]);
     }
+    const f32x4 z = meet(zs);
     const float b = a.decay_bias[cc];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = 16 * x + 4 * g + e;
-      sG[t * DS + c] = t < nt && c < d ? -a.decay_scale * LOG2E * mie_sigmoid(z[e] + b) : 0.f;
+      sG[t * DS + c] = t < nt && c < d ? expf(-a.decay_scale * mie_sigmoid(z[e] + b)) : 1.f;
     }
   }
   lds_barrier();
-  // ---- sums over the tokens of a 16 (differences of sums over all 64 would lose more to rounding)
+  // ---- products over the tokens of a 16 (over all 64 they could reach zero)
   if (tid < 4 * DP) {
     const int i = tid % DP, part = tid / DP;
-    float run = 0.f;
+    float run = 1.f, decay[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) decay[t] = sG[(16 * part + t) * DS + i];
+#pragma unroll
+    for (int t = 15; t >= 0; --t) {
+      sT[(16 * part + t) * DS + i] = run;
+      run *= decay[t];
+    }
+    run = 1.f;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-      float* at = sG + (16 * part + t) * DS + i;
-      run += *at;
-      *at = run;
+      run *= decay[t];
+      sG[(16 * part + t) * DS + i] = run;
     }
     so[part * DP + i] = run;
   }
@@ -470,44 +492,56 @@ chunk_solve_kernel(ChunkArgs a) {
     if (blk >= 10) break;
     const int x = blk < 4 ? 3 : blk < 7 ? 2 : blk < 9 ? 1 : 0, y = blk - (blk < 4 ? 0 : blk < 7 ? 4 : blk < 9 ? 7 : 9);
     const int t = 16 * x + n, s = 16 * y + n;
-    const float inside = n > 0 ? 1.f : 0.f;                        // the token before the 16's first: nothing
     const float* gb = sG + (t - (n > 0 ? 1 : 0)) * DS;
+    f32x4 pA[4] = {none, none, none, none}, pB[4] = {none, none, none, none}, pW[4] = {none, none, none, none}, pK[4] = {none, none, none, none};
+    const f32x4 ones = {1.f, 1.f, 1.f, 1.f};
 #pragma unroll
     for (int i = 4 * g; i < DP; i += 16) {
-      f32x4 between = none;                                         // the sum over the tokens from s's 16 up to t's
-      for (int z = y; z < x; ++z) between += *reinterpret_cast<const f32x4*>(so + z * DP + i);
-      const f32x4 gt = *reinterpret_cast<const f32x4*>(sG + t * DS + i), gp = *reinterpret_cast<const f32x4*>(gb + i) * inside;
-      const f32x4 gs = between - *reinterpret_cast<const f32x4*>(sG + s * DS + i);
+      f32x4 gp = *reinterpret_cast<const f32x4*>(gb + i);
+      if (n == 0) gp = ones;                                        // before the 16's first token: nothing
+      const f32x4 gt = *reinterpret_cast<const f32x4*>(sG + t * DS + i);
+      f32x4 es;                                                     // from s's next token to the end of its 16 and on to t's
+      if (x == y) {
+        const f32x4 gs = *reinterpret_cast<const f32x4*>(sG + s * DS + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) es[e] = reciprocal(gs[e]);
+      } else {
+        es = *reinterpret_cast<const f32x4*>(sT + s * DS + i);
+        for (int z = y + 1; z < x; ++z) es *= *reinterpret_cast<const f32x4*>(so + z * DP + i);
+      }
       const f32x4 u = *reinterpret_cast<const f32x4*>(sU + t * DS + i), r = *reinterpret_cast<const f32x4*>(sR + t * DS + i);
       const f32x4 w = *reinterpret_cast<const f32x4*>(sW + s * DS + i), k = *reinterpret_cast<const f32x4*>(sK + s * DS + i);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float lu = u[e] * pow2(gp[e]), lr = r[e] * pow2(gt[e]), es = pow2(gs[e]);
-        const float rw = w[e] * es, rk = k[e] * es;
-        accA[q] = mfma4(lu, rw, accA[q]);
-        accB[q] = mfma4(lu, rk, accB[q]);
-        accW[q] = mfma4(lr, rw, accW[q]);
-        accK[q] = mfma4(lr, rk, accK[q]);
+        const float lu = u[e] * gp[e], lr = r[e] * gt[e], rw = w[e] * es[e], rk = k[e] * es[e];
+        pA[e] = mfma4(lu, rw, pA[e]);
+        pB[e] = mfma4(lu, rk, pB[e]);
+        pW[e] = mfma4(lr, rw, pW[e]);
+        pK[e] = mfma4(lr, rk, pK[e]);
       }
     }
+    accA[q] = meet(pA);
+    accB[q] = meet(pB);
+    accW[q] = meet(pW);
+    accK[q] = meet(pK);
   }
   lds_barrier();
-  // ---- the vectors times their powers, in place, 2^G_end beside them
+  // ---- the vectors times their decays, in place, P_end beside them
   for (int e = tid; e < CH * DP; e += SOLVE_THREADS) {
     const int t = e / DP, i = e % DP, x = t >> 4;
-    float before = 0.f, after = so[x * DP + i] - sG[t * DS + i];
-    for (int z = 0; z < x; ++z) before += so[z * DP + i];
-    for (int z = x + 1; z < 4; ++z) after += so[z * DP + i];
-    const float G = sG[t * DS + i], Gb = t & 15 ? sG[(t - 1) * DS + i] : 0.f, to_end = pow2(after);
-    sU[t * DS + i] *= pow2(before + Gb);
-    sR[t * DS + i] *= pow2(before + G);
+    const float G = sG[t * DS + i], Gb = t & 15 ? sG[(t - 1) * DS + i] : 1.f;
+    float before = 1.f, to_end = sT[t * DS + i];
+    for (int z = 0; z < x; ++z) before *= so[z * DP + i];
+    for (int z = x + 1; z < 4; ++z) to_end *= so[z * DP + i];
+    sU[t * DS + i] *= before * Gb;
+    sR[t * DS + i] *= before * G;
     sK[t * DS + i] *= to_end;
     sW[t * DS + i] *= to_end;
-    if (t == CH - 1) so[4 * DP + i] = pow2(before + G);
+    if (t == CH - 1) so[4 * DP + i] = before * G;
   }
-  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) M[e] = X[e] = Qw[e] = Qk[e] = 0.f;
+  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) M[e] = X[e] = Qw[e] = 0.f;
   lds_barrier();
-  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) sG[e] = 0.f;
+  for (int e = tid; e < CH * MS; e += SOLVE_THREADS) sG[e] = Qk[e] = 0.f;
   lds_barrier();
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
@@ -545,12 +579,13 @@ chunk_solve_kernel(ChunkArgs a) {
   for (int dist = 1; dist < 4; ++dist) {
     if (wave + dist < 4) {
       const int x = wave + dist, y = wave;
-      f32x4 s = none, r = none;
+      f32x4 ps[4] = {none, none, none, none}, r = none;
       for (int c = y; c < x; ++c) {
         const f32x4 m = *reinterpret_cast<const f32x4*>(M + (16 * x + n) * MS + 16 * c + 4 * g);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s = mfma4(m[j], X[(16 * c + 4 * g + j) * MS + 16 * y + n], s);
+        for (int j = 0; j < 4; ++j) ps[j] = mfma4(m[j], X[(16 * c + 4 * g + j) * MS + 16 * y + n], ps[j]);
       }
+      const f32x4 s = meet(ps);
       // a result's rows 4 g + e are what the next product's operand wants as its rows 4 g + j
       const f32x4 xx = *reinterpret_cast<const f32x4*>(X + (16 * x + n) * MS + 16 * x + 4 * g);
 #pragma unroll
@@ -563,21 +598,27 @@ chunk_solve_kernel(ChunkArgs a) {
   // ---- the four matrices, a wave 16 columns: first W, R, P, then U, F, E
   auto lower = [&](const float* L, const f32x4 (&b)[4], f32x4 (&acc)[4], float sign) {      // acc += sign L b, L lower triangular
 #pragma unroll
-    for (int y = 0; y < 4; ++y)
+    for (int x = 0; x < 4; ++x) {
+      f32x4 p[4] = {none, none, none, none};
 #pragma unroll
-      for (int x = y; x < 4; ++x) {
+      for (int y = 0; y <= x; ++y) {
         const f32x4 m = *reinterpret_cast<const f32x4*>(L + (16 * x + n) * MS + 16 * y + 4 * g) * sign;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[x] = mfma4(m[j], b[y][j], acc[x]);
+        for (int j = 0; j < 4; ++j) p[j] = mfma4(m[j], b[y][j], p[j]);
       }
+      acc[x] += meet(p);
+    }
   };
   auto turned = [&](const float* T, const f32x4 (&b)[4], f32x4 (&acc)[CT], float sign) {    // acc += sign T^T b, T [64][DS]
 #pragma unroll
-    for (int y = 0; y < 4; ++y)
+    for (int x = 0; x < CT; ++x) {
+      f32x4 p[4] = {none, none, none, none};
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int y = 0; y < 4; ++y)
 #pragma unroll
-        for (int x = 0; x < CT; ++x) acc[x] = mfma4(sign * T[(16 * y + 4 * g + j) * DS + 16 * x + n], b[y][j], acc[x]);
+        for (int j = 0; j < 4; ++j) p[j] = mfma4(sign * T[(16 * y + 4 * g + j) * DS + 16 * x + n], b[y][j], p[j]);
+      acc[x] += meet(p);                 // (on top of the other sum, a chain would round at its size)
+    }
   };
   for (int ct = wave; ct < 2 * CT; ct += WAVES) {
     const bool of_v = ct >= CT;
@@ -608,16 +649,13 @@ chunk_solve_kernel(ChunkArgs a) {
           b[y][j] = sU[(16 * y + 4 * g + j) * DS + c];
           o[y][j] = sR[(16 * y + 4 * g + j) * DS + c];
         }
-#pragma unroll
-      for (int x = 0; x < CT; ++x)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[x][e] = 16 * x + 4 * g + e == c ? so[4 * DP + c] : 0.f;
     }
     lower(X, b, w, 1.f);                 // W or U
     lower(Qw, w, o, -1.f);
     turned(sW, w, st, -1.f);
     float* __restrict__ to = (of_v ? a.F : a.R) + unit * CH * DP + c;
     float* __restrict__ se = (of_v ? a.E : a.P) + unit * DP * DP + c;
+    const float diagonal = of_v ? 0.f : so[4 * DP + c];                  // P_end
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
@@ -625,7 +663,7 @@ chunk_solve_kernel(ChunkArgs a) {
 #pragma unroll
     for (int x = 0; x < CT; ++x)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) se[(size_t)(16 * x + 4 * g + e) * DP] = st[x][e];
+      for (int e = 0; e < 4; ++e) se[(size_t)(16 * x + 4 * g + e) * DP] = st[x][e] + (16 * x + 4 * g + e == c ? diagonal : 0.f);
   }
 }
 
@@ -666,17 +704,18 @@ chunk_fold_kernel(ChunkArgs a) {
       S0[(size_t)e * DP] = S[e];
     }
     lds_barrier();                       // (two buffers: the one written next was read before this barrier)
-    f32x4 acc[2] = {A.e, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[4] = {none, none, none, none};
     float right[KB][4];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) right[kb][j] = s[(16 * kb + 4 * g + j) * CS + n];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) acc[kb & 1] = mfma4(A.p[kb][j], right[kb][j], acc[kb & 1]);
-    S = acc[0] + acc[1];
+      for (int j = 0; j < 4; ++j) acc[j] = mfma4(A.p[kb][j], right[kb][j], acc[j]);
+    S = A.e + meet(acc);
     fetch(A, c + 2);
   };
   Ahead even, odd;
@@ -719,11 +758,15 @@ chunk_outputs_kernel(ChunkArgs a) {
   }
   __syncthreads();
 #pragma unroll
-  for (int kb = 0; kb < CT; ++kb)
+  for (int x = 0; x < CT; ++x) {
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    f32x4 p[4] = {none, none, none, none};
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int kb = 0; kb < CT; ++kb)
 #pragma unroll
-      for (int x = 0; x < CT; ++x) o[x] = mfma4(r[kb][j], sS[(16 * kb + 4 * g + j) * SS + 16 * x + n], o[x]);
+      for (int j = 0; j < 4; ++j) p[j] = mfma4(r[kb][j], sS[(16 * kb + 4 * g + j) * SS + 16 * x + n], p[j]);
+    o[x] += meet(p);
+  }
   float ss[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
