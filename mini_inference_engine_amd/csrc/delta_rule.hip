@@ -374,13 +374,35 @@ struct ChunkArgs {
   const float* norm_weight; float eps;
   float* state; const int* row_start; const int* slots; void* out;
   float *P, *E, *R, *F, *S0;       // [units * H][DP or 64][DP]; S0 [units * H][DP][DP]
-  int H, d, first_row, max_chunks, units;     // units: rows * max_chunks; the launch's rows begin at first_row
+  int H, d, first_row, rows, units;           // rows [first_row, first_row + rows), their chunks in `units` places
 };
+
+// Places for the chunks of `rows` rows of together `tokens` tokens.  The chunks of the rows' k-th begin at place
+// chunk_places(tokens before it, k): a row of n tokens is then ceil(n / 64) = chunk_places(n, 1) or more from the next one's,
+// without a sum over the rows' chunks, and what lies between is less than a place a row.  (As many places a row as the longest has
+// chunks were 2.1 GB a layer for a prompt of 1,000 tokens beside 100 portions of 10, 16 heads of 64; so 0.16 GB.)
+__host__ __device__ __forceinline__ int chunk_places(int tokens, int rows) { return (int)((tokens + (long)(CH - 1) * rows) / CH); }
+
+// Every wave looks for its place's row, 64 rows at a time: the last that begins at it or before
+__device__ __forceinline__ int row_of_place(const ChunkArgs& a, int place) {
+  if (a.rows == 1) return 0;           // (the prompt by itself need not wait for the loads below)
+  const int* __restrict__ start = a.row_start + a.first_row;
+  const int lane = threadIdx.x & 63, t0 = start[0];
+  int k = 0;
+  for (int base = 0; base < a.rows; base += 64) {
+    const int at = base + lane;
+    const int n = __popcll(__builtin_amdgcn_ballot_w64(at < a.rows && chunk_places(start[at < a.rows ? at : 0] - t0, at) <= place));
+    k += n;
+    if (n < 64) break;
+  }
+  return k - 1;
+}
 
 #define CHUNK_OF_ROW                                                                                                    \
   const int place = blockIdx.y + gridDim.y * blockIdx.z;                                                                \
   if (place >= a.units) return;                                                                                         \
-  const int rr = place / a.max_chunks, ci = place - rr * a.max_chunks, row = a.first_row + rr, h = blockIdx.x;          \
+  const int rr = row_of_place(a, place), row = a.first_row + rr, h = blockIdx.x;                                        \
+  const int ci = place - (rr ? chunk_places(a.row_start[row] - a.row_start[a.first_row], rr) : 0);                      \
   const int t0 = a.row_start[row] + ci * CH, t_end = a.row_start[row + 1];                                              \
   if (t0 >= t_end) return;                                                                                              \
   const int nt = t_end - t0 < CH ? t_end - t0 : CH;                                                                     \
@@ -678,6 +700,7 @@ chunk_fold_kernel(ChunkArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int d = a.d, tokens = a.row_start[row + 1] - a.row_start[row], chunks = (tokens + CH - 1) / CH;
   if (chunks <= 0) return;
+  const int place = rr ? chunk_places(a.row_start[row] - a.row_start[a.first_row], rr) : 0;
   float* __restrict__ st = a.state + ((size_t)a.slots[row] * a.H + h) * d * d;
   f32x4 S;
 #pragma unroll
@@ -687,7 +710,7 @@ chunk_fold_kernel(ChunkArgs a) {
   }
   struct Ahead { f32x4 p[KB], e; };      // what a chunk needs, asked for two chunks ahead
   auto fetch = [&](Ahead& A, int c) {
-    const size_t unit = ((size_t)rr * a.max_chunks + (c < chunks ? c : chunks - 1)) * a.H + h;
+    const size_t unit = (size_t)(place + (c < chunks ? c : chunks - 1)) * a.H + h;
     const float* __restrict__ P = a.P + unit * DP * DP + (size_t)(16 * wave + n) * DP + 4 * g;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) A.p[kb] = *reinterpret_cast<const f32x4*>(P + 16 * kb);
@@ -697,7 +720,7 @@ chunk_fold_kernel(ChunkArgs a) {
   };
   auto step = [&](Ahead& A, int c) {
     float* __restrict__ s = sS[c & 1];
-    float* __restrict__ S0 = a.S0 + (((size_t)rr * a.max_chunks + c) * a.H + h) * DP * DP + (size_t)(16 * wave + 4 * g) * DP + col;
+    float* __restrict__ S0 = a.S0 + ((size_t)(place + c) * a.H + h) * DP * DP + (size_t)(16 * wave + 4 * g) * DP + col;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       s[(16 * wave + 4 * g + e) * CS + n] = S[e];
@@ -822,26 +845,28 @@ static int chunks_launch(const ChunkArgs& a, int rows, int out_dtype, hipStream_
 MIE_EXPORT int mie_delta_rule_chunks_take(int d, int rank, float decay_scale) {
   return d >= 1 && d <= 64 && rank >= 16 && rank <= 64 && rank % 16 == 0 && decay_scale >= 0.f && decay_scale <= DELTA_SCALE_MAX;
 }
-// floats of scratch a (chunk, head) takes
+// places of the chunks of `rows` rows of together `tokens` tokens, and floats of scratch a (place, head) takes
+MIE_EXPORT int mie_delta_rule_places(int tokens, int rows) { return chunk_places(tokens, rows); }
 MIE_EXPORT int mie_delta_rule_unit_floats(int d) { const int DP = d <= 32 ? 32 : 64; return 2 * CH * DP + 3 * DP * DP; }
 
-// Rows [first_row, first_row + rows) in chunks of 64 tokens, at most max_chunks a row; scratch: rows * max_chunks * H *
-// mie_delta_rule_unit_floats(d) floats.
+// Rows [first_row, first_row + rows), of together `tokens` tokens, in chunks of 64 tokens; scratch: mie_delta_rule_places(tokens, rows)
+// * H * mie_delta_rule_unit_floats(d) floats.
 MIE_EXPORT int mie_delta_rule_chunks(const float* sums, long ld, int r_col, int k_col, int v_col, int g_col, int a_col, int w_col,
                                      const float* w_decay, int rank, const float* decay_bias, float decay_scale,
                                      const float* removal_bias, const float* norm_weight, float eps, float* state,
                                      const int* row_start, const int* slots, void* out, int out_dtype, int first_row, int rows,
-                                     int H, int d, int max_chunks, float* scratch, hipStream_t s) {
-  if (rows <= 0) return 0;
+                                     int H, int d, int tokens, float* scratch, hipStream_t s) {
+  if (rows <= 0 || tokens <= 0) return 0;
   if (H <= 0 || first_row < 0 || !mie_delta_rule_chunks_take(d, rank, decay_scale))
     MIE_FAIL("delta_rule: chunks of %d heads of %d, inner size %d, decays' scale %g", H, d, rank, (double)decay_scale);
-  if (rows > 65535 || H > 65535 || max_chunks < 1 || (long)rows * max_chunks > 2147483647L) MIE_FAIL("delta_rule: %d rows of %d chunks, %d heads are beyond the grid", rows, max_chunks, H);
+  if (rows > 65535 || H > 65535) MIE_FAIL("delta_rule: %d rows, %d heads are beyond the grid", rows, H);
   if (out_dtype != MIE_F32 && out_dtype != MIE_BF16) MIE_FAIL("delta_rule: out dtype code %d", out_dtype);
   if (!scratch || (((uintptr_t)scratch | (uintptr_t)w_decay) & 15)) MIE_FAIL("delta_rule: scratch and the decay's matrix must be 16-byte aligned");
   const int DP = d <= 32 ? 32 : 64;
-  const size_t units = (size_t)rows * max_chunks * H;
+  const int places = chunk_places(tokens, rows);
+  const size_t units = (size_t)places * H;
   ChunkArgs a{sums, ld, r_col, k_col, v_col, g_col, a_col, w_col, w_decay, rank, decay_bias, decay_scale, removal_bias, norm_weight,
-              eps, state, row_start, slots, out, nullptr, nullptr, nullptr, nullptr, nullptr, H, d, first_row, max_chunks, rows * max_chunks};
+              eps, state, row_start, slots, out, nullptr, nullptr, nullptr, nullptr, nullptr, H, d, first_row, rows, places};
   float* at = scratch;
   auto take = [&](size_t per) { float* q = at; at += units * per; return q; };
   a.P = take((size_t)DP * DP);

@@ -1323,12 +1323,12 @@ class HipBackend(KernelBackend):
                 and w_decay.data_ptr() % 16 == 0):
             # rows of many tokens, in chunks on the matrix cores; the single tokens that lead the step one by one, below
             whole = int(getattr(step, "num_decode_rows", 0) or 0)
-            chunks = -(-longest // 64)
-            scratch = torch.empty((rows - whole) * chunks * H * lib.mie_delta_rule_unit_floats(d), dtype=torch.float32, device=sums.device)
+            scratch = torch.empty(lib.mie_delta_rule_places(T - whole, rows - whole) * H * lib.mie_delta_rule_unit_floats(d),
+                                  dtype=torch.float32, device=sums.device)
             library.check(lib, lib.mie_delta_rule_chunks(
                 _ptr(sums), sums.stride(0), cols["r"], cols["k"], cols["v"], cols["g"], cols["a"], cols["w"], _ptr(w_decay), rank,
                 _ptr(decay_bias), float(decay_scale), _ptr(removal_bias), _ptr(norm_weight), float(eps), _ptr(state),
-                _ptr(step.row_start), _ptr(step.state_slots), _ptr(out), _code(out.dtype), whole, rows - whole, H, d, chunks,
+                _ptr(step.row_start), _ptr(step.state_slots), _ptr(out), _code(out.dtype), whole, rows - whole, H, d, T - whole,
                 _ptr(scratch), self._stream()))
             if not whole:
                 return out
@@ -1339,8 +1339,6 @@ class HipBackend(KernelBackend):
             chunk, chunks = self.DELTA_CHUNK, -(-longest // self.DELTA_CHUNK)
             scratch = torch.empty((3, step.num_rows * chunks * H, d, d), dtype=torch.float32, device=sums.device)
             summaries, starts = scratch[:2], scratch[2]
-        if whole:
-            chunk, chunks = 0, 0
         prep = torch.empty((tokens, 3 * n), dtype=torch.float32, device=sums.device)
         library.check(lib, lib.mie_delta_rule(
             _ptr(sums), sums.stride(0), cols["r"], cols["k"], cols["v"], cols["g"], cols["a"], cols["w"], _ptr(w_decay), rank,

@@ -82,6 +82,7 @@ register_kernel_module("attention_prep", {
 register_kernel_module("delta_rule", {
     "mie_delta_rule": [P, L, I, I, I, I, I, I, P, I, P, F, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P, P, P],
     "mie_delta_rule_chunks_take": [I, I, F],
+    "mie_delta_rule_places": [I, I],
     "mie_delta_rule_unit_floats": [I],
     "mie_delta_rule_chunks": [P, L, I, I, I, I, I, I, P, I, P, F, P, P, F, P, P, P, P, I, I, I, I, I, I, P, P],
 })

@@ -615,6 +615,37 @@ def test_delta_rule_in_chunks_on_the_matrix_cores(hip, H, d, rank, lens, scale):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[1, 1] + [3] * 63 + [700] + [2, 64, 5, 65, 63] * 2 + [129, 9], [700] + [2] * 60, [2] * 70 + [700]])
+def test_delta_rule_one_long_row_beside_many_short_ones(hip, lens):
+    """The chunks' scratch follows the step's tokens and rows, not rows times the longest row's chunks; results against 64 bits
+    wherever the long row stands among more rows than a wave looks through at once."""
+    ops, g = hip[torch.bfloat16], torch.Generator().manual_seed(len(lens))
+    H, d, rank, n = 2, 64, 16, 128
+    step = FakeStep(lens, list(range(len(lens), 0, -1)))
+    step.num_decode_rows = next(i for i, m in enumerate(lens) if m > 1)
+    T = step.num_tokens
+    cols = dict(r=0, k=n, v=2 * n, g=3 * n, a=4 * n, w=5 * n)
+    sums, w_decay = _rand((T, 5 * n + rank), torch.float32, g), _rand((n, rank), torch.float32, g, 1.5)
+    db, rb, nw = _rand((n,), torch.float32, g), _rand((n,), torch.float32, g), _rand((n,), torch.float32, g) + 1
+    state = _rand((len(lens) + 1, H, d, d), torch.float32, g, 0.5)
+    st_w = state.cpu().clone()
+    want = ref.ref_delta_rule(sums.cpu(), cols, H, d, w_decay.cpu(), db.cpu(), 0.6, rb.cpu(), nw.cpu(), 1e-5, st_w,
+                              step.host["row_start"], step.host["state_slots"], torch.float64)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    with counted(ops, "delta_rule", "mie_delta_rule_chunks") as calls:
+        got = ops.delta_rule(sums, cols, H, d, w_decay, db, 0.6, rb, nw, 1e-5, state, step)
+    assert len(calls) == 1
+    # 80 KB a chunk and head (two matrices of 64 x 64 and three of d x d floats), a chunk for every 64 tokens and one a row at most
+    most = (T // 64 + len(lens)) * H * 5 * 64 * 64 * 4 + got.numel() * 2 + 2 * 3 * n * 4
+    assert torch.cuda.max_memory_allocated() - before <= most + (8 << 20), "(and an allocator's block)"
+    close(got.double(), want, 1e-2, "delta rule")
+    close(state, st_w, 3e-5, "state")
+    assert torch.equal(state[0].cpu(), st_w[0]), "slots of no row are left alone"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("d,rank,weights,scale", [(64, 64, 1.5, 0.6065), (64, 64, 0.19, 1.0), (32, 16, 0.4, 0.6065), (48, 32, 1.5, 1.0)])
 def test_delta_rule_in_chunks_is_as_exact_as_token_by_token(hip, d, rank, weights, scale):
     """The float32 state that 512 tokens leave, computed in chunks by matrix products and token by token, against 64 bits: the
