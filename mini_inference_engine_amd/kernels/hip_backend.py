@@ -1801,14 +1801,14 @@ class HipBackend(KernelBackend):
 
     def _attention_f32(self, qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window) -> bool:
         """Plain causal (windowed) softmax attention of a float32 step on the 32-bit matrix unit (csrc/attention_f32.hip);
-        False where that does not take the operands, or a step does not say where its portions lie (the kernel of
-        attention.hip goes by tokens alone).  Head sizes, strides and alignment decide, never how many rows of how many tokens
+        False where that does not take the operands, or a step does not say where its portions lie or how far its contexts
+        reach (the kernel of attention.hip goes by tokens alone).  Head sizes, strides and alignment decide, never how many rows of how many tokens
         a step has: a request's tokens take the same arithmetic in every step of the engine."""
         T, window = qkv.shape[0], int(window or 0)
         single = step.num_decode_rows
         longest = int(getattr(step, "max_row_tokens", 0) or 0)
         if (D % 16 or D > 128 or page % 16 or qkv.stride(0) % 4 or any(t.data_ptr() % 16 for t in (qkv, k_cache, v_cache))
-                or Hkv * -(-(Hq // Hkv) // 16) > 65535 or single > 65535 or step.num_rows - single > 65535):
+                or Hkv * -(-(Hq // Hkv) // 16) > 65535 or single > 65535 or step.num_rows - single > 65535 or (single and step.max_context < 1)):
             return False
         if single < T and (longest < 1 or any(t is None or t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous()
                                               for t, n in ((step.row_start, step.num_rows + 1), (step.row_position, step.num_rows)))):

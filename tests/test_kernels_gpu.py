@@ -1194,12 +1194,12 @@ def test_attention_float32_matrix_unit(ops, geom, window):
 
 def test_attention_float32_of_a_step_that_does_not_describe_its_rows(ops):
     """What the float32 attention reads of a step beyond its tokens is only there to choose a faster kernel: without the longest
-    row's length, or with row arrays of another type, the result is the same."""
+    row's length or the largest context, or with row arrays of another type, the result is the same."""
     Hq, Hkv, D, page = 4, 2, 32, 16
     q, kc, vc, group, step = paged_setup([37, 64, 20], [1, 64, 5], Hq, Hkv, D, page, torch.float32, seed=2)
     expect = ref.ref_paged_attention(q, Hq, Hkv, D, kc, vc, group.block_tables, step.token_row, step.positions, 0.2, None, torch.float64)
     torch.full((70, Hq * D), float("nan"), device=DEV)          # what an unwritten result would be made of
-    for change in (dict(max_row_tokens=0), dict(row_start=step.row_start.long()), dict(row_position=None), dict(row_start=None)):
+    for change in (dict(max_row_tokens=0), dict(max_context=0), dict(row_start=step.row_start.long()), dict(row_position=None), dict(row_start=None)):
         out = ops[torch.float32].paged_attention(q, Hq, Hkv, D, kc, vc, group, SimpleNamespace(**{**vars(step), **change}), 0.2, None)
         torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
 
