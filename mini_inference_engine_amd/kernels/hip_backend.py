@@ -1799,6 +1799,10 @@ class HipBackend(KernelBackend):
                 library.check(lib, lib.mie_paged_attention(*args, self._stream()))
         return out
 
+    # What the results of single tokens' segments of 128 keys may take, bytes: rows beyond it wait for a launch of their own, which
+    # by then has hundreds of waves a compute unit (32 heads of 128 with contexts up to 8,192: 126 rows a launch)
+    F32_SEGMENT_BYTES = 128 << 20
+
     def _attention_f32(self, qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window) -> bool:
         """Plain causal (windowed) softmax attention of a float32 step on the 32-bit matrix unit (csrc/attention_f32.hip);
         False where that does not take the operands, or a step does not say where its portions lie or how far its contexts
@@ -1821,11 +1825,17 @@ class HipBackend(KernelBackend):
             if window:
                 splits = min(splits, (window - 1) // seg + 2)
             o_part = ml = None
+            at_once = single                    # as many rows a launch as their segments' results have room for
             if splits > 1:
-                o_part = torch.empty((single, Hq, splits, D), dtype=torch.float32, device=qkv.device)
-                ml = torch.empty((single, Hq, splits, 2), dtype=torch.float32, device=qkv.device)
-            library.check(lib, lib.mie_attention_f32_single(*caches, _ptr(step.token_row), _ptr(step.positions), single, Hq, Hkv, D,
-                                                            page, float(scale), window, splits, _ptr(o_part), _ptr(ml), self._stream()))
+                at_once = min(single, max(1, self.F32_SEGMENT_BYTES // (Hq * splits * (D + 2) * 4)))
+                o_part = torch.empty((at_once, Hq, splits, D), dtype=torch.float32, device=qkv.device)
+                ml = torch.empty((at_once, Hq, splits, 2), dtype=torch.float32, device=qkv.device)
+            for t in range(0, single, at_once):
+                q, o = qkv[t:], out[t:]
+                library.check(lib, lib.mie_attention_f32_single(
+                    _ptr(q), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(o), _ptr(bt), bt.shape[1], _ptr(step.token_row[t:]),
+                    _ptr(step.positions[t:]), min(at_once, single - t), Hq, Hkv, D, page, float(scale), window, splits,
+                    _ptr(o_part), _ptr(ml), self._stream()))
         if single < T:
             library.check(lib, lib.mie_attention_f32_portions(*caches, _ptr(step.row_start), _ptr(step.row_position), single,
                                                               step.num_rows, longest, Hq, Hkv, D, page, float(scale), window,

@@ -1204,6 +1204,26 @@ def test_attention_float32_of_a_step_that_does_not_describe_its_rows(ops):
         torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
 
 
+def test_attention_float32_single_tokens_in_bounded_memory(ops):
+    """Single tokens under a static bound on the context that makes their segments' results too many to lie side by side: the
+    same bits as under a tight bound, and no more memory than is set aside for them."""
+    Hq, Hkv, D, page, rows, bound = 32, 4, 64, 16, 37, 65536
+    o = ops[torch.float32]
+    q, kc, vc, group, step = paged_setup([(37 * r) % 700 + 1 for r in range(rows)], [1] * rows, Hq, Hkv, D, page, torch.float32, seed=4)
+    tight = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 0.125, None)
+    assert rows * Hq * (bound // 128) * (D + 2) * 4 > o.F32_SEGMENT_BYTES
+    bt = torch.nn.functional.pad(group.block_tables, (0, bound // page - group.block_tables.shape[1]))
+    wide = SimpleNamespace(block_tables=bt, max_blocks=bt.shape[1])
+    bounded = SimpleNamespace(**{**vars(step), "max_context": bound})
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    loose = o.paged_attention(q, Hq, Hkv, D, kc, vc, wide, bounded, 0.125, None)
+    assert torch.cuda.max_memory_allocated() - before <= o.F32_SEGMENT_BYTES + (4 << 20)
+    assert torch.equal(loose, tight)
+
+
 # 16 queries of a wave: 16, 2, 5 and 1 neighbouring tokens; a window whose first key lies inside a tile of 16 keys
 @pytest.mark.parametrize("window", [None, 21])
 @pytest.mark.parametrize("geom", [(4, 4, 64, 16), (32, 4, 64, 16), (3, 1, 32, 48), (32, 2, 16, 16)])
