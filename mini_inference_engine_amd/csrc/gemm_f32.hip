@@ -10,10 +10,10 @@
 // instruction takes them from 16-byte pieces: instruction j multiplies k = j, 4 + j, 8 + j, 12 + j.
 //
 // skinny_f32_kernel (M <= 16): the weights' bytes bound it.  A workgroup owns 16 rows of W; a wave streams a contiguous
-//   part of K through a ring of its own in the LDS, filled by loads that write the LDS directly (in the order lane
-//   4 r + b, row r, 16-byte block b: a quarter wave then reads 64 contiguous bytes of 4 rows, where the instruction's
-//   own order would touch 16 cache lines); segments meet in the LDS at the end.  Eight waves a workgroup (a deeper
-//   queue of loads a compute unit) while the tiles do not fill the compute units, four from there on.
+//   part of K through a ring of its own in the LDS, filled by loads that write the LDS directly: 8 rows of 32 k a load, lane
+//   8 r + b (whole cache lines, where the instruction's own order would touch 16 lines a quarter wave), block b of 16 bytes at
+//   8 r + (b ^ r % 8), so that the fragment reads spread over all banks; segments meet in the LDS at the end.  Eight waves a
+//   workgroup (a deeper queue of loads a compute unit) while the tiles do not fill the compute units, four from there on.
 // tile_f32_kernel (M > 16): the matrix unit bounds it.  BM x BN outputs a workgroup, two buffers of 32 k in the LDS, the
 //   next stage on its way to registers while one is multiplied; several waves a SIMD, since one alone waits out its reads
 //   of the LDS (128 x 128 on four waves: 44 to 60 TFLOP/s).  Few tiles: the grid is also cut over quarters or segments,
@@ -21,8 +21,8 @@
 //
 // Measured on MI355X against the vector-unit kernel gemm_nt_kernel (gemm.hip) with its 64 x 64 tiles walking all of K:
 // a step's products at 4 rows 47 -> 6.1 ms with the kernels beside them unchanged, and whole cache lines a load (half lines and
-// 16 rows of x before) took a whole step 2,057 -> 1,853 us; 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225 (105 TFLOP/s of the 157 that
-// the 32-bit matrix unit has).  Error against 64 bits of a 22-layer step's logits 2.5e-6 -> 2.1e-6.
+// 16 rows of x before) took a whole step 2,057 -> 1,853 us; 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225
+// (105 TFLOP/s of the 157 that the 32-bit matrix unit has).  Error against 64 bits of a 22-layer step's logits 2.5e-6 -> 2.1e-6.
 #include "common.hpp"
 #include <mutex>
 #include <set>
@@ -448,7 +448,7 @@ template <int EPI>
 static int launch_skinny(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int M, int N,
                          int K, hipStream_t s, const RopeArgs& rope = RopeArgs{}) {
   const int tiles = EPI == GF_SWIGLU ? (N + 7) / 8 : (N + 15) / 16;
-  // 8 waves, 144 KB of ring and one workgroup a compute unit, or 4 waves, 48 KB and three
+  // 8 waves, 144 KB of ring (128 from 9 rows on) and one workgroup a compute unit, or 4 waves, 48 KB and three
 #define GF_SKINNY(WAVES, SLOTS, XL)                                                                                       \
   {                                                                                                                       \
     auto kernel = skinny_f32_kernel<EPI, WAVES, SLOTS, XL>;                                                               \

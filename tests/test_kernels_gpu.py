@@ -15,6 +15,7 @@ import pytest
 import torch
 
 import torch_backend as ref
+from native_calls import counted
 
 pytestmark = pytest.mark.gpu
 
@@ -126,7 +127,9 @@ def test_linear_float32_matrix_unit(ops, shape):
     o = ops[torch.float32]
     torch.manual_seed(M + N)
     x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) / math.sqrt(K)
-    y = o.linear(x, w)
+    with counted(o, "gemm_f32", "mie_gemm_f32") as calls:
+        y = o.linear(x, w)
+    assert len(calls) == 1
     bound = (K / 16 + 32) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30
     assert bool(((y.double() - x.double() @ w.double().T).abs() <= bound).all())
     for a, b in ((0, 1), (M // 2, M // 2 + 1), (max(0, M - 17), M), (0, min(M, 16)), (0, M // 2 + 1)):
@@ -268,7 +271,9 @@ def test_tile_product_in_parts(engine_ops, shape):
     expect = stream.double() + x.double() @ w.double().T
     bound = (K + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -22 * expect.abs()
     plain = stream.clone()
-    assert o.linear(x, w, add_to=plain) is None
+    with counted(o, "tile_gemm_bf16", "mie_tile_gemm_units") as calls:
+        assert o.linear(x, w, add_to=plain) is None
+    assert len(calls) == 1
     assert bool(((plain.double() - expect).abs() <= bound).all())
     g = torch.randn(N, device=DEV).to(torch.bfloat16)
     normed = o.linear(x, w, add_to=Sink(stream, g, 1e-5))
@@ -300,11 +305,16 @@ def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
         torch.testing.assert_close(stream.double(), want, atol=1e-4, rtol=1e-4)
 
 
-@pytest.mark.parametrize("shape", [(129, 64, 104), (192, 2048, 5632), (300, 192, 96), (513, 128, 5640), (1300, 2048, 2816), (2047, 64, 1000)])
-def test_tile_product_swiglu(engine_ops, shape):
+# rows, K, columns; the rounds of the grid times a stage's time of the tile that is taken (128 x 128, 192 x 128, 256 x 128, 256 x 192
+# and 256 x 256 take 0.76, 0.98, 0.99, 1.33 and 1.57 us), and whether the product is better off on the own tiles
+@pytest.mark.parametrize("case", [(129, 64, 104, 0.76, True), (192, 2048, 5632, 0.76, True), (300, 192, 96, 0.76, True),
+                                  (380, 64, 5512, 0.98, True), (510, 128, 5512, 0.99, True), (513, 128, 5640, 1.33, True),
+                                  (1300, 2048, 2816, 1.33, False), (1020, 64, 6152, 1.57, True), (2047, 64, 1000, 0.76, True)])
+def test_tile_product_swiglu(engine_ops, case):
     """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
     sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
     from mini_inference_engine_amd.kernels import library
+    shape, stage_us, gains = case[:3], case[3], case[4]
     o, (M, K, inter) = engine_ops, shape
     torch.manual_seed(K + inter)
     x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
@@ -317,8 +327,13 @@ def test_tile_product_swiglu(engine_ops, shape):
     expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
     assert bool(((out[:, :inter].double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
     assert bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
-    if o._tile_swiglu_gains(x, w, inter):
-        assert torch.equal(o.linear_silu_mul(x, w, inter), out[:, :inter])
+    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 100 * stage_us * (K // 64)) <= 1, "the case must take the tile it is for"
+    assert o._tile_swiglu_gains(x, w, inter) == gains
+    with counted(o, "tile_gemm_bf16", "mie_tile_gemm_swiglu") as calls:
+        made = o.linear_silu_mul(x, w, inter)
+    assert len(calls) == gains
+    if gains:
+        assert torch.equal(made, out[:, :inter])
     assert lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K - 8, None) != 0
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
@@ -1177,7 +1192,9 @@ def test_attention_float32_matrix_unit(ops, geom, window):
     Hq, Hkv, D, page = geom
     o, n = ops[torch.float32], 389
     q, kc, vc, group, step = paged_setup([n, 131], [n, 131], Hq, Hkv, D, page, torch.float32, seed=D)
-    whole, expect = run_attention(ops, torch.float32, q, kc, vc, group, step, Hq, Hkv, D, 1 / math.sqrt(D), window)
+    with counted(o, "attention_f32", "mie_attention_f32_single", "mie_attention_f32_portions") as calls:
+        whole, expect = run_attention(ops, torch.float32, q, kc, vc, group, step, Hq, Hkv, D, 1 / math.sqrt(D), window)
+    assert calls == ["mie_attention_f32_portions"]
     torch.testing.assert_close(whole.double(), expect, **ATT_TOL[torch.float32])
     for a, b in ((0, 2), (2, 129), (129, 256), (256, n)):
         part = SimpleNamespace(token_row=step.token_row[a:b], positions=step.positions[a:b], num_rows=1, max_context=b, num_tokens=b - a,
@@ -1189,7 +1206,9 @@ def test_attention_float32_matrix_unit(ops, geom, window):
         wide.max_blocks = wide.block_tables.shape[1]
         single = SimpleNamespace(token_row=step.token_row, positions=step.positions, num_rows=2, max_context=bound, num_tokens=n + 131,
                                  num_decode_rows=n + 131, max_row_tokens=1, row_start=None, row_position=None)
-        assert torch.equal(o.paged_attention(q, Hq, Hkv, D, kc, vc, wide, single, 1 / math.sqrt(D), window), whole)
+        with counted(o, "attention_f32", "mie_attention_f32_single", "mie_attention_f32_portions") as calls:
+            out = o.paged_attention(q, Hq, Hkv, D, kc, vc, wide, single, 1 / math.sqrt(D), window)
+        assert calls == ["mie_attention_f32_single"] and torch.equal(out, whole)
 
 
 def test_attention_float32_of_a_step_that_does_not_describe_its_rows(ops):
