@@ -755,16 +755,65 @@ chunk_fold_kernel(ChunkArgs a) {
   }
 }
 
-// (3) a wave 16 tokens of a head: o = R S_0 + F, S_0 through the LDS; then the norm, the weight and the gate
+// A chunk's tokens one by one from S_0 (in the LDS, a stride of SS a row; used up), one wave, lane a channel and a column; vec: 5 DP.
+template <int DP, typename TO>
+__device__ __forceinline__ void chunk_one_by_one(const ChunkArgs& a, float* S, float* vec, int h, int t0, int nt) {
+  constexpr int SS = DP + 4;
+  const int lane = threadIdx.x & 63, d = a.d;
+  const bool live = lane < d;
+  const int c = h * d + (live ? lane : 0);
+  const float* __restrict__ wd = a.w_decay + (size_t)c * a.rank;
+#pragma unroll 1
+  for (int tt = 0; tt < nt; ++tt) {
+    const size_t t = t0 + tt;
+    const float* __restrict__ src = a.sums + t * a.ld;
+    const float k = live ? src[a.k_col + c] : 0.f, inner = lane < a.rank ? tanhf(src[a.w_col + lane]) : 0.f;
+    const float u = k / sqrtf(wave_sum(k * k) + 1e-6f);
+    float z = a.decay_bias[c];
+#pragma unroll 1
+    for (int j = 0; j < a.rank; ++j) z = fmaf(wd[j], __shfl(inner, j, 64), z);
+    if (live) {
+      vec[lane] = expf(-a.decay_scale * mie_sigmoid(z));
+      vec[DP + lane] = mie_sigmoid(src[a.a_col + c] + a.removal_bias[c]) * u;
+      vec[2 * DP + lane] = u;
+      vec[3 * DP + lane] = k;
+      vec[4 * DP + lane] = src[a.r_col + c];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // (one wave: what it wrote is there)
+    float o = 0.f;
+    if (live) {
+      const float v = src[a.v_col + c];
+      float seen = 0.f;
+#pragma unroll 1
+      for (int i = 0; i < d; ++i) seen = fmaf(vec[2 * DP + i], S[i * SS + lane], seen);
+#pragma unroll 1
+      for (int i = 0; i < d; ++i) {
+        const float x = fmaf(vec[3 * DP + i], v, fmaf(-vec[DP + i], seen, vec[i] * S[i * SS + lane]));
+        S[i * SS + lane] = x;
+        o = fmaf(x, vec[4 * DP + i], o);
+      }
+    }
+    const float rstd = 1.0f / sqrtf(wave_sum(o * o) / (float)d + a.eps);
+    if (live) ((TO*)a.out)[t * a.H * d + c] = from_float<TO>(o * rstd * a.norm_weight[c] * mie_sigmoid(src[a.g_col + c]));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
+// (3) a wave 16 tokens of a head: o = R S_0 + F, S_0 through the LDS; then the norm, the weight and the gate.  A product takes
+// 0 times what a later token of its 16 holds, and where that is not a number or infinite, 0 times it is not 0: a chunk with such a
+// result takes its tokens one by one, each from the state before it (the state behind such a token is no number either way).
 template <int DP, typename TO>
 __global__ void __launch_bounds__(256)
 chunk_outputs_kernel(ChunkArgs a) {
   constexpr int CT = DP / 16, SS = DP + 4;
   __shared__ __align__(16) float sS[DP * SS];
+  __shared__ float sVec[5 * DP];
+  __shared__ int sOdd;
   CHUNK_OF_ROW;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d = a.d;
+  if (tid == 0) sOdd = 0;
   const float* __restrict__ S0 = a.S0 + unit * DP * DP;
   const float* __restrict__ R = a.R + unit * CH * DP + (size_t)(16 * wave + n) * DP + 4 * g;
   const float* __restrict__ F = a.F + unit * CH * DP + (size_t)(16 * wave + 4 * g) * DP + n;
@@ -789,6 +838,17 @@ chunk_outputs_kernel(ChunkArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) p[j] = mfma4(r[kb][j], sS[(16 * kb + 4 * g + j) * SS + 16 * x + n], p[j]);
     o[x] += meet(p);
+  }
+  bool odd = false;
+#pragma unroll
+  for (int x = 0; x < CT; ++x)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) odd |= !(fabsf(o[x][e]) < INFINITY);     // (tokens and channels that are not there are zeros)
+  if (odd) sOdd = 1;
+  __syncthreads();
+  if (sOdd) {                            // the same for the whole workgroup
+    if (wave == 0) chunk_one_by_one<DP, TO>(a, sS, sVec, h, t0, nt);
+    return;
   }
   float ss[4];
 #pragma unroll

@@ -646,6 +646,42 @@ def test_delta_rule_one_long_row_beside_many_short_ones(hip, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("what", ["v", "k", "w", "r"])
+@pytest.mark.parametrize("H,d,rank", [(2, 64, 64), (3, 20, 16)])
+def test_delta_rule_in_chunks_keeps_later_tokens_out_of_earlier_ones(hip, H, d, rank, what):
+    """An infinite value, or a key, inner activation or query that is no number: the tokens before it, in its 16, its chunk and the
+    chunks before, and the row beside it get what they get without it; so do, behind a value, the state's other columns."""
+    ops, g = hip[torch.bfloat16], torch.Generator().manual_seed(d)
+    n, lens, at = H * d, [200, 70], 141
+    step = FakeStep(lens, [1, 2])
+    cols = dict(r=0, k=n, v=2 * n, g=3 * n, a=4 * n, w=5 * n)
+    sums, w_decay = _rand((270, 5 * n + rank), torch.float32, g), _rand((n, rank), torch.float32, g)
+    db, rb, nw = _rand((n,), torch.float32, g), _rand((n,), torch.float32, g), _rand((n,), torch.float32, g) + 1
+    start = _rand((3, H, d, d), torch.float32, g, 0.5)
+    st_w = start.cpu().clone()
+    want = ref.ref_delta_rule(sums.cpu(), cols, H, d, w_decay.cpu(), db.cpu(), 0.6, rb.cpu(), nw.cpu(), 1e-5, st_w,
+                              step.host["row_start"], step.host["state_slots"], torch.float64)
+    sums[at, cols[what] + 3] = float("inf") if what == "v" else float("nan")       # (of the first head)
+    state = start.clone()
+    with counted(ops, "delta_rule", "mie_delta_rule_chunks") as calls:
+        got = ops.delta_rule(sums, cols, H, d, w_decay, db, 0.6, rb, nw, 1e-5, state, step)
+    assert len(calls) == 1
+    close(got[:at].double(), want[:at], 1e-2, "tokens before")
+    close(got[200:].double(), want[200:], 1e-2, "the row beside")
+    assert not bool(torch.isfinite(got[at, :d].float()).all())
+    close(state[2], st_w[2], 3e-5, "the row beside's state")
+    if what != "w":
+        close(got[:200, d:].double(), want[:200, d:], 1e-2, "the other heads")
+    if what == "r":
+        close(got[at + 1:].double(), want[at + 1:], 1e-2, "tokens behind a query")
+        close(state, st_w, 3e-5, "state")
+    if what == "v":
+        others = [j for j in range(d) if j != 3]
+        close(state[1, 0][:, others], st_w[1, 0][:, others], 3e-5, "the state's other columns")
+        assert not bool(torch.isfinite(state[1, 0, :, 3]).any())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("d,rank,weights,scale", [(64, 64, 1.5, 0.6065), (64, 64, 0.19, 1.0), (32, 16, 0.4, 0.6065), (48, 32, 1.5, 1.0)])
 def test_delta_rule_in_chunks_is_as_exact_as_token_by_token(hip, d, rank, weights, scale):
     """The float32 state that 512 tokens leave, computed in chunks by matrix products and token by token, against 64 bits: the
