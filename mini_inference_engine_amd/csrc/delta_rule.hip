@@ -16,7 +16,7 @@
 // B (the recurrence on zero), a thread carrying the same column of both;  (2) per row and head, chunk after chunk, S_start(c + 1) = P_c S_start(c) + B_c from
 // state[slot] (16 columns a workgroup; columns do not mix);  (3) every chunk runs its tokens from its S_start and writes
 // the outputs, a row's last chunk leaves state[slot].  The two ways differ by the rounding of pass 2 alone.
-#include "common.hpp"
+#include "launch.hpp"
 
 constexpr int PT_MAX = 16;       // most tokens a workgroup of delta_prepare takes: a channel's row of the decay matrix is read once for all of them
 
@@ -882,14 +882,7 @@ MIE_EXPORT const char* delta_rule_last_error() { return g_mie_error; }
 template <int DP>
 static int chunks_launch(const ChunkArgs& a, int rows, int out_dtype, hipStream_t s) {
   const size_t lds = ((size_t)4 * CH * (DP + 4) + (size_t)5 * CH * MS + 5 * DP) * sizeof(float);
-  static bool allowed[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("delta_rule: no current device");
-  if (!allowed[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_solve_kernel<DP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) MIE_FAIL("delta_rule: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-    allowed[dev] = true;
-  }
+  if (mie_allow_lds(reinterpret_cast<const void*>(chunk_solve_kernel<DP>), (int)lds, "delta_rule")) return -1;
   const dim3 units(a.H, a.units < 32768 ? a.units : 32768, (a.units + 32767) / 32768);
   hipLaunchKernelGGL(chunk_solve_kernel<DP>, units, dim3(SOLVE_THREADS), lds, s, a);
   MIE_CHECK_LAUNCH("delta_rule (chunks: solve)");

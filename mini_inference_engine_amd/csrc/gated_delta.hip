@@ -20,7 +20,7 @@
 // No exponent is ever positive: within 16 tokens A and Q are taken pair by pair; for tokens s of an earlier 16 both factors are
 // taken against the sum R at the start of t's 16, e^(G_t - R) and e^(R - G_s), so that the product runs on the matrix cores.
 // The inverse is built from 16 x 16 blocks: the diagonal ones by substitution, X_ab = -X_aa sum_c M_ac X_cb below them.
-#include "common.hpp"
+#include "launch.hpp"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr float LOG2E = 1.4426950408889634f;
@@ -685,14 +685,7 @@ static int scan_launch(const DeltaArgs& a, int rows, hipStream_t s) {
 template <int DP, typename TO>
 static int chunks_launch(const ChunkArgs& p, int rows, hipStream_t s) {
   const size_t lds = ((size_t)3 * CH * (DP + 4) + (size_t)2 * CH * MS + CH + 4 * DP) * sizeof(float);
-  static bool allowed[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("gated_delta: no current device");
-  if (lds > 64 * 1024 && !allowed[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(chunk_solve_kernel<DP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) MIE_FAIL("gated_delta: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-    allowed[dev] = true;
-  }
+  if (lds > 64 * 1024 && mie_allow_lds(reinterpret_cast<const void*>(chunk_solve_kernel<DP>), (int)lds, "gated_delta")) return -1;
   const dim3 units(p.s.H, p.units < 32768 ? p.units : 32768, (p.units + 32767) / 32768);
   hipLaunchKernelGGL(chunk_solve_kernel<DP>, units, dim3(SOLVE_THREADS), lds, s, p);
   MIE_CHECK_LAUNCH("gated_delta (chunks: solve)");

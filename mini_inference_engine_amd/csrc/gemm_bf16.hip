@@ -30,19 +30,13 @@
 // The RMSNorm between two products is folded into them as well, see NormArgs below.  (A norm prologue that
 // converted the 32-bit stream inside every workgroup was measured and dropped: redoing the conversion of
 // all of x per workgroup cost more than a separate norm kernel.)
-#include "common.hpp"
-#include <mutex>
-#include <set>
-#include <utility>
+#include "launch.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // what a k-step beyond a wave's range or beyond K loads instead of weights, so that every load is unconditional
 __device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
-
-// wait until at most n vector memory loads of this wave are still on their way
-#define SG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 constexpr int SG_NONTEMPORAL = 2;  // the hint of loads whose lines nobody reads again: the weights
 
@@ -70,7 +64,7 @@ __device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1,
 // The wait of round `it` < SLOTS - 1 (the counter's limit must be a constant of the instruction).
 template <int SLOTS, int XL, int IT> struct RingStart {
   static __device__ __forceinline__ void wait(int it) {
-    if (it == IT) SG_VMCNT((SLOTS - 2 - IT) * XL + (IT + 1) * (2 + XL));
+    if (it == IT) MIE_VMCNT((SLOTS - 2 - IT) * XL + (IT + 1) * (2 + XL));
     else if constexpr (IT + 1 < SLOTS - 1) RingStart<SLOTS, XL, IT + 1>::wait(it);
   }
 };
@@ -250,7 +244,7 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     // Slot `it` has landed: all but the loads issued after its last one.  From round SLOTS - 1 on those are the
     // SLOTS - 1 slots after it; before, the x fragments of the first slots that follow its own and the slots
     // issued in the loop so far.  (Anything else asked for in between only makes this wait for more.)
-    if (it >= SLOTS - 1) SG_VMCNT((SLOTS - 1) * L);
+    if (it >= SLOTS - 1) MIE_VMCNT((SLOTS - 1) * L);
     else RingStart<SLOTS, XL, 0>::wait(it);
     sg_u32x4 f[2 * RING_U];
     const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
@@ -260,7 +254,7 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f[2 * u]), __builtin_bit_cast(bf16x8, f[2 * u + 1]),
                                                     acc, 0, 0, 0);
   }
-  SG_VMCNT(0);                                     // nothing of this wave may still be writing the LDS when it ends
+  MIE_VMCNT(0);                                     // nothing of this wave may still be writing the LDS when it ends
 
   if (NF && EPI != EPI_ADD) {
     // 1 / sqrt(mean of squares + eps) of every row, summed in a fixed order
@@ -346,18 +340,6 @@ MIE_EXPORT const char* gemm_bf16_last_error() { return g_mie_error; }
 MIE_EXPORT int mie_skinny_max_rows() { return 16; }
 
 // A kernel that wants more LDS than a launch gets by default is told so once per device.
-static int allow_lds(const void* kernel, int bytes) {
-  static std::mutex lock;
-  static std::set<std::pair<int, const void*>> done;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) MIE_FAIL("skinny_gemm: no current device");
-  std::lock_guard<std::mutex> g(lock);
-  if (done.count({dev, kernel})) return 0;
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) MIE_FAIL("skinny_gemm: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-  done.insert({dev, kernel});
-  return 0;
-}
 
 template <bool NF, int SLOTS, int XL>
 static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
@@ -365,8 +347,8 @@ static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx
   constexpr int lds = SG_WAVES * SLOTS * (2 + XL) * 1024;
 #define SG_LAUNCH(E)                                                                                                    \
   {                                                                                                                     \
-    auto kernel = skinny_gemm_kernel<E, NF, SLOTS, XL>;                                                                     \
-    if (allow_lds((const void*)kernel, lds)) return -1;                                                                 \
+    auto kernel = skinny_gemm_kernel<E, NF, SLOTS, XL>;                                                                 \
+    if (mie_allow_lds((const void*)kernel, lds, "skinny_gemm")) return -1;                                              \
     hipLaunchKernelGGL(kernel, grid, dim3(SG_THREADS), lds, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, nf); \
   }
   switch (epi) {
@@ -387,18 +369,8 @@ static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx
 // Slots a wave's ring has.  Four (64 KB a workgroup, two workgroups a compute unit; five of 60 KB for up to 8 rows) stream
 // best; three (48 KB, three workgroups a compute unit; four of 48 KB for up to 8 rows) when that lets all tiles run at once instead of in two rounds.  Chosen from
 // the weight's shape alone, never from the batch (the sums do not depend on it anyway).
-static int compute_units() {
-  static int units[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!units[dev]) {
-    int n = 0;
-    units[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-  }
-  return units[dev];
-}
 static int slots_for(int tiles) {
-  const int cu = compute_units();
+  const int cu = mie_compute_units();
   return tiles > 2 * cu && tiles <= 3 * cu ? 3 : 4;
 }
 

@@ -23,17 +23,12 @@
 // a step's products at 4 rows 47 -> 6.1 ms with the kernels beside them unchanged, and whole cache lines a load (half lines and
 // 16 rows of x before) took a whole step 2,057 -> 1,853 us; 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225
 // (105 TFLOP/s of the 157 that the 32-bit matrix unit has).  Error against 64 bits of a 22-layer step's logits 2.5e-6 -> 2.1e-6.
-#include "common.hpp"
-#include <mutex>
-#include <set>
-#include <utility>
+#include "launch.hpp"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
-
-#define GF_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 // The cut of K, in steps of 16: quarter q is steps [q * quarter, min((q + 1) * quarter, steps)), a segment `segment` steps.
 struct KCut {
@@ -156,7 +151,7 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
   const int rounds = ks1 > ks0 ? (ks1 - ks0 + GF_U - 1) / GF_U : 0;
   for (int it = 0; it < rounds; ++it) {
     issue(it + SLOTS - 1);                    // into the slot that was read a round ago
-    GF_VMCNT((SLOTS - 1) * L);                // slot `it` has landed
+    MIE_VMCNT((SLOTS - 1) * L);                // slot `it` has landed
     u32x4 f[2 * GF_U];
     const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
     ring_read(w0 + blk0, x0 + blk0, w0 + blk1, x0 + blk1, f);
@@ -170,7 +165,7 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
           acc[i] = step_mfma(w4, x4, acc[i]);
     }
   }
-  GF_VMCNT(0);                                // nothing of this wave is writing the LDS any more
+  MIE_VMCNT(0);                                // nothing of this wave is writing the LDS any more
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < SPW; ++i) *reinterpret_cast<f32x4*>(s_acc + (wave * SPW + i) * 256 + lane * 4) = acc[i];
@@ -404,19 +399,6 @@ reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long 
 // ------------------------------------------------------------------------------------------------ host
 MIE_EXPORT const char* gemm_f32_last_error() { return g_mie_error; }
 
-static int allow_lds(const void* kernel, int bytes) {
-  static std::mutex lock;
-  static std::set<std::pair<int, const void*>> done;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) MIE_FAIL("gemm_f32: no current device");
-  std::lock_guard<std::mutex> g(lock);
-  if (done.count({dev, kernel})) return 0;
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) MIE_FAIL("gemm_f32: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-  done.insert({dev, kernel});
-  return 0;
-}
-
 static int check_operands(const char* what, const void* X, long ldx, const void* W, long ldw, const void* out, long ldo, int N, int K) {
   if (K <= 0 || (K & 3) || (N & 3)) MIE_FAIL("%s: K = %d and N = %d must be positive multiples of 4", what, K, N);
   if (ldx < K || ldw < K || ldo < N || (ldx & 3) || (ldw & 3) || (ldo & 3)) MIE_FAIL("%s: leading dims %ld, %ld, %ld for K %d, N %d", what, ldx, ldw, ldo, K, N);
@@ -453,7 +435,7 @@ static int launch_skinny(const float* X, long ldx, const float* W, long ldw, flo
   {                                                                                                                       \
     auto kernel = skinny_f32_kernel<EPI, WAVES, SLOTS, XL>;                                                               \
     constexpr int lds = WAVES * SLOTS * (2 + XL) * 1024;                                                                  \
-    if (allow_lds((const void*)kernel, lds)) return -1;                                                                   \
+    if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;                                                   \
     hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, M, N, K, N, rope);  \
   }
   if (tiles <= 256) {
@@ -472,7 +454,7 @@ static int launch_tile(const float* X, long ldx, const float* W, long ldw, float
   constexpr int lds = 2 * (BM + BN) * 128;
   auto kernel = tile_f32_kernel<BM, BN, WR, WC, LEVELS>;
   if ((M + BM - 1) / BM > 65535) MIE_FAIL("gemm_f32: M = %d is beyond the grid", M);
-  if (allow_lds((const void*)kernel, lds)) return -1;
+  if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;
   hipLaunchKernelGGL(kernel, dim3((N + BN - 1) / BN, (M + BM - 1) / BM, units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, add, M, N, K);
   MIE_CHECK_LAUNCH("tile_f32");
   return 0;

@@ -21,7 +21,7 @@
 //   reduce_rows:     store (bfloat16 / float32), or add into the 32-bit stream, or add and RMSNorm for
 //                    the norm that reads the stream next (one workgroup a row, as the norm kernel);
 //   reduce_rope_kv:  the q/k/v projection: rotary on q and k, q out, k and v into their cache slots.
-#include "common.hpp"
+#include "launch.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -36,9 +36,6 @@ constexpr int MID_WAVES = 4;      // waves a workgroup = 16-row weight tiles a w
 constexpr int MID_KC = 2;         // k-steps (of 32) a stage
 constexpr int MID_STAGES = 4;     // stages in the ring (eight were measured: no faster)
 constexpr int FRAG_BYTES = 1024;  // one operand fragment: 64 lanes x 16 bytes
-
-// wait until at most n vector memory loads of this wave are still on their way
-#define MID_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 // The fragments of one k-step out of the LDS: the wave's weight fragment (at wbase) and the x fragments of all
 // row tiles (1 KB apart from xbase), read and waited for in one piece of assembly.  The compiler knows nothing
@@ -160,13 +157,13 @@ mid_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W
   // stages beyond the split's range load zeros only, so the ring is always filled and drained the same way
   for (int s = 0; s < MID_STAGES - 1; ++s) issue(s);
   for (int it = 0; it < nst; ++it) {
-    MID_VMCNT((MID_STAGES - 2) * L);           // this wave's loads of stage `it` have landed
+    MIE_VMCNT((MID_STAGES - 2) * L);           // this wave's loads of stage `it` have landed
     __builtin_amdgcn_s_barrier();              // and everybody else's; everybody is done reading stage it - 1
     issue(it + MID_STAGES - 1);                // into the buffer stage it - 1 used
     const uint32_t base = lds0 + (it % MID_STAGES) * STAGE_BYTES + rslot * 16;
     StageReader<MT, 0>::run(base, base + wave * FRAG_BYTES, acc);
   }
-  MID_VMCNT(0);                                // nothing of this wave may still be writing the LDS when it ends
+  MIE_VMCNT(0);                                // nothing of this wave may still be writing the LDS when it ends
   float* out = part + (size_t)blockIdx.y * M * N;
   // acc[mt][i]: x row mt * 16 + 4 kb + i (the A operand's rows), weight row n (the B operand's column)
 #pragma unroll

@@ -11,7 +11,7 @@
 //
 // route_topk, moe_align, moe_combine: choose a token's experts and their shares, sort (token, choice) pairs by
 // expert, and add a token's expert outputs back together in the order of its choices.
-#include "common.hpp"
+#include "launch.hpp"
 
 #define GG_T 64
 #define GG_K 16
@@ -175,7 +175,6 @@ union GGFrag {
 // Every output is the same chain of matrix instructions in increasing k wherever its tile lies, so a row's result
 // does not depend on the rows beside it.  K, the row strides and the group offsets are multiples of 8 and the
 // operands 16-byte aligned (checked by the caller).
-#define GG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 typedef uint32_t gg_u32x4 __attribute__((ext_vector_type(4)));
 
 template <int N> struct GGRead;
@@ -277,7 +276,7 @@ grouped_gemm_ring_kernel(GroupedArgs p) {
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s) issue(s);
   for (int it = 0; it < nk; ++it) {
-    GG_VMCNT(LPW * (STAGES - 2));      // this wave's loads of stage `it` have landed
+    MIE_VMCNT(LPW * (STAGES - 2));      // this wave's loads of stage `it` have landed
     __builtin_amdgcn_s_barrier();      // and everybody else's; everybody is done reading stage it - 1
     issue(it + STAGES - 1);            // into the buffer stage it - 1 used (zeros beyond K)
     const uint32_t base = lds0 + (it % STAGES) * STAGE_BYTES;
@@ -294,7 +293,7 @@ grouped_gemm_ring_kernel(GroupedArgs p) {
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[i][j], 0, 0, 0);
       }
   }
-  GG_VMCNT(0);                         // nothing of this wave may still be writing the LDS when it ends
+  MIE_VMCNT(0);                         // nothing of this wave may still be writing the LDS when it ends
   const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
   TC* C = (TC*)p.C + (size_t)g * p.c_group;
   if (p.glu) {

@@ -13,20 +13,15 @@
 // tried (the library's kernels move 11); reading the next fragments while one set is multiplied, across the barrier too,
 // changed nothing.  So what counts is bytes a workgroup brings in, and that every compute unit has one: TILE_STAGE_US, the
 // time of a stage of each tile, times the rounds of its grid picks the tile.
-#include "common.hpp"
-#include <mutex>
-#include <set>
-#include <utility>
+#include "launch.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define TG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
-
 enum { TG_F32, TG_SWIGLU };
 
 // 16 bytes a lane from base + offset into the LDS at byte `at` + 16 lane.  The compiler does not see that memory is on its
-// way: the waits are the kernel's own (TG_VMCNT and a barrier before a stage is read).  m0 is an output, so that the
+// way: the waits are the kernel's own (MIE_VMCNT and a barrier before a stage is read).  m0 is an output, so that the
 // compiler keeps nothing of its own there; as an input operand it costs the loop its order of moves and loads (2,048 rows of
 // [11264, 2048] 90.1 -> 93.0 us).
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t at) {
@@ -113,8 +108,8 @@ tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < nst) issue(s);
   for (int it = 0; it < nst; ++it) {
-    if (it + STAGES - 1 <= nst) TG_VMCNT((STAGES - 2) * L);      // this wave's loads of stage `it` have landed
-    else TG_VMCNT(0);
+    if (it + STAGES - 1 <= nst) MIE_VMCNT((STAGES - 2) * L);      // this wave's loads of stage `it` have landed
+    else MIE_VMCNT(0);
     __builtin_amdgcn_s_barrier();                                // and everybody else's; everybody is done with stage it - 1
     asm volatile("" ::: "memory");
     if (it + STAGES - 1 < nst) issue(it + STAGES - 1);
@@ -166,26 +161,13 @@ tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
 
 MIE_EXPORT const char* tile_gemm_bf16_last_error() { return g_mie_error; }
 
-static int allow_lds(const void* kernel, int bytes) {
-  static std::mutex lock;
-  static std::set<std::pair<int, const void*>> done;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) MIE_FAIL("tile_gemm: no current device");
-  std::lock_guard<std::mutex> g(lock);
-  if (done.count({dev, kernel})) return 0;
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) MIE_FAIL("tile_gemm: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-  done.insert({dev, kernel});
-  return 0;
-}
-
 template <int WR, int WC, int STAGES, int EPI>
 static int launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, long ldo, int M, int N, int K, int units, hipStream_t s) {
   constexpr int BM = WR * 64, BN = WC * 64, cols = EPI == TG_SWIGLU ? BN / 2 : BN;
   constexpr int lds = STAGES * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "LDS");
   auto kernel = tile_gemm_kernel<WR, WC, STAGES, EPI>;
-  if (allow_lds((const void*)kernel, lds)) return -1;
+  if (mie_allow_lds((const void*)kernel, lds, "tile_gemm")) return -1;
   const int mt = (M + BM - 1) / BM, nt = (N + cols - 1) / cols, stages = K / 64, per = (stages + units - 1) / units;
   if ((long)mt * nt * units > 0x7FFFFFFF) MIE_FAIL("tile_gemm: %d x %d tiles are beyond the grid", mt, nt);
   hipLaunchKernelGGL(kernel, dim3(mt * nt * units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, M, N, stages, per,
@@ -202,16 +184,6 @@ static int check_operands(const void* X, long ldx, const void* W, long ldw, cons
   return 0;
 }
 
-static int compute_units() {
-  static int units[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!units[dev]) {
-    int n = 0;
-    units[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-  }
-  return units[dev];
-}
 
 // Time of a stage (64 k) of a grid that gives every compute unit one workgroup, us: measured at 160 to 2,048 rows of
 // [11264, 2048] (MI355X).
@@ -223,7 +195,7 @@ static int best_tile(int M, long cols, float& us) {
   us = 1e30f;
   for (int i = 0; i < 5; ++i) {
     const long tiles = (long)((M + TILE_STAGE_US[i].bm - 1) / TILE_STAGE_US[i].bm) * ((cols + TILE_STAGE_US[i].bn - 1) / TILE_STAGE_US[i].bn);
-    const long rounds = (tiles + compute_units() - 1) / compute_units();
+    const long rounds = (tiles + mie_compute_units() - 1) / mie_compute_units();
     if (rounds * TILE_STAGE_US[i].us < us) {
       us = rounds * TILE_STAGE_US[i].us;
       best = i;
@@ -264,6 +236,6 @@ MIE_EXPORT int mie_tile_gemm_units(const void* X, long ldx, const void* W, long 
   const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
   // a workgroup a compute unit and a deep ring, or two and a short one
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * units;
-  return tiles <= compute_units() ? launch<2, 2, 4, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s)
+  return tiles <= mie_compute_units() ? launch<2, 2, 4, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s)
                                   : launch<2, 2, 2, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s);
 }
