@@ -346,7 +346,7 @@ delta_fold_kernel(const float* __restrict__ summaries, float* __restrict__ start
 // a third more exact with other weights (heads of 32, scale 4: 4.4 against 6.2), so they take what lies there.
 // What bounds it: the solve's chain of small products (about 440 matrix instructions a SIMD and chunk) and its 32-bit arithmetic,
 // a workgroup a compute unit.  2,048 tokens of 16 heads of 64 (MI355X): 40 + 168 + 142 + 175 us (preparation, summaries, fold,
-// chunks, token by token through the LDS) -> 73 + 27 + 17 us.  The token-by-token chunks stay for heads of 65 to 128, other inner
+// chunks, token by token through the LDS) -> 73 + 31 + 18 us.  The token-by-token chunks stay for heads of 65 to 128, other inner
 // sizes and stronger decays.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int CH = 64, MS = CH + 4;
