@@ -1,59 +1,120 @@
-// Matrix products of the float32 path on the 32-bit matrix instruction.
+// Matrix products of the float32 path on the bfloat16 matrix instruction, every operand in three parts.
 //
 //   y[m, n] = sum_k x[m, k] W[n, k]          x [M, K], W [N, K], y [M, N] float32
 //
+// A 32-bit number is the sum of three bfloat16 ones to its last bit or the one before (24 bits of mantissa in three pieces of
+// 8, the signs take up the roundings): v = h + m + l, h = bf16(v), m = bf16(v - h), l = bf16(v - h - m).  Of the nine
+// products six are taken, hh, hm, mh, mm, hl, lh; the three left out are below 2^-25 of |x w|.  A product of two bfloat16 numbers
+// is exact in 32 bits, so what rounds is the sums, and those of the five small products run in a chain of their own, where a
+// rounding is 2^-8 of one in the sums of hh.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles of a SIMD for what eight
+// v_mfma_f32_16x16x4_f32 (true 32-bit products) need 256 for.
+//
 // One order of summation for every kernel here, whatever M is, so that a row's result is bit-identical however the
-// batch around it is cut.  K is taken in steps of 16 (four v_mfma_f32_16x16x4_f32: the matrix unit adds true 32-bit
-// products); the steps are cut into four quarters and every quarter into four segments (sizes from K alone).  A
-// segment is one chain of matrix instructions, a quarter is ((s0 + s1) + s2) + s3 and the result ((q0 + q1) + q2) + q3:
-// the rounding error of a long sum grows with K / 16 + 16 terms.  Inside a step the sixteen k are taken as the
-// instruction takes them from 16-byte pieces: instruction j multiplies k = j, 4 + j, 8 + j, 12 + j.
+// batch around it is cut.  K is taken in steps of 32; the steps are cut into four quarters and every quarter into two
+// eighths (sizes from K alone).  An eighth is one chain of steps for hh and one for the small products and ends as their sum, a
+// quarter is e0 + e1 and the result ((q0 + q1) + q2) + q3.
+//
+// Numbers that bfloat16 cannot hold (infinities, and what rounds to one: 3.396e38 and above) have no such parts: their eighths
+// come out as NaN.  Every result that is one is computed again by 32-bit multiplications and additions (plain_unit): what is an
+// infinity stays one, and what is a NaN ends that at its first.  (Only there, where a finite number of 3.396e38 or more gives a
+// finite result, can the cut of the batch show in a last bit: a unit of K is computed again as a whole.)
 //
 // skinny_f32_kernel (M <= 16): the weights' bytes bound it.  A workgroup owns 16 rows of W; a wave streams a contiguous
 //   part of K through a ring of its own in the LDS, filled by loads that write the LDS directly: 8 rows of 32 k a load, lane
 //   8 r + b (whole cache lines, where the instruction's own order would touch 16 lines a quarter wave), block b of 16 bytes at
-//   8 r + (b ^ r % 8), so that the fragment reads spread over all banks; segments meet in the LDS at the end.  Eight waves a
+//   8 r + (b ^ r % 8), so that the fragment reads spread over all banks; parts of K meet in the LDS at the end.  Eight waves a
 //   workgroup (a deeper queue of loads a compute unit) while the tiles do not fill the compute units, four from there on.
-// tile_f32_kernel (M > 16): the matrix unit bounds it.  BM x BN outputs a workgroup, two buffers of 32 k in the LDS, the
-//   next stage on its way to registers while one is multiplied; several waves a SIMD, since one alone waits out its reads
-//   of the LDS (128 x 128 on four waves: 44 to 60 TFLOP/s).  Few tiles: the grid is also cut over quarters or segments,
-//   whose sums go to memory and meet in reduce_f32_kernel.
+// tile_f32_kernel (M > 16): the matrix unit bounds it.  BM x BN outputs a workgroup; a stage of 32 k comes into registers,
+//   is split there once for all waves, and goes into the LDS as three planes of bfloat16 (two buffers), while the stage
+//   before is multiplied.  Few tiles: the grid is also cut over quarters or eighths, whose sums go to memory and meet in
+//   reduce_f32_kernel.
 //
-// Measured on MI355X against the vector-unit kernel gemm_nt_kernel (gemm.hip) with its 64 x 64 tiles walking all of K:
-// a step's products at 4 rows 47 -> 6.1 ms with the kernels beside them unchanged, and whole cache lines a load (half lines and
-// 16 rows of x before) took a whole step 2,057 -> 1,853 us; 512 rows of [2048, 2048] 330 -> 50 us, of [11264, 2048] 475 -> 225
-// (105 TFLOP/s of the 157 that the 32-bit matrix unit has).  Error against 64 bits of a 22-layer step's logits 2.5e-6 -> 2.1e-6.
+// Measured on MI355X against the same kernels on v_mfma_f32_16x16x4_f32 (us; before / now): 512 rows of [11264, 2048] with SwiGLU
+// 237 / 175, [2048, 5632] 116 / 73, [2048, 2048] 51 / 35; 100 rows 69 / 59, 36 / 29, 21 / 16; 4 rows 21.9 / 19.2, 17.0 / 14.8, 8.8 / 8.3.
+// Steps of the engine, 22 layers of width 2,048: a prompt of 512 tokens 11,617 / 8,291, 4 rows 1,699 / 1,616.  Relative error of
+// [2048, 2048] against 64 bits 2.1e-7 / 1.0e-7, of [2048, 5632] 3.4e-7 / 1.6e-7, of a whole step's logits 2.1e-6 / 1.3e-6 (with the small
+// products in the chain of hh it would be 2.4e-7 and 4.1e-7).  What is left in the tile kernel: matrix instructions alone take 63 us
+// for 2,048 rows of [2048, 2048] (the clock falls with every compute unit at them), the fragment reads add 15, splitting 17.
 #include "launch.hpp"
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
 
-// The cut of K, in steps of 16: quarter q is steps [q * quarter, min((q + 1) * quarter, steps)), a segment `segment` steps.
+// The cut of K, in steps of 32: quarter q is steps [q * quarter, min((q + 1) * quarter, steps)), an eighth `eighth` steps.
 struct KCut {
-  int steps, quarter, segment;
+  int steps, quarter, eighth;
 };
 __host__ __device__ __forceinline__ KCut k_cut(int K) {
   KCut c;
-  c.steps = (K + 15) / 16;
+  c.steps = (K + 31) / 32;
   c.quarter = (c.steps + 3) / 4;
-  c.segment = (c.quarter + 3) / 4;
+  c.eighth = (c.quarter + 1) / 2;
   return c;
 }
 __host__ __device__ __forceinline__ int least(int a, int b) { return a < b ? a : b; }
 
-// steps [begin, end) of segment s (0 .. 15); may be empty
-__host__ __device__ __forceinline__ void segment_range(const KCut& c, int s, int& begin, int& end) {
-  const int q0 = least((s >> 2) * c.quarter, c.steps), q1 = least(q0 + c.quarter, c.steps);
-  begin = least(q0 + (s & 3) * c.segment, q1);
-  end = least(begin + c.segment, q1);
+// steps [begin, end) of eighth e (0 .. 7); may be empty
+__host__ __device__ __forceinline__ void eighth_range(const KCut& c, int e, int& begin, int& end) {
+  const int q0 = least((e >> 1) * c.quarter, c.steps), q1 = least(q0 + c.quarter, c.steps);
+  begin = least(q0 + (e & 1) * c.eighth, q1);
+  end = least(begin + c.eighth, q1);
 }
 
-__device__ __forceinline__ f32x4 step_mfma(const f32x4& w, const f32x4& x, f32x4 acc) {
+// two numbers as bfloat16, the first in the low half
+__device__ __forceinline__ uint32_t round2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+// h, m, l of two numbers
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = round2(a, b);
+  a -= __uint_as_float(h << 16);
+  b -= __uint_as_float(h & 0xFFFF0000u);
+  m = round2(a, b);
+  a -= __uint_as_float(m << 16);
+  b -= __uint_as_float(m & 0xFFFF0000u);
+  l = round2(a, b);
+}
+
+struct Parts {
+  bf16x8 h, m, l;
+};
+__device__ __forceinline__ Parts split8(const f32x4& a, const f32x4& b) {
+  u32x4 h, m, l;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], acc, 0, 0, 0);
-  return acc;
+  for (int i = 0; i < 4; ++i) {
+    const float p = i < 2 ? a[2 * i] : b[2 * i - 4], q = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    uint32_t hh, mm, ll;
+    split2(p, q, hh, mm, ll);
+    h[i] = hh, m[i] = mm, l[i] = ll;
+  }
+  return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+
+// The eighths [e0, e0 + n) of one result, n 1, 2 or 8, by 32-bit multiplications and additions, joined in the order of all
+// kernels here; a NaN, which stays one, ends it.
+__device__ __forceinline__ float plain_unit(const float* x, const float* w, int K, const KCut& cut, int e0, int n) {
+  float total = 0.f, quarter = 0.f;
+  for (int e = e0; e < e0 + n; ++e) {
+    int k0, k1;
+    eighth_range(cut, e, k0, k1);
+    k1 = least(k1 * 32, K);
+    float s = 0.f;
+    for (int k = k0 * 32; k < k1; ++k) {
+      s = fmaf(x[k], w[k], s);
+      if (s != s) return s;
+    }
+    quarter += s;
+    if (e & 1 || n == 1) {
+      total += quarter;
+      quarter = 0.f;
+    }
+  }
+  return total;
 }
 
 enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2, GF_ROPE = 3 };
@@ -69,11 +130,10 @@ struct RopeArgs {
 
 // ------------------------------------------------------------------------------------------------ few rows
 constexpr int GF_NONTEMPORAL = 2;             // the hint of loads whose lines nobody reads again: the weights
-constexpr int GF_U = 2;                       // steps a slot of a wave's ring
 
-// The fragments of a slot out of the LDS, read and waited for in one piece of assembly: the compiler knows nothing of the
-// loads that write the LDS and would wait for all of them at a read it could see.
-__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1, uint32_t x1, u32x4 (&f)[4]) {
+// Fragments out of the LDS, read and waited for in one piece of assembly: the compiler knows nothing of the loads that
+// write the LDS and would wait for all of them at a read it could see.
+__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t w1, uint32_t x0, uint32_t x1, u32x4 (&f)[4]) {
   asm volatile(
     "ds_read_b128 %0, %4\n\t"
     "ds_read_b128 %1, %5\n\t"
@@ -81,55 +141,79 @@ __device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1,
     "ds_read_b128 %3, %7\n\t"
     "s_waitcnt lgkmcnt(0)"
     : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
-    : "v"(w0), "v"(x0), "v"(w1), "v"(x1)
+    : "v"(w0), "v"(w1), "v"(x0), "v"(x1)
     : "memory");
 }
+__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t x0, uint32_t x1, u32x4 (&f)[6]) {
+  asm volatile(
+    "ds_read_b128 %0, %6\n\t"
+    "ds_read_b128 %1, %7\n\t"
+    "ds_read_b128 %4, %10\n\t"
+    "ds_read_b128 %5, %11\n\t"
+    "ds_read_b128 %2, %8\n\t"
+    "ds_read_b128 %3, %9\n\t"
+    "s_waitcnt lgkmcnt(0)"
+    : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5])
+    : "v"(w0), "v"(w1), "v"(w2), "v"(w3), "v"(x0), "v"(x1)
+    : "memory");
+}
+// the other half of every row of 16 lanes
+__device__ __forceinline__ bf16x8 other_half(const bf16x8& v) {
+  u32x4 r = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(0, r[i], 0x128, 0xF, 0xF, false);      // row_ror:8
+  return __builtin_bit_cast(bf16x8, r);
+}
 
-// XL: loads of x a slot: one for up to 8 rows (columns 8 to 15 of the tile then take rows 0 to 7 again), else two.
+// XL: loads of x a slot: two, or one for up to 8 rows.  Then two steps are taken at once: lanes of columns 0 to 7 read and split the
+// first one's x and those of columns 8 to 15 the second one's (an x row is split once, not twice; what columns 8 to 15 add up is
+// nobody's result), and one wait serves both: a step of 4 rows
+// (22 layers of width 2,048) 1,710 us with a step at a time, 1,616 with two.
 // SWIGLU: W is gate rows then up rows (up_offset apart); a tile is 8 gate rows and the 8 up rows of the same columns.
 template <int EPI, int WAVES, int SLOTS, int XL>
 __global__ void __launch_bounds__(WAVES * 64)
 skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ out,
                   long ldo, const float* __restrict__ bias, int M, int N, int K, int up_offset, RopeArgs rope) {
-  constexpr int SPW = 16 / WAVES;             // segments a wave
-  constexpr int L = 2 + XL, SLOT_BYTES = L * 1024;       // loads a slot: 16 weight rows of 128 bytes, then the x rows
+  constexpr int EPW = 8 / WAVES;              // eighths a wave
+  constexpr int U = XL == 1 ? 2 : 1;          // steps at once
+  constexpr int L = 2 + XL, SLOT_BYTES = L * 1024;       // loads a slot of 32 k: 16 weight rows of 128 bytes, then the x rows
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(16) char gf_lds[];
   char* ring = gf_lds;                                            // WAVES * SLOTS slots
-  float* s_acc = reinterpret_cast<float*>(gf_lds);                // [16][256], once every wave is done with its ring
+  float* s_acc = reinterpret_cast<float*>(gf_lds);                // [8][256], once every wave is done with its ring
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tile = blockIdx.x;
   const KCut cut = k_cut(K);
-  int seg_end[SPW], ks0, ks1;
+  int first_end, ks0, ks1;
   {
-    int b, e;
-    segment_range(cut, wave * SPW, ks0, e);
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) segment_range(cut, wave * SPW + i, b, seg_end[i]);
-    ks1 = seg_end[SPW - 1];
+    int b;
+    eighth_range(cut, wave * EPW, ks0, first_end);
+    eighth_range(cut, wave * EPW + EPW - 1, b, ks1);
   }
   const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;            // this lane's place in a load of 8 rows
-  const float *wsrc[2], *xsrc[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = lrow + 8 * j;
+  auto weight_row = [&](int r) {              // of the tile's row r; -1: there is none
     int wr = EPI == GF_SWIGLU ? tile * 8 + (r & 7) : tile * 16 + r;
     if (EPI == GF_ROPE) {
       const int per_head = rope.D >> 4, head = tile / per_head;
       wr = head * rope.D + (tile - head * per_head) * 8 + (r & 7) + (r >> 3) * (rope.D >> 1);
     }
-    if (wr >= N) wr = 0;                      // a row that does not exist is never stored
-    if (EPI == GF_SWIGLU) wr += (r >> 3) * up_offset;
-    wsrc[j] = W + (size_t)wr * ldw + lblk * 4;
+    if (wr >= N) return -1;
+    return EPI == GF_SWIGLU ? wr + (r >> 3) * up_offset : wr;
+  };
+  const float *wsrc[2], *xsrc[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = lrow + 8 * j, wr = weight_row(r);
+    wsrc[j] = W + (size_t)(wr < 0 ? 0 : wr) * ldw + lblk * 4;      // a row that does not exist is never stored
     xsrc[j] = X + (size_t)(r < M ? r : 0) * ldx + lblk * 4;
   }
   const float* zero = reinterpret_cast<const float*>(mie_zero_words) + lblk * 4;
   char* mine = ring + wave * SLOTS * SLOT_BYTES;
   auto issue = [&](int s) {
     char* base = mine + (s % SLOTS) * SLOT_BYTES;
-    const int ks = ks0 + s * GF_U;
-    const bool kok = ks + (lblk >> 2) < ks1 && ks * 16 + lblk * 4 < K;
-    const size_t k = (size_t)ks * 16;
+    const int ks = ks0 + s;
+    const bool kok = ks < ks1 && ks * 32 + lblk * 4 < K;
+    const size_t k = (size_t)ks * 32;
     const float* src[4] = {kok ? wsrc[0] + k : zero, kok ? wsrc[1] + k : zero, kok ? xsrc[0] + k : zero, kok ? xsrc[1] + k : zero};
 #pragma unroll
     for (int j = 0; j < L; ++j) {
@@ -140,35 +224,49 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
     }
   };
 #pragma unroll
-  for (int s = 0; s < SLOTS - 1; ++s) issue(s);
+  for (int s = 0; s < SLOTS - U; ++s) issue(s);
   const int col = lane & 15, kb = lane >> 4;
   const uint32_t ring0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine;
-  const uint32_t blk0 = (kb ^ (col & 7)) * 16, blk1 = ((4 + kb) ^ (col & 7)) * 16;
-  const uint32_t wrow0 = ring0 + col * 128, xrow0 = ring0 + 2048 + (XL == 1 ? col & 7 : col) * 128;
-  f32x4 acc[SPW];
+  const uint32_t blk0 = ((2 * kb) ^ (col & 7)) * 16, blk1 = ((2 * kb + 1) ^ (col & 7)) * 16;
+  const uint32_t wrow = ring0 + col * 128, xrow = ring0 + 2048 + (XL == 1 ? col & 7 : col) * 128;
+  f32x4 main[EPW], small[EPW];
 #pragma unroll
-  for (int i = 0; i < SPW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int rounds = ks1 > ks0 ? (ks1 - ks0 + GF_U - 1) / GF_U : 0;
-  for (int it = 0; it < rounds; ++it) {
-    issue(it + SLOTS - 1);                    // into the slot that was read a round ago
-    MIE_VMCNT((SLOTS - 1) * L);                // slot `it` has landed
-    u32x4 f[2 * GF_U];
-    const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
-    ring_read(w0 + blk0, x0 + blk0, w0 + blk1, x0 + blk1, f);
+  for (int i = 0; i < EPW; ++i) main[i] = small[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int ks, const Parts& w, const Parts& x) {       // (a step beyond ks1 is zeros)
 #pragma unroll
-    for (int u = 0; u < GF_U; ++u) {
-      const int ks = ks0 + it * GF_U + u;     // a step beyond ks1 loaded zeros and joins the last segment: it adds nothing
-      const f32x4 w4 = __builtin_bit_cast(f32x4, f[2 * u]), x4 = __builtin_bit_cast(f32x4, f[2 * u + 1]);
+    for (int i = 0; i < EPW; ++i)
+      if (EPW == 1 || (i == 0) == (ks < first_end)) {
+        main[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h, x.h, main[i], 0, 0, 0);
+        small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.m, x.h, small[i], 0, 0, 0);
+        small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h, x.m, small[i], 0, 0, 0);
+        small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.l, x.h, small[i], 0, 0, 0);
+        small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h, x.l, small[i], 0, 0, 0);
+        small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.m, x.m, small[i], 0, 0, 0);
+      }
+  };
+  auto parts = [](const u32x4& a, const u32x4& b) { return split8(__builtin_bit_cast(f32x4, a), __builtin_bit_cast(f32x4, b)); };
+  for (int it = 0; it < ks1 - ks0; it += U) {
 #pragma unroll
-      for (int i = 0; i < SPW; ++i)
-        if (i == SPW - 1 ? (SPW == 1 || ks >= seg_end[SPW > 1 ? SPW - 2 : 0]) : (ks < seg_end[i] && (i == 0 || ks >= seg_end[i > 0 ? i - 1 : 0])))
-          acc[i] = step_mfma(w4, x4, acc[i]);
+    for (int u = 0; u < U; ++u) issue(it + SLOTS - U + u);       // into the slots that were read a round ago
+    MIE_VMCNT((SLOTS - U) * L);                // slots `it` (and it + 1) have landed
+    const uint32_t at0 = (it % SLOTS) * SLOT_BYTES, at1 = ((it + 1) % SLOTS) * SLOT_BYTES;
+    if constexpr (U == 2) {
+      u32x4 f[6];
+      const uint32_t w0 = wrow + at0, w1 = wrow + at1, x0 = xrow + (col < 8 ? at0 : at1);
+      ring_read(w0 + blk0, w0 + blk1, w1 + blk0, w1 + blk1, x0 + blk0, x0 + blk1, f);
+      const Parts x = parts(f[4], f[5]);
+      step(ks0 + it, parts(f[0], f[1]), x);
+      step(ks0 + it + 1, parts(f[2], f[3]), {other_half(x.h), other_half(x.m), other_half(x.l)});
+    } else {
+      u32x4 f[4];
+      ring_read(wrow + at0 + blk0, wrow + at0 + blk1, xrow + at0 + blk0, xrow + at0 + blk1, f);
+      step(ks0 + it, parts(f[0], f[1]), parts(f[2], f[3]));
     }
   }
   MIE_VMCNT(0);                                // nothing of this wave is writing the LDS any more
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < SPW; ++i) *reinterpret_cast<f32x4*>(s_acc + (wave * SPW + i) * 256 + lane * 4) = acc[i];
+  for (int i = 0; i < EPW; ++i) *reinterpret_cast<f32x4*>(s_acc + (wave * EPW + i) * 256 + lane * 4) = main[i] + small[i];
   __syncthreads();
   if (threadIdx.x >= 256) return;
   // this thread's result: x row m, column c of the tile
@@ -179,9 +277,10 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
   for (int q = 0; q < 4; ++q) {
     float t = 0.f;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) t += s_acc[(4 * q + s) * 256 + src];
+    for (int e = 0; e < 2; ++e) t += s_acc[(2 * q + e) * 256 + src];
     v += t;
   }
+  if (v != v && m < M && weight_row(c) >= 0) v = plain_unit(X + (size_t)m * ldx, W + (size_t)weight_row(c) * ldw, K, cut, 0, 8);
   float other = 0.f;
   if (EPI == GF_SWIGLU || EPI == GF_ROPE) other = __shfl_xor(v, 8, 64);
   if (EPI == GF_ROPE) {
@@ -213,122 +312,139 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
 }
 
 // ------------------------------------------------------------------------------------------------ many rows
-// LEVELS 0: the unit is a segment (grid.z 16), 1: a quarter (grid.z 4), 2: all of K (grid.z 1, result or C += result).
-template <int BM, int BN, int WR, int WC, int LEVELS>
+// LEVELS 0: the unit is an eighth (grid.z 8), 1: a quarter (grid.z 4), 2: all of K (grid.z 1, result or C += result).
+// In the LDS, a buffer: planes h, m, l of BM + BN rows of 64 bytes; row r's block b of 16 bytes at 4 r + (b ^ (r / 2) % 4), so that
+// both the writes (a thread has 4 k) and the fragment reads (lane 16 g + r: row r, block g) spread over all banks.
+template <int BM, int BN, int WR, int WC, int LEVELS, bool TAIL>
 __global__ void __launch_bounds__(WR * WC * 64)
 tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ out,
                 long ldo, const float* __restrict__ bias, int add, int M, int N, int K) {
-  constexpr int THREADS = WR * WC * 64, WM = BM / WR, WN = BN / WC, TM = WM / 16, TN = WN / 16;
-  constexpr int XL = BM * 8 / THREADS, WL = BN * 8 / THREADS;      // 16-byte loads a thread and stage
+  constexpr int THREADS = WR * WC * 64, WM = BM / WR, WN = BN / WC, TM = WM / 16, TN = WN / 16, ROWS = BM + BN;
+  constexpr int PLANE = ROWS * 64, BUFFER = 3 * PLANE, XL = BM * 8 / THREADS, LOADS = ROWS * 8 / THREADS;      // 16-byte loads a thread and stage
+  static_assert(BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0, "loads of a thread are of x or of W");
   extern __shared__ __align__(16) char gf_lds[];
-  f32x4* xs = reinterpret_cast<f32x4*>(gf_lds);                    // [2][BM][8]: row r's block b at 8 r + (b ^ (r / 2) % 8)
-  f32x4* ws = xs + 2 * BM * 8;                                     // [2][BN][8]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const KCut cut = k_cut(K);
   int ks0, ks1;
-  if (LEVELS == 0) segment_range(cut, blockIdx.z, ks0, ks1);
+  if (LEVELS == 0) eighth_range(cut, blockIdx.z, ks0, ks1);
   else if (LEVELS == 1) { ks0 = least(blockIdx.z * cut.quarter, cut.steps); ks1 = least(ks0 + cut.quarter, cut.steps); }
   else { ks0 = 0; ks1 = cut.steps; }
 
-  const float* xsrc[XL];
-  const float* wsrc[WL];
-  int xat[XL], wat[WL], xblk[XL], wblk[WL];
+  const float* src[LOADS];
+  const int blk = tid & 7;                    // this thread's 4 k of every row it loads
+  int at[LOADS];
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int idx = tid + THREADS * i, r = idx >> 3, b = idx & 7, row = m0 + r;
-    xsrc[i] = X + (size_t)(row < M ? row : M - 1) * ldx + b * 4;
-    xblk[i] = b * 4;
-    xat[i] = r * 8 + (b ^ ((r >> 1) & 7));
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = (tid >> 3) + THREADS / 8 * i, row = i < XL ? m0 + r : n0 + r - BM;
+    src[i] = (i < XL ? X + (size_t)(row < M ? row : M - 1) * ldx : W + (size_t)(row < N ? row : N - 1) * ldw) + blk * 4;
+    at[i] = r * 64 + ((blk >> 1) ^ ((r >> 1) & 3)) * 16 + (blk & 1) * 8;
   }
-#pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int idx = tid + THREADS * i, r = idx >> 3, b = idx & 7, row = n0 + r;
-    wsrc[i] = W + (size_t)(row < N ? row : N - 1) * ldw + b * 4;
-    wblk[i] = b * 4;
-    wat[i] = r * 8 + (b ^ ((r >> 1) & 7));
-  }
-  f32x4 xr[XL], wreg[WL];
+  f32x4 staged[2][LOADS];                     // two steps on their way
   const f32x4 none = {0.f, 0.f, 0.f, 0.f};
-  auto fetch = [&](int ks) {                  // steps ks, ks + 1; what lies beyond K is zero, its load is from the row's end
-    const int k = ks * 16;
-    if (k + 32 <= K) {                        // (a unit may start at an odd step: the last stage can be cut short for any K)
+  auto fetch = [&](f32x4 (&staged)[LOADS], int ks) {      // step ks; TAIL: what lies beyond K is zero, its load is from the row's end
+    const int k = TAIL ? least(ks * 32, K - 4 - blk * 4) : ks * 32;
 #pragma unroll
-      for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const f32x4*>(xsrc[i] + k);
+    for (int i = 0; i < LOADS; ++i) staged[i] = *reinterpret_cast<const f32x4*>(src[i] + k);
+    if (TAIL && ks * 32 + blk * 4 >= K) {
 #pragma unroll
-      for (int i = 0; i < WL; ++i) wreg[i] = *reinterpret_cast<const f32x4*>(wsrc[i] + k);
-      return;
+      for (int i = 0; i < LOADS; ++i) staged[i] = none;
     }
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const f32x4*>(xsrc[i] + least(k, K - 4 - xblk[i]));
-#pragma unroll
-    for (int i = 0; i < WL; ++i) wreg[i] = *reinterpret_cast<const f32x4*>(wsrc[i] + least(k, K - 4 - wblk[i]));
-#pragma unroll
-    for (int i = 0; i < XL; ++i) if (k + xblk[i] >= K) xr[i] = none;
-#pragma unroll
-    for (int i = 0; i < WL; ++i) if (k + wblk[i] >= K) wreg[i] = none;
   };
-  auto put = [&](int buf) {
+  auto put = [&](const f32x4 (&staged)[LOADS], int buf) {
 #pragma unroll
-    for (int i = 0; i < XL; ++i) xs[buf * BM * 8 + xat[i]] = xr[i];
-#pragma unroll
-    for (int i = 0; i < WL; ++i) ws[buf * BN * 8 + wat[i]] = wreg[i];
+    for (int i = 0; i < LOADS; ++i) {
+      uint2 h, m, l;
+      split2(staged[i][0], staged[i][1], h.x, m.x, l.x);
+      split2(staged[i][2], staged[i][3], h.y, m.y, l.y);
+      char* p = gf_lds + buf * BUFFER + at[i];
+      *reinterpret_cast<uint2*>(p) = h;
+      *reinterpret_cast<uint2*>(p + PLANE) = m;
+      *reinterpret_cast<uint2*>(p + 2 * PLANE) = l;
+    }
   };
 
-  f32x4 acc[TN][TM], quarter[LEVELS >= 1 ? TN : 1][LEVELS >= 1 ? TM : 1], total[LEVELS >= 2 ? TN : 1][LEVELS >= 2 ? TM : 1];
+  f32x4 main[TN][TM], small[TN][TM], quarter[LEVELS >= 1 ? TN : 1][LEVELS >= 1 ? TM : 1], total[LEVELS >= 2 ? TN : 1][LEVELS >= 2 ? TM : 1];
 #pragma unroll
   for (int a = 0; a < TN; ++a)
 #pragma unroll
     for (int b = 0; b < TM; ++b) {
-      acc[a][b] = none;
+      main[a][b] = small[a][b] = none;
       if (LEVELS >= 1) quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0] = none;
       if (LEVELS >= 2) total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0] = none;
     }
   const int wm = (wave % WR) * WM, wn = (wave / WR) * WN;
   const int r16 = lane & 15, g = lane >> 4;
+  const int frag = r16 * 64 + (g ^ ((r16 >> 1) & 3)) * 16;
 
   int quarter_end = LEVELS >= 2 ? least(cut.quarter, cut.steps) : ks1;
-  int segment_end = LEVELS >= 1 ? least(ks0 + cut.segment, quarter_end) : ks1;
-  if (ks0 < ks1) fetch(ks0);
+  int eighth_end = LEVELS >= 1 ? least(ks0 + cut.eighth, quarter_end) : ks1;
+  bf16x8 wf[3][TN], xf[3][TM];
+  auto take = [&](int p, int buf) {           // this wave's fragments of plane p
+    const char* base = gf_lds + buf * BUFFER + p * PLANE + frag;
+#pragma unroll
+    for (int a = 0; a < TN; ++a) wf[p][a] = *reinterpret_cast<const bf16x8*>(base + (BM + wn + a * 16) * 64);
+#pragma unroll
+    for (int b = 0; b < TM; ++b) xf[p][b] = *reinterpret_cast<const bf16x8*>(base + (wm + b * 16) * 64);
+  };
+  auto products = [&](int p, int q, f32x4 (&acc)[TN][TM]) {
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+      for (int b = 0; b < TM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][a], xf[q][b], acc[a][b], 0, 0, 0);
+  };
+  if (ks0 < ks1) {                            // (behind the unit's end the last step once more, which nobody multiplies)
+    fetch(staged[0], ks0);
+    fetch(staged[1], least(ks0 + 1, ks1 - 1));
+    put(staged[0], 0);
+    fetch(staged[0], least(ks0 + 2, ks1 - 1));
+  }
+  __syncthreads();
   int buf = 0;
-  for (int ks = ks0; ks < ks1; ks += 2, buf ^= 1) {
-    put(buf);
-    __syncthreads();                          // (a buffer is written again two stages on, behind the barrier in between)
-    if (ks + 2 < ks1) fetch(ks + 2);
+  auto stage = [&](int ks, f32x4 (&next)[LOADS]) {       // next: the registers that hold step ks + 1
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (ks + u >= ks1) break;
-      f32x4 wf[TN], xf[TM];
+    for (int p = 0; p < 3; ++p) take(p, buf);
+    buf ^= 1;
+    put(next, buf);                           // (everybody has read this buffer before the last barrier)
+    fetch(next, least(ks + 3, ks1 - 1));
+    products(0, 0, main);
+    products(1, 0, small);
+    products(0, 1, small);
+    products(2, 0, small);
+    products(0, 2, small);
+    products(1, 1, small);
+    // matrix instructions and the splitting in turn
 #pragma unroll
-      for (int a = 0; a < TN; ++a) { const int r = wn + a * 16 + r16; wf[a] = ws[buf * BN * 8 + r * 8 + ((4 * u + g) ^ ((r >> 1) & 7))]; }
+    for (int i = 0; i < 6 * TM * TN; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    }
+    if (LEVELS >= 1 && ks + 1 == eighth_end) {
+      const bool quarter_done = LEVELS >= 2 && eighth_end == quarter_end;
 #pragma unroll
-      for (int b = 0; b < TM; ++b) { const int r = wm + b * 16 + r16; xf[b] = xs[buf * BM * 8 + r * 8 + ((4 * u + g) ^ ((r >> 1) & 7))]; }
+      for (int a = 0; a < TN; ++a)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-          for (int b = 0; b < TM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[a][j], xf[b][j], acc[a][b], 0, 0, 0);
-      if (LEVELS >= 1 && ks + u + 1 == segment_end) {
-        const bool quarter_done = LEVELS >= 2 && segment_end == quarter_end;
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-          for (int b = 0; b < TM; ++b) {
-            f32x4& q = quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0];
-            q += acc[a][b];
-            acc[a][b] = none;
-            if (quarter_done) {
-              total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0] += q;
-              q = none;
-            }
+        for (int b = 0; b < TM; ++b) {
+          f32x4& q = quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0];
+          q += main[a][b] + small[a][b];
+          main[a][b] = small[a][b] = none;
+          if (quarter_done) {
+            total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0] += q;
+            q = none;
           }
-        if (quarter_done) quarter_end = least(quarter_end + cut.quarter, cut.steps);
-        segment_end = least(segment_end + cut.segment, quarter_end);
-      }
+        }
+      if (quarter_done) quarter_end = least(quarter_end + cut.quarter, cut.steps);
+      eighth_end = least(eighth_end + cut.eighth, quarter_end);
+    }
+    __syncthreads();
+  };
+  for (int ks = ks0; ks < ks1;) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      stage(ks, staged[j ^ 1]);
+      if (++ks >= ks1) break;
     }
   }
-
   // acc[i] of lane (r16, g): weight row 4 g + i of the 16, x row r16
   float* dst = out + (LEVELS < 2 ? (size_t)blockIdx.z * M * N : 0);
   const long ld = LEVELS < 2 ? N : ldo;
@@ -340,8 +456,15 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
     for (int a = 0; a < TN; ++a) {
       const int n = n0 + wn + a * 16 + 4 * g;
       if (n >= N) continue;                   // N is a multiple of 4
-      f32x4 v = LEVELS == 0 ? acc[a][b] : LEVELS == 1 ? quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0]
-                                                      : total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0];
+      f32x4 v = LEVELS == 0 ? main[a][b] + small[a][b] : LEVELS == 1 ? quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0]
+                                                                     : total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0];
+      if (__any(v[0] + v[1] + v[2] + v[3] != v[0] + v[1] + v[2] + v[3])) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (v[i] != v[i])
+            v[i] = plain_unit(X + (size_t)m * ldx, W + (size_t)(n + i) * ldw, K, cut,
+                              LEVELS == 0 ? blockIdx.z : LEVELS == 1 ? 2 * blockIdx.z : 0, LEVELS == 0 ? 1 : LEVELS == 1 ? 2 : 8);
+      }
       f32x4* o = reinterpret_cast<f32x4*>(dst + (size_t)m * ld + n);
       if (LEVELS == 2) {
         if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
@@ -352,7 +475,7 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
   }
 }
 
-// The sums of PARTS (4 quarters or 16 segments) units joined in the order above, then stored, added into `out`, or, with
+// The sums of PARTS (4 quarters or 8 eighths) units joined in the order above, then stored, added into `out`, or, with
 // gate sums in columns [0, N) and up sums in [N, 2 N) (`part` has 2 N columns), silu(gate) * up.
 template <int PARTS>
 __device__ __forceinline__ f32x4 join_parts(const f32x4* p, size_t stride) {
@@ -367,7 +490,7 @@ __device__ __forceinline__ f32x4 join_parts(const f32x4* p, size_t stride) {
     if (PARTS == 4) t = v[q];
     else {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) t += v[(4 * q + s) % PARTS];
+      for (int e = 0; e < 2; ++e) t += v[(2 * q + e) % PARTS];
     }
     total += t;
   }
@@ -406,25 +529,38 @@ static int check_operands(const char* what, const void* X, long ldx, const void*
   return 0;
 }
 
-// The tile of a workgroup (wide: 128 rows of x by 64 of W and eight waves, else 64 by 64 and four) and how many units K is
-// cut into for M rows (more than 16): 1, 4 or 16.  Measured over 32 to 2,048 rows at [2560, 2048], [2048, 2048],
-// [11264, 2048] and [2048, 5632] (MI355X, us): the wide tile reads a third less out of the L2s and wins from two
-// workgroups a compute unit on (512 rows of [11264, 2048] 225 against 241, 2,048 rows of [2048, 2048] 150 against 165),
-// unless its last rows would be empty (300 rows of [11264, 2048] 184 against 157).  64 by 64 in quarters from 128 tiles
-// on (512 rows of [2048, 2048] 51 against 61 in segments and 62 whole, 200 of [11264, 2048] 121 against 127 whole),
-// in segments below (32 rows of [2048, 5632] 22 against 44).
-static void tile_plan(int M, int N, bool& wide, int& units) {
-  auto tiles = [&](int a, int b) { return (long)((M + a - 1) / a) * ((N + b - 1) / b); };
-  wide = tiles(128, 64) >= 512 && (M + 127) / 128 * 128 * 10 <= (M + 63) / 64 * 64 * 11;
-  const long t = tiles(64, 64);
-  units = wide || t >= 1024 ? 1 : t >= 128 ? 4 : 16;
+// The tile of a workgroup and how many units K is cut into (1, 4 or 8) for M rows (more than 16): the cheapest by what was
+// measured (MI355X, 17 to 2,048 rows of [11264, 2048], [2560, 2048], [2048, 2048], [2048, 5632], [768, 1536] and two small
+// weights).  A step of 32 k costs a compute unit fixed + each x the workgroups it has, whether they run side by side or in
+// turn; a start 2.9 us; units' sums cost a kernel of 1.9 us and 1.6 us a million of them.  Large tiles split and read an operand for more outputs, small ones and units of K give every compute unit
+// work: us of 128 x 128 / 128 x 64 / 64 x 64, each at its best cut: 512 rows of [11264, 2048] 176 / 169 / 180, 2,048 rows 543 / 638 /
+// 684, 512 rows of [2048, 2048] 35 / 40 / 39, 100 rows 20 / 17 / 16, 32 rows of [2048, 5632] 36 / 27 / 20.  gated: the product's
+// gate and up columns are joined where the units' sums are, else by a pass of its own.
+constexpr struct { int bm, bn; float fixed, each; } GF_TILES[3] = {{128, 128, 0.f, 1.40f}, {128, 64, 0.f, 0.87f}, {64, 64, 0.07f, 0.45f}};
+struct TilePlan {
+  int tile, units;
+};
+static TilePlan tile_plan(int M, int N, int K, bool gated) {
+  TilePlan best = {2, 8};
+  float least_us = 1e30f;
+  const KCut cut = k_cut(K);
+  const float outputs = (float)M * N;
+  for (int t = 0; t < 3; ++t) {
+    const long tiles = (long)((M + GF_TILES[t].bm - 1) / GF_TILES[t].bm) * ((N + GF_TILES[t].bn - 1) / GF_TILES[t].bn);
+    for (int units = 1; units <= 8; units += units == 1 ? 3 : 4) {
+      const int steps = units == 1 ? cut.steps : units == 4 ? cut.quarter : cut.eighth;
+      const long each = (tiles * units + mie_compute_units() - 1) / mie_compute_units();
+      float us = 2.9f + steps * (GF_TILES[t].fixed + GF_TILES[t].each * each);
+      if (units > 1 || gated) us += 1.9f + outputs * units * 1.6e-6f;
+      if (us < least_us) {
+        least_us = us;
+        best = {t, units};
+      }
+    }
+  }
+  return best;
 }
-MIE_EXPORT int mie_f32_units(int M, int N) {
-  bool wide;
-  int units;
-  tile_plan(M, N, wide, units);
-  return units;
-}
+MIE_EXPORT int mie_f32_units(int M, int N, int K, int gated) { return tile_plan(M, N, K, gated != 0).units; }
 
 template <int EPI>
 static int launch_skinny(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int M, int N,
@@ -451,8 +587,8 @@ static int launch_skinny(const float* X, long ldx, const float* W, long ldw, flo
 template <int BM, int BN, int WR, int WC, int LEVELS>
 static int launch_tile(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int add, int M,
                        int N, int K, int units, hipStream_t s) {
-  constexpr int lds = 2 * (BM + BN) * 128;
-  auto kernel = tile_f32_kernel<BM, BN, WR, WC, LEVELS>;
+  constexpr int lds = 2 * (BM + BN) * 192;
+  auto kernel = K & 31 ? tile_f32_kernel<BM, BN, WR, WC, LEVELS, true> : tile_f32_kernel<BM, BN, WR, WC, LEVELS, false>;
   if ((M + BM - 1) / BM > 65535) MIE_FAIL("gemm_f32: M = %d is beyond the grid", M);
   if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;
   hipLaunchKernelGGL(kernel, dim3((N + BN - 1) / BN, (M + BM - 1) / BM, units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, add, M, N, K);
@@ -461,11 +597,15 @@ static int launch_tile(const float* X, long ldx, const float* W, long ldw, float
 }
 
 static int launch_tiles(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int add, int M,
-                        int N, int K, bool wide, int units, hipStream_t s) {
-  if (wide) return launch_tile<128, 64, 4, 2, 2>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 1, s);
-  return units == 1   ? launch_tile<64, 64, 2, 2, 2>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 1, s)
-         : units == 4 ? launch_tile<64, 64, 2, 2, 1>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 4, s)
-                      : launch_tile<64, 64, 2, 2, 0>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 16, s);
+                        int N, int K, const TilePlan& plan, hipStream_t s) {
+#define GF_TILE(BM, BN, WR, WC)                                                                                             \
+  return plan.units == 1   ? launch_tile<BM, BN, WR, WC, 2>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 1, s)           \
+         : plan.units == 4 ? launch_tile<BM, BN, WR, WC, 1>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 4, s)           \
+                           : launch_tile<BM, BN, WR, WC, 0>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 8, s)
+  if (plan.tile == 0) GF_TILE(128, 128, 4, 2);
+  if (plan.tile == 1) GF_TILE(128, 64, 4, 2);
+  GF_TILE(64, 64, 2, 4);
+#undef GF_TILE
 }
 
 template <int EPI>
@@ -475,14 +615,14 @@ static int launch_reduce(int units, const float* part, float* out, long ldo, con
   if (units == 4)
     hipLaunchKernelGGL((reduce_f32_kernel<4, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N);
   else
-    hipLaunchKernelGGL((reduce_f32_kernel<16, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N);
+    hipLaunchKernelGGL((reduce_f32_kernel<8, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N);
   MIE_CHECK_LAUNCH("reduce_f32");
   return 0;
 }
 
 // epi 0: out = x W^T (+ bias), 1: out += x W^T (+ bias), 2: out = silu(gate) * up with W = [gate rows (N of them); up rows].
-// part: mie_f32_units(M, columns of x W^T) * M * columns floats, 16-byte aligned, when M > 16 and that is more than one
-// unit or epi is 2 (then at least one unit's worth).
+// part: mie_f32_units(M, columns of x W^T, K, epi == 2) * M * columns floats, 16-byte aligned, when M > 16 and that is more than
+// one unit.
 MIE_EXPORT int mie_gemm_f32(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, int epi, const float* bias,
                             float* part, int M, int N, int K, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
@@ -495,13 +635,12 @@ MIE_EXPORT int mie_gemm_f32(const float* X, long ldx, const float* W, long ldw, 
          : epi == GF_ADD ? launch_skinny<GF_ADD>(X, ldx, W, ldw, out, ldo, bias, M, N, K, s)
                          : launch_skinny<GF_SWIGLU>(X, ldx, W, ldw, out, ldo, bias, M, N, K, s);
   const int cols = epi == GF_SWIGLU ? 2 * N : N;
-  bool wide;
-  int units;
-  tile_plan(M, cols, wide, units);
-  if (units == 1 && epi != GF_SWIGLU) return launch_tiles(X, ldx, W, ldw, out, ldo, bias, epi == GF_ADD, M, N, K, wide, 1, s);
+  const TilePlan plan = tile_plan(M, cols, K, epi == GF_SWIGLU);
+  const int units = plan.units;
+  if (units == 1 && epi != GF_SWIGLU) return launch_tiles(X, ldx, W, ldw, out, ldo, bias, epi == GF_ADD, M, N, K, plan, s);
   if (epi == GF_SWIGLU && units == 1) MIE_FAIL("gemm_f32: %d rows of %d columns are one unit: take the product and silu_mul", M, cols);
   if (!part) MIE_FAIL("gemm_f32: %d units need memory for their sums", units);
-  if (launch_tiles(X, ldx, W, ldw, part, cols, nullptr, 0, M, cols, K, wide, units, s)) return -1;
+  if (launch_tiles(X, ldx, W, ldw, part, cols, nullptr, 0, M, cols, K, plan, s)) return -1;
   return epi == GF_STORE ? launch_reduce<GF_STORE>(units, part, out, ldo, bias, M, N, s)
        : epi == GF_ADD ? launch_reduce<GF_ADD>(units, part, out, ldo, bias, M, N, s)
                        : launch_reduce<GF_SWIGLU>(units, part, out, ldo, bias, M, N, s);

@@ -238,7 +238,7 @@ class HipBackend(KernelBackend):
         M, K = x.shape
         cols, part = w.shape[0], None
         if M > 16:
-            units = lib.mie_f32_units(M, cols)
+            units = lib.mie_f32_units(M, cols, K, int(epi == self.F32_SWIGLU))
             if units > 1:
                 part = torch.empty((units, M, cols), dtype=torch.float32, device=x.device)
             elif epi == self.F32_SWIGLU:

@@ -38,7 +38,7 @@ register_kernel_module("gemm", {
     "mie_clamped_glu_bf16": [P, L, P, L, I, I, F, F, F, P],
 })
 register_kernel_module("gemm_f32", {
-    "mie_f32_units": [I, I],
+    "mie_f32_units": [I, I, I, I],
     "mie_gemm_f32": [P, L, P, L, P, L, I, P, P, I, I, I, P],
     "mie_qkv_rope_f32": [P, L, P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, I, P],
 })

@@ -147,6 +147,47 @@ def test_linear_float32_matrix_unit(ops, shape):
     assert torch.equal(o.linear(x, w, bias=bias), y + bias)
 
 
+# rows that take the few-row kernel (two steps at once, one), the small tile in eighths and whole, the large ones in quarters and
+# whole; K with an odd number of steps for a wave, without any for most, and a step cut short
+F32_PARTS = [(3, 2080, 48), (12, 2080, 48), (40, 1056, 64), (20, 36, 352), (300, 2048, 2048), (1100, 96, 2304), (600, 352, 9000)]
+
+
+@pytest.mark.parametrize("shape", F32_PARTS)
+def test_linear_float32_in_three_parts(ops, shape):
+    """The float32 product as six bfloat16 ones: its error in the 2-norm is below that of chains of 32-bit products (a quarter of
+    the worst case, sqrt(terms) half ulps); numbers that bfloat16 cannot hold give the infinities, NaN and finite results that 32-bit
+    arithmetic gives them, and change no bit of another row or column."""
+    M, K, N = shape
+    o = ops[torch.float32]
+    torch.manual_seed(K + N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) / math.sqrt(K)
+    y, exact = o.linear(x, w), x.double() @ w.double().T
+    assert (y.double() - exact).norm() <= 2.0 ** -24 * math.sqrt(K / 16 + 8) * exact.norm()
+    for at, value in ((0, float("inf")), (K // 2, float("-inf")), (K - 1, float("nan")), (min(35, K - 1), 3.4e38)):
+        x2, w2 = x.clone(), w.clone()
+        x2[M // 2, at] = value
+        w2[N - 3, K - 1 - at] = value
+        w2[5, at] = 0.0 if at else 0.25              # an infinity times zero, and times a number bfloat16 holds whole
+        if value == 3.4e38:
+            w2[:, at] *= 2.0 ** -20                  # (finite results)
+            x2[:, K - 1 - at] *= 2.0 ** -20
+        got = o.linear(x2, w2)
+        want = x2.double() @ w2.double().T
+        large = want.abs() > 3.4028234663852886e38
+        want[large] = torch.sign(want[large]) * float("inf")
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(torch.where(got.isinf(), got, 0.0), torch.where(want.isinf(), want, 0.0).float())
+        finite = want.isfinite()
+        bound = (K / 16 + 32) * 2.0 ** -24 * (x2.double().abs() @ w2.double().abs().T) + 1e-30
+        assert bool(((got.double() - want).abs()[finite] <= bound[finite]).all())
+        if value != 3.4e38:
+            rows = torch.arange(M, device=DEV) != M // 2
+            cols = (torch.arange(N, device=DEV) != N - 3) & (torch.arange(N, device=DEV) != 5)
+            assert torch.equal(got[rows][:, cols], y[rows][:, cols])
+            alone = o.linear(x2[M // 2:M // 2 + 1].contiguous(), w2)
+            assert torch.equal(alone.nan_to_num(1e30), got[M // 2:M // 2 + 1].nan_to_num(1e30))
+
+
 def test_linear_mixed_storage(ops):
     """A matrix stored in 32-bit beside bfloat16 activations: computed, not refused."""
     torch.manual_seed(2)
