@@ -3,6 +3,7 @@
 // Caches: keys [pages, Hkv, page, D], values [pages, Hkv, D, page].
 //
 #include "attention_bf16_common.hpp"
+#include "launch.hpp"
 
 // prefill_attention: rows of several tokens, starting anywhere in their request.  With
 // v_mfma_f32_32x32x16_bf16 (A: 32 rows x 16 k, B: 16 k x 32 columns, C: 32 x 32, lane l holds column l % 32
@@ -56,12 +57,16 @@ constexpr int KS16 = D / 16;                        // 16-dim steps of q . k
 constexpr int DT32 = (D + 31) / 32;                 // 32-dim tiles of the output (the last may be half empty)
 constexpr int PF_KROW = 2 * D + 16;                 // bytes of a key row in the LDS
 constexpr int PF_VROW = 2 * PF_BK + 16;             // bytes of a value row (one dim, 64 keys) in the LDS
-constexpr int PF_KBYTES = PF_BK * PF_KROW;
-constexpr int PF_VBYTES = DT32 * 32 * PF_VROW;      // rows of dims beyond D stay zero
+constexpr bool PF_DIRECT = D == 64 || D == 128;     // blocks come in by loads that write the LDS themselves
+constexpr int PF_KBYTES = PF_DIRECT ? PF_BK * 2 * D : PF_BK * PF_KROW;
+constexpr int PF_VBYTES = PF_DIRECT ? PF_BK * 2 * D : DT32 * 32 * PF_VROW;      // rows of dims beyond D stay zero
 constexpr int PF_BUF = PF_KBYTES + PF_VBYTES;       // one buffer: keys, then values
 constexpr int PF_KPIECES = PF_BK * (D / 16);        // 32-byte pieces: 16 dims of one key
 constexpr int PF_VPIECES = D * (PF_BK / 16);        //                 16 keys of one dim
 constexpr int PF_PIECES = PF_KPIECES + PF_VPIECES;
+// sets of buffers for steps of `halves` blocks: one being computed, the others on their way
+constexpr int pf_sets(int halves) { return PF_DIRECT && 3 * halves * PF_BUF <= 96 * 1024 ? 3 : 2; }
+constexpr int pf_lds_bytes(int halves) { return pf_sets(halves) * halves * PF_BUF; }
 
 // max of three numbers none of which is a NaN, as one instruction
 __device__ __forceinline__ float max3_nn(float a, float b, float c) {
@@ -150,6 +155,29 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
     }
   }
 
+  // pages of a power of two (the usual 16): a key's page by a shift (the same for every lane)
+  const int page_shift = (page & (page - 1)) == 0 ? __builtin_ctz(page) : -1;
+  // PF_DIRECT: where this lane's pieces of a load come from and where its fragments lie
+  uint32_t k_from[D / 32 + 1], v_from = 0;
+  int k_lane = 0, v_lane = 0;
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)pf_lds;
+  if constexpr (PF_DIRECT) {
+    auto swizzle = [](int r) { return ((r & 3) ^ ((r >> 2) & 1)) | ((r >> 1) & 4) | (D == 128 ? (r << 1) & 8 : 0); };
+    auto swapped = [](int d) { return ((d >> 2) ^ (d >> 3)) & 1; };
+    constexpr int BLOCKS = D / 8;                              // 16-byte blocks of a key
+#pragma unroll
+    for (int j = 0; j < D / 32; ++j) {
+      const int r = (64 / BLOCKS) * j + lane / BLOCKS;
+      k_from[j] = r * 2 * D + ((lane % BLOCKS) ^ swizzle(r)) * 16;
+    }
+    v_from = (lane >> 1) * page * 2 + ((lane & 1) ^ swapped(lane >> 1)) * 16;
+    // row `col` of a score tile is key 8 (bit 2) + 4 (bit 3) + bits 0 and 1 of its 16: a lane's scores are then runs of
+    // eight keys, which the values' fragments read as they lie in the page
+    const int r = (col & 16) + ((col & 4) << 1) + ((col & 8) >> 1) + (col & 3);
+    k_lane = r * 2 * D + (g ^ swizzle(r & 15)) * 16;
+    v_lane = col * 32 + (g ^ swapped(col)) * 16;
+  }
+
   for (int pass = 0; pass < 2; ++pass) {
     const int s = pass == 0 ? NS - 1 - bx : bx;
     if (pass == 1 && (!paired || s >= NS - 1 - bx)) break;   // the middle stretch of an odd number has no partner
@@ -166,12 +194,15 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
     const int last_q = wave_q0 + PF_QW - 1 < q_len ? wave_q0 + PF_QW - 1 : q_len - 1;
     const int tile_first = p0 + wave_q0, tile_last = p0 + last_q;
     Frag qf[KS16];
+    auto load_queries = [&]() {
 #pragma unroll
-    for (int ks = 0; ks < KS16; ++ks) {
-      qf[ks].q = make_uint4(0, 0, 0, 0);
-      if (tile_ok)
-        qf[ks].q = *reinterpret_cast<const uint4*>(q + (size_t)qtok * q_stride + (size_t)head * D + ks * 16 + g * 8);
-    }
+      for (int ks = 0; ks < KS16; ++ks) {
+        qf[ks].q = make_uint4(0, 0, 0, 0);
+        if (tile_ok)
+          qf[ks].q = *reinterpret_cast<const uint4*>(q + (size_t)qtok * q_stride + (size_t)head * D + ks * 16 + g * 8);
+      }
+    };
+    if constexpr (!PF_DIRECT) load_queries();
     // keys the wave's queries can see, and the workgroup's (the union over its waves)
     const int wave_kmax = tile_ok ? tile_last : -1;            // -1: the wave has no query
     int wave_kmin = window > 0 ? tile_first - window + 1 : 0;
@@ -219,12 +250,51 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
     const float* __restrict__ db_row = DB ? dist_bias + (size_t)head * dist_n : nullptr;
     const float sl2 = DB ? 1.f : scale_log2;
 
+    // key of score i of score tile u of this lane, within its block
+    auto key_off = [&](int u, int i) {
+      return PF_DIRECT ? 32 * u + 16 * (i >> 3) + 8 * g + (i & 7) : 32 * u + 8 * (i >> 2) + 4 * g + (i & 3);
+    };
+
     float m = -INFINITY, l = 0.f;
     f32x16 O[DT32];
 #pragma unroll
     for (int dt = 0; dt < DT32; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[dt][i] = 0.f;
+
+    // ---- bringing a step into the LDS without registers between (PF_DIRECT).  16 keys of a page are one run of 32 D bytes;
+    // 16 keys of all dims of its values are D pieces of 32 (also one run, in pages of 16).  A wave brings the keys, the
+    // values or both of one such group, 1 KB a load, each from the page in a scalar register (looked up a step ahead).
+    // Keys stand as rows of 2 D bytes, block c of 16 bytes of key r at c ^ f(r), values as D rows of 32 bytes, the two halves
+    // of row d swapped by bits 2 and 3 of d: so the fragment reads, which take 16 lanes' worth of 16 bytes at a time, meet every bank once.
+    constexpr int GROUP_PARTS = KS * 8 / PF_WAVES;             // 1: keys or values of a group, 2: both
+    constexpr int LOADS = GROUP_PARTS * D / 32;                // of a wave and step
+    const int group = wave * GROUP_PARTS >> 1;
+    int page_at = 0, off_at = 0;
+    auto find_page = [&](int x) {
+      int key = key_of(x) + 16 * group;
+      key = key < (kmax & ~15) ? key : kmax & ~15;             // beyond the row's keys: its last ones again
+      const int idx = page_shift >= 0 ? key >> page_shift : key / page;
+      page_at = bt[idx];
+      off_at = key - idx * page;
+    };
+    auto bring = [&](int x, int set) {                         // in order, a step apart
+      const uint32_t to = lds0 + set * KS * PF_BUF + (group >> 2) * PF_BUF + (group & 3) * 32 * D;
+      const size_t head_at = (size_t)page_at * Hkv + kvh;
+#pragma unroll
+      for (int part = 0; part < GROUP_PARTS; ++part) {
+        if (GROUP_PARTS == 1 ? (wave & 1) == 0 : part == 0) {
+          const bf16* from = k_cache + (head_at * page + off_at) * D;
+#pragma unroll
+          for (int j = 0; j < D / 32; ++j) mie_load_to_lds(from, k_from[j], to + j * 1024);
+        } else {
+          const bf16* from = v_cache + head_at * D * page + off_at;
+#pragma unroll
+          for (int j = 0; j < D / 32; ++j) mie_load_to_lds(from + (size_t)j * 32 * page, v_from, to + PF_KBYTES + j * 1024);
+        }
+      }
+      find_page(x + FK);
+    };
 
     // ---- bringing a block into the LDS, by all threads: a piece is 32 bytes, 16 dims of one key or 16 keys
     // of one dim, so one page look-up and one address serve two loads.  Where a piece lies (page and place
@@ -238,8 +308,6 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
       uint4 lo[PF_PPT], hi[PF_PPT];
     };
     int walk_idx = blk0 / page, walk_start = walk_idx * page;
-    // pages of a power of two (the usual 16): a key's page by a shift (the same for every lane)
-    const int page_shift = (page & (page - 1)) == 0 ? __builtin_ctz(page) : -1;
     auto lookup = [&](Where& Wh, int blk) {            // blocks are looked up in order, 64 keys apart
       blk = key_of(blk);
       blk = blk < last_blk ? blk : last_blk;           // beyond the last block: the last one again
@@ -333,8 +401,8 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 
     // ---- one block of 64 keys for the wave's tile: the wave's half of the step in set `set`
     auto compute = [&](int set, int blk) {
-      const unsigned char* Kb = pf_lds + (set * KS + wk) * PF_BUF + col * PF_KROW + g * 16;
-      const unsigned char* Vb = pf_lds + (set * KS + wk) * PF_BUF + PF_KBYTES + col * PF_VROW + g * 16;
+      const unsigned char* Kb = pf_lds + (set * KS + wk) * PF_BUF + (PF_DIRECT ? 0 : col * PF_KROW + g * 16);
+      const unsigned char* Vb = pf_lds + (set * KS + wk) * PF_BUF + PF_KBYTES + (PF_DIRECT ? v_lane : col * PF_VROW + g * 16);
       // DB: the table's entries for this lane's 32 scores, in units of log2 e, asked for before the first product so that
       // they are there when the scores are: score * scale + table[min(distance, dist_n - 1)].  Three cases, each uniform
       // over the wave: every key of the block beyond the table's reach for every query of the tile (one number for all);
@@ -349,12 +417,12 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 #pragma unroll
             for (int i = 0; i < 16; ++i) tb[u][i] = far;
         } else if (tile_ok && blk + PF_BK - 1 <= tile_first && tile_last - blk <= dist_n - 1) {
-          const float* __restrict__ at = db_row + (qpos - blk) - 4 * g;
+          const float* __restrict__ at = db_row + (qpos - blk) - key_off(0, 0);
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              const Run4 r = *reinterpret_cast<const Run4*>(at - (32 * u + 8 * e + 3));
+              const Run4 r = *reinterpret_cast<const Run4*>(at - (key_off(u, 4 * e) - key_off(0, 0) + 3));
               tb[u][4 * e + 0] = r.d;
               tb[u][4 * e + 1] = r.c;
               tb[u][4 * e + 2] = r.b;
@@ -365,7 +433,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-              int n = qpos - (blk + 32 * u + 8 * (i >> 2) + 4 * g + (i & 3));
+              int n = qpos - (blk + key_off(u, i));
               n = n < 0 ? 0 : (n < dist_n ? n : dist_n - 1);          // a key after the query is masked below
               tb[u][i] = db_row[n];
             }
@@ -373,16 +441,71 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
       }
       f32x16 S[2];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[u][i] = 0.f;
+      constexpr int AHEAD = D == 64 ? 4 : DB ? 1 : 2;                  // PF_DIRECT: 16-key pieces of values read before the softmax
+      Frag va[PF_DIRECT ? DT32 : 1][4];
+      auto values = [&](int dt, int t) {
+        return *reinterpret_cast<const uint4*>(Vb + (PF_DIRECT ? t * 32 * D + dt * 1024 : dt * 32 * PF_VROW + t * 32));
+      };
+      if constexpr (PF_DIRECT) {
+        // all fragments asked for together, the values' before the softmax: nothing waits for the LDS in between
+        Frag ka[2][KS16];
 #pragma unroll
-        for (int ks = 0; ks < KS16; ++ks) {
-          Frag a;
-          a.q = *reinterpret_cast<const uint4*>(Kb + 32 * u * PF_KROW + ks * 32);
-          S[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, qf[ks].v, S[u], 0, 0, 0);
-        }
+        for (int ks = 0; ks < KS16; ++ks)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) ka[u][ks].q = *reinterpret_cast<const uint4*>(Kb + 64 * u * D + (k_lane ^ (ks * 32)));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < KS16; ++ks)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) S[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[u][ks].v, qf[ks].v, S[u], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t)
+#pragma unroll
+          for (int dt = 0; dt < DT32; ++dt) va[dt][t].q = values(dt, t);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int ks = 0; ks < KS16; ++ks) {
+            Frag a;
+            a.q = *reinterpret_cast<const uint4*>(Kb + 32 * u * PF_KROW + ks * 32);
+            S[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, qf[ks].v, S[u], 0, 0, 0);
+          }
       }
+      auto add_values = [&](const Frag (&pb)[4]) {
+        if constexpr (PF_DIRECT) {
+#pragma unroll
+          for (int t = AHEAD; t < 4; ++t)
+#pragma unroll
+            for (int dt = 0; dt < DT32; ++dt) va[dt][t].q = values(dt, t);
+          if (blk + PF_BK - 1 > vmax || blk < vmin) {
+            // values that nobody may look at (see stash): their weight is 0, but 0 * NaN would reach the sum
+            auto dead = [&](int key) { return key > vmax || (key < vmin && !(KEEP && key < keep)); };
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int key = blk + 16 * t + 8 * g + 2 * e;
+                const uint32_t bits = (dead(key) ? 0u : 0x0000FFFFu) | (dead(key + 1) ? 0u : 0xFFFF0000u);
+#pragma unroll
+                for (int dt = 0; dt < DT32; ++dt) va[dt][t].w[e] &= bits;
+              }
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int dt = 0; dt < DT32; ++dt) {
+            Frag a;
+            if constexpr (PF_DIRECT) a = va[dt][t];
+            else a.q = values(dt, t);
+            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, pb[t].v, O[dt], 0, 0, 0);
+          }
+      };
       // every query of the tile sees every key of the block (uniform over the wave)
       const bool whole = blk + PF_BK - 1 <= tile_first &&
                          (window <= 0 || blk >= tile_last - window + 1 || (KEEP && blk + PF_BK <= keep)) && (!(SIG || CHUNK) || blk >= tile_lo);
@@ -415,7 +538,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-              const int key = blk + 32 * u + 8 * (i >> 2) + 4 * g + (i & 3);
+              const int key = blk + key_off(u, i);
               S[u][i] = key >= lo && key <= hi ? S[u][i] : 0.f;
             }
         }
@@ -424,14 +547,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int e = 0; e < 8; ++e) pb[2 * u + (e >> 2)].w[e & 3] = pack_bf16(S[u][2 * e], S[u][2 * e + 1]);
-#pragma unroll
-        for (int dt = 0; dt < DT32; ++dt)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            Frag va;
-            va.q = *reinterpret_cast<const uint4*>(Vb + dt * 32 * PF_VROW + t * 32);
-            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va.v, pb[t].v, O[dt], 0, 0, 0);
-          }
+        add_values(pb);
         return;
       }
       float alpha;
@@ -458,7 +574,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const int key = blk + 32 * u + 8 * (i >> 2) + 4 * g + (i & 3);
+            const int key = blk + key_off(u, i);
             const bool ok = (key >= lo || (KEEP && key < keep)) && key <= hi;
             S[u][i] = ok ? S[u][i] : -INFINITY;
             mx = max_nn(mx, S[u][i]);
@@ -492,56 +608,76 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 #pragma unroll
           for (int i = 0; i < 16; ++i) O[dt][i] *= alpha;
       }
-#pragma unroll
-      for (int dt = 0; dt < DT32; ++dt)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          Frag va;
-          va.q = *reinterpret_cast<const uint4*>(Vb + dt * 32 * PF_VROW + t * 32);
-          O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va.v, pb[t].v, O[dt], 0, 0, 0);
-        }
+      add_values(pb);
     };
 
-    // ---- the steps, two sets of LDS buffers and two sets of registers: while step i is computed, step i + 1
-    // sits in registers (asked for an iteration ago, stored to the LDS after the computing), step i + 2 is
-    // on its way from memory and the pages of step i + 3 are looked up.  One barrier a step.
-    Where wh_;
-    Pieces pa, pb_;
-    lookup(wh_, blk0);
-    fetch(pa, wh_);                                    // step 0
-    lookup(wh_, blk0 + FK);
-    fetch(pb_, wh_);                                   // step 1 (clamped into the row if there is none)
-    lookup(wh_, blk0 + 2 * FK);
-    __syncthreads();                                   // the previous stretch is done with the buffers
-    stash(pa, 0, key_of(blk0));
-    __syncthreads();
     const int mine_off = wk * PF_BK;                   // this wave's block within a step
     auto mine = [&](int blk) { return blk <= wave_kmax && (blk + PF_BK > wave_kmin || (KEEP && blk < keep)); };
-    for (int blk = blk0; blk <= last_x; blk += 2 * FK) {       // every condition is uniform over the workgroup
-      // step blk from set 0; pb_ holds step blk + FK; pa is free for step blk + 2 FK
-      if (blk + 2 * FK <= last_x) {
-        fetch(pa, wh_);
-        lookup(wh_, blk + 3 * FK);
+    if constexpr (PF_DIRECT) {
+      // ---- the steps, a ring of sets of buffers: while step i is computed, the SETS - 1 after it are on their way.  One
+      // barrier a step: behind it everybody's loads of step i have landed and everybody is done with step i - 1.
+      constexpr int SETS = pf_sets(KS);
+      const int steps = (last_x - blk0) / FK + 1;
+      __syncthreads();                                 // the previous stretch is done with the buffers
+      find_page(blk0);
+      for (int i = 0; i < SETS - 1; ++i)
+        if (i < steps) bring(blk0 + i * FK, i);
+      load_queries();
+      // waited for here: a wait at their first use, within the loop, would be one for every load on its way, each time
+#pragma unroll
+      for (int ks = 0; ks < KS16; ++ks) asm volatile("" : "+v"(qf[ks].q.x), "+v"(qf[ks].q.y), "+v"(qf[ks].q.z), "+v"(qf[ks].q.w));
+      int set = 0;
+      for (int i = 0; i < steps; ++i) {
+        if (i + SETS - 1 <= steps) MIE_VMCNT((SETS - 2) * LOADS);
+        else MIE_VMCNT(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int blk = key_of(blk0 + i * FK) + mine_off;
+        if (i + SETS - 1 < steps) bring(blk0 + (i + SETS - 1) * FK, set == 0 ? SETS - 1 : set - 1);
+        if (mine(blk)) compute(set, blk);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // this wave has read the set before the next barrier
+        set = set + 1 < SETS ? set + 1 : 0;
       }
-      if (mine(key_of(blk) + mine_off)) compute(0, key_of(blk) + mine_off);
-      if (blk + FK > last_x) break;
-      stash(pb_, 1, key_of(blk + FK));
+    } else {
+      // ---- the steps, two sets of LDS buffers and two sets of registers: while step i is computed, step i + 1
+      // sits in registers (asked for an iteration ago, stored to the LDS after the computing), step i + 2 is
+      // on its way from memory and the pages of step i + 3 are looked up.  One barrier a step.
+      Where wh_;
+      Pieces pa, pb_;
+      lookup(wh_, blk0);
+      fetch(pa, wh_);                                    // step 0
+      lookup(wh_, blk0 + FK);
+      fetch(pb_, wh_);                                   // step 1 (clamped into the row if there is none)
+      lookup(wh_, blk0 + 2 * FK);
+      __syncthreads();                                   // the previous stretch is done with the buffers
+      stash(pa, 0, key_of(blk0));
       __syncthreads();
-      // step blk + FK from set 1; pa holds step blk + 2 FK; pb_ is free for step blk + 3 FK
-      if (blk + 3 * FK <= last_x) {
-        fetch(pb_, wh_);
-        lookup(wh_, blk + 4 * FK);
+      for (int blk = blk0; blk <= last_x; blk += 2 * FK) {       // every condition is uniform over the workgroup
+        // step blk from set 0; pb_ holds step blk + FK; pa is free for step blk + 2 FK
+        if (blk + 2 * FK <= last_x) {
+          fetch(pa, wh_);
+          lookup(wh_, blk + 3 * FK);
+        }
+        if (mine(key_of(blk) + mine_off)) compute(0, key_of(blk) + mine_off);
+        if (blk + FK > last_x) break;
+        stash(pb_, 1, key_of(blk + FK));
+        __syncthreads();
+        // step blk + FK from set 1; pa holds step blk + 2 FK; pb_ is free for step blk + 3 FK
+        if (blk + 3 * FK <= last_x) {
+          fetch(pb_, wh_);
+          lookup(wh_, blk + 4 * FK);
+        }
+        if (mine(key_of(blk + FK) + mine_off)) compute(1, key_of(blk + FK) + mine_off);
+        if (blk + 2 * FK <= last_x) stash(pa, 0, key_of(blk + 2 * FK));
+        __syncthreads();
       }
-      if (mine(key_of(blk + FK) + mine_off)) compute(1, key_of(blk + FK) + mine_off);
-      if (blk + 2 * FK <= last_x) stash(pa, 0, key_of(blk + 2 * FK));
-      __syncthreads();
     }
 
     if (KS == 2) {
       // The halves join: the second half's state goes through the LDS (item i of lane l at 4 (64 i + l), a
       // region a wave), the first half rescales both to the common maximum.  l and O are per-lane partial
       // sums, m is the same in a query's two lanes.
-      static_assert(KS == 1 || SUB_WAVES * 64 * (2 + 16 * DT32) * 4 <= 2 * KS * PF_BUF, "the halves' exchange must fit the buffers");
+      static_assert(KS == 1 || SUB_WAVES * 64 * (2 + 16 * DT32) * 4 <= pf_lds_bytes(KS), "the halves' exchange must fit the buffers");
       float* xch = reinterpret_cast<float*>(pf_lds) + wsub * (64 * (2 + 16 * DT32)) + lane;
       __syncthreads();                                 // everybody is done with the keys and values
       if (wk == 1) {
@@ -684,16 +820,16 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   int rc = 0;
   const bool plain = !sigmoid && !dist_bias && keep == 0 && !chunked;
   if constexpr (PF_MAX_WAVES == 8) {
-    if (kind == EIGHT_QUERIES && dist_bias) rc = launch(prefill_attention_kernel<8, 1, false, true>, 8, 2 * PF_BUF);
-    if (kind == EIGHT_KEYS && dist_bias) rc = launch(prefill_attention_kernel<8, 2, false, true>, 8, 4 * PF_BUF);
-    if (kind == EIGHT_QUERIES && plain) rc = launch(prefill_attention_kernel<8, 1, false>, 8, 2 * PF_BUF);
-    if (kind == EIGHT_KEYS && plain) rc = launch(prefill_attention_kernel<8, 2, false>, 8, 4 * PF_BUF);
-    if (kind == EIGHT_QUERIES && chunked) rc = launch(prefill_attention_kernel<8, 1, false, false, false, true>, 8, 2 * PF_BUF);
-    if (kind == EIGHT_KEYS && chunked) rc = launch(prefill_attention_kernel<8, 2, false, false, false, true>, 8, 4 * PF_BUF);
-    if (kind == EIGHT_QUERIES && keep > 0) rc = launch(prefill_attention_kernel<8, 1, false, false, true>, 8, 2 * PF_BUF);
-    if (kind == EIGHT_KEYS && keep > 0) rc = launch(prefill_attention_kernel<8, 2, false, false, true>, 8, 4 * PF_BUF);
-    if (kind == EIGHT_QUERIES && sigmoid) rc = launch(prefill_attention_kernel<8, 1, true>, 8, 2 * PF_BUF);
-    if (kind == EIGHT_KEYS && sigmoid) rc = launch(prefill_attention_kernel<8, 2, true>, 8, 4 * PF_BUF);
+    if (kind == EIGHT_QUERIES && dist_bias) rc = launch(prefill_attention_kernel<8, 1, false, true>, 8, pf_lds_bytes(1));
+    if (kind == EIGHT_KEYS && dist_bias) rc = launch(prefill_attention_kernel<8, 2, false, true>, 8, pf_lds_bytes(2));
+    if (kind == EIGHT_QUERIES && plain) rc = launch(prefill_attention_kernel<8, 1, false>, 8, pf_lds_bytes(1));
+    if (kind == EIGHT_KEYS && plain) rc = launch(prefill_attention_kernel<8, 2, false>, 8, pf_lds_bytes(2));
+    if (kind == EIGHT_QUERIES && chunked) rc = launch(prefill_attention_kernel<8, 1, false, false, false, true>, 8, pf_lds_bytes(1));
+    if (kind == EIGHT_KEYS && chunked) rc = launch(prefill_attention_kernel<8, 2, false, false, false, true>, 8, pf_lds_bytes(2));
+    if (kind == EIGHT_QUERIES && keep > 0) rc = launch(prefill_attention_kernel<8, 1, false, false, true>, 8, pf_lds_bytes(1));
+    if (kind == EIGHT_KEYS && keep > 0) rc = launch(prefill_attention_kernel<8, 2, false, false, true>, 8, pf_lds_bytes(2));
+    if (kind == EIGHT_QUERIES && sigmoid) rc = launch(prefill_attention_kernel<8, 1, true>, 8, pf_lds_bytes(1));
+    if (kind == EIGHT_KEYS && sigmoid) rc = launch(prefill_attention_kernel<8, 2, true>, 8, pf_lds_bytes(2));
   }
   if (kind == FOUR && dist_bias) rc = launch(prefill_attention_kernel<4, 1, false, true>, 4, 2 * PF_BUF);
   if (kind == FOUR && chunked) rc = launch(prefill_attention_kernel<4, 1, false, false, false, true>, 4, 2 * PF_BUF);

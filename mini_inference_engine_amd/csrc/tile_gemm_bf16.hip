@@ -20,21 +20,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 enum { TG_F32, TG_SWIGLU };
 
-// 16 bytes a lane from base + offset into the LDS at byte `at` + 16 lane.  The compiler does not see that memory is on its
-// way: the waits are the kernel's own (MIE_VMCNT and a barrier before a stage is read).  m0 is an output, so that the
-// compiler keeps nothing of its own there; as an input operand it costs the loop its order of moves and loads (2,048 rows of
-// [11264, 2048] 90.1 -> 93.0 us).
-__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t at) {
-  uint32_t written;
-  asm volatile(
-    "s_mov_b32 m0, %1\n\t"
-    "s_nop 0\n\t"
-    "global_load_lds_dwordx4 %2, %3"
-    : "={m0}"(written)
-    : "s"(at), "v"(offset), "s"(base)
-    : "memory");
-}
-
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return (uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(a)) | ((uint32_t)__builtin_bit_cast(uint16_t, __float2bfloat16(b)) << 16);
 }
@@ -94,7 +79,7 @@ tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
     const char* wb = reinterpret_cast<const char*>(W) + (size_t)(st0 + s) * 128;
     const uint32_t base = lds0 + (s % STAGES) * STAGE;
 #pragma unroll
-    for (int j = 0; j < L; ++j) load_to_lds(is_w[j] ? wb : xb, off[j], base + at[j]);
+    for (int j = 0; j < L; ++j) mie_load_to_lds(is_w[j] ? wb : xb, off[j], base + at[j]);
   };
   f32x4 acc[4][4];
 #pragma unroll
