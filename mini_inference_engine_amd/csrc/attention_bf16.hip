@@ -69,7 +69,8 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
   const int s = blockIdx.z;
   const int G = Hq / Hkv;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // the same in all lanes: kept in a scalar register
   const int col = lane & 15, kb = lane >> 4;
   const int g = ht * 16 + col;
   const bool head_ok = g < G;
@@ -90,38 +91,48 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
     Frag a[2][KS];      // keys: 16 keys x 32 dims each
     Frag va[DT];        // values: 16 dims x 32 keys each, in the order the probabilities sit in registers
   };
+  // Pages hold a multiple of 16 keys, so each half of a block lies in one page: looked up through the scalar unit, a block
+  // ahead.  Looked up by vector loads in front of a block's own, they made every block wait for all of the one before (vector
+  // loads return in order), and nothing was on its way beside the block being computed.
   const int last_page = max_blocks - 1;
-  auto load_block = [&](KeyBlock& B, int blk) {
+  const int page_shift = (page & (page - 1)) == 0 ? __builtin_ctz(page) : -1;
+  struct Places {
+    int pg[2], off[2];  // page and first key in it of keys 0 .. 15 and 16 .. 31 of a block
+  };
+  auto find = [&](int blk) {
+    Places p;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int key = blk + 16 * t + col;
-      int pi = key / page;
-      pi = pi < last_page ? pi : last_page;
-      const bf16* kp = k_cache + (((size_t)bt[pi] * Hkv + kvh) * page + key % page) * D;
+      const int key = blk + 16 * t, pi = page_shift >= 0 ? key >> page_shift : key / page;
+      p.pg[t] = bt[pi < last_page ? pi : last_page];
+      p.off[t] = key - pi * page;
+    }
+    return p;
+  };
+  auto load_block = [&](KeyBlock& B, const Places& p) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16* kp = k_cache + (((size_t)p.pg[t] * Hkv + kvh) * page + p.off[t]) * D;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const int d0 = ks * 32 + kb * 8;
-        B.a[t][ks].q = *reinterpret_cast<const uint4*>(kp + (d0 < D ? d0 : 0));
+        B.a[t][ks].q = *reinterpret_cast<const uint4*>(kp + (col * D + (d0 < D ? d0 : 0)));
       }
     }
-    const int k0 = blk + 4 * kb, k1 = blk + 16 + 4 * kb;
-    int p0 = k0 / page, p1 = k1 / page;
-    p0 = p0 < last_page ? p0 : last_page;
-    p1 = p1 < last_page ? p1 : last_page;
-    const bf16* v0 = v_cache + ((size_t)bt[p0] * Hkv + kvh) * D * page + k0 % page;
-    const bf16* v1 = v_cache + ((size_t)bt[p1] * Hkv + kvh) * D * page + k1 % page;
+    const bf16* v0 = v_cache + ((size_t)p.pg[0] * Hkv + kvh) * D * page + p.off[0];
+    const bf16* v1 = v_cache + ((size_t)p.pg[1] * Hkv + kvh) * D * page + p.off[1];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const size_t drow = (size_t)(dt * 16 + col) * page;
-      B.va[dt].h[0] = *reinterpret_cast<const uint2*>(v0 + drow);
-      B.va[dt].h[1] = *reinterpret_cast<const uint2*>(v1 + drow);
+      const int at = (dt * 16 + col) * page + 4 * kb;
+      B.va[dt].h[0] = *reinterpret_cast<const uint2*>(v0 + at);
+      B.va[dt].h[1] = *reinterpret_cast<const uint2*>(v1 + at);
     }
   };
   constexpr bool AHEAD = D <= 128;          // two blocks in registers; larger heads have no room for it
   KeyBlock b0, b1;
   const int pos_raw = positions[b];
   int begin0 = s * partition;               // the split's first key when there is no window
-  if (AHEAD && !CHUNK && window <= 0 && (!SIG || chunk <= 0)) load_block(b0, begin0 + BLOCK_KEYS * wave);
+  if (AHEAD && !CHUNK && window <= 0 && (!SIG || chunk <= 0)) load_block(b0, find(begin0 + BLOCK_KEYS * wave));
 
   const int pos = pos_raw;
   if (FROM_SUMS) {
@@ -302,19 +313,15 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
         }
         mx = fmaxf(mx, sv[t * 4 + i]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);                   // finite: every block taken holds a visible key
-    const float alpha = exp2f(m - m_new);
+    const float m_new = fmaxf(m, quad_max(mx));         // finite: every block taken holds a visible key
+    const float alpha = fast_exp2(m - m_new);
     float p[8], rs = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      p[j] = ok[j] ? exp2f(sv[j] - m_new) : 0.f;
+      p[j] = ok[j] ? fast_exp2(sv[j] - m_new) : 0.f;
       rs += p[j];
     }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l = l * alpha + rs;
+    l = l * alpha + rs;                                 // of this lane's keys; the head's four lanes join after the last block
     m = m_new;
     Frag pb;
 #pragma unroll
@@ -341,17 +348,20 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   constexpr int STEP = BLOCK_KEYS * NW;     // keys from one block of a wave to its next
   const int first = begin + BLOCK_KEYS * wave;
   if (AHEAD) {
-    if (CHUNK || window > 0 || (SIG && chunk > 0)) load_block(b0, key_of(first));  // with a window the split's start had to wait for the row's length
+    if (CHUNK || window > 0 || (SIG && chunk > 0)) load_block(b0, find(key_of(first)));  // with a window the split's start had to wait for the row's length
     const int part_end = begin + partition;   // nothing is asked for beyond the split's own keys
+    Places next = find(key_of(first + STEP));
     for (int blk = first; blk < end; blk += 2 * STEP) {
-      if (blk + STEP < part_end) load_block(b1, key_of(blk + STEP));           // in flight while block 0 is computed
+      if (blk + STEP < part_end) load_block(b1, next);                         // in flight while block 0 is computed
+      next = find(key_of(blk + 2 * STEP));
       compute(b0, key_of(blk));
-      if (blk + 2 * STEP < part_end) load_block(b0, key_of(blk + 2 * STEP));
+      if (blk + 2 * STEP < part_end) load_block(b0, next);
+      next = find(key_of(blk + 3 * STEP));
       if (blk + STEP < end) compute(b1, key_of(blk + STEP));
     }
   } else {
     for (int blk = first; blk < end; blk += STEP) {
-      load_block(b0, key_of(blk));
+      load_block(b0, find(key_of(blk)));
       compute(b0, key_of(blk));
     }
   }
@@ -360,6 +370,8 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   if constexpr (SIG) {
     m = 0.f;
     l = wave == 0 ? 1.f : 0.f;
+  } else {
+    l = quad_sum(l);
   }
   if (kb == 0) {
     s_m[wave][col] = m;
