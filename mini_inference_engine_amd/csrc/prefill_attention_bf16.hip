@@ -44,8 +44,8 @@
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 struct __attribute__((packed, aligned(4))) Run4 { float a, b, c, d; };      // four table entries in a row, 4-byte aligned
 
-// Waves a workgroup, at head sizes up to 128 (above, eight waves do not fit the registers: always 4):
-// 8 over twice the queries (twice the queries share each block that is brought in: at head size 128 and 8,192
+// Waves a workgroup, at head sizes up to 128 (above, eight waves do not fit the registers: always 4; at 128 sometimes, two
+// workgroups a compute unit: see the launcher): 8 over twice the queries (twice the queries share each block that is brought in: at head size 128 and 8,192
 // tokens 0.82 against 0.40 PFLOP/s); for rows so short that the grid of 4 waves gives no more workgroups than
 // there are compute units, 8 in two halves over the keys on that grid: a wave's chain of blocks is half as
 // long and every SIMD has two waves (2,048 tokens at head size 64: 47 against 56 us).  Both kinds of eight
@@ -64,9 +64,10 @@ constexpr int PF_BUF = PF_KBYTES + PF_VBYTES;       // one buffer: keys, then va
 constexpr int PF_KPIECES = PF_BK * (D / 16);        // 32-byte pieces: 16 dims of one key
 constexpr int PF_VPIECES = D * (PF_BK / 16);        //                 16 keys of one dim
 constexpr int PF_PIECES = PF_KPIECES + PF_VPIECES;
-// sets of buffers for steps of `halves` blocks: one being computed, the others on their way
-constexpr int pf_sets(int halves) { return PF_DIRECT && 3 * halves * PF_BUF <= 96 * 1024 ? 3 : 2; }
-constexpr int pf_lds_bytes(int halves) { return pf_sets(halves) * halves * PF_BUF; }
+// sets of buffers for steps of `halves` blocks: one being computed, the others on their way (workgroups of four waves leave
+// room for a second one)
+constexpr int pf_sets(int halves, int waves) { return PF_DIRECT && 3 * halves * PF_BUF <= (waves == 4 ? 64 : 96) * 1024 ? 3 : 2; }
+constexpr int pf_lds_bytes(int halves, int waves) { return pf_sets(halves, waves) * halves * PF_BUF; }
 
 // max of three numbers none of which is a NaN, as one instruction
 __device__ __forceinline__ float max3_nn(float a, float b, float c) {
@@ -75,10 +76,28 @@ __device__ __forceinline__ float max3_nn(float a, float b, float c) {
   return r;
 }
 
+// max of two, without the instruction the compiler puts before its own for signalling NaNs
+__device__ __forceinline__ float max2_nn(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // max / sum over the two lanes l, l ^ 32 (one query's lanes)
 __device__ __forceinline__ float pair_max(float x) {      // no NaN among the values
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return max_nn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  return max2_nn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// the largest of 32 numbers none of which is a NaN, by 16 instructions
+__device__ __forceinline__ float max32_nn(const f32x16 (&s)[2]) {
+  float t[12];
+#pragma unroll
+  for (int e = 0; e < 10; ++e)
+    t[e] = max3_nn(s[3 * e / 16][3 * e % 16], s[(3 * e + 1) / 16][(3 * e + 1) % 16], s[(3 * e + 2) / 16][(3 * e + 2) % 16]);
+  t[10] = s[1][14];
+  t[11] = s[1][15];
+  const float a = max3_nn(t[0], t[1], t[2]), b = max3_nn(t[3], t[4], t[5]), c = max3_nn(t[6], t[7], t[8]), d = max3_nn(t[9], t[10], t[11]);
+  return max2_nn(max3_nn(a, b, c), d);
 }
 __device__ __forceinline__ float pair_sum(float x) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -89,7 +108,7 @@ __device__ __forceinline__ float pair_sum(float x) {
 // brings 128 keys in, each half computes its 64) and join their results at the end: half the blocks a wave
 // for rows too short to give every SIMD two waves otherwise.
 template <int PF_WAVES, int KS, bool SIG, bool DB = false, bool KEEP = false, bool CHUNK = false>
-__global__ void __launch_bounds__(PF_WAVES * 64)
+__global__ void __launch_bounds__(PF_WAVES * 64, PF_DIRECT && PF_WAVES == 4 ? 2 : 1)
 prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* __restrict__ k_cache,
                          const bf16* __restrict__ v_cache, bf16* __restrict__ out,
                          const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ row_start,
@@ -484,12 +503,13 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
             for (int dt = 0; dt < DT32; ++dt) va[dt][t].q = values(dt, t);
           if (blk + PF_BK - 1 > vmax || blk < vmin) {
             // values that nobody may look at (see stash): their weight is 0, but 0 * NaN would reach the sum
-            auto dead = [&](int key) { return key > vmax || (key < vmin && !(KEEP && key < keep)); };
+            const int first_key = vmin - blk - 8 * g, last_key = vmax - blk - 8 * g, kept = keep - blk - 8 * g;
+            auto dead = [&](int key) { return key > last_key || (key < first_key && !(KEEP && key < kept)); };
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const int key = blk + 16 * t + 8 * g + 2 * e;
+                const int key = 16 * t + 2 * e;
                 const uint32_t bits = (dead(key) ? 0u : 0x0000FFFFu) | (dead(key + 1) ? 0u : 0xFFFF0000u);
 #pragma unroll
                 for (int dt = 0; dt < DT32; ++dt) va[dt][t].w[e] &= bits;
@@ -534,12 +554,13 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
           const int hi = tile_ok ? qpos : -1;                  // a tile that does not exist sees nothing
           int lo = window > 0 ? hi - window + 1 : 0;
           lo = lo > q_lo ? lo : q_lo;
+          const int first_key = lo - blk - key_off(0, 0), last_key = hi - blk - key_off(0, 0);
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-              const int key = blk + key_off(u, i);
-              S[u][i] = key >= lo && key <= hi ? S[u][i] : 0.f;
+              const int key = key_off(u, i) - key_off(0, 0);
+              S[u][i] = key >= first_key && key <= last_key ? S[u][i] : 0.f;
             }
         }
         Frag pb[4];
@@ -552,13 +573,9 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
       }
       float alpha;
       if (whole) {
-        float mx[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          mx[e] = max3_nn(max3_nn(S[0][4 * e], S[0][4 * e + 1], S[0][4 * e + 2]),
-                          max3_nn(S[0][4 * e + 3], S[1][4 * e], S[1][4 * e + 1]), max_nn(S[1][4 * e + 2], S[1][4 * e + 3]));
-        const float mxx = pair_max(max_nn(max_nn(mx[0], mx[1]), max_nn(mx[2], mx[3])));
-        const float m_new = max_nn(m, mxx * sl2);
+        // the first to read the products' results is assembly, before which the compiler puts no waits: at most 19 are asked for
+        asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(S[0]), "+v"(S[1]));
+        const float m_new = max2_nn(m, pair_max(max32_nn(S)) * sl2);
         alpha = fast_exp2(m - m_new);
         m = m_new;
 #pragma unroll
@@ -569,18 +586,17 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
         const int hi = tile_ok ? qpos : -1;                    // a tile that does not exist sees nothing
         int lo = window > 0 ? hi - window + 1 : 0;
         if constexpr (CHUNK) lo = lo > q_lo ? lo : q_lo;
-        float mx = -INFINITY;
+        // counted from the lane's first key, so that what a score is compared with stands in the instruction
+        const int first_key = lo - blk - key_off(0, 0), last_key = hi - blk - key_off(0, 0), kept = keep - blk - key_off(0, 0);
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const int key = blk + key_off(u, i);
-            const bool ok = (key >= lo || (KEEP && key < keep)) && key <= hi;
+            const int key = key_off(u, i) - key_off(0, 0);
+            const bool ok = (key >= first_key || (KEEP && key < kept)) && key <= last_key;
             S[u][i] = ok ? S[u][i] : -INFINITY;
-            mx = max_nn(mx, S[u][i]);
           }
-        mx = pair_max(mx);
-        const float m_new = max_nn(m, mx * sl2);
+        const float m_new = max2_nn(m, pair_max(max32_nn(S)) * sl2);
         // a query may see none of this block's keys (it lies before the block, or the block before its window)
         alpha = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
         m = m_new;
@@ -616,7 +632,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
     if constexpr (PF_DIRECT) {
       // ---- the steps, a ring of sets of buffers: while step i is computed, the SETS - 1 after it are on their way.  One
       // barrier a step: behind it everybody's loads of step i have landed and everybody is done with step i - 1.
-      constexpr int SETS = pf_sets(KS);
+      constexpr int SETS = pf_sets(KS, PF_WAVES);
       const int steps = (last_x - blk0) / FK + 1;
       __syncthreads();                                 // the previous stretch is done with the buffers
       find_page(blk0);
@@ -677,7 +693,7 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
       // The halves join: the second half's state goes through the LDS (item i of lane l at 4 (64 i + l), a
       // region a wave), the first half rescales both to the common maximum.  l and O are per-lane partial
       // sums, m is the same in a query's two lanes.
-      static_assert(KS == 1 || SUB_WAVES * 64 * (2 + 16 * DT32) * 4 <= pf_lds_bytes(KS), "the halves' exchange must fit the buffers");
+      static_assert(KS == 1 || SUB_WAVES * 64 * (2 + 16 * DT32) * 4 <= pf_lds_bytes(KS, PF_WAVES), "the halves' exchange must fit the buffers");
       float* xch = reinterpret_cast<float*>(pf_lds) + wsub * (64 * (2 + 16 * DT32)) + lane;
       __syncthreads();                                 // everybody is done with the keys and values
       if (wk == 1) {
@@ -783,7 +799,10 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   //     compute units and twice the chain (512 tokens of 32 / 4 heads of 64 19 -> 14, of 32 / 8 of 128 behind 4,096 283 -> 153);
   //   else above head size 64 twice the queries, a stretch a workgroup, while that is: a step brings half the keys in for the same
   //     products (2,048 tokens of 32 / 8 of 128 alone 87 in halves and pairs, 84; behind 4,096 344 -> 229; at head size 64
-  //     42 -> 55 and 150 -> 146, so not there);
+  //     42 -> 55 and 150 -> 146, so not there).  At 128 that is four waves a workgroup instead, two workgroups a compute unit: they
+  //     meet at no common barrier, so one's matrix instructions run beside the other's softmax (2,048 tokens alone 72 -> 62, behind
+  //     4,096 198 -> 190, 1,100 behind 4,000 151 -> 137, 32 / 32 heads 73 -> 62; with four workgroups a compute unit 124 -> 126, 4,096
+  //     tokens 153 -> 168, so not there; at 64, 2,048 tokens 38 -> 43);
   //   else two halves in pairs, while they are (two rounds of it, the second half empty, are slower: 2,560 tokens of 32 / 4 of 64
   //     95 us against 45 for 2,048);
   //   else twice the queries in pairs.
@@ -794,7 +813,7 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   if (PF_MAX_WAVES == 8) {
     const long units = compute_units[dev];
     if (plan(4, false, &waves_h, &grid) <= units) { kind = EIGHT_KEYS; paired = false; }
-    else if (D > 64 && plan(8, false, &waves_h, &grid) <= units) { kind = EIGHT_QUERIES; paired = false; }
+    else if (D > 64 && plan(8, false, &waves_h, &grid) <= units) { kind = PF_DIRECT ? FOUR : EIGHT_QUERIES; paired = false; }
     else kind = plan(4, true, &waves_h, &grid) <= units ? EIGHT_KEYS : EIGHT_QUERIES;
   }
   plan(kind == EIGHT_QUERIES ? 8 : 4, paired, &waves_h, &grid);
@@ -820,22 +839,22 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   int rc = 0;
   const bool plain = !sigmoid && !dist_bias && keep == 0 && !chunked;
   if constexpr (PF_MAX_WAVES == 8) {
-    if (kind == EIGHT_QUERIES && dist_bias) rc = launch(prefill_attention_kernel<8, 1, false, true>, 8, pf_lds_bytes(1));
-    if (kind == EIGHT_KEYS && dist_bias) rc = launch(prefill_attention_kernel<8, 2, false, true>, 8, pf_lds_bytes(2));
-    if (kind == EIGHT_QUERIES && plain) rc = launch(prefill_attention_kernel<8, 1, false>, 8, pf_lds_bytes(1));
-    if (kind == EIGHT_KEYS && plain) rc = launch(prefill_attention_kernel<8, 2, false>, 8, pf_lds_bytes(2));
-    if (kind == EIGHT_QUERIES && chunked) rc = launch(prefill_attention_kernel<8, 1, false, false, false, true>, 8, pf_lds_bytes(1));
-    if (kind == EIGHT_KEYS && chunked) rc = launch(prefill_attention_kernel<8, 2, false, false, false, true>, 8, pf_lds_bytes(2));
-    if (kind == EIGHT_QUERIES && keep > 0) rc = launch(prefill_attention_kernel<8, 1, false, false, true>, 8, pf_lds_bytes(1));
-    if (kind == EIGHT_KEYS && keep > 0) rc = launch(prefill_attention_kernel<8, 2, false, false, true>, 8, pf_lds_bytes(2));
-    if (kind == EIGHT_QUERIES && sigmoid) rc = launch(prefill_attention_kernel<8, 1, true>, 8, pf_lds_bytes(1));
-    if (kind == EIGHT_KEYS && sigmoid) rc = launch(prefill_attention_kernel<8, 2, true>, 8, pf_lds_bytes(2));
+    if (kind == EIGHT_QUERIES && dist_bias) rc = launch(prefill_attention_kernel<8, 1, false, true>, 8, pf_lds_bytes(1, 8));
+    if (kind == EIGHT_KEYS && dist_bias) rc = launch(prefill_attention_kernel<8, 2, false, true>, 8, pf_lds_bytes(2, 8));
+    if (kind == EIGHT_QUERIES && plain) rc = launch(prefill_attention_kernel<8, 1, false>, 8, pf_lds_bytes(1, 8));
+    if (kind == EIGHT_KEYS && plain) rc = launch(prefill_attention_kernel<8, 2, false>, 8, pf_lds_bytes(2, 8));
+    if (kind == EIGHT_QUERIES && chunked) rc = launch(prefill_attention_kernel<8, 1, false, false, false, true>, 8, pf_lds_bytes(1, 8));
+    if (kind == EIGHT_KEYS && chunked) rc = launch(prefill_attention_kernel<8, 2, false, false, false, true>, 8, pf_lds_bytes(2, 8));
+    if (kind == EIGHT_QUERIES && keep > 0) rc = launch(prefill_attention_kernel<8, 1, false, false, true>, 8, pf_lds_bytes(1, 8));
+    if (kind == EIGHT_KEYS && keep > 0) rc = launch(prefill_attention_kernel<8, 2, false, false, true>, 8, pf_lds_bytes(2, 8));
+    if (kind == EIGHT_QUERIES && sigmoid) rc = launch(prefill_attention_kernel<8, 1, true>, 8, pf_lds_bytes(1, 8));
+    if (kind == EIGHT_KEYS && sigmoid) rc = launch(prefill_attention_kernel<8, 2, true>, 8, pf_lds_bytes(2, 8));
   }
-  if (kind == FOUR && dist_bias) rc = launch(prefill_attention_kernel<4, 1, false, true>, 4, 2 * PF_BUF);
-  if (kind == FOUR && chunked) rc = launch(prefill_attention_kernel<4, 1, false, false, false, true>, 4, 2 * PF_BUF);
-  if (kind == FOUR && keep > 0) rc = launch(prefill_attention_kernel<4, 1, false, false, true>, 4, 2 * PF_BUF);
-  if (kind == FOUR && plain) rc = launch(prefill_attention_kernel<4, 1, false>, 4, 2 * PF_BUF);
-  if (kind == FOUR && sigmoid) rc = launch(prefill_attention_kernel<4, 1, true>, 4, 2 * PF_BUF);
+  if (kind == FOUR && dist_bias) rc = launch(prefill_attention_kernel<4, 1, false, true>, 4, pf_lds_bytes(1, 4));
+  if (kind == FOUR && chunked) rc = launch(prefill_attention_kernel<4, 1, false, false, false, true>, 4, pf_lds_bytes(1, 4));
+  if (kind == FOUR && keep > 0) rc = launch(prefill_attention_kernel<4, 1, false, false, true>, 4, pf_lds_bytes(1, 4));
+  if (kind == FOUR && plain) rc = launch(prefill_attention_kernel<4, 1, false>, 4, pf_lds_bytes(1, 4));
+  if (kind == FOUR && sigmoid) rc = launch(prefill_attention_kernel<4, 1, true>, 4, pf_lds_bytes(1, 4));
   if (rc) return rc;
   MIE_CHECK_LAUNCH("prefill_attention");
   return 0;
