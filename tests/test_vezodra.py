@@ -522,6 +522,28 @@ def test_conv_and_joined_norm_kernels(hip, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, K", [(2048, 4), (64, 1), (1028, 6), (2052, 4)])
+def test_joined_norms_of_many_tokens(hip, dtype, width, K):
+    """Steps of 1,024 tokens and more: four tokens a workgroup up to a width of 2,048 (2,052: one), rows that begin and end
+    anywhere in a workgroup's four, rows of one token and rows shorter than the convolution among them, a last workgroup that is not
+    full."""
+    ops, g = hip[dtype], torch.Generator().manual_seed(width + K)
+    step = FakeStep([1, 700, 1, 2, 3, 1, 330, 5], [4, 1, 3, 5, 2, 6, 8, 7])
+    stream = _rand((step.num_tokens, width), torch.float32, g, 2.0)
+    w1, w2 = _rand((width,), torch.float32, g) + 1, _rand((width,), torch.float32, g) + 1
+    taps, tail = _rand((width, K), torch.float32, g, 0.5), _rand((9, max(1, K - 1), width), torch.float32, g)
+    want_tail = tail.cpu().clone()
+    hn = ref.ref_add_rmsnorm(None, stream.cpu(), w1.cpu(), 1e-5, torch.float32)
+    want = ref.ref_residual_conv(hn, taps.cpu(), want_tail, step.host["row_start"], step.host["state_slots"], dtype)
+    x, y = ops.norm_pair_conv(stream, w1, w2, 1e-5, taps, tail, step)
+    close(x, want, TOL[dtype], "convolved")
+    close(y, ref.ref_add_rmsnorm(None, stream.cpu(), w2.cpu(), 1e-5, dtype), TOL[dtype], "second norm")
+    if K > 1:
+        close(tail, want_tail, 3e-6, "tail")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_preparation_kernels(hip, dtype):
     ops, g = hip[dtype], torch.Generator().manual_seed(2)
     cases = ((4, 2, 16, 24, 32, 4, "half", True, False, True, 37), (6, 3, 32, 32, 32, 8, "interleaved", False, True, False, 3),
