@@ -116,6 +116,138 @@ qkv_finish_kernel(FinishArgs a) {
   }
 }
 
+// The same where everything comes in pieces of 8 numbers: a thread a piece (four pairs that turn, or 8 numbers that do not, or
+// 8 values), up to ITERS of them, all asked for before the norms' sums.  The kernel above takes a wave a head and one head after
+// the other, each a trip to memory with half the lanes: nine in a row at 32 + 4 heads of 64 and one token a workgroup, which is what
+// bounded it.  2,048 tokens (MI355X, us): 32 + 4 heads of 64 with norms 33.8 / 16.2, 16 + 4 of 128 without 21.8 / 14.0.
+__device__ __forceinline__ void store4(float* p, const float* v) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void store4(bf16* p, const float* v) {
+  const bf16 o[4] = {__float2bfloat16(v[0]), __float2bfloat16(v[1]), __float2bfloat16(v[2]), __float2bfloat16(v[3])};
+  *reinterpret_cast<uint2*>(p) = *reinterpret_cast<const uint2*>(o);
+}
+
+template <typename TO, int ITERS>
+__global__ void __launch_bounds__(512)
+qkv_finish_pieces_kernel(FinishArgs a) {
+  __shared__ float parts[2][8];
+  extern __shared__ __align__(16) float cs[];   // cos [nf], sin [nf]
+  const int t = blockIdx.x, per_head = a.P >> 3, heads = a.Hq + a.Hkv, turned = a.nf >> 2;
+  const float* __restrict__ row = a.sums + (size_t)t * a.ld;
+  const int pos = a.positions[t], slot = a.slots[t];
+  float x[ITERS][8];
+  int head[ITERS], d1[ITERS], d2[ITERS];        // head: queries, keys, values; first numbers of the piece's halves; -1: none
+  float ssq = 0.f, ssk = 0.f, head_ss[ITERS];
+#pragma unroll
+  for (int n = 0; n < ITERS; ++n) {
+    const int job = threadIdx.x + n * blockDim.x, h = job / per_head, e = job - h * per_head;
+    head[n] = h < heads + a.Hkv ? h : -1;
+    const bool value = h >= heads, pairs = !value && e < turned;
+    d1[n] = pairs && a.layout == LAYOUT_HALF ? 4 * e : !value && !pairs ? 2 * a.nf + 8 * (e - turned) : 8 * e;
+    d2[n] = pairs && a.layout == LAYOUT_HALF ? d1[n] + a.nf : d1[n] + 4;
+    const int size = value ? a.vdim : a.dim;
+    const int col = h < a.Hq ? a.q_col + h * a.dim : !value ? a.k_col + (h - a.Hq) * a.dim
+                  : a.v_col < 0 ? a.k_col + (h - heads) * a.dim : a.v_col + (h - heads) * a.vdim;
+    float ss = 0.f;
+    const bool there = head[n] >= 0 && d1[n] < size;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (there) {
+        const int at = col + (half ? d2[n] : d1[n]);
+        v = *reinterpret_cast<const float4*>(row + at);
+        if (a.col_bias) {
+          const float4 b = *reinterpret_cast<const float4*>(a.col_bias + at);
+          v.x += b.x, v.y += b.y, v.z += b.z, v.w += b.w;
+        }
+      }
+      x[n][4 * half] = v.x, x[n][4 * half + 1] = v.y, x[n][4 * half + 2] = v.z, x[n][4 * half + 3] = v.w;
+      ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+    }
+    head_ss[n] = ss;
+    if (h < a.Hq) ssq += ss;
+    else if (h < heads) ssk += ss;
+  }
+  for (int i = threadIdx.x; i < a.nf; i += blockDim.x) sincosf((float)pos * a.inv_freq[i], &cs[a.nf + i], &cs[i]);
+  const bool whole = !a.norm_per_head && (a.q_norm || a.k_norm);
+  if (whole) {
+    ssq = wave_sum(ssq);
+    ssk = wave_sum(ssk);
+    if ((threadIdx.x & 63) == 0) {
+      parts[0][threadIdx.x >> 6] = ssq;
+      parts[1][threadIdx.x >> 6] = ssk;
+    }
+  }
+  __syncthreads();
+  float rq = 1.f, rk = 1.f;
+  if (whole) {
+    float q = 0.f, k = 0.f;
+    for (int w = 0; w < (int)(blockDim.x + 63) >> 6; ++w) {
+      q += parts[0][w];
+      k += parts[1][w];
+    }
+    if (a.q_norm) rq = 1.0f / sqrtf(q / (float)(a.Hq * a.dim) + a.eps);
+    if (a.k_norm) rk = 1.0f / sqrtf(k / (float)(a.Hkv * a.dim) + a.eps);
+  }
+  const float temperature = a.temp_every > 0 ? 1.0f + a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.0f) : 1.0f;
+  const size_t pg = slot / a.page, off = slot % a.page;
+#pragma unroll
+  for (int n = 0; n < ITERS; ++n) {
+    float r = 1.f;
+    if (a.norm_per_head) {                      // a head's pieces lie in neighbouring lanes, a power of two of them
+      float ss = head_ss[n];
+      for (int o = per_head >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      r = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
+    }
+    const int h = head[n];
+    if (h < 0) continue;
+    if (h >= heads) {
+      TO* __restrict__ vd = (TO*)a.v_cache + ((pg * a.Hkv + (h - heads)) * a.P + d1[n]) * a.page + off;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) vd[(size_t)i * a.page] = from_float<TO>(x[n][i]);
+      continue;
+    }
+    const bool is_q = h < a.Hq;
+    const float* __restrict__ w = is_q ? a.q_norm : a.k_norm;
+    float v[8];
+    if (w && d1[n] < a.dim) {
+      if (!a.norm_per_head) {
+        w += (size_t)(is_q ? h : h - a.Hq) * a.dim;
+        r = is_q ? rq : rk;
+      }
+      const float4 w1 = *reinterpret_cast<const float4*>(w + d1[n]), w2 = *reinterpret_cast<const float4*>(w + d2[n]);
+      const float ws[8] = {w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = x[n][i] * r * ws[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = x[n][i];
+    }
+    if (d1[n] < 2 * a.nf) {
+      const int f = a.layout == LAYOUT_HALF ? d1[n] : d1[n] >> 1;
+      const float4 c = *reinterpret_cast<const float4*>(cs + f), sn = *reinterpret_cast<const float4*>(cs + a.nf + f);
+      const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float o1, o2;
+        if (a.layout == LAYOUT_HALF) {
+          rotate_pair(v[i], v[4 + i], cc[i], ss[i], o1, o2);
+          v[i] = o1, v[4 + i] = o2;
+        } else {
+          rotate_pair(v[2 * i], v[2 * i + 1], cc[i], ss[i], o1, o2);
+          v[2 * i] = o1, v[2 * i + 1] = o2;
+        }
+      }
+    }
+    const float mult = is_q ? (a.q_head_scale ? a.q_head_scale[h] * temperature : temperature) : 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= mult;
+    TO* __restrict__ dst = is_q ? (TO*)a.q_out + ((size_t)t * a.Hq + h) * a.P
+                                : (TO*)a.k_cache + ((pg * a.Hkv + (h - a.Hq)) * a.page + off) * a.P;
+    store4(dst + d1[n], v);
+    store4(dst + d2[n], v + 4);
+  }
+}
+
 // ---- projections through a short convolution
 struct ConvFinishArgs {
   const float* sums; long ld; int col;                      // queries, keys, values side by side from column ``col`` on
@@ -415,6 +547,22 @@ MIE_EXPORT int mie_qkv_finish(const float* sums, long ld, int q_col, int k_col, 
   FinishArgs a{sums, ld, q_col, k_col, v_col, q_norm, k_norm, eps, norm_per_head, inv_freq, nf, layout, q_head_scale, col_bias, temp_coef, temp_every,
                positions, slots, q_out, k_cache, v_cache, Hq, Hkv, dim, vdim, P, page};
   const size_t lds = (size_t)2 * (nf > 0 ? nf : 1) * sizeof(float);
+  // Pieces of 8 numbers where sizes and addresses allow it and the tokens fill the GPU; fewer tokens are spread over it below.
+  const int per_head = P >> 3, pieces = (Hq + 2 * Hkv) * per_head;
+  const bool aligned = !(((uintptr_t)sums | (uintptr_t)q_norm | (uintptr_t)k_norm | (uintptr_t)col_bias | (uintptr_t)q_out |
+                          (uintptr_t)k_cache) & 15) && !((ld | q_col | k_col | (v_col < 0 ? 0 : v_col)) & 3);
+  if (tokens >= 256 && aligned && !((dim | vdim | P) & 7) && !(nf & 3) && pieces <= 2048 &&
+      (!norm_per_head || ((per_head & (per_head - 1)) == 0 && per_head <= 64))) {
+    const int iters = pieces <= 512 ? 1 : pieces <= 1024 ? 2 : 4;
+    const dim3 threads(((pieces + iters - 1) / iters + 63) & ~63);
+#define QKV_PIECES(TO_, N_) hipLaunchKernelGGL((qkv_finish_pieces_kernel<TO_, N_>), dim3(tokens), threads, lds, s, a)
+    if (dtype == MIE_F32) { if (iters == 1) QKV_PIECES(float, 1); else if (iters == 2) QKV_PIECES(float, 2); else QKV_PIECES(float, 4); }
+    else if (dtype == MIE_BF16) { if (iters == 1) QKV_PIECES(bf16, 1); else if (iters == 2) QKV_PIECES(bf16, 2); else QKV_PIECES(bf16, 4); }
+    else MIE_FAIL("qkv_finish: dtype code %d", dtype);
+#undef QKV_PIECES
+    MIE_CHECK_LAUNCH("qkv_finish");
+    return 0;
+  }
   // few tokens: several workgroups a token, so that a decode step's few rows are spread over the GPU
   int parts = tokens >= 256 ? 1 : (Hq + Hkv + 3) / 4;
   parts = parts < 1 ? 1 : parts > 8 ? 8 : parts;

@@ -544,6 +544,52 @@ def test_joined_norms_of_many_tokens(hip, dtype, width, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", [
+    # Hq, Hkv, dim, vdim, P, nf, layout, norms (whole, a head, none), own values, page
+    (32, 4, 64, 64, 64, 32, "half", "whole", True, 16), (16, 4, 128, 128, 128, 32, "interleaved", "none", False, 16),
+    (4, 2, 16, 24, 32, 4, "half", "head", True, 48), (3, 1, 40, 32, 48, 20, "interleaved", "whole", True, 16),
+    (40, 8, 128, 128, 128, 64, "half", "head", True, 16), (60, 10, 128, 128, 128, 0, "half", "whole", True, 32),
+    (6, 2, 40, 40, 48, 8, "half", "head", True, 16)])      # (pieces of a head no power of two: the wave a head)
+def test_attention_preparation_in_pieces(hip, dtype, form):
+    """Many tokens with sizes in pieces of 8: one, two and four pieces a thread, heads padded and partly turned, values of
+    their own size, and a row of sums whose columns are off 16 bytes (the wave a head) with the same result."""
+    Hq, Hkv, dim, vdim, P, nf, layout, norms, own_v, page = form
+    ops, g = hip[dtype], torch.Generator().manual_seed(Hq + dim + nf)
+    T = 261
+    inv_freq = (50.0 ** -(torch.arange(nf).double() * 2 / max(1, 2 * nf))).float().cuda() if nf else None
+    positions = torch.randint(0, 5000, (T,), generator=g).to(torch.int32).cuda()
+    slots = (torch.randperm((T // page + 2) * page, generator=g)[:T].to(torch.int32) + page).cuda()
+    per_head = norms == "head"
+    qn, kn = ((None, None) if norms == "none" else
+              tuple(_rand((dim if per_head else H * dim,), torch.float32, g) + 1 for H in (Hq, Hkv)))
+    hs = (torch.rand(Hq, generator=g) + 0.5).cuda()
+    numbers = _rand((T, Hq * dim + Hkv * dim + Hkv * vdim), torch.float32, g, 2.0)
+    bias = _rand((numbers.shape[1] + 8,), torch.float32, g)
+    for off in (4, 3):
+        sums = torch.zeros(T, numbers.shape[1] + 8, device="cuda")
+        sums[:, off:off + numbers.shape[1]] = numbers
+        q_col, k_col, v_col = off, off + Hq * dim, off + (Hq + Hkv) * dim if own_v else None
+        caches = [torch.full((T // page + 3, Hkv) + tail, 7.0, dtype=dtype).cuda() for tail in ((page, P), (P, page))]
+        want_caches = [c.clone() for c in caches]
+        shape = (sums, q_col, k_col, v_col, Hq, Hkv, dim, vdim, P, positions, inv_freq, layout)
+        if per_head:
+            shaped = sums.clone() + bias
+            for H, col, w in ((Hq, q_col, qn), (Hkv, k_col, kn)):
+                h = shaped[:, col:col + H * dim].view(T, H, dim).double()
+                if v_col is None and col == k_col:
+                    raise AssertionError("the oracle norms keys in place")
+                shaped[:, col:col + H * dim] = (h / torch.sqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()).float().view(T, H * dim)
+            want = ref.ref_qkv_finish(shaped, *shape[1:], *want_caches, slots, None, None, 1e-5, hs, dtype)
+        else:
+            want = ref.ref_qkv_finish(sums + bias, *shape[1:], *want_caches, slots, qn, kn, 1e-5, hs, dtype)
+        got = ops.qkv_finish(*shape, *caches, slots, q_norm=qn, k_norm=kn, eps=1e-5, q_head_scale=hs, col_bias=bias, norm_per_head=per_head)
+        close(got, want, TOL[dtype], f"queries, columns from {off}")
+        close(caches[0], want_caches[0], TOL[dtype], f"keys, columns from {off}")
+        close(caches[1], want_caches[1], TOL[dtype], f"values, columns from {off}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_preparation_kernels(hip, dtype):
     ops, g = hip[dtype], torch.Generator().manual_seed(2)
     cases = ((4, 2, 16, 24, 32, 4, "half", True, False, True, 37), (6, 3, 32, 32, 32, 8, "interleaved", False, True, False, 3),
