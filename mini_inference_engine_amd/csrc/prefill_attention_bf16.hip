@@ -19,11 +19,16 @@
 //
 // A workgroup of PF_WAVES waves serves one kv head and one stretch of queries of a row: its waves lie side by
 // side over the heads of the group and then over 32-query tiles.  All waves need the same keys: a block
-// of 64 keys and values is brought into the LDS once by all of them (two LDS buffers and two sets of
+// of 64 keys and values is brought into the LDS once by all of them.  At head sizes 64 and 128 (PF_DIRECT) by loads that
+// write the LDS, into a ring of two or three steps, as the keys and values lie in their pages; the score tile's rows are dealt
+// so that a lane's scores are runs of eight keys (row 4 g + j of 16 is key 8 g + j, row 8 + 4 g + j key 8 g + 4 + j), and the
+// values are taken in that order.  At other head sizes through registers (two LDS buffers and two sets of
 // registers: block i + 1 waits in registers while block i is computed, block i + 2 is on its way, the pages
 // of block i + 3 are looked up), in rows padded so that the fragment reads meet no bank conflict.  The more
-// queries share a block the better: what bounds the kernel at long contexts is the traffic from the L2 into
-// the workgroups.  Work per stretch grows with its place in the row (causal), so where stretches outnumber the
+// queries share a block the better for what comes out of the L2s.  What bounds it at head size 128 (2,048 tokens behind 4,096,
+// counters): matrix unit 46 % and vector unit 49 % of the cycles, one after the other behind the common barrier, the LDS reads of
+// 256 KB a step as long as either; at 64 (2,048 tokens): vector unit 50 %, matrix unit 21 %, and 8 of 39 us are starts and ends.
+// 2,048 tokens of 32 / 4 heads of 64 through registers / directly 45 / 39 us, of 32 / 8 of 128 behind 4,096 279 / 190 (MI355X).  Work per stretch grows with its place in the row (causal), so where stretches outnumber the
 // compute units a workgroup takes stretch NS - 1 - i and then stretch i: every workgroup of a row has the same number of blocks.  A block every
 // query of a wave sees whole takes a path without masks; the running maximum m is kept in units of
 // scale * log2(e); l is a per-lane partial sum, joined over a query's two lanes at the end.
