@@ -224,7 +224,7 @@ class HipBackend(KernelBackend):
 
     @staticmethod
     def _f32_ok(x, w, bias, out_dtype) -> bool:
-        """Whether the 32-bit matrix-unit kernels take x w^T: float32 throughout and 16-byte pieces everywhere.  What
+        """Whether the float32 product kernels take x w^T: float32 throughout and 16-byte pieces everywhere.  What
         they refuse goes to mie_gemm_nt.  Nothing here depends on the number of rows."""
         return (out_dtype == torch.float32 and x.dtype == torch.float32 and w.dtype == torch.float32
                 and w.shape[0] % 4 == 0 and w.shape[1] % 4 == 0 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
