@@ -14,10 +14,10 @@
 // eighths (sizes from K alone).  An eighth is one chain of steps for hh and one for the small products and ends as their sum, a
 // quarter is e0 + e1 and the result ((q0 + q1) + q2) + q3.
 //
-// Numbers that bfloat16 cannot hold (infinities, and what rounds to one: 3.396e38 and above) have no such parts: their eighths
-// come out as NaN.  Every result that is one is computed again by 32-bit multiplications and additions (plain_unit): what is an
-// infinity stays one, and what is a NaN ends that at its first.  (Only there, where a finite number of 3.396e38 or more gives a
-// finite result, can the cut of the batch show in a last bit: a unit of K is computed again as a whole.)
+// Results that are not finite are computed again, in 64 bits (plain_product): a number that bfloat16 cannot hold (an infinity, and what
+// rounds to one) has no such parts and gives NaN, and where h(x) h(w) or a sum of them rounds beyond the largest number the parts give an
+// infinity for what may be a finite result.  The rule looks at the whole sum over K alone (units' sums are looked at where they are
+// joined), so it is the same for every cut of the batch.
 //
 // skinny_f32_kernel (M <= 16): the weights' bytes bound it.  A workgroup owns 16 rows of W; a wave streams a contiguous
 //   part of K through a ring of its own in the LDS, filled by loads that write the LDS directly: 8 rows of 32 k a load, lane
@@ -95,26 +95,29 @@ __device__ __forceinline__ Parts split8(const f32x4& a, const f32x4& b) {
   return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-// The eighths [e0, e0 + n) of one result, n 1, 2 or 8, by 32-bit multiplications and additions, joined in the order of all
-// kernels here; a NaN, which stays one, ends it.
-__device__ __forceinline__ float plain_unit(const float* x, const float* w, int K, const KCut& cut, int e0, int n) {
-  float total = 0.f, quarter = 0.f;
-  for (int e = e0; e < e0 + n; ++e) {
-    int k0, k1;
-    eighth_range(cut, e, k0, k1);
-    k1 = least(k1 * 32, K);
-    float s = 0.f;
-    for (int k = k0 * 32; k < k1; ++k) {
-      s = fmaf(x[k], w[k], s);
-      if (s != s) return s;
-    }
-    quarter += s;
-    if (e & 1 || n == 1) {
-      total += quarter;
-      quarter = 0.f;
-    }
+// One result by 64-bit multiplications and additions, k ascending; a NaN, which stays one, ends it.
+__device__ __forceinline__ float plain_product(const float* x, const float* w, int K) {
+  double s = 0.0;
+  for (int k = 0; k < K; k += 4) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(x + k), b = *reinterpret_cast<const f32x4*>(w + k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s = fma((double)a[i], (double)b[i], s);
+    if (s != s) break;
   }
-  return total;
+  return (float)s;
+}
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
+// four results beside each other, x times the rows w, w + ldw, ...: those that are not finite computed again
+__device__ __forceinline__ void again_if_not_finite(f32x4& v, const float* x, const float* w, long ldw, int K) {
+  if (!__any(!(finite(v[0]) && finite(v[1]) && finite(v[2]) && finite(v[3])))) return;
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i) {
+    const float t = i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
+    if (finite(t)) continue;
+    const float r = plain_product(x, w + i * ldw, K);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = i == j ? r : v[j];
+  }
 }
 
 enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2, GF_ROPE = 3 };
@@ -280,7 +283,7 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
     for (int e = 0; e < 2; ++e) t += s_acc[(2 * q + e) * 256 + src];
     v += t;
   }
-  if (v != v && m < M && weight_row(c) >= 0) v = plain_unit(X + (size_t)m * ldx, W + (size_t)weight_row(c) * ldw, K, cut, 0, 8);
+  if (!finite(v) && m < M && weight_row(c) >= 0) v = plain_product(X + (size_t)m * ldx, W + (size_t)weight_row(c) * ldw, K);
   float other = 0.f;
   if (EPI == GF_SWIGLU || EPI == GF_ROPE) other = __shfl_xor(v, 8, 64);
   if (EPI == GF_ROPE) {
@@ -458,15 +461,9 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
       if (n >= N) continue;                   // N is a multiple of 4
       f32x4 v = LEVELS == 0 ? main[a][b] + small[a][b] : LEVELS == 1 ? quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0]
                                                                      : total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0];
-      if (__any(v[0] + v[1] + v[2] + v[3] != v[0] + v[1] + v[2] + v[3])) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (v[i] != v[i])
-            v[i] = plain_unit(X + (size_t)m * ldx, W + (size_t)(n + i) * ldw, K, cut,
-                              LEVELS == 0 ? blockIdx.z : LEVELS == 1 ? 2 * blockIdx.z : 0, LEVELS == 0 ? 1 : LEVELS == 1 ? 2 : 8);
-      }
       f32x4* o = reinterpret_cast<f32x4*>(dst + (size_t)m * ld + n);
       if (LEVELS == 2) {
+        again_if_not_finite(v, X + (size_t)m * ldx, W + (size_t)n * ldw, ldw, K);
         if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
         if (add) v = *o + v;
       }
@@ -499,16 +496,19 @@ __device__ __forceinline__ f32x4 join_parts(const f32x4* p, size_t stride) {
 
 template <int PARTS, int EPI>
 __global__ void __launch_bounds__(256)
-reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long ldo, const float* __restrict__ bias, int M, int N) {
+reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long ldo, const float* __restrict__ bias, int M, int N,
+                  const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, int K) {
   const int cols = EPI == GF_SWIGLU ? 2 * N : N, per_row = N >> 2;
   const size_t stride = (size_t)M * cols / 4, total = (size_t)M * per_row;
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (size_t)gridDim.x * 256) {
     const size_t m = e / per_row, n = (e - m * per_row) * 4;
     const f32x4* p = reinterpret_cast<const f32x4*>(part + m * cols + n);
     f32x4 v = join_parts<PARTS>(p, stride);
+    again_if_not_finite(v, X + m * ldx, W + n * ldw, ldw, K);
     f32x4* o = reinterpret_cast<f32x4*>(out + m * ldo + n);
     if (EPI == GF_SWIGLU) {
-      const f32x4 u = join_parts<PARTS>(p + (N >> 2), stride);
+      f32x4 u = join_parts<PARTS>(p + (N >> 2), stride);
+      again_if_not_finite(u, X + m * ldx, W + (N + n) * ldw, ldw, K);
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
       *o = v;
@@ -609,13 +609,14 @@ static int launch_tiles(const float* X, long ldx, const float* W, long ldw, floa
 }
 
 template <int EPI>
-static int launch_reduce(int units, const float* part, float* out, long ldo, const float* bias, int M, int N, hipStream_t s) {
+static int launch_reduce(int units, const float* part, float* out, long ldo, const float* bias, int M, int N, const float* X, long ldx,
+                         const float* W, long ldw, int K, hipStream_t s) {
   long blocks = ((long)M * (N / 4) + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   if (units == 4)
-    hipLaunchKernelGGL((reduce_f32_kernel<4, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N);
+    hipLaunchKernelGGL((reduce_f32_kernel<4, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K);
   else
-    hipLaunchKernelGGL((reduce_f32_kernel<8, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N);
+    hipLaunchKernelGGL((reduce_f32_kernel<8, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K);
   MIE_CHECK_LAUNCH("reduce_f32");
   return 0;
 }
@@ -641,9 +642,9 @@ MIE_EXPORT int mie_gemm_f32(const float* X, long ldx, const float* W, long ldw, 
   if (epi == GF_SWIGLU && units == 1) MIE_FAIL("gemm_f32: %d rows of %d columns are one unit: take the product and silu_mul", M, cols);
   if (!part) MIE_FAIL("gemm_f32: %d units need memory for their sums", units);
   if (launch_tiles(X, ldx, W, ldw, part, cols, nullptr, 0, M, cols, K, plan, s)) return -1;
-  return epi == GF_STORE ? launch_reduce<GF_STORE>(units, part, out, ldo, bias, M, N, s)
-       : epi == GF_ADD ? launch_reduce<GF_ADD>(units, part, out, ldo, bias, M, N, s)
-                       : launch_reduce<GF_SWIGLU>(units, part, out, ldo, bias, M, N, s);
+  return epi == GF_STORE ? launch_reduce<GF_STORE>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
+       : epi == GF_ADD ? launch_reduce<GF_ADD>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
+                       : launch_reduce<GF_SWIGLU>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s);
 }
 
 // The q/k/v projection of up to 16 rows with what follows it: W [(Hq + 2 Hkv) D, K]; q and k rotated (half-split pairs over the

@@ -188,6 +188,43 @@ def test_linear_float32_in_three_parts(ops, shape):
             assert torch.equal(alone.nan_to_num(1e30), got[M // 2:M // 2 + 1].nan_to_num(1e30))
 
 
+# (rows, K, N, parts of K that the product's plan takes): the few-row kernel (two steps at once, one), the tiles whole, in quarters
+# and in eighths
+F32_FORMS = [(3, 2080, 48, 0), (12, 2080, 48, 0), (600, 352, 9000, 1), (300, 2048, 2048, 4), (40, 1056, 64, 8)]
+
+
+def f32_parts_of_k(o, M, K, N):
+    return o.lib("gemm_f32").mie_f32_units(M, N, K, 0) if M > 16 else 0
+
+
+@pytest.mark.parametrize("shape", F32_FORMS)
+def test_linear_float32_just_below_the_largest_number(ops, shape):
+    """Results of 3.396e38 whose operands round up where they are cut: their first parts' product is an infinity, the results are
+    not, and they are the same bits in every cut, also where larger ones beside them are infinities."""
+    M, K, N, parts = shape
+    o = ops[torch.float32]
+    assert f32_parts_of_k(o, M, K, N) == parts
+    torch.manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    rows, cols = [0, M // 2, M - 1], [1, N // 2, N - 2]
+    for i, (r, c) in enumerate(zip(rows, cols)):
+        at = (i * K // 3 + 35) % K
+        x[:, at], w[:, at] = 0.0, 0.0
+        x[r, at], w[c, at] = 1.00395, 1.98829 * 2.0 ** 127 * (-1) ** i
+        w[c + 1, at] = 1.995 * 2.0 ** 127                 # times x[r, at]: beyond the largest number
+    y, want = o.linear(x, w), x.double() @ w.double().T
+    large = want.abs() > 3.4028234663852886e38
+    assert int(large.sum()) == 3 and float(want[~large].abs().max()) > 3.39e38
+    assert torch.equal(y[large].double(), want[large].sign() * float("inf"))
+    bound = (K / 16 + 32) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((y.double() - want).abs()[~large] <= bound[~large]).all())
+    for a, b in ((0, 1), (0, min(M, 16)), (M // 2, M // 2 + 1), (M // 2, M)):
+        assert torch.equal(o.linear(x[a:b].contiguous(), w), y[a:b])
+    assert torch.equal(o.linear(torch.cat([x, torch.randn(700, K, device=DEV)]), w)[:M], y)
+    silu = o.linear_silu_mul(x, w, N // 2)
+    assert torch.equal(silu.nan_to_num(1e30), o.silu_mul(y, N // 2).nan_to_num(1e30))
+
+
 def test_linear_mixed_storage(ops):
     """A matrix stored in 32-bit beside bfloat16 activations: computed, not refused."""
     torch.manual_seed(2)
