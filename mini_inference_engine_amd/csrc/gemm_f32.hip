@@ -2,10 +2,12 @@
 //
 //   y[m, n] = sum_k x[m, k] W[n, k]          x [M, K], W [N, K], y [M, N] float32
 //
-// A 32-bit number is the sum of three bfloat16 ones to its last bit or the one before (24 bits of mantissa in three pieces of
-// 8, the signs take up the roundings): v = h + m + l, h = bf16(v), m = bf16(v - h), l = bf16(v - h - m).  Of the nine
-// products six are taken, hh, hm, mh, mm, hl, lh; the three left out are below 2^-25 of |x w|.  A product of two bfloat16 numbers
-// is exact in 32 bits, so what rounds is the sums, and those of the five small products run in a chain of their own, where a
+// 2^16 times a 32-bit number v of less than 2^111 is the sum of three bfloat16 ones to its last bit (24 bits of mantissa in three
+// pieces of 8, the signs take up the roundings): h = bf16(2^16 v), m = bf16(2^16 v - h), l = 2^16 v - h - m.  Without the factor m and
+// l would fall below bfloat16's smallest number, 2^-133, for v below 2^-110 (the error of a product of operands of 1 and 2^-118 would be
+// 9e-6 for 1e-7); the sums lose the 2^32 of both operands at their end.  Of the nine products six are taken, hh, hm, mh, mm, hl, lh; the
+// three left out, ml, lm and ll, are together at most a little more than 2^-24 of |x w|.  A product of two bfloat16 numbers is
+// exact in 32 bits, so what rounds is the sums, and those of the five small products run in a chain of their own, where a
 // rounding is 2^-8 of one in the sums of hh.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles of a SIMD for what eight
 // v_mfma_f32_16x16x4_f32 (true 32-bit products) need 256 for.
 //
@@ -14,10 +16,11 @@
 // eighths (sizes from K alone).  An eighth is one chain of steps for hh and one for the small products and ends as their sum, a
 // quarter is e0 + e1 and the result ((q0 + q1) + q2) + q3.
 //
-// Results that are not finite are computed again, in 64 bits (plain_product): a number that bfloat16 cannot hold (an infinity, and what
-// rounds to one) has no such parts and gives NaN, and where h(x) h(w) or a sum of them rounds beyond the largest number the parts give an
-// infinity for what may be a finite result.  The rule looks at the whole sum over K alone (units' sums are looked at where they are
-// joined), so it is the same for every cut of the batch.
+// Results that are not finite are computed again, in 64 bits (plain_product): a number whose 2^16-fold bfloat16 cannot hold (2^111
+// and more, an infinity) has no such parts and gives NaN, and where h(x) h(w) or a sum of them goes beyond the largest number
+// (results of 2^95 and more) the parts give an infinity for what may be a finite result.  The rule looks at the whole sum over K alone
+// (units' sums are looked at where they are joined), so it is the same for every cut of the batch.  It is there to be right, not fast:
+// 512 rows of [2048, 2048] all of whose results are such take 1.2 ms for 0.035.
 //
 // skinny_f32_kernel (M <= 16): the weights' bytes bound it.  A workgroup owns 16 rows of W; a wave streams a contiguous
 //   part of K through a ring of its own in the LDS, filled by loads that write the LDS directly: 8 rows of 32 k a load, lane
@@ -69,14 +72,35 @@ __host__ __device__ __forceinline__ void eighth_range(const KCut& c, int e, int&
 __device__ __forceinline__ uint32_t round2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
-// h, m, l of two numbers
+constexpr float GF_SCALE = 65536.f, GF_UNSCALE = 1.f / (65536.f * 65536.f);      // of an operand; of what two scaled ones give
+// c minus the low or the high half of h (sel: -1 there, 0 in the other), exact where the difference is a 32-bit number: one
+// instruction for the shift or mask and the subtraction.  sel in a scalar register: as a constant the compiler writes -1.0 into the
+// instruction, which stands for another half.
+__device__ __forceinline__ float less_half(float c, uint32_t h, uint32_t sel) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, h), __builtin_bit_cast(bf16x2, sel), c, false);
+}
+struct Halves {
+  uint32_t low, high;
+};
+__device__ __forceinline__ Halves minus_one() {
+  Halves s;
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(s.low));
+  asm("s_mov_b32 %0, 0xbf800000" : "=s"(s.high));
+  return s;
+}
+// h, m, l of two numbers.  DOT: the differences by less_half, which pays where splitting bounds a kernel (tiles of 64 x 64 44.8 us against
+// 45.9 at 512 rows of [2560, 2048]) and not beside many matrix instructions (128 x 128 tiles 176 against 167 at 512 of [11264, 2048]).
+template <bool DOT>
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  const Halves minus = minus_one();
+  a *= GF_SCALE;
+  b *= GF_SCALE;
   h = round2(a, b);
-  a -= __uint_as_float(h << 16);
-  b -= __uint_as_float(h & 0xFFFF0000u);
+  a = DOT ? less_half(a, h, minus.low) : a - __uint_as_float(h << 16);
+  b = DOT ? less_half(b, h, minus.high) : b - __uint_as_float(h & 0xFFFF0000u);
   m = round2(a, b);
-  a -= __uint_as_float(m << 16);
-  b -= __uint_as_float(m & 0xFFFF0000u);
+  a = DOT ? less_half(a, m, minus.low) : a - __uint_as_float(m << 16);
+  b = DOT ? less_half(b, m, minus.high) : b - __uint_as_float(m & 0xFFFF0000u);
   l = round2(a, b);
 }
 
@@ -89,20 +113,20 @@ __device__ __forceinline__ Parts split8(const f32x4& a, const f32x4& b) {
   for (int i = 0; i < 4; ++i) {
     const float p = i < 2 ? a[2 * i] : b[2 * i - 4], q = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
     uint32_t hh, mm, ll;
-    split2(p, q, hh, mm, ll);
+    split2<true>(p, q, hh, mm, ll);
     h[i] = hh, m[i] = mm, l[i] = ll;
   }
   return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-// One result by 64-bit multiplications and additions, k ascending; a NaN, which stays one, ends it.
+// One result by 64-bit multiplications and additions, k ascending.
 __device__ __forceinline__ float plain_product(const float* x, const float* w, int K) {
   double s = 0.0;
+#pragma unroll 4
   for (int k = 0; k < K; k += 4) {
     const f32x4 a = *reinterpret_cast<const f32x4*>(x + k), b = *reinterpret_cast<const f32x4*>(w + k);
 #pragma unroll
     for (int i = 0; i < 4; ++i) s = fma((double)a[i], (double)b[i], s);
-    if (s != s) break;
   }
   return (float)s;
 }
@@ -283,6 +307,7 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
     for (int e = 0; e < 2; ++e) t += s_acc[(2 * q + e) * 256 + src];
     v += t;
   }
+  v *= GF_UNSCALE;
   if (!finite(v) && m < M && weight_row(c) >= 0) v = plain_product(X + (size_t)m * ldx, W + (size_t)weight_row(c) * ldw, K);
   float other = 0.f;
   if (EPI == GF_SWIGLU || EPI == GF_ROPE) other = __shfl_xor(v, 8, 64);
@@ -324,6 +349,7 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
                 long ldo, const float* __restrict__ bias, int add, int M, int N, int K) {
   constexpr int THREADS = WR * WC * 64, WM = BM / WR, WN = BN / WC, TM = WM / 16, TN = WN / 16, ROWS = BM + BN;
   constexpr int PLANE = ROWS * 64, BUFFER = 3 * PLANE, XL = BM * 8 / THREADS, LOADS = ROWS * 8 / THREADS;      // 16-byte loads a thread and stage
+  constexpr bool DOT = TM * TN <= 2;          // few matrix instructions a number that is split (see split2)
   static_assert(BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0, "loads of a thread are of x or of W");
   extern __shared__ __align__(16) char gf_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -358,8 +384,8 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       uint2 h, m, l;
-      split2(staged[i][0], staged[i][1], h.x, m.x, l.x);
-      split2(staged[i][2], staged[i][3], h.y, m.y, l.y);
+      split2<DOT>(staged[i][0], staged[i][1], h.x, m.x, l.x);
+      split2<DOT>(staged[i][2], staged[i][3], h.y, m.y, l.y);
       char* p = gf_lds + buf * BUFFER + at[i];
       *reinterpret_cast<uint2*>(p) = h;
       *reinterpret_cast<uint2*>(p + PLANE) = m;
@@ -416,11 +442,12 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
     products(2, 0, small);
     products(0, 2, small);
     products(1, 1, small);
-    // matrix instructions and the splitting in turn
+    // matrix instructions and the splitting in turn (two of it each: 172 us for 167 at 512 rows of [11264, 2048], in tiles of 64 x 64 46.0
+    // for 44.8 at 512 of [2560, 2048])
 #pragma unroll
     for (int i = 0; i < 6 * TM * TN; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, DOT ? 1 : 3, 0);
     }
     if (LEVELS >= 1 && ks + 1 == eighth_end) {
       const bool quarter_done = LEVELS >= 2 && eighth_end == quarter_end;
@@ -463,6 +490,7 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
                                                                      : total[LEVELS >= 2 ? a : 0][LEVELS >= 2 ? b : 0];
       f32x4* o = reinterpret_cast<f32x4*>(dst + (size_t)m * ld + n);
       if (LEVELS == 2) {
+        v *= GF_UNSCALE;
         again_if_not_finite(v, X + (size_t)m * ldx, W + (size_t)n * ldw, ldw, K);
         if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
         if (add) v = *o + v;
@@ -491,7 +519,7 @@ __device__ __forceinline__ f32x4 join_parts(const f32x4* p, size_t stride) {
     }
     total += t;
   }
-  return total;
+  return total * GF_UNSCALE;
 }
 
 template <int PARTS, int EPI>

@@ -225,6 +225,24 @@ def test_linear_float32_just_below_the_largest_number(ops, shape):
     assert torch.equal(silu.nan_to_num(1e30), o.silu_mul(y, N // 2).nan_to_num(1e30))
 
 
+@pytest.mark.parametrize("scales", [(60, -122), (-122, 60), (0, -110), (0, -118), (-118, 30), (-60, -60), (100, -140)])
+@pytest.mark.parametrize("shape", F32_FORMS)
+def test_linear_float32_of_tiny_operands(ops, shape, scales):
+    """Operands of 2^scales: as exact as at ordinary sizes (the bound of test_linear_float32_in_three_parts), down to numbers below
+    the smallest normal one (which hold the fewer bits that they hold; nothing more is lost), and the same bits in every cut."""
+    M, K, N, parts = shape
+    o = ops[torch.float32]
+    assert f32_parts_of_k(o, M, K, N) == parts
+    torch.manual_seed(K + N)
+    x, w = ((torch.randn(n, K, device=DEV, dtype=torch.float64) * 2.0 ** e).float() for n, e in ((M, scales[0]), (N, scales[1])))
+    y, exact = o.linear(x, w), x.double() @ w.double().T
+    scale = 2.0 ** -sum(scales)          # (a norm of numbers of 2^-120 is not taken as they are)
+    error, size = ((y.double() - exact) * scale).norm(), (exact * scale).norm()
+    assert error <= 2.0 ** -24 * math.sqrt(K / 16 + 8) * size, (float(error / size))
+    for a, b in ((0, 1), (0, min(M, 16)), (M // 2, M)):
+        assert torch.equal(o.linear(x[a:b].contiguous(), w), y[a:b])
+
+
 def test_linear_mixed_storage(ops):
     """A matrix stored in 32-bit beside bfloat16 activations: computed, not refused."""
     torch.manual_seed(2)
