@@ -560,10 +560,13 @@ static int check_operands(const char* what, const void* X, long ldx, const void*
 // The tile of a workgroup and how many units K is cut into (1, 4 or 8) for M rows (more than 16): the cheapest by what was
 // measured (MI355X, 17 to 2,048 rows of [11264, 2048], [2560, 2048], [2048, 2048], [2048, 5632], [768, 1536] and two small
 // weights).  A step of 32 k costs a compute unit fixed + each x the workgroups it has, whether they run side by side or in
-// turn; a start 2.9 us; units' sums cost a kernel of 1.9 us and 1.6 us a million of them.  Large tiles split and read an operand for more outputs, small ones and units of K give every compute unit
-// work: us of 128 x 128 / 128 x 64 / 64 x 64, each at its best cut: 512 rows of [11264, 2048] 176 / 169 / 180, 2,048 rows 543 / 638 /
-// 684, 512 rows of [2048, 2048] 35 / 40 / 39, 100 rows 20 / 17 / 16, 32 rows of [2048, 5632] 36 / 27 / 20.  gated: the product's
-// gate and up columns are joined where the units' sums are, else by a pass of its own.
+// turn; a start 2.9 us; units' sums cost a kernel of 1.9 us and 1.6 us a million of them.  Large tiles split and read an operand for
+// more outputs, small ones and units of K give every compute unit work: us of 128 x 128 / 128 x 64 / 64 x 64, each at its best cut: 512
+// rows of [11264, 2048] 176 / 169 / 180, 2,048 rows 543 / 638 / 684, 512 rows of [2048, 2048] 35 / 40 / 39, 100 rows 20 / 17 / 16, 32 rows of
+// [2048, 5632] 36 / 27 / 20.  gated: the product's gate and up columns are joined where the units' sums are, else by a pass of its own.
+// The units' sums take at most GF_PART_FLOATS, 128 MiB: 512 rows of [11264, 2048] have 92 MB of them (quarters 187 us, uncut 212 and a
+// pass of 10), and without a bound their memory would grow with the weight's size to gigabytes.
+constexpr long GF_PART_FLOATS = 1L << 25;
 constexpr struct { int bm, bn; float fixed, each; } GF_TILES[3] = {{128, 128, 0.f, 1.40f}, {128, 64, 0.f, 0.87f}, {64, 64, 0.07f, 0.45f}};
 struct TilePlan {
   int tile, units;
@@ -576,6 +579,7 @@ static TilePlan tile_plan(int M, int N, int K, bool gated) {
   for (int t = 0; t < 3; ++t) {
     const long tiles = (long)((M + GF_TILES[t].bm - 1) / GF_TILES[t].bm) * ((N + GF_TILES[t].bn - 1) / GF_TILES[t].bn);
     for (int units = 1; units <= 8; units += units == 1 ? 3 : 4) {
+      if (units > 1 && units * (long)M * N > GF_PART_FLOATS) break;
       const int steps = units == 1 ? cut.steps : units == 4 ? cut.quarter : cut.eighth;
       const long each = (tiles * units + mie_compute_units() - 1) / mie_compute_units();
       float us = 2.9f + steps * (GF_TILES[t].fixed + GF_TILES[t].each * each);

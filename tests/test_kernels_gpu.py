@@ -243,6 +243,27 @@ def test_linear_float32_of_tiny_operands(ops, shape, scales):
         assert torch.equal(o.linear(x[a:b].contiguous(), w), y[a:b])
 
 
+def test_linear_float32_in_parts_has_bounded_memory(ops):
+    """The sums of K's parts take at most 128 MiB, at any size; what is not cut for that is computed whole with the same bits."""
+    o = ops[torch.float32]
+    cut = set()
+    for M in (17, 100, 333, 512, 700, 1132, 1500, 2048, 4096, 8192):
+        for N in (64, 2048, 5632, 11264, 28672, 57344, 128256):
+            for K in (64, 2048, 5632, 14336, 28672):
+                for gated in (0, 1):
+                    parts = o.lib("gemm_f32").mie_f32_units(M, N, K, gated)
+                    assert parts == 1 or parts * M * N * 4 <= 1 << 27, (M, N, K, gated, parts)
+                    cut.add(parts)
+    assert cut == {1, 4, 8}
+    M, K, N = 1132, 4096, 8192
+    assert f32_parts_of_k(o, M, K, N) == 1 and f32_parts_of_k(o, 700, K, N) == 4
+    torch.manual_seed(0)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    y = o.linear(x, w)
+    for a, b in ((0, 700), (1100, 1132), (700, 709)):
+        assert torch.equal(o.linear(x[a:b].contiguous(), w), y[a:b])
+
+
 def test_linear_mixed_storage(ops):
     """A matrix stored in 32-bit beside bfloat16 activations: computed, not refused."""
     torch.manual_seed(2)
