@@ -119,24 +119,45 @@ qkv_finish_kernel(FinishArgs a) {
 // The same where everything comes in pieces of 8 numbers: a thread a piece (four pairs that turn, or 8 numbers that do not, or
 // 8 values), up to ITERS of them, all asked for before the norms' sums.  The kernel above takes a wave a head and one head after
 // the other, each a trip to memory with half the lanes: nine in a row at 32 + 4 heads of 64 and one token a workgroup, which is what
-// bounded it.  2,048 tokens (MI355X, us): 32 + 4 heads of 64 with norms 33.8 / 16.2, 16 + 4 of 128 without 21.8 / 14.0.
+// bounded it.  The norms' sums are taken out of the LDS in the order of the kernel above (256 lanes over a projection, 64 over a head),
+// so that a token's bits do not depend on how many others its step has (sums of a thread's own pieces: 12.7 us for the 13.8, 28.6 for
+// the 33.3).  The kernel above / this one at 2,048 tokens (MI355X, us): 32 + 4 heads of 64 with norms 26.4 / 13.8, 40 + 8 of 128 normed
+// head by head 52.4 / 33.3, 32 + 8 of 64 so 37.2 / 17.4, 16 + 4 of 128 without norms 15.4 / 13.7.
 __device__ __forceinline__ void store4(float* p, const float* v) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
 __device__ __forceinline__ void store4(bf16* p, const float* v) {
   const bf16 o[4] = {__float2bfloat16(v[0]), __float2bfloat16(v[1]), __float2bfloat16(v[2]), __float2bfloat16(v[3])};
   *reinterpret_cast<uint2*>(p) = *reinterpret_cast<const uint2*>(o);
 }
 
+// wave_sum with the same additions in the same order (lanes l and l ^ 32, then ^ 16, 8, 4, 2, 1) by swaps and rotations in
+// registers: the six trips through the LDS after one another are what the norms' sums below waited for (with them 14.2 us for the 13.8).
+__device__ __forceinline__ float swap_sum(float v) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+#define QKV_DPP(CTRL_) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL_, 0xF, 0xF, false))
+  QKV_DPP(0x128);      // row_ror:8
+  QKV_DPP(0x124);      // row_ror:4: lane l ^ 4's sum, now that lanes l and l ^ 8 hold the same
+  QKV_DPP(0x4E);       // quad_perm 2, 3, 0, 1
+  QKV_DPP(0xB1);       // quad_perm 1, 0, 3, 2
+#undef QKV_DPP
+  return v;
+}
+
 template <typename TO, int ITERS>
 __global__ void __launch_bounds__(512)
 qkv_finish_pieces_kernel(FinishArgs a) {
-  __shared__ float parts[2][8];
-  extern __shared__ __align__(16) float cs[];   // cos [nf], sin [nf]
+  __shared__ float parts[2][4];
+  extern __shared__ __align__(16) float cs[];   // cos [nf], sin [nf], with norms the queries and keys, with norms a head their sums
+  const bool normed = a.q_norm || a.k_norm;
+  float* const xs = cs + 2 * a.nf;              // [Hq + Hkv, dim]
+  float* const squares = xs + (a.Hq + a.Hkv) * a.dim;
   const int t = blockIdx.x, per_head = a.P >> 3, heads = a.Hq + a.Hkv, turned = a.nf >> 2;
   const float* __restrict__ row = a.sums + (size_t)t * a.ld;
   const int pos = a.positions[t], slot = a.slots[t];
   float x[ITERS][8];
   int head[ITERS], d1[ITERS], d2[ITERS];        // head: queries, keys, values; first numbers of the piece's halves; -1: none
-  float ssq = 0.f, ssk = 0.f, head_ss[ITERS];
 #pragma unroll
   for (int n = 0; n < ITERS; ++n) {
     const int job = threadIdx.x + n * blockDim.x, h = job / per_head, e = job - h * per_head;
@@ -147,7 +168,6 @@ qkv_finish_pieces_kernel(FinishArgs a) {
     const int size = value ? a.vdim : a.dim;
     const int col = h < a.Hq ? a.q_col + h * a.dim : !value ? a.k_col + (h - a.Hq) * a.dim
                   : a.v_col < 0 ? a.k_col + (h - heads) * a.dim : a.v_col + (h - heads) * a.vdim;
-    float ss = 0.f;
     const bool there = head[n] >= 0 && d1[n] < size;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -161,43 +181,48 @@ qkv_finish_pieces_kernel(FinishArgs a) {
         }
       }
       x[n][4 * half] = v.x, x[n][4 * half + 1] = v.y, x[n][4 * half + 2] = v.z, x[n][4 * half + 3] = v.w;
-      ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+      if (normed && there && !value) *reinterpret_cast<float4*>(xs + h * a.dim + (half ? d2[n] : d1[n])) = v;
     }
-    head_ss[n] = ss;
-    if (h < a.Hq) ssq += ss;
-    else if (h < heads) ssk += ss;
   }
   for (int i = threadIdx.x; i < a.nf; i += blockDim.x) sincosf((float)pos * a.inv_freq[i], &cs[a.nf + i], &cs[i]);
-  const bool whole = !a.norm_per_head && (a.q_norm || a.k_norm);
-  if (whole) {
-    ssq = wave_sum(ssq);
-    ssk = wave_sum(ssk);
-    if ((threadIdx.x & 63) == 0) {
-      parts[0][threadIdx.x >> 6] = ssq;
-      parts[1][threadIdx.x >> 6] = ssk;
-    }
-  }
   __syncthreads();
   float rq = 1.f, rk = 1.f;
-  if (whole) {
-    float q = 0.f, k = 0.f;
-    for (int w = 0; w < (int)(blockDim.x + 63) >> 6; ++w) {
-      q += parts[0][w];
-      k += parts[1][w];
+  if (normed) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if (a.norm_per_head) {
+#pragma unroll 4
+      for (int h = wave; h < heads; h += waves) {
+        float ss = 0.f;
+        for (int d = lane; d < a.dim; d += 64) ss = fmaf(xs[h * a.dim + d], xs[h * a.dim + d], ss);
+        ss = swap_sum(ss);
+        if (lane == 0) squares[h] = ss;
+      }
+    } else {
+      for (int job = wave; job < 8; job += waves) {             // queries, keys: a quarter of 256 lanes each
+        const int first = job < 4 ? 0 : a.Hq * a.dim, end = job < 4 ? a.Hq * a.dim : heads * a.dim;
+        float ss = 0.f;
+#pragma unroll 4
+        for (int i = first + (job & 3) * 64 + lane; i < end; i += 256) ss = fmaf(xs[i], xs[i], ss);
+        ss = swap_sum(ss);
+        if (lane == 0) parts[job >> 2][job & 3] = ss;
+      }
     }
-    if (a.q_norm) rq = 1.0f / sqrtf(q / (float)(a.Hq * a.dim) + a.eps);
-    if (a.k_norm) rk = 1.0f / sqrtf(k / (float)(a.Hkv * a.dim) + a.eps);
+    __syncthreads();
+    if (!a.norm_per_head) {
+      float q = 0.f, k = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        q += parts[0][w];
+        k += parts[1][w];
+      }
+      if (a.q_norm) rq = 1.0f / sqrtf(q / (float)(a.Hq * a.dim) + a.eps);
+      if (a.k_norm) rk = 1.0f / sqrtf(k / (float)(a.Hkv * a.dim) + a.eps);
+    }
   }
   const float temperature = a.temp_every > 0 ? 1.0f + a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.0f) : 1.0f;
   const size_t pg = slot / a.page, off = slot % a.page;
 #pragma unroll
   for (int n = 0; n < ITERS; ++n) {
-    float r = 1.f;
-    if (a.norm_per_head) {                      // a head's pieces lie in neighbouring lanes, a power of two of them
-      float ss = head_ss[n];
-      for (int o = per_head >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-      r = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
-    }
     const int h = head[n];
     if (h < 0) continue;
     if (h >= heads) {
@@ -210,10 +235,8 @@ qkv_finish_pieces_kernel(FinishArgs a) {
     const float* __restrict__ w = is_q ? a.q_norm : a.k_norm;
     float v[8];
     if (w && d1[n] < a.dim) {
-      if (!a.norm_per_head) {
-        w += (size_t)(is_q ? h : h - a.Hq) * a.dim;
-        r = is_q ? rq : rk;
-      }
+      const float r = a.norm_per_head ? 1.0f / sqrtf(squares[h] / (float)a.dim + a.eps) : is_q ? rq : rk;
+      if (!a.norm_per_head) w += (size_t)(is_q ? h : h - a.Hq) * a.dim;
       const float4 w1 = *reinterpret_cast<const float4*>(w + d1[n]), w2 = *reinterpret_cast<const float4*>(w + d2[n]);
       const float ws[8] = {w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
 #pragma unroll
@@ -547,15 +570,16 @@ MIE_EXPORT int mie_qkv_finish(const float* sums, long ld, int q_col, int k_col, 
   FinishArgs a{sums, ld, q_col, k_col, v_col, q_norm, k_norm, eps, norm_per_head, inv_freq, nf, layout, q_head_scale, col_bias, temp_coef, temp_every,
                positions, slots, q_out, k_cache, v_cache, Hq, Hkv, dim, vdim, P, page};
   const size_t lds = (size_t)2 * (nf > 0 ? nf : 1) * sizeof(float);
-  // Pieces of 8 numbers where sizes and addresses allow it and the tokens fill the GPU; fewer tokens are spread over it below.
+  // Pieces of 8 numbers where sizes and addresses allow it, the norms' operands fit the LDS that a kernel gets by default and the
+  // tokens fill the GPU; fewer tokens are spread over it below.
   const int per_head = P >> 3, pieces = (Hq + 2 * Hkv) * per_head;
   const bool aligned = !(((uintptr_t)sums | (uintptr_t)q_norm | (uintptr_t)k_norm | (uintptr_t)col_bias | (uintptr_t)q_out |
                           (uintptr_t)k_cache) & 15) && !((ld | q_col | k_col | (v_col < 0 ? 0 : v_col)) & 3);
-  if (tokens >= 256 && aligned && !((dim | vdim | P) & 7) && !(nf & 3) && pieces <= 2048 &&
-      (!norm_per_head || ((per_head & (per_head - 1)) == 0 && per_head <= 64))) {
+  const size_t pieces_lds = sizeof(float) * ((size_t)2 * nf + (q_norm || k_norm ? (size_t)(Hq + Hkv) * (dim + 1) : 0));
+  if (tokens >= 256 && aligned && !((dim | vdim | P) & 7) && !(nf & 3) && pieces <= 2048 && pieces_lds <= 60 * 1024) {
     const int iters = pieces <= 512 ? 1 : pieces <= 1024 ? 2 : 4;
     const dim3 threads(((pieces + iters - 1) / iters + 63) & ~63);
-#define QKV_PIECES(TO_, N_) hipLaunchKernelGGL((qkv_finish_pieces_kernel<TO_, N_>), dim3(tokens), threads, lds, s, a)
+#define QKV_PIECES(TO_, N_) hipLaunchKernelGGL((qkv_finish_pieces_kernel<TO_, N_>), dim3(tokens), threads, pieces_lds, s, a)
     if (dtype == MIE_F32) { if (iters == 1) QKV_PIECES(float, 1); else if (iters == 2) QKV_PIECES(float, 2); else QKV_PIECES(float, 4); }
     else if (dtype == MIE_BF16) { if (iters == 1) QKV_PIECES(bf16, 1); else if (iters == 2) QKV_PIECES(bf16, 2); else QKV_PIECES(bf16, 4); }
     else MIE_FAIL("qkv_finish: dtype code %d", dtype);

@@ -590,6 +590,40 @@ def test_attention_preparation_in_pieces(hip, dtype, form):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", [
+    # Hq, Hkv, dim, vdim, P, nf, layout, norms, own values
+    (32, 4, 64, 64, 64, 32, "half", "whole", True), (16, 4, 128, 128, 128, 32, "interleaved", "whole", False),
+    (4, 2, 16, 24, 32, 4, "half", "head", True), (3, 1, 40, 32, 48, 20, "interleaved", "whole", True),
+    (40, 8, 128, 128, 128, 64, "half", "head", True), (5, 3, 72, 72, 128, 36, "half", "head", True), (60, 10, 128, 128, 128, 0, "half", "whole", True)])
+def test_attention_preparation_does_not_depend_on_the_cut(hip, dtype, form):
+    """A token's queries, keys and values are the same bits in steps of few tokens and of many, and where rows lie off 16 bytes."""
+    Hq, Hkv, dim, vdim, P, nf, layout, norms, own_v = form
+    ops, g = hip[dtype], torch.Generator().manual_seed(Hq + dim)
+    T, page = 523, 16
+    inv_freq = (50.0 ** -(torch.arange(nf).double() * 2 / max(1, 2 * nf))).float().cuda() if nf else None
+    positions = torch.randint(0, 5000, (T,), generator=g).to(torch.int32).cuda()
+    slots = (torch.randperm((T // page + 2) * page, generator=g)[:T].to(torch.int32) + page).cuda()
+    qn, kn = (_rand((dim if norms == "head" else H * dim,), torch.float32, g) + 1 for H in (Hq, Hkv))
+    numbers = _rand((T, Hq * dim + Hkv * dim + Hkv * vdim), torch.float32, g, 2.0)
+    bias = _rand((numbers.shape[1] + 8,), torch.float32, g)
+    seen = []
+    for off, cuts in ((4, (0, T)), (4, (0, 100, 259, T)), (3, (0, T)), (4, (0, 260, T))):
+        sums = torch.zeros(T, numbers.shape[1] + 8, device="cuda")
+        sums[:, off:off + numbers.shape[1]] = numbers
+        biased = torch.zeros_like(bias)
+        biased[off:off + numbers.shape[1]] = bias[4:4 + numbers.shape[1]]
+        caches = [torch.full((T // page + 3, Hkv) + tail, 7.0, dtype=dtype).cuda() for tail in ((page, P), (P, page))]
+        q = [ops.qkv_finish(sums[a:b], off, off + Hq * dim, off + (Hq + Hkv) * dim if own_v else None, Hq, Hkv, dim, vdim, P,
+                            positions[a:b].contiguous(), inv_freq, layout, *caches, slots[a:b].contiguous(), q_norm=qn, k_norm=kn, eps=1e-5,
+                            col_bias=biased, norm_per_head=norms == "head") for a, b in zip(cuts, cuts[1:])]
+        seen.append([torch.cat(q), *caches])
+    for other in seen[1:]:
+        for a, b in zip(seen[0], other):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_preparation_kernels(hip, dtype):
     ops, g = hip[dtype], torch.Generator().manual_seed(2)
     cases = ((4, 2, 16, 24, 32, 4, "half", True, False, True, 37), (6, 3, 32, 32, 32, 8, "interleaved", False, True, False, 3),
