@@ -885,6 +885,41 @@ def test_decode_attention_split_count_and_static_bound(ops, ctx, splits):
     torch.testing.assert_close(out2.double(), expect, **ATT_TOL[dtype])
 
 
+@pytest.mark.parametrize("form", ["plain", "sink", "kept", "chunk", "biased"])
+@pytest.mark.parametrize("geom", [(32, 4, 64, 16), (8, 1, 128, 16), (4, 4, 256, 16), (2, 1, 48, 32)])
+def test_decode_attention_weights_below_the_smallest_normal_number(ops, geom, form):
+    """A key whose weight is e^-90 = 8.2e-40 beside keys of weight 1 (one, and one a block) without values: its value of 2^100 times
+    the weight comes out, within half a unit of the weight's bfloat16 (2^-134 of 8.2e-40: 5.6 %).  It stands in the block
+    of the largest score, and in an earlier one of the same wave (up to sixteen a workgroup, 32 keys each in turn), whose sums are
+    rescaled by e^-90."""
+    Hq, Hkv, D, page = geom
+    dtype = torch.bfloat16
+    n = 600
+    q, kc, vc, group, step = paged_setup([n], [1], Hq, Hkv, D, page, dtype, seed=D)
+    q.zero_()
+    q.view(1, Hq, D)[:, :, 0] = 1.0
+    window, kw = None, {}
+    if form == "sink":
+        kw = dict(sink=-100.0)
+    if form == "kept":
+        window, kw = n - 4, dict(keep_first=4)
+    if form == "chunk":
+        kw = dict(chunk=640)
+    if form == "biased":
+        kw = dict(distance_bias=torch.zeros(Hq, 30, device=DEV))
+    for small, ones in ((3, (9,)), (3, (515,)), (100, (20, 130))):
+        kc.zero_()
+        vc.zero_()
+        kc[..., 0] = -1000.0                             # the other keys: weights of e^-1000
+        for key, score, value in ((small, -90.0, 2.0 ** 100), *((k, 0.0, 0.0) for k in ones)):
+            pg, off = int(group.block_tables[0, key // page]), key % page
+            kc[pg, :, off, 0] = score
+            vc[pg, :, :, off] = value
+        out = ops[dtype].paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 1.0, window, num_splits=1, **kw)
+        want = math.exp(-90.0) * 2.0 ** 100 / len(ones)
+        assert bool(((out.double() / want - 1).abs() <= 0.056 + 2.0 ** -8).all()), (small, ones, float(out.double().min()), float(out.double().max()), want)
+
+
 LONG_DECODE = [  # (Hq, Hkv, D), contexts
     ((32, 4, 64), [4096]), ((32, 4, 64), [8192]), ((32, 8, 128), [8192]), ((32, 32, 128), [4096]),
     ((32, 8, 128), [8191, 5, 4097, 300, 6000, 64, 1, 2048]),
