@@ -755,6 +755,73 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 
 MIE_EXPORT const char* prefill_attention_bf16_last_error() { return g_mie_error; }
 
+enum PrefillKind { FOUR, EIGHT_QUERIES, EIGHT_KEYS };
+struct PrefillPlan {
+  PrefillKind kind;
+  bool paired;                // a workgroup takes a late stretch and an early one
+  int waves_h;
+  dim3 grid;
+};
+// How the stretches meet the compute units (a compute unit holds one workgroup of eight waves), at head sizes that leave room
+// for eight waves; measured at one row of 128 to 2,048 tokens behind 0, 1,000 and 4,096, 16 or 32 heads (MI355X, us):
+//   two halves over the keys, a stretch a workgroup, while that is no more than a workgroup a compute unit: in pairs half the
+//     compute units and twice the chain (512 tokens of 32 / 4 heads of 64 19 -> 14, of 32 / 8 of 128 behind 4,096 283 -> 153);
+//   else above head size 64 twice the queries, a stretch a workgroup, while that is: a step brings half the keys in for the same
+//     products (2,048 tokens of 32 / 8 of 128 alone 87 in halves and pairs, 84; behind 4,096 344 -> 229; at head size 64
+//     42 -> 55 and 150 -> 146, so not there).  At 128 that is four waves a workgroup instead, two workgroups a compute unit: they
+//     meet at no common barrier, so one's matrix instructions run beside the other's softmax (2,048 tokens alone 72 -> 62, behind
+//     4,096 198 -> 190, 1,100 behind 4,000 151 -> 137, 32 / 32 heads 73 -> 62; with four workgroups a compute unit 124 -> 126, 4,096
+//     tokens 153 -> 168, so not there; at 64, 2,048 tokens 38 -> 43);
+//   else two halves in pairs, while they are (two rounds of it, the second half empty, are slower: 2,560 tokens of 32 / 4 of 64
+//     95 us against 45 for 2,048);
+//   else twice the queries in pairs.
+static PrefillPlan prefill_plan(int rows, int max_row_tokens, int Hq, int Hkv, long units) {
+  const int G = Hq / Hkv;
+  PrefillPlan p{FOUR, true, 1, dim3(1)};
+  // the grid for `waves` waves a workgroup: waves side by side over the heads of a group (a power of two), the rest
+  // over 32-query tiles; a workgroup takes a late stretch and an early one (in pairs) or one stretch
+  auto plan = [&](int waves, bool in_pairs) {
+    int wh = 1;
+    while (wh < G && wh < waves) wh <<= 1;
+    const int head_chunks = (G + wh - 1) / wh;
+    const int stretch = (waves / wh) * PF_QW;
+    const long stretches = (max_row_tokens + stretch - 1) / stretch;
+    p.waves_h = wh;
+    p.grid = dim3((unsigned)(in_pairs ? (stretches + 1) / 2 : stretches), rows, Hkv * head_chunks);
+    return (long)p.grid.x * p.grid.y * p.grid.z;
+  };
+  if (PF_MAX_WAVES == 8) {
+    if (plan(4, false) <= units) { p.kind = EIGHT_KEYS; p.paired = false; }
+    else if (D > 64 && plan(8, false) <= units) { p.kind = PF_DIRECT ? FOUR : EIGHT_QUERIES; p.paired = false; }
+    else p.kind = plan(4, true) <= units ? EIGHT_KEYS : EIGHT_QUERIES;
+  }
+  plan(p.kind == EIGHT_QUERIES ? 8 : 4, p.paired);
+  return p;
+}
+static int device_compute_units(int& dev, long& units) {
+  dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("prefill_attention: no current device");
+  static int compute_units[64] = {};              // of each device, asked for once
+  if (compute_units[dev] <= 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      MIE_FAIL("prefill_attention: cannot read the number of compute units of device %d", dev);
+    compute_units[dev] = n;
+  }
+  units = compute_units[dev];
+  return 0;
+}
+// Which kernel rows of up to max_row_tokens tokens take: 0 four waves a workgroup, 1 eight over twice the queries, 2 eight in two
+// halves over the keys; 3, 4 and 5 the same with a late stretch and an early one a workgroup.
+MIE_EXPORT int mie_prefill_attention_kind(int rows, int max_row_tokens, int Hq, int Hkv) {
+  if (rows <= 0 || max_row_tokens <= 0 || Hkv <= 0 || Hq % Hkv) MIE_FAIL("prefill_attention: %d rows of %d tokens, %d / %d heads", rows, max_row_tokens, Hq, Hkv);
+  int dev;
+  long units;
+  if (device_compute_units(dev, units)) return -1;
+  const PrefillPlan p = prefill_plan(rows, max_row_tokens, Hq, Hkv, units);
+  return p.kind + (p.paired ? 3 : 0);
+}
+
 // Rows first_row .. first_row + rows - 1 of the step (those of more than one token).  q and out are
 // indexed by flat token; row_start [all rows + 1], row_position [all rows] as the step gives them, row_written (or null) [all
 // rows] too: a row's keys from there on are its padding tokens', which are not in its pages (null: rows have no padding tokens).
@@ -776,52 +843,12 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   if (q_stride < (long)Hq * D || (q_stride % 8) || ((uintptr_t)q % 16) || ((uintptr_t)out % 8))
     MIE_FAIL("prefill_attention: q stride %ld / alignment", q_stride);
   if (max_blocks <= 0) MIE_FAIL("prefill_attention: max_blocks %d", max_blocks);
-  const int G = Hq / Hkv;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("prefill_attention: no current device");
-  static int compute_units[64] = {};              // of each device, asked for once
-  if (compute_units[dev] <= 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      MIE_FAIL("prefill_attention: cannot read the number of compute units of device %d", dev);
-    compute_units[dev] = n;
-  }
-  // the grid for `waves` waves a workgroup: waves side by side over the heads of a group (a power of two), the rest
-  // over 32-query tiles; a workgroup takes a late stretch and an early one (in pairs) or one stretch
-  auto plan = [&](int waves, bool in_pairs, int* waves_h, dim3* grid) {
-    int wh = 1;
-    while (wh < G && wh < waves) wh <<= 1;
-    const int head_chunks = (G + wh - 1) / wh;
-    const int stretch = (waves / wh) * PF_QW;
-    const long stretches = (max_row_tokens + stretch - 1) / stretch;
-    *waves_h = wh;
-    *grid = dim3((unsigned)(in_pairs ? (stretches + 1) / 2 : stretches), rows, Hkv * head_chunks);
-    return (long)grid->x * grid->y * grid->z;
-  };
-  // How the stretches meet the compute units (a compute unit holds one workgroup of eight waves), at head sizes that leave room
-  // for eight waves; measured at one row of 128 to 2,048 tokens behind 0, 1,000 and 4,096, 16 or 32 heads (MI355X, us):
-  //   two halves over the keys, a stretch a workgroup, while that is no more than a workgroup a compute unit: in pairs half the
-  //     compute units and twice the chain (512 tokens of 32 / 4 heads of 64 19 -> 14, of 32 / 8 of 128 behind 4,096 283 -> 153);
-  //   else above head size 64 twice the queries, a stretch a workgroup, while that is: a step brings half the keys in for the same
-  //     products (2,048 tokens of 32 / 8 of 128 alone 87 in halves and pairs, 84; behind 4,096 344 -> 229; at head size 64
-  //     42 -> 55 and 150 -> 146, so not there).  At 128 that is four waves a workgroup instead, two workgroups a compute unit: they
-  //     meet at no common barrier, so one's matrix instructions run beside the other's softmax (2,048 tokens alone 72 -> 62, behind
-  //     4,096 198 -> 190, 1,100 behind 4,000 151 -> 137, 32 / 32 heads 73 -> 62; with four workgroups a compute unit 124 -> 126, 4,096
-  //     tokens 153 -> 168, so not there; at 64, 2,048 tokens 38 -> 43);
-  //   else two halves in pairs, while they are (two rounds of it, the second half empty, are slower: 2,560 tokens of 32 / 4 of 64
-  //     95 us against 45 for 2,048);
-  //   else twice the queries in pairs.
-  enum { FOUR, EIGHT_QUERIES, EIGHT_KEYS } kind = FOUR;
-  int waves_h;
-  dim3 grid;
-  bool paired = true;
-  if (PF_MAX_WAVES == 8) {
-    const long units = compute_units[dev];
-    if (plan(4, false, &waves_h, &grid) <= units) { kind = EIGHT_KEYS; paired = false; }
-    else if (D > 64 && plan(8, false, &waves_h, &grid) <= units) { kind = PF_DIRECT ? FOUR : EIGHT_QUERIES; paired = false; }
-    else kind = plan(4, true, &waves_h, &grid) <= units ? EIGHT_KEYS : EIGHT_QUERIES;
-  }
-  plan(kind == EIGHT_QUERIES ? 8 : 4, paired, &waves_h, &grid);
+  int dev;
+  long units;
+  if (device_compute_units(dev, units)) return -1;
+  const PrefillPlan plan = prefill_plan(rows, max_row_tokens, Hq, Hkv, units);
+  const PrefillKind kind = plan.kind;
+  const dim3 grid = plan.grid;
   if (grid.y > 65535 || grid.z > 65535) MIE_FAIL("prefill_attention: grid too large (%d rows)", rows);
   const float scale_log2 = sigmoid ? scale : scale * 1.4426950408889634f;      // the sigmoid kernels fold their own constants
   // more LDS than a kernel gets by default is asked for once per kernel and device
@@ -837,8 +864,8 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
     }
     hipLaunchKernelGGL(kernel, grid, dim3(waves * 64), lds_bytes, stream, (const bf16*)q, q_stride, (const bf16*)k_cache,
                        (const bf16*)v_cache, (bf16*)out, block_tables, max_blocks, row_start, row_position, row_written, first_row, Hq, Hkv,
-                       waves_h, page, scale_log2, window, sink_log2, chunk, softcap, head_bias, dist_bias, dist_n, keep,
-                       head_sinks, paired ? 1 : 0);
+                       plan.waves_h, page, scale_log2, window, sink_log2, chunk, softcap, head_bias, dist_bias, dist_n, keep,
+                       head_sinks, plan.paired ? 1 : 0);
     return 0;
   };
   int rc = 0;

@@ -1255,14 +1255,57 @@ def test_prefill_attention_ignores_stale_pages_bf16(ops):
     assert torch.equal(clean, dirty)
 
 
-# portions that take four waves, eight in two halves over the keys and eight over the queries; pages of 16 and 48; (kept keys, window,
-# chunk) of the forms that hide a row's first keys
-@pytest.mark.parametrize("form", ["plain", "window", "kept", "chunk", "sigmoid", "sigmoid chunk", "biased"])
-@pytest.mark.parametrize("geom", [(8, 2, 64, 16, 170, 29, 48), (32, 4, 64, 48, 600, 333, 512), (4, 4, 256, 16, 90, 35, 64), (16, 8, 128, 16, 1500, 1025, 1400)])
+# (heads, kv heads, head size, page, context, tokens of the step that are the row's own, with padding) and the kernel that each takes
+PREFILL_KINDS = {
+    "four waves, in pairs": (4, 4, 256, 16, 90, 35, 64), "four waves of size 128, two workgroups a compute unit": (32, 8, 128, 16, 1500, 1200, 1300),
+    "four waves, pages of 48": (32, 32, 128, 48, 1300, 1100, 1200),
+    "keys in halves": (8, 2, 64, 16, 170, 29, 48), "keys in halves, pages of 48": (32, 4, 64, 48, 600, 333, 512),
+    "keys in halves, size 128": (16, 8, 128, 16, 1500, 1025, 1400), "keys in halves, in pairs": (128, 128, 64, 48, 450, 300, 400),
+    "twice the queries": (96, 96, 80, 16, 640, 500, 512),
+    "twice the queries, in pairs": (128, 128, 64, 16, 700, 600, 650), "twice the queries, in pairs, size 128": (128, 128, 128, 16, 700, 600, 650)}
+PREFILL_KIND = {"four waves": 0, "four waves, in pairs": 3, "keys in halves": 2, "keys in halves, in pairs": 5, "twice the queries": 1,
+                "twice the queries, in pairs": 4}
+PREFILL_FORMS = ["plain", "window", "kept", "chunk", "sigmoid", "sigmoid chunk", "biased"]
+
+
+def prefill_case(ops, name):
+    """The geometry, after a look at whether its step takes the kernel that it is here for."""
+    geom = PREFILL_KINDS[name]
+    Hq, Hkv, D, _, _, _, padded = geom
+    what = max((k for k in PREFILL_KIND if name.startswith(k)), key=len)
+    lib = ops[torch.bfloat16].lib("prefill_attention_bf16", (f"-DHEAD_DIM={D}",))
+    assert lib.mie_prefill_attention_kind(1, padded, Hq, Hkv) == PREFILL_KIND[what], name
+    return geom
+
+
+@pytest.mark.parametrize("form", PREFILL_FORMS)
+@pytest.mark.parametrize("name", PREFILL_KINDS)
+def test_prefill_attention_kinds(ops, name, form):
+    """Every kernel that a portion can take, in every form, behind earlier keys: tokens at the edges of tiles and stretches and some
+    between, against 64 bits.  Half an ulp of bfloat16 each for a weight, for what their rounding adds to the denominator and for the
+    result is 3 * 2^-9 of a head's result in the 2-norm; 2^-7 allows for a token's values being few."""
+    Hq, Hkv, D, page, n, real, padded = prefill_case(ops, name)
+    n, real = n + padded - real, padded                # the whole length is the row's own
+    dtype = torch.bfloat16
+    q, kc, vc, group, step = paged_setup([n], [real], Hq, Hkv, D, page, dtype, seed=D + n)
+    window, kw = {"window": (45, {}), "kept": (70, dict(keep_first=5)), "chunk": (None, dict(chunk=72)), "sigmoid": (None, dict(weights="sigmoid")),
+                  "sigmoid chunk": (None, dict(weights="sigmoid", chunk=72)),
+                  "biased": (None, dict(distance_bias=torch.randn(Hq, 200, device=DEV)))}.get(form, (None, {}))
+    out = ops[dtype].paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 1.1 / math.sqrt(D), window, **kw)
+    at = sorted({t for e in (0, 32, 64, 128, 256, real // 2, real) for t in (e - 1, e, e + 1) if 0 <= t < real} | set(range(7, real, real // 12)))
+    want = ref.ref_paged_attention(q[at], Hq, Hkv, D, kc, vc, group.block_tables, step.token_row[at], step.positions[at], 1.1 / math.sqrt(D),
+                                   window, torch.float64, **kw).view(len(at), Hq, D)
+    error = (out[at].double().view(len(at), Hq, D) - want).norm(dim=-1) / want.norm(dim=-1)
+    assert float(error.max()) <= 2.0 ** -7, (at[int(error.max(1).values.argmax())], float(error.max()))
+
+
+# every kernel that a portion can take; (kept keys, window, chunk) of the forms that hide a row's first keys
+@pytest.mark.parametrize("form", PREFILL_FORMS)
+@pytest.mark.parametrize("geom", PREFILL_KINDS)
 def test_prefill_attention_looks_at_no_slot_its_row_did_not_write(ops, geom, form):
     """A row lengthened with padding tokens, whose keys are not in its pages, with NaN in every slot the row did not write and in
     the pages whose keys lie before all its queries' first: its own tokens get the bits they get from a cache of zeros there."""
-    Hq, Hkv, D, page, n, real, padded = geom
+    Hq, Hkv, D, page, n, real, padded = prefill_case(ops, geom)
     dtype = torch.bfloat16
     q, kc, vc, group, step = paged_setup([n], [real], Hq, Hkv, D, page, dtype, seed=D + n)
     window, kw, first = None, {}, 0
