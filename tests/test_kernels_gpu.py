@@ -113,16 +113,17 @@ def test_linear_float32_is_batch_invariant(ops):
     for a, b in ((0, 1), (63, 130), (199, 200), (17, 19)):
         assert torch.equal(ops[torch.float32].linear(x[a:b].contiguous(), w), whole[a:b])
 
-# (rows, K, N): few rows and many, K with quarters and segments missing (4, 16, 176), one step beyond a stage, tile edges
+# (rows, K, N): few rows and many, K with quarters and eighths missing (4, 64, 176: steps of 32, then quarters, then eighths), a step
+# cut short, tile edges
 F32_SHAPES = [(1, 2048, 2048), (16, 176, 64), (5, 4, 36), (17, 64, 132), (64, 1040, 260), (65, 528, 4100), (128, 2048, 96),
               (300, 332, 640), (513, 256, 8196)]
 
 
 @pytest.mark.parametrize("shape", F32_SHAPES)
 def test_linear_float32_matrix_unit(ops, shape):
-    """The 32-bit products on the matrix unit: against 64 bits within the worst case of their chains (K / 16 terms in a
-    segment, 32 joins; half an ulp each of the sum of magnitudes), a row the same bits in any cut (few-row kernel, tiles,
-    units of K), the added and the gated form the same bits as the product and a step of its own."""
+    """The float32 products on the matrix unit: against 64 bits within K / 16 + 32 half ulps of the sum of magnitudes (half the worst
+    case of an eighth's chain of K / 8 products; the joins, the small products' chain and the products left out, 2^-24 together), a row the
+    same bits in any cut (few-row kernel, tiles, units of K), the added and the gated form the same bits as the product and a step of its own."""
     M, K, N = shape
     o = ops[torch.float32]
     torch.manual_seed(M + N)
@@ -147,8 +148,8 @@ def test_linear_float32_matrix_unit(ops, shape):
     assert torch.equal(o.linear(x, w, bias=bias), y + bias)
 
 
-# rows that take the few-row kernel (two steps at once, one), the small tile in eighths and whole, the large ones in quarters and
-# whole; K with an odd number of steps for a wave, without any for most, and a step cut short
+# rows that take the few-row kernel (two steps at once, one), the tiles in eighths, whole and in quarters; K with an odd number of
+# steps for a wave, without any for most, and a step cut short
 F32_PARTS = [(3, 2080, 48), (12, 2080, 48), (40, 1056, 64), (20, 36, 352), (300, 2048, 2048), (1100, 96, 2304), (600, 352, 9000)]
 
 
@@ -195,6 +196,23 @@ F32_FORMS = [(3, 2080, 48, 0), (12, 2080, 48, 0), (600, 352, 9000, 1), (300, 204
 
 def f32_parts_of_k(o, M, K, N):
     return o.lib("gemm_f32").mie_f32_units(M, N, K, 0) if M > 16 else 0
+
+
+@pytest.mark.parametrize("K", [28, 36, 60, 68, 124, 132, 252, 260, 508, 516, 1020, 1028])
+def test_linear_float32_at_the_edges_of_the_cuts_of_k(ops, K):
+    """A step more or less than fills K's quarters and eighths: the few-row kernel, the tiles in eighths, in quarters and
+    whole give a row the same bits, as exact as K = 2,048 is asked to be."""
+    o = ops[torch.float32]
+    forms = [(3, 64), (12, 64), (40, 64), (300, 640), (700, 1100)]
+    assert f32_parts_of_k(o, 2100, K, 4100) == 1
+    assert f32_parts_of_k(o, 40, K, 64) == (1 if K < 128 else 8) and f32_parts_of_k(o, 300, K, 640) == (1 if K < 500 else 4)
+    torch.manual_seed(K)
+    x, w = torch.randn(2100, K, device=DEV), torch.randn(4100, K, device=DEV)
+    exact = x.double() @ w.double().T
+    whole = o.linear(x, w)
+    assert (whole.double() - exact).norm() <= 2.0 ** -24 * math.sqrt(K / 16 + 8) * exact.norm()
+    for M, N in forms:
+        assert torch.equal(o.linear(x[:M].contiguous(), w[:N].contiguous()), whole[:M, :N]), (M, N)
 
 
 @pytest.mark.parametrize("shape", F32_FORMS)

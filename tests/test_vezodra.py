@@ -544,15 +544,36 @@ def test_joined_norms_of_many_tokens(hip, dtype, width, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, K", [(2048, 4), (64, 1), (1028, 6)])
+def test_joined_norms_do_not_depend_on_the_cut(hip, dtype, width, K):
+    """A row's results and the tail it leaves are the same bits in a step of its own and in one of 1,024 tokens and more."""
+    ops, g = hip[dtype], torch.Generator().manual_seed(width + K)
+    counts, slots = [1, 700, 2, 330, 5], [4, 1, 3, 2, 7]
+    step = FakeStep(counts, slots)
+    stream = _rand((step.num_tokens, width), torch.float32, g, 2.0)
+    w1, w2 = _rand((width,), torch.float32, g) + 1, _rand((width,), torch.float32, g) + 1
+    taps, tail = _rand((width, K), torch.float32, g, 0.5), _rand((9, max(1, K - 1), width), torch.float32, g)
+    own_tail, seen, at = tail.clone(), [], 0
+    whole = ops.norm_pair_conv(stream, w1, w2, 1e-5, taps, tail, step)
+    for n, slot in zip(counts, slots):
+        seen.append(ops.norm_pair_conv(stream[at:at + n].contiguous(), w1, w2, 1e-5, taps, own_tail, FakeStep([n], [slot])))
+        at += n
+    for a, parts in zip(whole, zip(*seen)):
+        assert torch.equal(a, torch.cat(parts))
+    assert torch.equal(tail, own_tail)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("form", [
     # Hq, Hkv, dim, vdim, P, nf, layout, norms (whole, a head, none), own values, page
     (32, 4, 64, 64, 64, 32, "half", "whole", True, 16), (16, 4, 128, 128, 128, 32, "interleaved", "none", False, 16),
     (4, 2, 16, 24, 32, 4, "half", "head", True, 48), (3, 1, 40, 32, 48, 20, "interleaved", "whole", True, 16),
     (40, 8, 128, 128, 128, 64, "half", "head", True, 16), (60, 10, 128, 128, 128, 0, "half", "whole", True, 32),
-    (6, 2, 40, 40, 48, 8, "half", "head", True, 16)])      # (pieces of a head no power of two: the wave a head)
+    (6, 2, 40, 40, 48, 8, "half", "head", True, 16)])      # (pieces of a head no power of two)
 def test_attention_preparation_in_pieces(hip, dtype, form):
     """Many tokens with sizes in pieces of 8: one, two and four pieces a thread, heads padded and partly turned, values of
-    their own size, and a row of sums whose columns are off 16 bytes (the wave a head) with the same result."""
+    their own size, and a row of sums whose columns are off 16 bytes (the wave a head), each against the reference."""
     Hq, Hkv, dim, vdim, P, nf, layout, norms, own_v, page = form
     ops, g = hip[dtype], torch.Generator().manual_seed(Hq + dim + nf)
     T = 261
