@@ -872,6 +872,25 @@ def test_families_bfloat16_gpu(name, family, tmp_path):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", CONFIGS)
+def test_float32_logits_do_not_depend_on_the_cut_gpu(name):
+    """Prompts of 300 and 290 tokens whole, both in one step, in portions of 200, in small ones and token by token at their ends:
+    every logit has the same bits."""
+    raw, cfg, weights = make(name)
+    prompts = trace_util.random_prompts(raw["vocab"], [300, 290], seed=4)
+
+    def run(steps):
+        runner = ModelRunner(cfg, weights=weights, dtype="float32", device="cuda", num_pages=64, max_rows=4, max_step_tokens=640, max_model_len=320)
+        return trace_util.run_on_runner(runner, steps)
+    base = run(trace_util.whole(prompts))
+    together = [{"step": 0, "entries": [{"id": k, "tokens": t, "want": list(range(len(t)))} for k, t in prompts.items()], "end": list(prompts)}]
+    for what, steps in (("together", together), ("portions of 200", trace_util.portions(prompts, sizes=(200, 100))),
+                        ("portions", trace_util.portions(prompts)), ("tails", trace_util.decode_tail(prompts, 40))):
+        for key, row in run(steps).items():
+            assert torch.equal(row, base[key]), f"{what}: request {key[0]} position {key[1]} differs from whole"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_greedy_generation_gpu(dtype):
     eng = generate("A", "cuda", dtype)
