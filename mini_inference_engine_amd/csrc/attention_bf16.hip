@@ -8,8 +8,8 @@
 // The scores come out with lane % 16 = head and 4 consecutive keys per lane group; that is already
 // the layout P^T needs as the B operand of the second product if the 32 keys of its reduction are
 // taken in the order (lane group, tile, i), and the value operand is loaded in that same order, so the
-// probabilities never leave registers.  Softmax state (max, sum) is one value per lane (its head);
-// exponentials are base 2 with scale * log2(e) folded into the scores.  The waves of a workgroup are
+// probabilities never leave registers.  Softmax state is one value per lane: the maximum of its head, the sum over
+// its own keys of the head's (a head's four lanes join after the last block); exponentials are base 2 with scale * log2(e) folded into the scores.  The waves of a workgroup are
 // merged through LDS; splits write normalised partials and base-2 log-sum-exps, merged by a second,
 // small kernel.  Keys outside [lo, p] get probability 0 by selection and their values are zeroed, so stale
 // or poisoned slots never reach the sums.

@@ -643,7 +643,9 @@ norm_pair_conv_vec_kernel(const float* __restrict__ stream, const float* __restr
 // The same for steps of many tokens and widths up to 2048: a workgroup takes NT tokens in a row and holds them, and the K - 1
 // before them, in registers.  One token a workgroup reads K rows twice and all taps, 112 KB a token at a width of 2,048, and the
 // traffic out of the L2s bounds it; four tokens a workgroup read 7 rows once and the taps once, 26 KB a token, and every load is on
-// its way before the first is used.  2,048 tokens of 2,048, bfloat16 out (MI355X, us): 28.6 / 16.6.
+// its way before the first is used.  2,048 tokens of 2,048, bfloat16 out (MI355X, us): 28.6 / 16.6.  Twice the width would gain as well
+// (NPC_TILE_V 4, another harness: 2,048 tokens of 4,096 48.4 / 29.3, of 3,072 39.4 / 24.5, of 2,048 19.0 for 2 and 19.3 for 4) and is
+// not built.
 constexpr int NPC_TOKENS = 4, NPC_TILE_V = 2;
 template <typename TO, int K>
 __global__ void __launch_bounds__(NORM_THREADS)

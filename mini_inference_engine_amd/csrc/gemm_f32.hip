@@ -32,12 +32,14 @@
 //   before is multiplied.  Few tiles: the grid is also cut over quarters or eighths, whose sums go to memory and meet in
 //   reduce_f32_kernel.
 //
-// Measured on MI355X against the same kernels on v_mfma_f32_16x16x4_f32 (us; before / now): 512 rows of [11264, 2048] with SwiGLU
-// 237 / 175, [2048, 5632] 116 / 73, [2048, 2048] 51 / 35; 100 rows 69 / 59, 36 / 29, 21 / 16; 4 rows 21.9 / 19.2, 17.0 / 14.8, 8.8 / 8.3.
-// Steps of the engine, 22 layers of width 2,048: a prompt of 512 tokens 11,617 / 8,291, 4 rows 1,699 / 1,616.  Relative error of
-// [2048, 2048] against 64 bits 2.1e-7 / 1.0e-7, of [2048, 5632] 3.4e-7 / 1.6e-7, of a whole step's logits 2.1e-6 / 1.3e-6 (with the small
-// products in the chain of hh it would be 2.4e-7 and 4.1e-7).  What is left in the tile kernel: matrix instructions alone take 63 us
-// for 2,048 rows of [2048, 2048] (the clock falls with every compute unit at them), the fragment reads add 15, splitting 17.
+// Measured on MI355X against the same kernels on v_mfma_f32_16x16x4_f32, both without the factor of 2^16 (us; those / these): 512 rows of
+// [11264, 2048] with SwiGLU 237 / 175, [2048, 5632] 116 / 73, [2048, 2048] 51 / 35; 100 rows 69 / 59, 36 / 29, 21 / 16; 4 rows 21.9 / 19.2,
+// 17.0 / 14.8, 8.8 / 8.3.  Without / with the factor, another harness: 512 rows 171 / 166, 71.5 / 70.9, 33.3 / 33.2, 4 rows 18.0 / 18.1,
+// 14.9 / 15.1.  Steps of the engine, 22 layers of width 2,048, 32-bit instruction / these: a prompt of 512 tokens 11,637 / 8,775, 4
+// rows 1,700 / 1,628.  Relative error of [2048, 2048] against 64 bits 2.1e-7 / 1.0e-7, of [2048, 5632] 3.4e-7 / 1.6e-7, of a whole step's
+// logits 2.2e-6 / 1.5e-6 (with the small products in the chain of hh it would be 2.4e-7 and 4.1e-7).  What is left in the tile
+// kernel: matrix instructions alone take 63 us for 2,048 rows of [2048, 2048] (the clock falls with every compute unit at them), the
+// fragment reads add 15, the splitting the rest of its 93.
 #include "launch.hpp"
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));

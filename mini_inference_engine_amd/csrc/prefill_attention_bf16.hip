@@ -24,11 +24,15 @@
 // so that a lane's scores are runs of eight keys (row 4 g + j of 16 is key 8 g + j, row 8 + 4 g + j key 8 g + 4 + j), and the
 // values are taken in that order.  At other head sizes through registers (two LDS buffers and two sets of
 // registers: block i + 1 waits in registers while block i is computed, block i + 2 is on its way, the pages
-// of block i + 3 are looked up), in rows padded so that the fragment reads meet no bank conflict.  The more
-// queries share a block the better for what comes out of the L2s.  What bounds it at head size 128 (2,048 tokens behind 4,096,
-// counters): matrix unit 46 % and vector unit 49 % of the cycles, one after the other behind the common barrier, the LDS reads of
-// 256 KB a step as long as either; at 64 (2,048 tokens): vector unit 50 %, matrix unit 21 %, and 8 of 39 us are starts and ends.
-// 2,048 tokens of 32 / 4 heads of 64 through registers / directly 45 / 39 us, of 32 / 8 of 128 behind 4,096 279 / 190 (MI355X).  Work per stretch grows with its place in the row (causal), so where stretches outnumber the
+// of block i + 3 are looked up), in rows padded so that the fragment reads meet no bank conflict: the swizzle of the direct ring needs
+// rows of a power of two of 16-byte blocks, which 48, 80, 96, 112 and 192 have not; 16, 32 and 256 have them, but were not measured.  The
+// more queries share a block the better for what comes out of the L2s.  What bounds it at head size 128 (2,048 tokens behind 4,096, two
+// workgroups of four waves a compute unit, counters): matrix unit 46 % and vector unit 48 % of the cycles; the two workgroups overlap
+// them in part (209 us under the tracer; one workgroup of eight waves, where they follow each other behind the common barrier, 221), and
+// the LDS reads of 256 KB a step take as long as either.  At 64 (2,048 tokens): vector unit 45 %, matrix unit 21 %, and 8 of 39 us are
+// starts and ends.
+// 2,048 tokens of 32 / 4 heads of 64 through registers / directly 45 / 39 us, of 32 / 8 of 128 behind 4,096 279 / 190 (MI355X).
+// Work per stretch grows with its place in the row (causal), so where stretches outnumber the
 // compute units a workgroup takes stretch NS - 1 - i and then stretch i: every workgroup of a row has the same number of blocks.  A block every
 // query of a wave sees whole takes a path without masks; the running maximum m is kept in units of
 // scale * log2(e); l is a per-lane partial sum, joined over a query's two lanes at the end.
