@@ -615,7 +615,8 @@ def test_attention_preparation_in_pieces(hip, dtype, form):
     # Hq, Hkv, dim, vdim, P, nf, layout, norms, own values
     (32, 4, 64, 64, 64, 32, "half", "whole", True), (16, 4, 128, 128, 128, 32, "interleaved", "whole", False),
     (4, 2, 16, 24, 32, 4, "half", "head", True), (3, 1, 40, 32, 48, 20, "interleaved", "whole", True),
-    (40, 8, 128, 128, 128, 64, "half", "head", True), (5, 3, 72, 72, 128, 36, "half", "head", True), (60, 10, 128, 128, 128, 0, "half", "whole", True)])
+    (40, 8, 128, 128, 128, 64, "half", "head", True), (5, 3, 72, 72, 128, 36, "half", "head", True), (60, 10, 128, 128, 128, 0, "half", "whole", True),
+    (110, 8, 128, 128, 128, 64, "half", "whole", True), (112, 8, 128, 128, 128, 64, "half", "head", True)])      # 60 KB of LDS, and beyond
 def test_attention_preparation_does_not_depend_on_the_cut(hip, dtype, form):
     """A token's queries, keys and values are the same bits in steps of few tokens and of many, and where rows lie off 16 bytes."""
     Hq, Hkv, dim, vdim, P, nf, layout, norms, own_v = form
