@@ -1,21 +1,26 @@
-// Matrix products of the bfloat16 path with 17 to 128 rows and a narrow weight (N up to a few thousand):
-// decode steps of many requests.  The few-row kernel (gemm_bf16.hip) gives every 16 weight rows a
-// workgroup that reads all of x, which at 64 rows is four times the weights' bytes; a library product
-// runs such a shape on a few dozen workgroups.  Here
+// Matrix products of the bfloat16 path with 17 to 128 rows: decode steps of many requests.
 //
-//   part[s, m, n] = sum over the k of split s of x[m, k] W[n, k]
+//   part[s, m, n] = sum over the k of split s of x[m, k] W[n, k]         (narrow weights: q/k/v, o, down)
+//   out[m, j]     = silu(gate[m, j]) * up[m, j]  on their float32 sums   (gate and up, all of K in one workgroup)
 //
-// a workgroup of 4 waves owns 64 weight rows and one contiguous range of K (the split); k-steps of W
-// and of x (all rows) are brought into a ring of LDS stages by loads that write the LDS directly, 1 KB a
-// fragment (16 rows x 32 k), so x is read once per 64 weight rows; wave w multiplies its 16 weight rows
-// with v_mfma_f32_16x16x32_bf16.  The split's sums go out as float32 partial results.
-// A fragment is brought in by lane 4 r + b reading k-block b ^ (r / 4) % 4 of row r (16 bytes): a quarter
-// wave then reads 64 contiguous bytes of 4 rows (in the matrix instruction's own order, lane 16 b + r, it
-// touches 16 cache lines for 16 bytes each, and the address unit's line look-ups bound the kernel), and the
-// permutation of the blocks spreads the fragment reads (lane 16 b + r reads slot 4 r + (b ^ (r / 4) % 4))
-// over all banks.
-// The number of splits is chosen by the caller from the weight's shape alone, so a row's result does
-// not depend on the batch it is in.
+// The few-row kernel (gemm_bf16.hip) gives every 16 weight rows a workgroup that reads all of x, which at 64 rows is four
+// times the weights' bytes; a library product runs a narrow weight on a few dozen workgroups.  What a compute unit takes in
+// is what bounds these products: 58 bytes a nanosecond at most, out of the L2 as well as from memory (measured by a kernel
+// that only loads, whatever the access pattern, the depth or who shares the lines).  So a workgroup owns TW tiles of 16
+// weight rows, as many as give every compute unit one workgroup, and x is read once per 16 TW weight rows.
+//
+// Its waves share no loads and meet at no barrier in the loop: chunks of 64 k are dealt to them in turn, a wave brings a
+// chunk of all its weight rows and all x rows into its own slots of the LDS by loads that write the LDS directly (8 rows of
+// 128 bytes a load, whole cache lines; block b of row r at 16-byte place 8 r + (b ^ r % 8), so that the fragment reads are
+// spread over all banks), reads all fragments into registers, asks for the chunk after into the same slot at once and then
+// multiplies (v_mfma_f32_16x16x32_bf16).  The waves' sums meet in the LDS, in wave order.  Weights by nontemporal loads.
+// Before, four waves that shared a ring of stages met at a barrier a stage: a stage of 16 KB took 0.4 to 0.6 us whatever it
+// loaded.  Measured (MI355X, us, before / now): with the sums' kernel and the norm, 24 rows of [2048, 2048] 8.5 / 7.3, [2560, 2048]
+// 9.9 / 8.4, [2048, 5632] 11.9 / 9.7, [4096, 14336] 34.3 / 24.9; 64 rows 9.9 / 8.9, 11.2 / 10.2, 13.2 / 12.3, 33.4 / 30.2.  Gate and
+// up against the library's product and silu_mul: [11264, 2048] 17 / 64 / 128 rows 17.6 / 10.9, 19.9 / 13.7, 22.7 / 18.4;
+// [28672, 4096] 17 / 64 rows 55.4 / 43, 57.1 / 47.5.
+// The number of splits and of tiles a workgroup depends on the weight's shape alone and chunks go to waves by their place in
+// K, so a row's result does not depend on the batch it is in.
 //
 // The kernels that follow add the partial results up in split order and do what comes after the product:
 //   reduce_rows:     store (bfloat16 / float32), or add into the 32-bit stream, or add and RMSNorm for
@@ -27,165 +32,146 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-union Frag {
-  bf16x8 v;
-  uint4 q;
-};
-
-constexpr int MID_WAVES = 4;      // waves a workgroup = 16-row weight tiles a workgroup
-constexpr int MID_KC = 2;         // k-steps (of 32) a stage
-constexpr int MID_STAGES = 4;     // stages in the ring (eight were measured: no faster)
-constexpr int FRAG_BYTES = 1024;  // one operand fragment: 64 lanes x 16 bytes
-
-// The fragments of one k-step out of the LDS: the wave's weight fragment (at wbase) and the x fragments of all
-// row tiles (1 KB apart from xbase), read and waited for in one piece of assembly.  The compiler knows nothing
-// of the loads that write the LDS, so a read of the LDS it could see would make it wait for every load on its
-// way; and it must never see a register whose value is still to arrive (it may move it), so the wait is part
-// of the same piece.  OFF: byte offset of the k-step within the stage, XOFF: of its first x fragment.
-template <int MT, int OFF, int XOFF>
-struct LdsFragments;
-template <int OFF, int XOFF>
-struct LdsFragments<4, OFF, XOFF> {
-  static __device__ __forceinline__ void read(uint32_t wbase, uint32_t xbase, u32x4& w, u32x4 (&x)[4]) {
-    asm volatile(
-      "ds_read_b128 %0, %5 offset:%7\n\t"
-      "ds_read_b128 %1, %6 offset:%8\n\t"
-      "ds_read_b128 %2, %6 offset:%8+1024\n\t"
-      "ds_read_b128 %3, %6 offset:%8+2048\n\t"
-      "ds_read_b128 %4, %6 offset:%8+3072\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(w), "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
-      : "v"(wbase), "v"(xbase), "n"(OFF), "n"(XOFF)
-      : "memory");
-  }
-};
-template <int OFF, int XOFF>
-struct LdsFragments<8, OFF, XOFF> {
-  static __device__ __forceinline__ void read(uint32_t wbase, uint32_t xbase, u32x4& w, u32x4 (&x)[8]) {
-    asm volatile(
-      "ds_read_b128 %0, %9 offset:%11\n\t"
-      "ds_read_b128 %1, %10 offset:%12\n\t"
-      "ds_read_b128 %2, %10 offset:%12+1024\n\t"
-      "ds_read_b128 %3, %10 offset:%12+2048\n\t"
-      "ds_read_b128 %4, %10 offset:%12+3072\n\t"
-      "ds_read_b128 %5, %10 offset:%12+4096\n\t"
-      "ds_read_b128 %6, %10 offset:%12+5120\n\t"
-      "ds_read_b128 %7, %10 offset:%12+6144\n\t"
-      "ds_read_b128 %8, %10 offset:%12+7168\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(w), "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
-      : "v"(wbase), "v"(xbase), "n"(OFF), "n"(XOFF)
-      : "memory");
-  }
-};
-
-// One stage = KC k-steps; a k-step holds the waves' weight fragments, then the x fragments of the row tiles.
-template <int MT, int kc>
-struct StageReader {
-  static constexpr int SF = MID_WAVES + MT;
-  static_assert(FRAG_BYTES == 1024, "the offsets in LdsFragments");
-  static __device__ __forceinline__ void run(uint32_t base, uint32_t wbase, f32x4 (&acc)[MT]) {
-    u32x4 w, x[MT];
-    LdsFragments<MT, kc * SF * FRAG_BYTES, (kc * SF + MID_WAVES) * FRAG_BYTES>::read(wbase, base, w, x);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      Frag a, b;
-      a.q = *reinterpret_cast<uint4*>(&x[mt]);
-      b.q = *reinterpret_cast<uint4*>(&w);
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[mt], 0, 0, 0);
-    }
-    if constexpr (kc + 1 < MID_KC) StageReader<MT, kc + 1>::run(base, wbase, acc);
-  }
-};
-
-// grid (ceil(N / 64), splits).  zeros: 64 bytes of zeros in device memory (what a k-step beyond the range
-// or beyond K loads instead, so that every load is unconditional).  part [splits, M, N] float32.
-template <int MT>
-__global__ void __launch_bounds__(MID_WAVES * 64)
-mid_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, float* __restrict__ part,
-                int M, int N, int K, int kper, const bf16* __restrict__ zeros) {
-  extern __shared__ __align__(16) char lds[];
-  constexpr int SF = MID_WAVES + MT;                       // fragments a k-step
-  constexpr int STAGE_BYTES = MID_KC * SF * FRAG_BYTES;
-  static_assert((MT * MID_KC) % MID_WAVES == 0, "the x fragments of a stage must divide over the waves");
-  constexpr int XL = MT * MID_KC / MID_WAVES;              // x fragments a wave brings in per stage
-  constexpr int L = MID_KC + XL;                           // loads a wave issues per stage
-  static_assert((MID_STAGES - 2) * L <= 63, "more loads in flight than the counter holds");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 15, kb = lane >> 4;
-  const int lrow = lane >> 2, lkb = (lane & 3) ^ ((lrow >> 2) & 3);     // the row and k-block this lane brings in
-  const int rslot = col * 4 + (kb ^ ((col >> 2) & 3));                  // where this lane's piece of a fragment sits
-  const int ksteps = (K + 31) >> 5;
-  const int ksA = blockIdx.y * kper, ksB = ksA + kper < ksteps ? ksA + kper : ksteps;
-  const int nst = (ksB - ksA + MID_KC - 1) / MID_KC;
-  const int n = (blockIdx.x * MID_WAVES + wave) * 16 + col;
-  const int nl = (blockIdx.x * MID_WAVES + wave) * 16 + lrow;
-  const bf16* wrow = W + (size_t)(nl < N ? nl : N - 1) * ldw + lkb * 8;
-  const bf16* xptr[XL];
-  int xkc[XL], xlds[XL];
-#pragma unroll
-  for (int j = 0; j < XL; ++j) {
-    const int f = wave * XL + j, kc = f / MT, mt = f % MT;
-    const int m = mt * 16 + lrow;
-    xptr[j] = X + (size_t)(m < M ? m : 0) * ldx + kc * 32 + lkb * 8;
-    xkc[j] = kc;
-    xlds[j] = (kc * SF + MID_WAVES + mt) * FRAG_BYTES;
-  }
-  const bf16* zero_lane = zeros + lkb * 8;     // a per-lane address, so that choosing it is a select and no branch
-  auto issue = [&](int s) {
-    char* base = lds + (s % MID_STAGES) * STAGE_BYTES;
-    const int ks = ksA + s * MID_KC;
-#pragma unroll
-    for (int kc = 0; kc < MID_KC; ++kc) {
-      const bool ok = ks + kc < ksB && (ks + kc) * 32 + lkb * 8 < K;
-      const bf16* src = ok ? wrow + (size_t)(ks + kc) * 32 : zero_lane;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(base + (kc * SF + wave) * FRAG_BYTES), 16, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < XL; ++j) {
-      const bool ok = ks + xkc[j] < ksB && (ks + xkc[j]) * 32 + lkb * 8 < K;
-      const bf16* src = ok ? xptr[j] + (size_t)ks * 32 : zero_lane;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(base + xlds[j]), 16, 0, 0);
-    }
-  };
-  f32x4 acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
-  // stages beyond the split's range load zeros only, so the ring is always filled and drained the same way
-  for (int s = 0; s < MID_STAGES - 1; ++s) issue(s);
-  for (int it = 0; it < nst; ++it) {
-    MIE_VMCNT((MID_STAGES - 2) * L);           // this wave's loads of stage `it` have landed
-    __builtin_amdgcn_s_barrier();              // and everybody else's; everybody is done reading stage it - 1
-    issue(it + MID_STAGES - 1);                // into the buffer stage it - 1 used
-    const uint32_t base = lds0 + (it % MID_STAGES) * STAGE_BYTES + rslot * 16;
-    StageReader<MT, 0>::run(base, base + wave * FRAG_BYTES, acc);
-  }
-  MIE_VMCNT(0);                                // nothing of this wave may still be writing the LDS when it ends
-  float* out = part + (size_t)blockIdx.y * M * N;
-  // acc[mt][i]: x row mt * 16 + 4 kb + i (the A operand's rows), weight row n (the B operand's column)
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = mt * 16 + kb * 4 + i;
-      if (m < M && n < N) out[(size_t)m * N + n] = acc[mt][i];
-    }
-}
-
-// ---------------------------------------------------------------------------- after the product
-enum { RED_STORE_BF16 = 0, RED_STORE_F32 = 1, RED_ADD = 2, RED_ADD_NORM = 3 };
-constexpr int RED_THREADS = 512;
-constexpr int RED_VEC = 4;        // float4 a thread: rows up to 8192 wide
-
 __device__ __forceinline__ void store_bf16x4(bf16* p, float4 v) {
   uint2 u;
   u.x = (uint32_t)__bfloat16_as_ushort(__float2bfloat16(v.x)) | ((uint32_t)__bfloat16_as_ushort(__float2bfloat16(v.y)) << 16);
   u.y = (uint32_t)__bfloat16_as_ushort(__float2bfloat16(v.z)) | ((uint32_t)__bfloat16_as_ushort(__float2bfloat16(v.w)) << 16);
   *reinterpret_cast<uint2*>(p) = u;
 }
+
+enum { MID_PART = 0, MID_SWIGLU = 1 };
+constexpr int MID_WAVES = 4;      // more waves (six, eight) and fewer slots a wave: no faster at any shape
+
+// MT: tiles of 16 x rows.  TW: tiles of 16 weight rows; with SWIGLU a tile is 8 gate rows and the up rows of
+// the same columns, W = [gate rows (N of them); up rows].  TAIL: K is no multiple of 64.
+// grid (weight tiles / TW, splits), `per` chunks a split; part [splits, M, N] float32, or out [M, ldo] bfloat16.
+template <int TW, int MT, int SLOTS, int EPI, bool TAIL>
+__global__ void __launch_bounds__(MID_WAVES * 64)
+mid_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, void* __restrict__ outv, long ldo,
+                int M, int N, int K, int per) {
+  constexpr int SLOT = (TW + MT) * 2048, L = 2 * (TW + MT);
+  static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
+  extern __shared__ __align__(1024) char mid_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kb = lane >> 4;
+  const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;      // this lane's place in a load of 8 rows
+  constexpr int COLS = EPI == MID_SWIGLU ? 8 : 16;           // columns of a tile
+  const int j0 = blockIdx.x * TW * COLS;
+  const int all = (K + 63) >> 6, c0 = blockIdx.y * per, chunks = all - c0 < per ? all - c0 : per;
+
+  // offsets from the workgroup's first weight row (of the gate rows; the up rows lie a constant behind) and from x; a row that does
+  // not exist reads the last one and is never stored
+  constexpr int WO = EPI == MID_SWIGLU ? TW : 2 * TW;
+  uint32_t woff[WO], xoff[2 * MT];
+#pragma unroll
+  for (int t = 0; t < WO; ++t) {
+    const int r = t * 8 + lrow;
+    woff[t] = (uint32_t)((long)(j0 + r < N ? r : N - 1 - j0) * ldw * 2) + lblk * 16;
+  }
+#pragma unroll
+  for (int t = 0; t < 2 * MT; ++t) {
+    const int r = t * 8 + lrow;
+    xoff[t] = (uint32_t)((long)(r < M ? r : M - 1) * ldx * 2) + lblk * 16;
+  }
+  const char *wb = reinterpret_cast<const char*>(W + (size_t)j0 * ldw), *xb = reinterpret_cast<const char*>(X);
+  const char* ub = wb + (size_t)N * ldw * 2;
+  const uint32_t mine = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mid_lds + wave * SLOTS * SLOT;
+  auto issue = [&](int s) {
+    const int c = c0 + s * MID_WAVES + wave;
+    const size_t k = (size_t)c * 128;
+    const uint32_t base = mine + (s % SLOTS) * SLOT;
+    // blocks beyond K are read as the chunk's first block, and are zeros by the time they are multiplied
+    const uint32_t back = TAIL && c * 64 + lblk * 8 >= K ? lblk * 16 : 0;
+#pragma unroll
+    for (int t = 0; t < 2 * TW; ++t) {
+      if (EPI == MID_SWIGLU) mie_load_to_lds_nt((t & 1 ? ub : wb) + k, woff[t / (2 * TW / WO)] - back, base + t * 1024);
+      else mie_load_to_lds_nt(wb + k, woff[t / (2 * TW / WO)] - back, base + t * 1024);
+    }
+#pragma unroll
+    for (int t = 0; t < 2 * MT; ++t) mie_load_to_lds(xb + k, xoff[t] - back, base + TW * 2048 + t * 1024);
+  };
+
+  f32x4 acc[TW][MT];
+#pragma unroll
+  for (int a = 0; a < TW; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int n = (chunks - wave + MID_WAVES - 1) / MID_WAVES;      // this wave's chunks: wave, wave + 4, ...
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s)
+    if (s < n) issue(s);
+  for (int it = 0; it < n; ++it) {
+    if (it + SLOTS <= n) MIE_VMCNT((SLOTS - 1) * L);              // chunk `it` has landed
+    else MIE_VMCNT(0);
+    asm volatile("" ::: "memory");
+    const char* at = mid_lds + (wave * SLOTS + it % SLOTS) * SLOT;
+    bf16x8 f[2][TW + MT];
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const int blk = ((4 * kc + kb) ^ (col & 7)) * 16;
+#pragma unroll
+      for (int t = 0; t < TW; ++t) f[kc][t] = *reinterpret_cast<const bf16x8*>(at + t * 2048 + col * 128 + blk);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        f[kc][TW + t] = *reinterpret_cast<const bf16x8*>(at + TW * 2048 + t * 2048 + col * 128 + blk);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // read: the slot is free
+    if (it + SLOTS < n) issue(it + SLOTS);
+    if (TAIL && c0 + it * MID_WAVES + wave == all - 1) {
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc)
+        if ((all - 1) * 64 + (4 * kc + kb) * 8 >= K) {
+#pragma unroll
+          for (int t = 0; t < TW + MT; ++t) f[kc][t] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+        }
+    }
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+      for (int a = 0; a < TW; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[kc][a], f[kc][TW + b], acc[a][b], 0, 0, 0);
+  }
+
+  __syncthreads();                                               // every wave is done with its slots
+  // acc[a][b][i] of lane (col, kb): weight row 4 kb + i of tile a, x row 16 b + col
+  f32x4* sums = reinterpret_cast<f32x4*>(mid_lds);
+#pragma unroll
+  for (int a = 0; a < TW; ++a)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) sums[((wave * TW + a) * MT + b) * 64 + lane] = acc[a][b];
+  __syncthreads();
+  auto joined = [&](int a, int b, int l) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < MID_WAVES; ++w) v += sums[((w * TW + a) * MT + b) * 64 + l];
+    return v;
+  };
+  if (EPI == MID_SWIGLU) {
+    for (int i = threadIdx.x; i < TW * MT * 32; i += MID_WAVES * 64) {
+      const int l = i & 31, ab = i >> 5, a = ab % TW, b = ab / TW;
+      const int m = b * 16 + (l & 15), j = j0 + a * 8 + (l >> 4) * 4;
+      if (m >= M || j >= N) continue;
+      f32x4 g = joined(a, b, l), u = joined(a, b, l + 32);       // gate rows at kb 0 and 1, up rows at kb 2 and 3
+      float o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[q] = g[q] / (1.0f + expf(-g[q])) * u[q];
+      store_bf16x4(reinterpret_cast<bf16*>(outv) + (size_t)m * ldo + j, make_float4(o[0], o[1], o[2], o[3]));
+    }
+  } else {
+    float* out = reinterpret_cast<float*>(outv) + (size_t)blockIdx.y * M * N;
+    for (int i = threadIdx.x; i < TW * MT * 64; i += MID_WAVES * 64) {
+      const int q = i % (4 * TW), m = i / (4 * TW), j = j0 + q * 4;
+      if (m >= M || j >= N) continue;
+      *reinterpret_cast<f32x4*>(out + (size_t)m * N + j) = joined(q >> 2, m >> 4, (q & 3) * 16 + (m & 15));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------- after the product
+enum { RED_STORE_BF16 = 0, RED_STORE_F32 = 1, RED_ADD = 2, RED_ADD_NORM = 3 };
+constexpr int RED_THREADS = 512;
+constexpr int RED_VEC = 4;        // float4 a thread: rows up to 8192 wide
 
 // One workgroup a row; N a multiple of 4, at most 4 * RED_THREADS * RED_VEC.  y = sum of the splits in
 // split order.  STORE: out[m, :] = y.  ADD: stream[m, :] += y.  ADD_NORM: also x_next[m, :] =
@@ -286,58 +272,122 @@ reduce_rope_kv_kernel(const float* __restrict__ part, int splits, size_t split_s
 MIE_EXPORT const char* gemm_mid_bf16_last_error() { return g_mie_error; }
 MIE_EXPORT int mie_mid_max_rows() { return 128; }
 
-// How the caller has to cut K: k-steps a split for ``splits`` wanted splits, and the number of splits that gives.
-static void cut_k(int K, int wanted, int* kper, int* splits) {
-  const int ksteps = (K + 31) / 32;
-  int per = (ksteps + wanted - 1) / wanted;
-  per = (per + MID_KC - 1) / MID_KC * MID_KC;
-  *kper = per;
-  *splits = (ksteps + per - 1) / per;
+// Weight rows a workgroup of mie_mid_gemm owns, from the weight's rows alone: 32 while that many leave room for three splits on
+// a compute unit each, else 64 (24 rows of [4096, 4096] 12.6 us with 64 in four splits, 12.9 with 32 in two).
+static int tile_rows(int N) { return (N + 31) / 32 <= 85 ? 32 : 64; }
+MIE_EXPORT int mie_mid_tile_rows(int N) { return tile_rows(N); }
+
+// How the caller has to cut K: chunks of 64 k a split for ``splits`` wanted splits, and the number of splits that gives.
+static void cut_k(int K, int wanted, int* per, int* splits) {
+  const int chunks = (K + 63) / 64;
+  *per = (chunks + wanted - 1) / wanted;
+  *splits = (chunks + *per - 1) / *per;
 }
 
 // The number of splits mie_mid_gemm will really make of ``wanted`` (the caller sizes ``part`` by it).
 MIE_EXPORT int mie_mid_splits(int K, int wanted) {
   if (K <= 0 || wanted <= 0) return 0;
-  int kper, splits;
-  cut_k(K, wanted, &kper, &splits);
+  int per, splits;
+  cut_k(K, wanted, &per, &splits);
   return splits;
 }
 
-template <int MT>
-static int launch_mid(dim3 grid, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, float* part, int M, int N,
-                      int K, int kper, const bf16* zeros) {
-  constexpr int lds_bytes = MID_STAGES * MID_KC * (MID_WAVES + MT) * FRAG_BYTES;
-  if (lds_bytes > 64 * 1024) {
-    // more LDS than a kernel gets by default: asked for once per device
-    static bool raised[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) MIE_FAIL("mid_gemm: no current device");
-    if (!raised[dev]) {
-      hipError_t e = hipFuncSetAttribute((const void*)mid_gemm_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-      if (e != hipSuccess) MIE_FAIL("mid_gemm: %d bytes of LDS refused: %s", lds_bytes, hipGetErrorString(e));
-      raised[dev] = true;
-    }
+struct MidArgs {
+  const bf16 *X, *W;
+  long ldx, ldw, ldo;
+  void* out;
+  int M, N, K, per, splits;
+};
+
+template <int TW, int MT, int SLOTS, int EPI>
+static int launch_mid(const MidArgs& a, hipStream_t s) {
+  constexpr int ring = MID_WAVES * SLOTS * (TW + MT) * 2048, sums = MID_WAVES * TW * MT * 1024;
+  constexpr int lds = ring > sums ? ring : sums, rows = TW * (EPI == MID_SWIGLU ? 8 : 16);
+  if constexpr (lds > 160 * 1024) {
+    return launch_mid<TW, MT, SLOTS - 1, EPI>(a, s);
+  } else {
+    auto kernel = a.K & 63 ? mid_gemm_kernel<TW, MT, SLOTS, EPI, true> : mid_gemm_kernel<TW, MT, SLOTS, EPI, false>;
+    if (mie_allow_lds((const void*)kernel, lds, "mid_gemm")) return -1;
+    hipLaunchKernelGGL(kernel, dim3((a.N + rows - 1) / rows, a.splits), dim3(MID_WAVES * 64), lds, s, a.X, a.ldx, a.W, a.ldw, a.out, a.ldo,
+                       a.M, a.N, a.K, a.per);
+    MIE_CHECK_LAUNCH("mid_gemm");
+    return 0;
   }
-  hipLaunchKernelGGL((mid_gemm_kernel<MT>), grid, dim3(MID_WAVES * 64), lds_bytes, s, X, ldx, W, ldw, part, M, N, K, kper, zeros);
-  MIE_CHECK_LAUNCH("mid_gemm");
+}
+
+template <int TW, int SLOTS, int EPI>
+static int launch_rows(const MidArgs& a, hipStream_t s) {
+  if (a.M <= 32) return launch_mid<TW, 2, SLOTS, EPI>(a, s);
+  if (a.M <= 48) return launch_mid<TW, 3, SLOTS, EPI>(a, s);
+  if (a.M <= 64) return launch_mid<TW, 4, SLOTS, EPI>(a, s);
+  if constexpr (TW <= 4) {
+    if (a.M <= 96) return launch_mid<TW, 6, SLOTS, EPI>(a, s);
+    return launch_mid<TW, 8, SLOTS, EPI>(a, s);
+  }
+  MIE_FAIL("mid_gemm: %d rows with %d tiles", a.M, TW);
+}
+
+static int check_operands(const char* what, const void* X, long ldx, const void* W, long ldw, int M, int K) {
+  if (M > 128) MIE_FAIL("%s: %d rows (at most 128)", what, M);
+  if (K <= 0 || (K & 7)) MIE_FAIL("%s: K = %d must be a positive multiple of 8", what, K);
+  if (ldx < K || ldw < K || (ldw & 7) || (ldx & 7)) MIE_FAIL("%s: leading dims %ld, %ld for K %d", what, ldx, ldw, K);
+  if (ldx > 1L << 23 || ldw > 1L << 23) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^23)", what, ldx, ldw);      // 32-bit offsets
+  if (((uintptr_t)X | (uintptr_t)W) & 15) MIE_FAIL("%s: operands must be 16-byte aligned", what);
   return 0;
 }
 
-// X [M, K], W [N, K] bfloat16 (16-byte aligned, leading dims multiples of 8, K a multiple of 8), M <= 128.
-// part [mie_mid_splits(K, wanted_splits), M, N] float32.  zeros: 64 zero bytes of device memory.
+// X [M, K], W [N, K] bfloat16 (16-byte aligned, leading dims multiples of 8, K a multiple of 8), M <= 128, N a multiple of 4.
+// part [mie_mid_splits(K, wanted_splits), M, N] float32.  zeros has a place in the interface and is not read.
 MIE_EXPORT int mie_mid_gemm(const void* X, long ldx, const void* W, long ldw, float* part, int M, int N, int K,
                             int wanted_splits, const void* zeros, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 128) MIE_FAIL("mid_gemm: %d rows (at most 128)", M);
-  if (K <= 0 || (K & 7)) MIE_FAIL("mid_gemm: K = %d must be a positive multiple of 8", K);
-  if (ldx < K || ldw < K || (ldw & 7) || (ldx & 7)) MIE_FAIL("mid_gemm: leading dims %ld, %ld for K %d", ldx, ldw, K);
-  if ((((uintptr_t)X | (uintptr_t)W | (uintptr_t)zeros) & 15) || !zeros || !part) MIE_FAIL("mid_gemm: operands must be 16-byte aligned");
+  if (check_operands("mid_gemm", X, ldx, W, ldw, M, K)) return -1;
+  if (!part || ((uintptr_t)part & 15) || (N & 3)) MIE_FAIL("mid_gemm: partial sums of %d columns (16-byte aligned, a multiple of 4)", N);
   if (wanted_splits < 1 || wanted_splits > 64) MIE_FAIL("mid_gemm: %d splits", wanted_splits);
-  int kper, splits;
-  cut_k(K, wanted_splits, &kper, &splits);
-  dim3 grid((N + 16 * MID_WAVES - 1) / (16 * MID_WAVES), splits);
-  if (M <= 64) return launch_mid<4>(grid, s, (const bf16*)X, ldx, (const bf16*)W, ldw, part, M, N, K, kper, (const bf16*)zeros);
-  return launch_mid<8>(grid, s, (const bf16*)X, ldx, (const bf16*)W, ldw, part, M, N, K, kper, (const bf16*)zeros);
+  MidArgs a = {(const bf16*)X, (const bf16*)W, ldx, ldw, 0, part, M, N, K, 0, 0};
+  cut_k(K, wanted_splits, &a.per, &a.splits);
+  return tile_rows(N) == 32 ? launch_rows<2, 2, MID_PART>(a, s) : launch_rows<4, 2, MID_PART>(a, s);
+}
+
+// Tiles a workgroup of the gated product has: those for which rounds of the grid times what a workgroup brings in a chunk (its
+// weight rows and x) is least, of 1, 2, 3, 4, 6 and 7 (to 64 rows; to 4 beyond, where the waves' sums would not fit the LDS).  64 rows, us: [11264,
+// 2048] 3 tiles 13.6, 4 15.1, 2 15; [22016, 4096] 6 tiles 34.9, 3 42.0, 7 37.7; [28672, 4096] 7 tiles 47.5, 4 48.7, 3 56.5.
+static int swiglu_tiles(int M, int N) {
+  const long tiles = (N + 7) / 8, cu = mie_compute_units();
+  const int choices[6] = {1, 2, 3, 4, 6, 7}, x_tiles = (M + 15) / 16;
+  int best = 1;
+  long least = -1;
+  for (int i = 0; i < (M <= 64 ? 6 : 4); ++i) {
+    const long cost = ((tiles + choices[i] * cu - 1) / (choices[i] * cu)) * (choices[i] + x_tiles);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = choices[i];
+    }
+  }
+  return best;
+}
+MIE_EXPORT int mie_mid_swiglu_tiles(int M, int N) { return swiglu_tiles(M, N); }
+
+// out [M, ldo] bfloat16 = silu(x Wg^T) * (x Wu^T), W = [gate rows (N of them); up rows], N a multiple of 4.
+MIE_EXPORT int mie_mid_swiglu(const void* X, long ldx, const void* W, long ldw, void* out, long ldo, int M, int N, int K, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  if (check_operands("mid_swiglu", X, ldx, W, ldw, M, K)) return -1;
+  if (!out || ldo < N || (ldo & 3) || (N & 3) || ((uintptr_t)out & 7)) MIE_FAIL("mid_swiglu: output leading dim %ld for %d columns", ldo, N);
+  MidArgs a = {(const bf16*)X, (const bf16*)W, ldx, ldw, ldo, out, M, N, K, (K + 63) / 64, 1};
+  const int tiles = swiglu_tiles(M, N);
+  // two chunks of a wave on their way where a compute unit has one workgroup, one where it has two (64 rows of [28672, 4096] with four
+  // tiles: 51.9 us with two chunks, 48.7 with one)
+  const bool once = (long)tiles * 8 * mie_compute_units() >= N;
+#define MID_TILES(TW) return once ? launch_rows<TW, 2, MID_SWIGLU>(a, s) : launch_rows<TW, 1, MID_SWIGLU>(a, s)
+  switch (tiles) {
+    case 1: MID_TILES(1);
+    case 2: MID_TILES(2);
+    case 3: MID_TILES(3);
+    case 4: MID_TILES(4);
+    case 6: MID_TILES(6);
+    default: MID_TILES(7);
+  }
+#undef MID_TILES
 }
 
 // mode 0: out bfloat16 [M, ldo] = sum; 1: out float32; 2: stream [M, N] float32 += sum; 3: as 2, and

@@ -25,6 +25,18 @@ __device__ __forceinline__ void mie_load_to_lds(const void* base, uint32_t offse
     : "memory");
 }
 
+// the same with the hint of loads whose lines nobody reads again: weights that one workgroup takes
+__device__ __forceinline__ void mie_load_to_lds_nt(const void* base, uint32_t offset, uint32_t at) {
+  uint32_t written;
+  asm volatile(
+    "s_mov_b32 m0, %1\n\t"
+    "s_nop 0\n\t"
+    "global_load_lds_dwordx4 %2, %3 nt"
+    : "={m0}"(written)
+    : "s"(at), "v"(offset), "s"(base)
+    : "memory");
+}
+
 // Ask for `bytes` of dynamic LDS, once a kernel and device; `what` begins the message of a refusal.
 static inline int mie_allow_lds(const void* kernel, int bytes, const char* what) {
   static std::mutex lock;

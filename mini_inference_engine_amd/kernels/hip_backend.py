@@ -303,15 +303,27 @@ class HipBackend(KernelBackend):
         M = x.shape[0]
         return (not self.true_fp32 and bias is None and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
                 and self.SKINNY_MAX_ROWS < M <= self.MID_MAX_ROWS and w.shape[0] <= self.MID_MAX_COLS
-                and w.shape[0] % 4 == 0 and w.shape[1] % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) % 8 == 0
-                and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+                and self._mid_operands_ok(x, w))
 
     @staticmethod
-    def mid_splits(N: int, K: int) -> int:
-        """Splits of K wanted for a weight [N, K]: enough for 256 workgroups of 64 weight rows, each split
+    def _mid_operands_ok(x, w) -> bool:
+        return (w.shape[0] % 4 == 0 and w.shape[1] % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) % 8 == 0
+                and w.stride(0) <= 1 << 23 and x.stride(0) <= 1 << 23 and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+
+    def mid_splits(self, N: int, K: int) -> int:
+        """Splits of K wanted for a weight [N, K]: enough for 256 workgroups of the rows the kernel's workgroups own, each split
         at least 256 wide.  A function of the weight's shape alone: a row's sums do not depend on its batch."""
-        tiles = -(-N // 64)
+        tiles = -(-N // self.lib("gemm_mid_bf16").mie_mid_tile_rows(N))
         return max(1, min(8, 256 // tiles, K // 256))
+
+    def _mid_swiglu_ok(self, x, w, intermediate) -> bool:
+        """Whether the own gate/up product with SwiGLU on its sums takes x w^T: from 17 rows on to 64, to 128 up to K = 2,048, where
+        its workgroups still bring in less than the library and silu_mul cost (us, library and silu_mul / own: 64 rows of [28672,
+        4096] 56.9 / 48.6, of [22016, 4096] 48.6 / 37.4, 128 rows 59.1 / 65.6 and 54.0 / 57.3, but of [11264, 2048] 21.7 / 17.4)."""
+        M = x.shape[0]
+        return (not self.true_fp32 and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and M > self.SKINNY_MAX_ROWS
+                and (M <= 64 or M <= self.MID_MAX_ROWS and w.shape[1] <= 2048) and intermediate % 4 == 0
+                and self._mid_operands_ok(x, w))
 
     def _mid_partials(self, x, w):
         """part [splits, M, N] float32 of x w^T."""
@@ -501,6 +513,15 @@ class HipBackend(KernelBackend):
             out = torch.empty((x.shape[0], intermediate), dtype=torch.float32, device=w_gate_up.device)
             if self._f32_product(x, w_gate_up, self.F32_SWIGLU, out):
                 return out
+        if self._mid_swiglu_ok(x, w_gate_up, intermediate):
+            self._on_device(x, w_gate_up)
+            _rows_ok(x, "linear_silu_mul: x")
+            _rows_ok(w_gate_up, "linear_silu_mul: w")
+            out = torch.empty((x.shape[0], intermediate), dtype=torch.bfloat16, device=w_gate_up.device)
+            lib = self.lib("gemm_mid_bf16")
+            library.check(lib, lib.mie_mid_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0),
+                                                  x.shape[0], intermediate, x.shape[1], self._stream()))
+            return out
         if self._tile_swiglu_gains(x, w_gate_up, intermediate):
             self._on_device(x, w_gate_up)
             _rows_ok(x, "linear_silu_mul: x")

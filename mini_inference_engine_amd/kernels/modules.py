@@ -115,6 +115,9 @@ register_kernel_module("gemm_mid_bf16", {
     "mie_mid_reduce": [P, I, I, I, I, P, L, P, P, I, P, L, F, P],
     "mie_mid_reduce_rope_kv": [P, I, I, P, L, P, P, P, P, P, P, I, I, I, I, P],
     "mie_mid_splits": [I, I],
+    "mie_mid_tile_rows": [I],
+    "mie_mid_swiglu_tiles": [I, I],
+    "mie_mid_swiglu": [P, L, P, L, P, L, I, I, I, P],
     "mie_mid_max_rows": [],
 })
 register_kernel_module("attention_bf16", {

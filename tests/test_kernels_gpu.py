@@ -473,6 +473,35 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
+# rows, K, columns and the tiles of 16 weight rows a workgroup has
+@pytest.mark.parametrize("case", [(17, 64, 4, 1), (33, 72, 12, 1), (64, 2008, 3000, 2), (48, 328, 5632, 3), (128, 2048, 5632, 3),
+                                  (50, 8, 8188, 4), (97, 200, 8192, 4), (31, 136, 11008, 6), (64, 192, 11004, 6), (64, 256, 14336, 7)])
+def test_mid_product_swiglu(engine_ops, case):
+    """Gate and up of 17 to 128 rows with SwiGLU on the float32 sums: every number of tiles, edges in rows and columns, K that is
+    no multiple of a chunk, fewer chunks than waves; against 64 bits rounded once, and a row's bits whatever is beside it."""
+    o, (M, K, inter, tiles) = engine_ops, case
+    torch.manual_seed(K + inter)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    lib = o.lib("gemm_mid_bf16")
+    assert lib.mie_mid_swiglu_tiles(M, inter) == tiles, "the case must take the tiles it is for"
+    with counted(o, "gemm_mid_bf16", "mie_mid_swiglu") as calls:
+        y = o.linear_silu_mul(x, w, inter)
+    assert len(calls) == 1
+    gu = x.double() @ w.double().T
+    expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
+    assert bool(((y.double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
+    for a, b in ((0, 17), (max(0, M - 33), M)):
+        if b - a > 16:
+            assert torch.equal(o.linear_silu_mul(x[a:b].contiguous(), w, inter), y[a:b])
+    out = torch.full((M, inter + 4), 7.0, device=DEV, dtype=torch.bfloat16)
+    assert lib.mie_mid_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 4, M, inter, K,
+                              torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out[:, :inter], y) and bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
+    assert lib.mie_mid_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 4, 129, inter, K, None) != 0
+    assert lib.mie_mid_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 4, M, inter, K - 4, None) != 0
+
+
 def test_mid_linear_refuses_what_it_cannot_run(engine_ops):
     o = engine_ops
     lib = o.lib("gemm_mid_bf16")
