@@ -4,24 +4,24 @@
 //
 //   y[m, n] = sum_k x[m, k] W[n, k]          x [M, K], W [N, K] bfloat16 as stored in a checkpoint
 //
-// A workgroup of 4 waves owns 16 rows of W (one tile of C^T = W X^T); each wave streams one contiguous
-// quarter of K in 32-wide steps; v_mfma_f32_16x16x32_bf16 with A = 16 weight rows x 32 k and B = 32 k x 16
+// A workgroup of 4 waves owns one to three tiles of 16 rows of W (tiles of C^T = W X^T); each wave streams one contiguous
+// quarter of K in chunks of 64; v_mfma_f32_16x16x32_bf16 with A = 16 weight rows x 32 k and B = 32 k x 16
 // batch rows; the waves' accumulators are summed through LDS in a fixed order.  A row's result depends on
 // nothing but that row, K and the weights: it is bit-identical in any batch.
 //
 // How the operands reach the matrix instruction.  The instruction wants lane 16 b + r to hold k-block b (8
 // values, 16 bytes) of row r.  Loaded in that order, a quarter wave (16 lanes) touches 16 cache lines for 16
-// bytes each, and the address unit, which looks lines up one at a time, is then what bounds the kernel: the x
-// loads alone (all of them hits) cost a seventh to a third of its time, and the weights stream at 4.2 to
-// 4.7 TB/s where a plain read of the same bytes runs at 5.4 to 5.8.  So a load takes whole cache lines, 8 rows of
-// 64 k (lane 8 r + b), and writes the wave's own piece of the LDS directly (no registers, nothing the compiler
-// waits for): a ring of slots of two k-steps, all but one on their way while that one is multiplied.  Within a
-// row the eight blocks are permuted (block b at 16-byte slot 8 r + (b ^ r % 8)), so that the fragment reads
-// (lane 16 b + r) are spread over all banks.  No barrier in the loop: a wave reads only what it brought in itself.
-// Up to 8 rows bring in half as much x and a slot more of the weights.  Measured (decode steps of 1 / 8 rows at
-// TinyLlama sizes, 8 rows at four layers of Llama-3-8B's, us): half lines, 16 rows of 64 bytes a load, 936 / 1064 /
-// 821; whole lines 927 / 1021 / 795; the smaller slots beside that 898 / 999 / 786; the weights by nontemporal loads
-// beside that 862 / 995 / 755 (with half lines the hint had made the kernel slower: it dropped the line's other half).
+// bytes each, and the address unit, which looks lines up one at a time, is then what bounds the kernel.  So a load takes whole
+// cache lines, 8 rows of 64 k (lane 8 r + b), and writes the wave's own piece of the LDS directly (no registers, nothing the
+// compiler waits for): slots of one chunk.  A slot's fragments are read, the chunk SLOTS further on is asked for into the same
+// slot at once, and then they are multiplied.  Within a row the eight blocks are permuted (block b at 16-byte place
+// 8 r + (b ^ r % 8)), so that the fragment reads (lane 16 b + r) are spread over all banks.  No barrier in the loop: a wave
+// reads only what it brought in itself.  Up to 8 rows bring in half as much x.
+// Loads are all a compute unit can take in, 58 bytes a nanosecond, hits or not, so none is made for nothing: nothing behind a
+// wave's quarter is asked for (three slots of zeros a wave were, a quarter of all loads at K = 2,048), and tiles share a workgroup's
+// x.  Measured alone (MI355X, us, 1 / 8 / 16 rows, before and now): [2048, 2048] 4.5 / 4.7 / 5.1 and 4.1 / 4.5 / 4.9, [2048, 5632] 7.8 /
+// 8.2 / 9.7 and 7.0 / 7.9 / 9.6, [11264, 2048] 10.2 / 10.2 / 11.1 and 9.6 / 9.7 / 9.9, [32000, 2048] 24.9 / 25.1 / 27.2 and 21.7 / 21.3 /
+// 22.1, [6144, 4096] 11.4 / 12.6 / 14.4 and 10.8 / 11.2 / 12.3, [28672, 4096] 38.9 / 40.3 / 42.0 and 37.4 / 37.9 / 39.3.
 //
 // Epilogues: STORE (bfloat16 or float32 y), ADD (r[m, n] += y, the residual add of the 32-bit stream),
 //   SWIGLU (W holds gate rows then up rows; a tile is 8 gate rows and the matching 8 up rows, and the
@@ -31,43 +31,13 @@
 // converted the 32-bit stream inside every workgroup was measured and dropped: redoing the conversion of
 // all of x per workgroup cost more than a separate norm kernel.)
 #include "launch.hpp"
+#include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// what a k-step beyond a wave's range or beyond K loads instead of weights, so that every load is unconditional
-__device__ __align__(128) const uint32_t mie_zero_words[32] = {0};
-
-constexpr int SG_NONTEMPORAL = 2;  // the hint of loads whose lines nobody reads again: the weights
-
 constexpr int SG_WAVES = 4;       // waves a workgroup
 constexpr int SG_THREADS = SG_WAVES * 64;
-constexpr int RING_U = 2;         // k-steps a slot of a wave's ring
-
-// The fragments of a slot (U k-steps: weight fragment, x fragment, 1 KB each) out of the LDS, read and waited for
-// in one piece of assembly: the compiler knows nothing of the loads that write the LDS, so a read it could see
-// would make it wait for every load on its way, and it must never see a register whose value is still to arrive.
-typedef uint32_t sg_u32x4 __attribute__((ext_vector_type(4)));
-// w0 / w1, x0 / x1: this lane's pieces of the slot's first and second k-step.
-__device__ __forceinline__ void ring_read(uint32_t w0, uint32_t x0, uint32_t w1, uint32_t x1, sg_u32x4 (&f)[4]) {
-  asm volatile(
-    "ds_read_b128 %0, %4\n\t"
-    "ds_read_b128 %1, %5\n\t"
-    "ds_read_b128 %2, %6\n\t"
-    "ds_read_b128 %3, %7\n\t"
-    "s_waitcnt lgkmcnt(0)"
-    : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
-    : "v"(w0), "v"(x0), "v"(w1), "v"(x1)
-    : "memory");
-}
-
-// The wait of round `it` < SLOTS - 1 (the counter's limit must be a constant of the instruction).
-template <int SLOTS, int XL, int IT> struct RingStart {
-  static __device__ __forceinline__ void wait(int it) {
-    if (it == IT) MIE_VMCNT((SLOTS - 2 - IT) * XL + (IT + 1) * (2 + XL));
-    else if constexpr (IT + 1 < SLOTS - 1) RingStart<SLOTS, XL, IT + 1>::wait(it);
-  }
-};
 
 enum { EPI_STORE_BF16 = 0, EPI_STORE_F32 = 1, EPI_ADD = 2, EPI_SWIGLU = 3, EPI_ROPE = 4, EPI_GEGLU = 5, EPI_CLAMPGLU = 6 };
 // the gated epilogues differ in the function only: silu(g) u (SWIGLU), the tanh form of gelu(g) u (GEGLU), or, with g at most
@@ -107,163 +77,200 @@ struct NormArgs {
 
 // Which weight row column c (0 .. 15) of tile `tile` multiplies, and whether it exists.
 //   plain:  n = 16 tile + c
-//   SWIGLU: columns 0 .. 7 are gate rows j = 8 tile + c, columns 8 .. 15 the up rows of the same j
+//   gated:  columns 0 .. 7 are gate rows j = 8 tile + c, columns 8 .. 15 the up rows of the same j
 //   ROPE:   columns 0 .. 7 are the first members jd = 8 (tile % (D / 16)) + c of eight rotary pairs of head
 //           tile / (D / 16), columns 8 .. 15 their partners jd + D / 2
-// so that both members of a pair are lanes c and c ^ 8 of one wave after the reduction.
+// so that both members of a pair are lanes c and c ^ 8 of one wave after the reduction.  tile_row: the row of column 0 (h = 0) or
+// 8 (h = 1), `rows` the rows that exist from there on (may be none or negative).
 template <int EPI>
-__device__ __forceinline__ long tile_column(int tile, int c, int N, int up_offset, int D, bool& ok) {
+__device__ __forceinline__ long tile_row(int tile, int h, int N, int up_offset, int D, int& rows) {
   if (EPI_GATED(EPI)) {
-    const int j = tile * 8 + (c & 7);
-    ok = j < N;
-    return (long)(c >> 3) * up_offset + j;
+    rows = N - tile * 8;
+    return (long)h * up_offset + tile * 8;
   }
   if (EPI == EPI_ROPE) {
-    const int per_head = D >> 4, head = tile / per_head, jd = (tile - head * per_head) * 8 + (c & 7);
-    ok = true;
-    return (long)head * D + jd + (c >> 3) * (D >> 1);
+    const int per_head = D >> 4, head = tile / per_head, jd = (tile - head * per_head) * 8;
+    rows = head * D < N ? 8 : 0;
+    return (long)head * D + jd + h * (D >> 1);
   }
-  const int n = tile * 16 + c;
-  ok = n < N;
-  return n;
+  rows = N - (tile * 16 + h * 8);
+  return (long)tile * 16 + h * 8;
 }
 
-// XL: loads of x a slot: one for up to 8 rows (columns 8 to 15 of the tile then take rows 0 to 7 again), else two.
-template <int EPI, bool NF, int SLOTS, int XL>
+// XT: groups of 8 x rows: one for up to 8 (columns 8 to 15 of the tile then take rows 0 to 7 again), else two.
+// TW: tiles a workgroup, `tiles` of them in all.
+template <int EPI, bool NF, int TW, int XT, int SLOTS>
 __global__ void __launch_bounds__(SG_THREADS)
 skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, void* __restrict__ outv,
-                   long ldo, int M, int N, int K, int up_offset, RopeArgs rope, NormArgs nf) {
-  constexpr int L = 2 + XL;                                // loads a slot
-  constexpr int SLOT_BYTES = L * 1024;                     // 16 weight rows of 64 k (128 bytes), then the x rows
-  constexpr int WAVE_BYTES = SLOTS * SLOT_BYTES;
+                   long ldo, int M, int N, int K, int up_offset, int tiles, RopeArgs rope, NormArgs nf) {
+  constexpr int L = 2 * TW + XT, SLOT = L * 1024;          // of a slot: TW times 16 weight rows of 64 k (128 bytes), then the x rows
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
-  extern __shared__ __align__(16) char ring_lds[];         // WAVE_BYTES a wave
-  __shared__ float s_acc[SG_WAVES][256];
+  extern __shared__ __align__(1024) char ring_lds[];       // SLOTS slots a wave
+  __shared__ float s_acc[TW][SG_WAVES][256];
   __shared__ float s_rstd[16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kb = lane >> 4;
-  const int tile = blockIdx.x;
-  const int ksteps = (K + 31) >> 5;
-  const int per_wave = ((ksteps + SG_WAVES - 1) / SG_WAVES + 1) & ~1;       // whole cache lines of a row
-  const int ks0 = wave * per_wave;
-  const int ks1 = ks0 + per_wave < ksteps ? ks0 + per_wave : ksteps;
+  const int tile0 = blockIdx.x * TW;
+  const int all = (K + 63) >> 6, own = (all + SG_WAVES - 1) / SG_WAVES;
+  const int c0 = wave * own, chunks = all - c0 < own ? all - c0 : own;         // (none: negative or 0)
 
-  // What this lane brings in: rows lrow and lrow + 8 (of the weight tile; of x), block lblk of every 64 k.  And the one
-  // result this thread owns after the waves are summed: x row m, column c of the tile.  The gather of x's
-  // rows, if there is one, and the positions are the first things asked for: addresses depend on them.
+  // What this lane brings in: row lrow of each group of 8, block lblk of every 64 k.  And the results this thread owns after the
+  // waves are summed: x row m, column c of every tile.
   const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;
   const int m = threadIdx.x >> 4, c = threadIdx.x & 15;
   const bool gather = NF && EPI != EPI_ADD && nf.rows;
-  const int lsrc0 = lrow < M ? (gather ? nf.rows[lrow] : lrow) : 0;
-  const int lsrc1 = lrow + 8 < M ? (gather ? nf.rows[lrow + 8] : lrow + 8) : lsrc0;
+  uint32_t xoff[XT];
+#pragma unroll
+  for (int t = 0; t < XT; ++t) {
+    const int r = t * 8 + lrow < M ? t * 8 + lrow : 0;     // rows beyond M read another row along with the lanes that own it
+    xoff[t] = (uint32_t)((long)(gather ? nf.rows[r] : r) * ldx * 2) + lblk * 16;
+  }
   const int msrc = m < M ? (gather ? nf.rows[m] : m) : 0;
-
-  bool ok;
-  const long n = tile_column<EPI>(tile, c, N, up_offset, rope.D, ok);
-  const bool live = m < M && ok;
-  const int mc = live ? m : 0;
-  const long nc = live ? n : 0;
-  float e_old = 0.f, e_cos = 0.f, e_sin = 0.f;
-  uint32_t e_g = 0u;                       // raw bits of the next norm's weight (converted where it is used)
-  int e_slot = 0, e_pos = 0;
-  if (EPI == EPI_ROPE) {                   // the positions: further addresses depend on them too
-    e_pos = rope.positions[mc];
-    e_slot = rope.slots[mc];
-  }
-
-  // The ring.  Slots beyond the wave's range load zeros only, so that it is always filled and drained the
-  // same way.
-  bool lok0, lok1;
-  const long lwr0 = tile_column<EPI>(tile, lrow, N, up_offset, rope.D, lok0);
-  const long lwr1 = tile_column<EPI>(tile, lrow + 8, N, up_offset, rope.D, lok1);
-  // a row that does not exist is never stored; rows beyond M read another row along with the lanes that own it
-  const bf16* wsrc0 = W + (size_t)(lok0 ? lwr0 : 0) * ldw + lblk * 8;
-  const bf16* wsrc1 = W + (size_t)(lok1 ? lwr1 : 0) * ldw + lblk * 8;
-  const bf16* xsrc0 = X + (size_t)lsrc0 * ldx + lblk * 8;
-  const bf16* xsrc1 = X + (size_t)lsrc1 * ldx + lblk * 8;
-  const bf16* zero_lane = reinterpret_cast<const bf16*>(mie_zero_words) + lblk * 8;  // per lane, so that choosing it is a select
-  char* mine = ring_lds + wave * WAVE_BYTES;
-  // what: 1 the weights of slot s, 2 its x, 3 both
-  auto issue = [&](int s, int what) {
-    char* base = mine + (s % SLOTS) * SLOT_BYTES;
-    const int ks = ks0 + s * RING_U;
-    const bool kok = ks + (lblk >> 2) < ks1 && ks * 32 + lblk * 8 < K;
-    const size_t k = (size_t)ks * 32;
-    const bf16* src[4] = {kok ? wsrc0 + k : zero_lane, kok ? wsrc1 + k : zero_lane, kok ? xsrc0 + k : zero_lane, kok ? xsrc1 + k : zero_lane};
+  const char* wbase[TW][2];
+  uint32_t woff[TW][2];
+  long n_of[TW];
+  bool live[TW];
 #pragma unroll
-    for (int j = 0; j < L; ++j) {
-      const auto* from = (const __attribute__((address_space(1))) void*)src[j];
-      auto* to = (__attribute__((address_space(3))) void*)(base + j * 1024);
-      if (j < 2 && (what & 1)) __builtin_amdgcn_global_load_lds(from, to, 16, 0, SG_NONTEMPORAL);
-      if (j >= 2 && (what & 2)) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+  for (int a = 0; a < TW; ++a) {
+    const int tile = tile0 + a < tiles ? tile0 + a : tiles - 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int rows;
+      const long row = tile_row<EPI>(tile, h, N, up_offset, rope.D, rows);
+      // a row that does not exist is never stored: the tile's last one that does (or the weight's first) is read instead
+      wbase[a][h] = reinterpret_cast<const char*>(W + (size_t)(rows > 0 ? row : 0) * ldw);
+      woff[a][h] = (uint32_t)((long)(rows > 0 ? (lrow < rows ? lrow : rows - 1) : 0) * ldw * 2) + lblk * 16;
+      if (h == c >> 3) {
+        n_of[a] = row + (c & 7);
+        live[a] = tile0 + a < tiles && m < M && (c & 7) < rows;
+      }
     }
-  };
-  const int rounds = ks1 > ks0 ? (ks1 - ks0 + RING_U - 1) / RING_U : 0;
-  // this lane's pieces of a slot: row col, blocks kb and 4 + kb
-  const uint32_t ring0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine;
-  const uint32_t blk0 = (kb ^ (col & 7)) * 16, blk1 = ((4 + kb) ^ (col & 7)) * 16;
-  const uint32_t wrow0 = ring0 + col * 128, xrow0 = ring0 + 2048 + (XL == 1 ? col & 7 : col) * 128;
-  // The ring starts with the weights of its first slots; their x follows below, after what the epilogue reads
-  // has been asked for: all that waits for the row numbers of a gather, the weights do not.
-#pragma unroll
-  for (int s = 0; s < SLOTS - 1; ++s) issue(s, 1);
-  // What the epilogue reads beside the product is asked for next, so that it has arrived long before it is
-  // used and is older than the ring's x loads (the counter of loads on their way runs in issue order).
-  // Every load is unconditional, from an address clamped into the operand.
-  if (EPI == EPI_ADD) {
-    e_old = ((const float*)outv)[(size_t)mc * ldo + nc];
-    if (NF) e_g = nf.g_f32 ? ((const uint32_t*)nf.g)[nc] : (uint32_t)((const uint16_t*)nf.g)[nc];
   }
-  // Fused norm, consuming side: the partial sums of squares likewise.  16 lanes a row, lane c takes the
+
+  // What the epilogue reads beside the product is asked for before the ring, so that it has arrived long before it is used and a
+  // wait for it is no wait for the ring.  Every load is unconditional, from an address clamped into the operand.
+  float e_old[TW] = {}, e_cos[TW] = {}, e_sin[TW] = {};
+  uint32_t e_g[TW] = {};                   // raw bits of the next norm's weight (converted where it is used)
+  int e_slot = 0;
+  if (EPI == EPI_ROPE) {                   // positions and slots of the wave's four rows by scalar loads, and the angles
+    int pos[4], slot[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = wave * 4 + i < M ? wave * 4 + i : 0;
+      pos[i] = rope.positions[r];
+      slot[i] = rope.slots[r];
+    }
+    const int i = lane >> 4, e_pos = i == 0 ? pos[0] : i == 1 ? pos[1] : i == 2 ? pos[2] : pos[3];
+    e_slot = i == 0 ? slot[0] : i == 1 ? slot[1] : i == 2 ? slot[2] : slot[3];
+    const int half = rope.D >> 1, per_head = rope.D >> 4;
+#pragma unroll
+    for (int a = 0; a < TW; ++a) {
+      const int jd = ((tile0 + a) % per_head) * 8 + (c & 7);
+      e_cos[a] = rope.cos_t[(size_t)e_pos * half + jd];
+      e_sin[a] = rope.sin_t[(size_t)e_pos * half + jd];
+    }
+  }
+  if (EPI == EPI_ADD) {
+#pragma unroll
+    for (int a = 0; a < TW; ++a) {
+      const long nc = live[a] ? n_of[a] : 0;
+      e_old[a] = ((const float*)outv)[(size_t)(live[a] ? m : 0) * ldo + nc];
+      if (NF) e_g[a] = nf.g_f32 ? ((const uint32_t*)nf.g)[nc] : (uint32_t)((const uint16_t*)nf.g)[nc];
+    }
+  }
+  // Fused norm, consuming side: the partial sums of squares.  16 lanes a row, lane c takes the
   // tiles 4 (c + 16 i) .. + 3: the first SSP fours now, the rest (widths above 4096) after the loop.
   constexpr int SSP = 4;
-  float4 ssp[SSP];
+  f32x4 ssp[SSP];
   const int ss_ld = (nf.ss_tiles + 3) & ~3;
   if (NF && EPI != EPI_ADD) {
 #pragma unroll
     for (int i = 0; i < SSP; ++i) {
       const int t = 4 * (c + 16 * i);
-      ssp[i] = *reinterpret_cast<const float4*>(nf.ss_in + (size_t)msrc * ss_ld + (t < ss_ld ? t : 0));
+      ssp[i] = *reinterpret_cast<const f32x4*>(nf.ss_in + (size_t)msrc * ss_ld + (t < ss_ld ? t : 0));
     }
   }
 
-  // the x fragments of the ring's first slots
+  const char* xb = reinterpret_cast<const char*>(X);
+  const uint32_t mine = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)ring_lds + wave * SLOTS * SLOT;
+  auto issue = [&](int s) {
+    const size_t k = (size_t)(c0 + s) * 128;
+    const uint32_t base = mine + (s % SLOTS) * SLOT;
+    // blocks beyond K are read as the chunk's first block, and are zeros by the time they are multiplied
+    const uint32_t back = (c0 + s) * 64 + lblk * 8 >= K ? lblk * 16 : 0;
 #pragma unroll
-  for (int s = 0; s < SLOTS - 1; ++s) issue(s, 2);
-  if (EPI == EPI_ROPE) {
-    // the angles, once the positions are here (asked for before the ring: waiting for them does not wait for it)
-    const int half = rope.D >> 1;
-    const int per_head = rope.D >> 4;
-    const int jd = (tile % per_head) * 8 + (c & 7);
-    e_cos = rope.cos_t[(size_t)e_pos * half + jd];       // position 0 for the rows that do not count
-    e_sin = rope.sin_t[(size_t)e_pos * half + jd];
-  }
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int it = 0; it < rounds; ++it) {
-    issue(it + SLOTS - 1, 3);                      // into the slot that was read a round ago
-    // Slot `it` has landed: all but the loads issued after its last one.  From round SLOTS - 1 on those are the
-    // SLOTS - 1 slots after it; before, the x fragments of the first slots that follow its own and the slots
-    // issued in the loop so far.  (Anything else asked for in between only makes this wait for more.)
-    if (it >= SLOTS - 1) MIE_VMCNT((SLOTS - 1) * L);
-    else RingStart<SLOTS, XL, 0>::wait(it);
-    sg_u32x4 f[2 * RING_U];
-    const uint32_t w0 = wrow0 + (it % SLOTS) * SLOT_BYTES, x0 = xrow0 + (it % SLOTS) * SLOT_BYTES;
-    ring_read(w0 + blk0, x0 + blk0, w0 + blk1, x0 + blk1, f);
+    for (int a = 0; a < TW; ++a)
 #pragma unroll
-    for (int u = 0; u < RING_U; ++u)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f[2 * u]), __builtin_bit_cast(bf16x8, f[2 * u + 1]),
-                                                    acc, 0, 0, 0);
+      for (int h = 0; h < 2; ++h) mie_load_to_lds_nt(wbase[a][h] + k, woff[a][h] - back, base + (2 * a + h) * 1024);
+#pragma unroll
+    for (int t = 0; t < XT; ++t) mie_load_to_lds(xb + k, xoff[t] - back, base + (2 * TW + t) * 1024);
+  };
+  f32x4 acc[TW];
+#pragma unroll
+  for (int a = 0; a < TW; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s)
+    if (s < chunks) issue(s);
+  bf16x8 wf[2][TW], xf[2];
+  auto take = [&](int it) {                                // this lane's fragments of chunk `it`
+    const char* at = ring_lds + (wave * SLOTS + it % SLOTS) * SLOT;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int blk = ((4 * u + kb) ^ (col & 7)) * 16;
+#pragma unroll
+      for (int a = 0; a < TW; ++a) wf[u][a] = *reinterpret_cast<const bf16x8*>(at + a * 2048 + col * 128 + blk);
+      xf[u] = *reinterpret_cast<const bf16x8*>(at + TW * 2048 + (XT == 1 ? col & 7 : col) * 128 + blk);
+    }
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int a = 0; a < TW; ++a) acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][a], xf[u], acc[a], 0, 0, 0);
+  };
+  int it = 0;
+  for (; it + SLOTS < chunks; ++it) {
+    MIE_VMCNT((SLOTS - 1) * L);                            // chunk `it` has landed: at most those after it are on their way
+    asm volatile("" ::: "memory");
+    take(it);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // read: the slot is free
+    issue(it + SLOTS);
+    multiply();
   }
-  MIE_VMCNT(0);                                     // nothing of this wave may still be writing the LDS when it ends
+  // the last chunks, nothing behind them
+  auto last = [&](auto left) {
+    constexpr int LEFT = decltype(left)::value;            // chunks behind this one
+    if (LEFT >= SLOTS || LEFT >= chunks) return;
+    MIE_VMCNT(LEFT < SLOTS ? LEFT * L : 0);
+    asm volatile("" ::: "memory");
+    take(it++);
+    if (LEFT == 0 && c0 + chunks == all && (K & 63)) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if ((all - 1) * 64 + (4 * u + kb) * 8 >= K) {
+          xf[u] = __builtin_bit_cast(bf16x8, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int a = 0; a < TW; ++a) wf[u][a] = xf[u];
+        }
+    }
+    multiply();
+  };
+  static_assert(SLOTS <= 5, "the calls below");
+  last(std::integral_constant<int, 4>());
+  last(std::integral_constant<int, 3>());
+  last(std::integral_constant<int, 2>());
+  last(std::integral_constant<int, 1>());
+  last(std::integral_constant<int, 0>());
 
   if (NF && EPI != EPI_ADD) {
     // 1 / sqrt(mean of squares + eps) of every row, summed in a fixed order
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < SSP; ++i) {
+      asm volatile("" : "+v"(ssp[i]));                     // (not added up, and so not waited for, before the loop)
       const int t = 4 * (c + 16 * i);
-      sum += (t < nf.ss_tiles ? ssp[i].x : 0.f) + (t + 1 < nf.ss_tiles ? ssp[i].y : 0.f) +
-             (t + 2 < nf.ss_tiles ? ssp[i].z : 0.f) + (t + 3 < nf.ss_tiles ? ssp[i].w : 0.f);
+      sum += (t < nf.ss_tiles ? ssp[i][0] : 0.f) + (t + 1 < nf.ss_tiles ? ssp[i][1] : 0.f) +
+             (t + 2 < nf.ss_tiles ? ssp[i][2] : 0.f) + (t + 3 < nf.ss_tiles ? ssp[i][3] : 0.f);
     }
     if (nf.ss_tiles > 64 * SSP)
       for (int t = 64 * SSP + c; t < nf.ss_tiles; t += 16) sum += nf.ss_in[(size_t)msrc * ss_ld + t];
@@ -276,62 +283,66 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
 
   // sum the waves: acc[i] of lane (col, kb) is weight row 4 kb + i (column of the tile), x row col
 #pragma unroll
-  for (int i = 0; i < 4; ++i) s_acc[wave][lane * 4 + i] = acc[i];
+  for (int a = 0; a < TW; ++a) *reinterpret_cast<f32x4*>(&s_acc[a][wave][lane * 4]) = acc[a];
   __syncthreads();
-  float v = 0.f;
-  {
-    const int src = (((c >> 2) << 4) + m) * 4 + (c & 3);
+  const float rstd = NF && EPI != EPI_ADD ? s_rstd[m] : 1.f;
 #pragma unroll
-    for (int w = 0; w < SG_WAVES; ++w) v += s_acc[w][src];
-  }
+  for (int a = 0; a < TW; ++a) {
+    const long n = n_of[a];
+    float v = 0.f;
+    {
+      const int src = (((c >> 2) << 4) + m) * 4 + (c & 3);
+#pragma unroll
+      for (int w = 0; w < SG_WAVES; ++w) v += s_acc[a][w][src];
+    }
 
-  if (EPI == EPI_ADD) {
-    const float r = e_old + v;
-    if (live) ((float*)outv)[(size_t)m * ldo + n] = r;
-    if (NF) {
-      const float g = nf.g_f32 ? __uint_as_float(e_g) : __uint_as_float(e_g << 16);
-      if (live) nf.x_next[(size_t)m * nf.ldx_next + n] = __float2bfloat16(r * g);
-      float q = live ? r * r : 0.f;          // the 16 lanes of a row: sum of squares over this tile's columns
-      q += __shfl_xor(q, 1, 64);
-      q += __shfl_xor(q, 2, 64);
-      q += __shfl_xor(q, 4, 64);
-      q += __shfl_xor(q, 8, 64);
-      if (c == 0 && m < M) nf.ss_out[(size_t)m * ((gridDim.x + 3) & ~3) + tile] = q;
+    if (EPI == EPI_ADD) {
+      const float r = e_old[a] + v;
+      if (live[a]) ((float*)outv)[(size_t)m * ldo + n] = r;
+      if (NF) {
+        const float g = nf.g_f32 ? __uint_as_float(e_g[a]) : __uint_as_float(e_g[a] << 16);
+        if (live[a]) nf.x_next[(size_t)m * nf.ldx_next + n] = __float2bfloat16(r * g);
+        float q = live[a] ? r * r : 0.f;     // the 16 lanes of a row: sum of squares over this tile's columns
+        q += __shfl_xor(q, 1, 64);
+        q += __shfl_xor(q, 2, 64);
+        q += __shfl_xor(q, 4, 64);
+        q += __shfl_xor(q, 8, 64);
+        if (c == 0 && m < M && tile0 + a < tiles) nf.ss_out[(size_t)m * ((tiles + 3) & ~3) + tile0 + a] = q;
+      }
+      continue;
     }
-    return;
-  }
-  const float rstd = NF ? s_rstd[m] : 1.f;
-  const float mine_v = v * rstd;
-  float other = 0.f;
-  if (EPI == EPI_ROPE || EPI_GATED(EPI)) other = __shfl_xor(mine_v, 8, 64);   // the pair's other member
-  if (!live) return;
-  if (EPI == EPI_ROPE) {
-    const int D = rope.D;
-    const int head = (int)(n / D), jd = (int)(n - (long)head * D);   // column inside the head
-    const int slot = e_slot;
-    if (head < rope.Hq + rope.Hkv) {
-      // first member (c < 8): x1 cos - x2 sin; second: x2 cos + x1 sin, x1 being the first member's value
-      const float o = c < 8 ? mine_v * e_cos - other * e_sin : mine_v * e_cos + other * e_sin;
-      if (head < rope.Hq)
-        ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(o);
-      else
-        rope.k_cache[(((size_t)(slot / rope.page) * rope.Hkv + (head - rope.Hq)) * rope.page + slot % rope.page) * D + jd] =
-            __float2bfloat16(o);
-    } else {
-      rope.v_cache[(((size_t)(slot / rope.page) * rope.Hkv + (head - rope.Hq - rope.Hkv)) * D + jd) * rope.page +
-                   slot % rope.page] = __float2bfloat16(mine_v);
-    }
-  } else if (EPI == EPI_STORE_BF16) {
-    ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(mine_v);
-  } else if (EPI == EPI_STORE_F32) {
-    ((float*)outv)[(size_t)m * ldo + n] = mine_v;
-  } else if (c < 8) {                        // gated: mine = gate, other = up
-    if (EPI == EPI_CLAMPGLU) {
-      const float g = fminf(mine_v, nf.glu_limit), u = fminf(fmaxf(other, -nf.glu_limit), nf.glu_limit);
-      ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(g * mie_sigmoid(nf.glu_alpha * g) * (u + nf.glu_shift));
-    } else {
-      const float a = EPI == EPI_GEGLU ? mie_gelu_tanh(mine_v) : mine_v / (1.0f + expf(-mine_v));
-      ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(a * other);
+    const float mine_v = v * rstd;
+    float other = 0.f;
+    if (EPI == EPI_ROPE || EPI_GATED(EPI)) other = __shfl_xor(mine_v, 8, 64);   // the pair's other member
+    if (!live[a]) continue;
+    if (EPI == EPI_ROPE) {
+      const int D = rope.D;
+      const int head = (int)(n / D), jd = (int)(n - (long)head * D);   // column inside the head
+      const int slot = e_slot;
+      if (head < rope.Hq + rope.Hkv) {
+        // first member (c < 8): x1 cos - x2 sin; second: x2 cos + x1 sin, x1 being the first member's value
+        const float o = c < 8 ? mine_v * e_cos[a] - other * e_sin[a] : mine_v * e_cos[a] + other * e_sin[a];
+        if (head < rope.Hq)
+          ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(o);
+        else
+          rope.k_cache[(((size_t)(slot / rope.page) * rope.Hkv + (head - rope.Hq)) * rope.page + slot % rope.page) * D + jd] =
+              __float2bfloat16(o);
+      } else {
+        rope.v_cache[(((size_t)(slot / rope.page) * rope.Hkv + (head - rope.Hq - rope.Hkv)) * D + jd) * rope.page +
+                     slot % rope.page] = __float2bfloat16(mine_v);
+      }
+    } else if (EPI == EPI_STORE_BF16) {
+      ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(mine_v);
+    } else if (EPI == EPI_STORE_F32) {
+      ((float*)outv)[(size_t)m * ldo + n] = mine_v;
+    } else if (c < 8) {                      // gated: mine = gate, other = up
+      if (EPI == EPI_CLAMPGLU) {
+        const float g = fminf(mine_v, nf.glu_limit), u = fminf(fmaxf(other, -nf.glu_limit), nf.glu_limit);
+        ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(g * mie_sigmoid(nf.glu_alpha * g) * (u + nf.glu_shift));
+      } else {
+        const float f = EPI == EPI_GEGLU ? mie_gelu_tanh(mine_v) : mine_v / (1.0f + expf(-mine_v));
+        ((bf16*)outv)[(size_t)m * ldo + n] = __float2bfloat16(f * other);
+      }
     }
   }
 }
@@ -339,17 +350,16 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
 MIE_EXPORT const char* gemm_bf16_last_error() { return g_mie_error; }
 MIE_EXPORT int mie_skinny_max_rows() { return 16; }
 
-// A kernel that wants more LDS than a launch gets by default is told so once per device.
-
-template <bool NF, int SLOTS, int XL>
-static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
-                      long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& nf) {
-  constexpr int lds = SG_WAVES * SLOTS * (2 + XL) * 1024;
+template <bool NF, int TW, int XT, int SLOTS>
+static int launch_epi(int epi, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
+                      long ldo, int M, int N, int K, int up_offset, int tiles, const RopeArgs& rope, const NormArgs& nf) {
+  constexpr int lds = SG_WAVES * SLOTS * (2 * TW + XT) * 1024;
+  const dim3 grid((tiles + TW - 1) / TW);
 #define SG_LAUNCH(E)                                                                                                    \
   {                                                                                                                     \
-    auto kernel = skinny_gemm_kernel<E, NF, SLOTS, XL>;                                                                 \
+    auto kernel = skinny_gemm_kernel<E, NF, TW, XT, SLOTS>;                                                             \
     if (mie_allow_lds((const void*)kernel, lds, "skinny_gemm")) return -1;                                              \
-    hipLaunchKernelGGL(kernel, grid, dim3(SG_THREADS), lds, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, nf); \
+    hipLaunchKernelGGL(kernel, grid, dim3(SG_THREADS), lds, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, tiles, rope, nf); \
   }
   switch (epi) {
     case EPI_STORE_BF16: SG_LAUNCH(EPI_STORE_BF16); break;
@@ -366,22 +376,40 @@ static int launch_epi(int epi, dim3 grid, hipStream_t s, const bf16* X, long ldx
   return 0;
 }
 
-// Slots a wave's ring has.  Four (64 KB a workgroup, two workgroups a compute unit; five of 60 KB for up to 8 rows) stream
-// best; three (48 KB, three workgroups a compute unit; four of 48 KB for up to 8 rows) when that lets all tiles run at once instead of in two rounds.  Chosen from
-// the weight's shape alone, never from the batch (the sums do not depend on it anyway).
-static int slots_for(int tiles) {
+// Tiles a workgroup has.  One while every tile has a compute unit of its own; two where one would leave some compute units with
+// two workgroups and others with one ([6144, 4096] at 8 rows: 12.2 us with one tile, 11.2 with two).  Beyond, up to 8 rows one again,
+// three workgroups a compute unit ([28672, 4096] at 1 / 8 rows 37.4 / 37.9 us, two tiles 38.8 / 39.7), until the rounds are many
+// ([128256, 4096]: 160.8 / 157.3 with one, 157.6 / 155.5 with two); from 9 rows on x weighs twice as much: three tiles while
+// that gives every compute unit one workgroup ([11264, 2048] at 16 rows 10.7 with one, 9.9 with three), else two ([32000, 2048] 24.0,
+// 22.1).  The sums do not depend on it.
+static int tiles_for(int M, int tiles) {
   const int cu = mie_compute_units();
-  return tiles > 2 * cu && tiles <= 3 * cu ? 3 : 4;
+  if (tiles <= cu) return 1;
+  if (tiles <= 2 * cu) return 2;
+  if (M <= 8) return tiles <= 16 * cu ? 1 : 2;
+  return tiles <= 3 * cu ? 3 : 2;
 }
 
 static int launch_rows(int tiles, int epi, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
                        long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& n, bool fused) {
-  dim3 grid(tiles);
-  const bool three = slots_for(tiles) == 3;
-#define SG_ROWS(NF, SLOTS, XL) launch_epi<NF, SLOTS, XL>(epi, grid, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, rope, n)
-  if (M <= 8)             // a slot is a quarter smaller: as many workgroups a compute unit with one slot more
-    return three ? (fused ? SG_ROWS(true, 4, 1) : SG_ROWS(false, 4, 1)) : (fused ? SG_ROWS(true, 5, 1) : SG_ROWS(false, 5, 1));
-  return three ? (fused ? SG_ROWS(true, 3, 2) : SG_ROWS(false, 3, 2)) : (fused ? SG_ROWS(true, 4, 2) : SG_ROWS(false, 4, 2));
+  const int tw = tiles_for(M, tiles);
+#define SG_ROWS(NF, TW, XT, SLOTS) return launch_epi<NF, TW, XT, SLOTS>(epi, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, tiles, rope, n)
+#define SG_TILES(TW, XT, SLOTS)                  \
+  {                                              \
+    if (fused) SG_ROWS(true, TW, XT, SLOTS);     \
+    SG_ROWS(false, TW, XT, SLOTS);               \
+  }
+  // Slots: what lets a compute unit have its workgroups at once (48 to 72 KB each); one more where it has a single one ([2048, 5632] at 1
+  // row: four slots 8.1 us, five 7.1).
+  if (M <= 8) {
+    if (tw == 2) SG_TILES(2, 1, 3);
+    if (tiles <= mie_compute_units()) SG_TILES(1, 1, 5);
+    SG_TILES(1, 1, 4);
+  }
+  if (tw == 1) SG_TILES(1, 2, 5);
+  if (tw == 2) SG_TILES(2, 2, 3);
+  SG_TILES(3, 2, 2);
+#undef SG_TILES
 #undef SG_ROWS
 }
 
@@ -389,6 +417,7 @@ static int check_operands(const char* what, const void* X, long ldx, const void*
   if (M > 16) MIE_FAIL("%s: %d rows (at most 16)", what, M);
   if (K <= 0 || (K & 7)) MIE_FAIL("%s: K = %d must be a positive multiple of 8", what, K);
   if (ldx < K || ldw < K || (ldw & 7) || (ldx & 7)) MIE_FAIL("%s: leading dims %ld, %ld for K %d", what, ldx, ldw, K);
+  if (ldx > 1L << 24 || ldw > 1L << 24) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^24)", what, ldx, ldw);      // 32-bit offsets
   if (((uintptr_t)X | (uintptr_t)W) & 15) MIE_FAIL("%s: operands must be 16-byte aligned", what);
   return 0;
 }
