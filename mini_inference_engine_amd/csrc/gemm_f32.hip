@@ -27,10 +27,13 @@
 //   8 r + b (whole cache lines, where the instruction's own order would touch 16 lines a quarter wave), block b of 16 bytes at
 //   8 r + (b ^ r % 8), so that the fragment reads spread over all banks; parts of K meet in the LDS at the end.  Eight waves a
 //   workgroup (a deeper queue of loads a compute unit) while the tiles do not fill the compute units, four from there on.
+//   A product that goes into a stream whose norm is wanted next takes two workgroups a tile instead, half of K each (a narrow
+//   weight's tiles alone leave half of the compute units idle), and the kernel that joins the quarters adds and norms: product, add and
+//   norm at 4 rows, before / now: [2048, 2048] 10.6 / 8.9 us, [2048, 5632] 17.5 / 13.8.
 // tile_f32_kernel (M > 16): the matrix unit bounds it.  BM x BN outputs a workgroup; a stage of 32 k comes into registers,
 //   is split there once for all waves, and goes into the LDS as three planes of bfloat16 (two buffers), while the stage
 //   before is multiplied.  Few tiles: the grid is also cut over quarters or eighths, whose sums go to memory and meet in
-//   reduce_f32_kernel.
+//   reduce_f32_kernel, or with the norm that follows in reduce_add_norm_kernel (512 rows of [2048, 2048] with add and norm 38.5 / 36.0).
 //
 // Measured on MI355X against the same kernels on v_mfma_f32_16x16x4_f32, both without the factor of 2^16 (us; those / these): 512 rows of
 // [11264, 2048] with SwiGLU 237 / 175, [2048, 5632] 116 / 73, [2048, 2048] 51 / 35; 100 rows 69 / 59, 36 / 29, 21 / 16; 4 rows 21.9 / 19.2,
@@ -146,7 +149,7 @@ __device__ __forceinline__ void again_if_not_finite(f32x4& v, const float* x, co
   }
 }
 
-enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2, GF_ROPE = 3 };
+enum { GF_STORE = 0, GF_ADD = 1, GF_SWIGLU = 2, GF_ROPE = 3, GF_PART = 4 };
 
 // The q/k/v projection's epilogue: W's rows are q heads, k heads, v heads of D; a tile is 8 rotary pairs of one head.
 struct RopeArgs {
@@ -199,11 +202,12 @@ __device__ __forceinline__ bf16x8 other_half(const bf16x8& v) {
 // nobody's result), and one wait serves both: a step of 4 rows
 // (22 layers of width 2,048) 1,710 us with a step at a time, 1,616 with two.
 // SWIGLU: W is gate rows then up rows (up_offset apart); a tile is 8 gate rows and the 8 up rows of the same columns.
+// PART: a workgroup of four waves takes half of K (blockIdx.y), an eighth a wave, and leaves its two quarters' sums in out [4, M, N].
 template <int EPI, int WAVES, int SLOTS, int XL>
 __global__ void __launch_bounds__(WAVES * 64)
 skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ out,
                   long ldo, const float* __restrict__ bias, int M, int N, int K, int up_offset, RopeArgs rope) {
-  constexpr int EPW = 8 / WAVES;              // eighths a wave
+  constexpr int EPW = EPI == GF_PART ? 1 : 8 / WAVES;              // eighths a wave
   constexpr int U = XL == 1 ? 2 : 1;          // steps at once
   constexpr int L = 2 + XL, SLOT_BYTES = L * 1024;       // loads a slot of 32 k: 16 weight rows of 128 bytes, then the x rows
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
@@ -216,8 +220,9 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
   int first_end, ks0, ks1;
   {
     int b;
-    eighth_range(cut, wave * EPW, ks0, first_end);
-    eighth_range(cut, wave * EPW + EPW - 1, b, ks1);
+    const int e = wave * EPW + (EPI == GF_PART ? 4 * blockIdx.y : 0);
+    eighth_range(cut, e, ks0, first_end);
+    eighth_range(cut, e + EPW - 1, b, ks1);
   }
   const int lrow = lane >> 3, lblk = (lane & 7) ^ lrow;            // this lane's place in a load of 8 rows
   auto weight_row = [&](int r) {              // of the tile's row r; -1: there is none
@@ -301,6 +306,14 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
   // this thread's result: x row m, column c of the tile
   const int m = threadIdx.x >> 4, c = threadIdx.x & 15;
   const int src = (((c >> 2) << 4) + m) * 4 + (c & 3);
+  if (EPI == GF_PART) {
+    const int n = tile * 16 + c;
+    if (m >= M || n >= N) return;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      out[(size_t)(2 * blockIdx.y + q) * M * N + (size_t)m * N + n] = s_acc[2 * q * 256 + src] + s_acc[(2 * q + 1) * 256 + src];
+    return;
+  }
   float v = 0.f;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -549,6 +562,58 @@ reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long 
   }
 }
 
+// The same joined into the 32-bit stream [M, N], with the RMSNorm that reads the stream next: y [M, N] = stream * rsqrt(mean(stream^2) +
+// eps) * g.  A workgroup a row; threads, groups of four and the order of the squares' sum are those of the add + norm kernel
+// (embed_norm.hip), so a row has the same bits whichever of the two makes it.
+constexpr int GF_NORM_THREADS = 256, GF_NORM_MOST = 4 * GF_NORM_THREADS * 8;
+__device__ __forceinline__ f32x4 norm_weight4(const float* g) { return *reinterpret_cast<const f32x4*>(g); }
+__device__ __forceinline__ f32x4 norm_weight4(const bf16* g) {
+  const uint2 u = *reinterpret_cast<const uint2*>(g);
+  return f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xFFFF0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xFFFF0000u)};
+}
+template <int PARTS, typename TW, int VEC>
+__global__ void __launch_bounds__(GF_NORM_THREADS)
+reduce_add_norm_kernel(const float* __restrict__ part, float* __restrict__ stream, const TW* __restrict__ g, float* __restrict__ y, int M,
+                       int N, float eps, const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, int K) {
+  __shared__ float scratch[16];
+  const size_t m = blockIdx.x, stride = (size_t)M * N / 4;
+  f32x4 r[VEC], w[VEC], old[VEC];
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    const int i = (threadIdx.x + k * GF_NORM_THREADS) * 4;
+    r[k] = w[k] = old[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i < N) {
+      old[k] = *reinterpret_cast<const f32x4*>(stream + m * N + i);
+      w[k] = norm_weight4(g + i);
+      r[k] = join_parts<PARTS>(reinterpret_cast<const f32x4*>(part + m * N + i), stride);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    const int i = (threadIdx.x + k * GF_NORM_THREADS) * 4;
+    if (i < N) {
+      again_if_not_finite(r[k], X + m * ldx, W + (size_t)i * ldw, ldw, K);
+      r[k] = old[k] + r[k];
+      *reinterpret_cast<f32x4*>(stream + m * N + i) = r[k];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss = fmaf(r[k][j], r[k][j], ss);
+  }
+  const float total = block_sum(ss, scratch);
+  const float rstd = 1.0f / sqrtf(total / (float)N + eps);
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    const int i = (threadIdx.x + k * GF_NORM_THREADS) * 4;
+    if (i < N) {
+      f32x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = r[k][j] * rstd * w[k][j];
+      *reinterpret_cast<f32x4*>(y + m * N + i) = o;
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ host
 MIE_EXPORT const char* gemm_f32_last_error() { return g_mie_error; }
 
@@ -606,9 +671,11 @@ static int launch_skinny(const float* X, long ldx, const float* W, long ldw, flo
     auto kernel = skinny_f32_kernel<EPI, WAVES, SLOTS, XL>;                                                               \
     constexpr int lds = WAVES * SLOTS * (2 + XL) * 1024;                                                                  \
     if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;                                                   \
-    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, M, N, K, N, rope);  \
+    hipLaunchKernelGGL(kernel, dim3(tiles, EPI == GF_PART ? 2 : 1), dim3(WAVES * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, M, N, K, N, rope); \
   }
-  if (tiles <= 256) {
+  if constexpr (EPI == GF_PART) {             // (few slots: those behind a wave's few steps bring zeros; 6 to 12 are up to 1.4 us slower)
+    if (M <= 8) GF_SKINNY(4, 4, 1) else GF_SKINNY(4, 4, 2)
+  } else if (tiles <= 256) {
     if (M <= 8) GF_SKINNY(8, 6, 1) else GF_SKINNY(8, 4, 2)
   } else {
     if (M <= 8) GF_SKINNY(4, 4, 1) else GF_SKINNY(4, 3, 2)
@@ -679,6 +746,47 @@ MIE_EXPORT int mie_gemm_f32(const float* X, long ldx, const float* W, long ldw, 
   return epi == GF_STORE ? launch_reduce<GF_STORE>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
        : epi == GF_ADD ? launch_reduce<GF_ADD>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
                        : launch_reduce<GF_SWIGLU>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s);
+}
+
+// How many units K is cut into where the product is added into a stream whose RMSNorm is wanted next (mie_gemm_f32_add_norm), 0: the
+// product with the add and the norm by themselves.  More than 16 rows: the units that the product is cut into anyway.  Up to 16
+// rows: quarters, two a workgroup, while that gives every compute unit at most one workgroup and a wave some steps.
+MIE_EXPORT int mie_f32_norm_units(int M, int N, int K) {
+  if (M <= 0 || (N & 3) || N > GF_NORM_MOST || K <= 0) return 0;
+  if (M <= 16) return K >= 1024 && 2 * ((N + 15) / 16) <= mie_compute_units() ? 4 : 0;
+  const int units = tile_plan(M, N, K, false).units;
+  return units > 1 ? units : 0;
+}
+
+// stream [M, N] += x W^T and y [M, N] = RMSNorm(stream) with weight g (float32 if g_f32, else bfloat16).  part: mie_f32_norm_units(M, N, K)
+// (which is not 0) * M * N floats.  Everything 16-byte aligned.
+MIE_EXPORT int mie_gemm_f32_add_norm(const float* X, long ldx, const float* W, long ldw, float* stream, const void* g, int g_f32, float* y,
+                                     float* part, int M, int N, int K, float eps, hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  const int units = mie_f32_norm_units(M, N, K);
+  if (!units) MIE_FAIL("gemm_f32_add_norm: %d rows of [%d, %d] are not cut into units", M, N, K);
+  if (!stream || !g || !y || !part || ((uintptr_t)g | (uintptr_t)y | (uintptr_t)part) & 15) MIE_FAIL("gemm_f32_add_norm: operands must be 16-byte aligned");
+  if (check_operands("gemm_f32_add_norm", X, ldx, W, ldw, stream, N, N, K)) return -1;
+  if (M <= 16) {
+    if (launch_skinny<GF_PART>(X, ldx, W, ldw, part, N, nullptr, M, N, K, s)) return -1;
+  } else if (launch_tiles(X, ldx, W, ldw, part, N, nullptr, 0, M, N, K, tile_plan(M, N, K, false), s)) return -1;
+  const int groups = (N / 4 + GF_NORM_THREADS - 1) / GF_NORM_THREADS;
+#define GF_NORM(PARTS, TW, VEC)                                                                                                  \
+  hipLaunchKernelGGL((reduce_add_norm_kernel<PARTS, TW, VEC>), dim3(M), dim3(GF_NORM_THREADS), 0, s, part, stream, (const TW*)g, y, M, N, \
+                     eps, X, ldx, W, ldw, K)
+#define GF_NORM_VEC(PARTS, TW)                 \
+  if (groups <= 2) GF_NORM(PARTS, TW, 2);      \
+  else if (groups <= 4) GF_NORM(PARTS, TW, 4); \
+  else GF_NORM(PARTS, TW, 8)
+  if (units == 4) {
+    if (g_f32) { GF_NORM_VEC(4, float); } else { GF_NORM_VEC(4, bf16); }
+  } else {
+    if (g_f32) { GF_NORM_VEC(8, float); } else { GF_NORM_VEC(8, bf16); }
+  }
+#undef GF_NORM_VEC
+#undef GF_NORM
+  MIE_CHECK_LAUNCH("gemm_f32_add_norm");
+  return 0;
 }
 
 // The q/k/v projection of up to 16 rows with what follows it: W [(Hq + 2 Hkv) D, K]; q and k rotated (half-split pairs over the

@@ -247,6 +247,27 @@ class HipBackend(KernelBackend):
                                             _ptr(part), M, cols // 2 if epi == self.F32_SWIGLU else cols, K, self._stream()))
         return True
 
+    def _f32_add_norm(self, x, w, sink):
+        """The product added into the sink's stream and the norm that reads it next where the kernel that joins the product's
+        parts makes that norm too; None: nothing is done, the product and the norm are on their own."""
+        g, (M, K), N = sink.norm_weight, x.shape, w.shape[0]
+        if (g is None or g.dtype not in (torch.bfloat16, torch.float32) or tuple(g.shape) != (N,) or not g.is_contiguous()
+                or g.data_ptr() % 16):
+            return None
+        lib = self.lib("gemm_f32")
+        units = lib.mie_f32_norm_units(M, N, K)
+        if not units:
+            return None
+        self._on_device(g)
+        part = torch.empty((units, M, N), dtype=torch.float32, device=x.device)
+        normed = torch.empty((M, N), dtype=torch.float32, device=x.device)
+        library.check(lib, lib.mie_gemm_f32_add_norm(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(sink.stream), _ptr(g),
+                                                     int(g.dtype == torch.float32), _ptr(normed), _ptr(part), M, N, K,
+                                                     float(sink.norm_eps), self._stream()))
+        done = Normed(self, None, sink.stream, g, sink.norm_eps)
+        done._value = normed            # the norm is computed: materialize() hands this out
+        return done
+
     # ---- few-row products of the bfloat16 path: one fused kernel each
     SKINNY_MAX_ROWS = 16      # the kernel's own limit (one tile of rows); a decode step of 16 rows of 512 keys at the
                               # benchmark's sizes takes 1.15 ms, one of 17 rows with the split product 1.27
@@ -472,6 +493,9 @@ class HipBackend(KernelBackend):
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         if self._f32_ok(x, w, bias, out_dtype) and (sink is None or sink.stream.data_ptr() % 16 == 0):
             if sink is not None:
+                done = self._f32_add_norm(x, w, sink) if bias is None else None
+                if done is not None:
+                    return done
                 self._f32_product(x, w, self.F32_ADD, sink.stream, bias)
                 return None if sink.norm_weight is None else Normed(self, None, sink.stream, sink.norm_weight, sink.norm_eps)
             out = torch.empty((M, N), dtype=torch.float32, device=w.device)

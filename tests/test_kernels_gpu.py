@@ -473,6 +473,31 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
+@pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", [(1, 1024, 4, 4), (8, 2048, 2048, 4), (9, 1028, 1000, 4), (16, 5632, 516, 4), (17, 2052, 36, 8), (20, 1024, 4100, 8),
+                                  (100, 360, 2048, 4), (40, 1536, 8192, 4), (300, 200, 132, 8)])
+def test_float32_product_with_the_norm_behind_it(ops, case, g_dtype):
+    """A float32 product added into the stream whose norm follows: parts of K that meet in the kernel that adds and norms give
+    the bits of the product, the add and the norm by themselves (every width of a thread, quarters and eighths, edges of tiles)."""
+    from mini_inference_engine_amd.kernels.api import Sink
+    o, (M, K, N, units) = ops[torch.float32], case
+    lib = o.lib("gemm_f32")
+    assert lib.mie_f32_norm_units(M, N, K) == units, "the case must take the path it is for"
+    torch.manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) / math.sqrt(K)
+    x[M // 2, 3] = 3.0e38                       # results beyond what the parts can hold are computed again, here too
+    g = (1 + 0.1 * torch.randn(N, device=DEV)).to(g_dtype)
+    stream = torch.randn(M, N, device=DEV)
+    plain = stream.clone()
+    assert o.linear(x, w, add_to=plain) is None
+    with counted(o, "gemm_f32", "mie_gemm_f32_add_norm") as calls:
+        normed = o.linear(x, w, add_to=Sink(stream, g, 1e-5))
+    assert len(calls) == 1 and torch.equal(stream, plain)
+    assert torch.equal(normed.materialize(), o.add_rmsnorm(None, plain, g, 1e-5))
+    assert lib.mie_f32_norm_units(16, 8196, 2048) == 0 and lib.mie_f32_norm_units(4, 64, 512) == 0
+    assert lib.mie_gemm_f32_add_norm(x.data_ptr(), K, w.data_ptr(), K, stream.data_ptr(), g.data_ptr(), 1, None, x.data_ptr(), M, N, K, 1e-5, None) != 0
+
+
 # rows, K, columns and the tiles of 16 weight rows a workgroup has
 @pytest.mark.parametrize("case", [(17, 64, 4, 1), (33, 72, 12, 1), (64, 2008, 3000, 2), (48, 328, 5632, 3), (128, 2048, 5632, 3),
                                   (50, 8, 8188, 4), (97, 200, 8192, 4), (31, 136, 11008, 6), (64, 192, 11004, 6), (64, 256, 14336, 7)])
