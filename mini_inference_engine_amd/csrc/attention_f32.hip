@@ -10,14 +10,19 @@
 // A wave owns 16 queries of one kv head: the heads of its group, for as many neighbouring tokens as fit (16 / heads a
 // group).  S^T = K Q^T and O^T += V^T P^T by v_mfma_f32_16x16x4_f32: a lane of the scores' accumulator holds four keys
 // of one query, which is what the second product takes as its B operand, key 4 g + i of lane group g in instruction i;
-// K rows and the values (transposed within their page) are read from memory in exactly these 16-byte pieces, a page's
-// 16 keys at a time.  The queries of a group share every load; nothing goes through the LDS but the query fragments.
-//   portions: a wave walks its segments itself.     single tokens: a wave a segment, joined by merge_f32_kernel.
-// What bounds it is the latency of a wave's own loads (a segment's K, then its V, all of one issued together) and, for
-// portions, the reads out of the L2s.  The kernel of attention.hip, one wave a (token, head), reads every key once a head
-// and token, a quarter of a cache line a load: 512 tokens of 32 / 4 heads of 64 642 -> 38 us, 4 single tokens of 300 to
-// 900 keys 200 -> 11 + 5 (MI355X).
-#include "common.hpp"
+// K rows and the values (transposed within their page) are used in exactly these 16-byte pieces, a page's
+// 16 keys at a time.
+//   portions: four waves side by side (neighbouring tiles of 16 queries) walk their segments together.  A segment's K, then its V,
+//     come into a ring in the LDS by loads that write it directly, whole cache lines, each read once for all four waves and one to three
+//     of them on their way while one is used; the 16-byte blocks of a K row are turned by the row, those of a V row by a quarter of it,
+//     so that the fragment reads spread over all banks.  What bounds it: the longest workgroup's chain of segments, 3.4 us of matrix
+//     instructions and 1.5 of exponentials each.  Read by every wave for itself (16 cache lines a quarter wave and load) it
+//     took 41 us for 512 tokens of 32 / 4 heads of 64, now 30; 1,024 tokens 113 and 64, of 32 / 8 heads of 128 197 and 114.
+//   single tokens: a wave a segment, joined by merge_f32_kernel.  What bounds it is the latency of a wave's own loads (a segment's K,
+//     then its V, all of one issued together).
+// The kernel of attention.hip, one wave a (token, head), reads every key once a head and token, a quarter of a cache line a load: 512
+// tokens of 32 / 4 heads of 64 642 us, 4 single tokens of 300 to 900 keys 200 for 11 + 5 here (MI355X).
+#include "launch.hpp"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -32,6 +37,47 @@ struct AttArgs {
   int max_blocks, Hq, Hkv, page, window;
   float scale;
 };
+
+// The scores of a segment (lane column r16's query at position pos with keys from lo on) become exp(s - m); m and l.
+__device__ __forceinline__ void segment_weights(f32x4 (&s)[AF_TILES], int base, int pos, int lo, float scale, float& m, float& l) {
+  const int g = (threadIdx.x & 63) >> 4;
+  float top = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < AF_TILES; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = base + t * 16 + 4 * g + i;
+      s[t][i] = key <= pos && key >= lo ? __fmul_rn(s[t][i], scale) : -INFINITY;
+      top = fmaxf(top, s[t][i]);
+    }
+  top = fmaxf(top, __shfl_xor(top, 16, 64));
+  top = fmaxf(top, __shfl_xor(top, 32, 64));
+  m = top;
+  const float sub = top == -INFINITY ? 0.f : top;
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < AF_TILES; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[t][i] = expf(s[t][i] - sub);
+      sum += s[t][i];
+    }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+  l = sum;
+}
+
+// A value tile's fragment c (keys key .. key + 3 of this lane): what none of the 16 queries sees becomes zero; true if what only some
+// of them see is not finite.
+__device__ __forceinline__ bool clean_values(f32x4& v, int key, int first, int last, int all_lo, int all_pos) {
+  bool some = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = key + i >= first && key + i <= last ? v[i] : 0.f;
+    some |= !(fabsf(v[i]) < INFINITY) && (key + i < all_lo || key + i > all_pos);
+  }
+  return some;
+}
 
 // What segment `seg` gives 16 queries of kv head kvh: fragments qf, each lane's query at position pos (-1: none) with
 // keys from lo on; first / last: the smallest lo and the largest position among the 16.  Every query sees the keys from all_lo to
@@ -72,30 +118,7 @@ __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, in
 #pragma unroll
         for (int t = 0; t < AHEAD; ++t) s[u + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][c][j], qf[c][j], s[u + t], 0, 0, 0);
   }
-  float top = -INFINITY;
-#pragma unroll
-  for (int t = 0; t < AF_TILES; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = base + t * 16 + 4 * g + i;
-      s[t][i] = key <= pos && key >= lo ? __fmul_rn(s[t][i], a.scale) : -INFINITY;
-      top = fmaxf(top, s[t][i]);
-    }
-  top = fmaxf(top, __shfl_xor(top, 16, 64));
-  top = fmaxf(top, __shfl_xor(top, 32, 64));
-  m = top;
-  const float sub = top == -INFINITY ? 0.f : top;
-  float sum = 0.f;
-#pragma unroll
-  for (int t = 0; t < AF_TILES; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[t][i] = expf(s[t][i] - sub);
-      sum += s[t][i];
-    }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
-  l = sum;
+  segment_weights(s, base, pos, lo, a.scale, m, l);
 #pragma unroll
   for (int c = 0; c < DT; ++c) o[c] = none;
   bool some = false;
@@ -114,12 +137,7 @@ __device__ __forceinline__ void segment_sums(const AttArgs& a, const int* bt, in
       if (key - 4 * g < all_lo || key - 4 * g + 15 > all_pos) {
         // keys none of the queries sees: nobody wrote them, or their page went back; and keys some of them see
 #pragma unroll
-        for (int c = 0; c < DT; ++c)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            vf[t][c][i] = key + i >= first && key + i <= last ? vf[t][c][i] : 0.f;
-            some |= !(fabsf(vf[t][c][i]) < INFINITY) && (key + i < all_lo || key + i > all_pos);
-          }
+        for (int c = 0; c < DT; ++c) some |= clean_values(vf[t][c], key, first, last, all_lo, all_pos);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -150,65 +168,232 @@ __device__ __forceinline__ void load_queries(const AttArgs& a, int t, int h, f32
   }
 }
 
+// A portion's workgroup: AF_TILE_WAVES tiles of 16 queries side by side.  Up to head size 64 two waves a tile take the segments in turn, two
+// at a time; the second hands m, l and O to the first, which joins all in order: 512 tokens of 32 / 4 heads of 64 35.0 us with one
+// wave, 30.0 with two (33.1 with one of them at its scores while the other is at its values).  Beyond, the LDS holds no two segments
+// twice.
+constexpr int AF_TILE_WAVES = 4;
+template <int DT> constexpr int AF_SIDES = DT <= 4 ? 2 : 1;
+template <int DT> constexpr int AF_RING = DT <= 4 ? 2 : 160 / (8 * DT);      // steps: AF_SIDES segments' K or V
+template <int DT> constexpr int AF_EXCHANGE = DT <= 4 ? AF_TILE_WAVES * (4 * DT + 3) * 256 : 0;
+template <int DT> constexpr int AF_LDS = AF_RING<DT> * AF_SIDES<DT> * AF_SEG * DT * 64 + AF_EXCHANGE<DT>;
+
+// Workgroup (tile of AF_TILE_WAVES * per_tile tokens, the last first; kv head and tile of 16 heads), row blockIdx.y.
 template <int DT>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(AF_TILE_WAVES * AF_SIDES<DT> * 64)
 portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ row_start, const int* __restrict__ row_position,
-                   int row0, int per_tile) {
-  constexpr int D = DT * 16;
-  const int row = row0 + blockIdx.z, begin = row_start[row], n = row_start[row + 1] - begin;
-  const int rep = a.Hq / a.Hkv, head_tiles = per_tile > 1 ? 1 : (rep + 15) / 16;
-  const int kvh = blockIdx.y / head_tiles, h0 = (blockIdx.y - kvh * head_tiles) * 16;
-  // the last tokens see the most keys: their waves start first
-  const int tile = gridDim.x - 1 - blockIdx.x;
-  const int t0 = tile * per_tile;
-  if (t0 >= n) return;
-  const int lane = threadIdx.x, r16 = lane & 15, g = lane >> 4;
+                   int row0, int per_tile, int tiles) {
+  constexpr int D = DT * 16, BLOCKS = 4 * DT, RING = AF_RING<DT>, SIDES = AF_SIDES<DT>, BUFFER = AF_SEG * D * 4;
+  constexpr int WAVES = AF_TILE_WAVES * SIDES, OWN = AF_TILES / AF_TILE_WAVES, L = OWN * DT;      // tiles of 16 keys a wave brings in a step
+  static_assert((RING - 2) * L <= 63 && RING >= 2, "more loads in flight than the counter holds");
+  extern __shared__ __align__(1024) char af_lds[];
+  const int row = row0 + blockIdx.y, begin = row_start[row], n = row_start[row + 1] - begin;
+  const int rep = a.Hq / a.Hkv, head_tiles = per_tile > 1 ? 1 : (rep + 15) / 16, heads = a.Hkv * head_tiles;
+  const int tile = tiles - 1 - blockIdx.x / heads, hy = blockIdx.x % heads;
+  const int kvh = hy / head_tiles, h0 = (hy - kvh * head_tiles) * 16;
+  const int all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = all_waves % AF_TILE_WAVES, side = all_waves / AF_TILE_WAVES;
+  const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int T0 = tile * AF_TILE_WAVES * per_tile;
+  if (T0 >= n) return;
+  const auto first_of = [&](int p) { return a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0; };
+  // of the workgroup's queries, and of this wave's (none: last before first)
+  const int all_last = row_position[row] + T0 + (n - T0 < AF_TILE_WAVES * per_tile ? n - T0 : AF_TILE_WAVES * per_tile) - 1;
+  const int all_first = first_of(row_position[row] + T0);
+  const int t0 = T0 + wave * per_tile;
   const int ti = per_tile > 1 ? r16 / rep : 0, hi = per_tile > 1 ? r16 - ti * rep : h0 + r16;
   const bool live = hi < rep && ti < per_tile && t0 + ti < n;
   const int t = live ? begin + t0 + ti : -1, h = kvh * rep + hi;
   const int p0 = row_position[row] + t0;
-  const int last = p0 + (n - t0 < per_tile ? n - t0 : per_tile) - 1;
-  const int first = a.window > 0 && p0 - a.window + 1 > 0 ? p0 - a.window + 1 : 0;
-  const int pos = live ? p0 + ti : -1;
-  const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
+  const int last = t0 < n ? p0 + (n - t0 < per_tile ? n - t0 : per_tile) - 1 : -1;
+  const int first = first_of(p0), pos = live ? p0 + ti : -1, lo = first_of(pos);
   f32x4 qf[DT], O[DT];
   load_queries<DT>(a, t, h, qf);
-  float M = -INFINITY, L = 0.f;
+  float M = -INFINITY, L_sum = 0.f;
 #pragma unroll
   for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int* bt = a.block_tables + (size_t)row * a.max_blocks;
-  const auto first_of = [&](int p) { return a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0; };
+
+  // The ring: step 2 i is K of the workgroup's segments SIDES i and on (a side takes one), step 2 i + 1 their V.  A wave brings in two
+  // tiles of 16 keys a step.
+  // K: 16-byte block b of key r at place (b + r) % BLOCKS of its row.  V: block g of dim d at (g + d / 4) % 4.
+  const int seg0 = all_first / AF_SEG, segs = all_last / AF_SEG - seg0 + 1, steps = 2 * ((segs + SIDES - 1) / SIDES);
+  uint32_t koff[DT];
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    const int i = j * 64 + lane, r = i / BLOCKS, place = i - r * BLOCKS;
+    koff[j] = r * D * 4 + ((place + BLOCKS - r % BLOCKS) % BLOCKS) * 16;
+  }
+  const uint32_t voff = (lane >> 2) * a.page * 4 + (((lane & 3) - (lane >> 4)) & 3) * 16;
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)af_lds;
+  // pages are looked up through the scalar unit, a step ahead of their use: a vector load would come back after all that is on its way
+  const auto* pages = (const __attribute__((address_space(4))) int*)(uintptr_t)bt;
+  int own_page[OWN];
+  auto key_of = [&](int p, int u) {           // first key of the wave's tile u in step p
+    const int seg = (p >> 1) * SIDES + side, key = (seg0 + seg) * AF_SEG + (wave * OWN + u) * 16;
+    // a tile nobody sees stands for a neighbour: every table entry read is one of the request's
+    return key > all_last ? all_last & ~15 : key + 15 < all_first ? all_first & ~15 : key;
+  };
+  auto look_up = [&](int p) {
+#pragma unroll
+    for (int u = 0; u < OWN; ++u) own_page[u] = pages[key_of(p, u) / a.page];
+  };
+  auto issue = [&](int p) {
+    const bool v = p & 1;
+#pragma unroll
+    for (int u = 0; u < OWN; ++u) {
+      const int tt = wave * OWN + u, key = key_of(p, u);
+      const size_t at = ((size_t)own_page[u] * a.Hkv + kvh) * a.page * D;
+      const uint32_t to = lds0 + (p % RING * SIDES + side) * BUFFER + tt * 1024 * DT;
+      if (v) {
+        const float* vp = a.v_cache + at + key % a.page;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) mie_load_to_lds(vp + (size_t)(16 * j) * a.page, voff, to + j * 1024);
+      } else {
+        const float* kp = a.k_cache + at + (size_t)(key % a.page) * D;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) mie_load_to_lds(kp, koff[j], to + j * 1024);
+      }
+    }
+  };
+  look_up(0);
+  issue(0);
+#pragma unroll
+  for (int c = 0; c < DT; ++c) asm volatile("" : "+v"(qf[c]));      // the queries are waited for here, with the first K alone on its way
+#pragma unroll
+  for (int p = 1; p < RING - 1; ++p)
+    if (p < steps) {
+      look_up(p);
+      issue(p);
+    }
+  look_up(RING - 1);
+
+  int kat[DT];                                // of this lane's fragments: K block 4 c + g of key r16, V block g of dim r16
+#pragma unroll
+  for (int c = 0; c < DT; ++c) kat[c] = r16 * D * 4 + ((4 * c + g + r16) % BLOCKS) * 16;
+  const int vat = r16 * 64 + ((g + (r16 >> 2)) & 3) * 16;
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  f32x4 s[AF_TILES];
+  float m = 0.f, l = 0.f;
   bool odd = false;
-  auto add = [&](int seg, int qpos, int f, int e, int all_lo, int all_pos, bool mine) {
-    float m, l, wa, wb;
-    f32x4 o[DT];
-    segment_sums<DT>(a, bt, kvh, seg, qf, qpos, lo, f, e, all_lo, all_pos, m, l, o, odd);
-    if (!mine) return;
+  auto join = [&](float m, float l, const f32x4 (&o)[DT]) {
+    float wa, wb;
     join_weights(M, m, wa, wb);
-    L = joined(L, wa, l, wb);
+    L_sum = joined(L_sum, wa, l, wb);
 #pragma unroll
     for (int c = 0; c < DT; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) O[c][i] = joined(O[c][i], wa, o[c][i], wb);
   };
-  for (int seg = first / AF_SEG; seg * AF_SEG <= last && !odd; ++seg) add(seg, pos, first, last, first_of(last), p0, true);
+  // what the other side made of its segment, a barrier after it did: the next time it writes is two barriers on
+  float* exchange = reinterpret_cast<float*>(af_lds + RING * SIDES * BUFFER) + wave * (4 * DT + 3) * 64 + lane;
+  auto join_other = [&](int seg) {
+    const int base = (seg0 + seg) * AF_SEG;
+    if ( base > last || base + AF_SEG <= first) return;
+    f32x4 o[DT];
+#pragma unroll
+    for (int c = 0; c < DT; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[c][i] = exchange[(4 * c + i) * 64];
+    odd |= exchange[(4 * DT + 2) * 64] != 0.f;
+    join(exchange[4 * DT * 64], exchange[(4 * DT + 1) * 64], o);
+  };
+  for (int p = 0; p < steps; ++p) {
+    if (p + RING - 1 <= steps) MIE_VMCNT((RING - 2) * L);
+    else MIE_VMCNT(0);
+    __builtin_amdgcn_s_barrier();             // step p is in the LDS; everybody is done with step p - 1
+    asm volatile("" ::: "memory");
+    if (p + RING - 1 < steps) {
+      issue(p + RING - 1);
+      look_up(p + RING);
+    }
+    const bool values = p & 1;
+    const int seg = (p >> 1) * SIDES + side, base = (seg0 + seg) * AF_SEG;
+    if (SIDES == 2 && !side && !values && p) join_other(seg - 1);
+    const char* buf = af_lds + (p % RING * SIDES + side) * BUFFER;
+    const bool sees = base <= last && base + AF_SEG > first;
+    if (sees && !values) {
+#pragma unroll
+      for (int u = 0; u < AF_TILES; u += 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[u + k] = none;
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {
+          f32x4 kf[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) kf[k] = *reinterpret_cast<const f32x4*>(buf + (u + k) * 1024 * DT + kat[c]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s[u + k] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[k][j], qf[c][j], s[u + k], 0, 0, 0);
+        }
+      }
+      segment_weights(s, base, pos, lo, a.scale, m, l);
+    }
+    if (sees && values) {
+      f32x4 o[DT];
+      bool some = false;
+#pragma unroll
+      for (int c = 0; c < DT; ++c) o[c] = none;
+#pragma unroll
+      for (int u = 0; u < AF_TILES; ++u) {
+        f32x4 vf[DT];
+#pragma unroll
+        for (int c = 0; c < DT; ++c) vf[c] = *reinterpret_cast<const f32x4*>(buf + u * 1024 * DT + c * 1024 + vat);
+        const int key = base + u * 16;
+        if (key < first_of(last) || key + 15 > p0) {
+#pragma unroll
+          for (int c = 0; c < DT; ++c) some |= clean_values(vf[c], key + 4 * g, first, last, first_of(last), p0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int c = 0; c < DT; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[c][i], s[u][i], o[c], 0, 0, 0);
+      }
+      const bool bad = __builtin_amdgcn_ballot_w64(some) != 0;
+      if (SIDES == 2 && side) {
+#pragma unroll
+        for (int c = 0; c < DT; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) exchange[(4 * c + i) * 64] = o[c][i];
+        exchange[4 * DT * 64] = m;
+        exchange[(4 * DT + 1) * 64] = l;
+        exchange[(4 * DT + 2) * 64] = bad ? 1.f : 0.f;
+      } else {
+        odd |= bad;
+        join(m, l, o);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // this wave has read the buffer before the next barrier
+  }
+  if (SIDES == 2) {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (side) return;
+    join_other(steps - 1);                    // (the pair's second segment; not there: seen by nobody)
+  }
   if (odd) {
     // (values of the row's later tokens, or, beside padding tokens, of slots of its last page that nobody wrote)  All over
     // again, one token after the other: the same bits for what is a number
     M = -INFINITY;
-    L = 0.f;
+    L_sum = 0.f;
 #pragma unroll
     for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-    for (int p = p0; p <= last; ++p) {
-      const bool mine = pos == p;
-      const int f = first_of(p);
+    for (int q = p0; q <= last; ++q) {
+      const bool mine = pos == q;
+      const int f = first_of(q);
 #pragma unroll 1
-      for (int seg = f / AF_SEG; seg * AF_SEG <= p; ++seg) add(seg, mine ? pos : -1, f, p, f, p, mine);
+      for (int seg = f / AF_SEG; seg * AF_SEG <= q; ++seg) {
+        float sm, sl;
+        f32x4 o[DT];
+        bool again;                           // (of no account: all queries are one token's)
+        segment_sums<DT>(a, bt, kvh, seg, qf, mine ? pos : -1, lo, f, q, f, q, sm, sl, o, again);
+        if (mine) join(sm, sl, o);
+      }
     }
   }
   if (!live) return;
-  const float inv = 1.0f / L;
+  const float inv = 1.0f / L_sum;
   // O[c][i] of lane (r16, g): dim 16 c + 4 g + i of the lane's query
   float* op = out + ((size_t)t * a.Hq + h) * D + 4 * g;
 #pragma unroll
@@ -346,8 +531,16 @@ MIE_EXPORT int mie_attention_f32_portions(const float* q, long q_stride, const f
   if (check(a, out, D)) return -1;
   const int rep = Hq / Hkv, per_tile = rep <= 16 ? 16 / rep : 1, head_tiles = per_tile > 1 ? 1 : (rep + 15) / 16;
   if (Hkv * head_tiles > 65535 || rows - row0 > 65535) MIE_FAIL("attention_f32: %d kv heads, %d rows are beyond the grid", Hkv, rows - row0);
-  const dim3 grid((max_row_tokens + per_tile - 1) / per_tile, Hkv * head_tiles, rows - row0);
-#define AF_PORTIONS(DT) hipLaunchKernelGGL(portion_f32_kernel<DT>, grid, dim3(64), 0, s, a, out, row_start, row_position, row0, per_tile)
+  const int tiles = (max_row_tokens + AF_TILE_WAVES * per_tile - 1) / (AF_TILE_WAVES * per_tile);
+  if ((long)tiles * Hkv * head_tiles > 0x7FFFFFFF) MIE_FAIL("attention_f32: %d tokens are beyond the grid", max_row_tokens);
+  if ((long)page * D > 1L << 26) MIE_FAIL("attention_f32: pages of %d", page);      // 32-bit offsets within a page
+  const dim3 grid(tiles * Hkv * head_tiles, rows - row0);
+#define AF_PORTIONS(DT)                                                                                                              \
+  {                                                                                                                                  \
+    if (mie_allow_lds((const void*)portion_f32_kernel<DT>, AF_LDS<DT>, "attention_f32")) return -1;                                  \
+    hipLaunchKernelGGL(portion_f32_kernel<DT>, grid, dim3(AF_TILE_WAVES * AF_SIDES<DT> * 64), AF_LDS<DT>, s, a, out, row_start,      \
+                       row_position, row0, per_tile, tiles);                                                                         \
+  }
   AF_BY_HEAD(D, AF_PORTIONS)
   MIE_CHECK_LAUNCH("attention_f32 portions");
   return 0;
