@@ -13,7 +13,19 @@
 // merged through LDS; splits write normalised partials and base-2 log-sum-exps, merged by a second,
 // small kernel.  Keys outside [lo, p] get probability 0 by selection and their values are zeroed, so stale
 // or poisoned slots never reach the sums.
+//
+// How keys and values come in (head sizes 64, 96 and 128): each wave brings its blocks of 32 keys into slots of its own
+// in the LDS by loads that write the LDS directly, whole cache lines, and reads the fragments back; a slot is refilled as soon as
+// its fragments are in registers, so all of a wave's slots are on their way while it computes.  Straight into registers in the
+// matrix instruction's order a quarter wave touches 16 rows for 16 (keys) or 8 bytes (values), and the address unit's line look-ups
+// keep a compute unit below the 58 bytes a nanosecond that it can take in.  Measured (MI355X, attention and merge, us, before / now): 32 / 4
+// heads of 64, 64 rows of 200 to 1,990 keys 21.8 / 20.5, 96 rows 32.9 / 28.6, 32 rows of 150 to 900 13.4 / 11.8, 8 of 2,040 10.7 / 10.5; 32 / 8
+// heads of 128, 8 rows of 1,000 to 6,000 41.6 / 35.3, 64 of 200 to 1,990 73.0 / 63.9.  At head size 32 registers are the faster way (64
+// rows of 2,040 keys 17.3 us, 19.1 through the LDS).
+// The 32 keys of a block are dealt to the score tiles' rows so that a lane's eight probabilities belong to eight neighbouring keys,
+// 16 bytes of a value row: lane group g has keys 8 g .. 8 g + 7.
 #include "attention_bf16_common.hpp"
+#include "launch.hpp"
 
 constexpr int NW_SPLIT = D > 128 ? 2 : 4;    // waves per workgroup (bounded by the LDS the merge of the waves needs)
 // When rows and heads alone fill the GPU the context is not split and there is no second kernel; a workgroup then
@@ -22,7 +34,18 @@ constexpr int NW_SPLIT = D > 128 ? 2 : 4;    // waves per workgroup (bounded by 
 // workgroups, and four waves each are faster (256 rows x 4 kv heads of 512 keys: 24.8 against 32.9 us; 64 rows of
 // 2,048 keys: 27.8 against 24.1).
 constexpr int NW_WHOLE = D > 128 ? 2 : (D > 64 ? 4 : 8);
-constexpr long NW_WHOLE_BELOW = 512;         // workgroups from which on a workgroup is NW_SPLIT waves again
+constexpr bool RINGED = D % 32 == 0 && D >= 64 && D <= 128;
+// Blocks of a wave on their way: 32 to 64 KB a workgroup of four waves, 128 of eight (two blocks a wave of four leave room for two
+// workgroups a compute unit: head size 64, 128 rows of 100 to 1,990 keys 33.4 us with one, 36.5 with two, 256 of 512 29.1 and 33.6)
+constexpr int slots_of(int nw) { return !RINGED ? 0 : nw == 8 ? 2 : 1; }
+constexpr int BLOCK_LOADS = D / 8;           // of 1 KB: keys and values of 32 keys
+// Dynamic LDS of a workgroup of nw waves: the slots, and later, in the same place, the waves' sums.
+constexpr int da_lds_bytes(int nw) {
+  const int ring = nw * slots_of(nw) * BLOCK_KEYS * D * 4, sums = nw * 16 * (D + 1) * 4;
+  return ring > sums ? ring : sums;
+}
+// Workgroups up to which one is NW_WHOLE waves: while each has a compute unit's LDS to itself (ringed), or fewer than two a compute unit.
+static long whole_most() { return RINGED ? mie_compute_units() : 2L * mie_compute_units() - 1; }
 
 // What the kernel needs to finish the q/k/v projection of its row itself (FROM_SUMS): the projection's
 // float32 sums, split over K or not, instead of q; the angle tables; where the row's new key and value go.
@@ -62,7 +85,8 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   static_assert(!(KEEP && (SIG || FROM_SUMS || DB)), "kept first keys are built for the plain softmax over finished queries");
   static_assert(!(CHUNK && (SIG || FROM_SUMS || DB || KEEP)), "chunks are built for the plain softmax over finished queries, and for sigmoids");
   __shared__ float s_m[NW][16], s_l[NW][16], s_M[16], s_L[16];
-  __shared__ float s_o[NW][16][D + 1];
+  extern __shared__ __align__(1024) char da_lds[];               // the waves' slots, then s_o [NW][16][D + 1]
+  float* s_o = reinterpret_cast<float*>(da_lds);
   __shared__ __align__(16) bf16 s_q[FROM_SUMS ? 16 : 1][D];
   __shared__ __align__(16) bf16 s_k[FROM_SUMS ? D : 1], s_v[FROM_SUMS ? D : 1];   // the row's own new key and value
   const int b = blockIdx.x;
@@ -94,6 +118,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   // Pages hold a multiple of 16 keys, so each half of a block lies in one page: looked up through the scalar unit, a block
   // ahead.  Looked up by vector loads in front of a block's own, they made every block wait for all of the one before (vector
   // loads return in order), and nothing was on its way beside the block being computed.
+  const auto* pages = (const __attribute__((address_space(4))) int*)(uintptr_t)bt;
   const int last_page = max_blocks - 1;
   const int page_shift = (page & (page - 1)) == 0 ? __builtin_ctz(page) : -1;
   struct Places {
@@ -104,7 +129,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int key = blk + 16 * t, pi = page_shift >= 0 ? key >> page_shift : key / page;
-      p.pg[t] = bt[pi < last_page ? pi : last_page];
+      p.pg[t] = pages[pi < last_page ? pi : last_page];
       p.off[t] = key - pi * page;
     }
     return p;
@@ -128,11 +153,59 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
       B.va[dt].h[1] = *reinterpret_cast<const uint2*>(v1 + at);
     }
   };
-  constexpr bool AHEAD = D <= 128;          // two blocks in registers; larger heads have no room for it
+  // The slots.  Keys: row k of 32 as it stands in its page, 16-byte block b at place b ^ f(k) of it, f = k % 4 + 4 (k / 8 % 2) as far as
+  // the row's blocks allow; values: a page's 16 keys of a dim are two blocks, swapped for every second four dims.  Both so
+  // that eight lanes' fragment reads are in different banks.
+  constexpr int SLOTS = slots_of(NW), AHEAD_LOADS = RINGED ? (SLOTS - 1) * BLOCK_LOADS : 0;
+  static_assert(AHEAD_LOADS <= 63, "more loads in flight than the counter holds");
+  constexpr int NBLK = D / 8, TURN = NBLK % 8 == 0 ? 7 : 3, KL = RINGED ? D / 32 : 1;
+  uint32_t koff[KL];
+#pragma unroll
+  for (int j = 0; j < KL; ++j) {
+    const int i = j * 64 + lane, r = i / NBLK, place = i - r * NBLK;
+    koff[j] = r * D * 2 + (place ^ (((r & 3) | ((r >> 3) << 2)) & TURN)) * 16;
+  }
+  const uint32_t voff = (lane >> 1) * page * 2 + ((lane & 1) ^ ((lane >> 3) & 1)) * 16;
+  char* mine = da_lds + wave * SLOTS * 128 * D;
+  const uint32_t mine0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)mine;
+  auto issue = [&](int slot, const Places& p) {
+    const uint32_t to = mine0 + slot * 128 * D;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16* kp = k_cache + (((size_t)p.pg[t] * Hkv + kvh) * page + p.off[t]) * D;
+#pragma unroll
+      for (int j = 0; j < KL; ++j) mie_load_to_lds(kp, koff[j], to + t * 32 * D + j * 1024);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16* vp = v_cache + ((size_t)p.pg[t] * Hkv + kvh) * D * page + p.off[t];
+#pragma unroll
+      for (int j = 0; j < KL; ++j) mie_load_to_lds(vp + (size_t)32 * j * page, voff, to + 64 * D + t * 32 * D + j * 1024);
+    }
+  };
+  auto take = [&](KeyBlock& B, int slot) {
+    const char* at = mine + slot * 128 * D;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        B.a[t][ks].q = *reinterpret_cast<const uint4*>(at + (8 * (col >> 2) + 4 * t + (col & 3)) * D * 2 + ((4 * ks + kb) ^ (col & TURN)) * 16);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      B.va[dt].q = *reinterpret_cast<const uint4*>(at + 64 * D + (kb >> 1) * 32 * D + (dt * 16 + col) * 32 + ((kb & 1) ^ ((col >> 2) & 1)) * 16);
+  };
+  // which key of a block: a lane's j-th probability, and the row of score tile t that lane column c holds
+  auto key_at = [&](int blk, int j) { return RINGED ? blk + 8 * kb + j : blk + 16 * (j >> 2) + 4 * kb + (j & 3); };
+  auto row_key = [&](int blk, int t) { return RINGED ? blk + 8 * (col >> 2) + 4 * t + (col & 3) : blk + 16 * t + col; };
+  constexpr bool AHEAD = D <= 128;          // two blocks on their way; larger heads have no room for it
   KeyBlock b0, b1;
   const int pos_raw = positions[b];
   int begin0 = s * partition;               // the split's first key when there is no window
-  if (AHEAD && !CHUNK && window <= 0 && (!SIG || chunk <= 0)) load_block(b0, find(begin0 + BLOCK_KEYS * wave));
+  const bool early = AHEAD && !CHUNK && window <= 0 && (!SIG || chunk <= 0);
+  if (early) {
+    if constexpr (RINGED) issue(0, find(begin0 + BLOCK_KEYS * wave));
+    else load_block(b0, find(begin0 + BLOCK_KEYS * wave));
+  }
 
   const int pos = pos_raw;
   if (FROM_SUMS) {
@@ -207,7 +280,9 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   const int begin = (KEEP ? 0 : lo & ~(BLOCK_KEYS - 1)) + s * partition;
   const int end = begin + partition < last_x + 1 ? begin + partition : last_x + 1;
 
-  if (begin > last_x) {          // this split lies beyond the row's keys (uniform over the workgroup)
+  if (begin > last_x) {
+    if (RINGED) MIE_VMCNT(0);    // nothing of this wave may still be writing the LDS when it ends
+    // this split lies beyond the row's keys (uniform over the workgroup)
     if (num_splits > 1 && threadIdx.x < 16 && ht * 16 + (int)threadIdx.x < G)
       lse_part[((size_t)b * Hq + kvh * G + ht * 16 + threadIdx.x) * num_splits + s] = -INFINITY;
     return;
@@ -223,7 +298,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
       // what was loaded for the row's own key is whatever its slot held: the key and value come from the LDS
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        if (blk + 16 * t + col == pos) {
+        if (row_key(blk, t) == pos) {
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) {
             const int d0 = ks * 32 + kb * 8;
@@ -232,7 +307,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
         }
 #pragma unroll
       for (int wi = 0; wi < 4; ++wi) {                           // word wi of a value fragment: two keys
-        const int key = blk + 16 * (wi >> 1) + 4 * kb + 2 * (wi & 1);
+        const int key = key_at(blk, 2 * wi);
         const bool low = key == pos, high = key + 1 == pos;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
@@ -265,7 +340,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int key = blk + 16 * t + 4 * kb + i;
+          const int key = key_at(blk, 4 * t + i);
           ok[t * 4 + i] = key >= lo && key <= pos;
           float w;
           if (softcap > 0.f) {
@@ -302,7 +377,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int key = blk + 16 * t + 4 * kb + i;
+        const int key = key_at(blk, 4 * t + i);
         ok[t * 4 + i] = (key >= lo || (KEEP && key < keep)) && key <= pos;
         if constexpr (DB) {
           int n = pos - key;
@@ -350,7 +425,26 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
 
   constexpr int STEP = BLOCK_KEYS * NW;     // keys from one block of a wave to its next
   const int first = begin + BLOCK_KEYS * wave;
-  if (AHEAD) {
+  if constexpr (RINGED) {
+    const int count = first < end ? (end - first + STEP - 1) / STEP : 0;       // this wave's blocks: nothing beyond the split's own keys
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i)
+      if (i < count && !(i == 0 && early)) issue(i, find(key_of(first + i * STEP)));
+    Places next = find(key_of(first + SLOTS * STEP));
+    for (int it = 0; it < count; ++it) {
+      if (it + SLOTS <= count) MIE_VMCNT(AHEAD_LOADS);                  // block `it` has landed
+      else MIE_VMCNT(0);
+      asm volatile("" ::: "memory");
+      take(b0, it % SLOTS);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                       // read: the slot is free
+      if (it + SLOTS < count) {
+        issue(it % SLOTS, next);
+        next = find(key_of(first + (it + SLOTS + 1) * STEP));
+      }
+      compute(b0, key_of(first + it * STEP));
+    }
+    MIE_VMCNT(0);                           // (a wave without a block may have asked for one early)
+  } else if (AHEAD) {
     if (CHUNK || window > 0 || (SIG && chunk > 0)) load_block(b0, find(key_of(first)));  // with a window the split's start had to wait for the row's length
     const int part_end = begin + partition;   // nothing is asked for beyond the split's own keys
     Places next = find(key_of(first + STEP));
@@ -394,7 +488,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s_o[wave][col][dt * 16 + 4 * kb + i] = O[dt][i] * f;
+    for (int i = 0; i < 4; ++i) s_o[(wave * 16 + col) * (D + 1) + dt * 16 + 4 * kb + i] = O[dt][i] * f;
   if (wave == 0 && kb == 0) {
     s_M[col] = M;
     s_L[col] = L;
@@ -406,7 +500,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
     if (gg >= G) continue;
     float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) sum += s_o[w][hc][d];
+    for (int w = 0; w < NW; ++w) sum += s_o[(w * 16 + hc) * (D + 1) + d];
     const size_t hh = (size_t)b * Hq + kvh * G + gg;
     if (num_splits == 1) {
       // a sink (sink_log2 > -inf) is one more term in the denominator; with splits the merge kernel adds it
@@ -485,6 +579,13 @@ merge_splits_kernel(const float* __restrict__ o_part, const float* __restrict__ 
 
 MIE_EXPORT const char* attention_bf16_last_error() { return g_mie_error; }
 MIE_EXPORT int mie_attention_bf16_head_dim() { return D; }
+#define DA_LAUNCH(KERNEL, NW, STREAM, ...)                                                            \
+  do {                                                                                               \
+    auto kernel_ = KERNEL;                                                                           \
+    if (mie_allow_lds((const void*)kernel_, da_lds_bytes(NW), "decode_attention")) return -1;         \
+    hipLaunchKernelGGL(kernel_, grid, dim3(NW * 64), da_lds_bytes(NW), STREAM, __VA_ARGS__);         \
+  } while (0)
+
 MIE_EXPORT int mie_decode_block_keys() { return BLOCK_KEYS * NW_SPLIT; }
 
 // q: token b is row b (single-token rows lead the flattened batch).  partition: keys per split, a
@@ -516,55 +617,55 @@ static int decode_attention_launch(const void* q, long q_stride, const void* k_c
   // (the kernel writes the caches only when it is given the projection's sums)
   bf16* kc = (bf16*)const_cast<void*>(k_cache);
   bf16* vc = (bf16*)const_cast<void*>(v_cache);
-  const bool whole = num_splits == 1 && NW_WHOLE != NW_SPLIT && (long)rows * Hkv * head_tiles < NW_WHOLE_BELOW;
+  const bool whole = num_splits == 1 && NW_WHOLE != NW_SPLIT && (long)rows * Hkv * head_tiles <= whole_most();
   if (chunk > 0 && !sigmoid && (keep > 0 || dist_bias)) MIE_FAIL("decode_attention: chunks beside kept keys or a distance bias are not built");
   if (chunk > 0 && !sigmoid && whole)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, false, false, false, false, true>), grid, dim3(NW_WHOLE * 64), 0, stream,
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, false, false, true>), NW_WHOLE, stream,
                        (const bf16*)q, q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv,
                        head_tiles, page, scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else if (chunk > 0 && !sigmoid)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, false, false, false, false, true>), grid, dim3(NW_SPLIT * 64), 0, stream,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, false, false, true>), NW_SPLIT, stream,
                        (const bf16*)q, q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv,
                        head_tiles, page, scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else if (keep > 0 && whole)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, false, false, false, true>), grid, dim3(NW_WHOLE * 64), 0, stream, (const bf16*)q,
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, false, true>), NW_WHOLE, stream, (const bf16*)q,
                        q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, keep, head_sinks);
   else if (keep > 0)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, false, false, false, true>), grid, dim3(NW_SPLIT * 64), 0, stream, (const bf16*)q,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, false, true>), NW_SPLIT, stream, (const bf16*)q,
                        q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, keep, head_sinks);
   else if (dist_bias && whole)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, false, false, true>), grid, dim3(NW_WHOLE * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, true>), NW_WHOLE, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, dist_bias, dist_n, 0, head_sinks);
   else if (dist_bias)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, false, false, true>), grid, dim3(NW_SPLIT * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, true>), NW_SPLIT, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, dist_bias, dist_n, 0, head_sinks);
   else if (sigmoid && whole)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, false, true>), grid, dim3(NW_WHOLE * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, true>), NW_WHOLE, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, softcap, head_bias, (const float*)nullptr, 0, 0,
                        head_sinks);
   else if (sigmoid)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, false, true>), grid, dim3(NW_SPLIT * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, true>), NW_SPLIT, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, softcap, head_bias, (const float*)nullptr, 0, 0,
                        head_sinks);
   else if (whole)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, false>), grid, dim3(NW_WHOLE * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false>), NW_WHOLE, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, false>), grid, dim3(NW_SPLIT * 64), 0, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false>), NW_SPLIT, stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
@@ -632,13 +733,13 @@ MIE_EXPORT int mie_decode_attention_from_sums(const float* part, int splits, lon
   if (max_blocks <= 0 || Hkv > 65535) MIE_FAIL("decode_attention_from_sums: max_blocks %d, %d kv heads", max_blocks, Hkv);
   const ProjectionSums proj = {part, splits, (size_t)split_stride, ld, cos_t, sin_t, slots};
   dim3 grid(rows, Hkv, 1);
-  if ((long)rows * Hkv < NW_WHOLE_BELOW)
-    hipLaunchKernelGGL((decode_attention_kernel<NW_WHOLE, true>), grid, dim3(NW_WHOLE * 64), 0, stream, (const bf16*)nullptr, 0L,
+  if ((long)rows * Hkv <= whole_most())
+    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, true>), NW_WHOLE, stream, (const bf16*)nullptr, 0L,
                        (bf16*)k_cache, (bf16*)v_cache, (bf16*)out, (float*)nullptr, (float*)nullptr, block_tables, max_blocks,
                        positions, Hq, Hkv, 1, page, scale * 1.4426950408889634f, window, partition, 1, proj, -INFINITY, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, (const float*)nullptr);
   else
-    hipLaunchKernelGGL((decode_attention_kernel<NW_SPLIT, true>), grid, dim3(NW_SPLIT * 64), 0, stream, (const bf16*)nullptr, 0L,
+    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, true>), NW_SPLIT, stream, (const bf16*)nullptr, 0L,
                        (bf16*)k_cache, (bf16*)v_cache, (bf16*)out, (float*)nullptr, (float*)nullptr, block_tables, max_blocks,
                        positions, Hq, Hkv, 1, page, scale * 1.4426950408889634f, window, partition, 1, proj, -INFINITY, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, (const float*)nullptr);
