@@ -18,8 +18,8 @@
 //     so that the fragment reads spread over all banks.  What bounds it: the longest workgroup's chain of segments, 3.4 us of matrix
 //     instructions and 1.5 of exponentials each.  Read by every wave for itself (16 cache lines a quarter wave and load) it
 //     took 41 us for 512 tokens of 32 / 4 heads of 64, now 30; 1,024 tokens 113 and 64, of 32 / 8 heads of 128 197 and 114.
-//   single tokens: a wave a segment, joined by merge_f32_kernel.  What bounds it is the latency of a wave's own loads (a segment's K,
-//     then its V, all of one issued together).
+//   single tokens: a wave, or four, a segment, joined by merge_f32_kernel.  What bounds it is latency: the page table, K and V, matrix
+//     instructions, exponentials, one after the other.
 // The kernel of attention.hip, one wave a (token, head), reads every key once a head and token, a quarter of a cache line a load: 512
 // tokens of 32 / 4 heads of 64 642 us, 4 single tokens of 300 to 900 keys 200 for 11 + 5 here (MI355X).
 #include "launch.hpp"
@@ -435,6 +435,130 @@ single_f32_kernel(AttArgs a, float* __restrict__ out, float* __restrict__ o_part
   if (g == 0) *reinterpret_cast<float2*>(ml + 2 * at) = make_float2(m, l);
 }
 
+// The same by four waves, without another order of any sum: a wave makes the scores and exponentials of two of the eight tiles of 16
+// keys, all of them meet in the LDS, every wave adds them up as one wave would, and a wave takes every fourth tile of 16 dims of the
+// values.  4 tokens of 300 to 900 keys of 32 / 4 heads of 64 13.6 us with one wave and the kernel that joins, 10.0 with four; where the
+// segments are many, one wave each has less to exchange (64 tokens of 2,000 keys of 4 / 2 heads of 16: 15.2 and 20.9; 16 of 900
+// of 32 / 8 heads of 128: 34.6 and 37.4), so four take up to AF_FEW segments.
+constexpr long AF_FEW = 1024;
+constexpr int AF_SINGLE_WAVES = 4;
+template <int DT>
+__global__ void __launch_bounds__(AF_SINGLE_WAVES * 64)
+single_few_f32_kernel(AttArgs a, float* __restrict__ out, float* __restrict__ o_part, float* __restrict__ ml,
+                  const int* __restrict__ token_row, const int* __restrict__ positions, int splits) {
+  constexpr int D = DT * 16, OWN = AF_TILES / AF_SINGLE_WAVES, CT = (DT + AF_SINGLE_WAVES - 1) / AF_SINGLE_WAVES;
+  __shared__ __align__(16) float weights[AF_TILES * 64 * 4];
+  __shared__ float s_top[AF_SINGLE_WAVES][16];
+  const int t = blockIdx.z, rep = a.Hq / a.Hkv, head_tiles = (rep + 15) / 16;
+  const int kvh = blockIdx.y / head_tiles, h0 = (blockIdx.y - kvh * head_tiles) * 16;
+  const int p = positions[t];
+  const int first = a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0;
+  const int seg = first / AF_SEG + blockIdx.x;
+  if (seg * AF_SEG > p) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const bool live = h0 + r16 < rep;
+  const int h = kvh * rep + h0 + r16, base = seg * AF_SEG;
+  const int* bt = a.block_tables + (size_t)token_row[t] * a.max_blocks;
+  f32x4 qf[DT];
+  load_queries<DT>(a, live ? t : -1, h, qf);
+  size_t at[AF_TILES];                        // of the page stretch a tile of 16 keys lies in; a tile nobody sees stands for its neighbour
+  const int t0 = first > base ? (first - base) >> 4 : 0, t1 = p - base >= AF_SEG ? AF_TILES : ((p - base) >> 4) + 1;
+#pragma unroll
+  for (int u = 0; u < AF_TILES; ++u) {
+    const int tt = u < t0 ? t0 : u >= t1 ? t1 - 1 : u;
+    at[u] = ((size_t)bt[(base + tt * 16) / a.page] * a.Hkv + kvh) * a.page * D;
+  }
+  f32x4 kf[OWN][DT], vf[AF_TILES][CT], s[OWN];
+#pragma unroll
+  for (int u = 0; u < OWN; ++u) {
+    const int tile = wave * OWN + u;
+    size_t from = at[0];
+#pragma unroll
+    for (int k = 1; k < AF_TILES; ++k) from = tile == k ? at[k] : from;
+    const float* kp = a.k_cache + from + (size_t)((base + tile * 16) % a.page + r16) * D + 4 * g;
+#pragma unroll
+    for (int c = 0; c < DT; ++c) kf[u][c] = *reinterpret_cast<const f32x4*>(kp + 16 * c);
+  }
+#pragma unroll
+  for (int u = 0; u < AF_TILES; ++u) {
+    const float* vp = a.v_cache + at[u] + (size_t)r16 * a.page + (base + u * 16) % a.page + 4 * g;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const int c = wave + j * AF_SINGLE_WAVES;
+      vf[u][j] = *reinterpret_cast<const f32x4*>(vp + (size_t)(16 * (c < DT ? c : 0)) * a.page);
+    }
+  }
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < OWN; ++u) s[u] = none;
+#pragma unroll
+  for (int c = 0; c < DT; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][c][j], qf[c][j], s[u], 0, 0, 0);
+  const int pos = live ? p : -1;
+  float top = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < OWN; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = base + (wave * OWN + u) * 16 + 4 * g + i;
+      s[u][i] = key <= pos && key >= first ? __fmul_rn(s[u][i], a.scale) : -INFINITY;
+      top = fmaxf(top, s[u][i]);
+    }
+  top = fmaxf(top, __shfl_xor(top, 16, 64));
+  top = fmaxf(top, __shfl_xor(top, 32, 64));
+  if (g == 0) s_top[wave][r16] = top;
+  __syncthreads();
+  float m = s_top[0][r16];
+#pragma unroll
+  for (int w = 1; w < AF_SINGLE_WAVES; ++w) m = fmaxf(m, s_top[w][r16]);
+  const float sub = m == -INFINITY ? 0.f : m;
+#pragma unroll
+  for (int u = 0; u < OWN; ++u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[u][i] = expf(s[u][i] - sub);
+    *reinterpret_cast<f32x4*>(weights + ((wave * OWN + u) * 64 + lane) * 4) = s[u];
+  }
+  __syncthreads();
+  f32x4 o[CT], e[AF_TILES];
+#pragma unroll
+  for (int u = 0; u < AF_TILES; ++u) e[u] = *reinterpret_cast<const f32x4*>(weights + (u * 64 + lane) * 4);
+  float l = 0.f;
+#pragma unroll
+  for (int u = 0; u < AF_TILES; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l += e[u][i];
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+#pragma unroll
+  for (int j = 0; j < CT; ++j) o[j] = none;
+#pragma unroll
+  for (int u = 0; u < AF_TILES; ++u) {
+    const int key = base + u * 16;
+    if (key < first || key + 15 > p) {
+#pragma unroll
+      for (int j = 0; j < CT; ++j) clean_values(vf[u][j], key + 4 * g, first, p, first, p);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][j][i], e[u][i], o[j], 0, 0, 0);
+  }
+  if (!live) return;
+  const size_t part = ((size_t)t * a.Hq + h) * splits + blockIdx.x;
+  const float inv = 1.0f / l;                 // one segment, joined with nothing: O 0 + o 1, L 0 + l 1
+#pragma unroll
+  for (int j = 0; j < CT; ++j) {
+    const int c = wave + j * AF_SINGLE_WAVES;
+    if (c >= DT) break;
+    if (splits == 1) *reinterpret_cast<f32x4*>(out + ((size_t)t * a.Hq + h) * D + 16 * c + 4 * g) = o[j] * inv;
+    else *reinterpret_cast<f32x4*>(o_part + part * D + 16 * c + 4 * g) = o[j];
+  }
+  if (splits > 1 && wave == 0 && g == 0) *reinterpret_cast<float2*>(ml + 2 * part) = make_float2(m, l);
+}
+
 // Joins a token's segments in order: one wave a (token, head), lane d and d + 64 of the head.
 __global__ void __launch_bounds__(64)
 merge_f32_kernel(const float* __restrict__ o_part, const float* __restrict__ ml, float* __restrict__ out, const int* __restrict__ positions,
@@ -510,7 +634,10 @@ MIE_EXPORT int mie_attention_f32_single(const float* q, long q_stride, const flo
   const int rep = Hq / Hkv, head_tiles = (rep + 15) / 16;
   if (Hkv * head_tiles > 65535) MIE_FAIL("attention_f32: %d kv heads are beyond the grid", Hkv);
   const dim3 grid(splits, Hkv * head_tiles, tokens);
-#define AF_SINGLE(DT) hipLaunchKernelGGL(single_f32_kernel<DT>, grid, dim3(64), 0, s, a, out, o_part, ml, token_row, positions, splits)
+  const bool few = (long)splits * Hkv * head_tiles * tokens <= AF_FEW;
+#define AF_SINGLE(DT)                                                                                                                      \
+  if (few) hipLaunchKernelGGL(single_few_f32_kernel<DT>, grid, dim3(AF_SINGLE_WAVES * 64), 0, s, a, out, o_part, ml, token_row, positions, splits); \
+  else hipLaunchKernelGGL(single_f32_kernel<DT>, grid, dim3(64), 0, s, a, out, o_part, ml, token_row, positions, splits)
   AF_BY_HEAD(D, AF_SINGLE)
   MIE_CHECK_LAUNCH("attention_f32 single");
   if (splits > 1) {

@@ -1478,6 +1478,29 @@ def test_attention_float32_matrix_unit(ops, geom, window):
         assert calls == ["mie_attention_f32_single"] and torch.equal(out, whole)
 
 
+@pytest.mark.parametrize("window", [None, 1, 130])
+@pytest.mark.parametrize("geom", [(32, 4, 64, 16), (3, 1, 32, 16), (5, 5, 48, 32), (40, 2, 16, 16), (16, 1, 128, 16), (10, 2, 112, 48), (6, 2, 80, 16)])
+def test_attention_float32_few_single_tokens(ops, geom, window):
+    """Few single tokens (four waves a segment) beside the same ones among many (one wave): the same bits, for every head size's
+    number of value tiles a wave, segments that are begun, full and single keys."""
+    Hq, Hkv, D, page = geom
+    o, ctx = ops[torch.float32], [1, 127, 128, 129, 300]
+    many = ctx + [500] * 1100
+    q, kc, vc, group, step = paged_setup(many, [1] * len(many), Hq, Hkv, D, page, torch.float32, seed=D)
+    splits = -(-500 // 128)
+    heads = Hkv * -(-(Hq // Hkv) // 16)
+    assert splits * heads * len(ctx) <= 1024 < heads * len(many)
+    whole = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 1 / math.sqrt(D), window)
+    n = len(ctx)
+    few = SimpleNamespace(token_row=step.token_row[:n], positions=step.positions[:n], num_rows=n, max_context=500, num_tokens=n,
+                          num_decode_rows=n, max_row_tokens=1, row_start=None, row_position=None)
+    out = o.paged_attention(q[:n], Hq, Hkv, D, kc, vc, SimpleNamespace(block_tables=group.block_tables[:n].contiguous(), max_blocks=group.max_blocks),
+                            few, 1 / math.sqrt(D), window)
+    assert torch.equal(out, whole[:n])
+    expect = ref.ref_paged_attention(q[:n], Hq, Hkv, D, kc, vc, group.block_tables[:n], few.token_row, few.positions, 1 / math.sqrt(D), window, torch.float64)
+    torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
+
+
 def test_attention_float32_of_a_step_that_does_not_describe_its_rows(ops):
     """What the float32 attention reads of a step beyond its tokens is only there to choose a faster kernel: without the longest
     row's length or the largest context, or with row arrays of another type, the result is the same."""
