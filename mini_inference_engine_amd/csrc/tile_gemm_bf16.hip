@@ -9,9 +9,9 @@
 // (in halves of 64 bytes large tiles were up to a third slower: the L2s are asked twice for every line).  Row r's block b of
 // 16 bytes stands at 8 r + (b ^ r % 8), so that the fragment reads (lane 16 g + r: row r, block g) spread over all banks.
 //
-// What bounds it: the traffic from the L2s into the workgroups, 8 to 13 TB/s with every tile, ring and number of workgroups
-// tried (the library's kernels move 11); reading the next fragments while one set is multiplied, across the barrier too,
-// changed nothing.  So what counts is bytes a workgroup brings in, and that every compute unit has one: TILE_STAGE_US, the
+// What bounds it: what a compute unit takes in, 58 bytes a nanosecond at most (a kernel that only loads, whatever the access pattern
+// or who shares the lines), 36 to 48 with these tiles, rings and numbers of workgroups (the library's kernels move 43); reading the
+// next fragments while one set is multiplied, across the barrier too, changed nothing.  So what counts is bytes a workgroup brings in, and that every compute unit has one: TILE_STAGE_US, the
 // time of a stage of each tile, times the rounds of its grid picks the tile.
 #include "launch.hpp"
 
@@ -144,6 +144,111 @@ tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   }
 }
 
+// 256 x 384 outputs a workgroup of eight waves of 64 x 192, two stages of 64 k in all of the LDS: 80 KB a stage for the matrix
+// instructions of six 128 x 128 tiles, which bring in 192 KB, so the matrix cores come close to being the bound.  What it took (2,048 rows of
+// [11264, 2048], 240 tiles, MI355X; 256 x 192 tiles take 93.8 us): waves of 128 x 96 spill registers, 106 us; addresses by lane
+// arithmetic, too, 97; scalar addresses, all loads of the next stage at once 91, one between every four matrix instructions 85 (a load
+// that finds the queue full stops its wave), the second half's first fragments asked for in the first half 81.2.
+// SWIGLU only: a wave's 192 weight rows are 96 gate rows, then the up rows of the same columns.  N is a multiple of 8.
+constexpr int TW_A = 12, TW_B = 4, TW_WR = 4, TW_WC = 2;                    // 16-row tiles of W and of x a wave; waves
+constexpr int TW_BM = TW_WR * TW_B * 16, TW_BN = TW_WC * TW_A * 16;
+__global__ void __launch_bounds__(512)
+tile_wide_kernel(const bf16* __restrict__ X, uint32_t ldx, const bf16* __restrict__ W, uint32_t ldw, bf16* __restrict__ out, long ldo,
+                 int M, int N, int nst, int mt) {
+  constexpr int XL = TW_BM / 8, LOADS = XL + TW_BN / 8, L = LOADS / 8, STAGE = LOADS * 1024, HALF = TW_A * 8;
+  static_assert(LOADS % 8 == 0, "every wave brings in as many");
+  extern __shared__ __align__(1024) char tg_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kb = lane >> 4;
+  int id = blockIdx.x;
+  {
+    const int total = gridDim.x, q = total >> 3, r = total & 7, x = id & 7, y = id >> 3;
+    id = x * q + (x < r ? x : r) + y;
+  }
+  const int m0 = id % mt * TW_BM, n0 = id / mt * (TW_BN / 2);
+  const int lrow = lane >> 3;
+  const uint32_t lblk = ((lane & 7) ^ lrow) * 16;
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)tg_lds;
+  // a load of 8 rows from a scalar address; of x's last 8 some may not exist, and those read the last one that does
+  const int last_x = (M - 1) & ~7;
+  const uint32_t xo = lrow * ldx * 2 + lblk, wo = lrow * ldw * 2 + lblk, xo_last = (lrow < M - last_x ? lrow : M - 1 - last_x) * ldx * 2 + lblk;
+  auto load = [&](int s, int j) {              // the wave's j-th load of stage s
+    const int f = wave * L + j;
+    const uint32_t to = lds0 + (s & 1) * STAGE + f * 1024;
+    if (f < XL) {
+      const int g = m0 + f * 8, from = g < last_x ? g : last_x;
+      mie_load_to_lds(reinterpret_cast<const char*>(X) + (size_t)from * ldx * 2 + (size_t)s * 128, g + 8 <= M ? xo : xo_last, to);
+    } else {
+      // 8 rows of one wave's gate or up rows
+      const int r = (f - XL) * 8, w = r / (2 * HALF), at = r - w * 2 * HALF, up = at >= HALF;
+      const int g = n0 + w * HALF + at - up * HALF, from = (g < N ? g : N - 8) + (up ? N : 0);
+      mie_load_to_lds(reinterpret_cast<const char*>(W) + (size_t)from * ldw * 2 + (size_t)s * 128, wo, to);
+    }
+  };
+  f32x4 acc[TW_A][TW_B];
+#pragma unroll
+  for (int a = 0; a < TW_A; ++a)
+#pragma unroll
+    for (int b = 0; b < TW_B; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wr = wave % TW_WR, wc = wave / TW_WR;
+  const char* xl = tg_lds + (wr * TW_B * 16 + col) * 128;
+  const char* wl = tg_lds + (TW_BM + wc * TW_A * 16 + col) * 128;
+
+#pragma unroll
+  for (int j = 0; j < L; ++j) load(0, j);
+  for (int it = 0; it < nst; ++it) {
+    MIE_VMCNT(0);                              // this wave's loads of stage `it` have landed
+    __builtin_amdgcn_s_barrier();              // and everybody else's; everybody is done with stage it - 1
+    asm volatile("" ::: "memory");
+    const bool more = it + 1 < nst;
+    const int stage = (it & 1) * STAGE;
+    int next = 0;
+    bf16x8 xf[2][TW_B], wf[2];
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const int blk = stage + ((4 * kc + kb) ^ (col & 7)) * 16;
+      if (kc == 0) {
+#pragma unroll
+        for (int b = 0; b < TW_B; ++b) xf[0][b] = *reinterpret_cast<const bf16x8*>(xl + blk + b * 2048);
+        wf[0] = *reinterpret_cast<const bf16x8*>(wl + blk);
+      }
+      const int blk1 = stage + ((4 + kb) ^ (col & 7)) * 16;
+#pragma unroll
+      for (int a = 0; a < TW_A; ++a) {
+        if (a + 1 < TW_A) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk + (a + 1) * 2048);
+        else if (kc == 0) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk1);
+        if (kc == 0 && a + TW_B >= TW_A) xf[1][a + TW_B - TW_A] = *reinterpret_cast<const bf16x8*>(xl + blk1 + (a + TW_B - TW_A) * 2048);
+        if ((kc * TW_A + a) >= 1 && next < L) {
+          if (more) load(it + 1, next);
+          ++next;
+        }
+#pragma unroll
+        for (int b = 0; b < TW_B; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a & 1], xf[kc][b], acc[a][b], 0, 0, 0);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // this wave has read the stage before the next barrier
+  }
+
+  // acc[a][b][i] of lane (col, kb): weight row 16 a + 4 kb + i of the wave's 96, x row 16 b + col
+#pragma unroll
+  for (int b = 0; b < TW_B; ++b) {
+    const int m = m0 + (wr * TW_B + b) * 16 + col;
+    if (m >= M) continue;
+#pragma unroll
+    for (int a = 0; a < TW_A / 2; ++a) {
+      const int n = n0 + wc * HALF + a * 16 + 4 * kb;
+      if (n >= N) continue;
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float g = acc[a][b][i];
+        o[i] = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * acc[a + TW_A / 2][b][i];
+      }
+      *reinterpret_cast<uint2*>(out + (size_t)m * ldo + n) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+    }
+  }
+}
+
 MIE_EXPORT const char* tile_gemm_bf16_last_error() { return g_mie_error; }
 
 template <int WR, int WC, int STAGES, int EPI>
@@ -161,6 +266,17 @@ static int launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, l
   return 0;
 }
 
+static int launch_wide(const bf16* X, long ldx, const bf16* W, long ldw, bf16* out, long ldo, int M, int N, int K, hipStream_t s) {
+  constexpr int lds = 2 * (TW_BM + TW_BN) * 128;
+  static_assert(lds <= 160 * 1024, "LDS");
+  if (mie_allow_lds((const void*)tile_wide_kernel, lds, "tile_gemm")) return -1;
+  const int mt = (M + TW_BM - 1) / TW_BM, nt = (N + TW_BN / 2 - 1) / (TW_BN / 2);
+  if ((long)mt * nt > 0x7FFFFFFF) MIE_FAIL("tile_gemm: %d x %d tiles are beyond the grid", mt, nt);
+  hipLaunchKernelGGL(tile_wide_kernel, dim3(mt * nt), dim3(512), lds, s, X, (uint32_t)ldx, W, (uint32_t)ldw, out, ldo, M, N, K / 64, mt);
+  MIE_CHECK_LAUNCH("tile_gemm");
+  return 0;
+}
+
 static int check_operands(const void* X, long ldx, const void* W, long ldw, const void* out, int M, long w_rows, int N, int K) {
   if (K <= 0 || (K & 63) || (N & 7)) MIE_FAIL("tile_gemm: K = %d (multiples of 64), N = %d (of 8)", K, N);
   if (ldx < K || ldw < K || (ldx & 7) || (ldw & 7)) MIE_FAIL("tile_gemm: leading dims %ld, %ld for K %d", ldx, ldw, K);
@@ -172,13 +288,13 @@ static int check_operands(const void* X, long ldx, const void* W, long ldw, cons
 
 // Time of a stage (64 k) of a grid that gives every compute unit one workgroup, us: measured at 160 to 2,048 rows of
 // [11264, 2048] (MI355X).
-constexpr struct { int bm, bn; float us; } TILE_STAGE_US[5] = {
-  {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}};
+constexpr struct { int bm, bn; float us; } TILE_STAGE_US[6] = {
+  {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f}};
 
 static int best_tile(int M, long cols, float& us) {
   int best = 0;
   us = 1e30f;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < 6; ++i) {
     const long tiles = (long)((M + TILE_STAGE_US[i].bm - 1) / TILE_STAGE_US[i].bm) * ((cols + TILE_STAGE_US[i].bn - 1) / TILE_STAGE_US[i].bn);
     const long rounds = (tiles + mie_compute_units() - 1) / mie_compute_units();
     if (rounds * TILE_STAGE_US[i].us < us) {
@@ -208,7 +324,8 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
     case 1: return launch<3, 2, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 2: return launch<4, 2, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 3: return launch<4, 3, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
-    default: return launch<4, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 4: return launch<4, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    default: return launch_wide(x, ldx, w, ldw, (bf16*)out, ldo, M, N, K, s);
   }
 }
 

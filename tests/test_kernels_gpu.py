@@ -473,6 +473,26 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
+@pytest.mark.parametrize("case", [(2047, 192, 5640), (1281, 64, 7496), (1793, 128, 6144), (2048, 2048, 5632)])
+def test_wide_tile_product_swiglu(engine_ops, case):
+    """Gate and up on tiles of 256 x 384 (taken where they make one round of what other tiles need two for): edges in rows and
+    columns, one stage and many; against 64 bits rounded once."""
+    from mini_inference_engine_amd.kernels import library
+    o, (M, K, inter) = engine_ops, case
+    torch.manual_seed(K + inter)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    lib = o.lib("tile_gemm_bf16")
+    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 235 * (K // 64)) <= 1, "the case must take the tile it is for"
+    out = torch.full((M, inter + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    library.check(lib, lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K,
+                                                torch.cuda.current_stream().cuda_stream))
+    gu = x.double() @ w.double().T
+    expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
+    assert bool(((out[:, :inter].double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
+    assert bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
+
+
 @pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("case", [(1, 1024, 4, 4), (8, 2048, 2048, 4), (9, 1028, 1000, 4), (16, 5632, 516, 4), (17, 2052, 36, 8), (20, 1024, 4100, 8),
                                   (100, 360, 2048, 4), (40, 1536, 8192, 4), (300, 200, 132, 8)])
