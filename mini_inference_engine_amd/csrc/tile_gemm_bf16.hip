@@ -144,19 +144,23 @@ tile_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   }
 }
 
-// 256 x 384 outputs a workgroup of eight waves of 64 x 192, two stages of 64 k in all of the LDS: 80 KB a stage for the matrix
-// instructions of six 128 x 128 tiles, which bring in 192 KB, so the matrix cores come close to being the bound.  What it took (2,048 rows of
-// [11264, 2048], 240 tiles, MI355X; 256 x 192 tiles take 93.8 us): waves of 128 x 96 spill registers, 106 us; addresses by lane
-// arithmetic, too, 97; scalar addresses, all loads of the next stage at once 91, one between every four matrix instructions 85 (a load
-// that finds the queue full stops its wave), the second half's first fragments asked for in the first half 81.2.
-// SWIGLU only: a wave's 192 weight rows are 96 gate rows, then the up rows of the same columns.  N is a multiple of 8.
-constexpr int TW_A = 12, TW_B = 4, TW_WR = 4, TW_WC = 2;                    // 16-row tiles of W and of x a wave; waves
-constexpr int TW_BM = TW_WR * TW_B * 16, TW_BN = TW_WC * TW_A * 16;
+// The same by eight waves of TB x TA tiles of 16 x 16, four waves over x and two over W: wherever it was measured faster.  Three things
+// beside the shape: loads go out from scalar addresses (no lane arithmetic), one between every TB matrix instructions (a load that finds
+// the queue full stops its wave; all at once behind the barrier they stop every wave), and the second half's first fragments
+// are asked for in the first half.  What each gave at 256 x 384 (2,048 rows of [11264, 2048], 240 tiles, MI355X; 256 x 192 tiles of the kernel
+// above take 93.8 us): waves of 128 x 96, which spill registers, 106; addresses by lane arithmetic 97; scalar addresses, all loads at
+// once 91; between the matrix instructions 85; the fragments 81.  Tiles of 256 x 384 bring in 80 KB a stage for the matrix instructions of
+// six 128 x 128 tiles, which bring in 192 KB.
+// SWIGLU: a wave's weight rows are TA / 2 tiles of gate rows, then the up rows of the same columns.  N is a multiple of 8.
+template <int TA, int TB, int STAGES, int EPI>
 __global__ void __launch_bounds__(512)
-tile_wide_kernel(const bf16* __restrict__ X, uint32_t ldx, const bf16* __restrict__ W, uint32_t ldw, bf16* __restrict__ out, long ldo,
-                 int M, int N, int nst, int mt) {
-  constexpr int XL = TW_BM / 8, LOADS = XL + TW_BN / 8, L = LOADS / 8, STAGE = LOADS * 1024, HALF = TW_A * 8;
+tile_spread_kernel(const bf16* __restrict__ X, uint32_t ldx, const bf16* __restrict__ W, uint32_t ldw, void* __restrict__ outv, long ldo,
+                   int M, int N, int stages_all, int stages_unit, long unit_stride, int mt, int nt) {
+  constexpr int WR = 4, WC = 2, BM = WR * TB * 16, BN = WC * TA * 16, XL = BM / 8, LOADS = XL + BN / 8, L = LOADS / 8;
+  constexpr int STAGE = LOADS * 1024, HALF = TA * 8, COLS = EPI == TG_SWIGLU ? BN / 2 : BN;
   static_assert(LOADS % 8 == 0, "every wave brings in as many");
+  static_assert(L < 2 * TA, "a load between every TB matrix instructions, from the second on");
+  static_assert((STAGES - 2) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(1024) char tg_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kb = lane >> 4;
@@ -165,7 +169,9 @@ tile_wide_kernel(const bf16* __restrict__ X, uint32_t ldx, const bf16* __restric
     const int total = gridDim.x, q = total >> 3, r = total & 7, x = id & 7, y = id >> 3;
     id = x * q + (x < r ? x : r) + y;
   }
-  const int m0 = id % mt * TW_BM, n0 = id / mt * (TW_BN / 2);
+  const int tm = id % mt, rest = id / mt, tn = rest % nt, unit = rest / nt;
+  const int m0 = tm * BM, n0 = tn * COLS;
+  const int st0 = unit * stages_unit, nst = st0 + stages_unit < stages_all ? stages_unit : stages_all - st0;
   const int lrow = lane >> 3;
   const uint32_t lblk = ((lane & 7) ^ lrow) * 16;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)tg_lds;
@@ -174,77 +180,93 @@ tile_wide_kernel(const bf16* __restrict__ X, uint32_t ldx, const bf16* __restric
   const uint32_t xo = lrow * ldx * 2 + lblk, wo = lrow * ldw * 2 + lblk, xo_last = (lrow < M - last_x ? lrow : M - 1 - last_x) * ldx * 2 + lblk;
   auto load = [&](int s, int j) {              // the wave's j-th load of stage s
     const int f = wave * L + j;
-    const uint32_t to = lds0 + (s & 1) * STAGE + f * 1024;
+    const uint32_t to = lds0 + (s % STAGES) * STAGE + f * 1024;
+    const size_t k = (size_t)(st0 + s) * 128;
     if (f < XL) {
       const int g = m0 + f * 8, from = g < last_x ? g : last_x;
-      mie_load_to_lds(reinterpret_cast<const char*>(X) + (size_t)from * ldx * 2 + (size_t)s * 128, g + 8 <= M ? xo : xo_last, to);
+      mie_load_to_lds(reinterpret_cast<const char*>(X) + (size_t)from * ldx * 2 + k, g + 8 <= M ? xo : xo_last, to);
     } else {
-      // 8 rows of one wave's gate or up rows
-      const int r = (f - XL) * 8, w = r / (2 * HALF), at = r - w * 2 * HALF, up = at >= HALF;
-      const int g = n0 + w * HALF + at - up * HALF, from = (g < N ? g : N - 8) + (up ? N : 0);
-      mie_load_to_lds(reinterpret_cast<const char*>(W) + (size_t)from * ldw * 2 + (size_t)s * 128, wo, to);
+      const int r = (f - XL) * 8;
+      int g = n0 + r, behind = 0;
+      if (EPI == TG_SWIGLU) {                  // 8 rows of one wave's gate or up rows
+        const int w = r / (2 * HALF), at = r - w * 2 * HALF, up = at >= HALF;
+        g = n0 + w * HALF + at - up * HALF;
+        behind = up ? N : 0;
+      }
+      mie_load_to_lds(reinterpret_cast<const char*>(W) + (size_t)((g < N ? g : N - 8) + behind) * ldw * 2 + k, wo, to);
     }
   };
-  f32x4 acc[TW_A][TW_B];
+  f32x4 acc[TA][TB];
 #pragma unroll
-  for (int a = 0; a < TW_A; ++a)
+  for (int a = 0; a < TA; ++a)
 #pragma unroll
-    for (int b = 0; b < TW_B; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int wr = wave % TW_WR, wc = wave / TW_WR;
-  const char* xl = tg_lds + (wr * TW_B * 16 + col) * 128;
-  const char* wl = tg_lds + (TW_BM + wc * TW_A * 16 + col) * 128;
+    for (int b = 0; b < TB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wr = wave % WR, wc = wave / WR;
+  const char* xl = tg_lds + (wr * TB * 16 + col) * 128;
+  const char* wl = tg_lds + (BM + wc * TA * 16 + col) * 128;
 
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < nst)
 #pragma unroll
-  for (int j = 0; j < L; ++j) load(0, j);
+      for (int j = 0; j < L; ++j) load(t, j);
   for (int it = 0; it < nst; ++it) {
-    MIE_VMCNT(0);                              // this wave's loads of stage `it` have landed
-    __builtin_amdgcn_s_barrier();              // and everybody else's; everybody is done with stage it - 1
+    if (it + STAGES - 1 <= nst) MIE_VMCNT((STAGES - 2) * L);      // this wave's loads of stage `it` have landed
+    else MIE_VMCNT(0);
+    __builtin_amdgcn_s_barrier();                                // and everybody else's; everybody is done with stage it - 1
     asm volatile("" ::: "memory");
-    const bool more = it + 1 < nst;
-    const int stage = (it & 1) * STAGE;
+    const bool more = it + STAGES - 1 < nst;
+    const int stage = (it % STAGES) * STAGE, blk1 = stage + ((4 + kb) ^ (col & 7)) * 16;
     int next = 0;
-    bf16x8 xf[2][TW_B], wf[2];
+    bf16x8 xf[2][TB], wf[2];
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
       const int blk = stage + ((4 * kc + kb) ^ (col & 7)) * 16;
       if (kc == 0) {
 #pragma unroll
-        for (int b = 0; b < TW_B; ++b) xf[0][b] = *reinterpret_cast<const bf16x8*>(xl + blk + b * 2048);
+        for (int b = 0; b < TB; ++b) xf[0][b] = *reinterpret_cast<const bf16x8*>(xl + blk + b * 2048);
         wf[0] = *reinterpret_cast<const bf16x8*>(wl + blk);
       }
-      const int blk1 = stage + ((4 + kb) ^ (col & 7)) * 16;
 #pragma unroll
-      for (int a = 0; a < TW_A; ++a) {
-        if (a + 1 < TW_A) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk + (a + 1) * 2048);
+      for (int a = 0; a < TA; ++a) {
+        if (a + 1 < TA) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk + (a + 1) * 2048);
         else if (kc == 0) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk1);
-        if (kc == 0 && a + TW_B >= TW_A) xf[1][a + TW_B - TW_A] = *reinterpret_cast<const bf16x8*>(xl + blk1 + (a + TW_B - TW_A) * 2048);
-        if ((kc * TW_A + a) >= 1 && next < L) {
-          if (more) load(it + 1, next);
+        if (kc == 0 && a + TB >= TA) xf[1][a + TB - TA] = *reinterpret_cast<const bf16x8*>(xl + blk1 + (a + TB - TA) * 2048);
+        if (kc * TA + a >= 1 && next < L) {
+          if (more) load(it + STAGES - 1, next);
           ++next;
         }
 #pragma unroll
-        for (int b = 0; b < TW_B; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a & 1], xf[kc][b], acc[a][b], 0, 0, 0);
+        for (int b = 0; b < TB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a & 1], xf[kc][b], acc[a][b], 0, 0, 0);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // this wave has read the stage before the next barrier
   }
 
-  // acc[a][b][i] of lane (col, kb): weight row 16 a + 4 kb + i of the wave's 96, x row 16 b + col
+  // acc[a][b][i] of lane (col, kb): weight row 16 a + 4 kb + i of the wave's, x row 16 b + col
 #pragma unroll
-  for (int b = 0; b < TW_B; ++b) {
-    const int m = m0 + (wr * TW_B + b) * 16 + col;
+  for (int b = 0; b < TB; ++b) {
+    const int m = m0 + (wr * TB + b) * 16 + col;
     if (m >= M) continue;
+    if (EPI == TG_SWIGLU) {
 #pragma unroll
-    for (int a = 0; a < TW_A / 2; ++a) {
-      const int n = n0 + wc * HALF + a * 16 + 4 * kb;
-      if (n >= N) continue;
-      float o[4];
+      for (int a = 0; a < TA / 2; ++a) {
+        const int n = n0 + wc * HALF + a * 16 + 4 * kb;
+        if (n >= N) continue;
+        float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float g = acc[a][b][i];
-        o[i] = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * acc[a + TW_A / 2][b][i];
+        for (int i = 0; i < 4; ++i) {
+          const float g = acc[a][b][i];
+          o[i] = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * acc[a + TA / 2][b][i];
+        }
+        *reinterpret_cast<uint2*>((bf16*)outv + (size_t)m * ldo + n) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
       }
-      *reinterpret_cast<uint2*>(out + (size_t)m * ldo + n) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+      continue;
+    }
+#pragma unroll
+    for (int a = 0; a < TA; ++a) {
+      const int n = n0 + (wc * TA + a) * 16 + 4 * kb;
+      if (n >= N) continue;
+      *reinterpret_cast<f32x4*>((float*)outv + unit * unit_stride + (size_t)m * ldo + n) = acc[a][b];
     }
   }
 }
@@ -266,13 +288,16 @@ static int launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, l
   return 0;
 }
 
-static int launch_wide(const bf16* X, long ldx, const bf16* W, long ldw, bf16* out, long ldo, int M, int N, int K, hipStream_t s) {
-  constexpr int lds = 2 * (TW_BM + TW_BN) * 128;
+template <int TA, int TB, int STAGES, int EPI>
+static int launch_spread(const bf16* X, long ldx, const bf16* W, long ldw, void* out, long ldo, int M, int N, int K, int units, hipStream_t s) {
+  constexpr int BM = TB * 64, BN = TA * 32, cols = EPI == TG_SWIGLU ? BN / 2 : BN, lds = STAGES * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "LDS");
-  if (mie_allow_lds((const void*)tile_wide_kernel, lds, "tile_gemm")) return -1;
-  const int mt = (M + TW_BM - 1) / TW_BM, nt = (N + TW_BN / 2 - 1) / (TW_BN / 2);
-  if ((long)mt * nt > 0x7FFFFFFF) MIE_FAIL("tile_gemm: %d x %d tiles are beyond the grid", mt, nt);
-  hipLaunchKernelGGL(tile_wide_kernel, dim3(mt * nt), dim3(512), lds, s, X, (uint32_t)ldx, W, (uint32_t)ldw, out, ldo, M, N, K / 64, mt);
+  auto kernel = tile_spread_kernel<TA, TB, STAGES, EPI>;
+  if (mie_allow_lds((const void*)kernel, lds, "tile_gemm")) return -1;
+  const int mt = (M + BM - 1) / BM, nt = (N + cols - 1) / cols, stages = K / 64, per = (stages + units - 1) / units;
+  if ((long)mt * nt * units > 0x7FFFFFFF) MIE_FAIL("tile_gemm: %d x %d tiles are beyond the grid", mt, nt);
+  hipLaunchKernelGGL(kernel, dim3(mt * nt * units), dim3(512), lds, s, X, (uint32_t)ldx, W, (uint32_t)ldw, out, ldo, M, N, stages, per,
+                     (long)M * N, mt, nt);
   MIE_CHECK_LAUNCH("tile_gemm");
   return 0;
 }
@@ -286,15 +311,18 @@ static int check_operands(const void* X, long ldx, const void* W, long ldw, cons
 }
 
 
-// Time of a stage (64 k) of a grid that gives every compute unit one workgroup, us: measured at 160 to 2,048 rows of
-// [11264, 2048] (MI355X).
-constexpr struct { int bm, bn; float us; } TILE_STAGE_US[6] = {
-  {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f}};
+// Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: measured at
+// 160 to 2,048 rows of [11264, 2048] (MI355X).  The first five are tile_gemm_kernel's, the others tile_spread_kernel's.  Own tile of
+// before / now, us: 160 rows 25.2 / 22.4, 256 26.0 / 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9;
+// at 1,024 and 1,132 rows 256 x 256 of sixteen waves of 64 x 64 stays (45.6 and 50.5 us; of eight of 64 x 128 54.6 and 53.7).
+constexpr struct { int bm, bn; float us; } TILE_STAGE_US[10] = {
+  {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f},
+  {128, 128, 0.72f}, {128, 192, 0.96f}, {192, 192, 1.12f}, {256, 320, 1.94f}};
 
-static int best_tile(int M, long cols, float& us) {
+static int best_tile(int M, long cols, int choices, float& us) {
   int best = 0;
   us = 1e30f;
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < choices; ++i) {
     const long tiles = (long)((M + TILE_STAGE_US[i].bm - 1) / TILE_STAGE_US[i].bm) * ((cols + TILE_STAGE_US[i].bn - 1) / TILE_STAGE_US[i].bn);
     const long rounds = (tiles + mie_compute_units() - 1) / mie_compute_units();
     if (rounds * TILE_STAGE_US[i].us < us) {
@@ -305,10 +333,10 @@ static int best_tile(int M, long cols, float& us) {
   return best;
 }
 
-// Estimated time of mie_tile_gemm_swiglu, in units of 0.01 us.
+// What mie_tile_gemm_swiglu takes at most, in units of 0.01 us: by the tiles that the decision against the library was measured with.
 MIE_EXPORT int mie_tile_gemm_swiglu_cost(int M, int N, int K) {
   float us;
-  best_tile(M, 2L * N, us);
+  best_tile(M, 2L * N, 6, us);
   return (int)(100.f * us * (K / 64));
 }
 
@@ -319,13 +347,16 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   if (ldo < N || (ldo & 3)) MIE_FAIL("tile_gemm_swiglu: output leading dim %ld for %d columns", ldo, N);
   const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
   float us;
-  switch (best_tile(M, 2L * N, us)) {
-    case 0: return launch<2, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+  switch (best_tile(M, 2L * N, 10, us)) {
     case 1: return launch<3, 2, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 2: return launch<4, 2, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 3: return launch<4, 3, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 4: return launch<4, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
-    default: return launch_wide(x, ldx, w, ldw, (bf16*)out, ldo, M, N, K, s);
+    case 5: return launch_spread<12, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 0: case 6: return launch_spread<4, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 7: return launch_spread<6, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 8: return launch_spread<6, 3, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    default: return launch_spread<10, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
   }
 }
 
@@ -336,8 +367,9 @@ MIE_EXPORT int mie_tile_gemm_units(const void* X, long ldx, const void* W, long 
   const int stages = K / 64, per = units > 0 ? (stages + units - 1) / units : 0;
   if (units < 1 || (units - 1) * per >= stages) MIE_FAIL("tile_gemm_units: %d units of %d stages", units, stages);
   const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
-  // a workgroup a compute unit and a deep ring, or two and a short one
+  // a workgroup a compute unit and a deep ring, or two and a short one (512 rows of [2048, 5632] in four parts 21.4 us by four waves of 64 x
+  // 64, 20.7 by eight; of [4096, 14336] in two 81.1 and 77.1)
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * units;
-  return tiles <= mie_compute_units() ? launch<2, 2, 4, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s)
+  return tiles <= mie_compute_units() ? launch_spread<4, 2, 4, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s)
                                   : launch<2, 2, 2, TG_F32>(x, ldx, w, ldw, part, N, M, N, K, units, s);
 }
