@@ -356,19 +356,22 @@ skinny_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict
 
 // ------------------------------------------------------------------------------------------------ many rows
 // LEVELS 0: the unit is an eighth (grid.z 8), 1: a quarter (grid.z 4), 2: all of K (grid.z 1, result or C += result).
+// GATED (all of K): out = silu(gate) * up; of a wave's weight rows the first half are gate rows, the others the up rows of the same columns.
+// A row of W from `half` on lies `gap` rows further (gate and up rows of some columns of a larger weight; GATED: the up rows lie gap
+// behind).
 // In the LDS, a buffer: planes h, m, l of BM + BN rows of 64 bytes; row r's block b of 16 bytes at 4 r + (b ^ (r / 2) % 4), so that
 // both the writes (a thread has 4 k) and the fragment reads (lane 16 g + r: row r, block g) spread over all banks.
-template <int BM, int BN, int WR, int WC, int LEVELS, bool TAIL>
+template <int BM, int BN, int WR, int WC, int LEVELS, bool TAIL, bool GATED = false>
 __global__ void __launch_bounds__(WR * WC * 64)
 tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ out,
-                long ldo, const float* __restrict__ bias, int add, int M, int N, int K) {
+                long ldo, const float* __restrict__ bias, int add, int M, int N, int K, int half, long gap) {
   constexpr int THREADS = WR * WC * 64, WM = BM / WR, WN = BN / WC, TM = WM / 16, TN = WN / 16, ROWS = BM + BN;
   constexpr int PLANE = ROWS * 64, BUFFER = 3 * PLANE, XL = BM * 8 / THREADS, LOADS = ROWS * 8 / THREADS;      // 16-byte loads a thread and stage
   constexpr bool DOT = TM * TN <= 2;          // few matrix instructions a number that is split (see split2)
   static_assert(BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0, "loads of a thread are of x or of W");
   extern __shared__ __align__(16) char gf_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * (GATED ? BN / 2 : BN);
   const KCut cut = k_cut(K);
   int ks0, ks1;
   if (LEVELS == 0) eighth_range(cut, blockIdx.z, ks0, ks1);
@@ -380,8 +383,15 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
   int at[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    const int r = (tid >> 3) + THREADS / 8 * i, row = i < XL ? m0 + r : n0 + r - BM;
-    src[i] = (i < XL ? X + (size_t)(row < M ? row : M - 1) * ldx : W + (size_t)(row < N ? row : N - 1) * ldw) + blk * 4;
+    const int r = (tid >> 3) + THREADS / 8 * i;
+    if (i < XL) {
+      src[i] = X + (size_t)(m0 + r < M ? m0 + r : M - 1) * ldx + blk * 4;
+    } else {
+      const int c = r - BM, w = c / WN, in = c % WN;
+      int row = GATED ? n0 + w * (WN / 2) + in % (WN / 2) : n0 + c;
+      row = row < N ? row : N - 1;
+      src[i] = W + (size_t)(row + ((GATED ? in >= WN / 2 : row >= half) ? gap : 0)) * ldw + blk * 4;
+    }
     at[i] = r * 64 + ((blk >> 1) ^ ((r >> 1) & 3)) * 16 + (blk & 1) * 8;
   }
   f32x4 staged[2][LOADS];                     // two steps on their way
@@ -499,6 +509,17 @@ tile_f32_kernel(const float* __restrict__ X, long ldx, const float* __restrict__
     if (m >= M) continue;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
+      if constexpr (GATED) {
+        const int n = n0 + wn / 2 + a * 16 + 4 * g;
+        if (a >= TN / 2 || n >= N) continue;
+        f32x4 v = total[a][b] * GF_UNSCALE, u = total[(a + TN / 2) % TN][b] * GF_UNSCALE;
+        again_if_not_finite(v, X + (size_t)m * ldx, W + (size_t)n * ldw, ldw, K);
+        again_if_not_finite(u, X + (size_t)m * ldx, W + (size_t)(n + gap) * ldw, ldw, K);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
+        *reinterpret_cast<f32x4*>(dst + (size_t)m * ld + n) = v;
+        continue;
+      }
       const int n = n0 + wn + a * 16 + 4 * g;
       if (n >= N) continue;                   // N is a multiple of 4
       f32x4 v = LEVELS == 0 ? main[a][b] + small[a][b] : LEVELS == 1 ? quarter[LEVELS >= 1 ? a : 0][LEVELS >= 1 ? b : 0]
@@ -540,7 +561,7 @@ __device__ __forceinline__ f32x4 join_parts(const f32x4* p, size_t stride) {
 template <int PARTS, int EPI>
 __global__ void __launch_bounds__(256)
 reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long ldo, const float* __restrict__ bias, int M, int N,
-                  const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, int K) {
+                  const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, int K, long up_rows) {
   const int cols = EPI == GF_SWIGLU ? 2 * N : N, per_row = N >> 2;
   const size_t stride = (size_t)M * cols / 4, total = (size_t)M * per_row;
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (size_t)gridDim.x * 256) {
@@ -551,7 +572,7 @@ reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long 
     f32x4* o = reinterpret_cast<f32x4*>(out + m * ldo + n);
     if (EPI == GF_SWIGLU) {
       f32x4 u = join_parts<PARTS>(p + (N >> 2), stride);
-      again_if_not_finite(u, X + m * ldx, W + (N + n) * ldw, ldw, K);
+      again_if_not_finite(u, X + m * ldx, W + (up_rows + n) * ldw, ldw, K);
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
       *o = v;
@@ -638,7 +659,7 @@ constexpr struct { int bm, bn; float fixed, each; } GF_TILES[3] = {{128, 128, 0.
 struct TilePlan {
   int tile, units;
 };
-static TilePlan tile_plan(int M, int N, int K, bool gated) {
+static TilePlan tile_plan(int M, int N, int K, bool gated, float* cost = nullptr) {
   TilePlan best = {2, 8};
   float least_us = 1e30f;
   const KCut cut = k_cut(K);
@@ -657,8 +678,25 @@ static TilePlan tile_plan(int M, int N, int K, bool gated) {
       }
     }
   }
+  if (cost) *cost = least_us;
   return best;
 }
+
+// Columns of a gated product [M, N] (N gate and N up rows of W) that are made by uncut 128 x 128 tiles with silu(gate) * up behind them: as
+// many as fill whole rounds of the grid, where those and the others (the plan above) are estimated to take less than the plan for all
+// of them.  0: none.  A round uncut costs a tile's steps and no sums of parts in memory: 512 rows of [11264, 2048] are 256 tiles, one
+// round, and 96 that the plan cuts into quarters, 158 us; all in quarters, 5.5 rounds of 6 and 92 MB of sums, 178; 384 rows 115 and 150, 512 of [28672, 4096] 695 and 776.
+static int whole_columns(int M, int N, int K) {
+  float all_us, rest_us = 0.f;
+  tile_plan(M, 2 * N, K, true, &all_us);
+  const int mt = (M + 127) / 128, nt = (N + 63) / 64, cu = mie_compute_units();
+  const int rounds = (int)((long)mt * nt / cu), whole = rounds > 0 ? (int)((long)cu * rounds / mt) * 64 : 0;
+  if (M <= 16 || whole <= 0) return 0;
+  const int rest = whole < N ? N - whole : 0;
+  if (rest && tile_plan(M, 2 * rest, K, true, &rest_us).units == 1) return 0;
+  return rounds * (2.9f + k_cut(K).steps * GF_TILES[0].each) + rest_us < 0.97f * all_us ? N - rest : 0;
+}
+MIE_EXPORT int mie_f32_whole_columns(int M, int N, int K) { return whole_columns(M, N, K); }
 MIE_EXPORT int mie_f32_units(int M, int N, int K, int gated) { return tile_plan(M, N, K, gated != 0).units; }
 
 template <int EPI>
@@ -687,22 +725,22 @@ static int launch_skinny(const float* X, long ldx, const float* W, long ldw, flo
 
 template <int BM, int BN, int WR, int WC, int LEVELS>
 static int launch_tile(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int add, int M,
-                       int N, int K, int units, hipStream_t s) {
+                       int N, int K, int units, hipStream_t s, int half = 0x7FFFFFFF, long gap = 0) {
   constexpr int lds = 2 * (BM + BN) * 192;
   auto kernel = K & 31 ? tile_f32_kernel<BM, BN, WR, WC, LEVELS, true> : tile_f32_kernel<BM, BN, WR, WC, LEVELS, false>;
   if ((M + BM - 1) / BM > 65535) MIE_FAIL("gemm_f32: M = %d is beyond the grid", M);
   if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;
-  hipLaunchKernelGGL(kernel, dim3((N + BN - 1) / BN, (M + BM - 1) / BM, units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, add, M, N, K);
+  hipLaunchKernelGGL(kernel, dim3((N + BN - 1) / BN, (M + BM - 1) / BM, units), dim3(WR * WC * 64), lds, s, X, ldx, W, ldw, out, ldo, bias, add, M, N, K, half, gap);
   MIE_CHECK_LAUNCH("tile_f32");
   return 0;
 }
 
 static int launch_tiles(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, const float* bias, int add, int M,
-                        int N, int K, const TilePlan& plan, hipStream_t s) {
+                        int N, int K, const TilePlan& plan, hipStream_t s, int half = 0x7FFFFFFF, long gap = 0) {
 #define GF_TILE(BM, BN, WR, WC)                                                                                             \
-  return plan.units == 1   ? launch_tile<BM, BN, WR, WC, 2>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 1, s)           \
-         : plan.units == 4 ? launch_tile<BM, BN, WR, WC, 1>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 4, s)           \
-                           : launch_tile<BM, BN, WR, WC, 0>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 8, s)
+  return plan.units == 1   ? launch_tile<BM, BN, WR, WC, 2>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 1, s, half, gap)           \
+         : plan.units == 4 ? launch_tile<BM, BN, WR, WC, 1>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 4, s, half, gap)           \
+                           : launch_tile<BM, BN, WR, WC, 0>(X, ldx, W, ldw, out, ldo, bias, add, M, N, K, 8, s, half, gap)
   if (plan.tile == 0) GF_TILE(128, 128, 4, 2);
   if (plan.tile == 1) GF_TILE(128, 64, 4, 2);
   GF_TILE(64, 64, 2, 4);
@@ -711,13 +749,14 @@ static int launch_tiles(const float* X, long ldx, const float* W, long ldw, floa
 
 template <int EPI>
 static int launch_reduce(int units, const float* part, float* out, long ldo, const float* bias, int M, int N, const float* X, long ldx,
-                         const float* W, long ldw, int K, hipStream_t s) {
+                         const float* W, long ldw, int K, hipStream_t s, long up_rows = 0) {
+  if (!up_rows) up_rows = N;
   long blocks = ((long)M * (N / 4) + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   if (units == 4)
-    hipLaunchKernelGGL((reduce_f32_kernel<4, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K);
+    hipLaunchKernelGGL((reduce_f32_kernel<4, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, up_rows);
   else
-    hipLaunchKernelGGL((reduce_f32_kernel<8, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K);
+    hipLaunchKernelGGL((reduce_f32_kernel<8, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, up_rows);
   MIE_CHECK_LAUNCH("reduce_f32");
   return 0;
 }
@@ -746,6 +785,29 @@ MIE_EXPORT int mie_gemm_f32(const float* X, long ldx, const float* W, long ldw, 
   return epi == GF_STORE ? launch_reduce<GF_STORE>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
        : epi == GF_ADD ? launch_reduce<GF_ADD>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s)
                        : launch_reduce<GF_SWIGLU>(units, part, out, ldo, bias, M, N, X, ldx, W, ldw, K, s);
+}
+
+// out [M, N] = silu(x Wg^T) * (x Wu^T), its first mie_f32_whole_columns(M, N, K) columns (not 0) by uncut tiles, the others in
+// mie_f32_units(M, 2 * others, K, 1) units, whose sums take units * M * 2 * others floats of part (16-byte aligned).
+MIE_EXPORT int mie_gemm_f32_gated(const float* X, long ldx, const float* W, long ldw, float* out, long ldo, float* part, int M, int N, int K,
+                                  hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  if (check_operands("gemm_f32_gated", X, ldx, W, ldw, out, ldo, N, K)) return -1;
+  const int whole = whole_columns(M, N, K), rest = N - whole;
+  if (!whole) MIE_FAIL("gemm_f32_gated: no columns of %d rows of [%d, %d] fill the grid", M, 2 * N, K);
+  if (rest && (!part || ((uintptr_t)part & 15))) MIE_FAIL("gemm_f32_gated: the units' sums need memory, 16-byte aligned");
+  constexpr int lds = 2 * (128 + 128) * 192;
+  auto kernel = K & 31 ? tile_f32_kernel<128, 128, 4, 2, 2, true, true> : tile_f32_kernel<128, 128, 4, 2, 2, false, true>;
+  if ((M + 127) / 128 > 65535) MIE_FAIL("gemm_f32: M = %d is beyond the grid", M);
+  if (mie_allow_lds((const void*)kernel, lds, "gemm_f32")) return -1;
+  hipLaunchKernelGGL(kernel, dim3((whole + 63) / 64, (M + 127) / 128, 1), dim3(512), lds, s, X, ldx, W, ldw, out, ldo, nullptr, 0, M, whole, K,
+                     0, (long)N);
+  MIE_CHECK_LAUNCH("tile_f32");
+  if (!rest) return 0;
+  const TilePlan plan = tile_plan(M, 2 * rest, K, true);
+  const float* Wr = W + (size_t)whole * ldw;
+  if (launch_tiles(X, ldx, Wr, ldw, part, 2 * rest, nullptr, 0, M, 2 * rest, K, plan, s, rest, (long)whole)) return -1;
+  return launch_reduce<GF_SWIGLU>(plan.units, part, out + whole, ldo, nullptr, M, rest, X, ldx, Wr, ldw, K, s, N);
 }
 
 // How many units K is cut into where the product is added into a stream whose RMSNorm is wanted next (mie_gemm_f32_add_norm), 0: the

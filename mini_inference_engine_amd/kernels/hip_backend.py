@@ -237,6 +237,14 @@ class HipBackend(KernelBackend):
         lib = self.lib("gemm_f32")
         M, K = x.shape
         cols, part = w.shape[0], None
+        whole = lib.mie_f32_whole_columns(M, cols // 2, K) if epi == self.F32_SWIGLU and M > 16 else 0
+        if whole:
+            rest = cols // 2 - whole
+            if rest:
+                part = torch.empty((lib.mie_f32_units(M, 2 * rest, K, 1), M, 2 * rest), dtype=torch.float32, device=x.device)
+            library.check(lib, lib.mie_gemm_f32_gated(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), _ptr(part), M,
+                                                      cols // 2, K, self._stream()))
+            return True
         if M > 16:
             units = lib.mie_f32_units(M, cols, K, int(epi == self.F32_SWIGLU))
             if units > 1:

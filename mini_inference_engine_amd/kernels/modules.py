@@ -40,6 +40,8 @@ register_kernel_module("gemm", {
 register_kernel_module("gemm_f32", {
     "mie_f32_units": [I, I, I, I],
     "mie_f32_norm_units": [I, I, I],
+    "mie_f32_whole_columns": [I, I, I],
+    "mie_gemm_f32_gated": [P, L, P, L, P, L, P, I, I, I, P],
     "mie_gemm_f32_add_norm": [P, L, P, L, P, P, I, P, P, I, I, I, F, P],
     "mie_gemm_f32": [P, L, P, L, P, L, I, P, P, I, I, I, P],
     "mie_qkv_rope_f32": [P, L, P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, I, P],

@@ -473,6 +473,26 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
+# rows, K, columns and how many of them are made by uncut tiles
+@pytest.mark.parametrize("case", [(512, 2048, 5632, 4096), (384, 72, 5632, 5440), (260, 72, 7000, 0), (129, 96, 8256, 8192), (600, 64, 3300, 3264), (400, 200, 4096, 4096),
+                                  (520, 40, 3332, 3264), (2047, 200, 1000, 1000)])
+def test_float32_gated_product_partly_uncut(ops, case):
+    """Gate and up in float32 where the columns that fill the grid's rounds are uncut tiles with SwiGLU behind them and the others go in
+    parts: the bits of the product and silu_mul, edges in rows, columns and K, results beyond what the parts can hold too."""
+    o, (M, K, inter, whole) = ops[torch.float32], case
+    lib = o.lib("gemm_f32")
+    assert lib.mie_f32_whole_columns(M, inter, K) == whole, "the case must take the path it is for"
+    torch.manual_seed(M + K)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)
+    x[M // 2, 3] = 2.0e36
+    with counted(o, "gemm_f32", "mie_gemm_f32_gated") as calls:
+        y = o.linear_silu_mul(x, w, inter)
+    assert len(calls) == (whole > 0)
+    assert torch.equal(y, o.silu_mul(o.linear(x, w), inter))
+    assert lib.mie_f32_whole_columns(16, inter, K) == 0
+    assert lib.mie_gemm_f32_gated(x.data_ptr(), K, w.data_ptr(), K, y.data_ptr(), inter, None, 16, inter, K, None) != 0
+
+
 @pytest.mark.parametrize("case", [(2047, 192, 5640), (1281, 64, 7496), (1793, 128, 6144), (2048, 2048, 5632)])
 def test_wide_tile_product_swiglu(engine_ops, case):
     """Gate and up on tiles of 256 x 384 (taken where they make one round of what other tiles need two for): edges in rows and
