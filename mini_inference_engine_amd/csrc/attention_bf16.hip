@@ -780,6 +780,10 @@ static int scratch_for_current_device(float** ptr) {
 
 MIE_EXPORT int mie_decode_attention_static_setup(void) {
   float* p;
+  // (and the LDS beyond the default that the kernels ask for)
+  if (mie_allow_lds((const void*)decode_attention_kernel<NW_SPLIT, false>, da_lds_bytes(NW_SPLIT), "decode_attention_static") ||
+      mie_allow_lds((const void*)decode_attention_kernel<NW_WHOLE, false>, da_lds_bytes(NW_WHOLE), "decode_attention_static"))
+    return -1;
   return scratch_for_current_device(&p);
 }
 

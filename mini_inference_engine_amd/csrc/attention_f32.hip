@@ -660,7 +660,7 @@ MIE_EXPORT int mie_attention_f32_portions(const float* q, long q_stride, const f
   if (Hkv * head_tiles > 65535 || rows - row0 > 65535) MIE_FAIL("attention_f32: %d kv heads, %d rows are beyond the grid", Hkv, rows - row0);
   const int tiles = (max_row_tokens + AF_TILE_WAVES * per_tile - 1) / (AF_TILE_WAVES * per_tile);
   if ((long)tiles * Hkv * head_tiles > 0x7FFFFFFF) MIE_FAIL("attention_f32: %d tokens are beyond the grid", max_row_tokens);
-  if ((long)page * D > 1L << 26) MIE_FAIL("attention_f32: pages of %d", page);      // 32-bit offsets within a page
+  if (page > 1 << 24) MIE_FAIL("attention_f32: pages of %d", page);                 // 32-bit offsets within a page
   const dim3 grid(tiles * Hkv * head_tiles, rows - row0);
 #define AF_PORTIONS(DT)                                                                                                              \
   {                                                                                                                                  \

@@ -286,7 +286,8 @@ class HipBackend(KernelBackend):
         m = x.shape[0] if rows is None else rows.shape[0]
         return (not self.true_fp32 and bias is None and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
                 and m <= self.SKINNY_MAX_ROWS and x.shape[0] <= 64 and w.shape[1] % 8 == 0 and w.stride(0) % 8 == 0
-                and x.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+                and x.stride(0) % 8 == 0 and w.stride(0) <= 1 << 24 and x.stride(0) <= 1 << 24
+                and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
     def _prepared(self, x, w, bias):
         """If ``x`` is a Normed whose input an earlier product already prepared (weighted, rounded values
@@ -1683,7 +1684,7 @@ class HipBackend(KernelBackend):
         # The kernel rotates with the step's positions, takes the row's own key from its LDS and writes it to
         # pending.slots: that is the same result as finish() only if the projection was made for this very step
         # and this page group (same position and slot arrays, same caches).  Anything else takes finish().
-        if (forced or step.num_decode_rows != T or step.num_tokens != T or Hq // Hkv > 16
+        if (forced or (k_cache.data_ptr() | v_cache.data_ptr()) % 16 or step.num_decode_rows != T or step.num_tokens != T or Hq // Hkv > 16
                 or pending.k_cache is not k_cache or pending.v_cache is not v_cache
                 or pending.positions.data_ptr() != step.positions.data_ptr()
                 or pending.slots.data_ptr() != group.slot_mapping.data_ptr()
@@ -1768,6 +1769,8 @@ class HipBackend(KernelBackend):
             qkv = qkv.finish()
         self._on_device(qkv, k_cache, v_cache)
         T, page, bt = self._check_attention(qkv, Hq, Hkv, D, k_cache, v_cache, group, step)
+        if qkv.dtype == torch.bfloat16 and (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+            k_cache, v_cache = k_cache.clone(), v_cache.clone()         # (only read here) the kernels load 16 bytes at a time
         out = torch.empty((T, Hq * D), dtype=qkv.dtype, device=qkv.device)
         done = 0
         if D > 256:

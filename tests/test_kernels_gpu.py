@@ -1518,6 +1518,17 @@ def test_attention_float32_matrix_unit(ops, geom, window):
         assert calls == ["mie_attention_f32_single"] and torch.equal(out, whole)
 
 
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_decode_attention_of_caches_off_16_bytes(ops, D):
+    """Contiguous caches that begin 8 bytes into memory: the same result as of ones that begin on 16."""
+    q, kc, vc, group, step = paged_setup([70, 33, 200], [1, 1, 1], 8, 2, D, 16, torch.bfloat16, seed=D)
+    o = ops[torch.bfloat16]
+    want = o.paged_attention(q, 8, 2, D, kc, vc, group, step, D ** -0.5, None)
+    off = [torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t) for t in (kc, vc)]
+    assert all(t.data_ptr() % 16 for t in off)
+    assert torch.equal(o.paged_attention(q, 8, 2, D, *off, group, step, D ** -0.5, None), want)
+
+
 @pytest.mark.parametrize("window", [None, 1, 130])
 @pytest.mark.parametrize("geom", [(32, 4, 64, 16), (3, 1, 32, 16), (5, 5, 48, 32), (40, 2, 16, 16), (16, 1, 128, 16), (10, 2, 112, 48), (6, 2, 80, 16)])
 def test_attention_float32_few_single_tokens(ops, geom, window):
