@@ -37,12 +37,12 @@ constexpr int NW_WHOLE = D > 128 ? 2 : (D > 64 ? 4 : 8);
 constexpr bool RINGED = D % 32 == 0 && D >= 64 && D <= 128;
 // Blocks of a wave on their way: 32 to 64 KB a workgroup of four waves, 128 of eight (two blocks a wave of four leave room for two
 // workgroups a compute unit: head size 64, 128 rows of 100 to 1,990 keys 33.4 us with one, 36.5 with two, 256 of 512 29.1 and 33.6)
-constexpr int slots_of(int nw) { return !RINGED ? 0 : nw == 8 ? 2 : 1; }
+constexpr int slots_of(int nw, bool ring = RINGED) { return !ring ? 0 : nw == 8 ? 2 : 1; }
 constexpr int BLOCK_LOADS = D / 8;           // of 1 KB: keys and values of 32 keys
 // Dynamic LDS of a workgroup of nw waves: the slots, and later, in the same place, the waves' sums.
-constexpr int da_lds_bytes(int nw) {
-  const int ring = nw * slots_of(nw) * BLOCK_KEYS * D * 4, sums = nw * 16 * (D + 1) * 4;
-  return ring > sums ? ring : sums;
+constexpr int da_lds_bytes(int nw, bool ring) {
+  const int slots = nw * slots_of(nw, ring) * BLOCK_KEYS * D * 4, sums = nw * 16 * (D + 1) * 4;
+  return slots > sums ? slots : sums;
 }
 // Workgroups up to which one is NW_WHOLE waves: while each has a compute unit's LDS to itself (ringed), or fewer than two a compute unit.
 static long whole_most() { return RINGED ? mie_compute_units() : 2L * mie_compute_units() - 1; }
@@ -72,7 +72,9 @@ struct ProjectionSums {
 // window's in the order the splits and waves walk: index x of that order is key x up to the end of the kept blocks, key
 // x + gap behind it, gap a whole number of blocks.
 // CHUNK: the softmax over the keys of the row's own chunk of positions (from floor(position / chunk) chunk on).
-template <int NW, bool FROM_SUMS, bool SIG = false, bool DB = false, bool KEEP = false, bool CHUNK = false>
+// RING: keys and values through the slots.  Caches off 16 bytes, which those loads do not take, come into registers (RING false), at the
+// ringed head sizes in the slots' order of keys, so that the result has the same bits.
+template <int NW, bool FROM_SUMS, bool SIG, bool DB, bool KEEP, bool CHUNK, bool RING>
 __global__ void __launch_bounds__(NW * 64)
 decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache, bf16* v_cache,
                         bf16* __restrict__ out, float* __restrict__ o_part,
@@ -137,28 +139,30 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   auto load_block = [&](KeyBlock& B, const Places& p) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const bf16* kp = k_cache + (((size_t)p.pg[t] * Hkv + kvh) * page + p.off[t]) * D;
+      const int half = RINGED ? col >> 3 : t, r = RINGED ? (col >> 2 & 1) * 8 + 4 * t + (col & 3) : col;      // of the block; the key in it
+      const bf16* kp = k_cache + (((size_t)(half ? p.pg[1] : p.pg[0]) * Hkv + kvh) * page + (half ? p.off[1] : p.off[0])) * D;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const int d0 = ks * 32 + kb * 8;
-        B.a[t][ks].q = *reinterpret_cast<const uint4*>(kp + (col * D + (d0 < D ? d0 : 0)));
+        B.a[t][ks].q = *reinterpret_cast<const uint4*>(kp + (r * D + (d0 < D ? d0 : 0)));
       }
     }
     const bf16* v0 = v_cache + ((size_t)p.pg[0] * Hkv + kvh) * D * page + p.off[0];
     const bf16* v1 = v_cache + ((size_t)p.pg[1] * Hkv + kvh) * D * page + p.off[1];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const int at = (dt * 16 + col) * page + 4 * kb;
-      B.va[dt].h[0] = *reinterpret_cast<const uint2*>(v0 + at);
-      B.va[dt].h[1] = *reinterpret_cast<const uint2*>(v1 + at);
+      const int at = (dt * 16 + col) * page + (RINGED ? 8 * (kb & 1) : 4 * kb);
+      const bf16 *f0 = RINGED && kb >> 1 ? v1 : v0, *f1 = RINGED ? f0 + 4 : v1;
+      B.va[dt].h[0] = *reinterpret_cast<const uint2*>(f0 + at);
+      B.va[dt].h[1] = *reinterpret_cast<const uint2*>(f1 + at);
     }
   };
   // The slots.  Keys: row k of 32 as it stands in its page, 16-byte block b at place b ^ f(k) of it, f = k % 4 + 4 (k / 8 % 2) as far as
   // the row's blocks allow; values: a page's 16 keys of a dim are two blocks, swapped for every second four dims.  Both so
   // that eight lanes' fragment reads are in different banks.
-  constexpr int SLOTS = slots_of(NW), AHEAD_LOADS = RINGED ? (SLOTS - 1) * BLOCK_LOADS : 0;
+  constexpr int SLOTS = slots_of(NW, RING), AHEAD_LOADS = RING ? (SLOTS - 1) * BLOCK_LOADS : 0;
   static_assert(AHEAD_LOADS <= 63, "more loads in flight than the counter holds");
-  constexpr int NBLK = D / 8, TURN = NBLK % 8 == 0 ? 7 : 3, KL = RINGED ? D / 32 : 1;
+  constexpr int NBLK = D / 8, TURN = NBLK % 8 == 0 ? 7 : 3, KL = RING ? D / 32 : 1;
   uint32_t koff[KL];
 #pragma unroll
   for (int j = 0; j < KL; ++j) {
@@ -203,7 +207,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   int begin0 = s * partition;               // the split's first key when there is no window
   const bool early = AHEAD && !CHUNK && window <= 0 && (!SIG || chunk <= 0);
   if (early) {
-    if constexpr (RINGED) issue(0, find(begin0 + BLOCK_KEYS * wave));
+    if constexpr (RING) issue(0, find(begin0 + BLOCK_KEYS * wave));
     else load_block(b0, find(begin0 + BLOCK_KEYS * wave));
   }
 
@@ -281,7 +285,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
   const int end = begin + partition < last_x + 1 ? begin + partition : last_x + 1;
 
   if (begin > last_x) {
-    if (RINGED) MIE_VMCNT(0);    // nothing of this wave may still be writing the LDS when it ends
+    if (RING) MIE_VMCNT(0);      // nothing of this wave may still be writing the LDS when it ends
     // this split lies beyond the row's keys (uniform over the workgroup)
     if (num_splits > 1 && threadIdx.x < 16 && ht * 16 + (int)threadIdx.x < G)
       lse_part[((size_t)b * Hq + kvh * G + ht * 16 + threadIdx.x) * num_splits + s] = -INFINITY;
@@ -425,7 +429,7 @@ decode_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache
 
   constexpr int STEP = BLOCK_KEYS * NW;     // keys from one block of a wave to its next
   const int first = begin + BLOCK_KEYS * wave;
-  if constexpr (RINGED) {
+  if constexpr (RING) {
     const int count = first < end ? (end - first + STEP - 1) / STEP : 0;       // this wave's blocks: nothing beyond the split's own keys
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i)
@@ -579,12 +583,16 @@ merge_splits_kernel(const float* __restrict__ o_part, const float* __restrict__ 
 
 MIE_EXPORT const char* attention_bf16_last_error() { return g_mie_error; }
 MIE_EXPORT int mie_attention_bf16_head_dim() { return D; }
-#define DA_LAUNCH(KERNEL, NW, STREAM, ...)                                                            \
-  do {                                                                                               \
-    auto kernel_ = KERNEL;                                                                           \
-    if (mie_allow_lds((const void*)kernel_, da_lds_bytes(NW), "decode_attention")) return -1;         \
-    hipLaunchKernelGGL(kernel_, grid, dim3(NW * 64), da_lds_bytes(NW), STREAM, __VA_ARGS__);         \
+#define DA_KIND(...) __VA_ARGS__
+// KIND: FROM_SUMS, SIG, DB, KEEP, CHUNK in brackets; `off16` is the caller's
+#define DA_LAUNCH(NW, KIND, STREAM, ...)                                                                                           \
+  do {                                                                                                                             \
+    auto kernel_ = off16 ? decode_attention_kernel<NW, DA_KIND KIND, false> : decode_attention_kernel<NW, DA_KIND KIND, RINGED>;    \
+    const int lds_ = da_lds_bytes(NW, RINGED && !off16);                                                                           \
+    if (mie_allow_lds((const void*)kernel_, lds_, "decode_attention")) return -1;                                                   \
+    hipLaunchKernelGGL(kernel_, grid, dim3(NW * 64), lds_, STREAM, __VA_ARGS__);                                                   \
   } while (0)
+static bool caches_off16(const void* k_cache, const void* v_cache) { return RINGED && (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15); }
 
 MIE_EXPORT int mie_decode_block_keys() { return BLOCK_KEYS * NW_SPLIT; }
 
@@ -617,55 +625,56 @@ static int decode_attention_launch(const void* q, long q_stride, const void* k_c
   // (the kernel writes the caches only when it is given the projection's sums)
   bf16* kc = (bf16*)const_cast<void*>(k_cache);
   bf16* vc = (bf16*)const_cast<void*>(v_cache);
+  const bool off16 = caches_off16(k_cache, v_cache);
   const bool whole = num_splits == 1 && NW_WHOLE != NW_SPLIT && (long)rows * Hkv * head_tiles <= whole_most();
   if (chunk > 0 && !sigmoid && (keep > 0 || dist_bias)) MIE_FAIL("decode_attention: chunks beside kept keys or a distance bias are not built");
   if (chunk > 0 && !sigmoid && whole)
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, false, false, true>), NW_WHOLE, stream,
+    DA_LAUNCH(NW_WHOLE, (false, false, false, false, true), stream,
                        (const bf16*)q, q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv,
                        head_tiles, page, scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else if (chunk > 0 && !sigmoid)
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, false, false, true>), NW_SPLIT, stream,
+    DA_LAUNCH(NW_SPLIT, (false, false, false, false, true), stream,
                        (const bf16*)q, q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv,
                        head_tiles, page, scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else if (keep > 0 && whole)
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, false, true>), NW_WHOLE, stream, (const bf16*)q,
+    DA_LAUNCH(NW_WHOLE, (false, false, false, true, false), stream, (const bf16*)q,
                        q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, keep, head_sinks);
   else if (keep > 0)
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, false, true>), NW_SPLIT, stream, (const bf16*)q,
+    DA_LAUNCH(NW_SPLIT, (false, false, false, true, false), stream, (const bf16*)q,
                        q_stride, kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, keep, head_sinks);
   else if (dist_bias && whole)
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, false, true>), NW_WHOLE, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_WHOLE, (false, false, true, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, dist_bias, dist_n, 0, head_sinks);
   else if (dist_bias)
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, false, true>), NW_SPLIT, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_SPLIT, (false, false, true, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, dist_bias, dist_n, 0, head_sinks);
   else if (sigmoid && whole)
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false, true>), NW_WHOLE, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_WHOLE, (false, true, false, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, softcap, head_bias, (const float*)nullptr, 0, 0,
                        head_sinks);
   else if (sigmoid)
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false, true>), NW_SPLIT, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_SPLIT, (false, true, false, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale, window, partition, num_splits, ProjectionSums{}, sink_log2, chunk, softcap, head_bias, (const float*)nullptr, 0, 0,
                        head_sinks);
   else if (whole)
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, false>), NW_WHOLE, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_WHOLE, (false, false, false, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
   else
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, false>), NW_SPLIT, stream, (const bf16*)q, q_stride,
+    DA_LAUNCH(NW_SPLIT, (false, false, false, false, false), stream, (const bf16*)q, q_stride,
                        kc, vc, (bf16*)out, o_part, lse_part, block_tables, max_blocks, positions, Hq, Hkv, head_tiles, page,
                        scale * 1.4426950408889634f, window, partition, num_splits, ProjectionSums{}, sink_log2, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, head_sinks);
@@ -733,13 +742,14 @@ MIE_EXPORT int mie_decode_attention_from_sums(const float* part, int splits, lon
   if (max_blocks <= 0 || Hkv > 65535) MIE_FAIL("decode_attention_from_sums: max_blocks %d, %d kv heads", max_blocks, Hkv);
   const ProjectionSums proj = {part, splits, (size_t)split_stride, ld, cos_t, sin_t, slots};
   dim3 grid(rows, Hkv, 1);
+  const bool off16 = caches_off16(k_cache, v_cache);
   if ((long)rows * Hkv <= whole_most())
-    DA_LAUNCH((decode_attention_kernel<NW_WHOLE, true>), NW_WHOLE, stream, (const bf16*)nullptr, 0L,
+    DA_LAUNCH(NW_WHOLE, (true, false, false, false, false), stream, (const bf16*)nullptr, 0L,
                        (bf16*)k_cache, (bf16*)v_cache, (bf16*)out, (float*)nullptr, (float*)nullptr, block_tables, max_blocks,
                        positions, Hq, Hkv, 1, page, scale * 1.4426950408889634f, window, partition, 1, proj, -INFINITY, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, (const float*)nullptr);
   else
-    DA_LAUNCH((decode_attention_kernel<NW_SPLIT, true>), NW_SPLIT, stream, (const bf16*)nullptr, 0L,
+    DA_LAUNCH(NW_SPLIT, (true, false, false, false, false), stream, (const bf16*)nullptr, 0L,
                        (bf16*)k_cache, (bf16*)v_cache, (bf16*)out, (float*)nullptr, (float*)nullptr, block_tables, max_blocks,
                        positions, Hq, Hkv, 1, page, scale * 1.4426950408889634f, window, partition, 1, proj, -INFINITY, 0, 0.f,
                        (const float*)nullptr, (const float*)nullptr, 0, 0, (const float*)nullptr);
@@ -781,9 +791,10 @@ static int scratch_for_current_device(float** ptr) {
 MIE_EXPORT int mie_decode_attention_static_setup(void) {
   float* p;
   // (and the LDS beyond the default that the kernels ask for)
-  if (mie_allow_lds((const void*)decode_attention_kernel<NW_SPLIT, false>, da_lds_bytes(NW_SPLIT), "decode_attention_static") ||
-      mie_allow_lds((const void*)decode_attention_kernel<NW_WHOLE, false>, da_lds_bytes(NW_WHOLE), "decode_attention_static"))
-    return -1;
+#define DA_ALLOW(NW, RING) \
+  mie_allow_lds((const void*)decode_attention_kernel<NW, false, false, false, false, false, RING>, da_lds_bytes(NW, RING), "decode_attention_static")
+  if (DA_ALLOW(NW_SPLIT, RINGED) || DA_ALLOW(NW_WHOLE, RINGED) || DA_ALLOW(NW_SPLIT, false) || DA_ALLOW(NW_WHOLE, false)) return -1;
+#undef DA_ALLOW
   return scratch_for_current_device(&p);
 }
 

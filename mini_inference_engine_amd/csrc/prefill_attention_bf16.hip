@@ -66,7 +66,7 @@ constexpr int KS16 = D / 16;                        // 16-dim steps of q . k
 constexpr int DT32 = (D + 31) / 32;                 // 32-dim tiles of the output (the last may be half empty)
 constexpr int PF_KROW = 2 * D + 16;                 // bytes of a key row in the LDS
 constexpr int PF_VROW = 2 * PF_BK + 16;             // bytes of a value row (one dim, 64 keys) in the LDS
-constexpr bool PF_DIRECT = D == 64 || D == 128;     // blocks come in by loads that write the LDS themselves
+constexpr bool PF_DIRECT = D == 64 || D == 128;     // blocks come in by loads that write the LDS themselves, 16 bytes from multiples of 16
 constexpr int PF_KBYTES = PF_DIRECT ? PF_BK * 2 * D : PF_BK * PF_KROW;
 constexpr int PF_VBYTES = PF_DIRECT ? PF_BK * 2 * D : DT32 * 32 * PF_VROW;      // rows of dims beyond D stay zero
 constexpr int PF_BUF = PF_KBYTES + PF_VBYTES;       // one buffer: keys, then values
@@ -758,6 +758,8 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 }
 
 MIE_EXPORT const char* prefill_attention_bf16_last_error() { return g_mie_error; }
+// 1: the caches must be 16-byte aligned
+MIE_EXPORT int mie_prefill_needs_aligned_caches() { return PF_DIRECT; }
 
 enum PrefillKind { FOUR, EIGHT_QUERIES, EIGHT_KEYS };
 struct PrefillPlan {
@@ -846,6 +848,7 @@ static int prefill_attention_launch(const void* q, long q_stride, const void* k_
   if (page < 16 || page % 16) MIE_FAIL("prefill_attention: page size %d (multiples of 16)", page);
   if (q_stride < (long)Hq * D || (q_stride % 8) || ((uintptr_t)q % 16) || ((uintptr_t)out % 8))
     MIE_FAIL("prefill_attention: q stride %ld / alignment", q_stride);
+  if (PF_DIRECT && (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15)) MIE_FAIL("prefill_attention: caches must be 16-byte aligned");
   if (max_blocks <= 0) MIE_FAIL("prefill_attention: max_blocks %d", max_blocks);
   int dev;
   long units;

@@ -1684,7 +1684,7 @@ class HipBackend(KernelBackend):
         # The kernel rotates with the step's positions, takes the row's own key from its LDS and writes it to
         # pending.slots: that is the same result as finish() only if the projection was made for this very step
         # and this page group (same position and slot arrays, same caches).  Anything else takes finish().
-        if (forced or (k_cache.data_ptr() | v_cache.data_ptr()) % 16 or step.num_decode_rows != T or step.num_tokens != T or Hq // Hkv > 16
+        if (forced or step.num_decode_rows != T or step.num_tokens != T or Hq // Hkv > 16
                 or pending.k_cache is not k_cache or pending.v_cache is not v_cache
                 or pending.positions.data_ptr() != step.positions.data_ptr()
                 or pending.slots.data_ptr() != group.slot_mapping.data_ptr()
@@ -1707,6 +1707,17 @@ class HipBackend(KernelBackend):
             _ptr(pending.slots), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(bt), bt.shape[1], _ptr(step.positions), T,
             Hq, Hkv, D, pending.page, float(scale), int(window or 0), partition, self._stream()))
         return out
+
+    @staticmethod
+    def _pages_of_portions(k_cache, v_cache, bt, step, page):
+        """The pages that the step's rows of several tokens name, each row's side by side in memory of their own (16-byte aligned),
+        and block tables for them; both caches are only read."""
+        first, rows = step.num_decode_rows, step.num_rows
+        most = min(bt.shape[1], -(-step.max_context // page)) if step.max_context > 0 else bt.shape[1]
+        named = bt[first:rows, :most].reshape(-1)
+        table = torch.zeros((rows, bt.shape[1]), dtype=torch.int32, device=bt.device)
+        table[first:, :most] = torch.arange(named.shape[0], dtype=torch.int32, device=bt.device).view(rows - first, most)
+        return k_cache.index_select(0, named), v_cache.index_select(0, named), table
 
     def _in_log2(self, table):
         """A table the matrix-core kernels add to scores or sinks, in their units of log2 e; made once a table."""
@@ -1769,8 +1780,6 @@ class HipBackend(KernelBackend):
             qkv = qkv.finish()
         self._on_device(qkv, k_cache, v_cache)
         T, page, bt = self._check_attention(qkv, Hq, Hkv, D, k_cache, v_cache, group, step)
-        if qkv.dtype == torch.bfloat16 and (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
-            k_cache, v_cache = k_cache.clone(), v_cache.clone()         # (only read here) the kernels load 16 bytes at a time
         out = torch.empty((T, Hq * D), dtype=qkv.dtype, device=qkv.device)
         done = 0
         if D > 256:
@@ -1819,7 +1828,10 @@ class HipBackend(KernelBackend):
             if written is not None and (written.dtype != torch.int32 or written.shape[0] < step.num_rows or not written.is_contiguous()):
                 raise ValueError(f"paged_attention: row_written must be contiguous int32 [{step.num_rows}]")
             lib = self.lib("prefill_attention_bf16", (f"-DHEAD_DIM={D}",))
-            args = (_ptr(qkv), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(bt), bt.shape[1],
+            keys, values, table = k_cache, v_cache, bt
+            if (k_cache.data_ptr() | v_cache.data_ptr()) % 16 and lib.mie_prefill_needs_aligned_caches():
+                keys, values, table = self._pages_of_portions(k_cache, v_cache, bt, step, page)
+            args = (_ptr(qkv), qkv.stride(0), _ptr(keys), _ptr(values), _ptr(out), _ptr(table), table.shape[1],
                     _ptr(step.row_start), _ptr(step.row_position), _ptr(written), step.num_decode_rows,
                     step.num_rows - step.num_decode_rows, step.max_row_tokens, Hq, Hkv, D, page, float(scale),
                     int(window or 0))

@@ -141,6 +141,7 @@ register_kernel_module("attention_bf16", {
 # the compiler parks the outputs in accumulation registers and copies all of them back and forth around
 # every key block for the sake of the (rare) rescaling.
 register_kernel_module("prefill_attention_bf16", {
+    "mie_prefill_needs_aligned_caches": [],
     "mie_prefill_attention_kind": [I, I, I, I],
     "mie_prefill_attention": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P],
     "mie_prefill_attention_sink": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, F, P],

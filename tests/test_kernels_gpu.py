@@ -1148,7 +1148,7 @@ def test_decode_attention_finishes_the_projection(engine_ops, geom, window):
     and does rotary, cache write and attention itself.  Against the same step done by the kernels that are each
     checked against their references elsewhere: sum + rotary + cache write, then attention over the cache.
     Contexts of 1 key, around the kernel's first blocks (which it asks for before the new key is written),
-    at page edges, and long ones; fewer and more than 512 workgroups (eight waves a workgroup, or four)."""
+    at page edges, and long ones; fewer and more workgroups than those up to which one is eight waves."""
     from mini_inference_engine_amd.kernels.hip_backend import ProjectionSums
     from mini_inference_engine_amd.parts.rope import rotary_tables
     Hq, Hkv, D, page, M = geom
@@ -1527,6 +1527,60 @@ def test_decode_attention_of_caches_off_16_bytes(ops, D):
     off = [torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t) for t in (kc, vc)]
     assert all(t.data_ptr() % 16 for t in off)
     assert torch.equal(o.paged_attention(q, 8, 2, D, *off, group, step, D ** -0.5, None), want)
+
+
+def off_16_bytes(*caches):
+    off = [torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t) for t in caches]
+    assert all(t.data_ptr() % 16 for t in off)
+    return off
+
+
+@pytest.mark.parametrize("D", [64, 80, 96, 128])
+def test_attention_of_caches_off_16_bytes_keeps_bits_and_memory(ops, D):
+    """Caches that begin 8 bytes into memory, every kind of attention, split and whole contexts, eight and four waves, prompts: the
+    bits of caches that begin on 16, and never a copy of the caches."""
+    o, Hq, Hkv = ops[torch.bfloat16], 8, 2
+    table = torch.randn(Hq, 40, device=DEV)
+    kinds = [{}, dict(window=50), dict(weights="sigmoid", softcap=5.0), dict(weights="sigmoid", chunk=64), dict(distance_bias=table),
+             dict(window=40, keep_first=5), dict(chunk=48), dict(sink=0.5)]
+    for ctx, new in (([70, 33, 200], [1, 1, 1]), ([1, 16, 31, 33, 200] * 20, [1] * 100), ([100, 65] * 80, [1] * 160), ([90, 33, 200, 130], [1, 1, 64, 130])):
+        q, kc, vc, group, step = paged_setup(ctx, new, Hq, Hkv, D, 16, torch.bfloat16, num_pages=4096, seed=D)
+        off = off_16_bytes(kc, vc)
+        for kind in kinds:
+            kw = dict(kind)
+            window = kw.pop("window", None)
+            want = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, D ** -0.5, window, **kw)
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            got = o.paged_attention(q, Hq, Hkv, D, *off, group, step, D ** -0.5, window, **kw)
+            torch.cuda.synchronize()
+            assert torch.cuda.max_memory_allocated() - before < kc.numel()
+            assert torch.equal(got, want), (len(ctx), kind)
+
+
+@pytest.mark.parametrize("M", [64, 140])
+def test_decode_attention_from_sums_into_caches_off_16_bytes(engine_ops, M):
+    """The decode kernel that finishes the projection, on caches 8 bytes into memory: results and caches as on 16."""
+    from mini_inference_engine_amd.kernels.hip_backend import ProjectionSums
+    from mini_inference_engine_amd.parts.rope import rotary_tables
+    o, Hq, Hkv, D, page, K = engine_ops, 16, 4, 64, 16, 264
+    ctx = ([1, 16, 17, 33, 128, 300, 48] * 20)[:M]
+    _, kc, vc, group, step = paged_setup(ctx, [1] * M, Hq, Hkv, D, page, torch.bfloat16, seed=M)
+    cos, sin = (t.to(DEV) for t in rotary_tables(10000.0, D, max(ctx) + 1))
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn((Hq + 2 * Hkv) * D, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    pos = step.positions
+    group.slot_mapping = (group.block_tables[torch.arange(M, device=DEV), (pos // page).long()] * page + pos % page).to(torch.int32)
+    made = []
+    for caches in (off_16_bytes(kc, vc), (kc, vc)):
+        pending = o.linear_rotary_kv_store(x, w, pos, cos, sin, D, Hq, Hkv, D, *caches, group.slot_mapping, for_attention=True)
+        assert isinstance(pending, ProjectionSums)
+        with counted(o, "attention_bf16", "mie_decode_attention_from_sums", defines=("-DHEAD_DIM=64",)) as calls:
+            out = o.paged_attention(pending, Hq, Hkv, D, *caches, group, step, D ** -0.5, None)
+        assert len(calls) == 1
+        made.append((out, *caches))
+    assert all(torch.equal(a, b) for a, b in zip(*made))
 
 
 @pytest.mark.parametrize("window", [None, 1, 130])
