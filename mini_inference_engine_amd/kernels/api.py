@@ -44,7 +44,7 @@ class Normed:
         return (n, self.residual.shape[1])
 
     def materialize(self, out_dtype=None):
-        if self._value is None:
+        if self._value is None or (self.pending is None and out_dtype not in (None, self._value.dtype)):
             self._value = self.ops.add_rmsnorm(self.pending, self.residual, self.weight, self.eps,
                                                out_dtype=out_dtype, rows=self.rows)
             if self.rows is None:

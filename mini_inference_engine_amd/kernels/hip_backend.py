@@ -257,9 +257,10 @@ class HipBackend(KernelBackend):
 
     def _f32_add_norm(self, x, w, sink):
         """The product added into the sink's stream and the norm that reads it next where the kernel that joins the product's
-        parts makes that norm too; None: nothing is done, the product and the norm are on their own."""
+        parts makes that norm too (in float32: where that is what this backend's norms are in); None: nothing is done, the product
+        and the norm are on their own."""
         g, (M, K), N = sink.norm_weight, x.shape, w.shape[0]
-        if (g is None or g.dtype not in (torch.bfloat16, torch.float32) or tuple(g.shape) != (N,) or not g.is_contiguous()
+        if (self.act_dtype != torch.float32 or g is None or g.dtype not in (torch.bfloat16, torch.float32) or tuple(g.shape) != (N,) or not g.is_contiguous()
                 or g.data_ptr() % 16):
             return None
         lib = self.lib("gemm_f32")

@@ -538,6 +538,20 @@ def test_float32_product_with_the_norm_behind_it(ops, case, g_dtype):
     assert lib.mie_gemm_f32_add_norm(x.data_ptr(), K, w.data_ptr(), K, stream.data_ptr(), g.data_ptr(), 1, None, x.data_ptr(), M, N, K, 1e-5, None) != 0
 
 
+@pytest.mark.parametrize("M", [4, 100])
+def test_the_norm_behind_a_float32_product_is_of_the_wanted_type(ops, M):
+    """The norm that a float32 product's last kernel makes beside the add: of the backend's type where none is asked for, of another
+    where that is, the bits of the norm by itself."""
+    from mini_inference_engine_amd.kernels.api import Sink
+    torch.manual_seed(M)
+    x, w, g = torch.randn(M, 2048, device=DEV), torch.randn(256, 2048, device=DEV) / 45, torch.randn(256, device=DEV)
+    for dtype, asked in ((torch.float32, None), (torch.float32, torch.bfloat16), (torch.bfloat16, None), (torch.bfloat16, torch.float32)):
+        stream = torch.randn(M, 256, device=DEV)
+        y = ops[dtype].linear(x, w, out_dtype=torch.float32, add_to=Sink(stream, g, 1e-5)).materialize(asked)
+        assert y.dtype == (asked or dtype)
+        assert torch.equal(y, ops[dtype].add_rmsnorm(None, stream, g, 1e-5, out_dtype=y.dtype))
+
+
 # rows, K, columns and the tiles of 16 weight rows a workgroup has
 @pytest.mark.parametrize("case", [(17, 64, 4, 1), (33, 72, 12, 1), (64, 2008, 3000, 2), (48, 328, 5632, 3), (128, 2048, 5632, 3),
                                   (50, 8, 8188, 4), (97, 200, 8192, 4), (31, 136, 11008, 6), (64, 192, 11004, 6), (64, 256, 14336, 7)])
