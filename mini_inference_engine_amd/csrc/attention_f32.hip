@@ -168,6 +168,88 @@ __device__ __forceinline__ void load_queries(const AttArgs& a, int t, int h, f32
   }
 }
 
+// A segment's m, l and o join what the 16 queries have so far.
+template <int DT>
+__device__ __forceinline__ void join_segment(float& M, float& L, f32x4 (&O)[DT], float m, float l, const f32x4 (&o)[DT]) {
+  float wa, wb;
+  join_weights(M, m, wa, wb);
+  L = joined(L, wa, l, wb);
+#pragma unroll
+  for (int c = 0; c < DT; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) O[c][i] = joined(O[c][i], wa, o[c][i], wb);
+}
+
+__device__ __forceinline__ int first_key(const AttArgs& a, int p) { return a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0; }
+
+// All over again, one token after the other (values of the row's later tokens, or, beside padding tokens, of slots of its last page that
+// nobody wrote, are not finite): the same bits for what is a number.  The tile's tokens are at positions p0 .. last.
+template <int DT>
+__device__ __forceinline__ void one_by_one(const AttArgs& a, const int* bt, int kvh, const f32x4 (&qf)[DT], int pos, int lo, int p0, int last,
+                                           float& M, float& L, f32x4 (&O)[DT]) {
+  M = -INFINITY;
+  L = 0.f;
+#pragma unroll
+  for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int p = p0; p <= last; ++p) {
+    const bool mine = pos == p;
+    const int f = first_key(a, p);
+#pragma unroll 1
+    for (int seg = f / AF_SEG; seg * AF_SEG <= p; ++seg) {
+      float m, l;
+      f32x4 o[DT];
+      bool again;                             // (of no account: all queries are one token's)
+      segment_sums<DT>(a, bt, kvh, seg, qf, mine ? pos : -1, lo, f, p, f, p, m, l, o, again);
+      if (mine) join_segment<DT>(M, L, O, m, l, o);
+    }
+  }
+}
+
+// O[c][i] of lane (r16, g): dim 16 c + 4 g + i of the lane's query, head h of token t
+template <int DT>
+__device__ __forceinline__ void store_result(const AttArgs& a, float* out, int t, int h, float L, const f32x4 (&O)[DT]) {
+  const int g = (threadIdx.x & 63) >> 4;
+  const float inv = 1.0f / L;
+  float* op = out + ((size_t)t * a.Hq + h) * DT * 16 + 4 * g;
+#pragma unroll
+  for (int c = 0; c < DT; ++c) *reinterpret_cast<f32x4*>(op + 16 * c) = O[c] * inv;
+}
+
+// A portion by single waves: wave (tile of per_tile tokens, the last first: they see the most keys; kv head and tile of 16 heads; row) reads
+// every segment for itself.  The same bits as portion_f32_kernel, by addresses of any size: for pages whose offsets take more than 32 bits.
+template <int DT>
+__global__ void __launch_bounds__(64)
+portion_alone_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ row_start, const int* __restrict__ row_position,
+                         int row0, int per_tile) {
+  const int row = row0 + blockIdx.z, begin = row_start[row], n = row_start[row + 1] - begin;
+  const int rep = a.Hq / a.Hkv, head_tiles = per_tile > 1 ? 1 : (rep + 15) / 16;
+  const int kvh = blockIdx.y / head_tiles, h0 = (blockIdx.y - kvh * head_tiles) * 16;
+  const int t0 = (gridDim.x - 1 - blockIdx.x) * per_tile;
+  if (t0 >= n) return;
+  const int r16 = threadIdx.x & 15;
+  const int ti = per_tile > 1 ? r16 / rep : 0, hi = per_tile > 1 ? r16 - ti * rep : h0 + r16;
+  const bool live = hi < rep && ti < per_tile && t0 + ti < n;
+  const int t = live ? begin + t0 + ti : -1, h = kvh * rep + hi;
+  const int p0 = row_position[row] + t0, last = p0 + (n - t0 < per_tile ? n - t0 : per_tile) - 1;
+  const int first = first_key(a, p0), pos = live ? p0 + ti : -1, lo = first_key(a, pos);
+  const int* bt = a.block_tables + (size_t)row * a.max_blocks;
+  f32x4 qf[DT], O[DT];
+  load_queries<DT>(a, t, h, qf);
+  float M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bool odd = false;
+  for (int seg = first / AF_SEG; seg * AF_SEG <= last && !odd; ++seg) {
+    float m, l;
+    f32x4 o[DT];
+    segment_sums<DT>(a, bt, kvh, seg, qf, pos, lo, first, last, first_key(a, last), p0, m, l, o, odd);
+    join_segment<DT>(M, L, O, m, l, o);
+  }
+  if (odd) one_by_one<DT>(a, bt, kvh, qf, pos, lo, p0, last, M, L, O);
+  if (live) store_result<DT>(a, out, t, h, L, O);
+}
+
 // A portion's workgroup: AF_TILE_WAVES tiles of 16 queries side by side.  Up to head size 64 two waves a tile take the segments in turn, two
 // at a time; the second hands m, l and O to the first, which joins all in order: 512 tokens of 32 / 4 heads of 64 35.0 us with one
 // wave, 30.0 with two (33.1 with one of them at its scores while the other is at its values).  Beyond, the LDS holds no two segments
@@ -195,7 +277,7 @@ portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ r
   const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int T0 = tile * AF_TILE_WAVES * per_tile;
   if (T0 >= n) return;
-  const auto first_of = [&](int p) { return a.window > 0 && p - a.window + 1 > 0 ? p - a.window + 1 : 0; };
+  const auto first_of = [&](int p) { return first_key(a, p); };
   // of the workgroup's queries, and of this wave's (none: last before first)
   const int all_last = row_position[row] + T0 + (n - T0 < AF_TILE_WAVES * per_tile ? n - T0 : AF_TILE_WAVES * per_tile) - 1;
   const int all_first = first_of(row_position[row] + T0);
@@ -275,27 +357,18 @@ portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ r
   f32x4 s[AF_TILES];
   float m = 0.f, l = 0.f;
   bool odd = false;
-  auto join = [&](float m, float l, const f32x4 (&o)[DT]) {
-    float wa, wb;
-    join_weights(M, m, wa, wb);
-    L_sum = joined(L_sum, wa, l, wb);
-#pragma unroll
-    for (int c = 0; c < DT; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) O[c][i] = joined(O[c][i], wa, o[c][i], wb);
-  };
   // what the other side made of its segment, a barrier after it did: the next time it writes is two barriers on
   float* exchange = reinterpret_cast<float*>(af_lds + RING * SIDES * BUFFER) + wave * (4 * DT + 3) * 64 + lane;
   auto join_other = [&](int seg) {
     const int base = (seg0 + seg) * AF_SEG;
-    if ( base > last || base + AF_SEG <= first) return;
+    if (base > last || base + AF_SEG <= first) return;
     f32x4 o[DT];
 #pragma unroll
     for (int c = 0; c < DT; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[c][i] = exchange[(4 * c + i) * 64];
     odd |= exchange[(4 * DT + 2) * 64] != 0.f;
-    join(exchange[4 * DT * 64], exchange[(4 * DT + 1) * 64], o);
+    join_segment<DT>(M, L_sum, O, exchange[4 * DT * 64], exchange[(4 * DT + 1) * 64], o);
   };
   for (int p = 0; p < steps; ++p) {
     if (p + RING - 1 <= steps) MIE_VMCNT((RING - 2) * L);
@@ -360,7 +433,7 @@ portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ r
         exchange[(4 * DT + 2) * 64] = bad ? 1.f : 0.f;
       } else {
         odd |= bad;
-        join(m, l, o);
+        join_segment<DT>(M, L_sum, O, m, l, o);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // this wave has read the buffer before the next barrier
@@ -371,33 +444,8 @@ portion_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ r
     if (side) return;
     join_other(steps - 1);                    // (the pair's second segment; not there: seen by nobody)
   }
-  if (odd) {
-    // (values of the row's later tokens, or, beside padding tokens, of slots of its last page that nobody wrote)  All over
-    // again, one token after the other: the same bits for what is a number
-    M = -INFINITY;
-    L_sum = 0.f;
-#pragma unroll
-    for (int c = 0; c < DT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int q = p0; q <= last; ++q) {
-      const bool mine = pos == q;
-      const int f = first_of(q);
-#pragma unroll 1
-      for (int seg = f / AF_SEG; seg * AF_SEG <= q; ++seg) {
-        float sm, sl;
-        f32x4 o[DT];
-        bool again;                           // (of no account: all queries are one token's)
-        segment_sums<DT>(a, bt, kvh, seg, qf, mine ? pos : -1, lo, f, q, f, q, sm, sl, o, again);
-        if (mine) join(sm, sl, o);
-      }
-    }
-  }
-  if (!live) return;
-  const float inv = 1.0f / L_sum;
-  // O[c][i] of lane (r16, g): dim 16 c + 4 g + i of the lane's query
-  float* op = out + ((size_t)t * a.Hq + h) * D + 4 * g;
-#pragma unroll
-  for (int c = 0; c < DT; ++c) *reinterpret_cast<f32x4*>(op + 16 * c) = O[c] * inv;
+  if (odd) one_by_one<DT>(a, bt, kvh, qf, pos, lo, p0, last, M, L_sum, O);
+  if (live) store_result<DT>(a, out, t, h, L_sum, O);
 }
 
 // Single tokens: wave (split, kv head and tile of 16 heads, token).  Segment first / 128 + split of the token's keys;
@@ -660,7 +708,13 @@ MIE_EXPORT int mie_attention_f32_portions(const float* q, long q_stride, const f
   if (Hkv * head_tiles > 65535 || rows - row0 > 65535) MIE_FAIL("attention_f32: %d kv heads, %d rows are beyond the grid", Hkv, rows - row0);
   const int tiles = (max_row_tokens + AF_TILE_WAVES * per_tile - 1) / (AF_TILE_WAVES * per_tile);
   if ((long)tiles * Hkv * head_tiles > 0x7FFFFFFF) MIE_FAIL("attention_f32: %d tokens are beyond the grid", max_row_tokens);
-  if (page > 1 << 24) MIE_FAIL("attention_f32: pages of %d", page);                 // 32-bit offsets within a page
+  if (page > 1 << 24) {                       // 32-bit offsets within a page in portion_f32_kernel
+    const dim3 waves((max_row_tokens + per_tile - 1) / per_tile, Hkv * head_tiles, rows - row0);
+#define AF_ALONE(DT) hipLaunchKernelGGL(portion_alone_f32_kernel<DT>, waves, dim3(64), 0, s, a, out, row_start, row_position, row0, per_tile)
+    AF_BY_HEAD(D, AF_ALONE)
+    MIE_CHECK_LAUNCH("attention_f32 portions");
+    return 0;
+  }
   const dim3 grid(tiles * Hkv * head_tiles, rows - row0);
 #define AF_PORTIONS(DT)                                                                                                              \
   {                                                                                                                                  \

@@ -1620,6 +1620,21 @@ def test_attention_float32_few_single_tokens(ops, geom, window):
     torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
 
 
+def test_attention_float32_of_pages_beyond_32_bit_offsets(ops):
+    """A page of more than 2^24 tokens (one holds a whole cache): the bits of the same keys in small pages."""
+    Hq, Hkv, D, ctx, page = 4, 1, 16, 300, (1 << 24) + 16
+    q, kc, vc, group, step = paged_setup([ctx], [140], Hq, Hkv, D, 16, torch.float32, seed=5)
+    want = ops[torch.float32].paged_attention(q, Hq, Hkv, D, kc, vc, group, step, 0.25, None)
+    named = group.block_tables[0, :-(-ctx // 16)].long()
+    k, v = torch.zeros(1, Hkv, page, D, device=DEV), torch.zeros(1, Hkv, D, page, device=DEV)
+    k[0, 0, :16 * named.numel()] = kc[named, 0].reshape(-1, D)
+    v[0, 0, :, :16 * named.numel()] = vc[named, 0].permute(1, 0, 2).reshape(D, -1)
+    one = SimpleNamespace(block_tables=torch.zeros(1, 1, dtype=torch.int32, device=DEV), max_blocks=1)
+    with counted(ops[torch.float32], "attention_f32", "mie_attention_f32_portions") as calls:
+        got = ops[torch.float32].paged_attention(q, Hq, Hkv, D, k, v, one, step, 0.25, None)
+    assert len(calls) == 1 and torch.equal(got, want)
+
+
 def test_attention_float32_of_a_step_that_does_not_describe_its_rows(ops):
     """What the float32 attention reads of a step beyond its tokens is only there to choose a faster kernel: without the longest
     row's length or the largest context, or with row arrays of another type, the result is the same."""
