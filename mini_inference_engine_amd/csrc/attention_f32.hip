@@ -12,8 +12,8 @@
 // of one query, which is what the second product takes as its B operand, key 4 g + i of lane group g in instruction i;
 // K rows and the values (transposed within their page) are used in exactly these 16-byte pieces, a page's
 // 16 keys at a time.
-//   portions: four waves side by side (neighbouring tiles of 16 queries) walk their segments together.  A segment's K, then its V,
-//     come into a ring in the LDS by loads that write it directly, whole cache lines, each read once for all four waves and one to three
+//   portions: a wave by itself where there is little to share (alone()), else four waves side by side (neighbouring tiles of 16
+//     queries) that walk their segments together.  A segment's K, then its V, come into a ring in the LDS by loads that write it directly, whole cache lines, each read once for all four waves and one to three
 //     of them on their way while one is used; the 16-byte blocks of a K row are turned by the row, those of a V row by a quarter of it,
 //     so that the fragment reads spread over all banks.  What bounds it: the longest workgroup's chain of segments, 3.4 us of matrix
 //     instructions and 1.5 of exponentials each.  Read by every wave for itself (16 cache lines a quarter wave and load) it
@@ -217,7 +217,7 @@ __device__ __forceinline__ void store_result(const AttArgs& a, float* out, int t
 }
 
 // A portion by single waves: wave (tile of per_tile tokens, the last first: they see the most keys; kv head and tile of 16 heads; row) reads
-// every segment for itself.  The same bits as portion_f32_kernel, by addresses of any size: for pages whose offsets take more than 32 bits.
+// every segment for itself.  The same bits as portion_f32_kernel, for the steps that alone() names.
 template <int DT>
 __global__ void __launch_bounds__(64)
 portion_alone_f32_kernel(AttArgs a, float* __restrict__ out, const int* __restrict__ row_start, const int* __restrict__ row_position,
@@ -695,12 +695,37 @@ MIE_EXPORT int mie_attention_f32_single(const float* q, long q_stride, const flo
   return 0;
 }
 
+// Whether portions of up to max_row_tokens tokens go to single waves, not to workgroups of AF_TILE_WAVES tiles (max_context: of the longest
+// row, 0: not known).  A page's offsets take more than 32 bits; or
+//  - one segment at most, so that no sides take turns, and two waves a compute unit or small heads: a workgroup's start costs more than the
+//    shared loads save.  Four / one wave, us: 64 tokens of 32 / 4 heads of 64 13.4 / 12.2, of 4 / 2 of 16 8.5 / 7.4, 100 of
+//    32 / 8 of 128 19.4 / 18.8, but four rows of 100 of 32 / 4 of 64 (800 waves) 14.3 / 15.4;
+//  - more workgroups than compute units, whose waves are not all of them needed (rows of few tiles): 64 rows of 8 tokens of 12 / 12
+//    heads of 64 (one tile a workgroup) 34.5 / 14.0, of 32 / 8 of 128 (two) 37.1 / 24.1; behind 700 keys (one) 119.9 / 71.5.
+//    Of three tiles a workgroup, 192 rows of 32 / 4 heads of 64: one segment 39.2 / 40.4, 700 keys 1.47 times as long by one wave.
+// Over 567 steps measured 0.89 of four waves everywhere and 0.91 of one; up to 1.19 of one is left at thousands of tokens of ungrouped heads.
+static bool alone(int rows, int max_row_tokens, int Hq, int Hkv, int D, int page, int max_context) {
+  if (page > 1 << 24) return true;
+  const int rep = Hq / Hkv, per_tile = rep <= 16 ? 16 / rep : 1;
+  const long heads = (long)Hkv * (rep <= 16 ? 1 : (rep + 15) / 16), cu = mie_compute_units();
+  const long tiles = ((long)max_row_tokens + per_tile - 1) / per_tile, groups = (tiles + AF_TILE_WAVES - 1) / AF_TILE_WAVES;
+  const long workgroups = groups * heads * rows;
+  const bool one_segment = max_context > 0 && max_context <= AF_SEG;
+  if (one_segment && (D <= 32 || tiles * heads * rows <= 2 * cu)) return true;
+  if (workgroups <= cu) return false;
+  const int twice = D <= 32 ? 6 : workgroups <= 2 * cu ? 4 : one_segment ? 6 : 5;      // twice the tiles a workgroup up to which
+  return 2 * tiles <= twice * groups;
+}
+MIE_EXPORT int mie_attention_f32_alone(int rows, int max_row_tokens, int Hq, int Hkv, int D, int page, int max_context) {
+  return Hkv > 0 && Hq >= Hkv && alone(rows, max_row_tokens, Hq, Hkv, D, page, max_context);
+}
+
 // Rows [row0, rows) of the step: row r's tokens are [row_start[r], row_start[r + 1]) at positions from row_position[r] on,
-// at most max_row_tokens of them; q and out start at the step's token 0.
+// at most max_row_tokens of them; q and out start at the step's token 0.  max_context: no token is at a position beyond it, or 0.
 MIE_EXPORT int mie_attention_f32_portions(const float* q, long q_stride, const float* k_cache, const float* v_cache, float* out,
                                           const int* block_tables, int max_blocks, const int* row_start, const int* row_position,
                                           int row0, int rows, int max_row_tokens, int Hq, int Hkv, int D, int page, float scale,
-                                          int window, hipStream_t s) {
+                                          int window, int max_context, hipStream_t s) {
   if (rows <= row0 || max_row_tokens <= 0) return 0;
   AttArgs a = {q, q_stride, k_cache, v_cache, block_tables, max_blocks, Hq, Hkv, page, window, scale};
   if (check(a, out, D)) return -1;
@@ -708,7 +733,7 @@ MIE_EXPORT int mie_attention_f32_portions(const float* q, long q_stride, const f
   if (Hkv * head_tiles > 65535 || rows - row0 > 65535) MIE_FAIL("attention_f32: %d kv heads, %d rows are beyond the grid", Hkv, rows - row0);
   const int tiles = (max_row_tokens + AF_TILE_WAVES * per_tile - 1) / (AF_TILE_WAVES * per_tile);
   if ((long)tiles * Hkv * head_tiles > 0x7FFFFFFF) MIE_FAIL("attention_f32: %d tokens are beyond the grid", max_row_tokens);
-  if (page > 1 << 24) {                       // 32-bit offsets within a page in portion_f32_kernel
+  if (alone(rows - row0, max_row_tokens, Hq, Hkv, D, page, max_context)) {
     const dim3 waves((max_row_tokens + per_tile - 1) / per_tile, Hkv * head_tiles, rows - row0);
 #define AF_ALONE(DT) hipLaunchKernelGGL(portion_alone_f32_kernel<DT>, waves, dim3(64), 0, s, a, out, row_start, row_position, row0, per_tile)
     AF_BY_HEAD(D, AF_ALONE)

@@ -1908,7 +1908,7 @@ class HipBackend(KernelBackend):
         if single < T:
             library.check(lib, lib.mie_attention_f32_portions(*caches, _ptr(step.row_start), _ptr(step.row_position), single,
                                                               step.num_rows, longest, Hq, Hkv, D, page, float(scale), window,
-                                                              self._stream()))
+                                                              int(getattr(step, "max_context", 0) or 0), self._stream()))
         return True
 
     def sample(self, logits, temperatures, seeds, counters, out=None):

@@ -54,7 +54,8 @@ register_kernel_module("tile_gemm_bf16", {
 register_kernel_module("attention_f32", {
     "mie_attention_f32_segment": [],
     "mie_attention_f32_single": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, P, P],
-    "mie_attention_f32_portions": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, P],
+    "mie_attention_f32_alone": [I, I, I, I, I, I, I],
+    "mie_attention_f32_portions": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, I, P],
 })
 register_kernel_module("grouped_gemm", {
     "mie_grouped_linear": [P, I, L, L, I, P, I, L, L, P, I, L, L, P, P, L, P, P, I, I, I, I, I, I, P, P],

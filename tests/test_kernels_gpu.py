@@ -1620,6 +1620,38 @@ def test_attention_float32_few_single_tokens(ops, geom, window):
     torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
 
 
+# heads, kv heads, head size, page, rows, their tokens, keys before them: one segment at most; rows of one, two and a half and three tiles a
+# workgroup in more workgroups than there are compute units
+@pytest.mark.parametrize("window", [None, 37])
+@pytest.mark.parametrize("case", [(32, 4, 64, 16, 1, 128, 0), (40, 2, 16, 16, 3, 100, 28), (16, 1, 128, 16, 2, 33, 50), (12, 12, 64, 16, 32, 16, 250),
+                                  (32, 8, 128, 16, 40, 20, 300), (6, 2, 112, 16, 129, 5, 200), (3, 1, 32, 16, 300, 13, 130), (8, 2, 48, 48, 260, 9, 0)])
+def test_attention_float32_portions_by_single_waves(ops, case, window):
+    """Portions that single waves take against the same ones by workgroups of four tiles (a few of the rows, the context not said): the
+    same bits, also beside a later token's keys and values that are not finite; and against 64 bits."""
+    Hq, Hkv, D, page, rows, new, have = case
+    o, few, scale = ops[torch.float32], min(rows, 4), 1 / math.sqrt(D)
+    q, kc, vc, group, step = paged_setup([have + new] * rows, [new] * rows, Hq, Hkv, D, page, torch.float32, seed=D)
+    alone = o.lib("attention_f32").mie_attention_f32_alone
+    assert alone(rows, new, Hq, Hkv, D, page, have + new) == 1 and alone(few, new, Hq, Hkv, D, page, 0) == 0
+    part = SimpleNamespace(token_row=step.token_row[:few * new], positions=step.positions[:few * new], num_rows=few, max_context=0, num_tokens=few * new,
+                           num_decode_rows=0, max_row_tokens=new, row_start=step.row_start[:few + 1], row_position=step.row_position[:few])
+    tables = SimpleNamespace(block_tables=group.block_tables[:few].contiguous(), max_blocks=group.max_blocks)
+    out, expect = run_attention(ops, torch.float32, q, kc, vc, group, step, Hq, Hkv, D, scale, window)
+    torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
+    last = have + new - 1
+    for spoilt in (False, True):
+        if spoilt:
+            pages = group.block_tables[:, last // page].long()
+            kc[pages, :, last % page] = float("inf")
+            vc[pages, :, :, last % page] = float("nan")
+        a = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, scale, window)[:few * new]
+        b = o.paged_attention(q[:few * new], Hq, Hkv, D, kc, vc, tables, part, scale, window)
+        assert torch.equal(torch.nan_to_num(a, 7.0), torch.nan_to_num(b, 7.0))
+        assert spoilt or torch.equal(a, out[:few * new])
+        seen = a.view(few, new, -1)[:, :-1]
+        assert bool(torch.isfinite(seen).all()) and (not spoilt or torch.equal(seen, out.view(rows, new, -1)[:few, :-1]))
+
+
 def test_attention_float32_of_pages_beyond_32_bit_offsets(ops):
     """A page of more than 2^24 tokens (one holds a whole cache): the bits of the same keys in small pages."""
     Hq, Hkv, D, ctx, page = 4, 1, 16, 300, (1 << 24) + 16
