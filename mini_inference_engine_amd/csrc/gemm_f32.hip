@@ -585,8 +585,11 @@ reduce_f32_kernel(const float* __restrict__ part, float* __restrict__ out, long 
 
 // The same joined into the 32-bit stream [M, N], with the RMSNorm that reads the stream next: y [M, N] = stream * rsqrt(mean(stream^2) +
 // eps) * g.  A workgroup a row; threads, groups of four and the order of the squares' sum are those of the add + norm kernel
-// (embed_norm.hip), so a row has the same bits whichever of the two makes it.
-constexpr int GF_NORM_THREADS = 256, GF_NORM_MOST = 4 * GF_NORM_THREADS * 8;
+// (embed_norm.hip), so a row has the same bits whichever of the two makes it.  Rows of up to 4,096 numbers: of more, a thread's eight
+// groups and their parts do not fit the registers, and joining by itself has more workgroups than rows (product, add and norm, this
+// kernel / two: 20 rows of [6144, 2048] 28.3 / 25.4 us, of [8192, 2048] 32.0 / 28.9, of [5120, 13824] 88.0 / 85.5; 512 rows of [5120, 5120]
+// 193.5 / 189.0; but of [4096, 4096] 20 rows 27.7 / 28.4, 512 113.3 / 116.8).
+constexpr int GF_NORM_THREADS = 256, GF_NORM_MOST = 4 * GF_NORM_THREADS * 4;
 __device__ __forceinline__ f32x4 norm_weight4(const float* g) { return *reinterpret_cast<const f32x4*>(g); }
 __device__ __forceinline__ f32x4 norm_weight4(const bf16* g) {
   const uint2 u = *reinterpret_cast<const uint2*>(g);
@@ -836,10 +839,9 @@ MIE_EXPORT int mie_gemm_f32_add_norm(const float* X, long ldx, const float* W, l
 #define GF_NORM(PARTS, TW, VEC)                                                                                                  \
   hipLaunchKernelGGL((reduce_add_norm_kernel<PARTS, TW, VEC>), dim3(M), dim3(GF_NORM_THREADS), 0, s, part, stream, (const TW*)g, y, M, N, \
                      eps, X, ldx, W, ldw, K)
-#define GF_NORM_VEC(PARTS, TW)                 \
-  if (groups <= 2) GF_NORM(PARTS, TW, 2);      \
-  else if (groups <= 4) GF_NORM(PARTS, TW, 4); \
-  else GF_NORM(PARTS, TW, 8)
+#define GF_NORM_VEC(PARTS, TW)            \
+  if (groups <= 2) GF_NORM(PARTS, TW, 2); \
+  else GF_NORM(PARTS, TW, 4)
   if (units == 4) {
     if (g_f32) { GF_NORM_VEC(4, float); } else { GF_NORM_VEC(4, bf16); }
   } else {
