@@ -22,6 +22,8 @@
 // x.  Measured alone (MI355X, us, 1 / 8 / 16 rows, before and now): [2048, 2048] 4.5 / 4.7 / 5.1 and 4.1 / 4.5 / 4.9, [2048, 5632] 7.8 /
 // 8.2 / 9.7 and 7.0 / 7.9 / 9.6, [11264, 2048] 10.2 / 10.2 / 11.1 and 9.6 / 9.7 / 9.9, [32000, 2048] 24.9 / 25.1 / 27.2 and 21.7 / 21.3 /
 // 22.1, [6144, 4096] 11.4 / 12.6 / 14.4 and 10.8 / 11.2 / 12.3, [28672, 4096] 38.9 / 40.3 / 42.0 and 37.4 / 37.9 / 39.3.
+// With the norm in front fused in, as the engine runs them: [11264, 2048] 10.0 / 10.7 / 10.9, [32000, 2048] 23.3 / 24.5 / 26.5, [6144, 4096]
+// 11.7 / 12.5 / 14.4, [28672, 4096] 38.0 / 40.8 / 45.4.
 //
 // Epilogues: STORE (bfloat16 or float32 y), ADD (r[m, n] += y, the residual add of the 32-bit stream),
 //   SWIGLU (W holds gate rows then up rows; a tile is 8 gate rows and the matching 8 up rows, and the
@@ -107,7 +109,6 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
   static_assert((SLOTS - 1) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(1024) char ring_lds[];       // SLOTS slots a wave
   __shared__ float s_acc[TW][SG_WAVES][256];
-  __shared__ float s_rstd[16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kb = lane >> 4;
   const int tile0 = blockIdx.x * TW;
@@ -262,8 +263,9 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
   last(std::integral_constant<int, 1>());
   last(std::integral_constant<int, 0>());
 
+  float rstd = 1.f;
   if (NF && EPI != EPI_ADD) {
-    // 1 / sqrt(mean of squares + eps) of every row, summed in a fixed order
+    // 1 / sqrt(mean of squares + eps) of this thread's row, summed in a fixed order by the row's 16 lanes
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < SSP; ++i) {
@@ -278,14 +280,13 @@ skinny_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     sum += __shfl_xor(sum, 2, 64);
     sum += __shfl_xor(sum, 4, 64);
     sum += __shfl_xor(sum, 8, 64);
-    if (c == 0) s_rstd[m] = 1.0f / sqrtf(sum * nf.inv_width + nf.eps);
+    rstd = 1.0f / sqrtf(sum * nf.inv_width + nf.eps);
   }
 
   // sum the waves: acc[i] of lane (col, kb) is weight row 4 kb + i (column of the tile), x row col
 #pragma unroll
   for (int a = 0; a < TW; ++a) *reinterpret_cast<f32x4*>(&s_acc[a][wave][lane * 4]) = acc[a];
   __syncthreads();
-  const float rstd = NF && EPI != EPI_ADD ? s_rstd[m] : 1.f;
 #pragma unroll
   for (int a = 0; a < TW; ++a) {
     const long n = n_of[a];
@@ -352,13 +353,14 @@ MIE_EXPORT int mie_skinny_max_rows() { return 16; }
 
 template <bool NF, int TW, int XT, int SLOTS>
 static int launch_epi(int epi, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
-                      long ldo, int M, int N, int K, int up_offset, int tiles, const RopeArgs& rope, const NormArgs& nf) {
+                      long ldo, int M, int N, int K, int up_offset, int tiles, const RopeArgs& rope, const NormArgs& nf, int* held) {
   constexpr int lds = SG_WAVES * SLOTS * (2 * TW + XT) * 1024;
   const dim3 grid((tiles + TW - 1) / TW);
 #define SG_LAUNCH(E)                                                                                                    \
   {                                                                                                                     \
     auto kernel = skinny_gemm_kernel<E, NF, TW, XT, SLOTS>;                                                             \
     if (mie_allow_lds((const void*)kernel, lds, "skinny_gemm")) return -1;                                              \
+    if (held) return hipOccupancyMaxActiveBlocksPerMultiprocessor(held, kernel, SG_THREADS, lds) == hipSuccess ? 0 : -1; \
     hipLaunchKernelGGL(kernel, grid, dim3(SG_THREADS), lds, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, tiles, rope, nf); \
   }
   switch (epi) {
@@ -391,16 +393,19 @@ static int tiles_for(int M, int tiles) {
 }
 
 static int launch_rows(int tiles, int epi, hipStream_t s, const bf16* X, long ldx, const bf16* W, long ldw, void* out,
-                       long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& n, bool fused) {
+                       long ldo, int M, int N, int K, int up_offset, const RopeArgs& rope, const NormArgs& n, bool fused,
+                       int* held = nullptr) {        // held: nothing is launched, the workgroups that a compute unit holds at once
   const int tw = tiles_for(M, tiles);
-#define SG_ROWS(NF, TW, XT, SLOTS) return launch_epi<NF, TW, XT, SLOTS>(epi, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, tiles, rope, n)
+#define SG_ROWS(NF, TW, XT, SLOTS) return launch_epi<NF, TW, XT, SLOTS>(epi, s, X, ldx, W, ldw, out, ldo, M, N, K, up_offset, tiles, rope, n, held)
 #define SG_TILES(TW, XT, SLOTS)                  \
   {                                              \
     if (fused) SG_ROWS(true, TW, XT, SLOTS);     \
     SG_ROWS(false, TW, XT, SLOTS);               \
   }
-  // Slots: what lets a compute unit have its workgroups at once (48 to 72 KB each); one more where it has a single one ([2048, 5632] at 1
-  // row: four slots 8.1 us, five 7.1).
+  // Slots: what lets a compute unit have its workgroups at once (two of 80 KB at most, the waves' sums with them, or three of 52);
+  // one more where it has a single one ([2048, 5632] at 1 row: four slots 8.1 us, five 7.1).  So nothing else is in the LDS: with 64 bytes
+  // more, for the rows' factors, a compute unit held one workgroup of two tiles and 9 to 16 rows behind a norm ([28672, 4096] at 9 rows 46.2
+  // us for 42.0, [32000, 2048] at 16 30.5 for 26.5).
   if (M <= 8) {
     if (tw == 2) SG_TILES(2, 1, 3);
     if (tiles <= mie_compute_units()) SG_TILES(1, 1, 5);
@@ -458,6 +463,14 @@ MIE_EXPORT int mie_skinny_gemm(const void* X, long ldx, const void* W, long ldw,
   if (!fused && rows) MIE_FAIL("skinny_gemm: a row gather comes with the fused norm only");
   return launch_rows(EPI_GATED(epi) ? (N + 7) / 8 : (N + 15) / 16, epi, s, (const bf16*)X, ldx, (const bf16*)W, ldw, out, ldo, M, N, K, N, none,
                      nf, fused);
+}
+
+// Workgroups of a product of M rows on a weight [N, K] (gated epilogues: N columns of gate and up) that a compute unit holds at once,
+// with a norm fused in or not.
+MIE_EXPORT int mie_skinny_held(int epi, int M, int N, int fused) {
+  int held = 0;
+  const int tiles = EPI_GATED(epi) ? (N + 7) / 8 : (N + 15) / 16;
+  return launch_rows(tiles, epi, nullptr, nullptr, 0, nullptr, 0, nullptr, 0, M, N, 0, N, RopeArgs{}, NormArgs{}, fused != 0, &held) ? -1 : held;
 }
 
 // g sigmoid(alpha g) (u + shift) with g = min(gate, limit), u = clamp(up, -limit, limit); W = [gate rows (N of them); up rows],

@@ -341,6 +341,21 @@ def test_skinny_linear(ops, shape):
     torch.testing.assert_close(stream, expect, atol=2e-3, rtol=2e-3)
 
 
+def test_skinny_workgroups_a_compute_unit_holds(ops):
+    """The LDS of a few-row product's workgroup leaves a compute unit room for as many as its rule counts on: two of two tiles, three
+    of one tile and up to 8 rows, with a norm in front as without one."""
+    lib, cu = ops[torch.bfloat16].lib("gemm_bf16"), torch.cuda.get_device_properties(0).multi_processor_count
+    for epi, columns in ((0, 16), (1, 16), (3, 8), (5, 8)):
+        for fused in (0, 1):
+            for rows in (9, 16):                      # one tile to two a compute unit, and more than three
+                assert lib.mie_skinny_held(epi, rows, columns * 2 * cu, fused) >= 2
+                assert lib.mie_skinny_held(epi, rows, columns * 4 * cu, fused) >= 2
+            for rows in (1, 8):
+                assert lib.mie_skinny_held(epi, rows, columns * 2 * cu, fused) >= 2
+                assert lib.mie_skinny_held(epi, rows, columns * 4 * cu, fused) >= 3
+                assert lib.mie_skinny_held(epi, rows, columns * 20 * cu, fused) >= 2
+
+
 # --------------------------------------------------- products of 17 to 128 rows (bfloat16), split over K
 @pytest.fixture(scope="module")
 def engine_ops():
