@@ -134,17 +134,19 @@ mid_gemm_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W
   }
 
   __syncthreads();                                               // every wave is done with its slots
-  // acc[a][b][i] of lane (col, kb): weight row 4 kb + i of tile a, x row 16 b + col
+  // acc[a][b][i] of lane (col, kb): weight row 4 kb + i of tile a, x row 16 b + col.  PART reads neighbouring columns of a row together, 4 TW
+  // of them for every x row: a lane's place within its 16 turned by 4 a + kb, so that those are in different banks.
+  auto place = [&](int a, int l) { return EPI == MID_PART && TW <= 4 ? l ^ ((4 * a + (l >> 4)) * (4 / TW) & 15) : l; };
   f32x4* sums = reinterpret_cast<f32x4*>(mid_lds);
 #pragma unroll
   for (int a = 0; a < TW; ++a)
 #pragma unroll
-    for (int b = 0; b < MT; ++b) sums[((wave * TW + a) * MT + b) * 64 + lane] = acc[a][b];
+    for (int b = 0; b < MT; ++b) sums[((wave * TW + a) * MT + b) * 64 + place(a, lane)] = acc[a][b];
   __syncthreads();
   auto joined = [&](int a, int b, int l) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < MID_WAVES; ++w) v += sums[((w * TW + a) * MT + b) * 64 + l];
+    for (int w = 0; w < MID_WAVES; ++w) v += sums[((w * TW + a) * MT + b) * 64 + place(a, l)];
     return v;
   };
   if (EPI == MID_SWIGLU) {
