@@ -370,6 +370,13 @@ static int swiglu_tiles(int M, int N) {
 }
 MIE_EXPORT int mie_mid_swiglu_tiles(int M, int N) { return swiglu_tiles(M, N); }
 
+// Whether this product gains over the library's and silu_mul: to 64 rows at every width measured (N of 512 to 28,672, K of 512 to 8,192:
+// 0.44 to 0.99 of their time); beyond, where x is most of what a workgroup brings in, for K up to 2,048 and while the tiles are at most four
+// and a half a compute unit, one round of the grid and a little.  us, library and silu_mul / own, 128 rows: [11264, 2048] 21.7 / 17.4, [16384,
+// 2048] 23.9 / 22.9, [18432, 2048] 33.9 / 33.3, but [28672, 2048] 35.7 / 40.9, [28672, 1024] 21.8 / 24.4, [57344, 1024] 35.2 / 46.3, [22016, 2048]
+// 31.6 / 35.5 (at 65 rows 29.4 / 27.0), [28672, 4096] 59.1 / 65.6, [22016, 4096] 54.0 / 57.3.
+MIE_EXPORT int mie_mid_swiglu_gains(int M, int N, int K) { return M <= 64 || (K <= 2048 && 2L * ((N + 7) / 8) <= 9L * mie_compute_units()); }
+
 // out [M, ldo] bfloat16 = silu(x Wg^T) * (x Wu^T), W = [gate rows (N of them); up rows], N a multiple of 4.
 MIE_EXPORT int mie_mid_swiglu(const void* X, long ldx, const void* W, long ldw, void* out, long ldo, int M, int N, int K, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;

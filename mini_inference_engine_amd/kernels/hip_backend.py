@@ -348,13 +348,11 @@ class HipBackend(KernelBackend):
         return max(1, min(8, 256 // tiles, K // 256))
 
     def _mid_swiglu_ok(self, x, w, intermediate) -> bool:
-        """Whether the own gate/up product with SwiGLU on its sums takes x w^T: from 17 rows on to 64, to 128 up to K = 2,048, where
-        its workgroups still bring in less than the library and silu_mul cost (us, library and silu_mul / own: 64 rows of [28672,
-        4096] 56.9 / 48.6, of [22016, 4096] 48.6 / 37.4, 128 rows 59.1 / 65.6 and 54.0 / 57.3, but of [11264, 2048] 21.7 / 17.4)."""
+        """Whether the own gate/up product with SwiGLU on its sums takes x w^T: 17 to 128 rows where it gains."""
         M = x.shape[0]
-        return (not self.true_fp32 and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and M > self.SKINNY_MAX_ROWS
-                and (M <= 64 or M <= self.MID_MAX_ROWS and w.shape[1] <= 2048) and intermediate % 4 == 0
-                and self._mid_operands_ok(x, w))
+        return (not self.true_fp32 and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
+                and self.SKINNY_MAX_ROWS < M <= self.MID_MAX_ROWS and intermediate % 4 == 0 and self._mid_operands_ok(x, w)
+                and bool(self.lib("gemm_mid_bf16").mie_mid_swiglu_gains(M, intermediate, w.shape[1])))
 
     def _mid_partials(self, x, w):
         """part [splits, M, N] float32 of x w^T."""

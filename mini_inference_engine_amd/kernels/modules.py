@@ -123,6 +123,7 @@ register_kernel_module("gemm_mid_bf16", {
     "mie_mid_splits": [I, I],
     "mie_mid_tile_rows": [I],
     "mie_mid_swiglu_tiles": [I, I],
+    "mie_mid_swiglu_gains": [I, I, I],
     "mie_mid_swiglu": [P, L, P, L, P, L, I, I, I, P],
     "mie_mid_max_rows": [],
 })

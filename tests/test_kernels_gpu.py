@@ -597,6 +597,22 @@ def test_mid_product_swiglu(engine_ops, case):
     assert lib.mie_mid_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 4, M, inter, K - 4, None) != 0
 
 
+@pytest.mark.parametrize("case", [(64, 64, 9220, True), (65, 64, 9216, True), (65, 64, 9220, False), (128, 64, 14336, False), (128, 2048, 5632, True),
+                                  (128, 2056, 512, False)])
+def test_mid_product_swiglu_is_taken_where_it_gains(engine_ops, case):
+    """More than 64 rows of a weight that gives a compute unit more than four and a half tiles, or of a longer K, keep the library's
+    product and silu_mul."""
+    o, (M, K, inter, taken) = engine_ops, case
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    torch.manual_seed(M)
+    x, w = torch.randn(M, K, device=DEV).to(torch.bfloat16), (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    with counted(o, "gemm_mid_bf16", "mie_mid_swiglu") as calls:
+        y = o.linear_silu_mul(x, w, inter)
+    assert len(calls) == taken
+    gu = x.double() @ w.double().T
+    torch.testing.assert_close(y.double(), torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:], atol=2e-2, rtol=2e-2)
+
+
 def test_mid_linear_refuses_what_it_cannot_run(engine_ops):
     o = engine_ops
     lib = o.lib("gemm_mid_bf16")
