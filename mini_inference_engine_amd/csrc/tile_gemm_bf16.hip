@@ -312,17 +312,21 @@ static int check_operands(const void* X, long ldx, const void* W, long ldw, cons
 
 
 // Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: measured at
-// 160 to 2,048 rows of [11264, 2048] (MI355X).  The first five are tile_gemm_kernel's, the others tile_spread_kernel's.  Own tile of
+// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 384, the second 128 x 128 and those behind it are tile_spread_kernel's, the others
+// tile_gemm_kernel's, of which 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  Own tile of
 // before / now, us: 160 rows 25.2 / 22.4, 256 26.0 / 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9;
 // at 1,024 and 1,132 rows 256 x 256 of sixteen waves of 64 x 64 stays (45.6 and 50.5 us; of eight of 64 x 128 54.6 and 53.7).
-constexpr struct { int bm, bn; float us; } TILE_STAGE_US[10] = {
+constexpr struct { int bm, bn; float us; } TILE_STAGE_US[] = {
   {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f},
   {128, 128, 0.72f}, {128, 192, 0.96f}, {192, 192, 1.12f}, {256, 320, 1.94f}};
 
-static int best_tile(int M, long cols, int choices, float& us) {
-  int best = 0;
+constexpr int TILES_TAKEN = 1, TILES_ESTIMATED = 6, TILES = 10;       // taken: from the first on; estimated: those before the second
+
+// of tiles first .. behind - 1 the one with the least time
+static int best_tile(int M, long cols, int first, int behind, float& us) {
+  int best = first;
   us = 1e30f;
-  for (int i = 0; i < choices; ++i) {
+  for (int i = first; i < behind; ++i) {
     const long tiles = (long)((M + TILE_STAGE_US[i].bm - 1) / TILE_STAGE_US[i].bm) * ((cols + TILE_STAGE_US[i].bn - 1) / TILE_STAGE_US[i].bn);
     const long rounds = (tiles + mie_compute_units() - 1) / mie_compute_units();
     if (rounds * TILE_STAGE_US[i].us < us) {
@@ -333,11 +337,20 @@ static int best_tile(int M, long cols, int choices, float& us) {
   return best;
 }
 
-// What mie_tile_gemm_swiglu takes at most, in units of 0.01 us: by the tiles that the decision against the library was measured with.
+// What mie_tile_gemm_swiglu takes at most, in units of 0.01 us, for the decision against the library.  It leaves out the tiles of the spread
+// kernel but 256 x 384: with them the decision, whose estimate of the library is rough, would change for the better at some sizes and
+// for the worse at others (us, own / library / library's kernel chosen by timing: 1,300 rows of [11264, 2048] 63.8 / 71.7 / 72.6, 550 rows
+// 36.2 / 36.7 / 36.8, but 256 rows of [8192, 2048] 22.6 / 24.8 / 19.6).
 MIE_EXPORT int mie_tile_gemm_swiglu_cost(int M, int N, int K) {
   float us;
-  best_tile(M, 2L * N, 6, us);
+  best_tile(M, 2L * N, 0, TILES_ESTIMATED, us);
   return (int)(100.f * us * (K / 64));
+}
+// The tile that mie_tile_gemm_swiglu takes: 1,000 times its rows plus its columns.
+MIE_EXPORT int mie_tile_gemm_swiglu_tile(int M, int N) {
+  float us;
+  const auto& t = TILE_STAGE_US[best_tile(M, 2L * N, TILES_TAKEN, TILES, us)];
+  return t.bm * 1000 + t.bn;
 }
 
 // out [M, ldo] bfloat16 = silu(x Wg^T) * (x Wu^T), W = [gate rows (N of them); up rows].
@@ -347,13 +360,13 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   if (ldo < N || (ldo & 3)) MIE_FAIL("tile_gemm_swiglu: output leading dim %ld for %d columns", ldo, N);
   const bf16 *x = (const bf16*)X, *w = (const bf16*)W;
   float us;
-  switch (best_tile(M, 2L * N, 10, us)) {
+  switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {
     case 1: return launch<3, 2, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 2: return launch<4, 2, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 3: return launch<4, 3, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 4: return launch<4, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 5: return launch_spread<12, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
-    case 0: case 6: return launch_spread<4, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
+    case 6: return launch_spread<4, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 7: return launch_spread<6, 2, 4, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     case 8: return launch_spread<6, 3, 3, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);
     default: return launch_spread<10, 4, 2, TG_SWIGLU>(x, ldx, w, ldw, out, ldo, M, N, K, 1, s);

@@ -47,6 +47,7 @@ register_kernel_module("gemm_f32", {
     "mie_qkv_rope_f32": [P, L, P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, I, P],
 })
 register_kernel_module("tile_gemm_bf16", {
+    "mie_tile_gemm_swiglu_tile": [I, I],
     "mie_tile_gemm_swiglu_cost": [I, I, I],
     "mie_tile_gemm_swiglu": [P, L, P, L, P, L, I, I, I, P],
     "mie_tile_gemm_units": [P, L, P, L, P, I, I, I, I, P],

@@ -455,29 +455,31 @@ def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
         torch.testing.assert_close(stream.double(), want, atol=1e-4, rtol=1e-4)
 
 
-# rows, K, columns; the rounds of the grid times a stage's time of the tile that is taken (128 x 128, 192 x 128, 256 x 128, 256 x 192
-# and 256 x 256 take 0.76, 0.98, 0.99, 1.33 and 1.57 us), and whether the product is better off on the own tiles
-@pytest.mark.parametrize("case", [(129, 64, 104, 0.76, True), (192, 2048, 5632, 0.76, True), (300, 192, 96, 0.76, True),
-                                  (380, 64, 5512, 0.98, True), (510, 128, 5512, 0.99, True), (513, 128, 5640, 1.33, True),
-                                  (1300, 2048, 2816, 1.33, False), (1020, 64, 6152, 1.57, True), (2047, 64, 1000, 0.76, True)])
+# rows, K, columns; the estimate's time of a stage, whether the product is better off on the own tiles by it, and the tile that is taken
+@pytest.mark.parametrize("case", [(129, 64, 104, 0.76, True, 128128), (192, 2048, 5632, 0.76, True, 128128), (300, 192, 96, 0.76, True, 128128),
+                                  (380, 64, 5512, 0.98, True, 128192), (510, 128, 5512, 0.99, True, 128192), (513, 128, 5640, 1.33, True, 192192),
+                                  (1300, 2048, 2816, 1.33, False, 192192), (1020, 64, 6152, 1.57, True, 256256), (2047, 64, 1000, 0.76, True, 128128),
+                                  (525, 64, 5200, 0.98, True, 192128), (1307, 128, 2272, 0.98, True, 192128), (457, 192, 8184, 0.99, True, 256128),
+                                  (959, 64, 3896, 0.99, True, 256128), (690, 128, 7176, 1.33, True, 256192), (1193, 192, 3488, 1.33, True, 256192),
+                                  (1169, 64, 7880, 2.35, True, 256320), (1479, 192, 5976, 2.35, True, 256320)])
 def test_tile_product_swiglu(engine_ops, case):
     """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
     sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
     from mini_inference_engine_amd.kernels import library
-    shape, stage_us, gains = case[:3], case[3], case[4]
-    o, (M, K, inter) = engine_ops, shape
+    (M, K, inter, stage_us, gains, tile), o = case, engine_ops
     torch.manual_seed(K + inter)
     x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
     w = (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
     out = torch.full((M, inter + 8), 7.0, device=DEV, dtype=torch.bfloat16)
     lib = o.lib("tile_gemm_bf16")
+    assert lib.mie_tile_gemm_swiglu_tile(M, inter) == tile, "the case must take the tile it is for"
     library.check(lib, lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K,
                                                 torch.cuda.current_stream().cuda_stream))
     gu = x.double() @ w.double().T
     expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
     assert bool(((out[:, :inter].double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
     assert bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
-    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 100 * stage_us * (K // 64)) <= 1, "the case must take the tile it is for"
+    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 100 * stage_us * (K // 64)) <= 1
     assert o._tile_swiglu_gains(x, w, inter) == gains
     with counted(o, "tile_gemm_bf16", "mie_tile_gemm_swiglu") as calls:
         made = o.linear_silu_mul(x, w, inter)
@@ -518,7 +520,8 @@ def test_wide_tile_product_swiglu(engine_ops, case):
     x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
     w = (torch.randn(2 * inter, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
     lib = o.lib("tile_gemm_bf16")
-    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 235 * (K // 64)) <= 1, "the case must take the tile it is for"
+    assert lib.mie_tile_gemm_swiglu_tile(M, inter) == 256384, "the case must take the tile it is for"
+    assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 235 * (K // 64)) <= 1
     out = torch.full((M, inter + 8), 7.0, device=DEV, dtype=torch.bfloat16)
     library.check(lib, lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 8, M, inter, K,
                                                 torch.cuda.current_stream().cuda_stream))
