@@ -422,7 +422,8 @@ static int check_operands(const char* what, const void* X, long ldx, const void*
   if (M > 16) MIE_FAIL("%s: %d rows (at most 16)", what, M);
   if (K <= 0 || (K & 7)) MIE_FAIL("%s: K = %d must be a positive multiple of 8", what, K);
   if (ldx < K || ldw < K || (ldw & 7) || (ldx & 7)) MIE_FAIL("%s: leading dims %ld, %ld for K %d", what, ldx, ldw, K);
-  if (ldx > 1L << 24 || ldw > 1L << 24) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^24)", what, ldx, ldw);      // 32-bit offsets
+  // 32-bit offsets: of up to 64 gathered rows from x, of 8 weight rows from the first of them
+  if (ldx > 1L << 24 || ldw > 1L << 28) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^24, 2^28)", what, ldx, ldw);
   if (((uintptr_t)X | (uintptr_t)W) & 15) MIE_FAIL("%s: operands must be 16-byte aligned", what);
   return 0;
 }

@@ -333,7 +333,8 @@ static int check_operands(const char* what, const void* X, long ldx, const void*
   if (M > 128) MIE_FAIL("%s: %d rows (at most 128)", what, M);
   if (K <= 0 || (K & 7)) MIE_FAIL("%s: K = %d must be a positive multiple of 8", what, K);
   if (ldx < K || ldw < K || (ldw & 7) || (ldx & 7)) MIE_FAIL("%s: leading dims %ld, %ld for K %d", what, ldx, ldw, K);
-  if (ldx > 1L << 23 || ldw > 1L << 23) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^23)", what, ldx, ldw);      // 32-bit offsets
+  // 32-bit offsets: of up to 128 rows from x, of up to 64 weight rows from a workgroup's first
+  if (ldx > 1L << 24 || ldw > 1L << 24) MIE_FAIL("%s: leading dims %ld, %ld (at most 2^24)", what, ldx, ldw);
   if (((uintptr_t)X | (uintptr_t)W) & 15) MIE_FAIL("%s: operands must be 16-byte aligned", what);
   return 0;
 }

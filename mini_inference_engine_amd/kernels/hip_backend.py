@@ -287,7 +287,7 @@ class HipBackend(KernelBackend):
         m = x.shape[0] if rows is None else rows.shape[0]
         return (not self.true_fp32 and bias is None and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
                 and m <= self.SKINNY_MAX_ROWS and x.shape[0] <= 64 and w.shape[1] % 8 == 0 and w.stride(0) % 8 == 0
-                and x.stride(0) % 8 == 0 and w.stride(0) <= 1 << 24 and x.stride(0) <= 1 << 24
+                and x.stride(0) % 8 == 0 and w.stride(0) <= 1 << 28 and x.stride(0) <= 1 << 24
                 and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
     def _prepared(self, x, w, bias):
@@ -339,7 +339,7 @@ class HipBackend(KernelBackend):
     @staticmethod
     def _mid_operands_ok(x, w) -> bool:
         return (w.shape[0] % 4 == 0 and w.shape[1] % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) % 8 == 0
-                and w.stride(0) <= 1 << 23 and x.stride(0) <= 1 << 23 and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+                and w.stride(0) <= 1 << 24 and x.stride(0) <= 1 << 24 and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
     def mid_splits(self, N: int, K: int) -> int:
         """Splits of K wanted for a weight [N, K]: enough for 256 workgroups of the rows the kernel's workgroups own, each split

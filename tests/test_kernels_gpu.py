@@ -600,6 +600,34 @@ def test_mid_product_swiglu(engine_ops, case):
     assert lib.mie_mid_swiglu(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), inter + 4, M, inter, K - 4, None) != 0
 
 
+def far_rows(t, stride):
+    """The same matrix with its rows ``stride`` numbers apart."""
+    return torch.empty((t.shape[0] - 1) * stride + t.shape[1], dtype=t.dtype, device=DEV).as_strided(t.shape, (stride, 1)).copy_(t)
+
+
+# rows of x, K, weight rows and the strides of both: the largest that the kernels' 32-bit offsets reach
+@pytest.mark.parametrize("case", [(16, 72, 24, 72, 1 << 28), (16, 64, 40, 1 << 24, 64), (128, 136, 100, 136, 1 << 24), (128, 64, 72, 1 << 24, 1 << 24)])
+def test_products_of_rows_far_apart(engine_ops, case):
+    """Few-row and split products whose rows lie as far apart as they take: the bits of compact operands; further apart is refused
+    by the C entries and left to the library by the backend."""
+    o, (M, K, N, ldx, ldw) = engine_ops, case
+    torch.manual_seed(N)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    fx, fw = far_rows(x, ldx), far_rows(w, ldw)
+    ok = o._skinny_ok if M <= 16 else o._mid_ok
+    assert ok(fx, fw, None)
+    assert torch.equal(o.linear(fx, fw, out_dtype=torch.float32), o.linear(x, w, out_dtype=torch.float32))
+    assert torch.equal(o.linear_silu_mul(fx, fw, N // 2), o.linear_silu_mul(x, w, N // 2))
+    y, s = torch.empty(M, N, device=DEV), torch.cuda.current_stream().cuda_stream
+    far = max(ldx, ldw) + 8
+    args = (x.data_ptr(), far if ldx > K else K, w.data_ptr(), far if ldw > K else K)
+    if M <= 16:
+        assert o.lib("gemm_bf16").mie_skinny_gemm(*args, y.data_ptr(), N, 1, M, N, K, None, 0, None, 0, None, None, 0, 0.0, None, s) != 0
+    else:
+        assert o.lib("gemm_mid_bf16").mie_mid_gemm(*args, y.data_ptr(), M, N, K, 1, None, s) != 0
+
+
 @pytest.mark.parametrize("case", [(64, 64, 9220, True), (65, 64, 9216, True), (65, 64, 9220, False), (128, 64, 14336, False), (128, 2048, 5632, True),
                                   (128, 2056, 512, False)])
 def test_mid_product_swiglu_is_taken_where_it_gains(engine_ops, case):
