@@ -466,6 +466,9 @@ MIE_EXPORT int mie_skinny_gemm(const void* X, long ldx, const void* W, long ldw,
                      nf, fused);
 }
 
+// Tiles that a workgroup of such a product has.
+MIE_EXPORT int mie_skinny_tiles(int epi, int M, int N) { return tiles_for(M, EPI_GATED(epi) ? (N + 7) / 8 : (N + 15) / 16); }
+
 // Workgroups of a product of M rows on a weight [N, K] (gated epilogues: N columns of gate and up) that a compute unit holds at once,
 // with a norm fused in or not.
 MIE_EXPORT int mie_skinny_held(int epi, int M, int N, int fused) {

@@ -80,7 +80,7 @@ class HipBackend(KernelBackend):
         if not torch.cuda.is_available():
             raise RuntimeError("no GPU visible to torch: the engine needs an MI355X (gfx950)")
         self._libs = {}
-        self._zeros = None          # 256 zero bytes on the device, what masked loads of the mid-row product read
+        self._zeros = None          # 256 zero bytes on the device, what masked loads of grouped products read
         self._lt_workspace = None   # device memory the library's product kernels may use
         self._lt_rows = set()       # row counts whose library products get their kernel chosen by timing (prefer_rows)
         self._lt_tuned = set()      # (M, N, K, kind, leading dims) already chosen that way
@@ -362,10 +362,7 @@ class HipBackend(KernelBackend):
         wanted = self.mid_splits(N, K)
         splits = lib.mie_mid_splits(K, wanted)
         part = torch.empty((splits, M, N), dtype=torch.float32, device=w.device)
-        if self._zeros is None:
-            self._zeros = torch.zeros(64, dtype=torch.int32, device=w.device)
-        library.check(lib, lib.mie_mid_gemm(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(part), M, N, K, wanted,
-                                            _ptr(self._zeros), self._stream()))
+        library.check(lib, lib.mie_mid_gemm(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(part), M, N, K, wanted, None, self._stream()))
         return part
 
     def _mid_reduce(self, part, mode, out=None, stream=None, g=None, x_next=None, eps=0.0):

@@ -111,6 +111,7 @@ register_kernel_module("sampling", {
     "mie_sample": [P, L, P, P, P, P, I, I, P],
 })
 register_kernel_module("gemm_bf16", {
+    "mie_skinny_tiles": [I, I, I],
     "mie_skinny_held": [I, I, I, I],
     "mie_skinny_gemm": [P, L, P, L, P, L, I, I, I, I, P, I, P, L, P, P, I, F, P, P],
     "mie_skinny_qkv_rope": [P, L, P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, I, P, I, F, P],

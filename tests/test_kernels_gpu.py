@@ -313,8 +313,7 @@ def normed(ops, stream, w_norm, eps, rows=None, pending=None):
     return Normed(ops, pending, stream, w_norm, eps, rows)
 
 
-# (rows, K, N); 9,600 and 12,304 weight rows are 600 and 769 tiles: more than two, and more than three, a compute unit
-# (the kernel's ring is one slot shorter in between); K = 8 and 40: waves without a k-step of their own
+# (rows, K, N); K = 8 and 40: waves without a chunk of their own
 SKINNY_SHAPES = [(1, 64, 176), (7, 200, 331), (16, 2048, 2560), (13, 120, 96), (11, 5632, 2048), (16, 2048, 640),
                  (8, 176, 64), (3, 96, 384), (5, 264, 9600), (9, 72, 12304), (16, 4104, 48), (2, 8, 32), (6, 40, 16)]
 
@@ -339,6 +338,44 @@ def test_skinny_linear(ops, shape):
     expect = stream + ref.ref_linear(x, w, None, torch.float32)
     assert o.linear(x, w, add_to=stream) is None
     torch.testing.assert_close(stream, expect, atol=2e-3, rtol=2e-3)
+
+
+# rows, K, weight rows and the tiles a workgroup has: every number, a last workgroup with fewer and a last tile with fewer rows
+@pytest.mark.parametrize("case", [(12, 136, 9605, 3), (16, 2048, 8200, 3), (9, 72, 12305, 2), (16, 72, 4813, 2), (8, 2120, 4813, 2), (3, 40, 65575, 2),
+                                  (5, 264, 9605, 1), (16, 64, 4090, 1), (8, 1000, 12290, 1)])
+def test_skinny_tiles_a_workgroup(ops, case):
+    """Few-row products by one, two and three tiles a workgroup: plain, added, gated, with a norm in front and behind, and a row's bits by
+    itself, where the tiles are others."""
+    from mini_inference_engine_amd.kernels.api import Sink
+    o, (M, K, N, tiles) = ops[torch.bfloat16], case
+    I = (N + 1) // 2
+    lib = o.lib("gemm_bf16")
+    assert lib.mie_skinny_tiles(o.EPI_F32, M, N) == lib.mie_skinny_tiles(o.EPI_SWIGLU, M, I) == tiles, "the case must take the tiles it is for"
+    torch.manual_seed(N)
+    w, wg = ((torch.randn(n, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16) for n in (N, 2 * I))
+    x, g = torch.randn(M, K, device=DEV).to(torch.bfloat16), 1 + 0.1 * torch.randn(K, device=DEV)
+    y = o.linear(x, w, out_dtype=torch.float32)
+    torch.testing.assert_close(y.double(), x.double() @ w.double().T, atol=1e-4, rtol=1e-4)
+    assert torch.equal(o.linear(x[-1:].contiguous(), w, out_dtype=torch.float32), y[-1:])
+    a = o.linear_silu_mul(x, wg, I)
+    gu = x.double() @ wg.double().T
+    torch.testing.assert_close(a.double(), torch.nn.functional.silu(gu[:, :I]) * gu[:, I:], atol=1e-3, rtol=1e-2)
+    # added, with the norm behind it prepared
+    stream, gn = torch.randn(M, N, device=DEV), 1 + 0.1 * torch.randn(N, device=DEV)
+    want = stream.double() + y.double()
+    behind = o.linear(x, w, add_to=Sink(stream, gn, 1e-5))
+    torch.testing.assert_close(stream.double(), want, atol=1e-5, rtol=1e-5)
+    squares = behind.ready["ss"][:, :behind.ready["tiles"]].double().sum(1)
+    torch.testing.assert_close(squares, want.pow(2).sum(1), atol=0, rtol=1e-5)
+    torch.testing.assert_close(behind.ready["x"].double(), want * gn.double(), atol=1e-2, rtol=2.0 ** -8)
+    # a norm in front
+    first = torch.randn(M, K, device=DEV)
+    front = o.linear(x[:, :8].contiguous(), w[:K, :8].contiguous(), add_to=Sink(first, g, 1e-5))
+    assert front.ready is not None
+    xn = ref.ref_add_rmsnorm(None, first.clone(), g, 1e-5, torch.float64)
+    torch.testing.assert_close(o.linear(front, w, out_dtype=torch.float32).double(), xn @ w.double().T, atol=2e-2, rtol=1e-2)
+    gu = xn @ wg.double().T
+    torch.testing.assert_close(o.linear_silu_mul(front, wg, I).double(), torch.nn.functional.silu(gu[:, :I]) * gu[:, I:], atol=3e-2, rtol=2e-2)
 
 
 def test_skinny_workgroups_a_compute_unit_holds(ops):
