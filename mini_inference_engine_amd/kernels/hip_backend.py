@@ -1707,10 +1707,13 @@ class HipBackend(KernelBackend):
     @staticmethod
     def _pages_of_portions(k_cache, v_cache, bt, step, page):
         """The pages that the step's rows of several tokens name, each row's side by side in memory of their own (16-byte aligned),
-        and block tables for them; both caches are only read."""
-        first, rows = step.num_decode_rows, step.num_rows
+        and block tables for them; the whole caches and the step's tables where rows times the longest would be as many pages or more.
+        Both caches are only read."""
+        first, rows, pages = step.num_decode_rows, step.num_rows, k_cache.shape[0]
         most = min(bt.shape[1], -(-step.max_context // page)) if step.max_context > 0 else bt.shape[1]
-        named = bt[first:rows, :most].reshape(-1)
+        if (rows - first) * most >= pages:
+            return k_cache.clone(), v_cache.clone(), bt
+        named = bt[first:rows, :most].reshape(-1).clamp(0, pages - 1)       # (behind a row's own pages a table holds anything)
         table = torch.zeros((rows, bt.shape[1]), dtype=torch.int32, device=bt.device)
         table[first:, :most] = torch.arange(named.shape[0], dtype=torch.int32, device=bt.device).view(rows - first, most)
         return k_cache.index_select(0, named), v_cache.index_select(0, named), table
