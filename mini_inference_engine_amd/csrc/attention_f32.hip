@@ -199,7 +199,7 @@ __device__ __forceinline__ void one_by_one(const AttArgs& a, const int* bt, int 
     for (int seg = f / AF_SEG; seg * AF_SEG <= p; ++seg) {
       float m, l;
       f32x4 o[DT];
-      bool again = false;                     // (of no account: all queries are one token's)
+      bool again;                             // (of no account: all queries are one token's)
       segment_sums<DT>(a, bt, kvh, seg, qf, mine ? pos : -1, lo, f, p, f, p, m, l, o, again);
       if (mine) join_segment<DT>(M, L, O, m, l, o);
     }
