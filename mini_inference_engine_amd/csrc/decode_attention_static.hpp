@@ -32,7 +32,8 @@ MIE_EXPORT int mie_decode_attention_static_setup(void);
 // the array's size in bytes
 MIE_EXPORT long mie_decode_attention_static_capacity(void);
 
-// Arguments as mie_decode_attention without o_part and lse_part.
+// Arguments as mie_decode_attention without o_part and lse_part: q on 16 bytes; the caches at any address of a number, on 16 bytes
+// read through the LDS at head sizes 64, 96 and 128, else through registers, with the same bits.
 MIE_EXPORT int mie_decode_attention_static(const void* q, long q_stride, const void* k_cache, const void* v_cache,
                                            void* out, const int* block_tables, int max_blocks, const int* positions,
                                            int rows, int Hq, int Hkv, int head_dim, int page, float scale, int window,

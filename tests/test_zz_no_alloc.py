@@ -85,6 +85,29 @@ def test_static_decode_attention_equals_the_one_with_buffers():
         torch.testing.assert_close(out_b.double(), expect, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("splits", [1, 5])
+@pytest.mark.parametrize("behind", [8, 2])
+def test_static_decode_attention_takes_caches_off_16_bytes(splits, behind):
+    """Caches that begin ``behind`` bytes into memory, whole and split contexts, a workgroup's eight waves and four: the bits of the same
+    keys and values on 16 bytes."""
+    lib = _library()
+    assert lib.mie_decode_attention_static_setup() == 0, lib.attention_bf16_last_error()
+    for rows in (3, 70):
+        q, kc, vc, group, step = paged_setup([1 + 97 * r % 620 for r in range(rows)], [1] * rows, Hq, Hkv, D, PAGE, torch.bfloat16, seed=rows)
+        partition, n = _split(lib, 620, splits)
+        made = []
+        for skipped in (0, behind // 2):
+            k, v = (torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")[skipped:skipped + t.numel()].view(t.shape).copy_(t) for t in (kc, vc))
+            assert k.data_ptr() % 16 == v.data_ptr() % 16 == 2 * skipped
+            out = torch.zeros(rows, Hq * D, dtype=torch.bfloat16, device="cuda")
+            rc = lib.mie_decode_attention_static(*(c_void_p(q.data_ptr()), q.stride(0)), *(c_void_p(t.data_ptr()) for t in (k, v, out, group.block_tables)),
+                                                 group.block_tables.shape[1], c_void_p(step.positions.data_ptr()), rows, Hq, Hkv, D, PAGE,
+                                                 1 / math.sqrt(D), 0, partition, n, c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0, lib.attention_bf16_last_error()
+            made.append(out)
+        assert n == splits and torch.equal(*made)
+
+
 def test_static_decode_attention_inside_a_captured_graph():
     """The use the entry point is for: set-up once, then the call recorded into a graph (where an allocation is
     an error that ends the capture) and replayed with other inputs in the same buffers, with eager work and
