@@ -487,8 +487,7 @@ single_f32_kernel(AttArgs a, float* __restrict__ out, float* __restrict__ o_part
 // keys, all of them meet in the LDS, every wave adds them up as one wave would, and a wave takes every fourth tile of 16 dims of the
 // values.  4 tokens of 300 to 900 keys of 32 / 4 heads of 64 13.6 us with one wave and the kernel that joins, 10.0 with four; where the
 // segments are many, one wave each has less to exchange (64 tokens of 2,000 keys of 4 / 2 heads of 16: 15.2 and 20.9; 16 of 900
-// of 32 / 8 heads of 128: 34.6 and 37.4), so four take up to AF_FEW segments.
-constexpr long AF_FEW = 1024;
+// of 32 / 8 heads of 128: 34.6 and 37.4): four_waves() draws the line.
 constexpr int AF_SINGLE_WAVES = 4;
 template <int DT>
 __global__ void __launch_bounds__(AF_SINGLE_WAVES * 64)
@@ -668,6 +667,20 @@ static int check(const AttArgs& a, const void* out, int D) {
   return 0;
 }
 
+// Whether a segment of single tokens is four waves' work: while the segments are at most so many a compute unit.  The waves take tiles of
+// 16 dims in fours, so the fewer a head has, and 80 and 96 that take eight for five or six, the sooner one wave each is the better; and
+// the sooner where tokens have one segment, often a short one.  Four waves / one, at 1, 2, 3 and 4 segments a compute unit (MI355X, 80
+// shapes a head size; in brackets of one segment): 16 0.86, 1.01, 1.15, 1.29; 32 0.80, 0.91, 1.02, 1.09; 48 0.74, 0.86, 0.95, 1.01 (1.05); 64
+// 0.71, 0.82, 0.92, 0.97; 80 0.69, 0.86, 0.98 (1.01), 1.06; 96 0.67, 0.85, 0.99 (1.01), 1.05; 112 0.61, 0.78, 0.91, 0.98; 128 0.61, 0.80, 0.93, 0.99.
+static bool four_waves(int tokens, int Hq, int Hkv, int D, int splits) {
+  constexpr int most[2][8] = {{1, 2, 4, 4, 3, 3, 4, 4}, {1, 2, 3, 4, 2, 2, 4, 4}};      // of head size 16, 32, ...; the second: one segment
+  if (D < 16 || D > 128) return false;
+  return (long)splits * Hkv * ((Hq / Hkv + 15) / 16) * tokens <= (long)most[splits == 1][D / 16 - 1] * mie_compute_units();
+}
+MIE_EXPORT int mie_attention_f32_four_waves(int tokens, int Hq, int Hkv, int D, int splits) {
+  return Hkv > 0 && Hq >= Hkv && four_waves(tokens, Hq, Hkv, D, splits);
+}
+
 // Tokens [0, tokens) of the step, each by itself (row token_row[t], position positions[t]); splits: at least the number of
 // 128-key segments any of them sees; o_part and ml as above (not read or written for one split).
 MIE_EXPORT int mie_attention_f32_single(const float* q, long q_stride, const float* k_cache, const float* v_cache, float* out,
@@ -682,7 +695,7 @@ MIE_EXPORT int mie_attention_f32_single(const float* q, long q_stride, const flo
   const int rep = Hq / Hkv, head_tiles = (rep + 15) / 16;
   if (Hkv * head_tiles > 65535) MIE_FAIL("attention_f32: %d kv heads are beyond the grid", Hkv);
   const dim3 grid(splits, Hkv * head_tiles, tokens);
-  const bool few = (long)splits * Hkv * head_tiles * tokens <= AF_FEW;
+  const bool few = four_waves(tokens, Hq, Hkv, D, splits);
 #define AF_SINGLE(DT)                                                                                                                      \
   if (few) hipLaunchKernelGGL(single_few_f32_kernel<DT>, grid, dim3(AF_SINGLE_WAVES * 64), 0, s, a, out, o_part, ml, token_row, positions, splits); \
   else hipLaunchKernelGGL(single_f32_kernel<DT>, grid, dim3(64), 0, s, a, out, o_part, ml, token_row, positions, splits)

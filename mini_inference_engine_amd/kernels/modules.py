@@ -56,6 +56,7 @@ register_kernel_module("attention_f32", {
     "mie_attention_f32_segment": [],
     "mie_attention_f32_single": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, P, P],
     "mie_attention_f32_alone": [I, I, I, I, I, I, I],
+    "mie_attention_f32_four_waves": [I, I, I, I, I],
     "mie_attention_f32_portions": [P, L, P, P, P, P, I, P, P, I, I, I, I, I, I, I, F, I, I, P],
 })
 register_kernel_module("grouped_gemm", {

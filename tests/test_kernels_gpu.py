@@ -1720,6 +1720,24 @@ def test_attention_float32_few_single_tokens(ops, geom, window):
     torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.float32])
 
 
+# head size and the segments a compute unit up to which they are four waves' work, of several segments a token and of one
+@pytest.mark.parametrize("case", [(16, 1, 1), (32, 2, 2), (48, 4, 3), (64, 4, 4), (80, 3, 2), (96, 3, 2), (112, 4, 4), (128, 4, 4)])
+def test_attention_float32_of_as_many_single_tokens_as_four_waves_take(ops, case):
+    """Single tokens at the line between the two kernels and one token beyond it: the same bits."""
+    o, (D, several, one), cu = ops[torch.float32], case, torch.cuda.get_device_properties(0).multi_processor_count
+    four = o.lib("attention_f32").mie_attention_f32_four_waves
+    for ctx, splits, most in ((17, 1, one), (140, 2, several)):
+        n = most * cu // splits
+        assert four(n, 3, 1, D, splits) == 1 and four(n + 1, 3, 1, D, splits) == 0
+        q, kc, vc, group, step = paged_setup([ctx - r % 16 for r in range(n + 1)], [1] * (n + 1), 3, 1, D, 16, torch.float32, seed=D)
+        beyond, expect = run_attention(ops, torch.float32, q, kc, vc, group, step, 3, 1, D, D ** -0.5, None)
+        torch.testing.assert_close(beyond.double(), expect, **ATT_TOL[torch.float32])
+        few = SimpleNamespace(token_row=step.token_row[:n], positions=step.positions[:n], num_rows=n, max_context=ctx, num_tokens=n, num_decode_rows=n,
+                              max_row_tokens=1, row_start=None, row_position=None)
+        tables = SimpleNamespace(block_tables=group.block_tables[:n].contiguous(), max_blocks=group.max_blocks)
+        assert torch.equal(o.paged_attention(q[:n], 3, 1, D, kc, vc, tables, few, D ** -0.5, None), beyond[:n])
+
+
 # heads, kv heads, head size, page, rows, their tokens, keys before them: one segment at most; rows of one, two and a half and three tiles a
 # workgroup in more workgroups than there are compute units
 @pytest.mark.parametrize("window", [None, 37])
