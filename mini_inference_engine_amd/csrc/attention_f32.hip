@@ -714,19 +714,27 @@ MIE_EXPORT int mie_attention_f32_single(const float* q, long q_stride, const flo
 //    shared loads save.  Four / one wave, us: 64 tokens of 32 / 4 heads of 64 13.4 / 12.2, of 4 / 2 of 16 8.5 / 7.4, 100 of
 //    32 / 8 of 128 19.4 / 18.8, but four rows of 100 of 32 / 4 of 64 (800 waves) 14.3 / 15.4;
 //  - more workgroups than compute units, whose waves are not all of them needed (rows of few tiles): 64 rows of 8 tokens of 12 / 12
-//    heads of 64 (one tile a workgroup) 34.5 / 14.0, of 32 / 8 of 128 (two) 37.1 / 24.1; behind 700 keys (one) 119.9 / 71.5.
-//    Of three tiles a workgroup, 192 rows of 32 / 4 heads of 64: one segment 39.2 / 40.4, 700 keys 1.47 times as long by one wave.
-// Over 567 steps measured 0.89 of four waves everywhere and 0.91 of one; up to 1.19 of one is left at thousands of tokens of ungrouped heads.
+//    heads of 64 (one tile a workgroup) 34.5 / 14.0, of 32 / 8 of 128 (two) 37.1 / 24.1; 16 of 75 of 12 / 12 of 64 (two and a half)
+//    26.0 / 16.4; behind 700 keys (one) 119.9 / 71.5.  Of three tiles a workgroup, 192 rows of 32 / 4 heads of 64: one segment
+//    39.2 / 40.4, 700 keys 1.47 times as long by one wave;
+//  - more workgroups than compute units and little work in each: heads of 16 from two and a half workgroups a compute unit on (8 rows of
+//    250 of 40 / 2 heads 59.5 / 43.2, 3,000 tokens 453 / 368; 588 workgroups of 978 keys 0.89 of one wave, 720 of 476 1.02); of 48 and
+//    80, whose LDS leaves a compute unit one workgroup and most of it idle, up to two segments (64 rows of 43 of 40 / 2 of 48
+//    112 / 71, of 30 of 16 / 2 of 80 29.5 / 25.3, 8 rows of 250 44.7 / 40.3, and more than that on average not).
+// Over 700 steps drawn at random 0.93 of four waves everywhere and 0.94 of one, within 0.2 % of the better one of each; up to 1.12 of one
+// is left (heads of 80 behind thousands of keys).
 static bool alone(int rows, int max_row_tokens, int Hq, int Hkv, int D, int page, int max_context) {
   if (page > 1 << 24) return true;
   const int rep = Hq / Hkv, per_tile = rep <= 16 ? 16 / rep : 1;
   const long heads = (long)Hkv * (rep <= 16 ? 1 : (rep + 15) / 16), cu = mie_compute_units();
   const long tiles = ((long)max_row_tokens + per_tile - 1) / per_tile, groups = (tiles + AF_TILE_WAVES - 1) / AF_TILE_WAVES;
   const long workgroups = groups * heads * rows;
-  const bool one_segment = max_context > 0 && max_context <= AF_SEG;
+  const bool one_segment = max_context > 0 && max_context <= AF_SEG, two_segments = max_context > 0 && max_context <= 2 * AF_SEG;
   if (one_segment && (D <= 32 || tiles * heads * rows <= 2 * cu)) return true;
   if (workgroups <= cu) return false;
-  const int twice = D <= 32 ? 6 : workgroups <= 2 * cu ? 4 : one_segment ? 6 : 5;      // twice the tiles a workgroup up to which
+  if (D == 16 && 2 * workgroups > 5 * cu) return true;
+  if ((D == 48 || D == 80) && two_segments) return true;
+  const int twice = D <= 32 ? 6 : workgroups <= 2 * cu ? (one_segment ? 5 : 4) : one_segment ? 6 : 5;      // twice the tiles a workgroup up to which
   return 2 * tiles <= twice * groups;
 }
 MIE_EXPORT int mie_attention_f32_alone(int rows, int max_row_tokens, int Hq, int Hkv, int D, int page, int max_context) {

@@ -1739,10 +1739,11 @@ def test_attention_float32_of_as_many_single_tokens_as_four_waves_take(ops, case
 
 
 # heads, kv heads, head size, page, rows, their tokens, keys before them: one segment at most; rows of one, two and a half and three tiles a
-# workgroup in more workgroups than there are compute units
+# workgroup in more workgroups than there are compute units; many workgroups of heads of 16, and of 48 and 80 with two segments
 @pytest.mark.parametrize("window", [None, 37])
 @pytest.mark.parametrize("case", [(32, 4, 64, 16, 1, 128, 0), (40, 2, 16, 16, 3, 100, 28), (16, 1, 128, 16, 2, 33, 50), (12, 12, 64, 16, 32, 16, 250),
-                                  (32, 8, 128, 16, 40, 20, 300), (6, 2, 112, 16, 129, 5, 200), (3, 1, 32, 16, 300, 13, 130), (8, 2, 48, 48, 260, 9, 0)])
+                                  (32, 8, 128, 16, 40, 20, 300), (6, 2, 112, 16, 129, 5, 200), (3, 1, 32, 16, 300, 13, 130), (8, 2, 48, 48, 260, 9, 0),
+                                  (40, 2, 16, 16, 16, 60, 300), (8, 2, 48, 16, 80, 30, 200), (16, 2, 80, 16, 64, 30, 0), (12, 12, 64, 16, 16, 75, 0)])
 def test_attention_float32_portions_by_single_waves(ops, case, window):
     """Portions that single waves take against the same ones by workgroups of four tiles (a few of the rows, the context not said): the
     same bits, also beside a later token's keys and values that are not finite; and against 64 bits."""
