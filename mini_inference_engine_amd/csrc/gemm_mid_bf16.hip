@@ -16,7 +16,9 @@
 // multiplies (v_mfma_f32_16x16x32_bf16).  The waves' sums meet in the LDS, in wave order.  Weights by nontemporal loads.
 // Before, four waves that shared a ring of stages met at a barrier a stage: a stage of 16 KB took 0.4 to 0.6 us whatever it
 // loaded.  Measured (MI355X, us, before / now): with the sums' kernel and the norm, 24 rows of [2048, 2048] 8.5 / 7.3, [2560, 2048]
-// 9.9 / 8.4, [2048, 5632] 11.9 / 9.7, [4096, 14336] 34.3 / 24.9; 64 rows 9.9 / 8.9, 11.2 / 10.2, 13.2 / 12.3, 33.4 / 30.2.  Gate and
+// 9.9 / 8.4, [2048, 5632] 11.9 / 9.7, [4096, 14336] 34.3 / 24.9; 64 rows 9.9 / 8.9, 11.2 / 10.2, 13.2 / 12.3, 33.4 / 30.2.  Of
+// two or three chunks a wave 64 and 128 rows gain nothing ([3072, 3072] 13.4 / 13.8 and 17.3 / 18.3, [4096, 2048] 13.2 / 13.9 and 17.8 / 18.2,
+// but 32 and 96 rows 12.3 / 11.2 and 17.0 / 16.1, 11.9 / 11.3 and 16.6 / 16.1; other numbers of splits 0.1 to 0.4 us at most).  Gate and
 // up against the library's product and silu_mul: [11264, 2048] 17 / 64 / 128 rows 17.6 / 10.9, 19.9 / 13.7, 22.7 / 18.4;
 // [28672, 4096] 17 / 64 rows 55.4 / 43, 57.1 / 47.5.
 // The number of splits and of tiles a workgroup depends on the weight's shape alone and chunks go to waves by their place in
