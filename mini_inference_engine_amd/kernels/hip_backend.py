@@ -414,6 +414,11 @@ class HipBackend(KernelBackend):
         units = min(units, 8, K // 256)
         return -(-(K // 64) // -(-(K // 64) // units)) if units >= 2 else 0      # as many as their stages come out at
 
+    def _tile_takes(self, x, w, bias) -> bool:
+        """Whether the own tiles take x w^T with what follows it (added into the stream, or rotated): where one of them has no more
+        workgroups than run at once (tile_for in csrc/tile_gemm_bf16.hip has both sides measured)."""
+        return self._tile_ok(x, w, bias) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_tile(x.shape[0], w.shape[0], w.shape[1]))
+
     def _tile_swiglu_gains(self, x, w, intermediate) -> bool:
         """Whether the own gate/up product with SwiGLU on its sums beats the library's and silu_mul: its estimate (a stage's time
         of each tile times the rounds of its grid) against what the library was measured at, 7 us + weights at 3.5 TB/s +
@@ -481,7 +486,11 @@ class HipBackend(KernelBackend):
             if bias is None and sink is not None:
                 # the product adds its float32 sums to the stream itself (C = C + A B in place): the stream is
                 # not read and written once more by a kernel of its own
-                if own_call:
+                if sink.stream.data_ptr() % 16 == 0 and self._tile_takes(x, w, None):
+                    lib = self.lib("tile_gemm_bf16")
+                    library.check(lib, lib.mie_tile_gemm_add(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(sink.stream), N, M, N, K,
+                                                             self._stream()))
+                elif own_call:
                     self._lt_product(x, w, self.LT_ADD, sink.stream)
                 else:
                     torch.ops.aten.addmm.dtype_out(sink.stream, x, w.t(), torch.float32, out=sink.stream)
@@ -1512,13 +1521,22 @@ class HipBackend(KernelBackend):
                                              for_attention)
         if (not fused and can_rope and not self.true_fp32 and self.act_dtype == torch.bfloat16
                 and x.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16):
-            # many rows: library product with float32 sums, then rotary and cache write from those sums (q and k
-            # are rounded to bfloat16 once, after the rotation)
+            # many rows: rotary and cache write from the product's float32 sums (q and k are rounded to bfloat16 once, after
+            # the rotation), in its own kernel or, where the sums are the library's or wanted as they are, behind it
             self._on_device(x, w_qkv)
             self._on_device(positions, cos, sin, k_cache, v_cache, slot_mapping)
             M, K = x.shape
             page = self._check_rope_operands("linear_rotary_kv_store", M, K, w_qkv, positions, cos, sin, Hq, Hkv, D,
                                              k_cache, v_cache, slot_mapping)
+            if (not for_attention and self._lt_ok(x, w_qkv) and self._tile_takes(x, w_qkv, None) and D <= 256 and page % 16 == 0
+                    and not any(t.data_ptr() % 16 for t in (cos, sin, k_cache, v_cache))):
+                # rotation and cache write on the own tiles' float32 sums: the same expressions, one kernel and 8 us less
+                q = torch.empty((M, Hq * D), dtype=torch.bfloat16, device=x.device)
+                lib = self.lib("tile_gemm_bf16")
+                library.check(lib, lib.mie_tile_gemm_qkv_rope(
+                    _ptr(x), x.stride(0), _ptr(w_qkv), w_qkv.stride(0), _ptr(q), q.stride(0), _ptr(positions), _ptr(cos), _ptr(sin),
+                    _ptr(slot_mapping), _ptr(k_cache), _ptr(v_cache), M, Hq, Hkv, D, page, K, self._stream()))
+                return q
             if self._lt_ok(x, w_qkv):
                 sums = self._lt_product(x, w_qkv, self.LT_F32, torch.empty((M, w_qkv.shape[0]), dtype=torch.float32, device=x.device))
             else:

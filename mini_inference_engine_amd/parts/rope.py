@@ -51,9 +51,10 @@ class RotaryHalfSplit(PositionEncoding):
     def project_encode_store(self, ops, x, w_qkv, step, num_q_heads, num_kv_heads, k_cache, v_cache, slots):
         """Projection, encoding and cache write together; returns what the backend's paged_attention takes as
         its ``qkv`` (a tensor whose first Hq * D columns are the encoded q, or work the backend has put off
-        until then).  The backend may run it as one kernel."""
+        until then: only a step of single tokens has an attention that takes such work).  The backend may run it as one kernel."""
         return ops.linear_rotary_kv_store(x, w_qkv, step.positions, self.cos, self.sin, self.rotary_dim, num_q_heads,
-                                          num_kv_heads, self.head_dim, k_cache, v_cache, slots, for_attention=True)
+                                          num_kv_heads, self.head_dim, k_cache, v_cache, slots,
+                                          for_attention=step.num_decode_rows == step.num_tokens)
 
 
 @register_position_encoding("none")

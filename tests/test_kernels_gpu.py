@@ -527,6 +527,60 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
+# rows, columns, K and the tile: every tile, edges in rows and columns, K of one stage, of fewer and of more than the ring holds
+@pytest.mark.parametrize("case", [(137, 72, 64, 64064), (333, 2056, 320, 64064), (138, 5560, 64, 64080), (509, 2552, 576, 64080), (193, 5240, 192, 64096),
+                                  (263, 4912, 256, 64128), (513, 4520, 64, 80128), (1131, 2040, 1408, 80128), (520, 4624, 192, 96128), (483, 5392, 64, 128128),
+                                  (2047, 2040, 1088, 128128), (646, 5392, 1024, 128160), (642, 5488, 320, 128192), (1027, 5416, 448, 256128)])
+def test_tile_product_added(engine_ops, case):
+    """A product on the own tiles added into the stream: every tile; the float32 sums within the worst case of their additions, nothing
+    written beyond the last row."""
+    o, (M, N, K, tile) = engine_ops, case
+    lib = o.lib("tile_gemm_bf16")
+    assert lib.mie_tile_gemm_tile(M, N, K) == tile, "the case must take the tile it is for"
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K + 8, device=DEV).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K + 16, device=DEV) / math.sqrt(K)).to(torch.bfloat16)[:, :K]
+    held = torch.randn(M + 3, N, device=DEV)
+    behind, expect = held[M:].clone(), held[:M].double() + x.double() @ w.double().T
+    bound = (K + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -22 * expect.abs()
+    with counted(o, "tile_gemm_bf16", "mie_tile_gemm_add") as calls:
+        assert o.linear(x, w, add_to=held[:M]) is None
+    assert len(calls) == 1
+    assert bool(((held[:M].double() - expect).abs() <= bound).all()) and torch.equal(held[M:], behind)
+    assert lib.mie_tile_gemm_tile(4096, 8192, K) == 0 and lib.mie_tile_gemm_add(x.data_ptr(), K + 8, w.data_ptr(), K + 16, held.data_ptr(), N, M, N, K - 8, None) != 0
+
+
+@pytest.mark.parametrize("case", [(137, 2, 1, 16, 64), (333, 32, 4, 64, 320), (300, 3, 3, 80, 128), (512, 32, 4, 64, 192), (700, 5, 2, 48, 64), (1131, 32, 4, 64, 64),
+                                  (2040, 32, 4, 64, 128), (520, 32, 8, 128, 64), (1020, 32, 8, 128, 64), (260, 2, 2, 256, 128), (1500, 7, 1, 112, 64)])
+def test_tile_projection_rotary_store(engine_ops, case):
+    """The q/k/v projection of many rows with rotation and cache write on the own tiles' sums: against the same kernels' float32 sums
+    finished by a kernel of their own (one rounding of bfloat16 apart where the sums' order differs), other pages untouched."""
+    from mini_inference_engine_amd.parts.rope import rotary_tables
+    o, (M, Hq, Hkv, D, K) = engine_ops, case
+    torch.manual_seed(M + D)
+    N, page = (Hq + 2 * Hkv) * D, 32
+    assert o.lib("tile_gemm_bf16").mie_tile_gemm_tile(M, N, K) > 0
+    pages = -(-M // page) + 3
+    cos, sin = (t.to(DEV) for t in rotary_tables(10000.0, D, 3000))
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    pos = torch.randint(0, 3000, (M,), device=DEV, dtype=torch.int32)
+    slots = (torch.randperm((pages - 1) * page, device=DEV)[:M] + page).to(torch.int32)
+    kc, vc = make_cache(pages, Hkv, page, D, torch.bfloat16)
+    kc2, vc2 = kc.clone(), vc.clone()
+    with counted(o, "tile_gemm_bf16", "mie_tile_gemm_qkv_rope") as calls:
+        q = o.linear_rotary_kv_store(x, w, pos, cos, sin, D, Hq, Hkv, D, kc, vc, slots)
+    assert len(calls) == 1 and tuple(q.shape) == (M, Hq * D)
+    q2 = o.linear_rotary_kv_store(x, w, pos, cos, sin, D, Hq, Hkv, D, kc2, vc2, slots, for_attention=True).finish()
+    for a, b in ((q, q2), (kc, kc2), (vc, vc2)):
+        assert bool(((a.double() - b.double()).abs() <= 2.0 ** -7 * b.double().abs() + 1e-4).all())
+    fresh = torch.ones(pages * page, dtype=torch.bool, device=DEV)
+    fresh[slots.long()] = False
+    assert torch.equal(kc[0], kc2[0]) and torch.equal(vc[0], vc2[0])
+    at = fresh.view(pages, page)
+    assert torch.equal(kc.transpose(1, 2)[at], kc2.transpose(1, 2)[at]) and torch.equal(vc.permute(0, 3, 1, 2)[at], vc2.permute(0, 3, 1, 2)[at])
+
+
 # rows, K, columns and how many of them are made by uncut tiles
 @pytest.mark.parametrize("case", [(512, 2048, 5632, 4096), (384, 72, 5632, 5440), (260, 72, 7000, 0), (129, 96, 8256, 8192), (600, 64, 3300, 3264), (400, 200, 4096, 4096),
                                   (520, 40, 3332, 3264), (2047, 200, 1000, 1000)])
