@@ -2,8 +2,7 @@
 // cores of gfx950, for one head size per build (-DHEAD_DIM=N, a multiple of 16 up to 256).
 // Caches: keys [pages, Hkv, page, D], values [pages, Hkv, D, page].
 //
-#include "attention_bf16_common.hpp"
-#include "launch.hpp"
+#include "decode_attention_bf16.hpp"
 
 // prefill_attention: rows of several tokens, starting anywhere in their request.  With
 // v_mfma_f32_32x32x16_bf16 (A: 32 rows x 16 k, B: 16 k x 32 columns, C: 32 x 32, lane l holds column l % 32
@@ -117,8 +116,8 @@ __device__ __forceinline__ float pair_sum(float x) {
 // brings 128 keys in, each half computes its 64) and join their results at the end: half the blocks a wave
 // for rows too short to give every SIMD two waves otherwise.
 template <int PF_WAVES, int KS, bool SIG, bool DB = false, bool KEEP = false, bool CHUNK = false>
-__global__ void __launch_bounds__(PF_WAVES * 64, PF_DIRECT && PF_WAVES == 4 ? 2 : 1)
-prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* __restrict__ k_cache,
+__device__ __forceinline__ void
+prefill_attention_body(const dim3 place, const dim3 grid, const bf16* __restrict__ q, long q_stride, const bf16* __restrict__ k_cache,
                          const bf16* __restrict__ v_cache, bf16* __restrict__ out,
                          const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ row_start,
                          const int* __restrict__ row_position, const int* __restrict__ row_written, int first_row, int Hq, int Hkv, int waves_h,
@@ -139,10 +138,10 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
   // launch order with x fastest, and every XCD has an L2 of its own: all workgroups of one kv head read
   // the same keys and values, so they are placed on one XCD (or on 8 / Z of them when there are fewer
   // than eight z indices), and a block of keys is fetched into one L2 instead of all eight.
-  int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+  int bx = place.x, by = place.y, bz = place.z;
   {
-    const unsigned X = gridDim.x, Y = gridDim.y, Z = gridDim.z;
-    const unsigned w = blockIdx.x + X * (blockIdx.y + Y * blockIdx.z), total = X * Y * Z;
+    const unsigned X = grid.x, Y = grid.y, Z = grid.z;
+    const unsigned w = place.x + X * (place.y + Y * place.z), total = X * Y * Z;
     if (total % 8 == 0 && (Z % 8 == 0 || 8 % Z == 0)) {       // uniform over the grid
       unsigned r;
       if (Z % 8 == 0) {
@@ -757,6 +756,53 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
   }
 }
 
+template <int PF_WAVES, int KS, bool SIG, bool DB = false, bool KEEP = false, bool CHUNK = false>
+__global__ void __launch_bounds__(PF_WAVES * 64, PF_DIRECT && PF_WAVES == 4 ? 2 : 1)
+prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* __restrict__ k_cache,
+                         const bf16* __restrict__ v_cache, bf16* __restrict__ out,
+                         const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ row_start,
+                         const int* __restrict__ row_position, const int* __restrict__ row_written, int first_row, int Hq, int Hkv, int waves_h,
+                         int page, float scale_log2, int window, float sink_log2, int chunk, float softcap,
+                         const float* __restrict__ head_bias, const float* __restrict__ dist_bias, int dist_n, int keep,
+                         const float* __restrict__ head_sinks, int paired) {
+  prefill_attention_body<PF_WAVES, KS, SIG, DB, KEEP, CHUNK>(
+    dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), q, q_stride, k_cache, v_cache, out, block_tables,
+    max_blocks, row_start, row_position, row_written, first_row, Hq, Hkv, waves_h, page, scale_log2, window, sink_log2, chunk,
+    softcap, head_bias, dist_bias, dist_n, keep, head_sinks, paired);
+}
+
+// Rows of one token (decode_attention_bf16.hpp) beside the portions of the same step, in one launch: the first workgroups take the
+// portions, those behind them the single tokens, whose keys and values come in on compute units that the portions leave idle.  By themselves
+// the two kernels follow each other, each with a start and an end, and neither fills the chip: few stretches and long chains of blocks
+// here, a workgroup a row and kv head there.  32 / 4 heads of 64, us, two kernels (and a third that joins parts of contexts) / one: 32
+// rows of 150 to 900 keys beside 701 and 399 tokens 28.2 / 21.9, 8 of 1,500 beside 1,000 27.8 / 20.1, 1 of 900 beside 100 15.5 / 8.8, 64 of
+// 1,500 beside 1,800 55.3 / 51.3.
+struct SingleRows {
+  float *o_part, *lse_part;
+  const int* positions;
+  int rows, head_tiles, partition, splits;
+};
+template <int KS>
+__global__ void __launch_bounds__(512, 1)
+step_attention_kernel(const bf16* __restrict__ q, long q_stride, bf16* k_cache, bf16* v_cache, bf16* __restrict__ out,
+                      const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ row_start, const int* __restrict__ row_position,
+                      const int* __restrict__ row_written, int Hq, int Hkv, int waves_h, int page, float scale_log2, int window, float sink_log2,
+                      int paired, dim3 portions, SingleRows one) {
+  const unsigned id = blockIdx.x, P = portions.x * portions.y * portions.z;
+  if (id < P) {
+    const unsigned z = id / (portions.x * portions.y), rest = id - z * portions.x * portions.y;
+    prefill_attention_body<8, KS, false>(dim3(rest % portions.x, rest / portions.x, z), portions, q, q_stride, k_cache, v_cache, out, block_tables,
+                                         max_blocks, row_start, row_position, row_written, one.rows, Hq, Hkv, waves_h, page, scale_log2, window,
+                                         sink_log2, 0, 0.f, nullptr, nullptr, 0, 0, nullptr, paired);
+  } else {
+    const unsigned d = id - P, u = d / one.rows, units = Hkv * one.head_tiles;
+    decode_attention_body<8, false, false, false, false, false, RINGED>(d - u * one.rows, u % units, u / units, q, q_stride, k_cache, v_cache, out,
+                                                                       one.o_part, one.lse_part, block_tables, max_blocks, one.positions, Hq, Hkv,
+                                                                       one.head_tiles, page, scale_log2, window, one.partition, one.splits,
+                                                                       ProjectionSums{}, sink_log2, 0, 0.f, nullptr, nullptr, 0, 0, nullptr);
+  }
+}
+
 MIE_EXPORT const char* prefill_attention_bf16_last_error() { return g_mie_error; }
 // 1: the caches must be 16-byte aligned
 MIE_EXPORT int mie_prefill_needs_aligned_caches() { return PF_DIRECT; }
@@ -967,4 +1013,55 @@ MIE_EXPORT int mie_prefill_attention_chunked(const void* q, long q_stride, const
   return prefill_attention_launch(q, q_stride, k_cache, v_cache, out, block_tables, max_blocks, row_start, row_position,
                                   row_written, first_row, rows, max_row_tokens, Hq, Hkv, head_dim, page, scale, window, -INFINITY, stream,
                                   false, chunk);
+}
+
+// Whether a step's single tokens and portions go out together (mie_step_attention): at head size 64, where both kernels have eight waves,
+// while the single tokens' workgroups are no more than the compute units.
+MIE_EXPORT int mie_step_attention_takes(int singles, int rows, int max_row_tokens, int Hq, int Hkv, int splits) {
+  if (D != 64 || singles <= 0 || rows <= 0 || max_row_tokens <= 0 || splits <= 0 || Hkv <= 0 || Hq % Hkv) return 0;
+  if ((long)singles * Hkv * ((Hq / Hkv + 15) / 16) * splits > mie_compute_units()) return 0;
+  const PrefillPlan plan = prefill_plan(rows, max_row_tokens, Hq, Hkv, mie_compute_units());
+  return plan.kind != FOUR && (long)plan.grid.x * plan.grid.y * plan.grid.z < 1 << 22;
+}
+
+// Plain softmax attention (sink: one more term exp(sink) in every denominator, -infinity for none) of a step whose first `singles` rows
+// have one token each, at `positions`, and whose other `rows` have up to max_row_tokens.  partition, splits, o_part and lse_part are
+// those of mie_decode_attention, the other arguments those of mie_prefill_attention.
+MIE_EXPORT int mie_step_attention(const void* q, long q_stride, const void* k_cache, const void* v_cache, void* out, float* o_part,
+                                  float* lse_part, const int* block_tables, int max_blocks, const int* positions, int singles, int partition,
+                                  int splits, const int* row_start, const int* row_position, const int* row_written, int rows, int max_row_tokens,
+                                  int Hq, int Hkv, int head_dim, int page, float scale, int window, float sink, hipStream_t stream) {
+  if (head_dim != D) MIE_FAIL("step_attention: built for head_dim %d, called with %d", D, head_dim);
+  if (!mie_step_attention_takes(singles, rows, max_row_tokens, Hq, Hkv, splits))
+    MIE_FAIL("step_attention: %d single tokens, %d portions of %d, %d / %d heads of %d, %d splits", singles, rows, max_row_tokens, Hq, Hkv, D, splits);
+  if (page < 16 || page % 16) MIE_FAIL("step_attention: page size %d (multiples of 16)", page);
+  if (q_stride < (long)Hq * D || (q_stride % 8) || ((uintptr_t)q % 16) || ((uintptr_t)out % 8)) MIE_FAIL("step_attention: q stride %ld / alignment", q_stride);
+  if (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) MIE_FAIL("step_attention: caches must be 16-byte aligned");
+  if (max_blocks <= 0) MIE_FAIL("step_attention: max_blocks %d", max_blocks);
+  if (partition <= 0 || partition % (BLOCK_KEYS * NW_SPLIT)) MIE_FAIL("step_attention: partition %d is no multiple of %d", partition, BLOCK_KEYS * NW_SPLIT);
+  if (splits > 1 && (!o_part || !lse_part)) MIE_FAIL("step_attention: splits need partial buffers");
+  if constexpr (D == 64) {
+    const PrefillPlan plan = prefill_plan(rows, max_row_tokens, Hq, Hkv, mie_compute_units());
+    const int head_tiles = (Hq / Hkv + 15) / 16;
+    const long blocks = (long)plan.grid.x * plan.grid.y * plan.grid.z + (long)singles * Hkv * head_tiles * splits;
+    auto launch = [&](auto kernel, int lds) -> int {
+      if (mie_allow_lds((const void*)kernel, lds, "step_attention")) return -1;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(512), lds, stream, (const bf16*)q, q_stride, (bf16*)const_cast<void*>(k_cache),
+                         (bf16*)const_cast<void*>(v_cache), (bf16*)out, block_tables, max_blocks, row_start, row_position, row_written, Hq, Hkv,
+                         plan.waves_h, page, scale * 1.4426950408889634f, window, sink * 1.4426950408889634f, plan.paired ? 1 : 0, plan.grid,
+                         SingleRows{o_part, lse_part, positions, singles, head_tiles, partition, splits});
+      return 0;
+    };
+    auto most = [](int a, int b) { return a > b ? a : b; };
+    if (plan.kind == EIGHT_KEYS) {
+      if (launch(step_attention_kernel<2>, most(pf_lds_bytes(2, 8), da_lds_bytes(8, true)))) return -1;
+    } else if (launch(step_attention_kernel<1>, most(pf_lds_bytes(1, 8), da_lds_bytes(8, true)))) return -1;
+    MIE_CHECK_LAUNCH("step_attention");
+    if (splits > 1) {
+      hipLaunchKernelGGL(merge_splits_kernel, dim3(singles * Hq), dim3(64), 0, stream, o_part, lse_part, (bf16*)out, splits,
+                         sink * 1.4426950408889634f, 0, (const float*)nullptr, Hq);
+      MIE_CHECK_LAUNCH("merge_splits");
+    }
+  }
+  return 0;
 }

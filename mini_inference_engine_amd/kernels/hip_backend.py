@@ -1801,6 +1801,18 @@ class HipBackend(KernelBackend):
         done = 0
         if D > 256:
             force_generic = True            # beyond the matrix-core kernels' head sizes: the 32-bit kernel takes up to 1,024
+        written = None
+        if step.num_decode_rows < T and qkv.dtype == torch.bfloat16 and not force_generic:
+            for name, t, n in (("row_start", step.row_start, step.num_rows + 1),
+                               ("row_position", step.row_position, step.num_rows)):
+                if t is None or t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous():
+                    raise ValueError(f"paged_attention: {name} must be contiguous int32 [{n}]")
+            written = getattr(step, "row_written", None)        # where rows end that padding tokens lengthen
+            if written is not None and (written.dtype != torch.int32 or written.shape[0] < step.num_rows or not written.is_contiguous()):
+                raise ValueError(f"paged_attention: row_written must be contiguous int32 [{step.num_rows}]")
+            if (step.num_decode_rows > 0 and not scored and num_splits is None
+                    and self._step_attention(qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window, written, sink if has_sink else float("-inf"))):
+                return out
         if qkv.dtype == torch.bfloat16 and not force_generic and step.num_decode_rows > 0:
             done = step.num_decode_rows        # single-token rows lead the batch: token t is row t
             lib = self.lib("attention_bf16", (f"-DHEAD_DIM={D}",))
@@ -1837,13 +1849,6 @@ class HipBackend(KernelBackend):
         end = T                                # tokens [done, end) are left to the 32-bit kernel
         if step.num_decode_rows < T and qkv.dtype == torch.bfloat16 and not force_generic:
             # rows of several tokens: matrix-core kernel over their own and earlier portions' keys
-            for name, t, n in (("row_start", step.row_start, step.num_rows + 1),
-                               ("row_position", step.row_position, step.num_rows)):
-                if t is None or t.dtype != torch.int32 or t.shape[0] < n or not t.is_contiguous():
-                    raise ValueError(f"paged_attention: {name} must be contiguous int32 [{n}]")
-            written = getattr(step, "row_written", None)        # where rows end that padding tokens lengthen
-            if written is not None and (written.dtype != torch.int32 or written.shape[0] < step.num_rows or not written.is_contiguous()):
-                raise ValueError(f"paged_attention: row_written must be contiguous int32 [{step.num_rows}]")
             lib = self.lib("prefill_attention_bf16", (f"-DHEAD_DIM={D}",))
             keys, values, table = k_cache, v_cache, bt
             if (k_cache.data_ptr() | v_cache.data_ptr()) % 16 and lib.mie_prefill_needs_aligned_caches():
@@ -1883,6 +1888,35 @@ class HipBackend(KernelBackend):
             else:
                 library.check(lib, lib.mie_paged_attention(*args, self._stream()))
         return out
+
+    STEP_SPLIT_KEYS = 2048
+
+    def _step_attention(self, qkv, Hq, Hkv, D, k_cache, v_cache, out, bt, page, step, scale, window, written, sink) -> bool:
+        """Plain softmax attention of a step of single tokens and portions in one launch (csrc/prefill_attention_bf16.hip); False
+        where that does not take them.  Beside portions a single token's keys come in while others compute: contexts are cut
+        into no less than 2,048 keys a workgroup, and most steps need no kernel that joins the parts."""
+        lib = self.lib("prefill_attention_bf16", (f"-DHEAD_DIM={D}",))
+        singles = step.num_decode_rows
+        shape = (singles, step.num_rows - singles, int(step.max_row_tokens or 0), Hq, Hkv)
+        if (k_cache.data_ptr() | v_cache.data_ptr()) % 16 or not lib.mie_step_attention_takes(*shape, 1):
+            return False
+        block_keys = self.lib("attention_bf16", (f"-DHEAD_DIM={D}",)).mie_decode_block_keys()
+        partition, splits = self.decode_splits(singles, Hq, Hkv, step.max_context, window, block_keys, D)
+        if splits > 1:
+            bound = min(step.max_context, window + 32) if window else step.max_context
+            partition = max(partition, min(self.STEP_SPLIT_KEYS, -(-bound // block_keys) * block_keys))
+            splits = -(-bound // partition)
+            if not lib.mie_step_attention_takes(*shape, splits):
+                return False
+        o_part = lse_part = None
+        if splits > 1:
+            o_part = torch.empty((singles, Hq, splits, D), dtype=torch.float32, device=qkv.device)
+            lse_part = torch.empty((singles, Hq, splits), dtype=torch.float32, device=qkv.device)
+        library.check(lib, lib.mie_step_attention(
+            _ptr(qkv), qkv.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(o_part), _ptr(lse_part), _ptr(bt), bt.shape[1],
+            _ptr(step.positions), singles, partition, splits, _ptr(step.row_start), _ptr(step.row_position), _ptr(written),
+            step.num_rows - singles, step.max_row_tokens, Hq, Hkv, D, page, float(scale), int(window or 0), float(sink), self._stream()))
+        return True
 
     # What the results of single tokens' segments of 128 keys may take, bytes: rows beyond it wait for a launch of their own, which
     # by then has hundreds of waves a compute unit (32 heads of 128 with contexts up to 8,192: 126 rows a launch)

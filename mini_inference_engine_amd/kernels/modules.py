@@ -157,6 +157,8 @@ register_kernel_module("prefill_attention_bf16", {
     "mie_prefill_attention_sigmoid": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, F, P, P],
     "mie_prefill_attention_biased": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P, I, P],
     "mie_prefill_attention_chunked": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
+    "mie_step_attention_takes": [I, I, I, I, I, I],
+    "mie_step_attention": [P, L, P, P, P, P, P, P, I, P, I, I, I, P, P, P, I, I, I, I, I, I, F, I, F, P],
     "mie_prefill_attention_kept": [P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, P, P],
 }, variants=_head_variants, flags=["-mllvm", "-amdgpu-mfma-vgpr-form"])
 # lt_gemm: host code only, the engine's own way into the library's matrix products (hipBLASLt) with the choice of

@@ -1427,6 +1427,45 @@ def test_attention_mixed_rows(ops, dtype, geom):
     torch.testing.assert_close(out.double(), expect, **ATT_TOL[dtype])
 
 
+# single tokens' contexts; portions (tokens, tokens before them); heads; window; sink: one and many single tokens, contexts of one key, of whole
+# and broken blocks and pages, contexts cut at 2,048 keys, every grid of the portions, groups of more than 16 heads, as many workgroups as
+# compute units, and one single token more (two kernels)
+@pytest.mark.parametrize("case", [([1], [(2, 0)], (4, 1), 0, None), ([700, 64, 3], [(33, 0), (150, 77)], (32, 4), 0, None), ([900] * 32, [(701, 0), (399, 0)], (32, 4), 0, None),
+                                  ([2500, 31], [(65, 9)], (32, 4), 0, 0.7), ([4200], [(40, 300)], (8, 8), 0, None), ([2500, 800, 17], [(130, 1500)], (16, 4), 256, None),
+                                  ([333, 5000], [(70, 0), (2, 4000)], (40, 2), 1000, -0.5), ([50] * 64, [(1300, 0), (1290, 3)], (32, 4), 0, None),
+                                  ([50] * 65, [(40, 0)], (32, 4), 0, None)])
+@pytest.mark.parametrize("page", [16, 48])
+def test_attention_of_singles_beside_portions(ops, case, page):
+    """A step's single tokens and portions in one launch (head size 64): against 64 bits at the bound of the kernels alone, the single
+    tokens as near to their own kernel's, and no key that is not a request's reaches a result."""
+    contexts, portions, (Hq, Hkv), window, sink = case
+    o, D, n = ops[torch.bfloat16], 64, len(contexts)
+    ctx, new = contexts + [a + b for a, b in portions], [1] * n + [a for a, _ in portions]
+    q, kc, vc, group, step = paged_setup(ctx, new, Hq, Hkv, D, page, torch.bfloat16, seed=n + len(portions))
+    used = torch.zeros(kc.shape[0], dtype=torch.bool, device=DEV)
+    for r, c in enumerate(ctx):
+        pages = group.block_tables[r, :-(-c // page)].long()
+        used[pages] = True
+        if c % page:                            # behind a request's last key: numbers that must not reach a sum
+            kc[pages[-1], :, c % page:] = vc[pages[-1], :, :, c % page:] = float("nan")
+    kc[~used] = vc[~used] = float("nan")
+    fused = n * Hkv * -(-(Hq // Hkv) // 16) <= 256
+    with counted(o, "prefill_attention_bf16", "mie_step_attention", defines=("-DHEAD_DIM=64",)) as calls:
+        out = o.paged_attention(q, Hq, Hkv, D, kc, vc, group, step, D ** -0.5, window or None, sink=sink)
+    assert len(calls) == (1 if fused else 0)
+    plain_k, plain_v = kc.nan_to_num(0.0), vc.nan_to_num(0.0)
+    expect = ref.ref_paged_attention(q, Hq, Hkv, D, plain_k, plain_v, group.block_tables, step.token_row, step.positions, D ** -0.5, window or None,
+                                     torch.float64, **({} if sink is None else {"sink": sink}))
+    torch.testing.assert_close(out.double(), expect, **ATT_TOL[torch.bfloat16])
+    # the same by two kernels: the single tokens alone, then the portions
+    one = SimpleNamespace(token_row=step.token_row[:n], positions=step.positions[:n], num_rows=n, max_context=max(contexts), num_tokens=n, num_decode_rows=n,
+                          max_row_tokens=1, row_start=None, row_position=None)
+    alone = o.paged_attention(q[:n], Hq, Hkv, D, kc, vc, group, one, D ** -0.5, window or None, sink=sink)
+    # weights and results are rounded to bfloat16 on both sides: 2^-8 of the largest value a sum holds, each
+    bound = 4 * 2.0 ** -8 * float(vc[used].nan_to_num(0.0).abs().max())
+    assert float((alone.float() - out[:n].float()).abs().max()) <= bound
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("key", [0, 15, 16, 31, 255, 256, 700, 1022])
 def test_attention_finds_a_far_key(ops, dtype, key):
