@@ -627,10 +627,10 @@ MIE_EXPORT int mie_tile_gemm_qkv_rope(const void* X, long ldx, const void* W, lo
 }
 
 // Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: measured at
-// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 384, the second 128 x 128 and those behind it are tile_spread_kernel's, the others
-// tile_gemm_kernel's, of which 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  Own tile of
-// before / now, us: 160 rows 25.2 / 22.4, 256 26.0 / 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9;
-// at 1,024 and 1,132 rows 256 x 256 of sixteen waves of 64 x 64 stays (45.6 and 50.5 us; of eight of 64 x 128 54.6 and 53.7).
+// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 256, 256 x 320 and 256 x 384 are tile_wide_kernel's, the others tile_gemm_kernel's, of which
+// the first 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  Own tile of before / now, us: 160 rows 25.2 / 22.4, 256 26.0 /
+// 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9.  256 x 256, weights from memory, by eight waves of 64 x 128
+// / four of 128 x 128 with two sets of fragments: 1,132 rows 54.1 / 57.5, 1,200 54.3 / 57.8, 1,280 55.1 / 58.9.
 constexpr struct { int bm, bn; float us; } TILE_STAGE_US[] = {
   {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f},
   {128, 128, 0.72f}, {128, 192, 0.96f}, {192, 192, 1.12f}, {256, 320, 1.94f}};
@@ -652,8 +652,8 @@ static int best_tile(int M, long cols, int first, int behind, float& us) {
   return best;
 }
 
-// What mie_tile_gemm_swiglu takes at most, in units of 0.01 us, for the decision against the library.  It leaves out the tiles of the spread
-// kernel but 256 x 384: with them the decision, whose estimate of the library is rough, would change for the better at some sizes and
+// What mie_tile_gemm_swiglu takes at most, in units of 0.01 us, for the decision against the library.  It leaves out the
+// tiles behind 256 x 384: with them the decision, whose estimate of the library is rough, would change for the better at some sizes and
 // for the worse at others (us, own / library / library's kernel chosen by timing: 1,300 rows of [11264, 2048] 63.8 / 71.7 / 72.6, 550 rows
 // 36.2 / 36.7 / 36.8, but 256 rows of [8192, 2048] 22.6 / 24.8 / 19.6).
 MIE_EXPORT int mie_tile_gemm_swiglu_cost(int M, int N, int K) {
@@ -679,7 +679,7 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
     case 1: return launch<2, 2, 4, 6, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 2: return launch<4, 2, 4, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 3: return launch<4, 2, 6, 4, 2, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    case 4: return launch<2, 2, 8, 8, 2, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
+    case 4: return launch_wide<8, 4, 2>(t, K, s);
     case 5: return launch_wide<12, 4, 2>(t, K, s);
     case 6: return launch<2, 2, 4, 4, 4, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 7: return launch<2, 2, 6, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
