@@ -386,15 +386,22 @@ tile_gemm_kernel(TileArgs t, TileRope rope) {
   }
 }
 
-// Gate and up by eight waves whose sums leave no room for a second set of fragments: TB x TA tiles of 16 x 16 a wave, four waves over x and
-// two over W, the weight fragments read one ahead.
-template <int TA, int TB, int STAGES>
-__global__ void __launch_bounds__(512)
-tile_wide_kernel(TileArgs t) {
-  constexpr int WR = 4, WC = 2, BM = WR * TB * 16, BN = WC * TA * 16, XL = BM / 8, LOADS = XL + BN / 8, L = LOADS / 8;
+// Gate and up by waves without room for a second set of fragments: a stage is read behind its barrier, in one of two ways.
+//   SPREAD  few waves of many sums (256 x 320 and 256 x 384, eight of them): the weight fragments one ahead, a load between every TB matrix
+//           instructions; a load that finds the queue full stops its wave, and all at once behind the barrier they stop every wave.
+//   else    many waves (256 x 192 by twelve, 256 x 256 by sixteen of 64 x 64): while one waits another one multiplies, so each reads all
+//           fragments of half a stage before its products, and the loads of the next stage, which in a ring of two has only this stage's time
+//           to arrive, all go out first.  [11264, 2048], weights from memory, us, so / spread / by eight waves (of 64 x 96 with two sets
+//           of fragments, of 64 x 128 spread): 800 rows 46.4 / 49.8 / 50.3, 1,132 50.2 / 56.5 / 55.8, 1,280 51.7 / 57.3 / 57.5; [16384, 2048] 700 rows
+//           47.5 / 56.3 / 56.9, 2,048 107 / 117 / 120.
+template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD>
+__global__ void __launch_bounds__(WR * WC * 64)
+tile_lean_kernel(TileArgs t) {
+  constexpr int WAVES = WR * WC, BM = WR * TB * 16, BN = WC * TA * 16, XL = BM / 8, LOADS = XL + BN / 8, L = (LOADS + WAVES - 1) / WAVES;
   constexpr int STAGE = LOADS * 1024, HALF = TA * 8;
-  static_assert(LOADS % 8 == 0, "every wave brings in as many");
-  static_assert(L < 2 * TA, "a load between every TB matrix instructions, from the second on");
+  constexpr bool EVEN = LOADS % WAVES == 0;
+  static_assert(!SPREAD || L < 2 * TA, "a load between every TB matrix instructions, from the second on");
+  static_assert(!SPREAD || (TB <= TA && TA % 2 == 0), "the second half's x fragments are read in the first, its first weights in the slot that is free");
   static_assert((STAGES - 2) * L <= 63, "more loads in flight than the counter holds");
   extern __shared__ __align__(1024) char tg_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -413,7 +420,7 @@ tile_wide_kernel(TileArgs t) {
   uint32_t off[L];
 #pragma unroll
   for (int j = 0; j < L; ++j) {
-    const int f = wave * L + j;
+    const int f = EVEN || wave * L + j < LOADS ? wave * L + j : LOADS - 1;      // (the last one again)
     uint32_t row;
     if (f < XL) {
       row = m0 + f * 8 + lrow;
@@ -430,8 +437,12 @@ tile_wide_kernel(TileArgs t) {
   uint32_t ri = 0;
   auto load = [&](auto jc) {                   // the wave's j-th load of the stage that is asked for next
     constexpr int j = decltype(jc)::value;
-    load_to_ring<j * 1024>(wave * L + j < XL ? xb : wb, off[j], mine + ri);
+    const int f = wave * L + j;
+    const char* base = f < XL ? xb : wb;
+    if constexpr (EVEN) load_to_ring<j * 1024>(base, off[j], mine + ri);
+    else load_to_ring<0>(base, off[j], lds0 + (f < LOADS ? f : LOADS - 1) * 1024 + ri);
   };
+  auto loads = [&]() { [&]<int... J>(std::integer_sequence<int, J...>) { (load(Int<J>()), ...); }(std::make_integer_sequence<int, L>()); };
   auto advance = [&]() {
     xb += 128;
     wb += 128;
@@ -450,7 +461,7 @@ tile_wide_kernel(TileArgs t) {
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < nst) {
-      [&]<int... J>(std::integer_sequence<int, J...>) { (load(Int<J>()), ...); }(std::make_integer_sequence<int, L>());
+      loads();
       advance();
     }
   uint32_t stage = 0;
@@ -461,22 +472,39 @@ tile_wide_kernel(TileArgs t) {
     __builtin_amdgcn_s_barrier();                                // and everybody else's; everybody is done with the stage before
     asm volatile("" ::: "memory");
     const uint32_t blk0 = stage + (kb ^ (col & 7)) * 16, blk1 = stage + ((4 + kb) ^ (col & 7)) * 16;
-    bf16x8 xf[2][TB], wf[2];
+    if constexpr (SPREAD) {
+      bf16x8 xf[2][TB], wf[2];
 #pragma unroll
-    for (int b = 0; b < TB; ++b) xf[0][b] = *reinterpret_cast<const bf16x8*>(xl + blk0 + b * 2048);
-    wf[0] = *reinterpret_cast<const bf16x8*>(wl + blk0);
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-      ([&] {
-        constexpr int kc = I / TA, a = I % TA;
+      for (int b = 0; b < TB; ++b) xf[0][b] = *reinterpret_cast<const bf16x8*>(xl + blk0 + b * 2048);
+      wf[0] = *reinterpret_cast<const bf16x8*>(wl + blk0);
+      [&]<int... I>(std::integer_sequence<int, I...>) {
+        ([&] {
+          constexpr int kc = I / TA, a = I % TA;
+          const uint32_t blk = kc ? blk1 : blk0;
+          if constexpr (a + 1 < TA) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk + (a + 1) * 2048);
+          else if constexpr (kc == 0) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk1);
+          if constexpr (kc == 0 && a + TB >= TA) xf[1][a + TB - TA] = *reinterpret_cast<const bf16x8*>(xl + blk1 + (a + TB - TA) * 2048);
+          if constexpr (MORE && I >= 1 && I <= L) load(Int<I - 1>());
+#pragma unroll
+          for (int b = 0; b < TB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a & 1], xf[kc][b], acc[a][b], 0, 0, 0);
+        }(), ...);
+      }(std::make_integer_sequence<int, 2 * TA>());
+    } else {
+      if (MORE) loads();
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
         const uint32_t blk = kc ? blk1 : blk0;
-        if constexpr (a + 1 < TA) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk + (a + 1) * 2048);
-        else if constexpr (kc == 0) wf[(a + 1) & 1] = *reinterpret_cast<const bf16x8*>(wl + blk1);
-        if constexpr (kc == 0 && a + TB >= TA) xf[1][a + TB - TA] = *reinterpret_cast<const bf16x8*>(xl + blk1 + (a + TB - TA) * 2048);
-        if constexpr (MORE && I >= 1 && I <= L) load(Int<I - 1>());
+        bf16x8 xf[TB], wf[TA];
 #pragma unroll
-        for (int b = 0; b < TB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a & 1], xf[kc][b], acc[a][b], 0, 0, 0);
-      }(), ...);
-    }(std::make_integer_sequence<int, 2 * TA>());
+        for (int a = 0; a < TA; ++a) wf[a] = *reinterpret_cast<const bf16x8*>(wl + blk + a * 2048);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) xf[b] = *reinterpret_cast<const bf16x8*>(xl + blk + b * 2048);
+#pragma unroll
+        for (int a = 0; a < TA; ++a)
+#pragma unroll
+          for (int b = 0; b < TB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf[b], acc[a][b], 0, 0, 0);
+      }
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // this wave has read the stage before the next barrier
     if (MORE) advance();
     stage = stage + STAGE == STAGES * STAGE ? 0 : stage + STAGE;
@@ -520,15 +548,15 @@ static int launch(TileArgs t, const TileRope& rope, int K, int units, hipStream_
   return 0;
 }
 
-template <int TA, int TB, int STAGES>
-static int launch_wide(TileArgs t, int K, hipStream_t s) {
-  constexpr int BM = TB * 64, BN = TA * 32, lds = STAGES * (BM + BN) * 128;
+template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD>
+static int launch_lean(TileArgs t, int K, hipStream_t s) {
+  constexpr int BM = WR * TB * 16, BN = WC * TA * 16, lds = STAGES * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "LDS");
-  auto kernel = tile_wide_kernel<TA, TB, STAGES>;
+  auto kernel = tile_lean_kernel<WR, WC, TA, TB, STAGES, SPREAD>;
   if (mie_allow_lds((const void*)kernel, lds, "tile_gemm")) return -1;
   int grid;
   if (grid_of(t, BM, BN / 2, K, 1, &grid)) return -1;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, s, t);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(WR * WC * 64), lds, s, t);
   MIE_CHECK_LAUNCH("tile_gemm");
   return 0;
 }
@@ -627,10 +655,9 @@ MIE_EXPORT int mie_tile_gemm_qkv_rope(const void* X, long ldx, const void* W, lo
 }
 
 // Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: measured at
-// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 256, 256 x 320 and 256 x 384 are tile_wide_kernel's, the others tile_gemm_kernel's, of which
+// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 192 and wider are tile_lean_kernel's, the others tile_gemm_kernel's, of which
 // the first 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  Own tile of before / now, us: 160 rows 25.2 / 22.4, 256 26.0 /
-// 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9.  256 x 256, weights from memory, by eight waves of 64 x 128
-// / four of 128 x 128 with two sets of fragments: 1,132 rows 54.1 / 57.5, 1,200 54.3 / 57.8, 1,280 55.1 / 58.9.
+// 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9.
 constexpr struct { int bm, bn; float us; } TILE_STAGE_US[] = {
   {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f},
   {128, 128, 0.72f}, {128, 192, 0.96f}, {192, 192, 1.12f}, {256, 320, 1.94f}};
@@ -678,13 +705,13 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {
     case 1: return launch<2, 2, 4, 6, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 2: return launch<4, 2, 4, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    case 3: return launch<4, 2, 6, 4, 2, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    case 4: return launch_wide<8, 4, 2>(t, K, s);
-    case 5: return launch_wide<12, 4, 2>(t, K, s);
+    case 3: return launch_lean<4, 3, 4, 4, 2, false>(t, K, s);
+    case 4: return launch_lean<4, 4, 4, 4, 2, false>(t, K, s);
+    case 5: return launch_lean<4, 2, 12, 4, 2, true>(t, K, s);
     case 6: return launch<2, 2, 4, 4, 4, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 7: return launch<2, 2, 6, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 8: return launch<2, 2, 6, 6, 3, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    default: return launch_wide<10, 4, 2>(t, K, s);
+    default: return launch_lean<4, 2, 10, 4, 2, true>(t, K, s);
   }
 }
 
