@@ -548,6 +548,16 @@ static int launch(TileArgs t, const TileRope& rope, int K, int units, hipStream_
   return 0;
 }
 
+// The same with the wave that reads the weights ahead where three or more rows of tiles share that reading.  Of one or two rows each such wave
+// has 64 rows or more of every eight stages to itself, and the others wait for it at the barriers: [11264, 2048], us, with / without it (128 x 128):
+// 129 rows 23.9 / 18.9, 256 23.6 / 22.1; [16384, 2048] 129 rows 27.3 / 23.1, 256 27.3 / 24.2, 450 (256 x 128) 37.1 / 31.4.  Of three and more
+// 384 rows of [8192, 2048] 21.2 / 21.7, 512 21.0 / 21.5, 1,024 of [2048, 2048] 16.8 / 18.4.
+template <int WR, int WC, int TA, int TB, int RING, int EPI>
+static int launch_ahead(const TileArgs& t, int K, int units, hipStream_t s) {
+  return t.M <= 2 * WR * TB * 16 ? launch<WR, WC, TA, TB, RING, 0, EPI>(t, TileRope{}, K, units, s)
+                                 : launch<WR, WC, TA, TB, RING, 8, EPI>(t, TileRope{}, K, units, s);
+}
+
 template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD>
 static int launch_lean(TileArgs t, int K, hipStream_t s) {
   constexpr int BM = WR * TB * 16, BN = WC * TA * 16, lds = STAGES * (BM + BN) * 128;
@@ -704,11 +714,11 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   float us;
   switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {
     case 1: return launch<2, 2, 4, 6, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    case 2: return launch<4, 2, 4, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
+    case 2: return launch_ahead<4, 2, 4, 4, 3, TG_SWIGLU>(t, K, 1, s);
     case 3: return launch_lean<4, 3, 4, 4, 2, false>(t, K, s);
     case 4: return launch_lean<4, 4, 4, 4, 2, false>(t, K, s);
     case 5: return launch_lean<4, 2, 12, 4, 2, true>(t, K, s);
-    case 6: return launch<2, 2, 4, 4, 4, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
+    case 6: return launch_ahead<2, 2, 4, 4, 4, TG_SWIGLU>(t, K, 1, s);
     case 7: return launch<2, 2, 6, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 8: return launch<2, 2, 6, 6, 3, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     default: return launch_lean<4, 2, 10, 4, 2, true>(t, K, s);

@@ -499,7 +499,9 @@ def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
                                   (525, 64, 5200, 0.98, True, 192128), (1307, 128, 2272, 0.98, True, 192128), (457, 192, 8184, 0.99, True, 256128),
                                   (959, 64, 3896, 0.99, True, 256128), (690, 128, 7176, 1.33, True, 256192), (1193, 192, 3488, 1.33, True, 256192),
                                   (1169, 64, 7880, 2.35, True, 256320), (1479, 192, 5976, 2.35, True, 256320),
-                                  (790, 1152, 5640, 1.33, True, 256192), (1129, 1152, 5624, 1.57, True, 256256)])
+                                  (790, 1152, 5640, 1.33, True, 256192), (1129, 1152, 5624, 1.57, True, 256256),
+                                  (250, 1152, 5640, 0.76, True, 128128), (381, 1152, 4104, 0.76, True, 128128), (505, 1152, 8152, 0.99, True, 256128),
+                                  (1010, 1152, 4088, 0.99, True, 256128)])
 def test_tile_product_swiglu(engine_ops, case):
     """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
     sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
