@@ -386,15 +386,15 @@ tile_gemm_kernel(TileArgs t, TileRope rope) {
   }
 }
 
-// Gate and up by waves without room for a second set of fragments: a stage is read behind its barrier, in one of two ways.
+// Gate and up, and parts of K, by waves without room for a second set of fragments: a stage is read behind its barrier, in one of two ways.
 //   SPREAD  few waves of many sums (256 x 320 and 256 x 384, eight of them): the weight fragments one ahead, a load between every TB matrix
 //           instructions; a load that finds the queue full stops its wave, and all at once behind the barrier they stop every wave.
 //   else    many waves (256 x 192 by twelve, 256 x 256 by sixteen of 64 x 64): while one waits another one multiplies, so each reads all
 //           fragments of half a stage before its products, and the loads of the next stage, which in a ring of two has only this stage's time
 //           to arrive, all go out first.  [11264, 2048], weights from memory, us, so / spread / by eight waves (of 64 x 96 with two sets
 //           of fragments, of 64 x 128 spread): 800 rows 46.4 / 49.8 / 50.3, 1,132 50.2 / 56.5 / 55.8, 1,280 51.7 / 57.3 / 57.5; [16384, 2048] 700 rows
-//           47.5 / 56.3 / 56.9, 2,048 107 / 117 / 120.
-template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD>
+//           47.5 / 56.3 / 56.9, 2,048 107 / 117 / 120.  Two workgroups a compute unit, each with a ring of two, are the same at parts of K.
+template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD, int EPI>
 __global__ void __launch_bounds__(WR * WC * 64)
 tile_lean_kernel(TileArgs t) {
   constexpr int WAVES = WR * WC, BM = WR * TB * 16, BN = WC * TA * 16, XL = BM / 8, LOADS = XL + BN / 8, L = (LOADS + WAVES - 1) / WAVES;
@@ -403,6 +403,7 @@ tile_lean_kernel(TileArgs t) {
   static_assert(!SPREAD || L < 2 * TA, "a load between every TB matrix instructions, from the second on");
   static_assert(!SPREAD || (TB <= TA && TA % 2 == 0), "the second half's x fragments are read in the first, its first weights in the slot that is free");
   static_assert((STAGES - 2) * L <= 63, "more loads in flight than the counter holds");
+  static_assert(EPI == TG_SWIGLU || EPI == TG_F32, "what follows");
   extern __shared__ __align__(1024) char tg_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kb = lane >> 4;
@@ -411,12 +412,13 @@ tile_lean_kernel(TileArgs t) {
     const int total = gridDim.x, q = total >> 3, r = total & 7, x = id & 7, y = id >> 3;
     id = x * q + (x < r ? x : r) + y;
   }
-  const int tm = id % t.mt, tn = id / t.mt;
-  const int m0 = tm * BM, n0 = tn * (BN / 2), nst = t.stages_all;
+  const int tm = id % t.mt, rest = id / t.mt, unit = EPI == TG_F32 ? rest / t.nt : 0, tn = rest - unit * t.nt;
+  const int m0 = tm * BM, n0 = tn * (EPI == TG_SWIGLU ? BN / 2 : BN);
+  const int st0 = unit * t.stages_unit, left = t.stages_all - st0, nst = EPI == TG_F32 && t.stages_unit < left ? t.stages_unit : left;
   const int lrow = lane >> 3;
   const uint32_t lblk = ((lane & 7) ^ lrow) * 16;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)tg_lds;
-  const char *xb = reinterpret_cast<const char*>(t.X), *wb = reinterpret_cast<const char*>(t.W);
+  const char *xb = reinterpret_cast<const char*>(t.X) + (size_t)st0 * 128, *wb = reinterpret_cast<const char*>(t.W) + (size_t)st0 * 128;
   uint32_t off[L];
 #pragma unroll
   for (int j = 0; j < L; ++j) {
@@ -428,7 +430,7 @@ tile_lean_kernel(TileArgs t) {
       off[j] = row * t.ldx + lblk;
       continue;
     }
-    const int r = (f - XL) * 8, w = r / (2 * HALF), at = r - w * 2 * HALF, up = at >= HALF;
+    const int r = (f - XL) * 8, w = EPI == TG_SWIGLU ? r / (2 * HALF) : 0, at = r - w * 2 * HALF, up = EPI == TG_SWIGLU && at >= HALF;
     row = n0 + w * HALF + at - up * HALF + lrow;
     if ((int)row >= t.N) row = t.N - 1;
     off[j] = (row + up * t.N) * t.ldw + lblk;
@@ -516,7 +518,16 @@ tile_lean_kernel(TileArgs t) {
 #pragma unroll
   for (int b = 0; b < TB; ++b) {
     const int m = m0 + (wr * TB + b) * 16 + col;
-    store_swiglu<TA, TB>(t, acc, b, m, n0 + wc * HALF, kb);
+    if constexpr (EPI == TG_SWIGLU) {
+      store_swiglu<TA, TB>(t, acc, b, m, n0 + wc * HALF, kb);
+    } else if (m < t.M) {
+      float* row = (float*)t.out + unit * t.unit_stride + (size_t)m * t.ldo;
+#pragma unroll
+      for (int a = 0; a < TA; ++a) {
+        const int n = n0 + (wc * TA + a) * 16 + 4 * kb;
+        if (n < t.N) *reinterpret_cast<f32x4*>(row + n) = acc[a][b];       // N is a multiple of 8
+      }
+    }
   }
 }
 
@@ -551,21 +562,23 @@ static int launch(TileArgs t, const TileRope& rope, int K, int units, hipStream_
 // The same with the wave that reads the weights ahead where three or more rows of tiles share that reading.  Of one or two rows each such wave
 // has 64 rows or more of every eight stages to itself, and the others wait for it at the barriers: [11264, 2048], us, with / without it (128 x 128):
 // 129 rows 23.9 / 18.9, 256 23.6 / 22.1; [16384, 2048] 129 rows 27.3 / 23.1, 256 27.3 / 24.2, 450 (256 x 128) 37.1 / 31.4.  Of three and more
-// 384 rows of [8192, 2048] 21.2 / 21.7, 512 21.0 / 21.5, 1,024 of [2048, 2048] 16.8 / 18.4.
+// 384 rows of [8192, 2048] 21.2 / 21.7, 512 21.0 / 21.5, 1,024 of [2048, 2048] 16.8 / 18.4.  Parts of K: 129 rows of [4096, 14336] in
+// four 42.9 / 35.8, 256 45.3 / 42.2, 129 of [2048, 5632] in eight 13.2 / 12.3, 256 of [8192, 4096] in two 29.5 / 26.1; of four rows of tiles 512 of
+// [4096, 14336] in two 64.6 / 71.8.
 template <int WR, int WC, int TA, int TB, int RING, int EPI>
 static int launch_ahead(const TileArgs& t, int K, int units, hipStream_t s) {
   return t.M <= 2 * WR * TB * 16 ? launch<WR, WC, TA, TB, RING, 0, EPI>(t, TileRope{}, K, units, s)
                                  : launch<WR, WC, TA, TB, RING, 8, EPI>(t, TileRope{}, K, units, s);
 }
 
-template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD>
-static int launch_lean(TileArgs t, int K, hipStream_t s) {
+template <int WR, int WC, int TA, int TB, int STAGES, bool SPREAD, int EPI>
+static int launch_lean(TileArgs t, int K, int units, hipStream_t s) {
   constexpr int BM = WR * TB * 16, BN = WC * TA * 16, lds = STAGES * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "LDS");
-  auto kernel = tile_lean_kernel<WR, WC, TA, TB, STAGES, SPREAD>;
+  auto kernel = tile_lean_kernel<WR, WC, TA, TB, STAGES, SPREAD, EPI>;
   if (mie_allow_lds((const void*)kernel, lds, "tile_gemm")) return -1;
   int grid;
-  if (grid_of(t, BM, BN / 2, K, 1, &grid)) return -1;
+  if (grid_of(t, BM, EPI == TG_SWIGLU ? BN / 2 : BN, K, units, &grid)) return -1;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(WR * WC * 64), lds, s, t);
   MIE_CHECK_LAUNCH("tile_gemm");
   return 0;
@@ -715,13 +728,13 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {
     case 1: return launch<2, 2, 4, 6, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 2: return launch_ahead<4, 2, 4, 4, 3, TG_SWIGLU>(t, K, 1, s);
-    case 3: return launch_lean<4, 3, 4, 4, 2, false>(t, K, s);
-    case 4: return launch_lean<4, 4, 4, 4, 2, false>(t, K, s);
-    case 5: return launch_lean<4, 2, 12, 4, 2, true>(t, K, s);
+    case 3: return launch_lean<4, 3, 4, 4, 2, false, TG_SWIGLU>(t, K, 1, s);
+    case 4: return launch_lean<4, 4, 4, 4, 2, false, TG_SWIGLU>(t, K, 1, s);
+    case 5: return launch_lean<4, 2, 12, 4, 2, true, TG_SWIGLU>(t, K, 1, s);
     case 6: return launch_ahead<2, 2, 4, 4, 4, TG_SWIGLU>(t, K, 1, s);
     case 7: return launch<2, 2, 6, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     case 8: return launch<2, 2, 6, 6, 3, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
-    default: return launch_lean<4, 2, 10, 4, 2, true>(t, K, s);
+    default: return launch_lean<4, 2, 10, 4, 2, true, TG_SWIGLU>(t, K, 1, s);
   }
 }
 
@@ -733,5 +746,8 @@ MIE_EXPORT int mie_tile_gemm_units(const void* X, long ldx, const void* W, long 
   if (units < 1 || (units - 1) * per >= stages) MIE_FAIL("tile_gemm_units: %d units of %d stages", units, stages);
   TileArgs t = arguments(X, ldx, W, ldw, part, N, M, N);
   t.unit_stride = (long)M * N;
-  return launch<2, 2, 4, 4, 4, 8, TG_F32>(t, TileRope{}, K, units, s);
+  // a workgroup a compute unit and a deep ring, or two and a short one each: weights from memory, us, deep / short, 300 rows of [4096, 14336] in
+  // five parts 56.8 / 51.3, 384 65.7 / 53.9, of [4096, 4096] 26.3 / 20.9; 384 rows of [8192, 4096] in two 46.5 / 37.5
+  const long groups = (long)((M + 127) / 128) * ((N + 127) / 128) * units;
+  return groups > mie_compute_units() ? launch_lean<4, 2, 4, 2, 2, false, TG_F32>(t, K, units, s) : launch_ahead<2, 2, 4, 4, 4, TG_F32>(t, K, units, s);
 }

@@ -443,7 +443,7 @@ def test_mid_linear(engine_ops, shape):
         torch.testing.assert_close(out.materialize().double(), want, atol=2e-2, rtol=1e-2)
 
 
-@pytest.mark.parametrize("shape", [(129, 4096, 264), (300, 4160, 2048), (512, 5632, 136), (385, 4096, 4104)])
+@pytest.mark.parametrize("shape", [(129, 4096, 264), (300, 4160, 2048), (512, 5632, 136), (385, 4096, 4104), (255, 4672, 2056), (509, 4160, 5128)])
 def test_tile_product_in_parts(engine_ops, shape):
     """A long K in parts on the own tiles, added into the stream with and without the norm behind it: rows and columns beyond
     the tiles, K whose stages do not divide over the parts; the float32 sums within the worst case of their additions."""
