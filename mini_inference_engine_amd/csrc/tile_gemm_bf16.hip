@@ -636,6 +636,26 @@ MIE_EXPORT int mie_tile_gemm_tile(int M, int N, int K) {
   return i < 0 ? 0 : PRODUCT_TILES[i].bm * 1000 + PRODUCT_TILES[i].bn;
 }
 
+// Whether the tile that tile_for picks for a product that is added also beats the library's.  (One that is rotated saves a kernel of 8 us
+// beside it and does wherever there is a tile.)  It does not, us, weights from memory, own / library:
+//   - on a tenth to a quarter of the compute units with more than 16 stages each, where the library cuts K: 129 to 256 rows of [1024, 2048]
+//     9.2 / 8.4, of [1024, 3072] 14.7 / 10.4, of [1536, 1536] 7.9 / 7.5 (but of [1024, 1024] 6.3 / 8.2, 300 rows of [1024, 3072] 14.2 / 15.6);
+//   - on 256 x 128 tiles for three quarters of the compute units or fewer: 1,536 rows of [4096, 4096] 59.3 / 56.2, of [4096, 1024] 23.0 / 22.1, 768 of
+//     [8192, 8192] 114 / 102 (1,700 and 1,800 rows of [4096, 4096], 224 and 256 of them, 58.8 / 62.3 and 62.2 / 63.6);
+//   - on the two widest tiles for 8,192 columns and more over a K of 2,048 or less, whose start and end weigh most: 600 rows 32.4 / 29.8, 900 40.7 /
+//     38.8, 1,024 42.7 / 40.7 (of [8192, 8192] 123 / 127).
+// Of 397 products of 129 to 2,048 rows 8 remain that the library makes up to 15 % faster (384 rows of [4096, 2048] 16.4 / 15.7, 129 of [8192, 2048]
+// 20.0 / 17.0); all of them together take 0.88 times the library's time.
+MIE_EXPORT int mie_tile_gemm_add_gains(int M, int N, int K) {
+  const int i = tile_for(M, N, K);
+  if (i < 0) return 0;
+  const auto& p = PRODUCT_TILES[i];
+  const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), cu = mie_compute_units();
+  if (32 * tiles <= 9 * cu && K > 1024) return 0;
+  if (p.bm == 256 && 4 * tiles <= 3 * cu) return 0;
+  return !(p.bm * p.bn >= 128 * 192 && N >= 8192 && K <= 2048);
+}
+
 template <int EPI>
 static int launch_tile(const TileArgs& t, const TileRope& rope, int K, hipStream_t s) {
   switch (tile_for(t.M, t.N, K)) {

@@ -415,9 +415,13 @@ class HipBackend(KernelBackend):
         return -(-(K // 64) // -(-(K // 64) // units)) if units >= 2 else 0      # as many as their stages come out at
 
     def _tile_takes(self, x, w, bias) -> bool:
-        """Whether the own tiles take x w^T with what follows it (added into the stream, or rotated): where one of them has no more
-        workgroups than run at once (tile_for in csrc/tile_gemm_bf16.hip has both sides measured)."""
+        """Whether the own tiles take x w^T with the rotation behind it: where one of them has no more workgroups than run at once
+        (tile_for in csrc/tile_gemm_bf16.hip has both sides measured)."""
         return self._tile_ok(x, w, bias) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_tile(x.shape[0], w.shape[0], w.shape[1]))
+
+    def _tile_add_gains(self, x, w) -> bool:
+        """The same of x w^T that is added into the stream, where the library's product is not the faster one beside it."""
+        return self._tile_ok(x, w, None) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_add_gains(x.shape[0], w.shape[0], w.shape[1]))
 
     def _tile_swiglu_gains(self, x, w, intermediate) -> bool:
         """Whether the own gate/up product with SwiGLU on its sums beats the library's and silu_mul: its estimate (a stage's time
@@ -486,7 +490,7 @@ class HipBackend(KernelBackend):
             if bias is None and sink is not None:
                 # the product adds its float32 sums to the stream itself (C = C + A B in place): the stream is
                 # not read and written once more by a kernel of its own
-                if sink.stream.data_ptr() % 16 == 0 and self._tile_takes(x, w, None):
+                if sink.stream.data_ptr() % 16 == 0 and self._tile_add_gains(x, w):
                     lib = self.lib("tile_gemm_bf16")
                     library.check(lib, lib.mie_tile_gemm_add(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(sink.stream), N, M, N, K,
                                                              self._stream()))

@@ -1,0 +1,18 @@
+"""Which kernel a bfloat16 product of more than 128 rows takes: the rules of csrc/tile_gemm_bf16.hip, asked of the library itself
+(they are host code, for 256 compute units where there is no GPU to ask)."""
+import pytest
+
+from mini_inference_engine_amd.kernels import library, modules  # noqa: F401
+
+
+# rows, columns, K and whether the own tile adds into the stream faster than the library: few workgroups over a long K, the widest
+# tile on three quarters of the chip, the widest tiles of many columns over a short K, and each one's other side
+@pytest.mark.parametrize("case", [(129, 1024, 2048, False), (256, 1024, 3072, False), (192, 1536, 1536, False), (256, 1024, 1024, True), (300, 1024, 3072, True),
+                                  (1536, 4096, 4096, False), (1500, 4096, 14336, False), (768, 8192, 8192, False), (1700, 4096, 4096, True),
+                                  (2048, 4096, 14336, True), (600, 8192, 2048, False), (1024, 8192, 2048, False), (1024, 8192, 8192, True),
+                                  (129, 2048, 2048, True), (512, 2048, 2048, True), (1132, 2048, 5632, True), (2048, 2048, 5632, True), (4096, 8192, 1024, False)])
+def test_added_products_on_own_tiles_where_they_gain(case):
+    M, N, K, gains = case
+    lib = library.load("tile_gemm_bf16")
+    assert bool(lib.mie_tile_gemm_add_gains(M, N, K)) == gains
+    assert lib.mie_tile_gemm_tile(M, N, K) > 0 or not gains
