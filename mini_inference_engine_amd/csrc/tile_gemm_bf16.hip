@@ -656,6 +656,13 @@ MIE_EXPORT int mie_tile_gemm_add_gains(int M, int N, int K) {
   return !(p.bm * p.bn >= 128 * 192 && N >= 8192 && K <= 2048);
 }
 
+// Stages that a wave reads the weights of an added product ahead, 0: none does.  It saves the product time by itself at any size (2,048 rows of
+// [4096, 14336], weights from memory, 100 ms on end: 189 us with it, 197 without, 204 by the library), but a product of 200 us takes its power from
+// the kernels around it, and in whole steps of such products the saving was gone: 2,048 tokens behind 4,096 in four layers of [4096, 4096]
+// and [4096, 14336], three runs, us, with it / without for the second / library: 4,042 / 4,033 / 4,076, 4,055 / 4,010 / 4,086, 4,032 / 4,014 / 4,061.
+// Smaller ones keep it: [4096, 11008], 2,048 rows 3,295 / 3,376 / 3,445 a step, [4096, 14336], 1,700 rows 3,265 / 3,348 / 3,359.
+MIE_EXPORT int mie_tile_gemm_add_ahead(int M, int N, int K) { return (double)M * N * K > 1.1e11 ? 0 : 8; }
+
 template <int EPI>
 static int launch_tile(const TileArgs& t, const TileRope& rope, int K, hipStream_t s) {
   switch (tile_for(t.M, t.N, K)) {
@@ -668,7 +675,10 @@ static int launch_tile(const TileArgs& t, const TileRope& rope, int K, hipStream
     case 6: return launch<2, 2, 4, 4, 4, 8, EPI>(t, rope, K, 1, s);
     case 7: return launch<2, 2, 5, 4, 4, 8, EPI>(t, rope, K, 1, s);
     case 8: return launch<2, 2, 6, 4, 3, 8, EPI>(t, rope, K, 1, s);
-    case 9: return launch<4, 2, 4, 4, 3, 8, EPI>(t, rope, K, 1, s);
+    case 9:
+      if constexpr (EPI == TG_ADD)
+        if (!mie_tile_gemm_add_ahead(t.M, t.N, K)) return launch<4, 2, 4, 4, 3, 0, EPI>(t, rope, K, 1, s);
+      return launch<4, 2, 4, 4, 3, 8, EPI>(t, rope, K, 1, s);
   }
   MIE_FAIL("tile_gemm: %d rows of [%d, %d] are no one round of any tile", t.M, t.N, K);
 }

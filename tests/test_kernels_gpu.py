@@ -533,7 +533,7 @@ def test_tile_product_swiglu(engine_ops, case):
 # rows, columns, K and the tile: every tile, edges in rows and columns, K of one stage, of fewer and of more than the ring holds
 @pytest.mark.parametrize("case", [(137, 72, 64, 64064), (333, 2056, 320, 64064), (138, 5560, 64, 64080), (509, 2552, 576, 64080), (193, 5240, 192, 64096),
                                   (263, 4912, 256, 64128), (513, 4520, 64, 80128), (1131, 2040, 1408, 80128), (520, 4624, 192, 96128), (483, 5392, 64, 128128),
-                                  (2047, 2040, 1088, 128128), (646, 5392, 1024, 128160), (642, 5488, 320, 128192), (1027, 5416, 448, 256128)])
+                                  (2047, 2040, 1088, 128128), (646, 5392, 1024, 128160), (642, 5488, 320, 128192), (1027, 5416, 448, 256128), (2047, 4096, 14400, 256128)])
 def test_tile_product_added(engine_ops, case):
     """A product on the own tiles added into the stream: every tile; the float32 sums within the worst case of their additions, nothing
     written beyond the last row."""

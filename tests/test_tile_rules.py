@@ -16,3 +16,11 @@ def test_added_products_on_own_tiles_where_they_gain(case):
     lib = library.load("tile_gemm_bf16")
     assert bool(lib.mie_tile_gemm_add_gains(M, N, K)) == gains
     assert lib.mie_tile_gemm_tile(M, N, K) > 0 or not gains
+
+
+@pytest.mark.parametrize("case", [(2048, 4096, 14336, 0), (2047, 4096, 14336, 0), (1792, 4096, 14336, 8), (2048, 4096, 11008, 8), (2048, 4096, 4096, 8)])
+def test_added_products_read_weights_ahead_where_a_step_gains_by_it(case):
+    M, N, K, ahead = case
+    lib = library.load("tile_gemm_bf16")
+    assert lib.mie_tile_gemm_tile(M, N, K) == 256128, "the only tile that such products take"
+    assert lib.mie_tile_gemm_add_ahead(M, N, K) == ahead
