@@ -27,6 +27,8 @@
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_on_8 __attribute__((aligned(8)));      // 16 bytes that begin on 8: one store all the same
 
 enum { TG_F32, TG_ADD, TG_SWIGLU, TG_ROPE };
 
@@ -92,7 +94,7 @@ __device__ __forceinline__ void store_swiglu(const TileArgs& t, const f32x4 (&ac
   for (int a = 0; a + 1 < TA / 2; a += 2) {
     const uint4 v = eight_of_two(four(a), four(a + 1));
     const int at = n + (a + (kb & 1)) * 16 + 8 * (kb >> 1);          // N is a multiple of 8
-    if (m < t.M && at < t.N) *reinterpret_cast<uint4*>(row + at) = v;
+    if (m < t.M && at < t.N) *reinterpret_cast<u32x4_on_8*>(row + at) = u32x4_on_8{v.x, v.y, v.z, v.w};      // (ldo is one of 4)
   }
   if (TA / 2 % 2) {
     const uint2 v = four(TA / 2 - 1);
@@ -752,7 +754,7 @@ MIE_EXPORT int mie_tile_gemm_swiglu_tile(int M, int N) {
 MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long ldw, void* out, long ldo, int M, int N, int K, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
   if (check_operands(X, ldx, W, ldw, out, M, 2L * N, N, K)) return -1;
-  if (ldo < N || (ldo & 7)) MIE_FAIL("tile_gemm_swiglu: output leading dim %ld for %d columns", ldo, N);
+  if (ldo < N || (ldo & 3)) MIE_FAIL("tile_gemm_swiglu: output leading dim %ld for %d columns", ldo, N);
   const TileArgs t = arguments(X, ldx, W, ldw, out, ldo, M, N);
   float us;
   switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {

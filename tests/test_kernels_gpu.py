@@ -519,6 +519,10 @@ def test_tile_product_swiglu(engine_ops, case):
     expect = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
     assert bool(((out[:, :inter].double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-4).all())
     assert bool((out[:, inter:] == 7.0).all()), "nothing beyond the columns"
+    odd = torch.full((M, inter + 4), 7.0, device=DEV, dtype=torch.bfloat16)          # rows that begin on 8 bytes
+    library.check(lib, lib.mie_tile_gemm_swiglu(x.data_ptr(), K, w.data_ptr(), K, odd.data_ptr(), inter + 4, M, inter, K,
+                                                torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(odd[:, :inter], out[:, :inter]) and bool((odd[:, inter:] == 7.0).all())
     assert abs(lib.mie_tile_gemm_swiglu_cost(M, inter, K) - 100 * stage_us * (K // 64)) <= 1
     assert o._tile_swiglu_gains(x, w, inter) == gains
     with counted(o, "tile_gemm_bf16", "mie_tile_gemm_swiglu") as calls:
