@@ -1021,6 +1021,7 @@ MIE_EXPORT int mie_step_attention_takes(int singles, int rows, int max_row_token
   if (D != 64 || singles <= 0 || rows <= 0 || max_row_tokens <= 0 || splits <= 0 || Hkv <= 0 || Hq % Hkv) return 0;
   if ((long)singles * Hkv * ((Hq / Hkv + 15) / 16) * splits > mie_compute_units()) return 0;
   const PrefillPlan plan = prefill_plan(rows, max_row_tokens, Hq, Hkv, mie_compute_units());
+  if (plan.grid.y > 65535 || plan.grid.z > 65535) return 0;          // refused by the portions' own kernel
   return plan.kind != FOUR && (long)plan.grid.x * plan.grid.y * plan.grid.z < 1 << 22;
 }
 

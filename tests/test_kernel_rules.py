@@ -1,5 +1,4 @@
-"""Which kernel a bfloat16 product of more than 128 rows takes: the rules of csrc/tile_gemm_bf16.hip, asked of the library itself
-(they are host code, for 256 compute units where there is no GPU to ask)."""
+"""Which kernels a call takes: rules that the kernel libraries decide on the host (for 256 compute units where there is no GPU to ask)."""
 import pytest
 
 from mini_inference_engine_amd.kernels import library, modules  # noqa: F401
@@ -24,3 +23,13 @@ def test_added_products_read_weights_ahead_where_a_step_gains_by_it(case):
     lib = library.load("tile_gemm_bf16")
     assert lib.mie_tile_gemm_tile(M, N, K) == 256128, "the only tile that such products take"
     assert lib.mie_tile_gemm_add_ahead(M, N, K) == ahead
+
+
+# single tokens, portions, tokens of the longest, query and kv heads, splits: as many single workgroups as compute units and one more, and
+# more portions than a grid of the portions' own kernel has rows for
+@pytest.mark.parametrize("case", [(64, 1, 40, 32, 4, 1, True), (65, 1, 40, 32, 4, 1, False), (16, 1, 40, 32, 4, 4, True), (17, 1, 40, 32, 4, 4, False),
+                                  (1, 65535, 2, 4, 1, 1, True), (1, 65536, 2, 4, 1, 1, False), (1, 1, 0, 32, 4, 1, False), (0, 1, 40, 32, 4, 1, False)])
+def test_steps_whose_attention_is_one_launch(case):
+    lib = library.load("prefill_attention_bf16", ("-DHEAD_DIM=64",))
+    assert bool(lib.mie_step_attention_takes(*case[:-1])) == case[-1]
+    assert not library.load("prefill_attention_bf16", ("-DHEAD_DIM=128",)).mie_step_attention_takes(*case[:-1])
