@@ -501,10 +501,11 @@ def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
                                   (1169, 64, 7880, 2.35, True, 256320), (1479, 192, 5976, 2.35, True, 256320),
                                   (790, 1152, 5640, 1.33, True, 256192), (1129, 1152, 5624, 1.57, True, 256256),
                                   (250, 1152, 5640, 0.76, True, 128128), (381, 1152, 4104, 0.76, True, 128128), (505, 1152, 8152, 0.99, True, 256128),
-                                  (1010, 1152, 4088, 0.99, True, 256128)])
+                                  (1010, 1152, 4088, 0.99, True, 256128), (377, 1152, 5512, 0.98, True, 128192), (525, 1152, 5208, 0.98, True, 192128),
+                                  (1169, 1152, 7880, 2.35, True, 256320), (513, 1152, 5640, 1.33, True, 192192)])
 def test_tile_product_swiglu(engine_ops, case):
-    """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K) with SwiGLU on the float32
-    sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
+    """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K and one whose stages go round the ring)
+    with SwiGLU on the float32 sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
     from mini_inference_engine_amd.kernels import library
     (M, K, inter, stage_us, gains, tile), o = case, engine_ops
     torch.manual_seed(K + inter)
@@ -534,10 +535,13 @@ def test_tile_product_swiglu(engine_ops, case):
     assert lib.mie_tile_gemm_units(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), M, inter, K, K // 64 + 1, None) != 0
 
 
-# rows, columns, K and the tile: every tile, edges in rows and columns, K of one stage, of fewer and of more than the ring holds
+# rows, columns, K and the tile: every tile, edges in rows and columns, K of one stage or of no more than the ring holds, and of more than it
+# holds and is read ahead at once
 @pytest.mark.parametrize("case", [(137, 72, 64, 64064), (333, 2056, 320, 64064), (138, 5560, 64, 64080), (509, 2552, 576, 64080), (193, 5240, 192, 64096),
                                   (263, 4912, 256, 64128), (513, 4520, 64, 80128), (1131, 2040, 1408, 80128), (520, 4624, 192, 96128), (483, 5392, 64, 128128),
-                                  (2047, 2040, 1088, 128128), (646, 5392, 1024, 128160), (642, 5488, 320, 128192), (1027, 5416, 448, 256128), (2047, 4096, 14400, 256128)])
+                                  (2047, 2040, 1088, 128128), (646, 5392, 1024, 128160), (642, 5488, 320, 128192), (1027, 5416, 448, 256128), (2047, 4096, 14400, 256128),
+                                  (263, 3080, 1088, 64064), (395, 2552, 1088, 64080), (395, 3080, 1088, 64096), (333, 4104, 1088, 64128), (509, 5368, 1088, 96128),
+                                  (771, 4912, 1088, 128160), (901, 5368, 1088, 128192), (1290, 5368, 1088, 256128)])
 def test_tile_product_added(engine_ops, case):
     """A product on the own tiles added into the stream: every tile; the float32 sums within the worst case of their additions, nothing
     written beyond the last row."""
@@ -557,16 +561,21 @@ def test_tile_product_added(engine_ops, case):
     assert lib.mie_tile_gemm_tile(4096, 8192, K) == 0 and lib.mie_tile_gemm_add(x.data_ptr(), K + 8, w.data_ptr(), K + 16, held.data_ptr(), N, M, N, K - 8, None) != 0
 
 
-@pytest.mark.parametrize("case", [(137, 2, 1, 16, 64), (333, 32, 4, 64, 320), (300, 3, 3, 80, 128), (512, 32, 4, 64, 192), (700, 5, 2, 48, 64), (1131, 32, 4, 64, 64),
-                                  (2040, 32, 4, 64, 128), (520, 32, 8, 128, 64), (1020, 32, 8, 128, 64), (260, 2, 2, 256, 128), (1500, 7, 1, 112, 64)])
+# rows, q and kv heads, head size, K and the tile: every tile; pairs of tiles within a head, across heads, across q and k and across k and v, and the
+# lone last one of an odd number; K of one stage, of as many as the ring holds and of many more; edges in rows and columns
+@pytest.mark.parametrize("case", [(137, 2, 1, 16, 64, 64064), (333, 32, 4, 64, 320, 64064), (300, 3, 3, 80, 128, 64064), (700, 5, 2, 48, 64, 64064), (260, 2, 2, 256, 128, 64064),
+                                  (512, 32, 4, 64, 192, 64080), (410, 31, 5, 64, 2048, 64080), (560, 32, 4, 64, 2048, 64096), (1500, 7, 1, 112, 64, 64128),
+                                  (700, 32, 4, 64, 2048, 64128), (900, 32, 4, 64, 2048, 80128), (1131, 32, 4, 64, 64, 96128), (1131, 32, 4, 64, 1088, 96128),
+                                  (520, 32, 8, 128, 64, 128128), (1500, 32, 4, 64, 2048, 128128), (2047, 32, 4, 64, 2048, 128160), (1801, 33, 3, 64, 2048, 128160),
+                                  (2040, 32, 4, 64, 128, 128192), (1020, 32, 8, 128, 64, 128192), (1020, 32, 8, 128, 4096, 128192), (1100, 32, 8, 128, 4096, 256128)])
 def test_tile_projection_rotary_store(engine_ops, case):
     """The q/k/v projection of many rows with rotation and cache write on the own tiles' sums: against the same kernels' float32 sums
     finished by a kernel of their own (one rounding of bfloat16 apart where the sums' order differs), other pages untouched."""
     from mini_inference_engine_amd.parts.rope import rotary_tables
-    o, (M, Hq, Hkv, D, K) = engine_ops, case
+    o, (M, Hq, Hkv, D, K, tile) = engine_ops, case
     torch.manual_seed(M + D)
     N, page = (Hq + 2 * Hkv) * D, 32
-    assert o.lib("tile_gemm_bf16").mie_tile_gemm_tile(M, N, K) > 0
+    assert o.lib("tile_gemm_bf16").mie_tile_gemm_tile(M, N, K) == tile, "the case must take the tile it is for"
     pages = -(-M // page) + 3
     cos, sin = (t.to(DEV) for t in rotary_tables(10000.0, D, 3000))
     x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
