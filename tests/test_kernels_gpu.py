@@ -1477,9 +1477,27 @@ def test_attention_of_singles_beside_portions(ops, case, page):
     one = SimpleNamespace(token_row=step.token_row[:n], positions=step.positions[:n], num_rows=n, max_context=max(contexts), num_tokens=n, num_decode_rows=n,
                           max_row_tokens=1, row_start=None, row_position=None)
     alone = o.paged_attention(q[:n], Hq, Hkv, D, kc, vc, group, one, D ** -0.5, window or None, sink=sink)
-    # weights and results are rounded to bfloat16 on both sides: 2^-8 of the largest value a sum holds, each
-    bound = 4 * 2.0 ** -8 * float(vc[used].nan_to_num(0.0).abs().max())
-    assert float((alone.float() - out[:n].float()).abs().max()) <= bound
+    # on either side the weights, their sum's share in them and the result are rounded to bfloat16, 2^-9 of sum p |v| each at most; one
+    # more for the float32 sums of scores and weights
+    weighed = ref.ref_paged_attention(q[:n], Hq, Hkv, D, plain_k, plain_v.abs(), group.block_tables, step.token_row[:n], step.positions[:n], D ** -0.5,
+                                      window or None, torch.float64, **({} if sink is None else {"sink": sink}))
+    assert bool(((alone.double() - out[:n].double()).abs() <= 7 * 2.0 ** -9 * weighed).all())
+
+
+@pytest.mark.parametrize("key", [0, 31, 2047, 2048, 4095, 4096, 4490, 4499])
+def test_attention_of_singles_beside_portions_finds_a_far_key(ops, key):
+    """One key among 4,500 dominates a single token beside a portion, whose context is cut into three parts of 2,048 keys: a part that is
+    dropped or joined wrongly shows."""
+    o, Hq, Hkv, D, page = ops[torch.bfloat16], 8, 2, 64, 16
+    q, kc, vc, group, step = paged_setup([4500, 700], [1, 130], Hq, Hkv, D, page, torch.bfloat16, seed=key, spike=(0, key))
+    with counted(o, "prefill_attention_bf16", "mie_step_attention", defines=("-DHEAD_DIM=64",)) as calls:
+        out, expect = run_attention(ops, torch.bfloat16, q, kc, vc, group, step, Hq, Hkv, D, 1.0, None)
+    partition, splits = o.decode_splits(1, Hq, Hkv, 4500, None, o.lib("attention_bf16", ("-DHEAD_DIM=64",)).mie_decode_block_keys(), D)
+    assert len(calls) == 1 and splits > 1 and partition <= o.STEP_SPLIT_KEYS == 2048, "one launch, parts of 2,048 keys"
+    pg, off = int(group.block_tables[0, key // page]), key % page
+    v_key = vc[pg, :, :, off].double().repeat_interleave(Hq // Hkv, 0).reshape(-1)
+    assert (expect[0] - v_key).abs().max() < 5e-3, "the set-up must make that key dominate"
+    torch.testing.assert_close(out.double(), expect, **SPIKE_TOL[torch.bfloat16])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
