@@ -298,11 +298,13 @@ prefill_attention_body(const dim3 place, const dim3 grid, const bf16* __restrict
     constexpr int LOADS = GROUP_PARTS * D / 32;                // of a wave and step
     const int group = wave * GROUP_PARTS >> 1;
     int page_at = 0, off_at = 0;
+    // (scalar loads in every kernel that this is inlined into: a vector load waits for all loads to the LDS that are on their way)
+    const auto* pages = (const __attribute__((address_space(4))) int*)(uintptr_t)bt;
     auto find_page = [&](int x) {
       int key = key_of(x) + 16 * group;
       key = key < (kmax & ~15) ? key : kmax & ~15;             // beyond the row's keys: its last ones again
       const int idx = page_shift >= 0 ? key >> page_shift : key / page;
-      page_at = bt[idx];
+      page_at = pages[idx];
       off_at = key - idx * page;
     };
     auto bring = [&](int x, int set) {                         // in order, a step apart
@@ -775,8 +777,8 @@ prefill_attention_kernel(const bf16* __restrict__ q, long q_stride, const bf16* 
 // portions, those behind them the single tokens, whose keys and values come in on compute units that the portions leave idle.  By themselves
 // the two kernels follow each other, each with a start and an end, and neither fills the chip: few stretches and long chains of blocks
 // here, a workgroup a row and kv head there.  32 / 4 heads of 64, us, two kernels (and a third that joins parts of contexts) / one: 32
-// rows of 150 to 900 keys beside 701 and 399 tokens 28.2 / 21.9, 8 of 1,500 beside 1,000 27.8 / 20.1, 1 of 900 beside 100 15.5 / 8.8, 64 of
-// 1,500 beside 1,800 55.3 / 51.3.
+// rows of 150 to 900 keys beside 701 and 399 tokens 28.2 / 21.0, 8 of 1,500 beside 1,000 27.8 / 19.6, 1 of 900 beside 100 15.5 / 8.7, 64 of
+// 1,500 beside 1,800 55.9 / 48.7, 1 of 2,040 beside 100 behind 4,000 58.4 / 52.5, beside 1,024 behind 15,000 208 / 183.
 struct SingleRows {
   float *o_part, *lse_part;
   const int* positions;
