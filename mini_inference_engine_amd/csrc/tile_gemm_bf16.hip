@@ -609,6 +609,11 @@ constexpr struct { int bm, bn; float us, fixed; int held; } PRODUCT_TILES[] = {
   {96, 128, 0.375f, 6.0f, 1}, {128, 128, 0.45f, 8.0f, 1}, {128, 160, 0.54f, 10.0f, 1}, {128, 192, 0.68f, 8.5f, 1}, {256, 128, 0.78f, 12.0f, 1}};
 constexpr int PRODUCT_TILES_N = sizeof(PRODUCT_TILES) / sizeof(PRODUCT_TILES[0]);
 
+static long tiles_of(int i, int M, int N) {
+  const auto& p = PRODUCT_TILES[i];
+  return (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+}
+
 // The tile with the least estimate among those whose workgroups all run at once; -1 where none has so few: there the library's largest
 // tiles are faster (us, own / library: 2,048 rows of [6144, 4096] 103 / 88, of [8192, 4096] 122 / 114, of [28672, 4096] 480 / 428).  Two
 // workgroups a compute unit take 1.55 times one's time.  With one round, us, own / library (which for q/k/v leaves the rotation, 8 to 9 us
@@ -621,7 +626,7 @@ static int tile_for(int M, int N, int K) {
   float least = 1e30f;
   for (int i = 0; i < PRODUCT_TILES_N; ++i) {
     const auto& p = PRODUCT_TILES[i];
-    const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), cu = mie_compute_units();
+    const long tiles = tiles_of(i, M, N), cu = mie_compute_units();
     if (tiles > p.held * cu) continue;
     const float us = (p.us * (K / 64) + p.fixed) * (tiles > cu ? 1.55f : 1.f);
     if (us < least) {
@@ -638,8 +643,19 @@ MIE_EXPORT int mie_tile_gemm_tile(int M, int N, int K) {
   return i < 0 ? 0 : PRODUCT_TILES[i].bm * 1000 + PRODUCT_TILES[i].bn;
 }
 
-// Whether the tile that tile_for picks for a product that is added also beats the library's.  (One that is rotated saves a kernel of 8 us
-// beside it and does wherever there is a tile.)  It does not, us, weights from memory, own / library:
+// Whether the tile that tile_for picks for q/k/v also beats the library's product with the rotary kernel, 8 us, behind it.  It does not where
+// a few compute units walk a long K, which the library cuts, us, own / library and rotary kernel: 129 rows of [768, 3072] 13.4 / 12.3, of
+// [640, 2560] 12.5 / 10.9 (36 and 30 tiles), 300 rows of [768, 4096] 18.1 / 17.2, of [768, 8192] 30.5 / 25.0, 192 of [1280, 5120] 24.6 / 19.9 (60 tiles).  On the other
+// side 256 rows of [768, 3072] 13.2 / 13.4 (48 tiles), 350 of [768, 4096] 16.8 / 20.6 (72), 129 of [768, 2048] 10.2 / 12.8; of 365 products of 129 to 2,048
+// rows 2 remain that the library makes up to 1.6 % faster; all of them together take 0.72 times its time.
+MIE_EXPORT int mie_tile_gemm_rope_gains(int M, int N, int K) {
+  const int i = tile_for(M, N, K);
+  if (i < 0) return 0;
+  const long tiles = tiles_of(i, M, N), cu = mie_compute_units();
+  return !(64 * tiles <= 15 * cu && K > 3072) && !(64 * tiles <= 9 * cu && K > 2048);
+}
+
+// Whether the tile that tile_for picks for a product that is added also beats the library's.  It does not, us, weights from memory, own / library:
 //   - on a tenth to a quarter of the compute units with more than 16 stages each, where the library cuts K: 129 to 256 rows of [1024, 2048]
 //     9.2 / 8.4, of [1024, 3072] 14.7 / 10.4, of [1536, 1536] 7.9 / 7.5 (but of [1024, 1024] 6.3 / 8.2, 300 rows of [1024, 3072] 14.2 / 15.6);
 //   - on 256 x 128 tiles for three quarters of the compute units or fewer: 1,536 rows of [4096, 4096] 59.3 / 56.2, of [4096, 1024] 23.0 / 22.1, 768 of
@@ -652,7 +668,7 @@ MIE_EXPORT int mie_tile_gemm_add_gains(int M, int N, int K) {
   const int i = tile_for(M, N, K);
   if (i < 0) return 0;
   const auto& p = PRODUCT_TILES[i];
-  const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), cu = mie_compute_units();
+  const long tiles = tiles_of(i, M, N), cu = mie_compute_units();
   if (32 * tiles <= 9 * cu && K > 1024) return 0;
   if (p.bm == 256 && 4 * tiles <= 3 * cu) return 0;
   return !(p.bm * p.bn >= 128 * 192 && N >= 8192 && K <= 2048);

@@ -414,13 +414,13 @@ class HipBackend(KernelBackend):
         units = min(units, 8, K // 256)
         return -(-(K // 64) // -(-(K // 64) // units)) if units >= 2 else 0      # as many as their stages come out at
 
-    def _tile_takes(self, x, w, bias) -> bool:
-        """Whether the own tiles take x w^T with the rotation behind it: where one of them has no more workgroups than run at once
-        (tile_for in csrc/tile_gemm_bf16.hip has both sides measured)."""
-        return self._tile_ok(x, w, bias) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_tile(x.shape[0], w.shape[0], w.shape[1]))
+    def _tile_rope_gains(self, x, w) -> bool:
+        """Whether the own tiles take x w^T with the rotation behind it: where one of them has no more workgroups than run at once and
+        the library's product and the rotary kernel are not faster (csrc/tile_gemm_bf16.hip has both sides measured)."""
+        return self._tile_ok(x, w, None) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_rope_gains(x.shape[0], w.shape[0], w.shape[1]))
 
     def _tile_add_gains(self, x, w) -> bool:
-        """The same of x w^T that is added into the stream, where the library's product is not the faster one beside it."""
+        """The same of x w^T that is added into the stream."""
         return self._tile_ok(x, w, None) and bool(self.lib("tile_gemm_bf16").mie_tile_gemm_add_gains(x.shape[0], w.shape[0], w.shape[1]))
 
     def _tile_swiglu_gains(self, x, w, intermediate) -> bool:
@@ -1532,7 +1532,7 @@ class HipBackend(KernelBackend):
             M, K = x.shape
             page = self._check_rope_operands("linear_rotary_kv_store", M, K, w_qkv, positions, cos, sin, Hq, Hkv, D,
                                              k_cache, v_cache, slot_mapping)
-            if (not for_attention and self._lt_ok(x, w_qkv) and self._tile_takes(x, w_qkv, None) and D <= 256 and page % 16 == 0
+            if (not for_attention and self._lt_ok(x, w_qkv) and self._tile_rope_gains(x, w_qkv) and D <= 256 and page % 16 == 0
                     and not any(t.data_ptr() % 16 for t in (cos, sin, k_cache, v_cache))):
                 # rotation and cache write on the own tiles' float32 sums: the same expressions, one kernel and 8 us less
                 q = torch.empty((M, Hq * D), dtype=torch.bfloat16, device=x.device)

@@ -52,6 +52,7 @@ register_kernel_module("tile_gemm_bf16", {
     "mie_tile_gemm_swiglu": [P, L, P, L, P, L, I, I, I, P],
     "mie_tile_gemm_units": [P, L, P, L, P, I, I, I, I, P],
     "mie_tile_gemm_tile": [I, I, I],
+    "mie_tile_gemm_rope_gains": [I, I, I],
     "mie_tile_gemm_add_gains": [I, I, I],
     "mie_tile_gemm_add_ahead": [I, I, I],
     "mie_tile_gemm_add": [P, L, P, L, P, L, I, I, I, P],

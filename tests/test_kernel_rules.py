@@ -4,6 +4,17 @@ import pytest
 from mini_inference_engine_amd.kernels import library, modules  # noqa: F401
 
 
+# the same of q/k/v with the rotation behind it: few compute units over a long K, and more of them or a shorter one
+@pytest.mark.parametrize("case", [(129, 768, 3072, False), (129, 640, 2560, False), (300, 768, 4096, False), (192, 1280, 5120, False), (129, 896, 8192, False),
+                                  (256, 768, 3072, True), (350, 768, 4096, True), (129, 768, 2048, True), (129, 2560, 2048, True), (2048, 2560, 2048, True),
+                                  (512, 6144, 4096, True), (2048, 6144, 4096, False)])
+def test_rotated_products_on_own_tiles_where_they_gain(case):
+    M, N, K, gains = case
+    lib = library.load("tile_gemm_bf16")
+    assert bool(lib.mie_tile_gemm_rope_gains(M, N, K)) == gains
+    assert lib.mie_tile_gemm_tile(M, N, K) > 0 or not gains
+
+
 # rows, columns, K and whether the own tile adds into the stream faster than the library: few workgroups over a long K, the widest
 # tile on three quarters of the chip, the widest tiles of many columns over a short K, and each one's other side
 @pytest.mark.parametrize("case", [(129, 1024, 2048, False), (256, 1024, 3072, False), (192, 1536, 1536, False), (256, 1024, 1024, True), (300, 1024, 3072, True),
