@@ -563,8 +563,9 @@ static int launch(TileArgs t, const TileRope& rope, int K, int units, hipStream_
 
 // The same with the wave that reads the weights ahead where three or more rows of tiles share that reading.  Of one or two rows each such wave
 // has 64 rows or more of every eight stages to itself, and the others wait for it at the barriers: [11264, 2048], us, with / without it (128 x 128):
-// 129 rows 23.9 / 18.9, 256 23.6 / 22.1; [16384, 2048] 129 rows 27.3 / 23.1, 256 27.3 / 24.2, 450 (256 x 128) 37.1 / 31.4.  Of three and more
-// 384 rows of [8192, 2048] 21.2 / 21.7, 512 21.0 / 21.5, 1,024 of [2048, 2048] 16.8 / 18.4.  Parts of K: 129 rows of [4096, 14336] in
+// 129 rows 23.9 / 18.9, 256 23.6 / 22.1; [16384, 2048] 129 rows 27.3 / 23.1, 256 27.3 / 24.2, 450 (256 x 128) 37.1 / 31.4, 300 (192 x 128) 31.7 /
+// 26.4, 384 32.3 / 28.9; [28672, 2048] 160 rows (192 x 128) 40.6 / 32.9; [22528, 2048] 129 rows (128 x 192) 36.8 / 27.5, 256 37.6 / 31.7.  Of three and more
+// 450 rows of [11264, 2048] (128 x 192) 28.0 / 26.6, 512 28.3 / 28.2, of [5632, 2048] 22.8 / 24.0 and 23.1 / 26.2; 384 rows of [8192, 2048] 21.2 / 21.7, 512 21.0 / 21.5, 1,024 of [2048, 2048] 16.8 / 18.4.  Parts of K: 129 rows of [4096, 14336] in
 // four 42.9 / 35.8, 256 45.3 / 42.2, 129 of [2048, 5632] in eight 13.2 / 12.3, 256 of [8192, 4096] in two 29.5 / 26.1; of four rows of tiles 512 of
 // [4096, 14336] in two 64.6 / 71.8.
 template <int WR, int WC, int TA, int TB, int RING, int EPI>
@@ -774,13 +775,13 @@ MIE_EXPORT int mie_tile_gemm_swiglu(const void* X, long ldx, const void* W, long
   const TileArgs t = arguments(X, ldx, W, ldw, out, ldo, M, N);
   float us;
   switch (best_tile(M, 2L * N, TILES_TAKEN, TILES, us)) {
-    case 1: return launch<2, 2, 4, 6, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
+    case 1: return launch_ahead<2, 2, 4, 6, 3, TG_SWIGLU>(t, K, 1, s);
     case 2: return launch_ahead<4, 2, 4, 4, 3, TG_SWIGLU>(t, K, 1, s);
     case 3: return launch_lean<4, 3, 4, 4, 2, false, TG_SWIGLU>(t, K, 1, s);
     case 4: return launch_lean<4, 4, 4, 4, 2, false, TG_SWIGLU>(t, K, 1, s);
     case 5: return launch_lean<4, 2, 12, 4, 2, true, TG_SWIGLU>(t, K, 1, s);
     case 6: return launch_ahead<2, 2, 4, 4, 4, TG_SWIGLU>(t, K, 1, s);
-    case 7: return launch<2, 2, 6, 4, 3, 8, TG_SWIGLU>(t, TileRope{}, K, 1, s);
+    case 7: return launch_ahead<2, 2, 6, 4, 3, TG_SWIGLU>(t, K, 1, s);
     case 8: return launch<2, 2, 6, 6, 3, 0, TG_SWIGLU>(t, TileRope{}, K, 1, s);
     default: return launch_lean<4, 2, 10, 4, 2, true, TG_SWIGLU>(t, K, 1, s);
   }

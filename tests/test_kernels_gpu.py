@@ -502,7 +502,8 @@ def test_a_stream_off_16_bytes_is_added_to(engine_ops, ops, case):
                                   (790, 1152, 5640, 1.33, True, 256192), (1129, 1152, 5624, 1.57, True, 256256),
                                   (250, 1152, 5640, 0.76, True, 128128), (381, 1152, 4104, 0.76, True, 128128), (505, 1152, 8152, 0.99, True, 256128),
                                   (1010, 1152, 4088, 0.99, True, 256128), (377, 1152, 5512, 0.98, True, 128192), (525, 1152, 5208, 0.98, True, 192128),
-                                  (1169, 1152, 7880, 2.35, True, 256320), (513, 1152, 5640, 1.33, True, 192192)])
+                                  (1169, 1152, 7880, 2.35, True, 256320), (513, 1152, 5640, 1.33, True, 192192),
+                                  (160, 1152, 14328, 0.98, True, 192128), (383, 1152, 8184, 0.98, True, 192128), (255, 1152, 11256, 0.99, True, 128192)])
 def test_tile_product_swiglu(engine_ops, case):
     """Gate and up on the own tiles (every tile size, edges in rows and columns, the shortest K and one whose stages go round the ring)
     with SwiGLU on the float32 sums, against 64 bits rounded once (2^-8 of a value for bfloat16, and the hardware's exponential beside it)."""
