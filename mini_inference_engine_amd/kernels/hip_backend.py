@@ -397,11 +397,15 @@ class HipBackend(KernelBackend):
     TILE_SPLIT_MIN_K = 4096
 
     def _tile_split(self, x, w, bias, sink=None) -> int:
-        """Parts of K for a product that is added into the stream, 0: the library's.  The library walks all of a long K on few
-        workgroups; parts give every compute unit one, and their sums meet in the kernel that adds and norms anyway, until
-        those sums cost more than they save.  Product, add and norm against the library's and the norm kernel, us: 512 rows
-        of [2048, 5632] 27.9 / 29.6, 384 23.9 / 27.2, of [4096, 14336] 85 / 101 and 68 / 83; 768 rows 128 / 127, and of
-        [2048, 2048] 512 rows 21.4 / 16.7."""
+        """Parts of K for a product that is added into the stream, 0: the own tile's or the library's.  Those walk all of a long K
+        on few workgroups; parts give every compute unit one or two, and their sums meet in the kernel that adds and norms anyway, until
+        those sums cost more than they save.  Product, add and norm, weights from memory, us, parts / own tile / library, each with
+        the norm's kernel: [2048, 5632] 129 rows 18.7 / 28.3 / 23.3, 512 25.9 / 27.4 / 31.9; [4096, 14336] 129 rows 43.9 / 64.1 / 63.0, 384 67.0 /
+        85.4 / 83.5, 512 78.0 / 86.4 / 96.9; [4096, 4096] 129 rows 23.2 / 24.0 / 25.6, 256 24.3 / 24.3 / 27.0, 512 33.7 / 31.8 / 35.6; [2048, 4096] 129
+        rows 16.6 / 22.1 by the faster one, 512 22.8 / 21.6.  Two parts on two workgroups a compute unit leave a fifth to a third of the places empty
+        and lost everywhere (K of 4,096 to 14,336): 300 rows of [8192, 4096] 49.3 / 39.6, 384 of [8192, 14336] 130.7 / 124.6, 512 of [6144, 8192]
+        89.4 / 75.8.  Three to five so are 6 to 22 % faster for [4096, 6656] and longer rows, 450 rows of [3072, 11008] 54.4 / 60.2, [7168, 14336]
+        98 / 107; for K of 4,096 to 5,632 up to 18 % slower (384 rows of [4096, 4096] 31.2 / 30.3, 512 of [3072, 4096] 31.7 / 26.7)."""
         M, (N, K) = x.shape[0], w.shape
         if M > self.TILE_SPLIT_MAX_ROWS or K < self.TILE_SPLIT_MIN_K or N > 8192 or not self._tile_ok(x, w, bias):
             return 0
@@ -411,6 +415,8 @@ class HipBackend(KernelBackend):
         units = 256 // tiles
         if units * tiles < 205:                 # one workgroup a compute unit would leave many without: two
             units = 512 // tiles
+            if units < 3:
+                return 0
         units = min(units, 8, K // 256)
         return -(-(K // 64) // -(-(K // 64) // units)) if units >= 2 else 0      # as many as their stages come out at
 

@@ -1,10 +1,12 @@
 """Which kernels a call takes: rules that the kernel libraries decide on the host (for 256 compute units where there is no GPU to ask)."""
 import pytest
+import torch
 
 from mini_inference_engine_amd.kernels import library, modules  # noqa: F401
+from mini_inference_engine_amd.kernels.hip_backend import HipBackend
 
 
-# the same of q/k/v with the rotation behind it: few compute units over a long K, and more of them or a shorter one
+# rows, columns, K and whether the own tile makes q/k/v with the rotation behind it faster than the library: few compute units over a long K, and more of them or a shorter one
 @pytest.mark.parametrize("case", [(129, 768, 3072, False), (129, 640, 2560, False), (300, 768, 4096, False), (192, 1280, 5120, False), (129, 896, 8192, False),
                                   (256, 768, 3072, True), (350, 768, 4096, True), (129, 768, 2048, True), (129, 2560, 2048, True), (2048, 2560, 2048, True),
                                   (512, 6144, 4096, True), (2048, 6144, 4096, False)])
@@ -44,3 +46,14 @@ def test_steps_whose_attention_is_one_launch(case):
     lib = library.load("prefill_attention_bf16", ("-DHEAD_DIM=64",))
     assert bool(lib.mie_step_attention_takes(*case[:-1])) == case[-1]
     assert not library.load("prefill_attention_bf16", ("-DHEAD_DIM=128",)).mie_step_attention_takes(*case[:-1])
+
+
+# rows, columns, K and the parts that a long K is added in: one workgroup a compute unit, two of three to five parts, never two of two parts
+@pytest.mark.parametrize("case", [(129, 2048, 5632, 8), (512, 4096, 14336, 2), (384, 4096, 14336, 5), (385, 4104, 4096, 3), (300, 8192, 4096, 0), (384, 8192, 14336, 0),
+                                  (512, 6144, 8192, 0), (256, 8192, 4096, 2), (513, 4096, 4096, 0), (512, 8192, 4096, 0), (300, 4096, 4032, 0)])
+def test_parts_of_a_long_k(case):
+    M, N, K, units = case
+    o = HipBackend.__new__(HipBackend)
+    o.true_fp32 = False
+    x, w = (torch.empty(n, K, dtype=torch.bfloat16, device="meta") for n in (M, N))
+    assert o._tile_split(x, w, None) == units
