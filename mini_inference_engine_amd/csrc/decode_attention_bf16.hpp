@@ -19,7 +19,7 @@
 // in the LDS by loads that write the LDS directly, whole cache lines, and reads the fragments back; a slot is refilled as soon as
 // its fragments are in registers, so all of a wave's slots are on their way while it computes.  Straight into registers in the
 // matrix instruction's order a quarter wave touches 16 rows for 16 (keys) or 8 bytes (values), and the address unit's line look-ups
-// keep a compute unit below the 58 bytes a nanosecond that it can take in.  Measured (MI355X, attention and merge, us, before / now): 32 / 4
+// keep a compute unit far below the 75 to 97 bytes a nanosecond that whole lines come in at.  Measured (MI355X, attention and merge, us, before / now): 32 / 4
 // heads of 64, 64 rows of 200 to 1,990 keys 21.8 / 20.5, 96 rows 32.9 / 28.6, 32 rows of 150 to 900 13.4 / 11.8, 8 of 2,040 10.7 / 10.5; 32 / 8
 // heads of 128, 8 rows of 1,000 to 6,000 41.6 / 35.3, 64 of 200 to 1,990 73.0 / 63.9.  At head size 32 registers are the faster way (64
 // rows of 2,040 keys 17.3 us, 19.1 through the LDS).

@@ -17,9 +17,10 @@
 // slot at once, and then they are multiplied.  Within a row the eight blocks are permuted (block b at 16-byte place
 // 8 r + (b ^ r % 8)), so that the fragment reads (lane 16 b + r) are spread over all banks.  No barrier in the loop: a wave
 // reads only what it brought in itself.  Up to 8 rows bring in half as much x.
-// Loads are all a compute unit can take in, 58 bytes a nanosecond, hits or not, so none is made for nothing: nothing behind a
-// wave's quarter is asked for (three slots of zeros a wave were, a quarter of all loads at K = 2,048), and tiles share a workgroup's
-// x.  Measured alone (MI355X, us, 1 / 8 / 16 rows, before and now): [2048, 2048] 4.5 / 4.7 / 5.1 and 4.1 / 4.5 / 4.9, [2048, 5632] 7.8 /
+// Loads are what these kernels spend their time on (58 bytes a nanosecond and compute unit with their address arithmetic; whole lines
+// come in at 75 to 97 where an address is one addition, see tile_gemm_bf16.hip), so none is made for nothing: nothing behind a wave's
+// quarter is asked for (three slots of zeros a wave were, a quarter of all loads at K = 2,048), and tiles share a workgroup's x.
+// Measured alone (MI355X, us, 1 / 8 / 16 rows, before and now): [2048, 2048] 4.5 / 4.7 / 5.1 and 4.1 / 4.5 / 4.9, [2048, 5632] 7.8 /
 // 8.2 / 9.7 and 7.0 / 7.9 / 9.6, [11264, 2048] 10.2 / 10.2 / 11.1 and 9.6 / 9.7 / 9.9, [32000, 2048] 24.9 / 25.1 / 27.2 and 21.7 / 21.3 /
 // 22.1, [6144, 4096] 11.4 / 12.6 / 14.4 and 10.8 / 11.2 / 12.3, [28672, 4096] 38.9 / 40.3 / 42.0 and 37.4 / 37.9 / 39.3.
 // With the norm in front fused in, as the engine runs them: [11264, 2048] 10.0 / 10.7 / 10.9, [32000, 2048] 23.3 / 24.5 / 26.5, [6144, 4096]

@@ -5,8 +5,8 @@
 //
 // The few-row kernel (gemm_bf16.hip) gives every 16 weight rows a workgroup that reads all of x, which at 64 rows is four
 // times the weights' bytes; a library product runs a narrow weight on a few dozen workgroups.  What a compute unit takes in
-// is what bounds these products: 58 bytes a nanosecond at most, out of the L2 as well as from memory (measured by a kernel
-// that only loads, whatever the access pattern, the depth or who shares the lines).  So a workgroup owns TW tiles of 16
+// is what bounds these products: 58 bytes a nanosecond, out of the L2 as well as from memory, by loads whose addresses cost some
+// forty scalar instructions each as here (75 to 97 where an address is one addition, see tile_gemm_bf16.hip).  So a workgroup owns TW tiles of 16
 // weight rows, as many as give every compute unit one workgroup, and x is read once per 16 TW weight rows.
 //
 // Its waves share no loads and meet at no barrier in the loop: chunks of 64 k are dealt to them in turn, a wave brings a

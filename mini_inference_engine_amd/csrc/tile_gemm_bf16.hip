@@ -619,7 +619,7 @@ static long tiles_of(int i, int M, int N) {
 // tiles are faster (us, own / library: 2,048 rows of [6144, 4096] 103 / 88, of [8192, 4096] 122 / 114, of [28672, 4096] 480 / 428).  Two
 // workgroups a compute unit take 1.55 times one's time.  With one round, us, own / library (which for q/k/v leaves the rotation, 8 to 9 us
 // more, to a kernel of its own): added, [2048, 2048] 160 rows 9.7 / 12.3, 512 10.4 / 12.2, 1,132 16.9 / 19.5, 2,048 22.4 / 23.5; [2048, 5632]
-// 768 31.8 / 33.3, 1,132 35.7 / 44.7, 2,048 47.3 / 55.1; [4096, 4096] 512 26.4 / 30.0, 2,048 62.1 / 66.3; [4096, 14336] 1,024 113 / 132, 2,048
+// 768 31.8 / 33.3, 1,132 35.7 / 44.7, 2,048 47.3 / 55.1; [4096, 4096] 2,048 62.1 / 66.3; [4096, 14336] 1,024 113 / 132, 2,048
 // 187 / 197; q/k/v, [2560, 2048] 160 rows 10.7 / 12.7, 512 12.6 / 14.6, 1,132 19.6 / 20.8, 2,048 28.8 / 28.4; [6144, 4096] 256 27.8 / 26.7, 512
 // 38.5 / 36.6, 1,024 52.9 / 52.4.
 static int tile_for(int M, int N, int K) {
@@ -726,10 +726,13 @@ MIE_EXPORT int mie_tile_gemm_qkv_rope(const void* X, long ldx, const void* W, lo
   return launch_tile<TG_ROPE>(arguments(X, ldx, W, ldw, q_out, ldq, M, N), rope, K, s);
 }
 
-// Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: measured at
-// 160 to 2,048 rows of [11264, 2048] (MI355X).  256 x 192 and wider are tile_lean_kernel's, the others tile_gemm_kernel's, of which
-// the first 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  Own tile of before / now, us: 160 rows 25.2 / 22.4, 256 26.0 /
-// 23.9, 384 36.8 / 30.2, 512 34.1 / 31.1, 768 45.7 / 36.3, 1,536 73.0 / 62.6, 2,048 93.8 / 76.9.
+// Time of a stage (64 k) of a grid that gives every compute unit one workgroup, with its share of the start and the end, us: the numbers
+// that the choice goes by, measured on kernels before these.  256 x 192 and wider are tile_lean_kernel's, the others
+// tile_gemm_kernel's, of which the first 128 x 128 is for the estimate alone (mie_tile_gemm_swiglu_cost).  The present kernels' at [11264, 2048]
+// (MI355X, weights from memory, one round, few to all rows of the tiles): 128 x 128 0.58 to 0.71, 128 x 192 0.72 to 0.93, 192 x 128 0.73 to 0.85,
+// 256 x 128 0.84 to 0.95, 192 x 192 0.87 to 1.08, 256 x 192 1.29 to 1.48, 256 x 256 1.31 to 1.68, 256 x 320 1.79 to 2.06, 256 x 384 1.92 to 2.36.  The
+// order is the same, and so is the choice: of 22 numbers of rows from 129 to 2,048, with every tile timed, it was within 3 % of the best tile,
+// but at 300 and 333, where 192 x 128 takes 23.8 and 25.3 us for 26.2 of 128 x 192.
 constexpr struct { int bm, bn; float us; } TILE_STAGE_US[] = {
   {128, 128, 0.76f}, {192, 128, 0.98f}, {256, 128, 0.99f}, {256, 192, 1.33f}, {256, 256, 1.57f}, {256, 384, 2.35f},
   {128, 128, 0.72f}, {128, 192, 0.96f}, {192, 192, 1.12f}, {256, 320, 1.94f}};

@@ -432,9 +432,10 @@ class HipBackend(KernelBackend):
     def _tile_swiglu_gains(self, x, w, intermediate) -> bool:
         """Whether the own gate/up product with SwiGLU on its sums beats the library's and silu_mul: its estimate (a stage's time
         of each tile times the rounds of its grid) against what the library was measured at, 7 us + weights at 3.5 TB/s +
-        1.2 PFLOP/s, for K up to 2,048 (us, [11264, 2048]: 256 rows 25 / 30, 512 33.6 / 35.6, 1,132 55 / 60, 1,536 86 / 83 by
-        the library, 2,048 90 / 96; at K = 4,096 the library's largest tiles are as fast: 1,024 rows of [28672, 4096] 212 /
-        221, 2,048 403 / 395)."""
+        1.2 PFLOP/s, for K up to 2,048.  Weights from memory, us, own / library and silu_mul: [11264, 2048] 160 rows 19.4 / 27.8, 256 22.9 /
+        30.9, 512 28.7 / 37.0, 1,132 51.0 / 57.5, 1,536 63.7 / 82.4, 2,048 74.7 / 96.8; [16384, 2048] 1,024 56.7 / 67.4.  The estimate keeps
+        the library where it would lose, too (1,300 rows of [11264, 2048] 62.4 / 76.0).  At K = 4,096 the two are within 3 to 14 % of each
+        other, either way ([28672, 4096] 160 rows 77.3 / 64.0, 512 103.7 / 110.4, 2,048 363 / 376)."""
         M, K = x.shape
         if K > 2048 or intermediate % 8 or not self._tile_ok(x, w, None):
             return False
